@@ -248,6 +248,9 @@ const QmvRule kQmvRules[] = {
                                             // calls have passed, e.g. on operands that are not 16-byte aligned, or with the
                                             // diagonal and dot2 families switched off: this kernel is faster at long K,
                                             // 15.6 against 2 x 9 us at 8 rows of 14336 x 4096, but not row by row the same bytes)
+    {4, 32, 0, 3, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
+    {8, 32, 0, 2, 32, kFamTok},
+    {0, 128, 0, 5, 32, kFamTok},
     {0, 0, 0, 9, 64, kFamTilesLarge},       // 16 Mi codes and more: the 16-row block-MFMA kernel is bound by its 4x4x4 MFMAs
     {0, 0, 0, 2, 16, kFamBlk},              // the whole call in one launch of up to 16 rows (4 where K is long)
     {8, 0, 0, 1, 1, kFamBlk},               // (a single row of 4-bit codes is faster on the dot2 kernels)
@@ -325,10 +328,15 @@ int run_diag(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool g
     return kPass;
 }
 
+// Groups of 64 with a K that ends inside a run of 256 codes: matrices of fewer than 4 Mi codes stay with the families behind
+// (a workgroup per 16 rows does not fill the chip then, and its fixed cost is what is left).
+bool tok_small(int group_size, int K, int64_t rows) { return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20; }
+
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
     const int ti = forced >= 0 ? forced : aq::qmvt_pick(bits, a.M, a.K, a.N, ctx->cu_count);
-    if (gather || ti < 0 || !aq::qmvt_fits(a, bits, group_size, ti)) return kPass;
-    ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
+    if (gather || ti < 0 || !aq::qmvt_fits(a, bits, group_size, ti, forced >= 0)) return kPass;
+    if (forced < 0 && tok_small(group_size, a.K, a.N)) return kPass;
+    ctx->last_variant[0] = aq::qmvt_name(ti, a);
     AQ_HIP(aq::qmvt_launch(ti, a, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -379,6 +387,15 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
         if (rc != kPass) return rc;
     }
     return fail(AQ_ERR_UNSUPPORTED, "aq_qmv: no kernel for bits=%d group=%d rows=%d K=%d N=%d", bits, group_size, a.M, a.K, a.N);
+}
+
+// Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
+// the launch forms that put several matrices into one grid).
+bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows) {
+    if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(group_size, K, rows)) return false;
+    if (bits == 4 && group_size == 64) return M >= 9 && M <= 32;
+    if (bits == 8 && group_size == 64) return (M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0) && M >= 2 && M <= 32;
+    return M <= 32 && M >= (group_size == 128 ? 5 : bits == 4 ? 3 : 2);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -699,6 +716,38 @@ int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, c
     return launch_qmv_rows(ctx, a, group_size, bits, false);
 }
 
+namespace {
+aq::QmvMultiArgs multi_args(const void* x, int count, const void* const* packed, const void* const* scales,
+                            const void* const* biases, void* const* y, const int* N, int M, int K, int group_size, unsigned flags) {
+    aq::QmvMultiArgs ma{};
+    ma.common.x = static_cast<const uint16_t*>(x);
+    ma.common.K = K;
+    ma.common.M = M;
+    ma.common.gs_shift = is_pow2(group_size) ? ilog2(group_size) : 0;
+    ma.common.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
+    ma.common.routes = 1;
+    ma.common.tiled = (flags & AQ_W_TILED) ? 1 : 0;
+    ma.count = count;
+    for (int i = 0; i < count; i++) {
+        ma.w[i] = static_cast<const uint32_t*>(packed[i]);
+        ma.s[i] = static_cast<const uint16_t*>(scales[i]);
+        ma.b[i] = static_cast<const uint16_t*>(biases[i]);
+        ma.y[i] = y[i];
+        ma.N[i] = N[i];
+    }
+    return ma;
+}
+aq::QmvArgs multi_member(const aq::QmvMultiArgs& ma, int i) {
+    aq::QmvArgs one = ma.common;
+    one.w = ma.w[i];
+    one.s = ma.s[i];
+    one.b = ma.b[i];
+    one.y = ma.y[i];
+    one.N = ma.N[i];
+    return one;
+}
+}  // namespace
+
 int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packed, const void* const* scales,
                  const void* const* biases, void* const* y, const int* N, int M, int K, int group_size, int bits,
                  unsigned flags) {
@@ -737,29 +786,8 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             const int di = (ctx->families_off >> kFamDiag & 1) ? -1 : aq::qmvd_pick(M, K, (int)total);
             if (di >= 0 && aq::qmvd_multi_supported(di)) {
                 bool fits = true;
-                aq::QmvMultiArgs ma{};
-                ma.common.x = static_cast<const uint16_t*>(x);
-                ma.common.K = K;
-                ma.common.M = M;
-                ma.common.gs_shift = ilog2(group_size);
-                ma.common.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
-                ma.common.routes = 1;
-                ma.common.tiled = tiled ? 1 : 0;
-                ma.count = count;
-                for (int i = 0; i < count; i++) {
-                    ma.w[i] = static_cast<const uint32_t*>(packed[i]);
-                    ma.s[i] = static_cast<const uint16_t*>(scales[i]);
-                    ma.b[i] = static_cast<const uint16_t*>(biases[i]);
-                    ma.y[i] = y[i];
-                    ma.N[i] = N[i];
-                    aq::QmvArgs one = ma.common;
-                    one.w = ma.w[i];
-                    one.s = ma.s[i];
-                    one.b = ma.b[i];
-                    one.y = y[i];
-                    one.N = N[i];
-                    fits = fits && aq::qmvd_fits(one, bits, group_size, false, di);
-                }
+                const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
+                for (int i = 0; i < count; i++) fits = fits && aq::qmvd_fits(multi_member(ma, i), bits, group_size, false, di);
                 if (fits) {
                     ctx->last_variant[0] = "qmv_multi_diag";
                     AQ_HIP(aq::qmvd_multi_launch(di, ma, ctx->stream), "hipLaunchKernel");
@@ -769,25 +797,30 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             const int idx = M == 1 && !tiled ? pick_qmv_variant(ctx, bits, 1, false, (int)total, K, 1) : -1;
             const int rows = idx >= 0 ? aq::qmv_variant(idx)->rows : 0;
             if (rows > 0 && aq::qmv_multi_supported(bits, 1, rows)) {
-                aq::QmvMultiArgs ma{};
-                ma.common.x = static_cast<const uint16_t*>(x);
-                ma.common.K = K;
-                ma.common.M = 1;
-                ma.common.gs_shift = ilog2(group_size);
-                ma.common.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
-                ma.common.routes = 1;
-                ma.count = count;
-                for (int i = 0; i < count; i++) {
-                    ma.w[i] = static_cast<const uint32_t*>(packed[i]);
-                    ma.s[i] = static_cast<const uint16_t*>(scales[i]);
-                    ma.b[i] = static_cast<const uint16_t*>(biases[i]);
-                    ma.y[i] = y[i];
-                    ma.N[i] = N[i];
-                }
+                const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, 1, K, group_size, flags);
                 ctx->last_variant[0] = "qmv_multi_dot2";
                 AQ_HIP(aq::qmv_multi_launch(bits, 1, rows, ma, ctx->stream), "hipLaunchKernel");
                 return AQ_OK;
             }
+        }
+    }
+    if (!tiled && count > 1 && M > 1 && K > 0 && (bits == 4 || bits == 8) && check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK) {
+        // several rows: the token-tile kernels over all matrices in one grid
+        int64_t total = 0;
+        for (int i = 0; i < count; i++) total += N[i];
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        const int ti = total < (int64_t)1 << 30 && tok_runs(ctx, bits, group_size, M, K, total)
+                           ? aq::qmvt_pick(bits, M, K, (int)total, ctx->cu_count) : -1;
+        aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
+        bool fits = ti >= 0;
+        for (int i = 0; fits && i < count; i++) {
+            const aq::QmvArgs one = multi_member(ma, i);
+            fits = N[i] > 0 && aligned(y[i], 2) && aq::qmvt_fits(one, bits, group_size, ti, false);
+        }
+        if (fits) {
+            ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
+            AQ_HIP(aq::qmvt_multi_launch(ti, ma, ctx->stream), "hipLaunchKernel");
+            return AQ_OK;
         }
     }
     for (int i = 0; i < count; i++)
@@ -1058,6 +1091,32 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
             a.act = act;
             ctx->last_variant[0] = "qmv_gate_up_dot2";
             AQ_HIP(aq::qmv_act_launch(bits, 1, rows, false, a, ctx->stream), "hipLaunchKernel");
+            return AQ_OK;
+        }
+    }
+    if (M > 1 && tok_runs(ctx, bits, group_size, M, K, N)) {
+        // the token-tile kernels with half of a workgroup's rows in either matrix
+        aq::QmvArgs a{};
+        a.x = static_cast<const uint16_t*>(x);
+        a.w = static_cast<const uint32_t*>(gate_packed);
+        a.s = static_cast<const uint16_t*>(gate_scales);
+        a.b = static_cast<const uint16_t*>(gate_biases);
+        a.w2 = static_cast<const uint32_t*>(up_packed);
+        a.s2 = static_cast<const uint16_t*>(up_scales);
+        a.b2 = static_cast<const uint16_t*>(up_biases);
+        a.y = y;
+        a.K = K;
+        a.N = N;
+        a.M = M;
+        a.gs_shift = is_pow2(group_size) ? ilog2(group_size) : 0;
+        a.out_f32 = out_f32 ? 1 : 0;
+        a.routes = 1;
+        a.act = act;
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        const int ti = aq::qmvt_pick_pair(bits, M, K, N, ctx->cu_count);
+        if (ti >= 0 && aq::qmvt_pair_supported(ti) && aq::qmvt_fits(a, bits, group_size, ti, false)) {
+            ctx->last_variant[0] = "qmv_gate_up_tok";
+            AQ_HIP(aq::qmvt_pair_launch(ti, a, ctx->stream), "hipLaunchKernel");
             return AQ_OK;
         }
     }

@@ -10,6 +10,12 @@ namespace aq {
 // Operands of one affine matvec / gathered matvec launch.  Layouts follow the
 // MLX group-affine format (go/model/quant/mlxaffine/mlxaffine.go:14-20):
 //   w [rows, K*bits/32] u32, s/b [rows, K/group] bf16, x [x_rows, K] bf16.
+// Up to 32 (token-tile kernels) or more routes that name the same expert: places [first, first + count) of the list of
+// routes sorted by expert (aq_moe_group.hip).  count 0: behind the end of the list.
+struct RouteChunk {
+    int expert, first, count, pad;
+};
+
 struct QmvArgs {
     // (What a kernel needs before it can request its weights sits in the first 64 bytes of the kernel arguments: one
     // scalar load and one wait at the start of a wavefront instead of one per cache line.)
@@ -39,6 +45,11 @@ struct QmvArgs {
     const uint16_t* s2;
     const uint16_t* b2;
     int row_base2;       // pair fusion + gather: first `up` row inside an expert's slab
+    // routes grouped by expert (token-tile kernels): the chunks, and per place of the sorted list the row of x and the
+    // route (negative: the route's ids are out of range, its outputs are zeros; the route is the value without its sign bit)
+    const RouteChunk* chunks;
+    const int32_t* route_x;
+    const int32_t* route_of;
     int act;             // kActGeluTanh or kActSilu
     // head kernels only (aq_qmv_head.hip): y is uint64 best[M] (argmax) or uint64 scores[M, N]
     const int32_t* suppress;  // token ids that may not win, or nullptr
@@ -156,13 +167,21 @@ hipError_t head_fold_launch(const unsigned long long* partial, int count, unsign
 bool qmvd_multi_supported(int idx);
 hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
 
-// Token-tile MFMA matvec kernels (aq_qmv_tok.hip; group-64 codes of 4 or 8 bits, up to 32 activation rows as
-// the rows of 16x16x32 MFMAs, K a multiple of 256 up to 16384; one launch, no scratch memory).  kind 6 in QmvVariant.
+// Token-tile MFMA matvec kernels (aq_qmv_tok.hip; codes of 4 or 8 bits in groups of 32, 64 or 128, up to 32 activation rows
+// as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch, no scratch memory).  kind 6 in QmvVariant.
 int qmvt_variant_count();
 const QmvVariant* qmvt_variant(int idx);
-bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx);
+// (exact_only: groups of 64 with K a multiple of 256 only, what a forced variant takes)
+bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_only);
+const char* qmvt_name(int idx, const QmvArgs& a);  // the kernel qmvt_launch runs for this call
 hipError_t qmvt_launch(int idx, const QmvArgs& a, hipStream_t stream);
-int qmvt_pick(int bits, int M, int K, int N, int cu_count);
+int qmvt_pick(int bits, int M, int K, int rows, int cu_count);
+// Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
+// sums are those of qmvt_launch.
+hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
+int qmvt_pick_pair(int bits, int M, int K, int N, int cu_count);
+bool qmvt_pair_supported(int idx);
+hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream);
 
 // lm_head kernels (aq_qmv_head.hip), one activation row: the projection with its epilogue replaced by
 //   fuse 3: best[0] = max over rows of pack(score, row): every wavefront stores its own maximum into

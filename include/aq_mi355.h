@@ -131,8 +131,11 @@ int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, c
  * pointers.  Results are byte-identical to `count` separate aq_qmv calls.  This is the no-copy form of
  * running q|k|v or gate|up over model.ConcatQuantRows (go/model/quant_weight.go:32-62): at batch 1 the
  * narrow projections are bound by launch latency, not bandwidth, and one grid over all of them fills
- * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384);
- * shapes the fused kernels do not take are run as separate launches. */
+ * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384), and for
+ * the row counts the token-tile kernels run (9..32 rows of 4-bit group-64 codes, 3..32 of group 32, 5..32 of group 128,
+ * 2..32 of 8-bit codes); other shapes are run as separate launches.  (Byte-identity has one exception: 9..32 rows in
+ * groups of 64 with a K that is no multiple of 256, where a separate call on a matrix of under 4 Mi codes sums in another
+ * order.) */
 int aq_qmv_multi(aq_ctx *ctx, const void *x, int count, const void *const *packed, const void *const *scales,
                  const void *const *biases, void *const *y, const int *N, int M, int K, int group_size, int bits,
                  unsigned flags);
@@ -198,8 +201,8 @@ int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *sc
  * launch go/engine/hip/hip_projection_launch.go:3086-3160, packet contract/launch_abi.hipinc:634-657).
  * gate and up are [N, K*bits/32] with their own scales/biases; for a row-concatenated gate|up slab
  * (model.ConcatQuantRows, go/model/quant_weight.go:32-62) pass the slab for gate and slab + N rows for up.
- * M == 1 with 4/8-bit codes (up to 4 rows of 4-bit group-64 codes when K is a multiple of 256 between 1280 and 8192) runs as ONE launch
- * that reads every weight once; other shapes run the two
+ * M == 1 with 4/8-bit codes (up to 4 rows of 4-bit group-64 codes when K is a multiple of 256 between 1280 and 8192; up to 32
+ * rows where aq_qmv runs its token-tile kernels) runs as ONE launch that reads every weight once; other shapes run the two
  * projections and the element-wise step as separate launches through the context's workspace (which grows
  * on demand like aq_qmm's; not while a capture is open). */
 int aq_qmv_gate_up(aq_ctx *ctx, const void *x, const void *gate_packed, const void *gate_scales,

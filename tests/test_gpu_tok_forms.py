@@ -1,0 +1,72 @@
+"""The token-tile kernels beyond groups of 64 with whole runs of 256 codes: groups of 32 and 128, a K that ends inside a
+run, several matrices in one grid and the gated pair.  Accumulators within the stated bounds of the float64 reference."""
+import numpy as np
+import pytest
+
+import fixtures as F
+from gpu_util import DeviceAffine, check_accumulators, check_bf16_store, run_qmv, say
+
+pytestmark = pytest.mark.gpu
+
+# K: one piece of a run, a run and a piece, every number of 64-code blocks in the last run, one run per wavefront and more
+SHAPES = [(bits, 32, M, K, N) for bits in (4, 8) for M, K, N in ((3, 64, 40), (16, 192, 1030), (17, 320, 70), (32, 4096, 16), (9, 4032, 130))]
+SHAPES += [(bits, 128, M, K, N) for bits in (4, 8) for M, K, N in ((5, 128, 33), (16, 2944, 66), (32, 4096, 49))]
+SHAPES += [(bits, 64, M, K, N) for bits in (4, 8) for M, K, N in ((9, 960, 4400), (16, 2112, 2001), (32, 4032, 1056))]
+
+
+@pytest.mark.parametrize("bits,gs,M,K,N", SHAPES)
+def test_token_tile_forms(ctx, bits, gs, M, K, N):
+    say("token tile", bits, gs, M, K, N)
+    words, s, b = F.synthetic_affine(N, K, bits, gs, seed=2100 + K)
+    x = F.synthetic_x(M, K, seed=2101 + M)
+    ref = F.reference_f64(x, words, s, b, bits, gs, K)
+    dw = DeviceAffine(ctx, words, s, b)
+    acc = run_qmv(ctx, x, dw, M, K, N, gs, bits, True)
+    name = ctx.last_variant(0)
+    exact = gs == 64 and K % 256 == 0
+    assert name.startswith("qmvt_b%d_" % bits) and name.endswith("_s32" if gs == 32 else "_d2" if exact else "_any"), name
+    check_accumulators(acc, ref, name)
+    out = run_qmv(ctx, x, dw, M, K, N, gs, bits, False)
+    assert np.array_equal(out, F.f32_to_bf16_bits(acc).reshape(M, N))
+    dw.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K,Ns", [(4, 64, 12, 4032, (1056, 200, 17)), (4, 32, 4, 3840, (130, 64, 1)), (8, 64, 20, 2048, (512, 96)),
+                                            (8, 32, 2, 960, (40, 50, 60, 70)), (4, 128, 32, 1024, (256, 300))])
+def test_several_matrices_in_one_grid(ctx, bits, gs, M, K, Ns):
+    say("token tile multi", bits, gs, M, K, Ns)
+    mats = [F.synthetic_affine(n, K, bits, gs, seed=2200 + i) for i, n in enumerate(Ns)]
+    x = F.synthetic_x(M, K, seed=2250)
+    dws = [DeviceAffine(ctx, *m) for m in mats]
+    dx, ys = ctx.to_device(x), [ctx.alloc(M * n * 2) for n in Ns]
+    ctx.qmv_multi(dx, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, list(Ns), M, K, gs, bits)
+    ctx.sync()
+    assert ctx.last_variant(0).startswith("qmvt_"), ctx.last_variant(0)
+    for n, m, y in zip(Ns, mats, ys):
+        check_bf16_store(y.download(np.uint16, M * n), F.reference_f64(x, *m, bits, gs, K), "member of %d rows" % n)
+    for t in [dx] + ys + dws:
+        t.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K,N", [(4, 32, 21, 3840, 1000), (4, 64, 9, 4096, 77), (8, 64, 32, 960, 4400), (8, 32, 2, 192, 33),
+                                           (4, 128, 16, 640, 48)])
+def test_gated_pair(ctx, orc, bits, gs, M, K, N):
+    """act(gate . x) * (up . x) in one launch from the sums of the separate projections."""
+    say("token tile gate|up", bits, gs, M, K, N)
+    gate, up = F.synthetic_affine(N, K, bits, gs, seed=2300), F.synthetic_affine(N, K, bits, gs, seed=2301)
+    x = F.synthetic_x(M, K, seed=2302)
+    dg, du = DeviceAffine(ctx, *gate), DeviceAffine(ctx, *up)
+    g = run_qmv(ctx, x, dg, M, K, N, gs, bits, True)
+    u = run_qmv(ctx, x, du, M, K, N, gs, bits, True)
+    dx, dy = ctx.to_device(x), ctx.alloc(M * N * 4)
+    import aq_mi355
+    for act in (aq_mi355.AQ_ACT_GELU_TANH, aq_mi355.AQ_ACT_SILU):
+        ctx.qmv_gate_up(dx, (dg.w, dg.s, dg.b), (du.w, du.s, du.b), dy, M, K, N, gs, bits, act, aq_mi355.AQ_OUT_F32)
+        ctx.sync()
+        assert ctx.last_variant(0) == "qmv_gate_up_tok"
+        got = dy.download(np.float32, M * N).reshape(M, N)
+        want = orc.act_multiply(act, g, u)
+        # the same fp32 sums; tanh and exp of the device library against the oracle's: a few fp32 ulp
+        assert (np.abs(got - want) <= 4e-6 * np.abs(want) + 2.5e-7 * np.maximum(1.0, np.abs(g * u))).all()
+    for t in (dx, dy, dg, du):
+        t.free()
