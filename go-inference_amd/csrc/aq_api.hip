@@ -430,7 +430,7 @@ int launch_qmv_tiled(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits) {
             return fail(AQ_ERR_ARG, "aq_qmv: forced variant %d does not fit tile-major weights with rows=%d K=%d N=%d", forced, a.M,
                         a.K, a.N);
     }
-    const size_t region = aq::qmm_scratch_bytes(a.M, a.K, a.N);
+    const size_t region = aq::qmm_scratch_bytes(a.M, a.K, a.N, ctx->cu_count);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + untiled_bytes(a.N, a.K), fail)) return rc;
     if (int rc = untile_into_ws(ctx, region, a.w, a.N, a.K, &a.w, &a.s, &a.b)) return rc;
@@ -868,13 +868,13 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     if (M <= 0 || K <= 0) return fail(AQ_ERR_SHAPE, "aq_qmm_multi: M, N, K must be positive");
     if (int rc = check_geometry("aq_qmm_multi", K, group_size, bits)) return rc;
     if (!x || !aligned(x, 2)) return fail(AQ_ERR_ARG, "aq_qmm_multi: null or misaligned x");
-    size_t need = 0;
+    size_t need = 0, half_need = 0;
     for (int i = 0; i < count; i++) {
         if (N[i] <= 0) return fail(AQ_ERR_SHAPE, "aq_qmm_multi: M, N, K must be positive");
         if (!packed[i] || !scales[i] || !biases[i] || !y[i]) return fail(AQ_ERR_ARG, "aq_qmm_multi: null operand");
         if (!aligned(packed[i], 4) || !aligned(scales[i], 2) || !aligned(biases[i], 2) || !aligned(y[i], 2))
             return fail(AQ_ERR_ARG, "aq_qmm_multi: operand pointer is not element-aligned");
-        const size_t n = aq::qmm_scratch_bytes(M, K, N[i]);
+        const size_t n = aq::qmm_scratch_bytes(M, K, N[i], ctx->cu_count);
         need = n > need ? n : need;
     }
     if (M <= aq::kQmvMaxRows && ctx->forced[1] < 0) {
@@ -888,11 +888,44 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     }
     std::lock_guard<std::mutex> lk(ctx->mu);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    // the largest member's scratch first, so that no member makes the workspace move under the pass over x
-    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
+    // the members that the fp16-operand kernels take run as one grid (same bytes as on their own, see qmmh_split): narrow
+    // matrices (k and v beside q) then fill the rounds of tiles that the wide ones leave part-empty
+    aq::QmmHalfCall q{};
+    unsigned in_grid = 0;
+    if (ctx->forced[1] < 0)
+        for (int i = 0; i < count; i++) {
+            if (!aq::qmmh_takes(x, packed[i], K, group_size, bits) || !aq::qmmh_runs(M, K, N[i], group_size)) continue;
+            aq::QmmSegment& seg = q.seg[q.nseg++];
+            seg.w = static_cast<const uint32_t*>(packed[i]);
+            seg.s = static_cast<const uint16_t*>(scales[i]);
+            seg.b = static_cast<const uint16_t*>(biases[i]);
+            seg.y = y[i];
+            seg.N = N[i];
+            aq::qmmh_split(M, K, &seg, ctx->cu_count);
+            in_grid |= 1u << i;
+        }
+    if (q.nseg > 0) {
+        q.x = static_cast<const uint16_t*>(x);
+        q.M = M;
+        q.K = K;
+        q.group_size = group_size;
+        q.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
+        half_need = aq::qmm_scratch_bytes(M, K, 0, ctx->cu_count) + aq::qmmh_partial_bytes(q);
+        need = half_need > need ? half_need : need;
+    }
+    // the largest scratch first, so that no member makes the workspace move under the pass over x
+    if (!(q.nseg == count && !aq::workspace_may_grow(&ctx->ws, need, ctx->stream)))
+        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
     int x_state = aq::kXReadyNone;
+    if (q.nseg > 0) {
+        const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, -1, q, &ctx->last_variant[1], fail, &x_state);
+        if (rc != AQ_OK && rc != aq::kQmmhNoScratch) return rc;
+        if (rc == aq::kQmmhNoScratch) in_grid = 0;
+    }
     for (int i = 0; i < count; i++)
-        if (int rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], x, packed[i],
+        if (in_grid >> i & 1)
+            continue;
+        else if (int rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], x, packed[i],
                                       scales[i], biases[i], y[i], M, K, N[i], group_size, bits, (flags & AQ_OUT_F32) != 0, fail,
                                       nullptr, 0, &x_state))
             return rc;
@@ -967,7 +1000,7 @@ bool act_ok(int act) { return act == AQ_ACT_GELU_TANH || act == AQ_ACT_SILU; }
 
 // Bytes of the workspace the matmul path may claim for an M x K by N call (activations in fragment order,
 // partial tiles of a K split), 256-byte aligned: the unfused fallbacks keep their intermediates behind it.
-size_t qmm_region(int M, int K, int N) { return aq::qmm_scratch_bytes(M, K, N); }
+size_t qmm_region(const aq_ctx* ctx, int M, int K, int N) { return aq::qmm_scratch_bytes(M, K, N, ctx->cu_count); }
 
 // Rows per wavefront for the activation-fused dot2 kernels: `slots` row streams a wavefront of the
 // plain kernel would take for this much work, shared between the two matrices of a pair.
@@ -1057,7 +1090,8 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     if (tiled) {
         // no fused tile-major kernel for this call: the MLX arrays of both matrices are rebuilt behind the scratch
         // of the unfused route, which then runs as for any other call
-        const size_t region = qmm_region(M, K, N) + 2 * align256((size_t)M * N * 4);
+        // (a pair's partial tiles are twice a single matrix's)
+        const size_t region = 2 * qmm_region(ctx, M, K, N) + 2 * align256((size_t)M * N * 4);
         std::lock_guard<std::mutex> lk(ctx->mu);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * untiled_bytes(N, K), fail)) return rc;
@@ -1120,8 +1154,35 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
             return AQ_OK;
         }
     }
+    if (M > 32 && ctx->forced[0] < 0 && ctx->forced[1] < 0 && !(ctx->families_off >> kFamTiles & 1) &&
+        aq::qmmh_takes(x, up_packed, K, group_size, bits) && aq::qmmh_takes(x, gate_packed, K, group_size, bits) &&
+        aq::qmmh_runs(M, K, N, group_size)) {
+        // prefill sizes on the fp16-operand kernels: one launch, the tiles of which hold gate and up columns side by side; no
+        // intermediate reaches memory
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        aq::QmmHalfCall q{};
+        q.x = static_cast<const uint16_t*>(x);
+        q.M = M;
+        q.K = K;
+        q.group_size = group_size;
+        q.nseg = 2;
+        q.pair = 1;
+        q.act = act;
+        q.out_f32 = out_f32 ? 1 : 0;
+        q.seg[0].w = static_cast<const uint32_t*>(gate_packed);
+        q.seg[0].s = static_cast<const uint16_t*>(gate_scales);
+        q.seg[0].b = static_cast<const uint16_t*>(gate_biases);
+        q.seg[1].w = static_cast<const uint32_t*>(up_packed);
+        q.seg[1].s = static_cast<const uint16_t*>(up_scales);
+        q.seg[1].b = static_cast<const uint16_t*>(up_biases);
+        q.seg[0].y = q.seg[1].y = y;
+        q.seg[0].N = q.seg[1].N = N;
+        const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, -1, q, &ctx->last_variant[1], fail, nullptr);
+        if (rc == AQ_OK) ctx->last_variant[0] = "qmv_gate_up_tiles";
+        if (rc != aq::kQmmhNoScratch) return rc;
+    }
     // two projections into fp32 scratch, then the element-wise step
-    const size_t region = qmm_region(M, K, N);
+    const size_t region = qmm_region(ctx, M, K, N);
     const size_t each = (((size_t)M * N * 4) + 255) & ~(size_t)255;
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
@@ -1288,7 +1349,7 @@ int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* pa
             return AQ_OK;
         }
     }
-    const size_t region = qmm_region(M, K, N);
+    const size_t region = qmm_region(ctx, M, K, N);
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
@@ -1536,7 +1597,7 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
         }
     }
     // the projection as fp32 into scratch, then the same epilogue over it
-    const size_t region = qmm_region(M, K, N);
+    const size_t region = qmm_region(ctx, M, K, N);
     {
         std::lock_guard<std::mutex> lk(ctx->mu);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");

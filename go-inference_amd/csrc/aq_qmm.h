@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "aq_kernels.h"
+
 namespace aq {
 
 // Largest M the dot2 matvec kernels take in one pass; a matmul call of up to this many rows runs as a matvec.
@@ -24,7 +26,7 @@ struct QmmArgs {
 };
 
 // Which pass over x the workspace holds (QmmArgs.x_ready, and what a launch reports back through qmm_dispatch).
-enum { kXReadyNone = 0, kXReadyTile4 = 1, kXReadyTile8 = 2, kXReadyHalf = 3 };
+enum { kXReadyNone = 0, kXReadyTile4 = 1, kXReadyTile8 = 2, kXReadyHalf = 3, kXReadyHalf32 = 4 };
 
 struct QmmVariant {
     const char* name;
@@ -66,6 +68,7 @@ int qmmt_x_kind(int idx);
 // The same with K shared out over ksplit workgroups per tile and a second kernel that adds the partial
 // tiles: for few rows of x, where M x N tiles alone leave most of the chip idle.
 size_t qmmt_splitk_bytes(int M, int N, int ksplit);
+int qmmt_gsplit(int K, int ksplit);  // 64-code blocks of K per workgroup
 hipError_t qmmt_launch_splitk(int idx, const QmmArgs& a, void* workspace, int ksplit, hipStream_t stream);
 
 // Kernels for 5..64 rows of x whose LDS stages hold four blocks of K (aq_qmm_few.hip): listed behind the
@@ -75,9 +78,54 @@ const QmmVariant* qmmf_variant(int idx);
 hipError_t qmmf_launch_kernel(int idx, const QmmTileArgs& a, hipStream_t stream);
 
 // 4-bit kernels whose matrix-core operand carries scale * (code - 8) as fp16 (aq_qmm_half.hip); same workspace.
+constexpr int kQmmSegments = 8;  // weight matrices of one call
+struct QmmSegment {
+    const uint32_t* w;
+    const uint16_t* s;
+    const uint16_t* b;
+    void* y;
+    int N;
+    int ksplit, gsplit;    // workgroups that share a tile along K, 64-code blocks of K each takes (qmmh_split)
+    int strips, unit_end;  // filled by the launcher: column strips, and column units (strips x ksplit) up to and with this matrix
+    float* partial;        // filled by the launcher: partial tiles of a K split
+};
+struct QmmHalfArgs {
+    const uint16_t* xf;  // as in QmmTileArgs, fp16
+    const uint16_t* xs;
+    const float* rs;  // per row, the inverse of the power of two it was scaled by
+    QmmSegment seg[kQmmSegments];
+    int nseg, pair;  // pair: seg[0] is the gate matrix, seg[1] the up matrix of a gated MLP; one output
+    int M, K;
+    int gs_blocks, out_f32, act;
+    int mblks, tiles_m;
+    int units;    // column units of all matrices
+    int group_m;  // row bands of a group of tiles
+    // routes grouped by expert (aq_moe_group.hip), or null
+    const RouteChunk* chunks;
+    const int32_t* nchunks;
+    const int32_t* route_of;
+    int expert_rows, row_base, row_base2;
+};
+struct QmmHalfCall {
+    const uint16_t* x;
+    int M, K, group_size;
+    QmmSegment seg[kQmmSegments];
+    int nseg, pair, act, out_f32;
+    int x_ready;  // kXReady*
+    const RouteChunk* chunks;  // expert slabs: most_chunks and most_rows bound what the lists on the device hold
+    const int32_t *nchunks, *route_x, *route_of, *live_rows;
+    int most_chunks, most_rows, expert_rows, row_base, row_base2;
+};
 int qmmh_variant_count();
 const QmmVariant* qmmh_variant(int idx);
-hipError_t qmmh_launch(int idx, const QmmArgs& a, void* workspace, hipStream_t stream);
+int qmmh_rows(int idx);  // rows of x of a workgroup tile
+hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream);
+// How a matrix of seg->N columns shares K out for M rows of x: a function of M, K and N alone, so that the call of several
+// matrices, the gated pair and a call of its own add in the same order and give the same bytes.
+void qmmh_split(int M, int K, QmmSegment* seg, int cu_count);
+// The kernel for these matrices (the bytes of a result do not depend on it).
+int qmmh_pick(const QmmHalfCall& q, int cu_count);
+size_t qmmh_partial_bytes(const QmmHalfCall& q);
 
 // Scratch memory a context lends to the matmul path; grown on demand, never while a capture is open.
 // `generation` counts reallocations: a captured graph has the block's address in its kernel arguments and is
@@ -90,6 +138,10 @@ struct Workspace {
     bool touched = false;
 };
 
+// Whether ws holds `need` bytes or may be made to (not while the stream is being captured): for calls that have another
+// route that needs no scratch.
+bool workspace_may_grow(const Workspace* ws, size_t need, hipStream_t stream);
+
 hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream);
 
 typedef int (*FailFn)(int code, const char* fmt, ...);
@@ -101,7 +153,7 @@ int workspace_reserve(hipStream_t stream, Workspace* ws, size_t need, FailFn fai
 // Upper bound (256-byte aligned) of the workspace bytes qmm_dispatch may use for an M x K by N call: the
 // rewritten activations and, for few rows, the fp32 partial tiles of the K split.  Callers that keep their
 // own data in the same workspace place it behind this.
-size_t qmm_scratch_bytes(int M, int K, int N);
+size_t qmm_scratch_bytes(int M, int K, int N, int cu_count);
 
 // Sizes ws for activations of M x K ahead of time (not during capture).
 int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, FailFn fail);
@@ -115,6 +167,14 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
                  const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
                  int group_size, int bits, bool out_f32, FailFn fail, const float* gate = nullptr, int act = 0,
                  int* x_state = nullptr);
+// Whether the fp16-operand kernels take a call (4-bit codes, groups of 32, 64 or 128, K a multiple of 64).
+bool qmmh_takes(const void* x, const void* packed, int K, int group_size, int bits);
+// Whether an unforced call on one matrix runs on them (the choice among the families by shape).
+bool qmmh_runs(int M, int K, int N, int group_size);
+// One call of them over q.nseg matrices, or on expert slabs (idx < 0: qmmh_pick); x_state as in qmm_dispatch.  Scratch that
+// cannot be had because the stream is being captured: kQmmhNoScratch, nothing launched.
+constexpr int kQmmhNoScratch = INT32_MIN;
+int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCall& q, const char** last_variant, FailFn fail, int* x_state);
 // Whether qmm_dispatch runs this call on the tile kernels, whose stores can carry the gated-MLP epilogue.
 bool qmm_takes_gate(const void* x, const void* packed, int K, int group_size, int bits);
 

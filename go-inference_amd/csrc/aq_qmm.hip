@@ -62,11 +62,17 @@ static int grow_workspace(Workspace* ws, size_t need, hipStream_t stream, FailFn
     return AQ_OK;
 }
 
+bool workspace_may_grow(const Workspace* ws, size_t need, hipStream_t stream) {
+    if (ws->bytes >= need) return true;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    return !(stream != nullptr && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone);
+}
+
 int workspace_reserve(hipStream_t stream, Workspace* ws, size_t need, FailFn fail) {
     return grow_workspace(ws, need, stream, fail);
 }
 
-size_t qmm_scratch_bytes(int M, int K, int N) {
+size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
     const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;
     size_t partial = (M > 4 && M <= 64) ? qmmt_splitk_bytes(M, N, 16) : 0;
     if (M > 64 && (K / 64) % 8 == 0 && K >= 2048) {
@@ -74,6 +80,15 @@ size_t qmm_scratch_bytes(int M, int K, int N) {
         // (qmm_dispatch): k partial tiles of M x N with (M / 128) (N / 128) k <= 2 CUs, bounded here for up to 512 CUs
         const size_t by_k = qmmt_splitk_bytes(M, N, 8), by_cus = (size_t)2 * 512 * 128 * 128 * 4 + ((size_t)M + N) * 128 * 8 * 4;
         partial = by_k < by_cus ? by_k : by_cus;
+    }
+    if (M > 4) {  // the fp16-operand kernels' own split
+        QmmHalfCall q{};
+        q.M = M;
+        q.nseg = 1;
+        q.seg[0].N = N;
+        qmmh_split(M, K, &q.seg[0], cu_count);
+        const size_t half = qmmh_partial_bytes(q);
+        partial = half > partial ? half : partial;
     }
     return xbytes + ((partial + 255) & ~(size_t)255);
 }
@@ -96,6 +111,39 @@ static int find_qmmt_named(const char* name) {
     return -1;
 }
 
+bool qmmh_takes(const void* x, const void* packed, int K, int group_size, int bits) {
+    return bits == 4 && (group_size == 32 || group_size == 64 || group_size == 128) && K % 64 == 0 && K % group_size == 0 &&
+           (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0;
+}
+
+// Groups of 64 / 128 keep the bf16-code kernels where those are ahead: up to 64 rows with K in whole quads of blocks (the
+// few-rows kernels) or a handful of blocks of K, and up to 256 rows by a wide matrix with a short K, where the cheaper pass
+// over x shows (256 x 2048 x 14336; at K = 4096 and 128 x 128 tiles 69 us here against 72).
+bool qmmh_runs(int M, int K, int N, int group_size) {
+    if (group_size == 32) return true;
+    if (M <= 32) return false;
+    if (M <= 64) return K % 256 != 0 && K >= 512;
+    return !(M <= 256 && K <= 2048 && N >= 12288);
+}
+
+int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCall& q, const char** last_variant, FailFn fail, int* x_state) {
+    if (!q.chunks)
+        for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, &q.seg[i], cu_count);
+    const size_t xbytes = (qmmt_workspace_bytes(q.chunks ? q.most_rows : q.M, q.K) + 255) & ~(size_t)255;
+    const size_t need = xbytes + qmmh_partial_bytes(q);
+    if (!workspace_may_grow(ws, need, stream)) return kQmmhNoScratch;
+    const uint64_t generation = ws->generation;
+    if (int rc = grow_workspace(ws, need, stream, fail)) return rc;
+    // (a workspace that had to move no longer holds the earlier pass over x)
+    q.x_ready = x_state && ws->generation == generation ? *x_state : kXReadyNone;
+    if (idx < 0) idx = qmmh_pick(q, cu_count);
+    *last_variant = qmmh_variant(idx)->name;
+    hipError_t rc = qmmh_launch(idx, q, ws->ptr, stream);
+    if (rc != hipSuccess) return fail((int)rc, "rocm.hip.hipLaunchKernel: HIP returned %d (%s)", (int)rc, hipGetErrorString(rc));
+    if (x_state) *x_state = q.group_size == 32 ? kXReadyHalf32 : kXReadyHalf;
+    return AQ_OK;
+}
+
 bool qmm_takes_gate(const void* x, const void* packed, int K, int group_size, int bits) {
     return (bits == 4 || bits == 8) && (group_size == 64 || group_size == 128) && K % 64 == 0 &&
            (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0;
@@ -105,6 +153,22 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
                  const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
                  int group_size, int bits, bool out_f32, FailFn fail, const float* gate, int act, int* x_state) {
     const bool mfma_ok = qmm_takes_gate(x, packed, K, group_size, bits);
+    if (forced < 0 && !gate && qmmh_takes(x, packed, K, group_size, bits) && qmmh_runs(M, K, N, group_size)) {
+        QmmHalfCall q{};
+        q.x = static_cast<const uint16_t*>(x);
+        q.M = M;
+        q.K = K;
+        q.group_size = group_size;
+        q.seg[0].w = static_cast<const uint32_t*>(packed);
+        q.seg[0].s = static_cast<const uint16_t*>(scales);
+        q.seg[0].b = static_cast<const uint16_t*>(biases);
+        q.seg[0].y = y;
+        q.seg[0].N = N;
+        q.nseg = 1;
+        q.out_f32 = out_f32 ? 1 : 0;
+        const int rc = qmmh_run(stream, ws, cu_count, -1, q, last_variant, fail, x_state);
+        if (rc != kQmmhNoScratch) return rc;
+    }
     if (!mfma_ok) {
         if (gate) return fail(AQ_ERR_UNSUPPORTED, "aq_qmm: the gated epilogue needs the tile kernels (4 / 8 bit, groups of 64 / 128)");
         // any other geometry: the any-width matvec kernel walks the rows of x
@@ -144,33 +208,10 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
         const QmmVariant* v = qmmt_variant(tile_idx);
         if (!v || v->bits != bits) return fail(AQ_ERR_ARG, "aq_qmm: forced variant %d does not fit bits=%d", idx, bits);
     } else if (idx < 0 && M >= 64) {
-        // prefill sizes: the LDS-staged 128 x 128 tiles (four 64 x 64 wavefront tiles, two workgroups a CU);
-        // the 128 x 64 wavefront tiles need more registers than two wavefronts a SIMD leave and measure slower
+        // prefill sizes (8 bit; 4 bit where qmmh_runs passes): the LDS-staged 128 x 128 tiles (four 64 x 64 wavefront tiles,
+        // two workgroups a CU); the 128 x 64 wavefront tiles need more registers than two wavefronts a SIMD leave and
+        // measure slower
         tile_idx = find_qmmt(bits, 2, 2, 2, 2);
-        // 4 bit: the kernels whose MFMA operand carries scale * (code - 8) as fp16 (half the vector instructions per
-        // MFMA, no fp32 work on the accumulators) once their tiles cover enough of the chip.  A round of 256 x 256
-        // tiles (eight wavefronts, twice the MFMAs per byte of x copied into LDS) takes 0.121 ms at K = 4096 however
-        // few tiles it holds, a round of 256 x 128 tiles 0.094-0.107 ms, a round of up to 512 of the 128 x 128 tiles
-        // 0.07-0.115 ms; measured on one box, 256 x 256 / 256 x 128 / 128 x 128 (ms): 2048 x 14336 0.277 / 0.305 / 0.32,
-        // 1024 x 14336 0.139 / 0.150 / 0.196, 768 x 14336 0.125 / 0.135 / 0.158, 768 x 12288 0.122 / 0.129 / 0.148,
-        // 768 x 10240 0.122 / 0.103 / 0.110, 2048 x 4096 0.126 / 0.107 / 0.117, 1536 x 4096 0.121 / 0.098 / 0.103,
-        // 512 x 10240 0.121 / 0.094 / 0.094, 512 x 8192 0.121 / 0.095 / 0.071, 256 x 14336 0.120 / 0.094 / 0.067.
-        // Hence: 256 x 256 from 9/16 of a tile per CU, else 256 x 128 above 5/8 of a tile per CU.
-        const int cus = cu_count > 0 ? cu_count : 256;
-        const int64_t mb = (M + 255) / 256;
-        if (bits == 4 && mb * ((N + 255) / 256) * 16 >= (int64_t)cus * 9) {
-            const int wide = find_qmmt_named("qmmh_b4_mb4_nb2_wm2_wn4");
-            if (wide >= 0) tile_idx = wide;
-            // 192 x 256 tiles where their rounds cost a tenth less than those of the 256 x 256 tiles (a round of them
-            // takes 0.82 as long; 1536 x 14336: 0.224 against 0.256 ms, 768 x 14336: 0.117 against 0.126 ms)
-            const int64_t strips = (N + 255) / 256;
-            const int64_t rounds_large = (mb * strips + cus - 1) / cus, rounds_small = ((M + 191) / 192 * strips + cus - 1) / cus;
-            const int narrow = find_qmmt_named("qmmh_b4_mb3_nb2_wm2_wn4");
-            if (narrow >= 0 && rounds_small * 82 <= rounds_large * 90) tile_idx = narrow;
-        } else if (bits == 4 && mb * ((N + 127) / 128) * 8 > (int64_t)cus * 5) {
-            const int half = find_qmmt_named("qmmh_b4_mb4_nb2_wm2_wn2_s2c");
-            if (half >= 0) tile_idx = half;
-        }
     }
     // Few rows of x: M x N tiles alone would occupy a fraction of the chip (56 workgroups for 32 x 14336), so
     // K is shared out as well and a small kernel adds the partial tiles.
@@ -205,6 +246,12 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
         // fewer than 64 rows and a K that is no multiple of 256: 32 x 256 or 64 x 256 workgroup tiles
         tile_idx = M <= 32 ? find_qmmt(bits, 1, 2, 1, 4) : find_qmmt(bits, 2, 2, 1, 4);
         if (tile_idx < 0) return fail(AQ_ERR_UNSUPPORTED, "aq_qmm: no kernel variant for bits=%d", bits);
+        // their tiles are few (12 x 4032 x 1024: four workgroups, 60 us): K shared out like the few-rows kernels', whole quads
+        // of at least eight blocks each
+        const int tiles = (N + 255) / 256, cus = cu_count > 0 ? cu_count : 256;
+        if (idx < 0)
+            for (int k = 2; k <= 16; k++)
+                if (tiles * k <= cus && qmmt_gsplit(K, k) >= 8 && (int64_t)(k - 1) * qmmt_gsplit(K, k) * 64 < K) ksplit = k;
     }
     {
         const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;

@@ -30,6 +30,7 @@
 #include "aq_lds_copy.h"
 #include "aq_qmm.h"
 
+#include <cmath>
 #include <type_traits>
 
 namespace aq {
@@ -76,20 +77,30 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 //     x * 2^e with e chosen per row;
 // xs: [mblks * 32][ceil(G/4)][4 blocks][hi, lo] bf16: 2^e * sum of x over each 64-code block, hi + lo;
 // rs: [mblks * 32] fp32: 2^-e.
-constexpr int kPrepRows = 8;
-constexpr int kPrepThreads = 512;                     // eight wavefronts: 64 pieces of each of the eight rows per pass
-constexpr int kPrepStep = kPrepThreads / kPrepRows;   // pieces of a row between a thread's pieces
+//
+// GRP 32: xs holds the sums of the 32-code halves, [mblks * 32][ceil(G/4)][half][4 blocks][hi, lo].
+// ROWS rows of x per workgroup: eight, whose slots of a fragment are one 128-byte line of a store, or one where eight rows
+// a workgroup would leave most of the chip idle (21 x 15360: 4 workgroups).
+// GROUPED: row i of the fragments is row route_x[i] of x (the list of routes sorted by expert; negative: zeros), and rows
+// past *live_rows are left alone.
+constexpr int kPrepThreads = 512;
 constexpr int kPrepHold = 8;
+template <int ROWS, int GRP>
 __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xf,
-                                                         uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K) {
+                                                         uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K,
+                                                         const int32_t* __restrict__ route_x, const int32_t* __restrict__ live_rows) {
+    constexpr int STEP = kPrepThreads / ROWS;  // pieces of a row between a thread's pieces
+    if (live_rows && (int)blockIdx.x * ROWS >= *live_rows) return;
     const int tid = threadIdx.x;
-    const int r = tid & 7, p0 = tid >> 3;
-    const int row = (int)blockIdx.x * kPrepRows + r;
+    const int r = tid % ROWS, p0 = tid / ROWS;
+    const int row = (int)blockIdx.x * ROWS + r;
     const int G = K / 64;
     const int G4 = (G + 3) / 4;
     const int pieces = K / 8;
-    const bool live = row < M;
-    __shared__ uint32_t wave_mag[kPrepThreads / kWave][kPrepRows];
+    const int from = route_x ? (row < M ? route_x[row] : -1) : row;
+    const bool live = row < M && from >= 0;
+    const uint16_t* const xrow = x + (int64_t)(live ? from : 0) * K;
+    __shared__ uint32_t wave_mag[kPrepThreads / kWave][ROWS];
     uint32_t mag = 0;
     auto scan = [&](const uint4& v) {
         const uint32_t w[4] = {v.x, v.y, v.z, v.w};
@@ -100,32 +111,33 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
             if (hi < 0x7f80u) mag = max(mag, hi);
         }
     };
-    // up to kPrepHold pieces per thread (K up to 4096) are requested together and stay in registers for the second pass
-    const bool held = pieces <= kPrepStep * kPrepHold;
+    // up to kPrepHold pieces per thread (K up to 4096 with eight rows) are requested together and stay in registers for the
+    // second pass
+    const bool held = pieces <= STEP * kPrepHold;
     uint4 hold[kPrepHold];
     if (held) {
 #pragma unroll
         for (int i = 0; i < kPrepHold; i++) {
-            const int p = p0 + kPrepStep * i;
+            const int p = p0 + STEP * i;
             hold[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (live && p < pieces) hold[i] = *reinterpret_cast<const uint4*>(x + (int64_t)row * K + p * 8);
+            if (live && p < pieces) hold[i] = *reinterpret_cast<const uint4*>(xrow + p * 8);
         }
 #pragma unroll
         for (int i = 0; i < kPrepHold; i++) scan(hold[i]);
     } else if (live) {
-        for (int p = p0; p < pieces; p += kPrepStep) scan(*reinterpret_cast<const uint4*>(x + (int64_t)row * K + p * 8));
+        for (int p = p0; p < pieces; p += STEP) scan(*reinterpret_cast<const uint4*>(xrow + p * 8));
     }
-    // the eight threads of a wavefront that share a row are 8 lanes apart
+    // the threads of a wavefront that share a row are ROWS lanes apart
 #pragma unroll
-    for (int o = 8; o < kWave; o <<= 1) mag = max(mag, (uint32_t)__shfl_xor((int)mag, o, kWave));
-    if ((tid & (kWave - 1)) < kPrepRows) wave_mag[tid >> 6][r] = mag;
+    for (int o = ROWS; o < kWave; o <<= 1) mag = max(mag, (uint32_t)__shfl_xor((int)mag, o, kWave));
+    if ((tid & (kWave - 1)) < ROWS) wave_mag[tid >> 6][r] = mag;
     __syncthreads();
     mag = 0;
 #pragma unroll
     for (int w = 0; w < kPrepThreads / kWave; w++) mag = max(mag, wave_mag[w][r]);
     const int e = exponent_shift(mag, 14);
     const float up = pow2f(e);
-    if (tid < kPrepRows) rs[row] = live ? pow2f(-e) : 0.0f;
+    if (tid < ROWS) rs[row] = live ? pow2f(-e) : 0.0f;
 
     auto emit = [&](int p, const uint4& v) {
         const int g = p >> 3, c8 = p & 7;
@@ -134,15 +146,16 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
         sx = dot2_bf16(v.y, 0x3F803F80u, sx);
         sx = dot2_bf16(v.z, 0x3F803F80u, sx);
         sx = dot2_bf16(v.w, 0x3F803F80u, sx);
-        // the 8 pieces of a block of this row sit in the 8 lanes r, r + 8, ..., r + 56 of the wavefront
-        sx += __shfl_xor(sx, 8, kWave);
-        sx += __shfl_xor(sx, 16, kWave);
-        sx += __shfl_xor(sx, 32, kWave);
-        if (c8 == 0) {
+        // the 8 pieces of a block of this row sit in the 8 lanes ROWS apart
+        sx += __shfl_xor(sx, ROWS, kWave);
+        sx += __shfl_xor(sx, 2 * ROWS, kWave);
+        if (GRP == 64) sx += __shfl_xor(sx, 4 * ROWS, kWave);
+        if ((c8 & (GRP / 8 - 1)) == 0) {
             const float scaled = sx * up;
             const uint32_t hi = f32_to_bf16_bits(scaled);
             const uint32_t lo = f32_to_bf16_bits(scaled - bf16_bits_to_f32(hi));
-            uint32_t* dst = reinterpret_cast<uint32_t*>(xs) + ((int64_t)row * G4 + (g >> 2)) * 4;
+            const int64_t quad = (int64_t)row * G4 + (g >> 2);
+            uint32_t* dst = reinterpret_cast<uint32_t*>(xs) + (GRP == 64 ? quad : 2 * quad + (c8 >> 2)) * 4;
             dst[g & 3] = hi | (lo << 16);
             if (g == G - 1)
                 for (int q = (g & 3) + 1; q < 4; q++) dst[q] = 0u;
@@ -163,11 +176,11 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
     if (held) {
 #pragma unroll
         for (int i = 0; i < kPrepHold; i++)
-            if (p0 + kPrepStep * i < pieces) emit(p0 + kPrepStep * i, hold[i]);
+            if (p0 + STEP * i < pieces) emit(p0 + STEP * i, hold[i]);
     } else {
-        for (int p = p0; p < pieces; p += kPrepStep) {
+        for (int p = p0; p < pieces; p += STEP) {
             uint4 v = {0u, 0u, 0u, 0u};
-            if (live) v = *reinterpret_cast<const uint4*>(x + (int64_t)row * K + p * 8);
+            if (live) v = *reinterpret_cast<const uint4*>(xrow + p * 8);
             emit(p, v);
         }
     }
@@ -178,8 +191,18 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
 // the accumulation half of the register file).
 // SPREAD: the copies of the block requested in an iteration are issued a few at a time in front of every row block's
 // MFMAs instead of together at the top.
-template <int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD>
-__global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileArgs a) {
+// GRP 32: the codes a lane half h expands are those of one group (block g's half h), so that only its scale and bias differ:
+// the lane half keeps its own four scales per quad; the affine term takes its own sums on the A side and two MFMAs per quad
+// (sum x bias, sum x 8 scale) instead of one.
+// Several matrices (a.nseg > 1): the column tiles of all of them make one grid.
+// PAIR (a.pair): column block 0 of a wavefront's tile holds gate rows, column block 1 the up rows of the same outputs; the
+// store is act(gate) * up, from the accumulators as they lie.
+// Expert slabs (a.chunks): a row band is a chunk of up to BM places of the list of routes sorted by expert
+// (aq_moe_group.hip), its weights those of the chunk's expert, its outputs the rows of y that its routes name.
+template <int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
+__global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfArgs a) {
+    constexpr bool G32 = GRP == 32;
+    static_assert(NB == 2, "a pair is two column blocks");
     static_assert(STAGES == 2 || STAGES == 3 || STAGES == 4, "LDS stages");
     constexpr int AHEAD = STAGES - 1;  // iteration g requests block g + AHEAD
     constexpr int BM = WM * MB * 32;
@@ -207,12 +230,26 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
 
     // workgroups are dealt to the 8 XCDs round-robin, so every 8th one shares an L2; give each XCD a
     // contiguous run of tiles in row-band-major order
-    const int T = a.tiles_m * a.tiles_n;
+    // (a matrix with K shared out has ksplit column units per column strip: each stores fp32 partial tiles)
+    const int T = __builtin_amdgcn_readfirstlane((a.chunks ? *a.nchunks : a.tiles_m) * a.units);
     const int per_xcd = (T + 7) / 8;
-    const int tile = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if (tile >= T) return;
-    const int tm = tile / a.tiles_n;
-    const int tn = tile - tm * a.tiles_n;
+    const int id = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per_xcd || id >= T) return;
+    // tiles in groups of a.group_m row bands, column unit by column unit inside a group: the tiles an XCD works on at a
+    // time then cover a patch of the output that is about as tall as it is wide in bytes read
+    const int group = __builtin_amdgcn_readfirstlane(id / (a.group_m * a.units));
+    const int in_group = id - group * a.group_m * a.units;
+    const int bands = min(a.group_m, T / a.units - group * a.group_m);
+    int unit = __builtin_amdgcn_readfirstlane(in_group / bands);
+    const int tm = __builtin_amdgcn_readfirstlane(group * a.group_m + in_group - unit * bands);
+    int seg = 0;
+    while (seg + 1 < a.nseg && unit >= a.seg[seg].unit_end) seg++;
+    seg = __builtin_amdgcn_readfirstlane(seg);
+    if (seg > 0) unit -= a.seg[seg - 1].unit_end;
+    const int split = __builtin_amdgcn_readfirstlane(unit / a.seg[seg].strips);
+    const int tn = __builtin_amdgcn_readfirstlane(unit - split * a.seg[seg].strips);
+    float* const partial = a.seg[seg].partial;  // null: this workgroup's sums are whole
+    const bool pair = a.pair != 0;  // gate: seg[0], up: seg[1]
 
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
@@ -222,14 +259,39 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     const int j = lane & 31;
     const int h = lane >> 5;
 
-    const int K = a.K, M = a.M, N = a.N;
-    const int G = K / 64;
-    const int G4 = (G + 3) / 4;
+    const int K = a.K, N = a.seg[seg].N;
+    const int Gall = K / 64;
+    const int gb = split * a.seg[seg].gsplit;         // first block of K this workgroup multiplies (a multiple of 4)
+    const int G = min(Gall, gb + a.seg[seg].gsplit);  // one past its last block
+    const int G4 = (Gall + 3) / 4;
     const int ksteps = K / 16;
-    const int sb_per_row = G / a.gs_blocks;
+    const int sb_per_row = G32 ? Gall * 2 : Gall / a.gs_blocks;
     const int64_t words_per_row = (int64_t)K / 8;
-    const int m0 = tm * BM;
-    const int n0 = tn * BN;
+    // a pointer picked or computed per workgroup, back on the scalar unit
+    auto uniform = [](auto* p) {
+        const uint64_t u = reinterpret_cast<uint64_t>(p);
+        const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u), hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+        return reinterpret_cast<decltype(p)>((uint64_t)hi << 32 | lo);
+    };
+    int m0 = tm * BM, mend = a.M;  // rows [m0, min(mend, m0 + BM)) of the fragments
+    int64_t row1 = 0, row2 = 0;    // first weight row of the slab (PAIR: of either matrix)
+    if (a.chunks) {
+        const RouteChunk ch = a.chunks[tm];
+        m0 = __builtin_amdgcn_readfirstlane(ch.first);
+        mend = m0 + __builtin_amdgcn_readfirstlane(ch.count);
+        const int64_t base = (int64_t)__builtin_amdgcn_readfirstlane(ch.expert) * a.expert_rows;
+        row1 = base + a.row_base;
+        row2 = base + a.row_base2;
+    }
+    const int n0 = tn * (pair ? BN / 2 : BN);
+    // operands of column block 0 and 1 of the wavefronts' tiles
+    const uint32_t* const w1 = uniform(a.seg[seg].w + row1 * words_per_row);
+    const uint32_t* const w2 = uniform(pair ? a.seg[1].w + row2 * words_per_row : w1);
+    const uint16_t* const sb1[2] = {uniform(a.seg[seg].s + row1 * sb_per_row), uniform(a.seg[seg].b + row1 * sb_per_row)};
+    const uint16_t* const sb2[2] = {uniform(pair ? a.seg[1].s + row2 * sb_per_row : sb1[0]),
+                                    uniform(pair ? a.seg[1].b + row2 * sb_per_row : sb1[1])};
+    // weight row of column block nb, lane column c, for the wavefront column wn
+    auto weight_row = [&](int wn, int nb, int c) { return min(pair ? n0 + wn * 32 + c : n0 + (wn * NB + nb) * 32 + c, N - 1); };
 
     auto issue_a = [&](int g, int stage) {
 #pragma unroll
@@ -244,13 +306,14 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     // the tile's packed rows in 16-byte pieces; copy instruction i of this wavefront moves pieces
     // (i * NWAVE + wave) * 64 + lane to consecutive LDS slots, which leaves row r at r * 32 bytes
     // (rows past N repeat the last row; a tile spans well under 4 GiB, so the lane part fits 32 bits)
-    const uint32_t* const wtile = a.w + (int64_t)min(n0, N - 1) * words_per_row;
+    // (a copy instruction moves one column block of one wavefront column: 32 rows; an odd wavefront's are column blocks 1)
+    static_assert(NWAVE % 2 == 0, "a wavefront copies column blocks of one parity");
+    const uint32_t* const wtile = uniform(((wave & 1) ? w2 : w1) + (int64_t)min(n0, N - 1) * words_per_row);
     uint32_t woff[WPT];
 #pragma unroll
     for (int i = 0; i < WPT; i++) {
-        const int p = (i * NWAVE + wave) * kWave + lane;
-        const int r = p >> 1, q = p & 1;
-        const int n = min(n0 + r, N - 1);
+        const int q = lane & 1;
+        const int n = weight_row((i * NWAVE + wave) / NB, (i * NWAVE + wave) % NB, lane >> 1);
         woff[i] = (uint32_t)(n - min(n0, N - 1)) * (uint32_t)(words_per_row * 4) + (uint32_t)q * 16u;
     }
     auto issue_b = [&](int g, int stage) {
@@ -276,23 +339,25 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     // the first blocks are on their way while the prologue scans the scale rows
 #pragma unroll
     for (int d = 0; d < AHEAD; d++) {
-        issue_a(d < K / 64 ? d : K / 64 - 1, d);
-        issue_b(d < K / 64 ? d : K / 64 - 1, d);
+        issue_a(gb + d < G ? gb + d : G - 1, d);
+        issue_b(gb + d < G ? gb + d : G - 1, d);
     }
 
-    // this lane's weight rows (one per column block), and the power of two that brings the row's largest scale
-    // into [2^10, 2^11): lane half h scans its half of the row's scales
+    // this lane's weight rows (one per column block), and the power of two that brings the row's largest scale (of this
+    // workgroup's range of K) into [2^10, 2^11): lane half h scans its half of the row's scales
     uint32_t sboff[NB];  // element offset of the row's scales (and biases): a 32-bit lane part next to a uniform base
     float col_up[NB];
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) {
-        const int n = min(n0 + (wave_n * NB + nb) * 32 + j, N - 1);
+        const uint16_t* const sbase = nb ? sb2[0] : sb1[0];
+        const int n = weight_row(wave_n, nb, j);
         sboff[nb] = (uint32_t)n * (uint32_t)sb_per_row;
-        const uint16_t* srow = a.s + sboff[nb];
+        const uint16_t* srow = sbase + sboff[nb];
         uint32_t mag = 0;
-        if ((sb_per_row & 15) == 0 && ((uintptr_t)a.s & 15) == 0) {
-            const uint4* p = reinterpret_cast<const uint4*>(srow) + h * (sb_per_row >> 4);
-            for (int i = 0; i < (sb_per_row >> 4); i++) {
+        const int first = G32 ? gb * 2 : gb / a.gs_blocks, last = G32 ? G * 2 : (G + a.gs_blocks - 1) / a.gs_blocks;
+        if (((sb_per_row | first | last) & 7) == 0 && ((uintptr_t)sbase & 15) == 0) {
+            const uint4* p = reinterpret_cast<const uint4*>(srow);
+            for (int i = (first >> 3) + h; i < (last >> 3); i += 2) {
                 const uint4 v = p[i];
                 const uint32_t w[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
@@ -303,7 +368,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
                 }
             }
         } else {
-            for (int i = h; i < sb_per_row; i += 2) {
+            for (int i = first + h; i < last; i += 2) {
                 const uint32_t v = srow[i] & 0x7fffu;
                 if (v < 0x7f80u) mag = max(mag, v);
             }
@@ -316,21 +381,32 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     // in two words per column block (8-byte loads where the rows allow it).  Biases and the (hi, lo) block sums
     // of x are needed once per quad, by the affine MFMA behind its last block, and are fetched for the quad under
     // way.
-    const bool quad_loads = a.gs_blocks == 1 && (G & 3) == 0 && (((uintptr_t)a.s | (uintptr_t)a.b) & 7) == 0;
+    // (groups of 32: this lane half's four of the quad's eight, picked out of one 16-byte load)
+    const uintptr_t sb_bits = (uintptr_t)sb1[0] | (uintptr_t)sb1[1] | (uintptr_t)sb2[0] | (uintptr_t)sb2[1];
+    const bool quad_loads = (Gall & 3) == 0 && (G32 ? (sb_bits & 15) == 0 : a.gs_blocks == 1 && (sb_bits & 7) == 0);
+    const uint32_t half_sel = h ? 0x07060302u : 0x05040100u;
     uint2 s_cur[NB], s_nxt[NB], b_cur[NB];
-    auto load_quad = [&](const uint16_t* base, int quad, uint2 (&dst)[NB]) {
+    auto load_quad = [&](int which, int quad, uint2 (&dst)[NB]) {
         if (quad_loads) {
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) dst[nb] = *reinterpret_cast<const uint2*>(base + sboff[nb] + quad * 4);
+            for (int nb = 0; nb < NB; nb++) {
+                const uint16_t* const base = nb ? sb2[which] : sb1[which];
+                if constexpr (G32) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(base + sboff[nb] + quad * 8);
+                    dst[nb] = make_uint2(__builtin_amdgcn_perm(v.y, v.x, half_sel), __builtin_amdgcn_perm(v.w, v.z, half_sel));
+                } else {
+                    dst[nb] = *reinterpret_cast<const uint2*>(base + sboff[nb] + quad * 4);
+                }
+            }
         } else {
 #pragma unroll
             for (int nb = 0; nb < NB; nb++) {
                 uint32_t v[4];
 #pragma unroll
                 for (int k = 0; k < 4; k++) {
-                    int idx = (quad * 4 + k) / a.gs_blocks;
+                    int idx = G32 ? (quad * 4 + k) * 2 + h : (quad * 4 + k) / a.gs_blocks;
                     idx = idx < sb_per_row ? idx : sb_per_row - 1;  // blocks past K: never used
-                    v[k] = base[sboff[nb] + idx];
+                    v[k] = (nb ? sb2[which] : sb1[which])[sboff[nb] + idx];
                 }
                 dst[nb] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
             }
@@ -346,12 +422,12 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     for (int mb = 0; mb < MB; mb++) {
         int row = m0 + (wave_m * MB + mb) * 32 + j;
         row = row < a.mblks * 32 ? row : a.mblks * 32 - 1;
-        xsoff[mb] = (uint32_t)row * (uint32_t)G4;
+        xsoff[mb] = (uint32_t)row * (uint32_t)(G32 ? 2 * G4 : G4) + (G32 ? (uint32_t)h : 0u);
     }
     uint4 xs_cur[MB];
     auto load_xs = [&](int quad) {
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + quad];
+        for (int mb = 0; mb < MB; mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + (G32 ? 2 * quad : quad)];
     };
 
     f32x16_t out[MB][NB];
@@ -367,22 +443,24 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     // (both times the row's power of two: exact); blocks past Q (only at the end of K) contribute zeros.
     auto affine = [&](auto q_tag) {
         constexpr int Q = decltype(q_tag)::value;
-        bf16x8_t bbf[NB];
+        bf16x8_t bbf[NB], ebf[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
-            uint32_t v[4];
+            uint32_t v[4], ve[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if (q <= Q) {
                     const uint32_t eight = __float_as_uint(__uint_as_float(quad_hi(s_cur[nb], q)) * (8.0f * col_up[nb])) >> 16;
                     const uint32_t bia = __float_as_uint(__uint_as_float(quad_hi(b_cur[nb], q)) * col_up[nb]) >> 16;
-                    v[q] = dup16(h ? eight : bia);
+                    v[q] = dup16(!G32 && h ? eight : bia);
+                    ve[q] = dup16(eight);
                 } else {
-                    v[q] = 0u;
+                    v[q] = ve[q] = 0u;
                 }
             }
-            const uint4 u = {v[0], v[1], v[2], v[3]};
+            const uint4 u = {v[0], v[1], v[2], v[3]}, ue = {ve[0], ve[1], ve[2], ve[3]};
             bbf[nb] = __builtin_bit_cast(bf16x8_t, u);
+            ebf[nb] = __builtin_bit_cast(bf16x8_t, ue);
         }
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) {
@@ -390,6 +468,11 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
 #pragma unroll
             for (int nb = 0; nb < NB; nb++)
                 out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aa, bbf[nb], out[mb][nb], 0, 0, 0);
+            if constexpr (G32) {
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++)
+                    out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aa, ebf[nb], out[mb][nb], 0, 0, 0);
+            }
         }
     };
 
@@ -417,8 +500,8 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
         }
         if constexpr (Q == 1) {
             const int nq = (g >> 2) + 1 < G4 ? (g >> 2) + 1 : G4 - 1;
-            load_quad(a.s, nq, s_nxt);
-            load_quad(a.b, g >> 2, b_cur);
+            load_quad(0, nq, s_nxt);
+            load_quad(1, g >> 2, b_cur);
             load_xs(g >> 2);
         }
         // the copies of block g + AHEAD: together at the top, or (SPREAD) a few in front of every row block's
@@ -482,7 +565,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
         }
         if (Q == 3 || !more) {
             if (Q < 1) {  // K ends inside a quad before its biases and sums were asked for
-                load_quad(a.b, g >> 2, b_cur);
+                load_quad(1, g >> 2, b_cur);
                 load_xs(g >> 2);
             }
             affine(q_tag);
@@ -497,14 +580,14 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     };
     // the first quad's scales; blocks 0 .. AHEAD-1 were requested before the scan of the scale rows (any wait of
     // the compiler's for the loads since then has drained those copies too: all the better)
-    load_quad(a.s, 0, s_nxt);
+    load_quad(0, gb >> 2, s_nxt);
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(s_nxt[nb].x), "+v"(s_nxt[nb].y));
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * GROUP_OPS) : "memory");  // block 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    for (int g = 0; g < G; g += 4) {
+    for (int g = gb; g < G; g += 4) {
         iteration(std::integral_constant<int, 0>{}, g);
         if (g + 1 < G) iteration(std::integral_constant<int, 1>{}, g + 1);
         if (g + 2 < G) iteration(std::integral_constant<int, 2>{}, g + 2);
@@ -522,85 +605,154 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmTileA
     // stores, whole 128-byte lines per eight lanes.
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    constexpr int CW = NB * 32;       // columns of the wavefront's tile
-    constexpr int LPR = CW / 8;       // lanes that share a row, eight columns each
-    constexpr int RPP = kWave / LPR;  // rows per pass
+    constexpr int CW = NB * 32;  // columns of the wavefront's tile
     static_assert(NWAVE * 32 * CW * 4 <= STAGES * (A_STAGE + B_STAGE), "staging area fits the stages");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * CW);
-    const bool wide = (reinterpret_cast<uintptr_t>(a.y) & 15) == 0 && (a.out_f32 ? (N & 3) == 0 : (N & 7) == 0);
-    const int row_in = lane / LPR, c8 = (lane % LPR) * 8;
-    const int n = n0 + wave_n * CW + c8;
+    const int stride = partial && pair ? 2 * N : N;
+    void* const ybase = partial ? static_cast<void*>(partial + (int64_t)split * a.M * stride) : a.seg[seg].y;
+    const bool y_f32 = partial != nullptr || a.out_f32 != 0;
+    // COLS columns of the wavefront's tile leave together, eight consecutive ones per lane; `gated`: act(gate) * up of the two
+    // column blocks.  (Partial tiles of a pair keep both sums: the gate columns of all outputs, then the up columns.)
+    auto store_tile = [&](auto gated_tag) {
+        constexpr bool GATED = decltype(gated_tag)::value;
+        constexpr int COLS = GATED ? CW / 2 : CW;
+        constexpr int LPR = COLS / 8;     // lanes that share a row
+        constexpr int RPP = kWave / LPR;  // rows per pass
+        const int row_in = lane / LPR, c8 = (lane % LPR) * 8;
+        const bool halves = pair && !GATED;
+        const int n = n0 + (pair ? wave_n * 32 + (halves ? c8 % 32 : c8) : wave_n * CW + c8);
+        const int col = halves && c8 >= 32 ? N + n : n;
+        const bool wide = (reinterpret_cast<uintptr_t>(ybase) & 15) == 0 && (y_f32 ? (N & 3) == 0 : (N & 7) == 0);
 #pragma unroll
-    for (int mb = 0; mb < MB; mb++) {
-        const int mtop = m0 + (wave_m * MB + mb) * 32;  // < mblks * 32 unless the whole block lies past M
-        float4 down[4];
+        for (int mb = 0; mb < MB; mb++) {
+            const int mtop = m0 + (wave_m * MB + mb) * 32;  // < mblks * 32 unless the whole block lies past the last row
+            float4 down[4];
 #pragma unroll
-        for (int q = 0; q < 4; q++) {
-            const int m = mtop + 4 * h + 8 * q;
-            down[q] = m < a.mblks * 32 ? *reinterpret_cast<const float4*>(a.rs + m) : make_float4(0.f, 0.f, 0.f, 0.f);
-        }
-#pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const float col_down = 1.0f / col_up[nb];
+            for (int q = 0; q < 4; q++) {
+                const int m = mtop + 4 * h + 8 * q;
+                down[q] = m < a.mblks * 32 ? *reinterpret_cast<const float4*>(a.rs + m) : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            const float col_down[2] = {1.0f / col_up[0], 1.0f / col_up[1]};
 #pragma unroll
             for (int r = 0; r < 16; r++) {
                 const float4 d4 = down[r >> 2];
                 const float dm = (r & 3) == 0 ? d4.x : (r & 3) == 1 ? d4.y : (r & 3) == 2 ? d4.z : d4.w;
-                stage[(8 * (r >> 2) + 4 * h + (r & 3)) * CW + nb * 32 + j] = out[mb][nb][r] * dm * col_down;
-            }
-        }
-#pragma unroll
-        for (int p = 0; p < 32 / RPP; p++) {
-            const int row = p * RPP + row_in;
-            const int m = mtop + row;
-            float4 lo = *reinterpret_cast<const float4*>(stage + row * CW + c8);
-            float4 hi = *reinterpret_cast<const float4*>(stage + row * CW + c8 + 4);
-            if (m >= M || n >= N) continue;
-            const int64_t o = (int64_t)m * N + n;
-            if (a.gate && !a.partial) gate_mul8(a.gate, a.act, o, n, N, lo, hi);
-            if (wide && n + 8 <= N) {
-                if (a.out_f32) {
-                    float4* dst = reinterpret_cast<float4*>(reinterpret_cast<float*>(a.y) + o);
-                    dst[0] = lo;
-                    dst[1] = hi;
+                const int at = (8 * (r >> 2) + 4 * h + (r & 3)) * COLS + j;
+                if constexpr (GATED) {
+                    stage[at] = fmul_unfused(act_value(a.act, out[mb][0][r] * dm * col_down[0]), out[mb][1][r] * dm * col_down[1]);
                 } else {
-                    uint4 u;
-                    u.x = pack_bf16x2(lo.x, lo.y);
-                    u.y = pack_bf16x2(lo.z, lo.w);
-                    u.z = pack_bf16x2(hi.x, hi.y);
-                    u.w = pack_bf16x2(hi.z, hi.w);
-                    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(a.y) + o) = u;
-                }
-            } else {
-                const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    if (n + e < N) {
-                        if (a.out_f32) {
-                            reinterpret_cast<float*>(a.y)[o + e] = v[e];
-                        } else {
-                            reinterpret_cast<uint16_t*>(a.y)[o + e] = f32_to_bf16_bits(v[e]);
+                    for (int nb = 0; nb < NB; nb++) stage[at + nb * 32] = out[mb][nb][r] * dm * col_down[nb];
+                }
+            }
+#pragma unroll
+            for (int p = 0; p < 32 / RPP; p++) {
+                const int row = p * RPP + row_in;
+                const int m = mtop + row;
+                float4 lo = *reinterpret_cast<const float4*>(stage + row * COLS + c8);
+                float4 hi = *reinterpret_cast<const float4*>(stage + row * COLS + c8 + 4);
+                if (m >= mend || n >= N) continue;
+                int64_t y_row = m;
+                if (a.chunks) {
+                    const int route = a.route_of[m];
+                    if (route < 0) lo = hi = make_float4(0.f, 0.f, 0.f, 0.f);  // an expert id or a row of x out of range
+                    y_row = route & INT32_MAX;
+                }
+                const int64_t o = y_row * stride + col;
+                if (wide && n + 8 <= N) {
+                    if (y_f32) {
+                        float4* dst = reinterpret_cast<float4*>(reinterpret_cast<float*>(ybase) + o);
+                        dst[0] = lo;
+                        dst[1] = hi;
+                    } else {
+                        uint4 u;
+                        u.x = pack_bf16x2(lo.x, lo.y);
+                        u.y = pack_bf16x2(lo.z, lo.w);
+                        u.z = pack_bf16x2(hi.x, hi.y);
+                        u.w = pack_bf16x2(hi.z, hi.w);
+                        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(ybase) + o) = u;
+                    }
+                } else {
+                    const float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+                    for (int e = 0; e < 8; e++) {
+                        if (n + e < N) {
+                            if (y_f32) {
+                                reinterpret_cast<float*>(ybase)[o + e] = v[e];
+                            } else {
+                                reinterpret_cast<uint16_t*>(ybase)[o + e] = f32_to_bf16_bits(v[e]);
+                            }
                         }
                     }
                 }
             }
+        }
+    };
+    if (pair && !partial) {
+        store_tile(std::true_type{});
+    } else {
+        store_tile(std::false_type{});
+    }
+}
+
+// ---- adding the partial tiles of a K split --------------------------------------------------------------------------
+// A matrix's partial tiles [ksplit][M][N] ([ksplit][M][gate N | up N] for a pair), added in split order; four columns a
+// thread where N allows it.  grid.y: the matrices.
+template <int V>
+__global__ __launch_bounds__(256) void qmmh_reduce_kernel(const QmmHalfArgs a) {
+    const QmmSegment& seg = a.seg[blockIdx.y];
+    if (!seg.partial) return;
+    const int N = seg.N, stride = a.pair ? 2 * N : N, per_row = N / V;
+    const int64_t total = (int64_t)a.M * per_row;
+    const int64_t mn = (int64_t)a.M * stride;
+    auto sum = [&](int64_t at, float (&v)[V]) {
+        for (int s = 0; s < seg.ksplit; s++) {
+            float t[V];
+            if constexpr (V == 4) {
+                const float4 f = *reinterpret_cast<const float4*>(seg.partial + (int64_t)s * mn + at);
+                t[0] = f.x, t[1] = f.y, t[2] = f.z, t[3] = f.w;
+            } else {
+                t[0] = seg.partial[(int64_t)s * mn + at];
+            }
+#pragma unroll
+            for (int i = 0; i < V; i++) v[i] = s ? v[i] + t[i] : t[i];
+        }
+    };
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        const int m = (int)(i / per_row), c = (int)(i - (int64_t)m * per_row) * V;
+        float v[V];
+        sum((int64_t)m * stride + c, v);
+        if (a.pair) {
+            float u[V];
+            sum((int64_t)m * stride + N + c, u);
+#pragma unroll
+            for (int e = 0; e < V; e++) v[e] = fmul_unfused(act_value(a.act, v[e]), u[e]);
+        }
+        const int64_t o = (int64_t)m * N + c;
+        if (a.out_f32) {
+#pragma unroll
+            for (int e = 0; e < V; e++) static_cast<float*>(seg.y)[o + e] = v[e];
+        } else {
+#pragma unroll
+            for (int e = 0; e < V; e++) static_cast<uint16_t*>(seg.y)[o + e] = f32_to_bf16_bits(v[e]);
         }
     }
 }
 
 // ---- variant table ----------------------------------------------------------------------------
 
-typedef void (*QmmHalfKernel)(const QmmTileArgs);
+typedef void (*QmmHalfKernel)(const QmmHalfArgs);
 struct QmmHalfEntry {
     QmmVariant v;
-    QmmHalfKernel fn;
+    QmmHalfKernel fn, fn32;  // groups of 64 / 128, groups of 32
     int lds_bytes;
 };
 
 #define AQ_QMMH(MB, NB, WM, WN, ST, OCC, SPREAD, SUFFIX)                                               \
     {                                                                                                 \
         {"qmmh_b4_mb" #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, 4, MB, NB, WM, WN},                   \
-            qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD>, ST*((WM * MB * 4096) + (WN * NB * 32 * 32)) \
+            qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 64>, qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 32>, \
+            ST*((WM * MB * 4096) + (WN * NB * 32 * 32))                                               \
     }
 
 static const QmmHalfEntry kQmmHalfTable[] = {
@@ -608,6 +760,9 @@ static const QmmHalfEntry kQmmHalfTable[] = {
     AQ_QMMH(4, 2, 2, 4, 3, 2, false, ""),     // 256 x 256, eight wavefronts, three stages (120 KiB): an A tile feeds twice the MFMAs
     AQ_QMMH(3, 2, 2, 4, 3, 2, false, ""),     // 192 x 256: a round of these takes 0.82 of a round of those; for row counts
                                               // that fill their rounds better (1536 rows: 8 bands instead of 6 of 256)
+    AQ_QMMH(2, 2, 2, 2, 3, 2, false, ""),     // 128 x 128
+    AQ_QMMH(2, 2, 1, 4, 3, 2, false, ""),     // 64 x 256
+    AQ_QMMH(1, 2, 1, 4, 3, 2, false, ""),     // 32 x 256
 };
 
 int qmmh_variant_count() { return (int)(sizeof(kQmmHalfTable) / sizeof(kQmmHalfTable[0])); }
@@ -615,50 +770,159 @@ const QmmVariant* qmmh_variant(int idx) {
     if (idx < 0 || idx >= qmmh_variant_count()) return nullptr;
     return &kQmmHalfTable[idx].v;
 }
+int qmmh_rows(int idx) { return kQmmHalfTable[idx].v.wm * kQmmHalfTable[idx].v.mb * 32; }
+size_t qmmh_partial_bytes(const QmmHalfCall& q) {
+    size_t bytes = 0;
+    for (int i = 0; i < (q.pair ? 1 : q.nseg); i++)
+        if (q.seg[i].ksplit > 1) bytes += ((size_t)q.seg[i].ksplit * q.M * q.seg[i].N * (q.pair ? 2 : 1) * 4 + 255) & ~(size_t)255;
+    return bytes;
+}
 
-// workspace: fragments, block sums, then the row factors (the layout qmmt_workspace_bytes sizes)
-hipError_t qmmh_launch(int idx, const QmmArgs& q, void* workspace, hipStream_t stream) {
-    if (idx < 0 || idx >= qmmh_variant_count()) return hipErrorInvalidValue;
+// What a workgroup tile of each kernel takes: microseconds per 64-code block of K alone on its CU, the same per tile when the
+// CU has more of them, and outside the loop.  From runs at K = 1024 and 4096 with 1/2, 1, 2, 3 and 4 tiles per CU (a CU's
+// clock and its share of L2 depend on how busy the rest of the chip is: 256 x 256 tiles take 1.77 on half the CUs, 2.2 on all).
+struct QmmHalfCost {
+    double solo, full, fixed;
+};
+static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0}};
+
+// Microseconds of kernel i over `tiles` tiles of `blocks` blocks each.
+static double half_cost(int i, int64_t tiles, int blocks, int cus) {
+    const double load = (double)tiles / cus, per_cu = load > 1.0 ? ceil(load) : load;
+    const double work = kQmmHalfCost[i].full * per_cu, least = kQmmHalfCost[i].solo;
+    return kQmmHalfCost[i].fixed + blocks * (work > least ? work : least);
+}
+static int64_t half_strips(int i, int N, bool pair) {
+    const int bn = kQmmHalfTable[i].v.wn * kQmmHalfTable[i].v.nb * 32 / (pair ? 2 : 1);
+    return (N + bn - 1) / bn;
+}
+static int64_t half_bands(int i, int M) { return (M + qmmh_rows(i) - 1) / qmmh_rows(i); }
+
+void qmmh_split(int M, int K, QmmSegment* seg, int cu_count) {
+    const int cus = cu_count > 0 ? cu_count : 256;
+    const int G = K / 64;
+    double best_us = 1e30;
+    seg->ksplit = 1;
+    seg->gsplit = (G + 3) / 4 * 4;
+    for (int i = 0; i < qmmh_variant_count(); i++) {
+        const int64_t tiles = half_bands(i, M) * half_strips(i, seg->N, false);
+        for (int ks = 1; ks <= 16; ks++) {
+            const int gsplit = ((G + ks - 1) / ks + 3) / 4 * 4;
+            if (ks > 1 && (gsplit < 8 || (int64_t)(ks - 1) * gsplit >= G || (int64_t)tiles * ks > 4 * cus)) continue;
+            double us = half_cost(i, tiles * ks, ks > 1 ? gsplit : G, cus);
+            // partial tiles: written and read once at about 3 bytes per nanosecond, one more launch
+            if (ks > 1) us += 3.0 + (double)ks * M * (double)seg->N * 8 / 3e6;
+            if (us < best_us) best_us = us, seg->ksplit = ks, seg->gsplit = gsplit;
+        }
+    }
+}
+
+int qmmh_pick(const QmmHalfCall& q, int cu_count) {
+    const int cus = cu_count > 0 ? cu_count : 256;
+    int best = -1;
+    double best_us = 1e30;
+    for (int i = 0; i < qmmh_variant_count(); i++) {
+        int64_t tiles = 0;
+        int blocks = 0;
+        for (int k = 0; k < (q.pair ? 1 : q.nseg); k++) {
+            tiles += half_bands(i, q.M) * half_strips(i, q.seg[k].N, q.pair) * q.seg[k].ksplit;
+            const int b = q.seg[k].ksplit > 1 ? q.seg[k].gsplit : q.K / 64;
+            blocks = b > blocks ? b : blocks;
+        }
+        const double us = half_cost(i, tiles, blocks, cus);
+        if (us < best_us) best_us = us, best = i;
+    }
+    return best;
+}
+
+
+// workspace: fragments, block sums, row factors (qmmt_workspace_bytes sizes them), then the partial tiles of a K split
+hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream) {
+    if (idx < 0 || idx >= qmmh_variant_count() || q.nseg < 1 || q.nseg > kQmmSegments || (q.pair && q.nseg != 2)) return hipErrorInvalidValue;
     const QmmHalfEntry& e = kQmmHalfTable[idx];
-    const int mblks = (q.M + 31) / 32;
+    const bool g32 = q.group_size == 32;
+    const int rows = q.chunks ? q.most_rows : q.M;  // rows of the fragments
+    const int mblks = (rows + 31) / 32;
     const size_t g4 = ((size_t)q.K / 64 + 3) / 4;
     uint16_t* xf = static_cast<uint16_t*>(workspace);
     uint16_t* xs = xf + (size_t)mblks * 32 * q.K;
-    float* rs = reinterpret_cast<float*>(xs + (size_t)mblks * 32 * g4 * 8);
+    float* rs = reinterpret_cast<float*>(xs + (size_t)mblks * 32 * g4 * (g32 ? 16 : 8));
     hipError_t rc = hipSuccess;
-    if (q.x_ready != kXReadyHalf) {
-        hipLaunchKernelGGL(qmmh_prep_kernel, dim3((unsigned)(mblks * 32 / kPrepRows)), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, q.M, q.K);
+    if (q.x_ready != (g32 ? kXReadyHalf32 : kXReadyHalf)) {
+        // one row a workgroup while eight would leave CUs idle
+        const bool narrow = mblks * 4 < 128;
+        auto* const fn = narrow ? (g32 ? qmmh_prep_kernel<1, 32> : qmmh_prep_kernel<1, 64>) : (g32 ? qmmh_prep_kernel<8, 32> : qmmh_prep_kernel<8, 64>);
+        hipLaunchKernelGGL(fn, dim3((unsigned)(narrow ? mblks * 32 : mblks * 4)), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows,
+                           q.K, q.route_x, q.live_rows);
         rc = hipGetLastError();
         if (rc != hipSuccess) return rc;
     }
 
-    QmmTileArgs a{};
+    QmmHalfArgs a{};
     a.xf = xf;
     a.xs = xs;
     a.rs = rs;
-    a.w = q.w;
-    a.s = q.s;
-    a.b = q.b;
-    a.y = q.y;
+    a.nseg = q.pair ? 1 : q.nseg;  // (a pair is one run of column units; the up matrix is a.seg[1])
+    a.pair = q.pair;
     a.M = q.M;
     a.K = q.K;
-    a.N = q.N;
-    a.gs_blocks = q.gs_blocks;
+    a.gs_blocks = g32 ? 1 : q.group_size / 64;
     a.out_f32 = q.out_f32;
-    a.gate = q.gate;
     a.act = q.act;
     a.mblks = mblks;
-    const int bm = e.v.wm * e.v.mb * 32, bn = e.v.wn * e.v.nb * 32;
-    a.tiles_m = (q.M + bm - 1) / bm;
-    a.tiles_n = (q.N + bn - 1) / bn;
-    a.ksplit = 1;
-    a.gsplit = (q.K / 64 + 3) / 4 * 4;
-    a.partial = nullptr;
-    const int T = a.tiles_m * a.tiles_n;
+    const int bm = qmmh_rows(idx), bn = e.v.wn * e.v.nb * 32;
+    char* partial = static_cast<char*>(workspace) + ((qmmt_workspace_bytes(rows, q.K) + 255) & ~(size_t)255);
+    int units = 0, split_segments = 0;
+    int64_t split_work = 0;
+    bool by4 = true;
+    for (int i = 0; i < q.nseg; i++) {
+        QmmSegment& seg = a.seg[i];
+        seg = q.seg[i];
+        seg.partial = nullptr;
+        seg.strips = (int)half_strips(idx, seg.N, q.pair);
+        if (seg.ksplit <= 1) seg.ksplit = 1, seg.gsplit = (q.K / 64 + 3) / 4 * 4;
+        if (q.pair && i == 1) break;
+        units += seg.strips * seg.ksplit;
+        seg.unit_end = units;
+        if (seg.ksplit > 1) {
+            if (q.chunks || seg.gsplit % 4 != 0 || (int64_t)(seg.ksplit - 1) * seg.gsplit * 64 >= q.K) return hipErrorInvalidValue;
+            seg.partial = reinterpret_cast<float*>(partial);
+            partial += ((size_t)seg.ksplit * q.M * seg.N * (q.pair ? 2 : 1) * 4 + 255) & ~(size_t)255;
+            split_segments++;
+            split_work = (int64_t)q.M * seg.N > split_work ? (int64_t)q.M * seg.N : split_work;
+            by4 = by4 && seg.N % 4 == 0;
+        }
+    }
+    a.units = units;
+    a.tiles_m = (rows + bm - 1) / bm;
+    {
+        // the patch an XCD's 32 CUs work on at a time: group_m row bands by the rest in column strips, fewest bytes per step
+        // of K (4096 x 4096 x 16384: 598 -> 571 us against one band, 1024 x 4096 x 16384 on 64-row tiles 284 -> 201 us)
+        const int at_once = 32 * (160 * 1024 / e.lds_bytes);
+        int64_t least = INT64_MAX;
+        a.group_m = 1;
+        for (int gm = 1; gm <= a.tiles_m && gm <= at_once && !q.chunks; gm++) {
+            const int64_t cost = (int64_t)gm * bm * 32 + (int64_t)((at_once + gm - 1) / gm) * bn * 9;  // in 1/16 bytes: fp16 rows, 4.5-bit columns
+            if (cost < least) least = cost, a.group_m = gm;
+        }
+    }
+    a.chunks = q.chunks;
+    a.nchunks = q.nchunks;
+    a.route_of = q.route_of;
+    a.expert_rows = q.expert_rows;
+    a.row_base = q.row_base;
+    a.row_base2 = q.row_base2;
+    const int T = (q.chunks ? q.most_chunks : a.tiles_m) * units;
     const unsigned grid = (unsigned)(((T + 7) / 8) * 8);
-    rc = ensure_dynamic_lds(reinterpret_cast<const void*>(e.fn), (size_t)e.lds_bytes);
+    const QmmHalfKernel fn = g32 ? e.fn32 : e.fn;
+    rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), (size_t)e.lds_bytes);
     if (rc != hipSuccess) return rc;
-    hipLaunchKernelGGL(e.fn, dim3(grid), dim3((unsigned)(e.v.wm * e.v.wn * kWave)), (size_t)e.lds_bytes, stream, a);
+    hipLaunchKernelGGL(fn, dim3(grid), dim3((unsigned)(e.v.wm * e.v.wn * kWave)), (size_t)e.lds_bytes, stream, a);
+    rc = hipGetLastError();
+    if (rc != hipSuccess || split_segments == 0) return rc;
+    int64_t blocks = (split_work / (by4 ? 4 : 1) + 255) / 256;
+    if (blocks > 4096) blocks = 4096;
+    hipLaunchKernelGGL(by4 ? qmmh_reduce_kernel<4> : qmmh_reduce_kernel<1>, dim3((unsigned)blocks, (unsigned)a.nseg), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
 

@@ -505,7 +505,7 @@ const QmmVariant* qmmt_variant(int idx) {
 size_t qmmt_workspace_bytes(int M, int K) {
     const size_t mblks = ((size_t)M + 31) / 32;
     const size_t g4 = ((size_t)K / 64 + 3) / 4;
-    return mblks * 32 * (size_t)K * 2 + mblks * 32 * g4 * 16 + mblks * 32 * 4;
+    return mblks * 32 * (size_t)K * 2 + mblks * 32 * g4 * 32 + mblks * 32 * 4;  // (groups of 32: a sum per half block)
 }
 
 // Adds the ksplit partial tiles [ksplit][M*N] in split order and stores bf16 or fp32.
@@ -537,17 +537,34 @@ int qmmt_x_kind(int idx) {
     return v->bits == 4 ? kXReadyTile4 : kXReadyTile8;
 }
 
-// ksplit > 1: K/64 must be a multiple of 4 * ksplit; the fp32 partial tiles live in the workspace behind the
+int qmmt_gsplit(int K, int ksplit) {
+    const int G = K / 64;
+    return ((G + ksplit - 1) / (ksplit > 0 ? ksplit : 1) + 3) / 4 * 4;
+}
+
+// ksplit > 1: every share of K is whole quads of blocks (qmmt_gsplit) and none is empty; the fp32 partial tiles live in the workspace behind the
 // rewritten activations (qmmt_workspace_bytes(M, K) rounded up to 256, then qmmt_splitk_bytes).
 hipError_t qmmt_launch_splitk(int idx, const QmmArgs& q, void* workspace, int ksplit, hipStream_t stream) {
     if (idx < 0 || idx >= qmmt_variant_count()) return hipErrorInvalidValue;
-    if (idx >= tile_variants() && idx < tile_variants() + qmmh_variant_count())
-        return ksplit == 1 ? qmmh_launch(idx - tile_variants(), q, workspace, stream) : hipErrorInvalidValue;
+    if (idx >= tile_variants() && idx < tile_variants() + qmmh_variant_count()) {
+        if (ksplit != 1 || q.gate) return hipErrorInvalidValue;
+        QmmHalfCall c{};
+        c.x = q.x;
+        c.M = q.M;
+        c.K = q.K;
+        c.group_size = q.gs_blocks * 64;
+        c.seg[0] = {q.w, q.s, q.b, q.y, q.N, 1, 0, 0, 0, nullptr};
+        c.nseg = 1;
+        c.out_f32 = q.out_f32;
+        c.x_ready = q.x_ready;
+        return qmmh_launch(idx - tile_variants(), c, workspace, stream);
+    }
     const int few = idx >= tile_variants() ? idx - tile_variants() - qmmh_variant_count() : -1;
     static const QmmTileEntry kNone{};
     const QmmTileEntry& e = few < 0 ? kQmmTileTable[idx] : kNone;
     const QmmVariant& v = few < 0 ? e.v : *qmmf_variant(few);
-    if (ksplit < 1 || (ksplit > 1 && (q.K / 64) % (4 * ksplit) != 0)) return hipErrorInvalidValue;
+    const int gsplit = qmmt_gsplit(q.K, ksplit);
+    if (ksplit < 1 || (int64_t)(ksplit - 1) * gsplit * 64 >= q.K) return hipErrorInvalidValue;
     const int mblks = (q.M + 31) / 32;
     uint16_t* xf = static_cast<uint16_t*>(workspace);
     uint16_t* xs = xf + (size_t)mblks * 32 * q.K;
@@ -582,7 +599,7 @@ hipError_t qmmt_launch_splitk(int idx, const QmmArgs& q, void* workspace, int ks
     a.tiles_m = (q.M + bm - 1) / bm;
     a.tiles_n = (q.N + bn - 1) / bn;
     a.ksplit = ksplit;
-    a.gsplit = ksplit > 1 ? (q.K / 64) / ksplit : (q.K / 64 + 3) / 4 * 4;
+    a.gsplit = gsplit;
     a.partial = nullptr;
     if (ksplit > 1) {
         const size_t off = (qmmt_workspace_bytes(q.M, q.K) + 255) & ~(size_t)255;
