@@ -75,10 +75,11 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // workgroup wrote 16 bytes per kilobyte and took 18 us for 34 MB).
 // xf: [mblks][K/16][64 lanes][8] fp16, the A-fragment order of the tile kernels (4-bit slot order), values
 //     x * 2^e with e chosen per row;
-// xs: [mblks * 32][ceil(G/4)][4 blocks][hi, lo] bf16: 2^e * sum of x over each 64-code block, hi + lo;
+// xs: [mblks][ceil(G/4)][32 rows][4 blocks][hi, lo] bf16: 2^e * sum of x over each 64-code block, hi + lo (a wavefront's
+//     load of 32 rows is four lines; row-major it was 32);
 // rs: [mblks * 32] fp32: 2^-e.
 //
-// GRP 32: xs holds the sums of the 32-code halves, [mblks * 32][ceil(G/4)][half][4 blocks][hi, lo].
+// GRP 32: xs holds the sums of the 32-code halves, [mblks][ceil(G/4)][half][32 rows][4 blocks][hi, lo].
 // ROWS rows of x per workgroup: eight, whose slots of a fragment are one 128-byte line of a store, or one where eight rows
 // a workgroup would leave most of the chip idle (21 x 15360: 4 workgroups).
 // GROUPED: row i of the fragments is row route_x[i] of x (the list of routes sorted by expert; negative: zeros), and rows
@@ -154,8 +155,8 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
             const float scaled = sx * up;
             const uint32_t hi = f32_to_bf16_bits(scaled);
             const uint32_t lo = f32_to_bf16_bits(scaled - bf16_bits_to_f32(hi));
-            const int64_t quad = (int64_t)row * G4 + (g >> 2);
-            uint32_t* dst = reinterpret_cast<uint32_t*>(xs) + (GRP == 64 ? quad : 2 * quad + (c8 >> 2)) * 4;
+            const int64_t quad = (int64_t)(row >> 5) * G4 + (g >> 2);
+            uint32_t* dst = reinterpret_cast<uint32_t*>(xs) + ((GRP == 64 ? quad : 2 * quad + (c8 >> 2)) * 32 + (row & 31)) * 4;
             dst[g & 3] = hi | (lo << 16);
             if (g == G - 1)
                 for (int q = (g & 3) + 1; q < 4; q++) dst[q] = 0u;
@@ -199,6 +200,14 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
 // store is act(gate) * up, from the accumulators as they lie.
 // Expert slabs (a.chunks): a row band is a chunk of up to BM places of the list of routes sorted by expert
 // (aq_moe_group.hip), its weights those of the chunk's expert, its outputs the rows of y that its routes name.
+// Packed weights are staged two 64-code blocks at a time.  The L1 charges a copy instruction per line it touches, about four
+// clocks each: 32 bytes of each of 32 rows per instruction (one block at a time) cost 32 lines for 1 KiB, which was most of
+// what the small tiles' loop took (32 x 256 tiles: 288 lines x 4 clocks of 1320 per block) and half the copies' time in the
+// large ones; two blocks are 64-byte halves of sixteen rows (2048 x 4096 x 14336: 281 -> 265 us; 4096 x 4096 x 16384: 571 ->
+// 558; 512 x 4096 x 16384 on 32 x 256 tiles: 155 -> 138; whole lines, four blocks at a time, measured the same on the small
+// tiles and 623 us on the large ones, whose LDS addresses then are no constants).  The 16-byte pieces of a row are rotated
+// against those of its neighbours (the piece a lane fetches, not the place it lands in), so that a wavefront's reads of one
+// block hit all banks.
 template <int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
 __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfArgs a) {
     constexpr bool G32 = GRP == 32;
@@ -208,21 +217,26 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     constexpr int BM = WM * MB * 32;
     constexpr int BN = WN * NB * 32;
     constexpr int NWAVE = WM * WN;
-    constexpr int NT = NWAVE * kWave;
     constexpr int A_STAGE = (BM / 32) * 4096;
-    constexpr int B_STAGE = BN * 32;         // packed codes of one 64-code block
+    constexpr int QB = 2;                    // blocks of packed weights per stage
+    constexpr int B_ROW = QB * 32;           // bytes of a weight row per stage
+    constexpr int B_STAGE = BN * B_ROW;      // packed codes of QB 64-code blocks
     constexpr int A_BLOCKS = (BM / 32) * 4;  // 1 KiB fragments of A per stage
-    constexpr int WPB = 8;                   // packed words per row and 64-code block
-    constexpr int W_PIECES = BN * WPB / 4;   // 16-byte pieces of packed weights per stage
-    constexpr int WPT = W_PIECES / NT;       // per thread
+    constexpr int PPR = 2 * QB;              // 16-byte pieces of a row per stage
+    constexpr int RPI = kWave / PPR;         // rows a copy instruction covers
+    constexpr int NBC = B_STAGE / 1024 / NWAVE;  // B copies a wavefront issues per stage
     static_assert(A_BLOCKS % NWAVE == 0, "A fragments must divide among the wavefronts");
-    static_assert(W_PIECES % NT == 0 && WPT >= 1, "weight pieces must divide among the threads");
+    static_assert(B_STAGE % (1024 * NWAVE) == 0 && NBC >= 1, "weight pieces must divide among the wavefronts");
     constexpr int NA = A_BLOCKS / NWAVE;  // A copies a wavefront issues per block
-    constexpr int GROUP_OPS = NA + WPT;   // LDS copies a wavefront issues per block
+    // B's next stage is issued in a stage's first block, behind that iteration's A copies.  still_out: the copies that may be
+    // on their way at the end of the iteration of block Q of a quad, which are those newer than A of the next block, and in a
+    // stage's second block none of B's.
+    static_assert(AHEAD <= 2, "waits are counted for one or two blocks ahead");
+    auto still_out = [=](int q) constexpr { return (AHEAD - 1) * NA + ((q & 1) == 0 ? NBC : 0); };
 
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* const abuf = lds;                     // [STAGES][A_STAGE]
-    uint8_t* const bbuf = lds + STAGES * A_STAGE;  // [STAGES][B_STAGE]
+    uint8_t* const bbuf = lds + STAGES * A_STAGE;  // [2][B_STAGE]
     // the same as LDS byte addresses: the copy instructions take theirs from a scalar register, and plain integer
     // arithmetic keeps it on the scalar unit (a pointer would be converted, null check included, per copy)
     const uint32_t abuf_at = __builtin_amdgcn_readfirstlane(lds_offset(lds));
@@ -293,55 +307,44 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     // weight row of column block nb, lane column c, for the wavefront column wn
     auto weight_row = [&](int wn, int nb, int c) { return min(pair ? n0 + wn * 32 + c : n0 + (wn * NB + nb) * 32 + c, N - 1); };
 
-    auto issue_a = [&](int g, int stage) {
+    // The tile's packed rows in 16-byte pieces: copy c of this wavefront fills 1 KiB, RPI rows of a stage, row r at r * B_ROW
+    // bytes, its piece p at slot p ^ turn(r).  (Rows past N repeat the last row, pieces past K the last piece; a tile spans
+    // well under 4 GiB, so the lane part fits 32 bits.  The RPI rows belong to one column block, hence to one matrix.)
+    auto turn = [](int r) { return (r >> 2) & 3; };
+    const int64_t first_row = (int64_t)min(n0, N - 1) * words_per_row;
+    const uint32_t* const wtile1 = uniform(w1 + first_row);
+    const uint32_t* const wtile2 = uniform(w2 + first_row);
+    const uint32_t row_bytes = (uint32_t)(words_per_row * 4);
+    uint32_t wrow[NBC], wpiece[NBC];
 #pragma unroll
-        for (int q = 0; q < NA; q++) {
-            const int blk = wave + q * NWAVE;
-            int mblk = m0 / 32 + (blk >> 2);
-            mblk = mblk < a.mblks ? mblk : a.mblks - 1;  // past the end: any valid rows, never stored
-            const uint16_t* src = a.xf + ((int64_t)mblk * ksteps + g * 4 + (blk & 3)) * 512;
-            copy16_to_lds(src, (uint32_t)lane * 16u, abuf_at + (uint32_t)(stage * A_STAGE + blk * 1024));
-        }
-    };
-    // the tile's packed rows in 16-byte pieces; copy instruction i of this wavefront moves pieces
-    // (i * NWAVE + wave) * 64 + lane to consecutive LDS slots, which leaves row r at r * 32 bytes
-    // (rows past N repeat the last row; a tile spans well under 4 GiB, so the lane part fits 32 bits)
-    // (a copy instruction moves one column block of one wavefront column: 32 rows; an odd wavefront's are column blocks 1)
-    static_assert(NWAVE % 2 == 0, "a wavefront copies column blocks of one parity");
-    const uint32_t* const wtile = uniform(((wave & 1) ? w2 : w1) + (int64_t)min(n0, N - 1) * words_per_row);
-    uint32_t woff[WPT];
-#pragma unroll
-    for (int i = 0; i < WPT; i++) {
-        const int q = lane & 1;
-        const int n = weight_row((i * NWAVE + wave) / NB, (i * NWAVE + wave) % NB, lane >> 1);
-        woff[i] = (uint32_t)(n - min(n0, N - 1)) * (uint32_t)(words_per_row * 4) + (uint32_t)q * 16u;
+    for (int c = 0; c < NBC; c++) {
+        const int r = (c * NWAVE + wave) * RPI + lane / PPR;  // row of the tile: column block r / 32
+        wrow[c] = (uint32_t)(weight_row((r >> 5) / NB, (r >> 5) % NB, r & 31) - min(n0, N - 1)) * row_bytes;
+        wpiece[c] = (uint32_t)((lane % PPR) ^ turn(r)) * 16u;
     }
-    auto issue_b = [&](int g, int stage) {
-#pragma unroll
-        for (int i = 0; i < WPT; i++)
-            copy16_to_lds(wtile + (int64_t)g * WPB, woff[i], bbuf_at + (uint32_t)(stage * B_STAGE + (i * NWAVE + wave) * 1024));
+    // copy c of stage st (64-code blocks QB * st ..) into buffer `buf`
+    auto issue_b = [&](int c, int st, int buf) {
+        const uint32_t in_row = min((uint32_t)(st * B_ROW) + wpiece[c], row_bytes - 16u);
+        const int block = (c * NWAVE + wave) * RPI >> 5;
+        copy16_to_lds((block & 1) ? wtile2 : wtile1, wrow[c] + in_row, bbuf_at + (uint32_t)(buf * B_STAGE + (c * NWAVE + wave) * 1024));
     };
-    // copy number c (0 .. GROUP_OPS-1) of a block: the A fragments first, then the codes
-    auto issue_one = [&](int c, int g, int stage) {
-        if (c < NA) {
-            const int blk = wave + c * NWAVE;
-            int mblk = m0 / 32 + (blk >> 2);
-            mblk = mblk < a.mblks ? mblk : a.mblks - 1;
-            const uint16_t* src = a.xf + ((int64_t)mblk * ksteps + g * 4 + (blk & 3)) * 512;
-            copy16_to_lds(src, (uint32_t)lane * 16u, abuf_at + (uint32_t)(stage * A_STAGE + blk * 1024));
-        } else {
-            const int i = c - NA;
-            copy16_to_lds(wtile + (int64_t)g * WPB, woff[i], bbuf_at + (uint32_t)(stage * B_STAGE + (i * NWAVE + wave) * 1024));
-        }
+    // copy c of A's block g
+    auto issue_a1 = [&](int c, int g, int stage) {
+        const int blk = wave + c * NWAVE;
+        int mblk = m0 / 32 + (blk >> 2);
+        mblk = mblk < a.mblks ? mblk : a.mblks - 1;  // past the end: any valid rows, never stored
+        const uint16_t* src = a.xf + ((int64_t)mblk * ksteps + g * 4 + (blk & 3)) * 512;
+        copy16_to_lds(src, (uint32_t)lane * 16u, abuf_at + (uint32_t)(stage * A_STAGE + blk * 1024));
     };
     const uint32_t mask_s = opaque_s(kMaskH);
     const uint32_t magic_v = opaque_v(kMagicH);
     // the first blocks are on their way while the prologue scans the scale rows
 #pragma unroll
-    for (int d = 0; d < AHEAD; d++) {
-        issue_a(gb + d < G ? gb + d : G - 1, d);
-        issue_b(gb + d < G ? gb + d : G - 1, d);
-    }
+    for (int c = 0; c < NBC; c++) issue_b(c, gb / QB, 0);
+#pragma unroll
+    for (int d = 0; d < AHEAD; d++)
+#pragma unroll
+        for (int c = 0; c < NA; c++) issue_a1(c, gb + d < G ? gb + d : G - 1, d);
 
     // this lane's weight rows (one per column block), and the power of two that brings the row's largest scale (of this
     // workgroup's range of K) into [2^10, 2^11): lane half h scans its half of the row's scales
@@ -420,14 +423,13 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     uint32_t xsoff[MB];  // in 16-byte units
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
-        int row = m0 + (wave_m * MB + mb) * 32 + j;
-        row = row < a.mblks * 32 ? row : a.mblks * 32 - 1;
-        xsoff[mb] = (uint32_t)row * (uint32_t)(G32 ? 2 * G4 : G4) + (G32 ? (uint32_t)h : 0u);
+        const int mblk = min(m0 / 32 + wave_m * MB + mb, a.mblks - 1);
+        xsoff[mb] = (uint32_t)mblk * (uint32_t)(G32 ? 2 * G4 : G4) * 32u + (G32 ? (uint32_t)h * 32u : 0u) + (uint32_t)j;
     }
     uint4 xs_cur[MB];
     auto load_xs = [&](int quad) {
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + (G32 ? 2 * quad : quad)];
+        for (int mb = 0; mb < MB; mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + (G32 ? 64 * quad : 32 * quad)];
     };
 
     f32x16_t out[MB][NB];
@@ -484,6 +486,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     // until NOTHING is outstanding, copies included.  Iteration Q = 1 is therefore ordered: loads, MFMAs, first
     // use of the loaded registers (forced), and only then this iteration's copies - the forced wait then covers
     // the loads, a block of MFMAs old, and the copies of block g+1, which the end of the iteration needs anyway.
+    // (Loads at Q = 0, or the forced use at Q = 2, measured 3 to 4 % slower on the large tiles and no better on the small.)
     // With two or four stages the stage of block g is g & 3 modulo the stages, static like Q, and every LDS address
     // of the loop is a constant; with three it is carried along.
     const int glast = G - 1;
@@ -508,17 +511,26 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         // MFMAs, so that they do not queue up behind those of the other wavefronts
         const int g2 = g + AHEAD < G ? g + AHEAD : glast;
         const int st2 = sa == 0 ? STAGES - 1 : sa - 1;  // stage (sa + AHEAD) % STAGES: read last in iteration g-1
-        if constexpr (!SPREAD && !LATE) {
-            issue_a(g2, st2);
-            issue_b(g2, st2);
-        }
+        // B's next stage into the buffer that was read last in the stage before this one (past the end of K: the last again)
+        constexpr int NBQ = (Q & 1) == 0 ? NBC : 0, bcur = Q >> 1;
+        const int bst = min(g / QB + 1, (Gall - 1) / QB);
+        auto issue_some = [&](int from, int to) {  // A's copies first, then B's
+#pragma unroll
+            for (int c = from; c < to; c++) {
+                if (c < NA)
+                    issue_a1(c, g2, st2);
+                else
+                    issue_b(c - NA, bst, bcur ^ 1);
+            }
+        };
+        if constexpr (!SPREAD && !LATE) issue_some(0, NA + NBQ);
         const uint8_t* ab = abuf + sa * A_STAGE + (wave_m * MB) * 4096 + lane * 16;
         // this lane's codes: row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3
-        const uint8_t* bb = bbuf + sa * B_STAGE + ((wave_n * NB) * 32 + j) * 32 + h * 16;
+        const uint8_t* bb = bbuf + bcur * B_STAGE + ((wave_n * NB) * 32 + j) * B_ROW + (((Q % QB * 2 + h) ^ turn(j)) * 16);
         f16x8_t bfrag[NB][4];
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
-            const uint4 cw = *reinterpret_cast<const uint4*>(bb + nb * 32 * 32);
+            const uint4 cw = *reinterpret_cast<const uint4*>(bb + nb * 32 * B_ROW);
             // the block's scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
             const float sv = __uint_as_float(quad_hi(s_cur[nb], Q)) * col_up[nb];
             const f16x2_t s2 = {(_Float16)sv, (_Float16)sv};
@@ -541,10 +553,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
                     afrag[(mb + 1) & 1][t] = *reinterpret_cast<const f16x8_t*>(ab + ((mb + 1) * 4 + t) * 1024);
                 __builtin_amdgcn_sched_barrier(0);  // or the scheduler sinks the reads back to their first use
             }
-            if constexpr (SPREAD && !LATE) {
-#pragma unroll
-                for (int c = mb * GROUP_OPS / MB; c < (mb + 1) * GROUP_OPS / MB; c++) issue_one(c, g2, st2);
-            }
+            if constexpr (SPREAD && !LATE) issue_some(mb * (NA + NBQ) / MB, (mb + 1) * (NA + NBQ) / MB);
 #pragma unroll
             for (int t = 0; t < 4; t++)
 #pragma unroll
@@ -560,8 +569,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
             for (int mb = 0; mb < MB; mb++)
                 asm volatile("" : "+v"(xs_cur[mb].x), "+v"(xs_cur[mb].y), "+v"(xs_cur[mb].z), "+v"(xs_cur[mb].w));
             __builtin_amdgcn_sched_barrier(0);
-            issue_a(g2, st2);
-            issue_b(g2, st2);
+            issue_some(0, NA + NBQ);
         }
         if (Q == 3 || !more) {
             if (Q < 1) {  // K ends inside a quad before its biases and sums were asked for
@@ -571,10 +579,9 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
             affine(q_tag);
         }
         sa_carried = sa == STAGES - 1 ? 0 : sa + 1;
-        // Block g+1 has landed once at most the copies of the AHEAD-1 newest blocks are outstanding; this
-        // iteration's LDS reads have returned.  A bare s_barrier on purpose: __syncthreads() carries a workgroup
+        // Block g+1 has landed once only newer copies are outstanding (still_out); this iteration's LDS reads have returned.  A bare s_barrier on purpose: __syncthreads() carries a workgroup
         // fence, for which the compiler drains ALL outstanding copies into LDS.
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * GROUP_OPS) : "memory");
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(still_out(Q)) : "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
@@ -584,7 +591,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(s_nxt[nb].x), "+v"(s_nxt[nb].y));
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * GROUP_OPS) : "memory");  // block 0 has landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * NA) : "memory");  // block 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     for (int g = gb; g < G; g += 4) {
@@ -606,7 +613,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     constexpr int CW = NB * 32;  // columns of the wavefront's tile
-    static_assert(NWAVE * 32 * CW * 4 <= STAGES * (A_STAGE + B_STAGE), "staging area fits the stages");
+    static_assert(NWAVE * 32 * CW * 4 <= STAGES * A_STAGE + 2 * B_STAGE, "staging area fits the stages");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * CW);
     const int stride = partial && pair ? 2 * N : N;
     void* const ybase = partial ? static_cast<void*>(partial + (int64_t)split * a.M * stride) : a.seg[seg].y;
@@ -752,7 +759,7 @@ struct QmmHalfEntry {
     {                                                                                                 \
         {"qmmh_b4_mb" #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, 4, MB, NB, WM, WN},                   \
             qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 64>, qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 32>, \
-            ST*((WM * MB * 4096) + (WN * NB * 32 * 32))                                               \
+            ST*(WM * MB * 4096) + 2 * (WN * NB * 32 * 64)                                               \
     }
 
 static const QmmHalfEntry kQmmHalfTable[] = {
