@@ -955,6 +955,105 @@ size_t aq_workspace_bytes(aq_ctx* ctx) {
     return ctx->ws.bytes + ctx->head_ws.bytes;
 }
 
+namespace {
+
+// A gathered call of many routes: grouped by expert on the device, so that an expert's weights are read once per chunk of
+// its routes instead of once per route.  `a` as the per-route kernels take it (pair: w = w2 and row_base2 set).  kPass: the
+// per-route kernels run the call, as they do up to 64 routes, whose outputs keep the bytes of the sliced expert's own call.
+//
+// Where the lines lie (128 experts, gate|up 2816 -> 2 x 704 and down 704 -> 2816, us per route / grouped on token tiles of 16
+// / on matmul tiles of 32 / of 64 rows):
+//                    gate|up                        down
+//   256 routes       78 /  92 / 120 / 130         114 / 101 /  60 /  75
+//   512             163 / 103 / 134 / 144         220 / 116 /  68 /  83
+//   1024            329 / 106 / 135 / 147         440 / 125 /  69 /  84
+//   4096           1306 / 272 / 160 / 159        1695 / 328 /  94 /  95
+// The per-route kernels stop paying at about two and a half routes per expert that is named at all, where their fast form
+// takes the shape, and at about one where it does not (K = 704 here); few routes per expert go to the token tiles while K
+// gives their eight wavefronts a run each, everything else to the matmul tiles whose rows an expert's routes fill.
+int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair) {
+    if (a.routes <= 64 || ctx->forced[0] >= 0 || ctx->forced[1] >= 0 || a.num_experts > aq::kGroupMaxExperts) return kPass;
+    a.gs_shift = is_pow2(group_size) ? ilog2(group_size) : 0;
+    const double named = a.num_experts * (1.0 - pow(1.0 - 1.0 / a.num_experts, a.routes));  // experts with a route, ids at random
+    const bool fast_routes = bits == 4 && group_size == 64 && !(ctx->families_off >> kFamDiag & 1) && aq::qmvd_pick_gather(a.K) >= 0;
+    if (a.routes < (fast_routes ? 2.5 : 1.15) * named) return kPass;
+    const double per_expert = a.routes / named;
+    const int groups = a.num_experts < a.routes ? a.num_experts : a.routes;
+    const bool tiles_fit = aq::qmmh_takes(a.x, a.w, a.K, group_size, bits) && !(ctx->families_off >> kFamTiles & 1);
+    const bool tok_fits = aq::qmvt_grouped_fits(a, bits, group_size, pair) && !(ctx->families_off >> kFamTok & 1);
+    if (!tiles_fit && !tok_fits) return kPass;
+    const bool tiles = tiles_fit && !(tok_fits && per_expert <= 12 && a.K >= 2048);
+    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= 32 ? 32 : per_expert <= 96 ? 64 : per_expert <= 384 ? 128 : 256;
+    const int pad = tiles ? 32 : 1;
+    const int most_chunks = a.routes / chunk + groups;
+    const int most_rows = a.routes + groups * (pad - 1);
+    const size_t xbytes = tiles ? (aq::qmmt_workspace_bytes(most_rows, a.K) + 255) & ~(size_t)255 : 0;
+    const size_t list = align256((size_t)most_chunks * sizeof(aq::RouteChunk)), places = align256((size_t)most_rows * 4);
+    const size_t need = xbytes + list + 256 + 2 * places;
+    if (!aq::workspace_may_grow(&ctx->ws, need, ctx->stream)) return kPass;
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
+    char* p = static_cast<char*>(ctx->ws.ptr) + xbytes;
+    aq::RouteGroupArgs g{};
+    g.lhs = a.lhs;
+    g.rhs = a.rhs;
+    g.routes = a.routes;
+    g.x_rows = a.x_rows;
+    g.num_experts = a.num_experts;
+    g.chunk_rows = chunk;
+    g.pad = pad;
+    g.most_chunks = most_chunks;
+    g.chunks = reinterpret_cast<aq::RouteChunk*>(p);
+    g.nchunks = reinterpret_cast<int32_t*>(p + list);
+    g.live_rows = g.nchunks + 1;
+    g.route_x = reinterpret_cast<int32_t*>(p + list + 256);
+    g.route_of = reinterpret_cast<int32_t*>(p + list + 256 + places);
+    AQ_HIP(aq::moe_group_launch(g, ctx->stream), "hipLaunchKernel");
+    if (!tiles) {
+        a.chunks = g.chunks;
+        a.route_x = g.route_x;
+        a.route_of = g.route_of;
+        ctx->last_variant[0] = pair ? "gather_gate_up_grouped_tok" : "gather_grouped_tok";
+        AQ_HIP(aq::qmvt_grouped_launch(bits, chunk, pair, most_chunks, a, ctx->stream), "hipLaunchKernel");
+        return AQ_OK;
+    }
+    aq::QmmHalfCall q{};
+    q.x = a.x;
+    q.M = most_rows;
+    q.K = a.K;
+    q.group_size = group_size;
+    q.nseg = pair ? 2 : 1;
+    q.pair = pair ? 1 : 0;
+    q.act = a.act;
+    q.out_f32 = a.out_f32;
+    for (int i = 0; i < q.nseg; i++) {
+        q.seg[i].w = a.w;
+        q.seg[i].s = a.s;
+        q.seg[i].b = a.b;
+        q.seg[i].y = a.y;
+        q.seg[i].N = a.N;
+    }
+    q.chunks = g.chunks;
+    q.nchunks = g.nchunks;
+    q.route_x = g.route_x;
+    q.route_of = g.route_of;
+    q.live_rows = g.live_rows;
+    q.most_chunks = most_chunks;
+    q.most_rows = most_rows;
+    q.expert_rows = a.expert_rows;
+    q.row_base = a.row_base;
+    q.row_base2 = a.row_base2;
+    int idx = 0;
+    while (idx < aq::qmmh_variant_count() && !(aq::qmmh_rows(idx) == chunk && (chunk != 256 || aq::qmmh_variant(idx)->wn == 4))) idx++;
+    if (idx >= aq::qmmh_variant_count()) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv: no tiles of %d rows", chunk);
+    const char* name = nullptr;
+    const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, idx, q, &name, fail, nullptr);
+    if (rc == AQ_OK) ctx->last_variant[0] = pair ? "gather_gate_up_grouped_tiles" : "gather_grouped_tiles";
+    return rc;
+}
+
+}  // namespace
+
 int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
                   const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
                   int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags) {
@@ -990,6 +1089,7 @@ int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* sc
     a.row_base = row_base;
     a.x_rows = x_rows;
     a.routes = routes;
+    if (const int rc = run_grouped(ctx, a, group_size, bits, false); rc != kPass) return rc;
     // every expert slab must keep 16-byte row alignment for the dot2 kernels
     return launch_qmv_rows(ctx, a, group_size, bits, true);
 }
@@ -1259,6 +1359,10 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
         a.x_rows = x_rows;
         a.routes = routes;
         a.act = act;
+        {
+            std::lock_guard<std::mutex> lk(ctx->mu);
+            if (const int rc = run_grouped(ctx, a, group_size, bits, true); rc != kPass) return rc;
+        }
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, true, di)) {
             std::lock_guard<std::mutex> lk(ctx->mu);
             ctx->last_variant[0] = "gather_gate_up_diag";

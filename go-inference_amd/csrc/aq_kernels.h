@@ -182,6 +182,10 @@ hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
 int qmvt_pick_pair(int bits, int M, int K, int N, int cu_count);
 bool qmvt_pair_supported(int idx);
 hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream);
+// Expert slabs with the routes grouped by expert (a.chunks, a.route_x, a.route_of; chunks of up to `tokens` = 16 or 32
+// routes; most_chunks entries in the list); pair as above.
+bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair);
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream);
 
 // lm_head kernels (aq_qmv_head.hip), one activation row: the projection with its epilogue replaced by
 //   fuse 3: best[0] = max over rows of pack(score, row): every wavefront stores its own maximum into
@@ -235,6 +239,16 @@ struct MoeCombineArgs {
     int in_f32, out_f32, bf16_steps;
 };
 hipError_t moe_route_launch(const MoeRouteArgs& a, hipStream_t stream);
+// Routes grouped by expert (aq_moe_group.hip).  The lists hold most_chunks chunks of up to chunk_rows routes and
+// routes + min(num_experts, routes) * (pad - 1) places; every expert's run starts at a multiple of pad.
+constexpr int kGroupMaxExperts = 4096;
+struct RouteGroupArgs {
+    const int32_t *lhs, *rhs;  // lhs may be null (every route reads row 0)
+    int routes, x_rows, num_experts, chunk_rows, pad, most_chunks;
+    RouteChunk* chunks;
+    int32_t *nchunks, *live_rows, *route_x, *route_of;
+};
+hipError_t moe_group_launch(const RouteGroupArgs& a, hipStream_t stream);
 hipError_t moe_combine_launch(const MoeCombineArgs& a, hipStream_t stream);
 
 // Any-width (2..8 bit, codes may straddle words), any-group fallback.

@@ -149,7 +149,7 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
         }
     // x: lane (i, q) of load `ab` of token set ts reads token 16 ts + (i % 8) + 8 ab, bytes 64 (i / 8) + 16 q of a
     // 128-byte step pair (TS sets of 16 tokens share every expanded weight)
-    auto x_row = [&](int t) { return GROUPED ? (uint32_t)a.route_x[first_route + t] : (uint32_t)t; };
+    auto x_row = [&](int t) { return GROUPED ? (uint32_t)max(a.route_x[first_route + t], 0) : (uint32_t)t; };
     uint32_t x_lane[TS][2];
 #pragma unroll
     for (int ts = 0; ts < TS; ts++)

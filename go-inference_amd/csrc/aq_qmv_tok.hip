@@ -100,6 +100,33 @@ hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair) {
+    if ((bits != 4 && bits != 8) || (group_size != 32 && group_size != 64 && group_size != 128)) return false;
+    if (a.N < 1 || a.K < 64 || a.K % 64 != 0 || a.K % group_size != 0 || a.K > kTokMaxK) return false;
+    const uintptr_t al = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.s) |
+                         reinterpret_cast<uintptr_t>(a.b);
+    if (al & 15) return false;
+    // 32-bit byte offsets into an expert's rows and into x
+    if ((uint64_t)a.expert_rows * (uint64_t)(a.K * bits / 8) >= (1ull << 32) || (uint64_t)a.x_rows * (uint64_t)a.K * 2 >= (1ull << 32)) return false;
+    // an expert's scales are read in 16-byte pieces from its first row on
+    const int64_t groups = a.K / group_size;
+    if ((a.expert_rows * groups) % 8 || (a.row_base * groups) % 8 || (pair && (a.row_base2 * groups) % 8)) return false;
+    return tok_lds_bytes(tok_entry(0), a.K, group_size == 32 ? kTokG32 : kTokAny) <= 160 * 1024;
+}
+
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream) {
+    const int idx = (bits == 8 ? kTokPerWidth : 0) + (tokens == 32 ? 3 : 0);  // (four sets of rows: the first of a token count)
+    const QmvTokEntry& e = tok_entry(idx);
+    const int form = a.gs_shift == 5 ? kTokG32 : kTokAny;
+    const QmvTokKernel fn = e.grouped[form == kTokG32][pair ? 1 : 0];
+    if (!fn || e.v.m != tokens) return hipErrorInvalidValue;
+    const size_t lds = tok_lds_bytes(e, a.K, form);
+    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
+    const int outs = e.wg_rows / (pair ? 2 : 1);
+    hipLaunchKernelGGL(fn, dim3((unsigned)((a.N + outs - 1) / outs), (unsigned)most_chunks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
+    return hipGetLastError();
+}
+
 // The variant for `rows` weight rows in all, or -1.
 int qmvt_pick(int bits, int M, int K, int rows, int cu_count) {
     if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK) return -1;

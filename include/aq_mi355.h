@@ -182,7 +182,11 @@ size_t aq_workspace_bytes(aq_ctx *ctx);
  * rocm_moe_mlx_affine_routes path (go/engine/hip/hip_gemma4_moe.go:294-446).
  * A route whose expert id or x row is out of range yields zeros (the host
  * cannot see device ids; the by-index helper of qmv_gather.go:405-409 checks
- * on the host instead). */
+ * on the host instead).
+ * Calls of more than 64 routes (a prompt, a decode batch larger than the expert count) may run grouped by expert: the
+ * routes are sorted on the device and an expert's weights read once per 16 to 256 of its routes; scratch comes from the
+ * context's workspace (about 2 * K bytes a route; during a capture that would have to grow it, the per-route kernels run).
+ * Up to 64 routes every output has the bytes of aq_qmv on the sliced expert. */
 int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, const void *biases,
                   const int32_t *lhs, const int32_t *rhs, void *y, int routes, int x_rows, int K, int N,
                   int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags);

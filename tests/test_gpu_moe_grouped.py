@@ -1,0 +1,105 @@
+"""Gathered projections of many routes, grouped by expert on the device: against the per-route kernels' contract (the
+float64 reference per route), with ids and rows of x out of range, experts without a route and experts with more routes than
+a tile has rows."""
+import numpy as np
+import pytest
+
+import fixtures as F
+from gpu_util import DeviceAffine, check_accumulators, say
+
+pytestmark = pytest.mark.gpu
+
+
+def _ids(rng, routes, E, skew):
+    """Expert of each route: at random, or most of them one expert with some experts left out."""
+    if not skew:
+        return rng.integers(0, E, routes).astype(np.int32)
+    ids = rng.integers(0, max(1, E // 2), routes)
+    ids[rng.random(routes) < 0.6] = E - 1
+    return ids.astype(np.int32)
+
+
+# tiles of 32, 64, 128 and 256 rows, token tiles of 16 and 32; K and N that end inside a tile; every width and group size
+CASES = [(4, 64, 300, 8, 704, 130, False), (4, 64, 300, 8, 704, 130, True), (4, 32, 700, 6, 512, 264, True), (4, 128, 90, 3, 256, 40, False),
+         (4, 64, 70, 16, 2816, 72, False), (4, 32, 65, 40, 2048, 64, True), (8, 64, 200, 32, 1088, 96, True), (8, 32, 700, 8, 320, 33, False),
+         (4, 64, 1000, 2, 192, 515, True)]
+
+
+@pytest.mark.parametrize("bits,gs,routes,E,K,N,skew", CASES)
+def test_grouped_gather(ctx, orc, bits, gs, routes, E, K, N, skew):
+    import aq_mi355
+    say("grouped gather", bits, gs, routes, E, K, N, skew)
+    rng = np.random.default_rng(routes + K)
+    expert_rows, gate_base, up_base = 2 * ((N + 15) // 16 * 16), 0, (N + 15) // 16 * 16
+    words, s, b = F.synthetic_affine(E * expert_rows, K, bits, gs, seed=2800 + K)
+    x_rows = routes // 2
+    x = F.synthetic_x(x_rows, K, seed=2801)
+    rhs, lhs = _ids(rng, routes, E, skew), rng.integers(0, x_rows, routes).astype(np.int32)
+    bad = {3: "rhs", 11: "rhs", 20: "lhs", routes - 1: "lhs"}
+    rhs[3], rhs[11], lhs[20], lhs[routes - 1] = -1, E, x_rows, -5
+    dw = DeviceAffine(ctx, words, s, b)
+    dx, dl, dr, dy = ctx.to_device(x), ctx.to_device(lhs), ctx.to_device(rhs), ctx.alloc(routes * N * 4)
+    refs = {}
+    for base in (gate_base, up_base):
+        ctx.fill_zero(dy)
+        ctx.gather_qmv(dx, dw.w, dw.s, dw.b, dl, dr, dy, routes, x_rows, K, N, E, expert_rows, base, gs, bits, aq_mi355.AQ_OUT_F32)
+        ctx.sync()
+        assert "grouped" in ctx.last_variant(0), ctx.last_variant(0)
+        got = dy.download(np.float32, routes * N).reshape(routes, N)
+        ref = np.zeros((routes, N))
+        for e in range(E):
+            z = [r for r in np.nonzero(rhs == e)[0] if r not in bad]
+            if z:
+                rows = slice(e * expert_rows + base, e * expert_rows + base + N)
+                ref[z] = F.reference_f64(x[lhs[z]], words[rows], s[rows], b[rows], bits, gs, K)
+        assert not got[list(bad)].any(), "ids out of range give zeros"
+        check_accumulators(got, ref, "grouped gather, rows from %d" % base)
+        refs[base] = got
+        out = ctx.alloc(routes * N * 2)
+        ctx.gather_qmv(dx, dw.w, dw.s, dw.b, dl, dr, out, routes, x_rows, K, N, E, expert_rows, base, gs, bits)
+        ctx.sync()
+        assert np.array_equal(out.download(np.uint16, routes * N), F.f32_to_bf16_bits(got).reshape(-1))
+        out.free()
+    ctx.fill_zero(dy)
+    ctx.gather_qmv_gate_up(dx, dw.w, dw.s, dw.b, dl, dr, dy, routes, x_rows, K, N, E, expert_rows, gate_base, up_base, gs, bits,
+                           aq_mi355.AQ_ACT_SILU, aq_mi355.AQ_OUT_F32)
+    ctx.sync()
+    assert "grouped" in ctx.last_variant(0), ctx.last_variant(0)
+    got = dy.download(np.float32, routes * N).reshape(routes, N)
+    g, u = refs[gate_base], refs[up_base]
+    want = orc.act_multiply(aq_mi355.AQ_ACT_SILU, g.reshape(-1), u.reshape(-1)).reshape(routes, N)
+    # the same fp32 sums; exp of the device library against the oracle's: a few fp32 ulp
+    assert (np.abs(got - want) <= 4e-6 * np.abs(want) + 2.5e-7 * np.maximum(1.0, np.abs(g * u))).all()
+    for t in (dx, dl, dr, dy, dw):
+        t.free()
+
+
+def test_grouped_gather_captured(ctx):
+    """Recorded into a graph and replayed over changing ids: every replay equals the eager call."""
+    import aq_mi355
+    routes, E, K, N = 130, 4, 512, 64
+    say("grouped gather in a graph")
+    rng = np.random.default_rng(5)
+    words, s, b = F.synthetic_affine(E * N, K, 4, 64, seed=2900)
+    x = F.synthetic_x(routes, K, seed=2901)
+    dw = DeviceAffine(ctx, words, s, b)
+    dx, dl, dr, dy = ctx.to_device(x), ctx.to_device(np.arange(routes, dtype=np.int32)), ctx.alloc(routes * 4), ctx.alloc(routes * N * 4)
+    call = lambda: ctx.gather_qmv(dx, dw.w, dw.s, dw.b, dl, dr, dy, routes, routes, K, N, E, N, 0, 64, 4, aq_mi355.AQ_OUT_F32)
+    eager, sets = [], [rng.integers(0, E, routes).astype(np.int32) for _ in range(3)]
+    for ids in sets:
+        dr.upload(ids)
+        call()
+        ctx.sync()
+        eager.append(dy.download(np.float32, routes * N).copy())
+    ctx.capture_begin()
+    call()
+    graph = ctx.capture_end()
+    for ids, want in zip(sets, eager):
+        ctx.fill_zero(dy)
+        dr.upload(ids)
+        ctx.graph_launch(graph)
+        ctx.sync()
+        assert np.array_equal(dy.download(np.uint32, routes * N), want.view(np.uint32))
+    ctx.graph_destroy(graph)
+    for t in (dx, dl, dr, dy, dw):
+        t.free()
