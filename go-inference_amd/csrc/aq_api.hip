@@ -16,6 +16,7 @@
 #include <string>
 #include <vector>
 
+#include "aq_host_stage.h"
 #include "aq_kernels.h"
 #include "aq_qmm.h"
 #include "aq_tile.h"
@@ -79,6 +80,8 @@ struct aq_ctx {
     void* head_fold = nullptr;     // aq_qmv_greedy's fold tickets and slots (aq::kHeadFoldBytes, kept zeroed by the kernel)
     unsigned char* static_scratch = nullptr;  // this device's copy of `scratch` (hipGetSymbolAddress at creation)
     char name[256] = {0};
+    std::mutex host_mu;     // one staged host call at a time
+    aq::HostStage* host = nullptr;
 };
 
 namespace {
@@ -510,6 +513,7 @@ void aq_destroy(aq_ctx* ctx) {
         (void)hipStreamSynchronize(ctx->own_stream);
         (void)hipStreamDestroy(ctx->own_stream);
     }
+    delete ctx->host;
     if (ctx->ws.ptr) (void)hipFree(ctx->ws.ptr);
     if (ctx->head_ws.ptr) (void)hipFree(ctx->head_ws.ptr);
     if (ctx->head_fold) (void)hipFree(ctx->head_fold);
@@ -2067,6 +2071,74 @@ int aq_gguf_to_affine(aq_ctx* ctx, int gguf_type, const void* src, uint64_t src_
     return AQ_OK;
 }
 
+namespace {
+
+// y = x . dequant(weights)^T with everything in host memory: one staged upload (aq_host_stage.h), the call, one download.
+// x is bf16, or fp32 rounded to bf16 on the way (f32); out likewise.
+int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, const uint8_t* packed, size_t packed_len, const uint8_t* scales,
+                     const uint8_t* biases, size_t sb_len, int M, int K, int N, int group_size, int bits, void* out, bool out_f32) {
+    const size_t x_bytes = (size_t)M * K * 2, y_bytes = (size_t)M * N * 2;
+    const size_t at_s = align256(x_bytes), at_b = at_s + align256(sb_len), at_w = at_b + align256(sb_len), total = at_w + align256(packed_len);
+    const aq::HostPart parts[4] = {{x, x_bytes, 0, x_f32}, {scales, sb_len, at_s, false}, {biases, sb_len, at_b, false}, {packed, packed_len, at_w, false}};
+    std::lock_guard<std::mutex> host_lk(ctx->host_mu);
+    if (!ctx->host) ctx->host = new (std::nothrow) aq::HostStage();
+    if (!ctx->host) return fail(AQ_ERR_NOMEM, "%s: out of host memory", op);
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    hipStream_t stream;
+    {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        stream = ctx->stream;
+    }
+    // small results are stored to pinned host memory by the kernel itself; larger ones cross in one copy, which fills the
+    // link better than a tile's stores
+    const bool direct = y_bytes <= ((size_t)64 << 10);
+    char* dev = nullptr;
+    void* host_y = nullptr;
+    AQ_HIP(ctx->host->results(y_bytes, &host_y), "hipHostMalloc");
+    const size_t dev_total = total + (direct ? 0 : align256(y_bytes));
+    AQ_HIP(ctx->host->reserve_device(dev_total), "hipMalloc");
+    const hipError_t up = ctx->host->upload(parts, 4, total, stream, &dev);
+    int rc = AQ_OK;
+    if (up != hipSuccess) {
+        rc = hip_fail(up, "hipMemcpyHtoD");
+    } else {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        if (ctx->stream != stream) (void)hipStreamSynchronize(stream);  // (the caller moved the context meanwhile)
+        stream = ctx->stream;
+        aq::QmvArgs a{};
+        a.x = reinterpret_cast<const uint16_t*>(dev);
+        a.s = reinterpret_cast<const uint16_t*>(dev + at_s);
+        a.b = reinterpret_cast<const uint16_t*>(dev + at_b);
+        a.w = reinterpret_cast<const uint32_t*>(dev + at_w);
+        a.y = direct ? host_y : dev + total;
+        a.K = K;
+        a.N = N;
+        a.M = M;
+        a.routes = 1;
+        if (M <= aq::kQmvMaxRows && (M == 1 || ctx->forced[1] < 0))
+            rc = launch_qmv_rows(ctx, a, group_size, bits, false);
+        else
+            rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], a.x, a.w, a.s, a.b, a.y, M, K, N,
+                                  group_size, bits, false, fail);
+        if (rc == AQ_OK && !direct) {
+            const hipError_t down = hipMemcpyAsync(host_y, dev + total, y_bytes, hipMemcpyDeviceToHost, stream);
+            if (down != hipSuccess) rc = hip_fail(down, "hipMemcpyDtoH");
+        }
+    }
+    const hipError_t done = hipStreamSynchronize(stream);
+    if (rc == AQ_OK && done != hipSuccess) rc = hip_fail(done, "hipStreamSynchronize");
+    if (rc == AQ_OK) {
+        if (out_f32)
+            ctx->host->widen(static_cast<float*>(out), static_cast<const uint16_t*>(host_y), (size_t)M * N);
+        else
+            memcpy(out, host_y, y_bytes);
+    }
+    ctx->host->finish();
+    return rc;
+}
+
+}  // namespace
+
 int aq_matvec_host(aq_ctx* ctx, const uint8_t* x, size_t x_len, const uint8_t* packed, size_t packed_len,
                    const uint8_t* scales, size_t scales_len, const uint8_t* biases, size_t biases_len, int out_dim,
                    int in_dim, int group_size, int bits, uint8_t* out, size_t out_len) {
@@ -2087,19 +2159,8 @@ int aq_matvec_host(aq_ctx* ctx, const uint8_t* x, size_t x_len, const uint8_t* p
     if (out_len < (size_t)out_dim * 2) return fail(AQ_ERR_SIZE, "aq_matvec_host: out holds fewer than outDim bf16 values");
     if (!x || !packed || !scales || !biases || !out) return fail(AQ_ERR_ARG, "aq_matvec_host: null operand");
     if (int rc = check_geometry("aq_matvec_host", in_dim, group_size, bits)) return rc;
-    DevBuf dx, dw, ds, db, dy;
-    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    AQ_HIP(dx.alloc(x_len), "hipMalloc");
-    AQ_HIP(dw.alloc(packed_len), "hipMalloc");
-    AQ_HIP(ds.alloc(scales_len), "hipMalloc");
-    AQ_HIP(db.alloc(biases_len), "hipMalloc");
-    AQ_HIP(dy.alloc((size_t)out_dim * 2), "hipMalloc");
-    if (int rc = aq_h2d(ctx, dx.p, x, x_len)) return rc;
-    if (int rc = aq_h2d(ctx, dw.p, packed, packed_len)) return rc;
-    if (int rc = aq_h2d(ctx, ds.p, scales, scales_len)) return rc;
-    if (int rc = aq_h2d(ctx, db.p, biases, biases_len)) return rc;
-    if (int rc = aq_qmv(ctx, dx.p, dw.p, ds.p, db.p, dy.p, 1, in_dim, out_dim, group_size, bits, 0)) return rc;
-    return aq_d2h(ctx, out, dy.p, (size_t)out_dim * 2);
+    return staged_host_call(ctx, "aq_matvec_host", x, false, packed, packed_len, scales, biases, scales_len, 1, in_dim, out_dim, group_size,
+                            bits, out, false);
 }
 
 int aq_proj_quant_matmul_host(aq_ctx* ctx, float* out, const float* x, size_t x_len, const uint8_t* packed,
@@ -2117,39 +2178,9 @@ int aq_proj_quant_matmul_host(aq_ctx* ctx, float* out, const float* x, size_t x_
     if (packed_len != want_packed || scales_len != want_sb || biases_len != want_sb)
         return fail(AQ_ERR_SIZE, "aq_proj_quant_matmul_host: packed/scales/biases size mismatch");
     if (!out || !x || !packed || !scales || !biases) return fail(AQ_ERR_ARG, "aq_proj_quant_matmul_host: null operand");
-    // f32 -> bf16 RNE at the seam (quant_seam_backend.go:50,66-74; codec mlxaffine.go:229-237)
-    std::vector<uint16_t> xb((size_t)M * K);
-    for (size_t i = 0; i < xb.size(); i++) {
-        uint32_t u;
-        memcpy(&u, &x[i], 4);
-        if ((u & 0x7fffffffu) > 0x7f800000u) {
-            xb[i] = (uint16_t)((u >> 16) | 0x0040u);
-        } else {
-            u += 0x7fffu + ((u >> 16) & 1u);
-            xb[i] = (uint16_t)(u >> 16);
-        }
-    }
-    DevBuf dx, dw, ds, db, dy;
-    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    AQ_HIP(dx.alloc(xb.size() * 2), "hipMalloc");
-    AQ_HIP(dw.alloc(packed_len), "hipMalloc");
-    AQ_HIP(ds.alloc(scales_len), "hipMalloc");
-    AQ_HIP(db.alloc(biases_len), "hipMalloc");
-    AQ_HIP(dy.alloc((size_t)M * N * 2), "hipMalloc");
-    if (int rc = aq_h2d(ctx, dx.p, xb.data(), xb.size() * 2)) return rc;
-    if (int rc = aq_h2d(ctx, dw.p, packed, packed_len)) return rc;
-    if (int rc = aq_h2d(ctx, ds.p, scales, scales_len)) return rc;
-    if (int rc = aq_h2d(ctx, db.p, biases, biases_len)) return rc;
-    int rc = (M == 1) ? aq_qmv(ctx, dx.p, dw.p, ds.p, db.p, dy.p, 1, K, N, group_size, bits, 0)
-                      : aq_qmm(ctx, dx.p, dw.p, ds.p, db.p, dy.p, M, K, N, group_size, bits, 0);
-    if (rc) return rc;
-    std::vector<uint16_t> yb((size_t)M * N);
-    if (int rc2 = aq_d2h(ctx, yb.data(), dy.p, yb.size() * 2)) return rc2;
-    for (size_t i = 0; i < yb.size(); i++) {
-        uint32_t u = (uint32_t)yb[i] << 16;
-        memcpy(&out[i], &u, 4);
-    }
-    return AQ_OK;
+    // f32 -> bf16 RNE at the seam (quant_seam_backend.go:50,66-74; codec mlxaffine.go:229-237), bf16 -> f32 on the way back
+    return staged_host_call(ctx, "aq_proj_quant_matmul_host", x, true, packed, packed_len, scales, biases, scales_len, M, K, N, group_size,
+                            bits, out, true);
 }
 
 int aq_variant_count(int op) {
