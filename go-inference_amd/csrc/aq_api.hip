@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <exception>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -2076,7 +2077,7 @@ namespace {
 // y = x . dequant(weights)^T with everything in host memory: one staged upload (aq_host_stage.h), the call, one download.
 // x is bf16, or fp32 rounded to bf16 on the way (f32); out likewise.
 int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, const uint8_t* packed, size_t packed_len, const uint8_t* scales,
-                     const uint8_t* biases, size_t sb_len, int M, int K, int N, int group_size, int bits, void* out, bool out_f32) {
+                     const uint8_t* biases, size_t sb_len, int M, int K, int N, int group_size, int bits, void* out, bool out_f32) try {
     const size_t x_bytes = (size_t)M * K * 2, y_bytes = (size_t)M * N * 2;
     const size_t at_s = align256(x_bytes), at_b = at_s + align256(sb_len), at_w = at_b + align256(sb_len), total = at_w + align256(packed_len);
     const aq::HostPart parts[4] = {{x, x_bytes, 0, x_f32}, {scales, sb_len, at_s, false}, {biases, sb_len, at_b, false}, {packed, packed_len, at_w, false}};
@@ -2094,7 +2095,8 @@ int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, con
     const bool direct = y_bytes <= ((size_t)64 << 10);
     char* dev = nullptr;
     void* host_y = nullptr;
-    AQ_HIP(ctx->host->results(y_bytes, &host_y), "hipHostMalloc");
+    const size_t y_piece = y_bytes < aq::HostStage::kMostResults ? y_bytes : aq::HostStage::kMostResults;
+    AQ_HIP(ctx->host->results(y_piece, &host_y), "hipHostMalloc");
     const size_t dev_total = total + (direct ? 0 : align256(y_bytes));
     AQ_HIP(ctx->host->reserve_device(dev_total), "hipMalloc");
     const hipError_t up = ctx->host->upload(parts, 4, total, stream, &dev);
@@ -2120,21 +2122,25 @@ int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, con
         else
             rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], a.x, a.w, a.s, a.b, a.y, M, K, N,
                                   group_size, bits, false, fail);
-        if (rc == AQ_OK && !direct) {
-            const hipError_t down = hipMemcpyAsync(host_y, dev + total, y_bytes, hipMemcpyDeviceToHost, stream);
-            if (down != hipSuccess) rc = hip_fail(down, "hipMemcpyDtoH");
-        }
     }
-    const hipError_t done = hipStreamSynchronize(stream);
-    if (rc == AQ_OK && done != hipSuccess) rc = hip_fail(done, "hipStreamSynchronize");
-    if (rc == AQ_OK) {
+    // the result crosses in pieces of the pinned block (one, but for results of many rows)
+    for (size_t at = 0; at < y_bytes && rc == AQ_OK; at += y_piece) {
+        const size_t n = y_bytes - at < y_piece ? y_bytes - at : y_piece;
+        hipError_t down = direct ? hipSuccess : hipMemcpyAsync(host_y, dev + total + at, n, hipMemcpyDeviceToHost, stream);
+        if (down != hipSuccess) rc = hip_fail(down, "hipMemcpyDtoH");
+        down = hipStreamSynchronize(stream);
+        if (rc == AQ_OK && down != hipSuccess) rc = hip_fail(down, "hipStreamSynchronize");
+        if (rc != AQ_OK) break;
         if (out_f32)
-            ctx->host->widen(static_cast<float*>(out), static_cast<const uint16_t*>(host_y), (size_t)M * N);
+            ctx->host->widen(static_cast<float*>(out) + at / 2, static_cast<const uint16_t*>(host_y), n / 2);
         else
-            memcpy(out, host_y, y_bytes);
+            memcpy(static_cast<char*>(out) + at, host_y, n);
     }
+    if (rc != AQ_OK) (void)hipStreamSynchronize(stream);  // the uploads that went out before the error read the ring
     ctx->host->finish();
     return rc;
+} catch (const std::exception&) {  // no memory for the upload's bookkeeping: thrown before anything is queued, or after it is done
+    return fail(AQ_ERR_NOMEM, "%s: out of host memory", op);
 }
 
 }  // namespace

@@ -23,11 +23,12 @@ public:
     // Queues the parts' upload on `stream`; *dev is the device block of `total` bytes (a multiple of 256).  The host slices
     // have been read when it returns.
     hipError_t upload(const HostPart* parts, int count, size_t total, hipStream_t stream, char** dev);
-    // Pinned host memory of at least `bytes` that kernels may write, for results.
+    // Pinned host memory of at least `bytes` (at most kMostResults) that kernels may write, for results.
+    static constexpr size_t kMostResults = (size_t)16 << 20;
     hipError_t results(size_t bytes, void** host);
     // out[i] = fp32 of n bf16 values, shared out over the worker threads when there are many.
     void widen(float* out, const uint16_t* in, size_t n);
-    // Ends a call (the stream has been waited for): blocks larger than what is kept between calls are freed.
+    // Ends a call (the stream has been waited for): a device block larger than what is kept between calls is freed.
     void finish();
 
 private:

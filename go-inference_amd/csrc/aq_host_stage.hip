@@ -14,6 +14,7 @@
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -25,7 +26,6 @@ constexpr size_t kPiece = (size_t)128 << 10;     // bytes a thread copies at a t
 constexpr int kFirstRun = 3, kLongRun = 32;      // pieces of the first copy kernel, and of a long one
 constexpr size_t kRing = (size_t)64 << 20;       // pinned memory at most
 constexpr size_t kKeepDevice = (size_t)256 << 20;  // device memory kept between calls at most
-constexpr size_t kKeepOut = (size_t)16 << 20;    // pinned memory for results kept between calls at most
 constexpr size_t kAlone = (size_t)384 << 10;     // the caller copies this much by itself: waking threads costs about as much
 constexpr int kWorkers = 5;
 
@@ -62,7 +62,12 @@ struct HostStage::Pool {
     std::atomic<int> next{0}, limit{0}, busy{0}, units{0};  // units below `limit` may be taken
 
     Pool() {
-        for (int i = 0; i < kWorkers; i++) threads.emplace_back([this] { run(); });
+        threads.reserve(kWorkers);
+        try {
+            for (int i = 0; i < kWorkers; i++) threads.emplace_back([this] { run(); });
+        } catch (const std::system_error&) {
+            // the process may start no more threads: those there are, or the caller alone, do the work
+        }
     }
     ~Pool() {
         {
@@ -239,11 +244,6 @@ void HostStage::finish() {
         (void)hipFree(dev_);
         dev_ = nullptr;
         dev_bytes_ = 0;
-    }
-    if (out_bytes_ > kKeepOut) {
-        (void)hipHostFree(out_);
-        out_ = nullptr;
-        out_bytes_ = 0;
     }
 }
 

@@ -11,9 +11,10 @@ from gpu_util import DeviceAffine, run_qmv, say
 pytestmark = pytest.mark.gpu
 
 
-# one copy by the caller; just beyond it; a few runs; the last piece short; beyond the ring of 64 MiB
+# one copy by the caller; just beyond it; a few runs; the last piece short; beyond the ring of 64 MiB; a result beyond the
+# pinned block of 16 MiB
 @pytest.mark.parametrize("M,K,N,bits,gs", [(1, 64, 8, 4, 64), (1, 1024, 700, 4, 64), (3, 1024, 800, 4, 32), (1, 4096, 4096, 8, 64), (70, 2048, 3001, 4, 64),
-                                           (1, 4096, 33000, 4, 64)])
+                                           (1, 4096, 33000, 4, 64), (300, 64, 33001, 4, 64)])
 def test_staged_call_has_the_bytes_of_the_resident_call(ctx, M, K, N, bits, gs):
     say("host slices", M, K, N, bits, gs)
     words, s, b = F.synthetic_affine(N, K, bits, gs, seed=3000 + N)
