@@ -899,14 +899,14 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     unsigned in_grid = 0;
     if (ctx->forced[1] < 0)
         for (int i = 0; i < count; i++) {
-            if (!aq::qmmh_takes(x, packed[i], K, group_size, bits) || !aq::qmmh_runs(M, K, N[i], group_size)) continue;
+            if (!aq::qmmh_takes(x, packed[i], K, group_size, bits) || !aq::qmmh_runs(M, K, N[i], group_size, bits)) continue;
             aq::QmmSegment& seg = q.seg[q.nseg++];
             seg.w = static_cast<const uint32_t*>(packed[i]);
             seg.s = static_cast<const uint16_t*>(scales[i]);
             seg.b = static_cast<const uint16_t*>(biases[i]);
             seg.y = y[i];
             seg.N = N[i];
-            aq::qmmh_split(M, K, &seg, ctx->cu_count);
+            aq::qmmh_split(M, K, bits, &seg, ctx->cu_count);
             in_grid |= 1u << i;
         }
     if (q.nseg > 0) {
@@ -914,6 +914,7 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         q.M = M;
         q.K = K;
         q.group_size = group_size;
+        q.bits = bits;
         q.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
         half_need = aq::qmm_scratch_bytes(M, K, 0, ctx->cu_count) + aq::qmmh_partial_bytes(q);
         need = half_need > need ? half_need : need;
@@ -988,7 +989,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     const bool tok_fits = aq::qmvt_grouped_fits(a, bits, group_size, pair) && !(ctx->families_off >> kFamTok & 1);
     if (!tiles_fit && !tok_fits) return kPass;
     const bool tiles = tiles_fit && !(tok_fits && per_expert <= 12 && a.K >= 2048);
-    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= 32 ? 32 : per_expert <= 96 ? 64 : per_expert <= 384 ? 128 : 256;
+    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= 32 ? 32 : per_expert <= 96 ? 64 : per_expert <= 384 || bits == 8 ? 128 : 256;
     const int pad = tiles ? 32 : 1;
     const int most_chunks = a.routes / chunk + groups;
     const int most_rows = a.routes + groups * (pad - 1);
@@ -1027,6 +1028,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     q.M = most_rows;
     q.K = a.K;
     q.group_size = group_size;
+    q.bits = bits;
     q.nseg = pair ? 2 : 1;
     q.pair = pair ? 1 : 0;
     q.act = a.act;
@@ -1049,7 +1051,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     q.row_base = a.row_base;
     q.row_base2 = a.row_base2;
     int idx = 0;
-    while (idx < aq::qmmh_variant_count() && !(aq::qmmh_rows(idx) == chunk && (chunk != 256 || aq::qmmh_variant(idx)->wn == 4))) idx++;
+    while (idx < aq::qmmh_variant_count() && !(aq::qmmh_variant(idx)->bits == bits && aq::qmmh_rows(idx) == chunk && (chunk != 256 || aq::qmmh_variant(idx)->wn == 4))) idx++;
     if (idx >= aq::qmmh_variant_count()) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv: no tiles of %d rows", chunk);
     const char* name = nullptr;
     const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, idx, q, &name, fail, nullptr);
@@ -1261,7 +1263,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     }
     if (M > 32 && ctx->forced[0] < 0 && ctx->forced[1] < 0 && !(ctx->families_off >> kFamTiles & 1) &&
         aq::qmmh_takes(x, up_packed, K, group_size, bits) && aq::qmmh_takes(x, gate_packed, K, group_size, bits) &&
-        aq::qmmh_runs(M, K, N, group_size)) {
+        aq::qmmh_runs(M, K, N, group_size, bits)) {
         // prefill sizes on the fp16-operand kernels: one launch, the tiles of which hold gate and up columns side by side; no
         // intermediate reaches memory
         std::lock_guard<std::mutex> lk(ctx->mu);
@@ -1270,6 +1272,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         q.M = M;
         q.K = K;
         q.group_size = group_size;
+        q.bits = bits;
         q.nseg = 2;
         q.pair = 1;
         q.act = act;

@@ -26,7 +26,7 @@ struct QmmArgs {
 };
 
 // Which pass over x the workspace holds (QmmArgs.x_ready, and what a launch reports back through qmm_dispatch).
-enum { kXReadyNone = 0, kXReadyTile4 = 1, kXReadyTile8 = 2, kXReadyHalf = 3, kXReadyHalf32 = 4 };
+enum { kXReadyNone = 0, kXReadyTile4 = 1, kXReadyTile8 = 2, kXReadyHalf = 3, kXReadyHalf32 = 4, kXReadyHalf8 = 5, kXReadyHalf8G32 = 6 };
 
 struct QmmVariant {
     const char* name;
@@ -77,7 +77,7 @@ int qmmf_variant_count();
 const QmmVariant* qmmf_variant(int idx);
 hipError_t qmmf_launch_kernel(int idx, const QmmTileArgs& a, hipStream_t stream);
 
-// 4-bit kernels whose matrix-core operand carries scale * (code - 8) as fp16 (aq_qmm_half.hip); same workspace.
+// Kernels with fp16 matrix-core operands (aq_qmm_half.hip): 4 bit, scale * (code - 8); 8 bit, code - 128.  Same workspace.
 constexpr int kQmmSegments = 8;  // weight matrices of one call
 struct QmmSegment {
     const uint32_t* w;
@@ -108,7 +108,7 @@ struct QmmHalfArgs {
 };
 struct QmmHalfCall {
     const uint16_t* x;
-    int M, K, group_size;
+    int M, K, group_size, bits;
     QmmSegment seg[kQmmSegments];
     int nseg, pair, act, out_f32;
     int x_ready;  // kXReady*
@@ -118,11 +118,12 @@ struct QmmHalfCall {
 };
 int qmmh_variant_count();
 const QmmVariant* qmmh_variant(int idx);
+int qmmh_x_kind(int bits, int group_size);  // the pass over x their kernels need (kXReady*)
 int qmmh_rows(int idx);  // rows of x of a workgroup tile
 hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream);
-// How a matrix of seg->N columns shares K out for M rows of x: a function of M, K and N alone, so that the call of several
+// How a matrix of seg->N columns shares K out for M rows of x: a function of M, K, N and the code width alone, so that the call of several
 // matrices, the gated pair and a call of its own add in the same order and give the same bytes.
-void qmmh_split(int M, int K, QmmSegment* seg, int cu_count);
+void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count);
 // The kernel for these matrices (the bytes of a result do not depend on it).
 int qmmh_pick(const QmmHalfCall& q, int cu_count);
 size_t qmmh_partial_bytes(const QmmHalfCall& q);
@@ -167,10 +168,10 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
                  const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
                  int group_size, int bits, bool out_f32, FailFn fail, const float* gate = nullptr, int act = 0,
                  int* x_state = nullptr);
-// Whether the fp16-operand kernels take a call (4-bit codes, groups of 32, 64 or 128, K a multiple of 64).
+// Whether the fp16-operand kernels take a call (4- or 8-bit codes, groups of 32, 64 or 128, K a multiple of 64).
 bool qmmh_takes(const void* x, const void* packed, int K, int group_size, int bits);
 // Whether an unforced call on one matrix runs on them (the choice among the families by shape).
-bool qmmh_runs(int M, int K, int N, int group_size);
+bool qmmh_runs(int M, int K, int N, int group_size, int bits);
 // One call of them over q.nseg matrices, or on expert slabs (idx < 0: qmmh_pick); x_state as in qmm_dispatch.  Scratch that
 // cannot be had because the stream is being captured: kQmmhNoScratch, nothing launched.
 constexpr int kQmmhNoScratch = INT32_MIN;

@@ -4,8 +4,8 @@
 // Replaces the selector of rocm_mlx_q4_projection_batch* (go/engine/hip/hip_projection_launch.go:5192-5287; kernels
 // go/engine/hip/kernels/quant/affine_projection_tuned.hipinc:166-1109) with the semantics of MLX affine_qmm_t
 // (go/engine/metal/quant_seam_backend.go:77-109, go/engine/metal/attention.go:731-751).  The kernels themselves are in
-// aq_qmm_tile.hip (bf16 codes as MFMA operands, fp32 scaling of the partial products), aq_qmm_half.hip (4 bit:
-// scale * (code - 8) as fp16 operands) and aq_qmm_few.hip (5..64 rows of x, K shared out over workgroups).
+// aq_qmm_tile.hip (bf16 codes as MFMA operands, fp32 scaling of the partial products), aq_qmm_half.hip (fp16 operands:
+// 4 bit scale * (code - 8), 8 bit code - 128) and aq_qmm_few.hip (5..64 rows of x, K shared out over workgroups).
 #include "aq_device.h"
 #include "aq_kernels.h"
 #include "aq_qmm.h"
@@ -86,9 +86,11 @@ size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
         q.M = M;
         q.nseg = 1;
         q.seg[0].N = N;
-        qmmh_split(M, K, &q.seg[0], cu_count);
-        const size_t half = qmmh_partial_bytes(q);
-        partial = half > partial ? half : partial;
+        for (int bits : {4, 8}) {
+            qmmh_split(M, K, bits, &q.seg[0], cu_count);
+            const size_t half = qmmh_partial_bytes(q);
+            partial = half > partial ? half : partial;
+        }
     }
     return xbytes + ((partial + 255) & ~(size_t)255);
 }
@@ -112,23 +114,26 @@ static int find_qmmt_named(const char* name) {
 }
 
 bool qmmh_takes(const void* x, const void* packed, int K, int group_size, int bits) {
-    return bits == 4 && (group_size == 32 || group_size == 64 || group_size == 128) && K % 64 == 0 && K % group_size == 0 &&
+    return (bits == 4 || bits == 8) && (group_size == 32 || group_size == 64 || group_size == 128) && K % 64 == 0 && K % group_size == 0 &&
            (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(packed) & 15) == 0;
 }
 
 // Groups of 64 / 128 keep the bf16-code kernels where those are ahead: up to 64 rows with K in whole quads of blocks (the
-// few-rows kernels) or a handful of blocks of K, and up to 256 rows by a wide matrix with a short K, where the cheaper pass
-// over x shows (256 x 2048 x 14336; at K = 4096 and 128 x 128 tiles 69 us here against 72).
-bool qmmh_runs(int M, int K, int N, int group_size) {
+// few-rows kernels) or a handful of blocks of K (8 bit, 300 x 320 x 4096: 13.7 us against 15.6, 2048 x 320 x 14336: 49
+// against 58), and up to 256 rows by a wide matrix with a short K, where the cheaper pass over x shows (256 x 2048 x 14336;
+// at K = 4096 and 128 x 128 tiles 69 us here against 72; 8 bit 256 x 1024 x 14336: 22.1 against 25.2, but 100 x 2048 x 14336
+// 35 against 30 on 32 x 256 tiles).
+bool qmmh_runs(int M, int K, int N, int group_size, int bits) {
     if (group_size == 32) return true;
     if (M <= 32) return false;
-    if (M <= 64) return K % 256 != 0 && K >= 512;
-    return !(M <= 256 && K <= 2048 && N >= 12288);
+    if (M <= 64) return bits == 4 && K % 256 != 0 && K >= 512;
+    if (bits == 8 && K < 512) return false;
+    return !(M <= 256 && (bits == 4 || M > 128) && K <= 2048 && N >= 12288);
 }
 
 int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCall& q, const char** last_variant, FailFn fail, int* x_state) {
     if (!q.chunks)
-        for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, &q.seg[i], cu_count);
+        for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, q.bits, &q.seg[i], cu_count);
     const size_t xbytes = (qmmt_workspace_bytes(q.chunks ? q.most_rows : q.M, q.K) + 255) & ~(size_t)255;
     const size_t need = xbytes + qmmh_partial_bytes(q);
     if (!workspace_may_grow(ws, need, stream)) return kQmmhNoScratch;
@@ -140,7 +145,7 @@ int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCa
     *last_variant = qmmh_variant(idx)->name;
     hipError_t rc = qmmh_launch(idx, q, ws->ptr, stream);
     if (rc != hipSuccess) return fail((int)rc, "rocm.hip.hipLaunchKernel: HIP returned %d (%s)", (int)rc, hipGetErrorString(rc));
-    if (x_state) *x_state = q.group_size == 32 ? kXReadyHalf32 : kXReadyHalf;
+    if (x_state) *x_state = qmmh_x_kind(q.bits, q.group_size);
     return AQ_OK;
 }
 
@@ -153,12 +158,13 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
                  const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
                  int group_size, int bits, bool out_f32, FailFn fail, const float* gate, int act, int* x_state) {
     const bool mfma_ok = qmm_takes_gate(x, packed, K, group_size, bits);
-    if (forced < 0 && !gate && qmmh_takes(x, packed, K, group_size, bits) && qmmh_runs(M, K, N, group_size)) {
+    if (forced < 0 && !gate && qmmh_takes(x, packed, K, group_size, bits) && qmmh_runs(M, K, N, group_size, bits)) {
         QmmHalfCall q{};
         q.x = static_cast<const uint16_t*>(x);
         q.M = M;
         q.K = K;
         q.group_size = group_size;
+        q.bits = bits;
         q.seg[0].w = static_cast<const uint32_t*>(packed);
         q.seg[0].s = static_cast<const uint16_t*>(scales);
         q.seg[0].b = static_cast<const uint16_t*>(biases);

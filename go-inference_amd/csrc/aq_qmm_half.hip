@@ -1,4 +1,5 @@
-// affine_qmm for gfx950, 4-bit codes, prefill sizes: the scale rides inside the matrix-core operand.
+// affine_qmm for gfx950, prefill sizes, fp16 matrix-core operands; 4-bit codes: the scale rides inside the operand (8-bit
+// codes: see BITS 8 at the kernel).
 //
 // Same contract as the tile kernels of aq_qmm_tile.hip (MLX affine_qmm_t,
 // go/engine/metal/quant_seam_backend.go:77-109; replaces rocm_mlx_q4_projection_batch*,
@@ -53,6 +54,17 @@ __device__ __forceinline__ uint4 expand_word(uint32_t w, uint32_t mask_s, uint32
     return v;
 }
 
+// 8 codes of two packed words of 8-bit codes -> 8 fp16 values code - 128 in their natural order: the bytes go into the
+// mantissa of fp16 1024.0, whose unit in the last place is 1, and 1152 comes off again; both steps are exact
+__device__ __forceinline__ f16x8_t expand_bytes(uint2 w) {
+    const f16x2_t off = {(_Float16)-1152.0f, (_Float16)-1152.0f};
+    auto two = [&](uint32_t v, uint32_t sel) {
+        return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2_t, __builtin_amdgcn_perm(0x64646464u, v, sel)) + off);
+    };
+    const uint4 u = {two(w.x, 0x04010400u), two(w.x, 0x04030402u), two(w.y, 0x04010400u), two(w.y, 0x04030402u)};
+    return __builtin_bit_cast(f16x8_t, u);
+}
+
 __device__ __forceinline__ uint32_t dup16(uint32_t h) { return (h & 0xffffu) | (h << 16); }
 
 // 2^e for the largest finite magnitude `mag` (bf16 bits without the sign) such that mag * 2^e has binary
@@ -86,7 +98,9 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // past *live_rows are left alone.
 constexpr int kPrepThreads = 512;
 constexpr int kPrepHold = 8;
-template <int ROWS, int GRP>
+// BITS 8: the order in which the 8-bit kernels take x: a step of 16 codes is 16 consecutive ones (half h the second eight),
+// values in their natural order.
+template <int ROWS, int GRP, int BITS>
 __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xf,
                                                          uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K,
                                                          const int32_t* __restrict__ route_x, const int32_t* __restrict__ live_rows) {
@@ -169,8 +183,9 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
             hv[2 * i + 1] = (_Float16)(bf16_bits_to_f32(w[i] >> 16) * up);
         }
         // slot order (x0,x4)(x1,x5)(x2,x6)(x3,x7): the order in which expand_word emits the codes of a word
-        const f16x8_t o = {hv[0], hv[4], hv[1], hv[5], hv[2], hv[6], hv[3], hv[7]};
-        const int t = c8 & 3, h = c8 >> 2;
+        const f16x8_t o = BITS == 4 ? f16x8_t{hv[0], hv[4], hv[1], hv[5], hv[2], hv[6], hv[3], hv[7]}
+                                    : f16x8_t{hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], hv[6], hv[7]};
+        const int t = BITS == 4 ? c8 & 3 : c8 >> 1, h = BITS == 4 ? c8 >> 2 : c8 & 1;
         const int64_t frag = (int64_t)(row >> 5) * (K / 16) + g * 4 + t;
         *reinterpret_cast<f16x8_t*>(xf + (frag * 64 + h * 32 + (row & 31)) * 8) = o;
     };
@@ -208,9 +223,21 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
 // tiles and 623 us on the large ones, whose LDS addresses then are no constants).  The 16-byte pieces of a row are rotated
 // against those of its neighbours (the piece a lane fetches, not the place it lands in), so that a wavefront's reads of one
 // block hit all banks.
-template <int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
+//
+// BITS 8: scale * (code - 128) has 16 significant bits, more than fp16 holds, so the operand is code - 128 alone (exact) and a
+// group's partial sums P are multiplied by the fp32 scale: out += scale * P, one FMA per output element and group, as in the
+// tile kernels of aq_qmm_tile.hip.  Against those: two vector instructions per pair of codes instead of three, several
+// matrices in one grid, the gated pair, groups of 32 and expert slabs.  A step of the MFMA is 16 consecutive codes, so that
+// groups of 32 are two steps each; bytes are staged one 64-code block at a time, in as many stages as A.
+// Measured (us; bf16-code tiles -> here): 2048 x 4096 x 14336 395 -> 341, a layer of 777 rows (2560 / 10240) 461 -> 375, of 400
+// rows (1472 / 4032) 274 -> 130, of 300 rows in groups of 32 (2048 / 8192) 24.9 ms on the any-width kernel -> 174, 512 tokens
+// through 128 experts (2816 / 704) 3749 -> 338.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
+// instructions of expansion and 64 of scaling; a block takes 0.72 us of a CU for 0.23 us of matrix pipe.
+template <int BITS, int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
 __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfArgs a) {
     constexpr bool G32 = GRP == 32;
+    constexpr bool B8 = BITS == 8;
+    constexpr float CENTRE = B8 ? 128.0f : 8.0f;  // the operand's codes are code - CENTRE
     static_assert(NB == 2, "a pair is two column blocks");
     static_assert(STAGES == 2 || STAGES == 3 || STAGES == 4, "LDS stages");
     constexpr int AHEAD = STAGES - 1;  // iteration g requests block g + AHEAD
@@ -218,11 +245,12 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     constexpr int BN = WN * NB * 32;
     constexpr int NWAVE = WM * WN;
     constexpr int A_STAGE = (BM / 32) * 4096;
-    constexpr int QB = 2;                    // blocks of packed weights per stage
-    constexpr int B_ROW = QB * 32;           // bytes of a weight row per stage
+    constexpr int QB = B8 ? 1 : 2;           // blocks of packed weights per stage
+    constexpr int B_ROW = QB * 8 * BITS;     // bytes of a weight row per stage
+    constexpr int B_BUFS = B8 ? STAGES : 2;
     constexpr int B_STAGE = BN * B_ROW;      // packed codes of QB 64-code blocks
     constexpr int A_BLOCKS = (BM / 32) * 4;  // 1 KiB fragments of A per stage
-    constexpr int PPR = 2 * QB;              // 16-byte pieces of a row per stage
+    constexpr int PPR = B_ROW / 16;          // 16-byte pieces of a row per stage
     constexpr int RPI = kWave / PPR;         // rows a copy instruction covers
     constexpr int NBC = B_STAGE / 1024 / NWAVE;  // B copies a wavefront issues per stage
     static_assert(A_BLOCKS % NWAVE == 0, "A fragments must divide among the wavefronts");
@@ -232,11 +260,12 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     // on their way at the end of the iteration of block Q of a quad, which are those newer than A of the next block, and in a
     // stage's second block none of B's.
     static_assert(AHEAD <= 2, "waits are counted for one or two blocks ahead");
-    auto still_out = [=](int q) constexpr { return (AHEAD - 1) * NA + ((q & 1) == 0 ? NBC : 0); };
+    // BITS 8: iteration g requests A and B of block g + AHEAD.
+    auto still_out = [=](int q) constexpr { return B8 ? (AHEAD - 1) * (NA + NBC) : (AHEAD - 1) * NA + ((q & 1) == 0 ? NBC : 0); };
 
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* const abuf = lds;                     // [STAGES][A_STAGE]
-    uint8_t* const bbuf = lds + STAGES * A_STAGE;  // [2][B_STAGE]
+    uint8_t* const bbuf = lds + STAGES * A_STAGE;  // [B_BUFS][B_STAGE]
     // the same as LDS byte addresses: the copy instructions take theirs from a scalar register, and plain integer
     // arithmetic keeps it on the scalar unit (a pointer would be converted, null check included, per copy)
     const uint32_t abuf_at = __builtin_amdgcn_readfirstlane(lds_offset(lds));
@@ -280,7 +309,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     const int G4 = (Gall + 3) / 4;
     const int ksteps = K / 16;
     const int sb_per_row = G32 ? Gall * 2 : Gall / a.gs_blocks;
-    const int64_t words_per_row = (int64_t)K / 8;
+    const int64_t words_per_row = (int64_t)K * BITS / 32;
     // a pointer picked or computed per workgroup, back on the scalar unit
     auto uniform = [](auto* p) {
         const uint64_t u = reinterpret_cast<uint64_t>(p);
@@ -339,12 +368,17 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     const uint32_t mask_s = opaque_s(kMaskH);
     const uint32_t magic_v = opaque_v(kMagicH);
     // the first blocks are on their way while the prologue scans the scale rows
+    if constexpr (!B8)
 #pragma unroll
-    for (int c = 0; c < NBC; c++) issue_b(c, gb / QB, 0);
+        for (int c = 0; c < NBC; c++) issue_b(c, gb / QB, 0);
 #pragma unroll
-    for (int d = 0; d < AHEAD; d++)
+    for (int d = 0; d < AHEAD; d++) {
 #pragma unroll
         for (int c = 0; c < NA; c++) issue_a1(c, gb + d < G ? gb + d : G - 1, d);
+        if constexpr (B8)
+#pragma unroll
+            for (int c = 0; c < NBC; c++) issue_b(c, gb + d < G ? gb + d : G - 1, d);
+    }
 
     // this lane's weight rows (one per column block), and the power of two that brings the row's largest scale (of this
     // workgroup's range of K) into [2^10, 2^11): lane half h scans its half of the row's scales
@@ -355,6 +389,10 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         const uint16_t* const sbase = nb ? sb2[0] : sb1[0];
         const int n = weight_row(wave_n, nb, j);
         sboff[nb] = (uint32_t)n * (uint32_t)sb_per_row;
+        if constexpr (B8) {  // the scales stay fp32
+            col_up[nb] = 1.0f;
+            continue;
+        }
         const uint16_t* srow = sbase + sboff[nb];
         uint32_t mag = 0;
         const int first = G32 ? gb * 2 : gb / a.gs_blocks, last = G32 ? G * 2 : (G + a.gs_blocks - 1) / a.gs_blocks;
@@ -452,7 +490,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
 #pragma unroll
             for (int q = 0; q < 4; q++) {
                 if (q <= Q) {
-                    const uint32_t eight = __float_as_uint(__uint_as_float(quad_hi(s_cur[nb], q)) * (8.0f * col_up[nb])) >> 16;
+                    const uint32_t eight = __float_as_uint(__uint_as_float(quad_hi(s_cur[nb], q)) * (CENTRE * col_up[nb])) >> 16;
                     const uint32_t bia = __float_as_uint(__uint_as_float(quad_hi(b_cur[nb], q)) * col_up[nb]) >> 16;
                     v[q] = dup16(!G32 && h ? eight : bia);
                     ve[q] = dup16(eight);
@@ -512,35 +550,65 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         const int g2 = g + AHEAD < G ? g + AHEAD : glast;
         const int st2 = sa == 0 ? STAGES - 1 : sa - 1;  // stage (sa + AHEAD) % STAGES: read last in iteration g-1
         // B's next stage into the buffer that was read last in the stage before this one (past the end of K: the last again)
-        constexpr int NBQ = (Q & 1) == 0 ? NBC : 0, bcur = Q >> 1;
-        const int bst = min(g / QB + 1, (Gall - 1) / QB);
+        constexpr int NBQ = B8 || (Q & 1) == 0 ? NBC : 0;
+        const int bcur = B8 ? sa : Q >> 1, bnxt = B8 ? st2 : (Q >> 1) ^ 1;
+        const int bst = B8 ? g2 : min(g / QB + 1, (Gall - 1) / QB);
         auto issue_some = [&](int from, int to) {  // A's copies first, then B's
 #pragma unroll
             for (int c = from; c < to; c++) {
                 if (c < NA)
                     issue_a1(c, g2, st2);
                 else
-                    issue_b(c - NA, bst, bcur ^ 1);
+                    issue_b(c - NA, bst, bnxt);
             }
         };
         if constexpr (!SPREAD && !LATE) issue_some(0, NA + NBQ);
         const uint8_t* ab = abuf + sa * A_STAGE + (wave_m * MB) * 4096 + lane * 16;
-        // this lane's codes: row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3
-        const uint8_t* bb = bbuf + bcur * B_STAGE + ((wave_n * NB) * 32 + j) * B_ROW + (((Q % QB * 2 + h) ^ turn(j)) * 16);
+        const uint8_t* const brow = bbuf + bcur * B_STAGE + ((wave_n * NB) * 32 + j) * B_ROW;
         f16x8_t bfrag[NB][4];
+        [[maybe_unused]] float scale[NB][G32 ? 2 : 1];  // BITS 8: of the block's groups
+        if constexpr (B8) {
+            // row (wave_n * NB + nb) * 32 + j, eight codes from 16 t + 8 h on for step t
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) {
-            const uint4 cw = *reinterpret_cast<const uint4*>(bb + nb * 32 * B_ROW);
-            // the block's scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
-            const float sv = __uint_as_float(quad_hi(s_cur[nb], Q)) * col_up[nb];
-            const f16x2_t s2 = {(_Float16)sv, (_Float16)sv};
-            const float mv = sv * -24.0f;
-            const f16x2_t m24 = {(_Float16)mv, (_Float16)mv};
-            bfrag[nb][0] = __builtin_bit_cast(f16x8_t, expand_word(cw.x, mask_s, magic_v, s2, m24));
-            bfrag[nb][1] = __builtin_bit_cast(f16x8_t, expand_word(cw.y, mask_s, magic_v, s2, m24));
-            bfrag[nb][2] = __builtin_bit_cast(f16x8_t, expand_word(cw.z, mask_s, magic_v, s2, m24));
-            bfrag[nb][3] = __builtin_bit_cast(f16x8_t, expand_word(cw.w, mask_s, magic_v, s2, m24));
+            for (int nb = 0; nb < NB; nb++) {
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+                    bfrag[nb][t] = expand_bytes(*reinterpret_cast<const uint2*>(brow + nb * 32 * B_ROW + ((t ^ turn(j)) * 16) + h * 8));
+                const uint32_t sv = quad_hi(s_cur[nb], Q);
+                if constexpr (G32) {  // the lane halves hold the two groups' scales
+                    const auto both = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
+                    scale[nb][0] = __uint_as_float(both[0]);
+                    scale[nb][1] = __uint_as_float(both[1]);
+                } else {
+                    scale[nb][0] = __uint_as_float(sv);
+                }
+            }
+        } else {
+            // this lane's codes: row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3
+            const uint8_t* bb = brow + (((Q % QB * 2 + h) ^ turn(j)) * 16);
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) {
+                const uint4 cw = *reinterpret_cast<const uint4*>(bb + nb * 32 * B_ROW);
+                // the block's scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
+                const float sv = __uint_as_float(quad_hi(s_cur[nb], Q)) * col_up[nb];
+                const f16x2_t s2 = {(_Float16)sv, (_Float16)sv};
+                const float mv = sv * -24.0f;
+                const f16x2_t m24 = {(_Float16)mv, (_Float16)mv};
+                bfrag[nb][0] = __builtin_bit_cast(f16x8_t, expand_word(cw.x, mask_s, magic_v, s2, m24));
+                bfrag[nb][1] = __builtin_bit_cast(f16x8_t, expand_word(cw.y, mask_s, magic_v, s2, m24));
+                bfrag[nb][2] = __builtin_bit_cast(f16x8_t, expand_word(cw.z, mask_s, magic_v, s2, m24));
+                bfrag[nb][3] = __builtin_bit_cast(f16x8_t, expand_word(cw.w, mask_s, magic_v, s2, m24));
+            }
         }
+        constexpr int GROUPS = G32 ? 2 : 1;  // of a block
+        [[maybe_unused]] f32x16_t part[2][NB];
+        [[maybe_unused]] auto scale_part = [&](int u) {
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                for (int r = 0; r < 16; r++)
+                    out[u / GROUPS][nb][r] = __builtin_fmaf(scale[nb][u % GROUPS], part[u & 1][nb][r], out[u / GROUPS][nb][r]);
+        };
         // the A fragments of row block mb+1 are read while row block mb is multiplied
         f16x8_t afrag[2][4];
 #pragma unroll
@@ -554,11 +622,28 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
                 __builtin_amdgcn_sched_barrier(0);  // or the scheduler sinks the reads back to their first use
             }
             if constexpr (SPREAD && !LATE) issue_some(mb * (NA + NBQ) / MB, (mb + 1) * (NA + NBQ) / MB);
+            if constexpr (B8) {
+                // a group's sums are scaled while the matrix cores work on the next group's
 #pragma unroll
-            for (int t = 0; t < 4; t++)
+                for (int grp = 0; grp < GROUPS; grp++) {
+                    constexpr int STEPS = 4 / GROUPS;
+                    const int u = mb * GROUPS + grp;
 #pragma unroll
-                for (int nb = 0; nb < NB; nb++)
-                    out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag[mb & 1][t], bfrag[nb][t], out[mb][nb], 0, 0, 0);
+                    for (int t = 0; t < STEPS; t++)
+#pragma unroll
+                        for (int nb = 0; nb < NB; nb++)
+                            part[u & 1][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag[mb & 1][grp * STEPS + t], bfrag[nb][grp * STEPS + t],
+                                                                                     t ? part[u & 1][nb] : f32x16_t{}, 0, 0, 0);
+                    if (u > 0) scale_part(u - 1);
+                }
+                if (mb == MB - 1) scale_part(MB * GROUPS - 1);
+            } else {
+#pragma unroll
+                for (int t = 0; t < 4; t++)
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++)
+                        out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag[mb & 1][t], bfrag[nb][t], out[mb][nb], 0, 0, 0);
+            }
         }
         if constexpr (LATE) {
             __builtin_amdgcn_sched_barrier(0);
@@ -591,7 +676,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
 #pragma unroll
     for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(s_nxt[nb].x), "+v"(s_nxt[nb].y));
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * NA) : "memory");  // block 0 has landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * (B8 ? NA + NBC : NA)) : "memory");  // block 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     for (int g = gb; g < G; g += 4) {
@@ -613,7 +698,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     constexpr int CW = NB * 32;  // columns of the wavefront's tile
-    static_assert(NWAVE * 32 * CW * 4 <= STAGES * A_STAGE + 2 * B_STAGE, "staging area fits the stages");
+    static_assert(NWAVE * 32 * CW * 4 <= STAGES * A_STAGE + B_BUFS * B_STAGE, "staging area fits the stages");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * CW);
     const int stride = partial && pair ? 2 * N : N;
     void* const ybase = partial ? static_cast<void*>(partial + (int64_t)split * a.M * stride) : a.seg[seg].y;
@@ -755,27 +840,37 @@ struct QmmHalfEntry {
     int lds_bytes;
 };
 
-#define AQ_QMMH(MB, NB, WM, WN, ST, OCC, SPREAD, SUFFIX)                                               \
-    {                                                                                                 \
-        {"qmmh_b4_mb" #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, 4, MB, NB, WM, WN},                   \
-            qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 64>, qmmh_kernel<MB, NB, WM, WN, ST, OCC, SPREAD, 32>, \
-            ST*(WM * MB * 4096) + 2 * (WN * NB * 32 * 64)                                               \
+#define AQ_QMMH(PREFIX, BITS, MB, NB, WM, WN, ST, OCC, SPREAD, SUFFIX)                                                        \
+    {                                                                                                                        \
+        {PREFIX #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, BITS, MB, NB, WM, WN},                                             \
+            qmmh_kernel<BITS, MB, NB, WM, WN, ST, OCC, SPREAD, 64>, qmmh_kernel<BITS, MB, NB, WM, WN, ST, OCC, SPREAD, 32>,  \
+            ST*(WM * MB * 4096) + (BITS == 8 ? ST : 2) * (WN * NB * 32 * 64)                                                  \
     }
+#define AQ_QMMH4(...) AQ_QMMH("qmmh_b4_mb", 4, __VA_ARGS__)
+#define AQ_QMMH8(...) AQ_QMMH("qmmh8_b8_mb", 8, __VA_ARGS__)
 
 static const QmmHalfEntry kQmmHalfTable[] = {
-    AQ_QMMH(4, 2, 2, 2, 2, 2, true, "_s2c"),  // 256 x 128, four wavefronts, two stages (every LDS address a constant)
-    AQ_QMMH(4, 2, 2, 4, 3, 2, false, ""),     // 256 x 256, eight wavefronts, three stages (120 KiB): an A tile feeds twice the MFMAs
-    AQ_QMMH(3, 2, 2, 4, 3, 2, false, ""),     // 192 x 256: a round of these takes 0.82 of a round of those; for row counts
+    AQ_QMMH4(4, 2, 2, 2, 2, 2, true, "_s2c"),  // 256 x 128, four wavefronts, two stages (every LDS address a constant)
+    AQ_QMMH4(4, 2, 2, 4, 3, 2, false, ""),     // 256 x 256, eight wavefronts, three stages (120 KiB): an A tile feeds twice the MFMAs
+    AQ_QMMH4(3, 2, 2, 4, 3, 2, false, ""),     // 192 x 256: a round of these takes 0.82 of a round of those; for row counts
                                               // that fill their rounds better (1536 rows: 8 bands instead of 6 of 256)
-    AQ_QMMH(2, 2, 2, 2, 3, 2, false, ""),     // 128 x 128
-    AQ_QMMH(2, 2, 1, 4, 3, 2, false, ""),     // 64 x 256
-    AQ_QMMH(1, 2, 1, 4, 3, 2, false, ""),     // 32 x 256
+    AQ_QMMH4(2, 2, 2, 2, 3, 2, false, ""),     // 128 x 128
+    AQ_QMMH4(2, 2, 1, 4, 3, 2, false, ""),     // 64 x 256
+    AQ_QMMH4(1, 2, 1, 4, 3, 2, false, ""),     // 32 x 256
+    // 8-bit codes (a wavefront's partial sums take 64 registers: 96 or 128 rows a wavefront would spill)
+    AQ_QMMH8(2, 2, 2, 2, 3, 2, false, ""),
+    AQ_QMMH8(2, 2, 2, 4, 3, 2, false, ""),     // 128 x 256, eight wavefronts
+    AQ_QMMH8(2, 2, 1, 4, 3, 2, false, ""),
+    AQ_QMMH8(1, 2, 1, 4, 3, 2, false, ""),
 };
 
 int qmmh_variant_count() { return (int)(sizeof(kQmmHalfTable) / sizeof(kQmmHalfTable[0])); }
 const QmmVariant* qmmh_variant(int idx) {
     if (idx < 0 || idx >= qmmh_variant_count()) return nullptr;
     return &kQmmHalfTable[idx].v;
+}
+int qmmh_x_kind(int bits, int group_size) {
+    return bits == 8 ? (group_size == 32 ? kXReadyHalf8G32 : kXReadyHalf8) : (group_size == 32 ? kXReadyHalf32 : kXReadyHalf);
 }
 int qmmh_rows(int idx) { return kQmmHalfTable[idx].v.wm * kQmmHalfTable[idx].v.mb * 32; }
 size_t qmmh_partial_bytes(const QmmHalfCall& q) {
@@ -791,7 +886,8 @@ size_t qmmh_partial_bytes(const QmmHalfCall& q) {
 struct QmmHalfCost {
     double solo, full, fixed;
 };
-static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0}};
+static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0},
+                                           {1.02, 0.72, 5.0}, {1.25, 1.35, 6.0}, {1.01, 0.74, 5.0}, {0.78, 0.51, 4.0}};
 
 // Microseconds of kernel i over `tiles` tiles of `blocks` blocks each.
 static double half_cost(int i, int64_t tiles, int blocks, int cus) {
@@ -805,13 +901,14 @@ static int64_t half_strips(int i, int N, bool pair) {
 }
 static int64_t half_bands(int i, int M) { return (M + qmmh_rows(i) - 1) / qmmh_rows(i); }
 
-void qmmh_split(int M, int K, QmmSegment* seg, int cu_count) {
+void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count) {
     const int cus = cu_count > 0 ? cu_count : 256;
     const int G = K / 64;
     double best_us = 1e30;
     seg->ksplit = 1;
     seg->gsplit = (G + 3) / 4 * 4;
     for (int i = 0; i < qmmh_variant_count(); i++) {
+        if (kQmmHalfTable[i].v.bits != bits) continue;
         const int64_t tiles = half_bands(i, M) * half_strips(i, seg->N, false);
         for (int ks = 1; ks <= 16; ks++) {
             const int gsplit = ((G + ks - 1) / ks + 3) / 4 * 4;
@@ -829,6 +926,7 @@ int qmmh_pick(const QmmHalfCall& q, int cu_count) {
     int best = -1;
     double best_us = 1e30;
     for (int i = 0; i < qmmh_variant_count(); i++) {
+        if (kQmmHalfTable[i].v.bits != q.bits) continue;
         int64_t tiles = 0;
         int blocks = 0;
         for (int k = 0; k < (q.pair ? 1 : q.nseg); k++) {
@@ -847,6 +945,7 @@ int qmmh_pick(const QmmHalfCall& q, int cu_count) {
 hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream) {
     if (idx < 0 || idx >= qmmh_variant_count() || q.nseg < 1 || q.nseg > kQmmSegments || (q.pair && q.nseg != 2)) return hipErrorInvalidValue;
     const QmmHalfEntry& e = kQmmHalfTable[idx];
+    if (e.v.bits != q.bits) return hipErrorInvalidValue;
     const bool g32 = q.group_size == 32;
     const int rows = q.chunks ? q.most_rows : q.M;  // rows of the fragments
     const int mblks = (rows + 31) / 32;
@@ -855,10 +954,13 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     uint16_t* xs = xf + (size_t)mblks * 32 * q.K;
     float* rs = reinterpret_cast<float*>(xs + (size_t)mblks * 32 * g4 * (g32 ? 16 : 8));
     hipError_t rc = hipSuccess;
-    if (q.x_ready != (g32 ? kXReadyHalf32 : kXReadyHalf)) {
+    if (q.x_ready != qmmh_x_kind(q.bits, q.group_size)) {
         // one row a workgroup while eight would leave CUs idle
         const bool narrow = mblks * 4 < 128;
-        auto* const fn = narrow ? (g32 ? qmmh_prep_kernel<1, 32> : qmmh_prep_kernel<1, 64>) : (g32 ? qmmh_prep_kernel<8, 32> : qmmh_prep_kernel<8, 64>);
+        typedef void (*PrepKernel)(const uint16_t*, uint16_t*, uint16_t*, float*, int, int, const int32_t*, const int32_t*);
+        static const PrepKernel kPrep[2][2][2] = {{{qmmh_prep_kernel<8, 64, 4>, qmmh_prep_kernel<8, 64, 8>}, {qmmh_prep_kernel<8, 32, 4>, qmmh_prep_kernel<8, 32, 8>}},
+                                                  {{qmmh_prep_kernel<1, 64, 4>, qmmh_prep_kernel<1, 64, 8>}, {qmmh_prep_kernel<1, 32, 4>, qmmh_prep_kernel<1, 32, 8>}}};
+        const PrepKernel fn = kPrep[narrow][g32][q.bits == 8];
         hipLaunchKernelGGL(fn, dim3((unsigned)(narrow ? mblks * 32 : mblks * 4)), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows,
                            q.K, q.route_x, q.live_rows);
         rc = hipGetLastError();
@@ -909,7 +1011,7 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
         int64_t least = INT64_MAX;
         a.group_m = 1;
         for (int gm = 1; gm <= a.tiles_m && gm <= at_once && !q.chunks; gm++) {
-            const int64_t cost = (int64_t)gm * bm * 32 + (int64_t)((at_once + gm - 1) / gm) * bn * 9;  // in 1/16 bytes: fp16 rows, 4.5-bit columns
+            const int64_t cost = (int64_t)gm * bm * 32 + (int64_t)((at_once + gm - 1) / gm) * bn * (2 * q.bits + 1);  // in 1/16 bytes: fp16 rows, 4.5- or 8.5-bit columns
             if (cost < least) least = cost, a.group_m = gm;
         }
     }

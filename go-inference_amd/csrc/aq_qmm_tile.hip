@@ -533,7 +533,7 @@ hipError_t qmmt_launch(int idx, const QmmArgs& q, void* workspace, hipStream_t s
 int qmmt_x_kind(int idx) {
     const QmmVariant* v = qmmt_variant(idx);
     if (!v) return kXReadyNone;
-    if (idx >= tile_variants() && idx < tile_variants() + qmmh_variant_count()) return kXReadyHalf;
+    if (idx >= tile_variants() && idx < tile_variants() + qmmh_variant_count()) return qmmh_x_kind(v->bits, 64);
     return v->bits == 4 ? kXReadyTile4 : kXReadyTile8;
 }
 
@@ -553,6 +553,7 @@ hipError_t qmmt_launch_splitk(int idx, const QmmArgs& q, void* workspace, int ks
         c.M = q.M;
         c.K = q.K;
         c.group_size = q.gs_blocks * 64;
+        c.bits = qmmt_variant(idx)->bits;
         c.seg[0] = {q.w, q.s, q.b, q.y, q.N, 1, 0, 0, 0, nullptr};
         c.nseg = 1;
         c.out_f32 = q.out_f32;
