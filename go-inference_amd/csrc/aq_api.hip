@@ -976,7 +976,10 @@ namespace {
 //   4096           1306 / 272 / 160 / 159        1695 / 328 /  94 /  95
 // The per-route kernels stop paying at about two and a half routes per expert that is named at all, where their fast form
 // takes the shape, and at about one where it does not (K = 704 here); few routes per expert go to the token tiles while K
-// gives their eight wavefronts a run each, everything else to the matmul tiles whose rows an expert's routes fill.
+// gives their eight wavefronts a run each, everything else to matmul tiles.  Their rows (a whole block with router and combine,
+// us on tiles of 32 / 64 / 128 rows): 32 routes per expert (128 experts, 2816 / 704) 272 / 280 / 392, 64 (32 experts, 2048 /
+// 704) 95 / 105 / 108, 256 (16 experts) 144 / 135 / 140; 8 bit, 32 per expert: 340 / 313 (64 x 128) / 394: small tiles win
+// until an expert's routes fill several, since more workgroups are resident and hide each other's waits.
 int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair) {
     if (a.routes <= 64 || ctx->forced[0] >= 0 || ctx->forced[1] >= 0 || a.num_experts > aq::kGroupMaxExperts) return kPass;
     a.gs_shift = is_pow2(group_size) ? ilog2(group_size) : 0;
@@ -989,7 +992,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     const bool tok_fits = aq::qmvt_grouped_fits(a, bits, group_size, pair) && !(ctx->families_off >> kFamTok & 1);
     if (!tiles_fit && !tok_fits) return kPass;
     const bool tiles = tiles_fit && !(tok_fits && per_expert <= 12 && a.K >= 2048);
-    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= 32 ? 32 : per_expert <= 96 ? 64 : per_expert <= 384 || bits == 8 ? 128 : 256;
+    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= (bits == 4 ? 96 : 16) ? 32 : per_expert <= 384 ? 64 : bits == 8 ? 128 : 256;
     const int pad = tiles ? 32 : 1;
     const int most_chunks = a.routes / chunk + groups;
     const int most_rows = a.routes + groups * (pad - 1);
@@ -1050,8 +1053,11 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     q.expert_rows = a.expert_rows;
     q.row_base = a.row_base;
     q.row_base2 = a.row_base2;
+    const int wn = chunk == 128 || (chunk == 64 && bits == 8) ? 2 : 4;  // 128 columns, or 256
     int idx = 0;
-    while (idx < aq::qmmh_variant_count() && !(aq::qmmh_variant(idx)->bits == bits && aq::qmmh_rows(idx) == chunk && (chunk != 256 || aq::qmmh_variant(idx)->wn == 4))) idx++;
+    while (idx < aq::qmmh_variant_count() &&
+           !(aq::qmmh_variant(idx)->bits == bits && aq::qmmh_rows(idx) == chunk && aq::qmmh_variant(idx)->wn == wn))
+        idx++;
     if (idx >= aq::qmmh_variant_count()) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv: no tiles of %d rows", chunk);
     const char* name = nullptr;
     const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, idx, q, &name, fail, nullptr);
