@@ -225,8 +225,8 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
 // sorts its kTopKPerLane values in registers; then, top_k times, the wavefront takes the largest of the 64
 // list heads (high words first, then the low words of the lanes that hold that high word) and the winning
 // lane drops its head.  Entries past `count` read as 0, which is also the "no candidate" value.
-__device__ __forceinline__ void topk_reduce_segment(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                    unsigned long long* __restrict__ out, int64_t segment, int lane) {
+__device__ __forceinline__ void topk_reduce_segment(const unsigned long long* in, int64_t count, int top_k, unsigned long long* out,
+                                                    int64_t segment, int lane) {
     constexpr int V = kTopKPerLane;
     const int64_t begin = segment * kTopKSegment;
     if (begin >= count) return;  // whole wavefronts
@@ -272,11 +272,9 @@ __device__ __forceinline__ void topk_reduce_segment(const unsigned long long* __
     if (lane < top_k) out[segment * top_k + lane] = mine;
 }
 
-// A round of the segment-by-segment reduction.  With `gate` set the round only runs when the candidate list of
-// the threshold path below has overflowed (*gate > kTopKCandidates); otherwise it leaves at once.
+// A round of the segment-by-segment reduction.
 __global__ __launch_bounds__(256) void packed_topk_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                          unsigned long long* __restrict__ out, const uint32_t* gate) {
-    if (gate && *gate <= (uint32_t)kTopKCandidates) return;
+                                                          unsigned long long* __restrict__ out) {
     topk_reduce_segment(in, count, top_k, out, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & (kWave - 1));
 }
 
@@ -285,7 +283,8 @@ __global__ __launch_bounds__(256) void packed_topk_kernel(const unsigned long lo
 // >= T; for scores that are not arranged by rank that set is a little over top_k entries, and one workgroup
 // orders it by counting.  Three launches: maxima, filter, finish.  When more than kTopKCandidates entries
 // reach T (long runs of equal scores, an input sorted by score) the finish launch runs the first round of the
-// segment-by-segment reduction instead and the gated rounds after it complete the answer.
+// segment-by-segment reduction instead, and the workgroup that ends it last the rounds that are left (as launches of their
+// own, which left at once where there was nothing to do, those rounds took 1.6 us each of every call).
 // A wavefront of these two kernels takes a piece of 64 * V entries: V is the largest of 16, 4, 1 that leaves at
 // least top_k pieces.
 template <int V>
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(256) void topk_segment_max_kernel(const unsigned lo
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t segment = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int64_t begin = segment * (kWave * V);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0;
+    if (blockIdx.x == 0 && threadIdx.x < 2) counter[threadIdx.x] = 0;  // candidates; workgroups past the first round
     if (begin >= count) return;
     unsigned long long m = 0;
 #pragma unroll
@@ -377,14 +376,33 @@ __global__ __launch_bounds__(256) void topk_filter_kernel(const unsigned long lo
 // The candidates are distinct unless the input repeats a value, so an entry's place in the output is the number
 // of candidates above it (equal values take consecutive places in list order).
 __global__ __launch_bounds__(256) void topk_finish_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                          const uint32_t* counter, const unsigned long long* __restrict__ cand,
-                                                          unsigned long long* __restrict__ out,
-                                                          unsigned long long* __restrict__ round_out) {
+                                                          uint32_t* counter, const unsigned long long* __restrict__ cand,
+                                                          unsigned long long* __restrict__ out, unsigned long long* round1,
+                                                          unsigned long long* round2) {
     const uint32_t n = *counter;
     if (n > (uint32_t)kTopKCandidates) {
-        topk_reduce_segment(in, count, top_k, round_out, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6),
-                            threadIdx.x & (kWave - 1));
-        return;
+        const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+        topk_reduce_segment(in, count, top_k, round1, (int64_t)blockIdx.x * 4 + wave, lane);
+        __shared__ uint32_t arrived;
+        __threadfence();  // this workgroup's share of round1 is visible before its ticket is
+        __syncthreads();
+        if (threadIdx.x == 0) arrived = atomicAdd(counter + 1, 1u);
+        __syncthreads();
+        if (arrived + 1 != gridDim.x) return;
+        __threadfence();
+        unsigned long long *from = round1, *to = round2;
+        int64_t left = (count + kTopKSegment - 1) / kTopKSegment * top_k;
+        while (true) {
+            const int64_t segments = (left + kTopKSegment - 1) / kTopKSegment;
+            unsigned long long* const dst = segments == 1 ? out : to;
+            for (int64_t s = wave; s < segments; s += 4) topk_reduce_segment(from, left, top_k, dst, s, lane);
+            if (segments == 1) return;
+            __threadfence_block();
+            __syncthreads();
+            to = from;
+            from = dst;
+            left = segments * top_k;
+        }
     }
     if (blockIdx.x != 0) return;
     constexpr int PER = kTopKCandidates / 256;
@@ -428,7 +446,7 @@ static int topk_threshold_per_lane(int64_t count, int top_k) {
     return 0;
 }
 
-constexpr int kTopKHeader = 2;  // scratch[0]: candidate counter (its low word)
+constexpr int kTopKHeader = 2;  // scratch[0]: candidate counter, workgroups past the first round
 
 size_t packed_topk_scratch_entries(int64_t count, int top_k) {
     if (count <= kTopKSegment) return 0;
@@ -455,7 +473,6 @@ hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int t
     const int64_t first = topk_segments(count);
     const int64_t c1 = first * top_k;
     unsigned long long* bufs[2] = {scratch, scratch + c1};
-    const uint32_t* gate = nullptr;
     int which = 0;
     const unsigned long long* src = in;
     int64_t n = count;
@@ -469,19 +486,13 @@ hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int t
         else if (per_lane == 4) topk_threshold_launch<4>(in, count, top_k, segmax, counter, cand, stream);
         else topk_threshold_launch<1>(in, count, top_k, segmax, counter, cand, stream);
         hipLaunchKernelGGL(topk_finish_kernel, dim3((unsigned)((first + 3) / 4)), dim3(256), 0, stream, in, count, top_k, counter,
-                           cand, out, bufs[0]);
-        hipError_t rc = hipGetLastError();
-        if (rc != hipSuccess) return rc;
-        gate = counter;
-        src = bufs[0];
-        n = c1;
-        which = 1;
+                           cand, out, bufs[0], bufs[1]);
+        return hipGetLastError();
     }
     while (true) {
         const int64_t segments = topk_segments(n);
         unsigned long long* dst = segments == 1 ? out : bufs[which];
-        hipLaunchKernelGGL(packed_topk_kernel, dim3((unsigned)((segments + 3) / 4)), dim3(256), 0, stream, src, n, top_k, dst,
-                           gate);
+        hipLaunchKernelGGL(packed_topk_kernel, dim3((unsigned)((segments + 3) / 4)), dim3(256), 0, stream, src, n, top_k, dst);
         hipError_t rc = hipGetLastError();
         if (rc != hipSuccess || segments == 1) return rc;
         src = dst;
