@@ -857,13 +857,13 @@ static const QmmHalfEntry kQmmHalfTable[] = {
     AQ_QMMH4(2, 2, 2, 2, 3, 2, false, ""),     // 128 x 128
     AQ_QMMH4(2, 2, 1, 4, 3, 2, false, ""),     // 64 x 256
     AQ_QMMH4(1, 2, 1, 4, 3, 2, false, ""),     // 32 x 256
-    AQ_QMMH4(1, 2, 2, 2, 3, 2, false, ""),     // 64 x 128 (four workgroups a CU): long K on few tiles
     // 8-bit codes (a wavefront's partial sums take 64 registers: 96 or 128 rows a wavefront would spill)
-    AQ_QMMH8(2, 2, 2, 2, 3, 2, false, ""),
+    AQ_QMMH8(2, 2, 2, 2, 3, 2, true, ""),      // (copies spread: 343 -> 329 us on 2048 x 4096 x 14336)
     AQ_QMMH8(2, 2, 2, 4, 3, 2, false, ""),     // 128 x 256, eight wavefronts
     AQ_QMMH8(2, 2, 1, 4, 3, 2, false, ""),
     AQ_QMMH8(1, 2, 1, 4, 3, 2, false, ""),
-    AQ_QMMH8(1, 2, 2, 2, 3, 2, false, ""),     // 64 x 128
+    AQ_QMMH8(1, 2, 2, 2, 3, 2, false, ""),     // 64 x 128 (4-bit tiles of that size, unsplit 167 -> 152 us on 509 x 15360 x 3840, lost to
+                                               // 128 x 128 and 192 x 256 with shares of K: 117 -> 142)
 };
 
 int qmmh_variant_count() { return (int)(sizeof(kQmmHalfTable) / sizeof(kQmmHalfTable[0])); }
@@ -888,7 +888,7 @@ size_t qmmh_partial_bytes(const QmmHalfCall& q) {
 struct QmmHalfCost {
     double solo, full, fixed;
 };
-static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0}, {0.58, 0.39, 4.0},
+static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0},
                                            {1.02, 0.72, 5.0}, {1.25, 1.35, 6.0}, {1.01, 0.74, 5.0}, {0.78, 0.51, 4.0}, {0.66, 0.41, 4.0}};
 
 // Microseconds of kernel i over `tiles` tiles of `blocks` blocks each.
