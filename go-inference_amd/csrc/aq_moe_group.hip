@@ -8,7 +8,8 @@
 // entries as the ids ask for; the launches behind it are sized for the most there can be and read the count here.
 //
 // Bound: latency.  Two passes over 4 bytes a route with LDS counters and one scan over the experts, one workgroup because
-// the passes depend on each other through the counters (4096 routes: 6 us; a grid-wide meeting costs more than that).
+// the passes depend on each other through the counters (4096 routes over 128 experts: 11 us in a kernel trace; a grid-wide
+// meeting costs more than that).
 #include "aq_device.h"
 #include "aq_kernels.h"
 

@@ -229,9 +229,9 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
 // tile kernels of aq_qmm_tile.hip.  Against those: two vector instructions per pair of codes instead of three, several
 // matrices in one grid, the gated pair, groups of 32 and expert slabs.  A step of the MFMA is 16 consecutive codes, so that
 // groups of 32 are two steps each; bytes are staged one 64-code block at a time, in as many stages as A.
-// Measured (us; bf16-code tiles -> here): 2048 x 4096 x 14336 395 -> 341, a layer of 777 rows (2560 / 10240) 461 -> 375, of 400
-// rows (1472 / 4032) 274 -> 130, of 300 rows in groups of 32 (2048 / 8192) 24.9 ms on the any-width kernel -> 174, 512 tokens
-// through 128 experts (2816 / 704) 3749 -> 338.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
+// Measured (us; bf16-code tiles -> here): 2048 x 4096 x 14336 395 -> 329, a layer of 777 rows (2560 / 10240) 453 -> 358, of 400
+// rows (1472 / 4032) 274 -> 125, of 300 rows in groups of 32 (2048 / 8192) 24.7 ms on the any-width kernel -> 159, 512 tokens
+// through 128 experts (2816 / 704) 3692 -> 314.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
 // instructions of expansion and 64 of scaling; a block takes 0.72 us of a CU for 0.23 us of matrix pipe.
 template <int BITS, int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
 __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfArgs a) {
