@@ -809,8 +809,8 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             }
         }
     }
-    if (!tiled && count > 1 && M > 1 && K > 0 && (bits == 4 || bits == 8) && check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK) {
-        // several rows: the token-tile kernels over all matrices in one grid
+    if (x && !tiled && count > 1 && M > 1 && K > 0 && (bits == 4 || bits == 8) && check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK) {
+        // several rows: the token-tile kernels over all matrices in one grid (aq_qmv names what is wrong with a call)
         int64_t total = 0;
         for (int i = 0; i < count; i++) total += N[i];
         std::lock_guard<std::mutex> lk(ctx->mu);

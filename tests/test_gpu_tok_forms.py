@@ -70,3 +70,19 @@ def test_gated_pair(ctx, orc, bits, gs, M, K, N):
         assert (np.abs(got - want) <= 4e-6 * np.abs(want) + 2.5e-7 * np.maximum(1.0, np.abs(g * u))).all()
     for t in (dx, dy, dg, du):
         t.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K", [(4, 64, 9, 4096), (8, 64, 2, 4096), (4, 32, 3, 960), (4, 128, 32, 1024), (4, 64, 1, 4096), (4, 64, 48, 4096)])
+def test_several_matrices_without_x_are_refused(ctx, bits, gs, M, K):
+    import aq_mi355
+    say("token tile multi without x", bits, gs, M, K)
+    dws, ys = [], []
+    for n in (48, 16):
+        dws.append(DeviceAffine(ctx, *F.synthetic_affine(n, K, bits, gs, seed=2260)))
+        ys.append(ctx.alloc(M * n * 2))
+    with pytest.raises(aq_mi355.AqError) as e:
+        ctx.qmv_multi(None, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, [48, 16], M, K, gs, bits)
+    assert e.value.code == aq_mi355.AQ_ERR_ARG and "null operand" in str(e.value)
+    ctx.sync()
+    for t in ys + dws:
+        t.free()
