@@ -809,27 +809,46 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             }
         }
     }
-    if (x && !tiled && count > 1 && M > 1 && K > 0 && (bits == 4 || bits == 8) && check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK) {
-        // several rows: the token-tile kernels over all matrices in one grid (aq_qmv names what is wrong with a call)
-        int64_t total = 0;
-        for (int i = 0; i < count; i++) total += N[i];
+    // several rows: the token-tile kernels over all matrices in one grid (aq_qmv names what is wrong with a call).  A member
+    // belongs to it if its own call runs on them: the choice by the rows of all members together would move members across a
+    // line of the selection (40 Mi and 4 Mi codes), and so to sums in another order.  The others run first, one by one.
+    const bool tok = x && !tiled && count > 1 && M > 1 && K > 0 && (bits == 4 || bits == 8) &&
+                     check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK;
+    unsigned in_grid = 0;
+    int members = 0, ti = -1;
+    aq::QmvMultiArgs grid{};
+    if (tok) {
         std::lock_guard<std::mutex> lk(ctx->mu);
-        const int ti = total < (int64_t)1 << 30 && tok_runs(ctx, bits, group_size, M, K, total)
-                           ? aq::qmvt_pick(bits, M, K, (int)total, ctx->cu_count) : -1;
-        aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
-        bool fits = ti >= 0;
-        for (int i = 0; fits && i < count; i++) {
-            const aq::QmvArgs one = multi_member(ma, i);
-            fits = N[i] > 0 && aligned(y[i], 2) && aq::qmvt_fits(one, bits, group_size, ti, false);
+        const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
+        int64_t total = 0;
+        grid.common = all.common;
+        for (int i = 0; i < count; i++) {
+            if (N[i] == 0 || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i])) continue;
+            const int own = aq::qmvt_pick(bits, M, K, N[i], ctx->cu_count);
+            if (own < 0 || !aq::qmvt_fits(multi_member(all, i), bits, group_size, own, false)) continue;
+            in_grid |= 1u << i;
+            grid.w[members] = all.w[i];
+            grid.s[members] = all.s[i];
+            grid.b[members] = all.b[i];
+            grid.y[members] = all.y[i];
+            grid.N[members++] = N[i];
+            total += N[i];
         }
-        if (fits) {
-            ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
-            AQ_HIP(aq::qmvt_multi_launch(ti, ma, ctx->stream), "hipLaunchKernel");
-            return AQ_OK;
-        }
+        grid.count = members;
+        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, M, K, (int)total, ctx->cu_count) : -1;
+        for (int i = 0; ti >= 0 && i < members; i++)
+            if (!aq::qmvt_fits(multi_member(grid, i), bits, group_size, ti, false)) ti = -1;
+        if (ti < 0) in_grid = 0;
     }
-    for (int i = 0; i < count; i++)
+    for (int i = 0; i < count; i++) {
+        if (in_grid >> i & 1) continue;
         if (int rc = aq_qmv(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
+    }
+    if (in_grid) {
+        std::lock_guard<std::mutex> lk(ctx->mu);
+        ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
+        AQ_HIP(aq::qmvt_multi_launch(ti, grid, ctx->stream), "hipLaunchKernel");
+    }
     return AQ_OK;
 }
 

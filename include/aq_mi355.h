@@ -133,9 +133,8 @@ int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, c
  * narrow projections are bound by launch latency, not bandwidth, and one grid over all of them fills
  * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384), and for
  * the row counts the token-tile kernels run (9..32 rows of 4-bit group-64 codes, 3..32 of group 32, 5..32 of group 128,
- * 2..32 of 8-bit codes); other shapes are run as separate launches.  (Byte-identity has one exception: 9..32 rows in
- * groups of 64 with a K that is no multiple of 256, where a separate call on a matrix of under 4 Mi codes sums in another
- * order.) */
+ * 2..32 of 8-bit codes) over those members whose own call runs on them; other shapes and members are run as separate
+ * launches. */
 int aq_qmv_multi(aq_ctx *ctx, const void *x, int count, const void *const *packed, const void *const *scales,
                  const void *const *biases, void *const *y, const int *N, int M, int K, int group_size, int bits,
                  unsigned flags);

@@ -86,3 +86,24 @@ def test_several_matrices_without_x_are_refused(ctx, bits, gs, M, K):
     ctx.sync()
     for t in ys + dws:
         t.free()
+
+
+# the sum of the rows on one side of a line of the selection and every member on the other (40 Mi and 4 Mi codes), members on
+# both sides of it, and shapes without such a line
+@pytest.mark.parametrize("bits,gs,M,K,Ns", [(8, 64, 2, 4096, (4096, 4096, 4096)), (8, 64, 4, 8192, (2048, 3100, 512)), (8, 64, 2, 2112, (900, 1100, 400)),
+                                            (8, 64, 8, 4032, (520, 520, 600)), (4, 64, 12, 4032, (520, 520, 600)), (4, 64, 32, 2112, (2100, 300)),
+                                            (4, 64, 6, 4032, (520, 600)), (4, 32, 5, 3840, (130, 64, 1)), (8, 32, 2, 960, (40, 50)), (4, 128, 5, 1024, (256, 300)),
+                                            (8, 128, 3, 1024, (256, 300)), (4, 64, 16, 4096, (1000, 17))])
+def test_members_have_the_bytes_of_their_own_calls(ctx, bits, gs, M, K, Ns):
+    import aq_mi355
+    say("token tile multi, bytes", bits, gs, M, K, Ns)
+    x = F.synthetic_x(M, K, seed=2270)
+    dws = [DeviceAffine(ctx, *F.synthetic_affine(n, K, bits, gs, seed=2271 + i)) for i, n in enumerate(Ns)]
+    alone = [run_qmv(ctx, x, d, M, K, n, gs, bits, True) for d, n in zip(dws, Ns)]
+    dx, ys = ctx.to_device(x), [ctx.alloc(M * n * 4) for n in Ns]
+    ctx.qmv_multi(dx, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, list(Ns), M, K, gs, bits, aq_mi355.AQ_OUT_F32)
+    ctx.sync()
+    for n, y, one in zip(Ns, ys, alone):
+        assert np.array_equal(y.download(np.uint32, M * n), one.view(np.uint32).reshape(-1)), "member of %d rows" % n
+    for t in [dx] + ys + dws:
+        t.free()
