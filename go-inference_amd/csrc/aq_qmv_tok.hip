@@ -14,8 +14,10 @@ const QmvVariant* qmvt_variant(int idx) {
     return &tok_entry(idx).v;
 }
 
+// (of a gated pair: one form for both matrices, so the alignment of either decides it)
 static int tok_form(const QmvArgs& a) {
-    const uintptr_t al8 = reinterpret_cast<uintptr_t>(a.s) | reinterpret_cast<uintptr_t>(a.b);
+    const uintptr_t al8 = reinterpret_cast<uintptr_t>(a.s) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.s2) |
+                          reinterpret_cast<uintptr_t>(a.b2);
     if (a.gs_shift == 6 && a.K % 256 == 0 && (al8 & 7) == 0) return kTokExact;
     return a.gs_shift == 5 ? kTokG32 : kTokAny;
 }
@@ -88,10 +90,7 @@ bool qmvt_pair_supported(int idx) { return idx >= 0 && idx < qmvt_variant_count(
 hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream) {
     if (!qmvt_pair_supported(idx)) return hipErrorInvalidValue;
     const QmvTokEntry& e = tok_entry(idx);
-    QmvArgs up = a;
-    up.s = a.s2;
-    up.b = a.b2;
-    const int f1 = tok_form(a), f2 = tok_form(up), form = f1 > f2 ? f1 : f2;
+    const int form = tok_form(a);
     const QmvTokKernel fn = e.pair[form];
     const size_t lds = tok_lds_bytes(e, a.K, form);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;

@@ -107,3 +107,30 @@ def test_members_have_the_bytes_of_their_own_calls(ctx, bits, gs, M, K, Ns):
         assert np.array_equal(y.download(np.uint32, M * n), one.view(np.uint32).reshape(-1)), "member of %d rows" % n
     for t in [dx] + ys + dws:
         t.free()
+
+
+@pytest.mark.parametrize("off_gate,off_up,fused", [(0, 0, True), (8, 8, True), (8, 0, True), (8, 2, False), (2, 8, False), (4, 4, False)])
+def test_gated_pair_scales_of_any_alignment(ctx, orc, off_gate, off_up, fused):
+    """Scales and biases of the two matrices at their own byte offsets: the one launch asks the same of both, and the separate
+    projections run where either falls short of it."""
+    import aq_mi355
+    M, K, N, gs, bits = 12, 1024, 200, 64, 4
+    say("token tile gate|up, alignment", off_gate, off_up)
+    x = F.synthetic_x(M, K, seed=2350)
+    mats = [F.synthetic_affine(N, K, bits, gs, seed=2351 + i) for i in range(2)]
+    g, u = (F.reference_f64(x, *m, bits, gs, K) for m in mats)
+    held, args = [], []
+    for (words, s, b), off in zip(mats, (off_gate, off_up)):
+        sb = [ctx.to_device(np.concatenate([np.zeros(off // 2, np.uint16), np.ravel(t)])) for t in (s, b)]
+        held += [ctx.to_device(words)] + sb
+        args.append((held[-3], sb[0].ptr + off, sb[1].ptr + off))
+    dx, dy = ctx.to_device(x), ctx.alloc(M * N * 4)
+    ctx.qmv_gate_up(dx, args[0], args[1], dy, M, K, N, gs, bits, aq_mi355.AQ_ACT_SILU, aq_mi355.AQ_OUT_F32)
+    ctx.sync()
+    assert (ctx.last_variant(0) == "qmv_gate_up_tok") == fused, ctx.last_variant(0)
+    want = g / (1.0 + np.exp(-g)) * u
+    got = dy.download(np.float32, M * N).reshape(M, N)
+    # 1e-4: twice the fp32 sums' error over K = 1024 against float64 (1.2e-5 of the result's scale on the code-128 kernels)
+    assert (np.abs(got - want) <= 1e-4 * np.maximum(1.0, np.abs(g * u) + np.abs(g) + np.abs(u))).all()
+    for t in held + [dx, dy]:
+        t.free()
