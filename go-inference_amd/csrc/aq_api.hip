@@ -490,9 +490,9 @@ int aq_create(int device, aq_ctx** out) {
     if (rc == hipSuccess) rc = hipMemset(ctx->head_fold, 0, aq::kHeadFoldBytes);
     if (rc == hipSuccess) {
         // room for the argmax partials of a 1M-row vocabulary at two rows per wavefront
-        rc = hipMalloc(&ctx->head_ws.ptr, (size_t)4 << 20);
-        if (rc == hipSuccess) ctx->head_ws.bytes = (size_t)4 << 20;
+        rc = aq::workspace_open(&ctx->head_ws, (size_t)4 << 20);
     }
+    if (rc == hipSuccess) rc = aq::workspace_open(&ctx->ws, 0);
     if (rc != hipSuccess) {
         aq_destroy(ctx);
         return hip_fail(rc, "hipStreamCreate");
@@ -515,26 +515,37 @@ void aq_destroy(aq_ctx* ctx) {
         (void)hipStreamDestroy(ctx->own_stream);
     }
     delete ctx->host;
-    if (ctx->ws.ptr) (void)hipFree(ctx->ws.ptr);
-    if (ctx->head_ws.ptr) (void)hipFree(ctx->head_ws.ptr);
+    aq::workspace_close(&ctx->ws);
+    aq::workspace_close(&ctx->head_ws);
     if (ctx->head_fold) (void)hipFree(ctx->head_fold);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
     delete ctx;
 }
 
+namespace {
+// The context's scratch blocks stay in order across streams: what the stream that is left still does with them, the next
+// call that uses them on another stream waits for.
+int go_to_stream(aq_ctx* ctx, hipStream_t stream) {
+    const hipStream_t old = ctx->stream;
+    ctx->stream = stream;
+    if (stream == old) return AQ_OK;
+    const hipError_t rc = aq::workspace_leave(old, &ctx->ws), rc_head = aq::workspace_leave(old, &ctx->head_ws);
+    if (rc != hipSuccess || rc_head != hipSuccess) return hip_fail(rc != hipSuccess ? rc : rc_head, "hipEventRecord");
+    return AQ_OK;
+}
+}  // namespace
+
 int aq_use_stream(aq_ctx* ctx, void* hip_stream) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_use_stream: ctx is null");
     std::lock_guard<std::mutex> lk(ctx->mu);
-    ctx->stream = static_cast<hipStream_t>(hip_stream);
-    return AQ_OK;
+    return go_to_stream(ctx, static_cast<hipStream_t>(hip_stream));
 }
 
 int aq_use_own_stream(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_use_own_stream: ctx is null");
     std::lock_guard<std::mutex> lk(ctx->mu);
-    ctx->stream = ctx->own_stream;
-    return AQ_OK;
+    return go_to_stream(ctx, ctx->own_stream);
 }
 
 int aq_device_name(aq_ctx* ctx, char* buf, size_t buf_len) {
@@ -627,6 +638,8 @@ int aq_capture_begin(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_capture_begin: ctx is null");
     std::lock_guard<std::mutex> lk(ctx->mu);
     if (ctx->stream == nullptr) return fail(AQ_ERR_UNSUPPORTED, "aq_capture_begin: the legacy default stream cannot be captured");
+    AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->ws), "hipEventRecord");
+    AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->head_ws), "hipEventRecord");
     AQ_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     ctx->ws.touched = ctx->head_ws.touched = false;
     return AQ_OK;
@@ -666,6 +679,8 @@ int aq_graph_launch(aq_ctx* ctx, aq_graph* graph) {
                     "aq_graph_launch: the context's workspace was reallocated after this graph was captured (a later call "
                     "needed more room); the graph's kernels still point at the freed block: capture it again, and reserve "
                     "the largest workspace first (aq_reserve_workspace / aq_reserve_workspace_bytes)");
+    if (graph->uses_ws) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->ws), "hipStreamWaitEvent");
+    if (graph->uses_head_ws) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->head_ws), "hipStreamWaitEvent");
     AQ_HIP(hipGraphLaunch(graph->exec, ctx->stream), "hipGraphLaunch");
     return AQ_OK;
 }

@@ -4,6 +4,7 @@
 #include <stdint.h>
 
 #include "aq_kernels.h"
+#include "aq_workspace.h"
 
 namespace aq {
 
@@ -128,28 +129,7 @@ void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count);
 int qmmh_pick(const QmmHalfCall& q, int cu_count);
 size_t qmmh_partial_bytes(const QmmHalfCall& q);
 
-// Scratch memory a context lends to the matmul path; grown on demand, never while a capture is open.
-// `generation` counts reallocations: a captured graph has the block's address in its kernel arguments and is
-// only valid while the generation it was captured under stands.  `touched` is set by every reserve call, so
-// that the owner can tell whether a capture used the block.
-struct Workspace {
-    void* ptr = nullptr;
-    size_t bytes = 0;
-    uint64_t generation = 0;
-    bool touched = false;
-};
-
-// Whether ws holds `need` bytes or may be made to (not while the stream is being captured): for calls that have another
-// route that needs no scratch.
-bool workspace_may_grow(const Workspace* ws, size_t need, hipStream_t stream);
-
 hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream);
-
-typedef int (*FailFn)(int code, const char* fmt, ...);
-
-// Makes ws hold at least `need` bytes (drains the stream and reallocates when it must grow; refused
-// while the stream is being captured).
-int workspace_reserve(hipStream_t stream, Workspace* ws, size_t need, FailFn fail);
 
 // Upper bound (256-byte aligned) of the workspace bytes qmm_dispatch may use for an M x K by N call: the
 // rewritten activations and, for few rows, the fp32 partial tiles of the K split.  Callers that keep their

@@ -39,39 +39,6 @@ hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream) {
     return hipGetLastError();
 }
 
-// Makes ws hold at least `need` bytes.  Growing frees the old block, so everything queued on the stream
-// is drained first; a stream that is being captured cannot be drained.
-static int grow_workspace(Workspace* ws, size_t need, hipStream_t stream, FailFn fail) {
-    ws->touched = true;
-    if (ws->bytes >= need) return AQ_OK;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    if (stream != nullptr && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone)
-        return fail(AQ_ERR_UNSUPPORTED,
-                    "the context's workspace must grow to %zu bytes, which cannot happen during stream capture; "
-                    "run the call once, or call aq_reserve_workspace / aq_reserve_workspace_bytes, before capturing", need);
-    hipError_t rc = hipStreamSynchronize(stream);
-    if (rc != hipSuccess) return fail((int)rc, "rocm.hip.hipStreamSynchronize: HIP returned %d", (int)rc);
-    if (ws->ptr) (void)hipFree(ws->ptr);
-    ws->ptr = nullptr;
-    ws->bytes = 0;
-    ws->generation++;  // graphs captured over the old block must not run again
-    const size_t want = need + need / 4;  // headroom: prompts grow a little from call to call
-    rc = hipMalloc(&ws->ptr, want);
-    if (rc != hipSuccess) return fail(AQ_ERR_NOMEM, "aq_qmm: cannot allocate a %zu-byte workspace (HIP %d)", want, (int)rc);
-    ws->bytes = want;
-    return AQ_OK;
-}
-
-bool workspace_may_grow(const Workspace* ws, size_t need, hipStream_t stream) {
-    if (ws->bytes >= need) return true;
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    return !(stream != nullptr && hipStreamIsCapturing(stream, &cs) == hipSuccess && cs != hipStreamCaptureStatusNone);
-}
-
-int workspace_reserve(hipStream_t stream, Workspace* ws, size_t need, FailFn fail) {
-    return grow_workspace(ws, need, stream, fail);
-}
-
 size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
     const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;
     size_t partial = (M > 4 && M <= 64) ? qmmt_splitk_bytes(M, N, 16) : 0;
@@ -96,7 +63,7 @@ size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
 }
 
 int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, FailFn fail) {
-    return grow_workspace(ws, qmmt_workspace_bytes(M, K), stream, fail);
+    return workspace_reserve(stream, ws, qmmt_workspace_bytes(M, K), fail);
 }
 
 static int find_qmmt(int bits, int mb, int nb, int wm, int wn) {
@@ -138,7 +105,7 @@ int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCa
     const size_t need = xbytes + qmmh_partial_bytes(q);
     if (!workspace_may_grow(ws, need, stream)) return kQmmhNoScratch;
     const uint64_t generation = ws->generation;
-    if (int rc = grow_workspace(ws, need, stream, fail)) return rc;
+    if (int rc = workspace_reserve(stream, ws, need, fail)) return rc;
     // (a workspace that had to move no longer holds the earlier pass over x)
     q.x_ready = x_state && ws->generation == generation ? *x_state : kXReadyNone;
     if (idx < 0) idx = qmmh_pick(q, cu_count);
@@ -262,7 +229,7 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
     {
         const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;
         const uint64_t generation = ws->generation;
-        if (int rc = grow_workspace(ws, xbytes + qmmt_splitk_bytes(M, N, ksplit), stream, fail)) return rc;
+        if (int rc = workspace_reserve(stream, ws, xbytes + qmmt_splitk_bytes(M, N, ksplit), fail)) return rc;
         // (a workspace that had to move no longer holds the earlier pass over x)
         a.x_ready = x_state && ws->generation == generation ? *x_state : kXReadyNone;
         *last_variant = qmmt_variant(tile_idx)->name;

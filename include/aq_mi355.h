@@ -64,7 +64,9 @@ int aq_create(int device, aq_ctx **out);
 void aq_destroy(aq_ctx *ctx);
 /* Enqueue on a caller-owned hipStream_t instead of the context's own stream
  * (pass NULL for the legacy default stream the reference launches on,
- * go/engine/hip/hip_driver_cgo.go:452-478).  aq_use_own_stream() goes back. */
+ * go/engine/hip/hip_driver_cgo.go:452-478).  aq_use_own_stream() goes back.
+ * Calls that go through the context's workspace stay in order across a switch: the first of them on the new stream waits
+ * (on the device) for what the old one still does.  All other calls on the two streams are independent of each other. */
 int aq_use_stream(aq_ctx *ctx, void *hip_stream);
 int aq_use_own_stream(aq_ctx *ctx);
 int aq_device_name(aq_ctx *ctx, char *buf, size_t buf_len);

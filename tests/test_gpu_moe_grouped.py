@@ -103,3 +103,46 @@ def test_grouped_gather_captured(ctx):
     ctx.graph_destroy(graph)
     for t in (dx, dl, dr, dy, dw):
         t.free()
+
+
+def test_two_streams_share_one_workspace(ctx):
+    """Grouped gathers keep their lists in the context's workspace: calls that alternate between two streams give what they
+    give on one."""
+    import ctypes
+    say("grouped gathers on two streams")
+    hip = ctypes.CDLL("libamdhip64.so")
+    streams = [ctypes.c_void_p() for _ in range(2)]
+    for st in streams:
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0
+    jobs = []
+    for i, (routes, E, K, N) in enumerate([(2000, 4, 1024, 512), (300, 16, 512, 256)]):
+        rng = np.random.default_rng(60 + i)
+        dw = DeviceAffine(ctx, *F.synthetic_affine(E * N, K, 4, 64, seed=2950 + i))
+        held = [ctx.to_device(F.synthetic_x(routes, K, seed=2960 + i)), ctx.to_device(np.arange(routes, dtype=np.int32)),
+                ctx.to_device(rng.integers(0, E, routes).astype(np.int32)), ctx.alloc(routes * N * 2)]
+        dx, dl, dr, dy = held
+        call = lambda a=(dx, dw.w, dw.s, dw.b, dl, dr, dy, routes, routes, K, N, E, N, 0, 64, 4): ctx.gather_qmv(*a)
+        call()
+        ctx.sync()
+        jobs.append((call, dy, dy.download(np.uint16).copy(), held + [dw]))
+    try:
+        for _ in range(10):
+            for _, dy, _, _ in jobs:
+                ctx.fill_zero(dy)
+            ctx.sync()
+            for _ in range(3):
+                for st, (call, _, _, _) in zip(streams, jobs):
+                    assert ctx.lib.aq_use_stream(ctx.handle, st) == 0
+                    call()
+            for st, (_, dy, want, _) in zip(streams, jobs):
+                assert hip.hipStreamSynchronize(st) == 0
+            assert ctx.lib.aq_use_own_stream(ctx.handle) == 0
+            for _, dy, want, _ in jobs:
+                assert np.array_equal(dy.download(np.uint16), want)
+    finally:
+        ctx.lib.aq_use_own_stream(ctx.handle)
+    for st in streams:
+        hip.hipStreamDestroy(st)
+    for _, _, _, held in jobs:
+        for t in held:
+            t.free()
