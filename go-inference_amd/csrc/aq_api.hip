@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <exception>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -629,9 +630,20 @@ int aq_timer_stop(aq_ctx* ctx, float* elapsed_ms) {
 struct aq_graph {
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    // the context workspaces whose addresses the captured kernels carry, and the generation they were captured under
-    bool uses_ws = false, uses_head_ws = false;
-    uint64_t ws_generation = 0, head_ws_generation = 0;
+    // what the captured kernels have of one of the context's workspaces: the block whose address they carry, kept until the
+    // graph is destroyed, and the generation it was captured under, which calls that cannot do without scratch are held to
+    struct Scratch {
+        bool used = false, required = false;
+        uint64_t generation = 0;
+        std::shared_ptr<aq::WorkspaceBlock> block;
+        void note(const aq::Workspace& ws) {
+            used = ws.touched;
+            required = ws.required;
+            generation = ws.generation;
+            if (used) block = ws.block;
+        }
+        bool stale(const aq::Workspace& ws) const { return required && generation != ws.generation; }
+    } ws, head_ws;
 };
 
 int aq_capture_begin(aq_ctx* ctx) {
@@ -641,7 +653,7 @@ int aq_capture_begin(aq_ctx* ctx) {
     AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->ws), "hipEventRecord");
     AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->head_ws), "hipEventRecord");
     AQ_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    ctx->ws.touched = ctx->head_ws.touched = false;
+    ctx->ws.touched = ctx->ws.required = ctx->head_ws.touched = ctx->head_ws.required = false;
     return AQ_OK;
 }
 
@@ -657,10 +669,8 @@ int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
         return fail(AQ_ERR_NOMEM, "aq_capture_end: out of host memory");
     }
     ag->graph = g;
-    ag->uses_ws = ctx->ws.touched;
-    ag->uses_head_ws = ctx->head_ws.touched;
-    ag->ws_generation = ctx->ws.generation;
-    ag->head_ws_generation = ctx->head_ws.generation;
+    ag->ws.note(ctx->ws);
+    ag->head_ws.note(ctx->head_ws);
     hipError_t rc = hipGraphInstantiate(&ag->exec, g, nullptr, nullptr, 0);
     if (rc != hipSuccess) {
         aq_graph_destroy(ag);
@@ -673,14 +683,13 @@ int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
 int aq_graph_launch(aq_ctx* ctx, aq_graph* graph) {
     if (!ctx || !graph || !graph->exec) return fail(AQ_ERR_ARG, "aq_graph_launch: bad argument");
     std::lock_guard<std::mutex> lk(ctx->mu);
-    if ((graph->uses_ws && graph->ws_generation != ctx->ws.generation) ||
-        (graph->uses_head_ws && graph->head_ws_generation != ctx->head_ws.generation))
+    if (graph->ws.stale(ctx->ws) || graph->head_ws.stale(ctx->head_ws))
         return fail(AQ_ERR_UNSUPPORTED,
                     "aq_graph_launch: the context's workspace was reallocated after this graph was captured (a later call "
-                    "needed more room); the graph's kernels still point at the freed block: capture it again, and reserve "
+                    "needed more room); the graph's kernels still point at the old block: capture it again, and reserve "
                     "the largest workspace first (aq_reserve_workspace / aq_reserve_workspace_bytes)");
-    if (graph->uses_ws) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->ws), "hipStreamWaitEvent");
-    if (graph->uses_head_ws) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->head_ws), "hipStreamWaitEvent");
+    if (graph->ws.used) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->ws), "hipStreamWaitEvent");
+    if (graph->head_ws.used) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->head_ws), "hipStreamWaitEvent");
     AQ_HIP(hipGraphLaunch(graph->exec, ctx->stream), "hipGraphLaunch");
     return AQ_OK;
 }
@@ -951,11 +960,18 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         q.bits = bits;
         q.out_f32 = (flags & AQ_OUT_F32) ? 1 : 0;
         half_need = aq::qmm_scratch_bytes(M, K, 0, ctx->cu_count) + aq::qmmh_partial_bytes(q);
-        need = half_need > need ? half_need : need;
     }
-    // the largest scratch first, so that no member makes the workspace move under the pass over x
-    if (!(q.nseg == count && !aq::workspace_may_grow(&ctx->ws, need, ctx->stream)))
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
+    // the largest scratch first, so that no member makes the workspace move under the pass over x (groups of 32 do without:
+    // the grid asks for its own, and the any-width kernel runs members that cannot have it)
+    if (group_size != 32 && !(q.nseg == count && !aq::workspace_may_grow(&ctx->ws, half_need, ctx->stream))) {
+        const int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, half_need > need ? half_need : need, fail);
+        if (rc == AQ_ERR_NOMEM) {
+            in_grid = 0;  // one member at a time, each with the scratch it can have
+            q.nseg = 0;
+        } else if (rc != AQ_OK) {
+            return rc;
+        }
+    }
     int x_state = aq::kXReadyNone;
     if (q.nseg > 0) {
         const int rc = aq::qmmh_run(ctx->stream, &ctx->ws, ctx->cu_count, -1, q, &ctx->last_variant[1], fail, &x_state);
@@ -1033,9 +1049,8 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     const size_t xbytes = tiles ? (aq::qmmt_workspace_bytes(most_rows, a.K) + 255) & ~(size_t)255 : 0;
     const size_t list = align256((size_t)most_chunks * sizeof(aq::RouteChunk)), places = align256((size_t)most_rows * 4);
     const size_t need = xbytes + list + 256 + 2 * places;
-    if (!aq::workspace_may_grow(&ctx->ws, need, ctx->stream)) return kPass;
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
+    if (!aq::workspace_offer(ctx->stream, &ctx->ws, need)) return kPass;  // the per-route kernels need no scratch
     char* p = static_cast<char*>(ctx->ws.ptr) + xbytes;
     aq::RouteGroupArgs g{};
     g.lhs = a.lhs;

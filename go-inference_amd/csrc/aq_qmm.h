@@ -153,7 +153,7 @@ bool qmmh_takes(const void* x, const void* packed, int K, int group_size, int bi
 // Whether an unforced call on one matrix runs on them (the choice among the families by shape).
 bool qmmh_runs(int M, int K, int N, int group_size, int bits);
 // One call of them over q.nseg matrices, or on expert slabs (idx < 0: qmmh_pick); x_state as in qmm_dispatch.  Scratch that
-// cannot be had because the stream is being captured: kQmmhNoScratch, nothing launched.
+// cannot be had (the stream is being captured, or there is no memory): kQmmhNoScratch, nothing launched.
 constexpr int kQmmhNoScratch = INT32_MIN;
 int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCall& q, const char** last_variant, FailFn fail, int* x_state);
 // Whether qmm_dispatch runs this call on the tile kernels, whose stores can carry the gated-MLP epilogue.

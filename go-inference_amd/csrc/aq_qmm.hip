@@ -103,11 +103,18 @@ int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCa
         for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, q.bits, &q.seg[i], cu_count);
     const size_t xbytes = (qmmt_workspace_bytes(q.chunks ? q.most_rows : q.M, q.K) + 255) & ~(size_t)255;
     const size_t need = xbytes + qmmh_partial_bytes(q);
-    if (!workspace_may_grow(ws, need, stream)) return kQmmhNoScratch;
-    const uint64_t generation = ws->generation;
-    if (int rc = workspace_reserve(stream, ws, need, fail)) return rc;
+    const uint64_t moves = ws->moves;
+    if (q.group_size == 32 || q.chunks) {
+        // (what runs these calls otherwise, the any-width and the per-route kernels, needs no scratch)
+        if (!workspace_offer(stream, ws, need)) return kQmmhNoScratch;
+    } else {
+        if (!workspace_may_grow(ws, need, stream)) return kQmmhNoScratch;
+        const int rc = workspace_reserve(stream, ws, need, fail);
+        if (rc == AQ_ERR_NOMEM) return kQmmhNoScratch;  // the tile kernels ask for less
+        if (rc != AQ_OK) return rc;
+    }
     // (a workspace that had to move no longer holds the earlier pass over x)
-    q.x_ready = x_state && ws->generation == generation ? *x_state : kXReadyNone;
+    q.x_ready = x_state && ws->moves == moves ? *x_state : kXReadyNone;
     if (idx < 0) idx = qmmh_pick(q, cu_count);
     *last_variant = qmmh_variant(idx)->name;
     hipError_t rc = qmmh_launch(idx, q, ws->ptr, stream);
@@ -228,10 +235,10 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
     }
     {
         const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;
-        const uint64_t generation = ws->generation;
+        const uint64_t moves = ws->moves;
         if (int rc = workspace_reserve(stream, ws, xbytes + qmmt_splitk_bytes(M, N, ksplit), fail)) return rc;
         // (a workspace that had to move no longer holds the earlier pass over x)
-        a.x_ready = x_state && ws->generation == generation ? *x_state : kXReadyNone;
+        a.x_ready = x_state && ws->moves == moves ? *x_state : kXReadyNone;
         *last_variant = qmmt_variant(tile_idx)->name;
         hipError_t rc = qmmt_launch_splitk(tile_idx, a, ws->ptr, ksplit, stream);
         if (rc != hipSuccess) return fail((int)rc, "rocm.hip.hipLaunchKernel: HIP returned %d (%s)", (int)rc, hipGetErrorString(rc));

@@ -96,9 +96,13 @@ int aq_timer_stop(aq_ctx *ctx, float *elapsed_ms); /* records, waits, reports */
  * may be called while capturing; the pointers they were given must stay valid for replays.
  * Calls that go through the context's workspace (aq_qmm, aq_qmv with many rows, aq_packed_topk, aq_qmv_greedy,
  * the unfused fallbacks) record the workspace's address: the workspace cannot grow during a capture (the call
- * fails with a message), and when a later call makes it grow, every graph captured over the old block is
+ * fails with a message), and when a later such call makes it grow, every graph captured over the old block is
  * refused by aq_graph_launch with AQ_ERR_UNSUPPORTED - reserve the largest workspace first
- * (aq_reserve_workspace / aq_reserve_workspace_bytes), or capture again. */
+ * (aq_reserve_workspace / aq_reserve_workspace_bytes), or capture again.
+ * Gathers of more than 64 routes (aq_gather_qmv, aq_gather_qmv_gate_up) and matmuls in groups of 32 use the workspace
+ * where they can have it and run without it where they cannot (during a capture that would have to grow it, or for want of
+ * memory): they are never refused for it, and neither is a graph of them.  A graph keeps the block that it was captured over
+ * until it is destroyed. */
 typedef struct aq_graph aq_graph;
 int aq_capture_begin(aq_ctx *ctx);
 int aq_capture_end(aq_ctx *ctx, aq_graph **out);
@@ -186,7 +190,7 @@ size_t aq_workspace_bytes(aq_ctx *ctx);
  * on the host instead).
  * Calls of more than 64 routes (a prompt, a decode batch larger than the expert count) may run grouped by expert: the
  * routes are sorted on the device and an expert's weights read once per 16 to 256 of its routes; scratch comes from the
- * context's workspace (about 2 * K bytes a route; during a capture that would have to grow it, the per-route kernels run).
+ * context's workspace (about 2 * K bytes a route; where it cannot be had, the per-route kernels run).
  * Up to 64 routes every output has the bytes of aq_qmv on the sliced expert. */
 int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, const void *biases,
                   const int32_t *lhs, const int32_t *rhs, void *y, int routes, int x_rows, int K, int N,

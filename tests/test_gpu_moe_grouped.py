@@ -146,3 +146,65 @@ def test_two_streams_share_one_workspace(ctx):
     for _, _, _, held in jobs:
         for t in held:
             t.free()
+
+
+def test_recorded_calls_outlive_a_larger_workspace(orc):
+    """A gather of many routes and matmuls in groups of 32, recorded over the workspace, are replayed after it has moved (other
+    calls asked for more); recorded where it has no room they run on the kernels that need none."""
+    import aq_mi355
+    say("recorded calls, workspace moved")
+    fresh = aq_mi355.Context(0)
+    try:
+        routes, E, K, N, M = 300, 4, 512, 64, 40
+        rng = np.random.default_rng(6)
+        x = F.synthetic_x(routes, K, seed=2970)
+        rhs = rng.integers(0, E, routes).astype(np.int32)
+        mats = [F.synthetic_affine(E * N, K, 4, 64, seed=2971), F.synthetic_affine(N, K, 4, 32, seed=2972), F.synthetic_affine(2 * N, K, 4, 32, seed=2973)]
+        dws = [DeviceAffine(fresh, *m) for m in mats]
+        dx, dl, dr = fresh.to_device(x), fresh.to_device(np.arange(routes, dtype=np.int32)), fresh.to_device(rhs)
+        ys = [fresh.alloc(routes * N * 4), fresh.alloc(M * N * 4), fresh.alloc(M * 2 * N * 4)]
+        gather64 = np.zeros((routes, N))
+        for e in range(E):
+            rows = slice(e * N, (e + 1) * N)
+            gather64[rhs == e] = F.reference_f64(x[rhs == e], mats[0][0][rows], mats[0][1][rows], mats[0][2][rows], 4, 64, K)
+        want = [gather64] + [F.reference_f64(x[:M], *m, 4, 32, K) for m in mats[1:]]
+
+        def step():
+            d = dws[0]
+            fresh.gather_qmv(dx, d.w, d.s, d.b, dl, dr, ys[0], routes, routes, K, N, E, N, 0, 64, 4, aq_mi355.AQ_OUT_F32)
+            names = [fresh.last_variant(0)]
+            fresh.qmm_multi(dx, [d.w for d in dws[1:]], [d.s for d in dws[1:]], [d.b for d in dws[1:]], ys[1:], [N, 2 * N], M, K, 32, 4,
+                            aq_mi355.AQ_OUT_F32)
+            return names + [fresh.last_variant(1)]
+
+        def record():
+            fresh.capture_begin()
+            names = step()
+            return fresh.capture_end(), names
+
+        def replay(graph, what):
+            for i in range(3):
+                for y in ys:
+                    fresh.fill_zero(y)
+                fresh.graph_launch(graph)
+                fresh.sync()
+                for y, ref in zip(ys, want):
+                    check_accumulators(y.download(np.float32, ref.size), ref, "%s, replay %d" % (what, i))
+
+        bare, names = record()  # a context that has run nothing: no workspace
+        assert "grouped" not in names[0] and names[1] == "qmv_generic", names
+        step()
+        fresh.sync()
+        over, names = record()
+        assert "grouped" in names[0] and names[1].startswith("qmmh_"), names
+        replay(over, "before")
+        fresh.reserve_workspace_bytes(64 << 20)
+        fresh.gather_qmv(dx, dws[0].w, dws[0].s, dws[0].b, dl, dr, ys[0], routes, routes, K, N, E, N, 0, 64, 4, aq_mi355.AQ_OUT_F32)
+        replay(over, "after")
+        replay(bare, "without scratch")
+        for g in (over, bare):
+            fresh.graph_destroy(g)
+        for t in [dx, dl, dr] + ys + dws:
+            t.free()
+    finally:
+        fresh.close()

@@ -2,6 +2,8 @@
 // here and write down what they were asked, so that order, growth and refusals can be checked without a GPU.
 #include "aq_workspace.h"
 
+#include "../include/aq_mi355.h"
+
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -137,7 +139,53 @@ static void captured_uses_wait_for_nothing_and_are_ordered_when_replayed() {
     EXPECT(live_blocks == 0);
 }
 
+static void an_offer_that_cannot_be_met_changes_nothing() {
+    aq::Workspace ws;
+    EXPECT(aq::workspace_open(&ws, 0) == hipSuccess);
+    EXPECT(aq::workspace_reserve(A, &ws, 400, quiet) == 0 && seen({"sync A", "malloc 500"}));
+    const void* const before = ws.ptr;
+    const uint64_t generation = ws.generation, moves = ws.moves;
+    capturing_stream = A;
+    EXPECT(!aq::workspace_offer(A, &ws, 501) && aq::workspace_offer(A, &ws, 500) && seen({}));
+    capturing_stream = nullptr;
+    const size_t all = memory;
+    memory = 700;
+    EXPECT(!aq::workspace_offer(A, &ws, 701) && seen({}));
+    EXPECT(ws.ptr == before && ws.bytes == 500 && ws.moves == moves && ws.generation == generation);
+    EXPECT(aq::workspace_offer(A, &ws, 700) && ws.bytes == 700);  // no room for more than the call needs
+    EXPECT(seen({"malloc 700", "sync A", "free"}));
+    EXPECT(ws.moves != moves && ws.generation == generation);
+    memory = all;
+    EXPECT(aq::workspace_reserve(A, &ws, 701, quiet) == 0 && ws.generation == generation + 1);
+    memory = 0;
+    EXPECT(aq::workspace_reserve(A, &ws, 5000, quiet) == AQ_ERR_NOMEM && ws.bytes == 0 && ws.ptr == nullptr);
+    memory = all;
+    EXPECT(aq::workspace_reserve(A, &ws, 100, quiet) == 0 && ws.bytes == 125);
+    aq::workspace_close(&ws);
+    calls.clear();
+    EXPECT(live_blocks == 0);
+}
+
+static void a_block_that_a_graph_keeps_outlives_growth() {
+    aq::Workspace ws;
+    EXPECT(aq::workspace_open(&ws, 1000) == hipSuccess);
+    ws.touched = ws.required = false;  // a capture begins
+    capturing_stream = A;
+    EXPECT(aq::workspace_offer(A, &ws, 900) && ws.touched && !ws.required);
+    capturing_stream = nullptr;
+    std::shared_ptr<aq::WorkspaceBlock> kept = ws.block;
+    EXPECT(aq::workspace_offer(A, &ws, 2000) && live_blocks == 2 && ws.ptr != kept->ptr);
+    EXPECT(aq::workspace_reserve(A, &ws, 4000, quiet) == 0 && live_blocks == 2 && ws.required);
+    kept.reset();  // the graph is destroyed
+    EXPECT(live_blocks == 1);
+    aq::workspace_close(&ws);
+    calls.clear();
+    EXPECT(live_blocks == 0);
+}
+
 int main() {
+    an_offer_that_cannot_be_met_changes_nothing();
+    a_block_that_a_graph_keeps_outlives_growth();
     use_on_another_stream_waits_for_the_last_one();
     captured_uses_wait_for_nothing_and_are_ordered_when_replayed();
     puts("ok");
