@@ -1116,9 +1116,12 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
 
 }  // namespace
 
-int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
-                  const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
-                  int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags) {
+namespace {
+// grouped: whether the routes may be grouped by expert, which puts lists and a copy of x at the start of the context's
+// workspace; not for callers whose x or y lies there.
+int gather_call(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
+                const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
+                int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags, bool grouped) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_gather_qmv: ctx is null");
     if (routes < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_gather_qmv: routes, K, N must be non-negative");
     if (routes == 0 || N == 0 || K == 0) return AQ_OK;  // qmv_gather.go:422-424
@@ -1151,9 +1154,18 @@ int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* sc
     a.row_base = row_base;
     a.x_rows = x_rows;
     a.routes = routes;
-    if (const int rc = run_grouped(ctx, a, group_size, bits, false); rc != kPass) return rc;
+    if (grouped)
+        if (const int rc = run_grouped(ctx, a, group_size, bits, false); rc != kPass) return rc;
     // every expert slab must keep 16-byte row alignment for the dot2 kernels
     return launch_qmv_rows(ctx, a, group_size, bits, true);
+}
+}  // namespace
+
+int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
+                  const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
+                  int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags) {
+    return gather_call(ctx, x, packed, scales, biases, lhs, rhs, y, routes, x_rows, K, N, num_experts, expert_rows, row_base,
+                       group_size, bits, flags, true);
 }
 
 namespace {
@@ -1470,11 +1482,11 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
     }
     float* g = static_cast<float*>(ctx->ws.ptr);
     float* u = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + each);
-    if (int rc = aq_gather_qmv(ctx, x, packed, scales, biases, lhs, rhs, g, routes, x_rows, K, N, num_experts, expert_rows,
-                               gate_row_base, group_size, bits, AQ_OUT_F32))
+    if (int rc = gather_call(ctx, x, packed, scales, biases, lhs, rhs, g, routes, x_rows, K, N, num_experts, expert_rows,
+                             gate_row_base, group_size, bits, AQ_OUT_F32, false))
         return rc;
-    if (int rc = aq_gather_qmv(ctx, x, packed, scales, biases, lhs, rhs, u, routes, x_rows, K, N, num_experts, expert_rows,
-                               up_row_base, group_size, bits, AQ_OUT_F32))
+    if (int rc = gather_call(ctx, x, packed, scales, biases, lhs, rhs, u, routes, x_rows, K, N, num_experts, expert_rows,
+                             up_row_base, group_size, bits, AQ_OUT_F32, false))
         return rc;
     std::lock_guard<std::mutex> lk(ctx->mu);
     AQ_HIP(aq::act_mul_f32_launch(g, u, y, (int64_t)routes * N, act, out_f32 ? 1 : 0, ctx->stream), "hipLaunchKernel");
@@ -1582,8 +1594,8 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, (size_t)x_rows * K * 2, fail)) return rc;
     }
     if (int rc = aq_act_mul(ctx, gate_x, up_x, ctx->ws.ptr, (int64_t)x_rows * K, act)) return rc;
-    return aq_gather_qmv(ctx, ctx->ws.ptr, packed, scales, biases, lhs, rhs, y, routes, x_rows, K, N, num_experts,
-                         expert_rows, row_base, group_size, bits, flags);
+    return gather_call(ctx, ctx->ws.ptr, packed, scales, biases, lhs, rhs, y, routes, x_rows, K, N, num_experts, expert_rows,
+                       row_base, group_size, bits, flags, false);
 }
 
 int aq_moe_route(aq_ctx* ctx, const void* logits, int rows, int num_experts, int top_k, const float* expert_scales,

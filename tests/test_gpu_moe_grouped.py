@@ -208,3 +208,35 @@ def test_recorded_calls_outlive_a_larger_workspace(orc):
             t.free()
     finally:
         fresh.close()
+
+
+@pytest.mark.parametrize("offset", [0, 2])
+def test_gather_act_of_many_routes(ctx, orc, offset):
+    """bf16(act(gate) * up) gathered: where the activations are not 16-byte aligned the product lies in the workspace, and the
+    gather behind it leaves that alone."""
+    import aq_mi355
+    routes, E, K, N = 200, 4, 512, 72
+    say("gather of formed activations", offset)
+    rng = np.random.default_rng(8)
+    words, s, b = F.synthetic_affine(E * N, K, 4, 64, seed=2980)
+    gate, up = F.synthetic_x(routes, K, seed=2981), F.synthetic_x(routes, K, seed=2982)
+    rhs, lhs = rng.integers(0, E, routes).astype(np.int32), rng.permutation(routes).astype(np.int32)
+    pad = lambda a: np.concatenate([np.zeros(offset // 2, np.uint16), a.reshape(-1)])
+    dw = DeviceAffine(ctx, words, s, b)
+    dg, du, dl, dr, dy = (ctx.to_device(pad(gate)), ctx.to_device(pad(up)), ctx.to_device(lhs), ctx.to_device(rhs), ctx.alloc(routes * N * 4))
+    product = ctx.alloc(routes * K * 2)
+    ctx.act_mul(dg.ptr + offset, du.ptr + offset, product, routes * K, aq_mi355.AQ_ACT_SILU)
+    ctx.sync()
+    x = product.download(np.uint16, routes * K).reshape(routes, K)
+    ref = np.zeros((routes, N))
+    for e in range(E):
+        z, rows = np.nonzero(rhs == e)[0], slice(e * N, (e + 1) * N)
+        ref[z] = F.reference_f64(x[lhs[z]], words[rows], s[rows], b[rows], 4, 64, K)
+    for _ in range(2):
+        ctx.fill_zero(dy)
+        ctx.gather_qmv_act(dg.ptr + offset, du.ptr + offset, dw.w, dw.s, dw.b, dl, dr, dy, routes, routes, K, N, E, N, 0, 64, 4,
+                           aq_mi355.AQ_ACT_SILU, aq_mi355.AQ_OUT_F32)
+        ctx.sync()
+        check_accumulators(dy.download(np.float32, routes * N), ref, "gather of formed activations")
+    for t in (dg, du, dl, dr, dy, product, dw):
+        t.free()
