@@ -87,6 +87,27 @@ __device__ __forceinline__ void unpack8_word(uint32_t w, uint32_t p[2]) {
     p[1] = __builtin_amdgcn_perm(f3, f2, 0x07060302u);
 }
 
+// The same with the codes centred on zero, for sums that must not lose what the bias takes off again: 16 * (code - 8) of the
+// eight 4-bit codes in the order of unpack4_word (a signed nibble in the upper half of a byte), code - 128 of four 8-bit codes.
+// Both have at most 8 significant bits: exact in bf16.
+__device__ __forceinline__ uint32_t signed_bytes_to_bf16(uint32_t w, int i, int j) {
+    const float f = (float)(int8_t)(w >> (8 * i)), g = (float)(int8_t)(w >> (8 * j));
+    return __builtin_amdgcn_perm(__float_as_uint(g), __float_as_uint(f), 0x07060302u);
+}
+__device__ __forceinline__ void unpack4_centred(uint32_t w, uint32_t p[4]) {
+    w ^= 0x88888888u;
+    const uint32_t even = (w << 4) & 0xf0f0f0f0u, odd = w & 0xf0f0f0f0u;
+    p[0] = signed_bytes_to_bf16(even, 0, 2);
+    p[1] = signed_bytes_to_bf16(odd, 0, 2);
+    p[2] = signed_bytes_to_bf16(even, 1, 3);
+    p[3] = signed_bytes_to_bf16(odd, 1, 3);
+}
+__device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
+    w ^= 0x80808080u;
+    p[0] = signed_bytes_to_bf16(w, 0, 1);
+    p[1] = signed_bytes_to_bf16(w, 2, 3);
+}
+
 // Activations of the fused kernels.  1: tanh-approximated GELU with the operation order of
 // rocm_gelu_tanh_value (go/engine/hip/kernels/common/math.hipinc:3-9); 2: SiLU, v / (1 + exp(-v))
 // (go/model/attn/gated_delta.go:228).  Contraction is off, so every step is one fp32 operation and each

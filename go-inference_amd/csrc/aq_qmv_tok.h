@@ -89,6 +89,11 @@ __host__ __device__ constexpr int tok16_stage_pieces(int nw) { return nw >= 16 ?
 // its four FMAs, and the affine term is two MFMAs per run.  8-bit codes: a lane's 16 codes lie in one group, but the step
 // of 32 codes that is group 0 of a block of 64 has to come from lane blocks 0 and 1 alone: a swap of 32-lane halves
 // between the two steps' registers moves the second 8 codes of those lanes to lane blocks 2 and 3 (x takes the same swap).
+// The operand of these forms holds the codes centred on zero, 16 (code - 8) or code - 128 (aq_device.h), and the affine term
+// bias + 8 scale (128 scale): a weight is near zero on average, and what 128 + code has beside it comes off again out of sums
+// 28 times the result (21 x 3840 x 512, groups of 32: 2.1e-6 from the float64 product, centred 1.0e-7, the any-width kernel
+// that this shape had 0.9e-7; 8 bit 1.6e-7 -> 1.0e-7, any-width 1.35e-7).  It costs 16 vector instructions a word instead of 7:
+// a layer of 21 rows (3840 / 15360, groups of 32) 97.7 -> 103.4 us.
 // Measured (graph replay, weights from HBM): 21 x 3840 x 15360 in groups of 32 19.4 us (the any-width kernel this shape had:
 // 0.48 ms a matrix), 32 x 4096 x 14336 21.0 us against 16.9 us for groups of 64: four more FMAs a lane per 32 codes; 32 x
 // 4032 x 14336 18.9 us, 2 us over whole runs for the element-wise staging.
@@ -102,6 +107,7 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
     static_assert(GRP == 64 || (GRP == 32 && ANY), "group size");
     constexpr bool G32 = GRP == 32;
     constexpr int GPR = 256 / GRP;  // groups of a run
+    constexpr bool CENTRED = ANY;   // the operand's codes: 16 (code - 8) or code - 128, else 128 + code or code
     static_assert(!PAIR || RS % 2 == 0, "a pair shares its sets of rows between two matrices");
     constexpr int PAIRS = PAIR ? 2 : 1;
     constexpr int LINES = BITS / 4;  // 128-byte lines of a row per run of 256 codes
@@ -409,13 +415,15 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
             transpose(t0, t1, t2, t3);
             float X = (__uint_as_float(t0) + __uint_as_float(t1)) + (__uint_as_float(t2) + __uint_as_float(t3));
             if (!live[j]) X = 0.0f;
+            constexpr float kUnit = CENTRED && BITS == 4 ? 16.0f : 1.0f;  // what the operand has 1 of a code as
+            X *= kUnit;
             const uint32_t u0 = __float_as_uint(X) & 0xffff0000u;
             const float r1 = X - __uint_as_float(u0);
             const uint32_t u1 = __float_as_uint(r1) & 0xffff0000u;
             const float r2 = r1 - __uint_as_float(u1);
             const uint32_t u2 = __float_as_uint(r2) & 0xffff0000u;
-            // 4 bit: the expanded codes are 128 + code
-            const float off = BITS == 4 ? -128.0f : 0.0f;
+            // what the operand's codes lack of the codes
+            const float off = CENTRED ? (BITS == 4 ? 8.0f : 128.0f) : BITS == 4 ? -128.0f : 0.0f;
             const uint32_t m0 = __float_as_uint(off * __uint_as_float(u0));
             const uint32_t m1 = __float_as_uint(off * __uint_as_float(u1));
             const uint32_t m2 = __float_as_uint(off * __uint_as_float(u2));
@@ -480,8 +488,13 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
 #pragma unroll
                     for (int half = 0; half < 2; half++) {
                         uint32_t e[4];
-                        if constexpr (BITS == 4) {
+                        if constexpr (BITS == 4 && CENTRED) {
+                            unpack4_centred(ww[2 * g + half], e);
+                        } else if constexpr (BITS == 4) {
                             unpack4_word(ww[2 * g + half], mask, magic, e);
+                        } else if constexpr (CENTRED) {
+                            unpack8_centred(ww[4 * g + 2 * half], e);
+                            unpack8_centred(ww[4 * g + 2 * half + 1], e + 2);
                         } else {
                             unpack8_word(ww[4 * g + 2 * half], e);
                             unpack8_word(ww[4 * g + 2 * half + 1], e + 2);
@@ -558,7 +571,7 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
         float total = red[t * TSTRIDE + column];
 #pragma unroll
         for (int p = 1; p < NW; p++) total += red[(p * 16 * TS + t) * TSTRIDE + column];
-        return total;
+        return CENTRED && BITS == 4 ? total * 0.0625f : total;
     };
     for (int o = tid; o < 16 * TS * OUTS; o += NW * kWave) {
         const int t = o / OUTS, rl = o - t * OUTS;

@@ -134,3 +134,22 @@ def test_gated_pair_scales_of_any_alignment(ctx, orc, off_gate, off_up, fused):
     assert (np.abs(got - want) <= 1e-4 * np.maximum(1.0, np.abs(g * u) + np.abs(g) + np.abs(u))).all()
     for t in held + [dx, dy]:
         t.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K,N", [(4, 32, 3, 3840, 300), (4, 32, 21, 3840, 300), (4, 32, 32, 1024, 300), (4, 32, 21, 15360, 64), (4, 128, 12, 2944, 300),
+                                           (4, 64, 20, 4032, 1056), (8, 32, 21, 3840, 300), (8, 64, 3, 4032, 1056), (8, 128, 32, 2944, 300)])
+def test_sums_keep_fp32_accuracy(ctx, bits, gs, M, K, N):
+    """Weights centred on zero, as GGUF tensors and the synthetic ones are: what the operand's codes carry beside the weight
+    must not be taken off again out of a sum many times the result.  2^-21 = 4.8e-7 of the result's 2-norm: eight roundings of
+    2^-24 on the way (the fp32 sums of the any-width kernel end at 0.7e-7 to 2.5e-7, sums over 128 + code at 2e-6)."""
+    say("token tile accuracy", bits, gs, M, K, N)
+    words, s, b = F.synthetic_affine(N, K, bits, gs, seed=2390 + K)
+    x = F.synthetic_x(M, K, seed=2391 + M)
+    dw = DeviceAffine(ctx, words, s, b)
+    got = run_qmv(ctx, x, dw, M, K, N, gs, bits, True).astype(np.float64)
+    assert ctx.last_variant(0).startswith("qmvt_"), ctx.last_variant(0)
+    ref = F.reference_f64(x, words, s, b, bits, gs, K)
+    err = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    print("error %.2e" % err)
+    assert err <= 2.0 ** -21
+    dw.free()
