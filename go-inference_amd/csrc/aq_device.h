@@ -108,6 +108,37 @@ __device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
     p[1] = signed_bytes_to_bf16(w, 2, 3);
 }
 
+// scale * code + bias in two roundings.
+__device__ __forceinline__ float affine_weight(float scale, float code, float bias) {
+#pragma clang fp contract(off)
+    const float prod = scale * code;
+    return prod + bias;
+}
+
+// x . w of one weight row in groups of 32, as the any-width kernel forms it: fp32 weights, fp32 sums.  For the outputs that sums
+// over codes leave without a finite value: with an infinity in x (or products beyond fp32) the part that the bias takes off
+// again is infinite as well, and the difference NaN whatever the sign of the weight.
+__device__ __forceinline__ bool not_finite(float v) { return (__float_as_uint(v) & 0x7f800000u) == 0x7f800000u; }
+__device__ __forceinline__ float plain_dot_g32(const uint16_t* x, const uint32_t* w, const uint16_t* s, const uint16_t* b, int K, int bits) {
+    float sum = 0.0f;
+    const uint32_t mask = (1u << bits) - 1u;
+#pragma nounroll
+    for (int g = 0; g < K / 32 && sum == sum; g++) {
+        const float sc = bf16_bits_to_f32(s[g]), bi = bf16_bits_to_f32(b[g]);
+#pragma nounroll
+        for (int i = 0; i < bits; i++) {
+            const uint32_t word = w[g * bits + i];
+            const uint16_t* const xi = x + g * 32 + i * (32 / bits);
+#pragma nounroll
+            for (int c = 0; c * bits < 32; c++) {
+                const float code = (float)((word >> (c * bits)) & mask);
+                sum = __fmaf_rn(affine_weight(sc, code, bi), bf16_bits_to_f32(xi[c]), sum);
+            }
+        }
+    }
+    return sum;
+}
+
 // Activations of the fused kernels.  1: tanh-approximated GELU with the operation order of
 // rocm_gelu_tanh_value (go/engine/hip/kernels/common/math.hipinc:3-9); 2: SiLU, v / (1 + exp(-v))
 // (go/model/attn/gated_delta.go:228).  Contraction is off, so every step is one fp32 operation and each

@@ -37,13 +37,6 @@ hipError_t ensure_dynamic_lds(const void* fn, size_t lds) {
     return rc;
 }
 
-
-__device__ __forceinline__ float affine_weight(float scale, float code, float bias) {
-#pragma clang fp contract(off)
-    const float prod = scale * code;
-    return prod + bias;
-}
-
 // Code `col` of a packed row, any width 1..8, codes may cross a word boundary.
 __device__ __forceinline__ uint32_t extract_code(const uint32_t* row, int64_t words, int64_t col, int bits) {
     const int64_t bit = col * bits;

@@ -94,10 +94,11 @@ struct QmmHalfArgs {
     const uint16_t* xf;  // as in QmmTileArgs, fp16
     const uint16_t* xs;
     const float* rs;  // per row, the inverse of the power of two it was scaled by
+    const uint16_t* x;  // groups of 32 (not expert slabs): x itself, for outputs without a finite value; else null
     QmmSegment seg[kQmmSegments];
     int nseg, pair;  // pair: seg[0] is the gate matrix, seg[1] the up matrix of a gated MLP; one output
     int M, K;
-    int gs_blocks, out_f32, act;
+    int bits, gs_blocks, out_f32, act;
     int mblks, tiles_m;
     int units;    // column units of all matrices
     int group_m;  // row bands of a group of tiles

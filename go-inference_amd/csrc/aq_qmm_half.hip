@@ -202,6 +202,28 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
     }
 }
 
+// Output (m, n) of a matrix (pair: of the gated pair) formed again from x itself, if what is stored there is not finite: dense
+// calls in groups of 32 ran on the any-width kernel, which keeps infinities (plain_dot_g32).  The test costs a prompt of 509
+// tokens 4 of 420 us (3840 / 15360); rows with an infinity cost what the any-width kernel took for them.
+__device__ __forceinline__ void fix_output(const QmmHalfArgs& a, const QmmSegment& seg, int m, int n) {
+    const int64_t at = (int64_t)m * seg.N + n;
+    if (!not_finite(a.out_f32 ? static_cast<const float*>(seg.y)[at] : bf16_bits_to_f32(static_cast<const uint16_t*>(seg.y)[at]))) return;
+    const uint16_t* const x = a.x + (int64_t)m * a.K;
+    const int64_t word = (int64_t)n * (a.K / 32 * a.bits), group = (int64_t)n * (a.K / 32);
+    float v[2];
+#pragma nounroll
+    for (int i = 0; i < (a.pair ? 2 : 1); i++) {
+        const QmmSegment& from = i ? a.seg[1] : seg;
+        const float d = plain_dot_g32(x, from.w + word, from.s + group, from.b + group, a.K, a.bits);
+        if (i) v[1] = d; else v[0] = d;
+    }
+    const float y = a.pair ? fmul_unfused(act_value(a.act, v[0]), v[1]) : v[0];
+    if (a.out_f32)
+        static_cast<float*>(seg.y)[at] = y;
+    else
+        static_cast<uint16_t*>(seg.y)[at] = f32_to_bf16_bits(y);
+}
+
 // ---- main kernel ----------------------------------------------------------------------------
 // OCC: wavefronts per SIMD the register budget is cut for (2: 256 registers, 1: 512, the accumulators then live in
 // the accumulation half of the register file).
@@ -705,6 +727,7 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     const bool y_f32 = partial != nullptr || a.out_f32 != 0;
     // COLS columns of the wavefront's tile leave together, eight consecutive ones per lane; `gated`: act(gate) * up of the two
     // column blocks.  (Partial tiles of a pair keep both sums: the gate columns of all outputs, then the up columns.)
+    [[maybe_unused]] bool odd_one = false;  // this lane has stored a value that may not be finite
     auto store_tile = [&](auto gated_tag) {
         constexpr bool GATED = decltype(gated_tag)::value;
         constexpr int COLS = GATED ? CW / 2 : CW;
@@ -750,6 +773,8 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
                     if (route < 0) lo = hi = make_float4(0.f, 0.f, 0.f, 0.f);  // an expert id or a row of x out of range
                     y_row = route & INT32_MAX;
                 }
+                if (G32 && !partial)  // (one test for the eight; fix_output looks at each)
+                    odd_one |= not_finite(((fabsf(lo.x) + fabsf(lo.y)) + (fabsf(lo.z) + fabsf(lo.w))) + ((fabsf(hi.x) + fabsf(hi.y)) + (fabsf(hi.z) + fabsf(hi.w))));
                 const int64_t o = y_row * stride + col;
                 if (wide && n + 8 <= N) {
                     if (y_f32) {
@@ -784,6 +809,20 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         store_tile(std::true_type{});
     } else {
         store_tile(std::false_type{});
+    }
+    if constexpr (G32) {
+        // Dense groups of 32 keep what the any-width kernel makes of infinities: a lane goes over what it has stored once more.
+        // (Partial tiles: qmmh_reduce_kernel does.)
+        if (a.x && !partial && odd_one) {
+            const int lanes = pair ? 4 : 8, row_in = lane / lanes, c8 = (lane % lanes) * 8;
+            const int first = n0 + wave_n * (pair ? 32 : CW) + c8;
+#pragma nounroll
+            for (int r = row_in; r < MB * 32; r += kWave / lanes) {
+                const int m = m0 + wave_m * MB * 32 + r;
+#pragma nounroll
+                for (int n = first; n < first + 8 && n < N && m < mend; n++) fix_output(a, a.seg[seg], m, n);
+            }
+        }
     }
 }
 
@@ -827,6 +866,13 @@ __global__ __launch_bounds__(256) void qmmh_reduce_kernel(const QmmHalfArgs a) {
         } else {
 #pragma unroll
             for (int e = 0; e < V; e++) static_cast<uint16_t*>(seg.y)[o + e] = f32_to_bf16_bits(v[e]);
+        }
+        float all = 0.0f;
+#pragma unroll
+        for (int e = 0; e < V; e++) all += fabsf(v[e]);
+        if (a.x && not_finite(all)) {
+#pragma nounroll
+            for (int e = 0; e < V; e++) fix_output(a, seg, m, c + e);
         }
     }
 }
@@ -977,6 +1023,8 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     a.pair = q.pair;
     a.M = q.M;
     a.K = q.K;
+    a.bits = q.bits;
+    a.x = g32 && !q.chunks ? q.x : nullptr;
     a.gs_blocks = g32 ? 1 : q.group_size / 64;
     a.out_f32 = q.out_f32;
     a.act = q.act;

@@ -93,7 +93,8 @@ __host__ __device__ constexpr int tok16_stage_pieces(int nw) { return nw >= 16 ?
 // bias + 8 scale (128 scale): a weight is near zero on average, and what 128 + code has beside it comes off again out of sums
 // 28 times the result (21 x 3840 x 512, groups of 32: 2.1e-6 from the float64 product, centred 1.0e-7, the any-width kernel
 // that this shape had 0.9e-7; 8 bit 1.6e-7 -> 1.0e-7, any-width 1.35e-7).  It costs 16 vector instructions a word instead of 7:
-// a layer of 21 rows (3840 / 15360, groups of 32) 97.7 -> 103.4 us.
+// a layer of 21 rows (3840 / 15360, groups of 32) 97.7 -> 103.4 us (104.5 with the
+// test of every sum of dense groups of 32 for infinities, which the any-width kernel keeps: see plain_dot_g32).
 // Measured (graph replay, weights from HBM): 21 x 3840 x 15360 in groups of 32 19.4 us (the any-width kernel this shape had:
 // 0.48 ms a matrix), 32 x 4096 x 14336 21.0 us against 16.9 us for groups of 64: four more FMAs a lane per 32 codes; 32 x
 // 4032 x 14336 18.9 us, 2 us over whole runs for the element-wise staging.
@@ -578,7 +579,17 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
         const int row = row0 + rl;
         if (t >= M || row >= N) continue;
         float total = total_of(t, rl);
-        if constexpr (PAIR) total = fmul_unfused(act_value(a.act, total), total_of(t, OUTS + rl));
+        [[maybe_unused]] float up = PAIR ? total_of(t, OUTS + rl) : 0.0f;
+        if constexpr (G32 && !GROUPED) {  // (dense groups of 32 keep what the any-width kernel makes of infinities)
+#pragma nounroll
+            for (int part = 0; part < PAIRS; part++) {
+                if (!not_finite(part ? up : total)) continue;
+                const float v = plain_dot_g32(a.x + (size_t)t * K, (PAIR && part ? a.w2 : a.w) + (size_t)row * (row_bytes / 4),
+                                              (PAIR && part ? a.s2 : a.s) + (size_t)row * sgroups, (PAIR && part ? a.b2 : a.b) + (size_t)row * sgroups, K, BITS);
+                if (part) up = v; else total = v;
+            }
+        }
+        if constexpr (PAIR) total = fmul_unfused(act_value(a.act, total), up);
         size_t y_row = (size_t)t;
         if constexpr (GROUPED) {
             const int route = a.route_of[first_route + t];
