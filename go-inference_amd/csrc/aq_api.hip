@@ -994,7 +994,7 @@ int aq_reserve_workspace(aq_ctx* ctx, int M, int K) {
     if (M == 0 || K == 0) return AQ_OK;
     std::lock_guard<std::mutex> lk(ctx->mu);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    return aq::qmm_reserve(ctx->stream, &ctx->ws, M, K, fail);
+    return aq::qmm_reserve(ctx->stream, &ctx->ws, M, K, ctx->cu_count, fail);
 }
 
 int aq_reserve_workspace_bytes(aq_ctx* ctx, size_t bytes) {

@@ -129,6 +129,8 @@ void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count);
 // The kernel for these matrices (the bytes of a result do not depend on it).
 int qmmh_pick(const QmmHalfCall& q, int cu_count);
 size_t qmmh_partial_bytes(const QmmHalfCall& q);
+// What one matrix of any N needs at most with up to M rows of up to K columns.
+size_t qmmh_partial_most(int M, int K, int cu_count);
 
 hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream);
 
@@ -137,8 +139,8 @@ hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream);
 // own data in the same workspace place it behind this.
 size_t qmm_scratch_bytes(int M, int K, int N, int cu_count);
 
-// Sizes ws for activations of M x K ahead of time (not during capture).
-int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, FailFn fail);
+// Sizes ws for prefill calls with activations of up to M x K ahead of time (not during capture).
+int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, int cu_count, FailFn fail);
 
 // Validated-shape dispatch used by aq_qmm and by aq_qmv for calls the matvec families pass on.
 // Returns an AQ_* / hipError_t code through `fail`.

@@ -62,8 +62,10 @@ size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
     return xbytes + ((partial + 255) & ~(size_t)255);
 }
 
-int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, FailFn fail) {
-    return workspace_reserve(stream, ws, qmmt_workspace_bytes(M, K), fail);
+int qmm_reserve(hipStream_t stream, Workspace* ws, int M, int K, int cu_count, FailFn fail) {
+    const size_t xbytes = (qmmt_workspace_bytes(M, K) + 255) & ~(size_t)255;
+    const int rc = workspace_reserve(stream, ws, xbytes + qmmh_partial_most(M, K, cu_count), fail);
+    return rc == AQ_ERR_NOMEM ? workspace_reserve(stream, ws, xbytes, fail) : rc;  // without shares of K, on the tile kernels
 }
 
 static int find_qmmt(int bits, int mb, int nb, int wm, int wn) {

@@ -969,6 +969,19 @@ void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count) {
     }
 }
 
+size_t qmmh_partial_most(int M, int K, int cu_count) {
+    if (K / 64 <= 8) return 0;  // no share of fewer than eight blocks
+    const int cus = cu_count > 0 ? cu_count : 256;
+    // qmmh_split: strips x bands x shares <= 4 CUs, so that shares x N <= 4 CUs x columns of a tile / bands of M rows
+    size_t most = 0;
+    for (int i = 0; i < qmmh_variant_count(); i++) {
+        const size_t rows = qmmh_rows(i), bn = (size_t)kQmmHalfTable[i].v.wn * kQmmHalfTable[i].v.nb * 32;
+        const size_t bytes = (size_t)4 * cus * bn * ((size_t)M < rows ? (size_t)M : rows) * 4;
+        most = bytes > most ? bytes : most;
+    }
+    return (most + 255) & ~(size_t)255;
+}
+
 int qmmh_pick(const QmmHalfCall& q, int cu_count) {
     const int cus = cu_count > 0 ? cu_count : 256;
     int best = -1;

@@ -161,15 +161,18 @@ int aq_qmm_multi(aq_ctx *ctx, const void *x, int count, const void *const *packe
                  const void *const *biases, void *const *y, const int *N, int M, int K, int group_size, int bits,
                  unsigned flags);
 
-/* Prefill-sized aq_qmm / aq_qmv calls (M >= 64) rewrite x into MFMA operand order first and keep that
- * copy (about M*K*2 bytes) in a workspace the context owns.  The workspace grows on demand, which
+/* Prefill-sized aq_qmm / aq_qmv calls (more than 64 rows; 33 where K is no multiple of 256; any in groups of 32) rewrite x into
+ * MFMA operand order first and keep that copy (about M*K*2 bytes) in a workspace the context owns, and beside it, where the
+ * tiles of a matrix leave CUs idle, the fp32 partial tiles of shares of K.  The workspace grows on demand, which
  * drains the stream and allocates: not allowed while a capture is open and unwelcome in a serving
- * loop.  This call sizes it ahead of time for activations of up to M x K.  The reference sizes its
+ * loop.  This call sizes it ahead of time for one matrix of any N and activations of up to M x K (the copy and at most
+ * 16 KiB * min(M, 256) * CUs of partial tiles: 268 MB at M >= 256 on 256 CUs).  The reference sizes its
  * own scratch the same way at model load (hipMLXQ4DeviceWeightConfig and the batch scratch of
  * go/engine/hip/hip_projection_launch.go:2671-2720). */
 int aq_reserve_workspace(aq_ctx *ctx, int M, int K);
-/* The same by size.  Besides the prefill copy of x the workspace holds: the fp32 partial tiles of calls with
- * 5..64 rows whose K is shared out over workgroups (up to 64*M*N bytes), the intermediates of the unfused
+/* The same by size.  Besides those the workspace holds: the partial tiles of the few-rows kernels (5..64 rows, up to 64*M*N
+ * bytes), those of all members of an aq_qmm_multi call and of both matrices of an aq_qmv_gate_up call, the lists of gathers of
+ * more than 64 routes, the intermediates of the unfused
  * fallbacks of the fused MLP / lm_head entry points, and the scratch of aq_packed_topk.  A call that needs
  * more than is there grows it (not possible while a capture is open): run such a call once before capturing,
  * or reserve its bytes here. */

@@ -105,3 +105,41 @@ def test_ragged_shares_of_k_few_rows(ctx):
     assert ctx.last_variant(0).startswith("qmmt_"), ctx.last_variant(0)
     check_accumulators(acc, F.reference_f64(x, words, s, b, 4, 64, K), "ragged shares")
     dw.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K,N", [(4, 64, 300, 4096, 4096), (4, 128, 130, 8192, 1024), (8, 64, 300, 4096, 4096), (4, 64, 40, 4032, 512),
+                                           (4, 64, 97, 15360, 3840)])
+def test_reserved_by_rows_and_columns_a_call_is_captured_on_its_kernels(bits, gs, M, K, N):
+    """aq_reserve_workspace(M, K) holds all that a prefill call of that size needs, its partial tiles included: recorded into a
+    graph it runs on the kernels of the eager call and gives its bytes; so does a call of fewer rows."""
+    import aq_mi355
+    say("qmm in a graph after reserving", bits, gs, M, K, N)
+    words, s, b = F.synthetic_affine(N, K, bits, gs, seed=2720)
+    x = F.synthetic_x(M, K, seed=2721)
+    fresh = aq_mi355.Context(0)
+    try:
+        dw = DeviceAffine(fresh, words, s, b)
+        dx, dy = fresh.to_device(x), fresh.alloc(M * N * 4)
+        fresh.reserve_workspace(M, K)
+        held = fresh.workspace_bytes()
+        recorded = []
+        for rows in (M, M - 3):
+            fresh.capture_begin()
+            fresh.qmm(dx, dw.w, dw.s, dw.b, dy, rows, K, N, gs, bits, aq_mi355.AQ_OUT_F32)
+            recorded.append((rows, fresh.last_variant(1), fresh.capture_end()))
+        for rows, name, graph in recorded:
+            fresh.qmm(dx, dw.w, dw.s, dw.b, dy, rows, K, N, gs, bits, aq_mi355.AQ_OUT_F32)
+            fresh.sync()
+            want = dy.download(np.uint32, rows * N)
+            assert name == fresh.last_variant(1) and name.startswith("qmmh"), (name, fresh.last_variant(1))
+            assert fresh.workspace_bytes() == held
+            for _ in range(3):
+                fresh.fill_zero(dy)
+                fresh.graph_launch(graph)
+                fresh.sync()
+                assert np.array_equal(dy.download(np.uint32, rows * N), want)
+            fresh.graph_destroy(graph)
+        for t in (dx, dy, dw):
+            t.free()
+    finally:
+        fresh.close()
