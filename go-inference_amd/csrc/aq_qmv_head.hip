@@ -282,18 +282,24 @@ __global__ __launch_bounds__(256) void packed_topk_kernel(const unsigned long lo
 // at least top_k entries reach (the maxima themselves), so the top_k largest entries all lie among the entries
 // >= T; for scores that are not arranged by rank that set is a little over top_k entries, and one workgroup
 // orders it by counting.  Three launches: maxima, filter, finish.  When more than kTopKCandidates entries
-// reach T (long runs of equal scores, an input sorted by score) the finish launch runs the first round of the
-// segment-by-segment reduction instead, and the workgroup that ends it last the rounds that are left (as launches of their
-// own, which left at once where there was nothing to do, those rounds took 1.6 us each of every call).
+// reach T (long runs of equal scores, an input sorted by score) the finish launch runs the segment-by-segment reduction
+// instead, all its rounds: as launches of their own, which left at once where there was nothing to do, the later ones took
+// 1.6 us each of every call.  Measured, us for 262144 entries and the best 40 in random order / sorted by score: rounds as
+// launches 16.8 / 53.4, in the workgroup that ends the first round last 13.7 / 83.0, as the tree 14.0 / 54.2 (best 8: 14.5 /
+// 27.9, 10.8 / 30.8, 10.9 / 29.6; best 64: 19.4 / 70.0, 16.4 / 127.5, 16.3 / 71.2).
 // A wavefront of these two kernels takes a piece of 64 * V entries: V is the largest of 16, 4, 1 that leaves at
 // least top_k pieces.
+// Head of the threshold path's scratch in 8-byte entries: the candidate counter and the tickets of the tree's nodes, 4 bytes
+// each (at most 1024 segments in nodes of 16 lists or more: 64 + 4 + 1).
+constexpr int kTopKHeader = 40;
+static_assert(kTopKMax <= kTopKSegment / 16 && kTopKThresholdSegments <= 1024 && 1 + 64 + 4 + 1 <= 2 * kTopKHeader && 2 * kTopKHeader <= 256, "tickets");
 template <int V>
 __global__ __launch_bounds__(256) void topk_segment_max_kernel(const unsigned long long* __restrict__ in, int64_t count,
                                                                unsigned long long* __restrict__ segmax, uint32_t* counter) {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t segment = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     const int64_t begin = segment * (kWave * V);
-    if (blockIdx.x == 0 && threadIdx.x < 2) counter[threadIdx.x] = 0;  // candidates; workgroups past the first round
+    if (blockIdx.x == 0 && threadIdx.x < kTopKHeader * 2) counter[threadIdx.x] = 0;  // candidates, then the tickets of the tree
     if (begin >= count) return;
     unsigned long long m = 0;
 #pragma unroll
@@ -376,32 +382,32 @@ __global__ __launch_bounds__(256) void topk_filter_kernel(const unsigned long lo
 // The candidates are distinct unless the input repeats a value, so an entry's place in the output is the number
 // of candidates above it (equal values take consecutive places in list order).
 __global__ __launch_bounds__(256) void topk_finish_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                          uint32_t* counter, const unsigned long long* __restrict__ cand,
-                                                          unsigned long long* __restrict__ out, unsigned long long* round1,
-                                                          unsigned long long* round2) {
+                                                          const uint32_t* counter, const unsigned long long* __restrict__ cand,
+                                                          unsigned long long* __restrict__ out, unsigned long long* tree,
+                                                          uint32_t* tickets) {
     const uint32_t n = *counter;
     if (n > (uint32_t)kTopKCandidates) {
-        const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-        topk_reduce_segment(in, count, top_k, round1, (int64_t)blockIdx.x * 4 + wave, lane);
-        __shared__ uint32_t arrived;
-        __threadfence();  // this workgroup's share of round1 is visible before its ticket is
-        __syncthreads();
-        if (threadIdx.x == 0) arrived = atomicAdd(counter + 1, 1u);
-        __syncthreads();
-        if (arrived + 1 != gridDim.x) return;
-        __threadfence();
-        unsigned long long *from = round1, *to = round2;
-        int64_t left = (count + kTopKSegment - 1) / kTopKSegment * top_k;
+        // A tree of lists: every wavefront reduces its segment, and the one that completes the children of a node (as many
+        // lists as fill a segment) reduces those too and goes on from there.  Every list has a place of its own.
+        const int lane = threadIdx.x & (kWave - 1), fan = kTopKSegment / top_k;
+        int64_t lists = (count + kTopKSegment - 1) / kTopKSegment, at = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+        if (at >= lists) return;
+        topk_reduce_segment(in, count, top_k, tree, at, lane);
         while (true) {
-            const int64_t segments = (left + kTopKSegment - 1) / kTopKSegment;
-            unsigned long long* const dst = segments == 1 ? out : to;
-            for (int64_t s = wave; s < segments; s += 4) topk_reduce_segment(from, left, top_k, dst, s, lane);
-            if (segments == 1) return;
-            __threadfence_block();
-            __syncthreads();
-            to = from;
-            from = dst;
-            left = segments * top_k;
+            const int64_t node = at / fan, first = node * fan, nodes = (lists + fan - 1) / fan;
+            const int children = (int)(lists - first < fan ? lists - first : fan);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // this wavefront's list is visible before its ticket is
+            uint32_t before = 0;
+            if (lane == 0) before = atomicAdd(tickets + node, 1u);
+            if (__builtin_amdgcn_readfirstlane((int)before) + 1 != children) return;
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            unsigned long long* const dst = nodes == 1 ? out : tree + lists * top_k;
+            topk_reduce_segment(tree + first * top_k, (int64_t)children * top_k, top_k, dst + node * top_k, 0, lane);
+            if (nodes == 1) return;
+            tree = dst;
+            tickets += nodes;
+            lists = nodes;
+            at = node;
         }
     }
     if (blockIdx.x != 0) return;
@@ -446,16 +452,22 @@ static int topk_threshold_per_lane(int64_t count, int top_k) {
     return 0;
 }
 
-constexpr int kTopKHeader = 2;  // scratch[0]: candidate counter, workgroups past the first round
+// Entries of the tree of lists (topk_finish_kernel; the last list is the call's output).
+static int64_t topk_tree_entries(int64_t count, int top_k) {
+    const int64_t fan = kTopKSegment / top_k;
+    int64_t total = 0;
+    for (int64_t lists = topk_segments(count); lists > 1; lists = (lists + fan - 1) / fan) total += lists * top_k;
+    return total;
+}
 
 size_t packed_topk_scratch_entries(int64_t count, int top_k) {
     if (count <= kTopKSegment) return 0;
     // first round's output, then the second round's beside it (every later round is smaller)
     const int64_t c1 = topk_segments(count) * top_k;
     const int64_t c2 = c1 > kTopKSegment ? topk_segments(c1) * top_k : 0;
-    int64_t total = c1 + c2;
-    if (topk_threshold_per_lane(count, top_k)) total += kTopKHeader + kTopKThresholdSegments + kTopKCandidates;
-    return (size_t)total;
+    if (topk_threshold_per_lane(count, top_k))
+        return (size_t)(topk_tree_entries(count, top_k) + kTopKHeader + kTopKThresholdSegments + kTopKCandidates);
+    return (size_t)(c1 + c2);
 }
 
 template <int V>
@@ -477,8 +489,7 @@ hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int t
     const unsigned long long* src = in;
     int64_t n = count;
     if (const int per_lane = topk_threshold_per_lane(count, top_k)) {
-        const int64_t c2 = c1 > kTopKSegment ? topk_segments(c1) * top_k : 0;
-        unsigned long long* extra = scratch + c1 + c2;
+        unsigned long long* extra = scratch + topk_tree_entries(count, top_k);
         uint32_t* counter = reinterpret_cast<uint32_t*>(extra);
         unsigned long long* segmax = extra + kTopKHeader;
         unsigned long long* cand = segmax + kTopKThresholdSegments;
@@ -486,7 +497,7 @@ hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int t
         else if (per_lane == 4) topk_threshold_launch<4>(in, count, top_k, segmax, counter, cand, stream);
         else topk_threshold_launch<1>(in, count, top_k, segmax, counter, cand, stream);
         hipLaunchKernelGGL(topk_finish_kernel, dim3((unsigned)((first + 3) / 4)), dim3(256), 0, stream, in, count, top_k, counter,
-                           cand, out, bufs[0], bufs[1]);
+                           cand, out, scratch, counter + 1);
         return hipGetLastError();
     }
     while (true) {

@@ -187,6 +187,32 @@ def test_packed_topk_arranged_inputs(ctx, shape, count, top_k):
     dout.free()
 
 
+@pytest.mark.parametrize("count,top_k", [(1048571, 64), (700001, 33), (1048576, 50), (262144, 1), (263000, 64), (17000, 64), (30000, 7)])
+def test_packed_topk_tree_of_lists(ctx, count, top_k):
+    """More entries than the threshold path orders in one workgroup: two to four levels of lists, the last node of each short,
+    replayed from a graph over inputs that take it and one that does not."""
+    say("packed topk, tree", count, top_k)
+    rng = np.random.default_rng(count + top_k)
+    idx = np.arange(count, dtype=np.uint64)
+    inputs = [((np.uint64(0x80000000) + idx) << np.uint64(32)) | (np.uint64(0xFFFFFFFF) - idx), rng.integers(1, 2 ** 63, count, dtype=np.uint64),
+              np.full(count, 5 << 40, np.uint64)]
+    din, dout = ctx.to_device(inputs[0]), ctx.alloc(top_k * 8)
+    ctx.packed_topk(din, count, top_k, dout)
+    ctx.sync()
+    ctx.capture_begin()
+    ctx.packed_topk(din, count, top_k, dout)
+    graph = ctx.capture_end()
+    for packed in inputs + inputs[:2]:
+        din.upload(packed)
+        ctx.fill_zero(dout)
+        ctx.graph_launch(graph)
+        ctx.sync()
+        assert np.array_equal(_u64(dout, top_k), np.sort(packed)[::-1][:top_k])
+    ctx.graph_destroy(graph)
+    din.free()
+    dout.free()
+
+
 def test_head_top_k_pipeline_and_errors(ctx, orc):
     """scores -> top-k: the k best tokens of the projection, in order, without the logits leaving the device."""
     import aq_mi355
