@@ -1007,8 +1007,9 @@ int aq_reserve_workspace_bytes(aq_ctx* ctx, size_t bytes) {
 
 size_t aq_workspace_bytes(aq_ctx* ctx) {
     if (!ctx) return 0;
+    std::lock_guard<std::mutex> host_lk(ctx->host_mu);
     std::lock_guard<std::mutex> lk(ctx->mu);
-    return ctx->ws.bytes + ctx->head_ws.bytes;
+    return ctx->ws.bytes + ctx->head_ws.bytes + (ctx->host ? ctx->host->device_bytes() : 0);
 }
 
 namespace {

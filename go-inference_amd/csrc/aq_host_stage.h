@@ -30,6 +30,8 @@ public:
     void widen(float* out, const uint16_t* in, size_t n);
     // Ends a call (the stream has been waited for): a device block larger than what is kept between calls is freed.
     void finish();
+    // Device memory kept between calls.
+    size_t device_bytes() const { return dev_bytes_; }
 
 private:
     struct Pool;

@@ -177,8 +177,9 @@ int aq_reserve_workspace(aq_ctx *ctx, int M, int K);
  * more than is there grows it (not possible while a capture is open): run such a call once before capturing,
  * or reserve its bytes here. */
 int aq_reserve_workspace_bytes(aq_ctx *ctx, size_t bytes);
-/* Device bytes the context holds as scratch right now (the workspace above plus the partial maxima of
- * aq_qmv_greedy): lets a caller, or a test, see whether a call made either of them grow.  No reference counterpart. */
+/* Device bytes the context holds as scratch right now (the workspace above, the partial maxima of
+ * aq_qmv_greedy, and the block that host-slice calls upload to, of which up to 256 MB stay between calls): lets a caller, or a
+ * test, see whether a call made any of them grow.  No reference counterpart. */
 size_t aq_workspace_bytes(aq_ctx *ctx);
 
 /* gather_qmv: for each route z, y[z,:N] = x[lhs[z] or 0, :K] . dequant(W_e)^T with

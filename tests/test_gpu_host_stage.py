@@ -66,3 +66,18 @@ def test_nan_activations_stay_nan(ctx):
     x[1, 0] = 1.0
     y = ctx.proj_quant_matmul_host(x, words, s, b, 2, K, N, 64, 4)
     assert np.isnan(y[0]).all() and np.isfinite(y[1]).all()
+
+
+def test_kept_device_block_is_counted():
+    import aq_mi355
+    say("host slices, bytes held")
+    c = aq_mi355.Context(0)
+    try:
+        K, held = 2048, [c.workspace_bytes()]
+        for N in (512, 4096, 100):
+            words, s, b = F.synthetic_affine(N, K, 4, 64, seed=3300 + N)
+            c.matvec_host(F.synthetic_x(1, K, seed=3301), words, s, b, N, K, 64, 4)
+            held.append(c.workspace_bytes())
+        assert held[1] - held[0] >= 512 * K // 2 and held[2] - held[0] >= 4096 * K // 2 and held[3] == held[2]
+    finally:
+        c.close()
