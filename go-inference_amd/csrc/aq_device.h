@@ -87,25 +87,38 @@ __device__ __forceinline__ void unpack8_word(uint32_t w, uint32_t p[2]) {
     p[1] = __builtin_amdgcn_perm(f3, f2, 0x07060302u);
 }
 
-// The same with the codes centred on zero, for sums that must not lose what the bias takes off again: 16 * (code - 8) of the
-// eight 4-bit codes in the order of unpack4_word (a signed nibble in the upper half of a byte), code - 128 of four 8-bit codes.
-// Both have at most 8 significant bits: exact in bf16.
-__device__ __forceinline__ uint32_t signed_bytes_to_bf16(uint32_t w, int i, int j) {
-    const float f = (float)(int8_t)(w >> (8 * i)), g = (float)(int8_t)(w >> (8 * j));
-    return __builtin_amdgcn_perm(__float_as_uint(g), __float_as_uint(f), 0x07060302u);
+// The same as 16 + code, exact as well: one shift more, and an eighth of the part that comes off again.
+constexpr uint32_t kMask16 = 0x00780078u;   // a nibble moved to mantissa bits [6:3]
+constexpr uint32_t kMagic16 = 0x41804180u;  // bf16 16.0 in both halves
+__device__ __forceinline__ uint4 unpack_word4(uint32_t w, uint32_t mask_s, uint32_t magic_v) {
+    uint4 v;
+    v.x = and_or(w << 3, mask_s, magic_v);
+    v.y = and_or(w >> 1, mask_s, magic_v);
+    v.z = and_or(w >> 5, mask_s, magic_v);
+    v.w = and_or(w >> 9, mask_s, magic_v);
+    return v;
+}
+
+// Codes centred on zero, for sums that must not lose what the bias takes off again: (code - 8) / 16 of the eight 4-bit codes in
+// the order of unpack4_word, code - 128 of four 8-bit codes.  Both have at most 8 significant bits: exact in bf16.
+__device__ __forceinline__ uint32_t high_halves(float lo, float hi) {
+    return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
 }
 __device__ __forceinline__ void unpack4_centred(uint32_t w, uint32_t p[4]) {
-    w ^= 0x88888888u;
-    const uint32_t even = (w << 4) & 0xf0f0f0f0u, odd = w & 0xf0f0f0f0u;
-    p[0] = signed_bytes_to_bf16(even, 0, 2);
-    p[1] = signed_bytes_to_bf16(odd, 0, 2);
-    p[2] = signed_bytes_to_bf16(even, 1, 3);
-    p[3] = signed_bytes_to_bf16(odd, 1, 3);
+    w ^= 0x88888888u;  // signed nibbles
+    uint32_t odd = w >> 4;
+    asm("" : "+v"(odd));  // (or eight shifts take the place of the byte selections)
+    auto at = [](uint32_t v, int byte) { return __builtin_amdgcn_cvt_off_f32_i4(byte ? (int)((v >> (8 * byte)) & 0xffu) : (int)v); };
+    p[0] = high_halves(at(w, 0), at(w, 2));
+    p[1] = high_halves(at(odd, 0), at(odd, 2));
+    p[2] = high_halves(at(w, 1), at(w, 3));
+    p[3] = high_halves(at(odd, 1), at(odd, 3));
 }
 __device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
-    w ^= 0x80808080u;
-    p[0] = signed_bytes_to_bf16(w, 0, 1);
-    p[1] = signed_bytes_to_bf16(w, 2, 3);
+    w ^= 0x80808080u;  // signed bytes
+    auto at = [&](int byte) { return (float)(int8_t)(w >> (8 * byte)); };
+    p[0] = high_halves(at(0), at(1));
+    p[1] = high_halves(at(2), at(3));
 }
 
 // scale * code + bias in two roundings.

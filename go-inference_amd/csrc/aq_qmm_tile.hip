@@ -35,19 +35,6 @@ namespace aq {
 
 namespace {
 
-constexpr uint32_t kMask16 = 0x00780078u;   // a nibble moved to mantissa bits [6:3]
-constexpr uint32_t kMagic16 = 0x41804180u;  // bf16 16.0 in both halves: 16 + code, exact
-
-// 8 codes of one packed word -> 8 bf16 (16 + c) in slot order (c0,c4)(c1,c5)(c2,c6)(c3,c7)
-__device__ __forceinline__ uint4 unpack_word4(uint32_t w, uint32_t mask_s, uint32_t magic_v) {
-    uint4 v;
-    v.x = and_or(w << 3, mask_s, magic_v);
-    v.y = and_or(w >> 1, mask_s, magic_v);
-    v.z = and_or(w >> 5, mask_s, magic_v);
-    v.w = and_or(w >> 9, mask_s, magic_v);
-    return v;
-}
-
 __device__ __forceinline__ uint4 unpack_words8(uint32_t w0, uint32_t w1) {
     uint32_t p[4];
     unpack8_word(w0, p);

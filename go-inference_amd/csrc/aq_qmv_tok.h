@@ -89,15 +89,17 @@ __host__ __device__ constexpr int tok16_stage_pieces(int nw) { return nw >= 16 ?
 // its four FMAs, and the affine term is two MFMAs per run.  8-bit codes: a lane's 16 codes lie in one group, but the step
 // of 32 codes that is group 0 of a block of 64 has to come from lane blocks 0 and 1 alone: a swap of 32-lane halves
 // between the two steps' registers moves the second 8 codes of those lanes to lane blocks 2 and 3 (x takes the same swap).
-// The operand of these forms holds the codes centred on zero, 16 (code - 8) or code - 128 (aq_device.h), and the affine term
-// bias + 8 scale (128 scale): a weight is near zero on average, and what 128 + code has beside it comes off again out of sums
-// 28 times the result (21 x 3840 x 512, groups of 32: 2.1e-6 from the float64 product, centred 1.0e-7, the any-width kernel
-// that this shape had 0.9e-7; 8 bit 1.6e-7 -> 1.0e-7, any-width 1.35e-7).  It costs 16 vector instructions a word instead of 7:
-// a layer of 21 rows (3840 / 15360, groups of 32) 97.7 -> 103.4 us (104.5 with the
-// test of every sum of dense groups of 32 for infinities, which the any-width kernel keeps: see plain_dot_g32).
-// Measured (graph replay, weights from HBM): 21 x 3840 x 15360 in groups of 32 19.4 us (the any-width kernel this shape had:
-// 0.48 ms a matrix), 32 x 4096 x 14336 21.0 us against 16.9 us for groups of 64: four more FMAs a lane per 32 codes; 32 x
-// 4032 x 14336 18.9 us, 2 us over whole runs for the element-wise staging.
+// What the operand holds of a code, and why.  A weight is near zero on average: what 128 + code has beside it comes off again,
+// in the affine term, out of sums 28 times the result.  Errors against the float64 product (fp32 results, relative; in brackets
+// the kernels these shapes had before this one): 4 bit, groups of 32 2.1e-6 with 128 + code, 1.0e-7 with (code - 8) / 16 (3..4
+// rows 8.3e-7, more rows 0.9e-7); groups of 64 and 128 1.8e-6, 2.8e-7 with 16 + code (5..16 rows 8.3e-7, more 1.2e-5); 8 bit
+// 1.6e-7 with the code, 0.9-1.0e-7 with code - 128 (0.9-1.4e-7).  Vector instructions per word of 4-bit codes: 7, 8 for 16 +
+// code, 14 for (code - 8) / 16, which is therefore only where groups of 32 need it.
+// Measured (us, graph replay over 640 MB of weights; 128 + code or the plain 8-bit code -> here): 21 x 3840 x 15360 in groups of
+// 32 20.4 -> 21.9 (the any-width kernel this shape had: 0.48 ms a matrix), 32 x 4096 x 14336 21.5 -> 23.0 against 16.8 for groups
+// of 64: four more FMAs a lane per 32 codes; 32 x 4032 x 14336 in groups of 64 18.4 -> 18.7, 2 us over whole runs for the
+// element-wise staging; 16 x 4032 x 14336 13.6 -> 13.7, 8 bit 17.6 -> 17.8; 12 x 4096 x 14336 in groups of 128 12.3 -> 12.5.
+// Dense groups of 32 also test every sum for infinities, which the any-width kernel keeps (plain_dot_g32).
 // PAIR: the first half of the workgroup's sets of rows belongs to the gate matrix, the second half to the same rows of the
 // up matrix, and the store is act(gate) * up: one pass over x and one launch for a gated MLP's two projections.
 // GROUPED (expert slabs): the rows of x of a launch are the routes of one chunk of the list a.chunks (aq_moe_group.hip):
@@ -108,7 +110,10 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
     static_assert(GRP == 64 || (GRP == 32 && ANY), "group size");
     constexpr bool G32 = GRP == 32;
     constexpr int GPR = 256 / GRP;  // groups of a run
-    constexpr bool CENTRED = ANY;   // the operand's codes: 16 (code - 8) or code - 128, else 128 + code or code
+    // what the operand holds of a code: 4 bit 128 + code; ANY 16 + code, in groups of 32 (code - 8) / 16; 8 bit code; ANY code - 128
+    constexpr bool CENTRED = BITS == 8 ? ANY : G32;
+    constexpr float kUnit = CENTRED && BITS == 4 ? 1.0f / 16 : 1.0f;
+    constexpr float kLacks = CENTRED ? (BITS == 4 ? 8.0f : 128.0f) : BITS == 8 ? 0.0f : ANY ? -16.0f : -128.0f;  // in codes
     static_assert(!PAIR || RS % 2 == 0, "a pair shares its sets of rows between two matrices");
     constexpr int PAIRS = PAIR ? 2 : 1;
     constexpr int LINES = BITS / 4;  // 128-byte lines of a row per run of 256 codes
@@ -166,8 +171,8 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
                              (BITS == 4 ? (uint32_t)(n >> 3) * 64u + (uint32_t)q * 16u   // step pair: first 64 bytes | second
                                         : (uint32_t)q * 32u + (uint32_t)(n >> 3) * 16u);  // group: first 16 of the lane's 32 | second
 
-    const uint32_t mask = opaque_s(kNibbleMask);
-    const uint32_t magic = opaque_v(kMagic128);
+    const uint32_t mask = opaque_s(ANY ? kMask16 : kNibbleMask);
+    const uint32_t magic = opaque_v(ANY ? kMagic16 : kMagic128);
     const uint32_t ones = 0x3f803f80u;
     // picks element q of four bf16 values in two registers, twice
     const uint32_t sel_q = 0x01000100u + 0x02020202u * (uint32_t)q;
@@ -416,18 +421,15 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
             transpose(t0, t1, t2, t3);
             float X = (__uint_as_float(t0) + __uint_as_float(t1)) + (__uint_as_float(t2) + __uint_as_float(t3));
             if (!live[j]) X = 0.0f;
-            constexpr float kUnit = CENTRED && BITS == 4 ? 16.0f : 1.0f;  // what the operand has 1 of a code as
             X *= kUnit;
             const uint32_t u0 = __float_as_uint(X) & 0xffff0000u;
             const float r1 = X - __uint_as_float(u0);
             const uint32_t u1 = __float_as_uint(r1) & 0xffff0000u;
             const float r2 = r1 - __uint_as_float(u1);
             const uint32_t u2 = __float_as_uint(r2) & 0xffff0000u;
-            // what the operand's codes lack of the codes
-            const float off = CENTRED ? (BITS == 4 ? 8.0f : 128.0f) : BITS == 4 ? -128.0f : 0.0f;
-            const uint32_t m0 = __float_as_uint(off * __uint_as_float(u0));
-            const uint32_t m1 = __float_as_uint(off * __uint_as_float(u1));
-            const uint32_t m2 = __float_as_uint(off * __uint_as_float(u2));
+            const uint32_t m0 = __float_as_uint(kLacks * __uint_as_float(u0));
+            const uint32_t m1 = __float_as_uint(kLacks * __uint_as_float(u1));
+            const uint32_t m2 = __float_as_uint(kLacks * __uint_as_float(u2));
             a2[ts][j][g4] = as_bf16x8((u0 >> 16) | u1, (u2 >> 16) | m0, (m1 >> 16) | m2, 0u);
             }
         }
@@ -491,6 +493,9 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
                         uint32_t e[4];
                         if constexpr (BITS == 4 && CENTRED) {
                             unpack4_centred(ww[2 * g + half], e);
+                        } else if constexpr (BITS == 4 && ANY) {
+                            const uint4 v = unpack_word4(ww[2 * g + half], mask, magic);
+                            e[0] = v.x, e[1] = v.y, e[2] = v.z, e[3] = v.w;
                         } else if constexpr (BITS == 4) {
                             unpack4_word(ww[2 * g + half], mask, magic, e);
                         } else if constexpr (CENTRED) {
@@ -572,7 +577,7 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
         float total = red[t * TSTRIDE + column];
 #pragma unroll
         for (int p = 1; p < NW; p++) total += red[(p * 16 * TS + t) * TSTRIDE + column];
-        return CENTRED && BITS == 4 ? total * 0.0625f : total;
+        return kUnit != 1.0f ? total * (1.0f / kUnit) : total;
     };
     for (int o = tid; o < 16 * TS * OUTS; o += NW * kWave) {
         const int t = o / OUTS, rl = o - t * OUTS;
