@@ -333,14 +333,20 @@ int run_diag(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool g
     return kPass;
 }
 
-// Groups of 64 with a K that ends inside a run of 256 codes: matrices of fewer than 4 Mi codes stay with the families behind
-// (a workgroup per 16 rows does not fill the chip then, and its fixed cost is what is left).
-bool tok_small(int group_size, int K, int64_t rows) { return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20; }
+// Groups of 64 with a K that ends inside a run of 256 codes: calls on matrices of fewer than 4 Mi codes that stay with the
+// families behind.  8 bit: up to four rows, where the dot2 kernels are ahead (us, dot2 / here: 2 rows of 960 x 512 2.8 / 4.5, of
+// 4032 x 1024 4.4 / 6.7; 4 rows 3.2 / 4.5, 5.8 / 7.0); from five rows on what is behind are tiles, a pass over x and a sum of
+// shares of K in three launches (8 rows 14.6 / 4.6, 17.6 / 7.3; 32 rows 15.0 / 6.7, 18.1 / 11.9).  4 bit: up to 528 rows of
+// weights; the tiles are behind there as well (9 rows of x by 960 x 512 13.6 / 4.6, by 960 x 2048 14.3 / 4.6, 32 by 4032 x 1024
+// 17.4 / 11.1), but the choice for those sizes is one that tests/test_gpu_selection.py states.
+bool tok_small(int bits, int group_size, int M, int K, int64_t rows) {
+    return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20 && (bits == 8 ? M <= 4 : rows <= 528);
+}
 
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
     const int ti = forced >= 0 ? forced : aq::qmvt_pick(bits, a.M, a.K, a.N, ctx->cu_count);
     if (gather || ti < 0 || !aq::qmvt_fits(a, bits, group_size, ti, forced >= 0)) return kPass;
-    if (forced < 0 && tok_small(group_size, a.K, a.N)) return kPass;
+    if (forced < 0 && tok_small(bits, group_size, a.M, a.K, a.N)) return kPass;
     ctx->last_variant[0] = aq::qmvt_name(ti, a);
     AQ_HIP(aq::qmvt_launch(ti, a, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
@@ -397,7 +403,7 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
 // Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
 // the launch forms that put several matrices into one grid).
 bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows) {
-    if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(group_size, K, rows)) return false;
+    if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(bits, group_size, M, K, rows)) return false;
     if (bits == 4 && group_size == 64) return M >= 9 && M <= 32;
     if (bits == 8 && group_size == 64) return (M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0) && M >= 2 && M <= 32;
     return M <= 32 && M >= (group_size == 128 ? 5 : bits == 4 ? 3 : 2);

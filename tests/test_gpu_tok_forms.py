@@ -12,6 +12,8 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(bits, 32, M, K, N) for bits in (4, 8) for M, K, N in ((3, 64, 40), (16, 192, 1030), (17, 320, 70), (32, 4096, 16), (9, 4032, 130))]
 SHAPES += [(bits, 128, M, K, N) for bits in (4, 8) for M, K, N in ((5, 128, 33), (16, 2944, 66), (32, 4096, 49))]
 SHAPES += [(bits, 64, M, K, N) for bits in (4, 8) for M, K, N in ((9, 960, 4400), (16, 2112, 2001), (32, 4032, 1056))]
+# small matrices with such a K, from the first size that runs here
+SHAPES += [(4, 64, 9, 320, 529), (4, 64, 32, 4160, 600), (8, 64, 5, 64, 1), (8, 64, 5, 320, 24), (8, 64, 32, 4160, 48)]
 
 
 @pytest.mark.parametrize("bits,gs,M,K,N", SHAPES)
