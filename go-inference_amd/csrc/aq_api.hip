@@ -968,15 +968,14 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         half_need = aq::qmm_scratch_bytes(M, K, 0, ctx->cu_count) + aq::qmmh_partial_bytes(q);
     }
     // the largest scratch first, so that no member makes the workspace move under the pass over x (groups of 32 do without:
-    // the grid asks for its own, and the any-width kernel runs members that cannot have it)
-    if (group_size != 32 && !(q.nseg == count && !aq::workspace_may_grow(&ctx->ws, half_need, ctx->stream))) {
-        const int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, half_need > need ? half_need : need, fail);
-        if (rc == AQ_ERR_NOMEM) {
-            in_grid = 0;  // one member at a time, each with the scratch it can have
-            q.nseg = 0;
-        } else if (rc != AQ_OK) {
-            return rc;
-        }
+    // the grid asks for its own, and the any-width kernel runs members that cannot have it).  Where it is not to be had (the
+    // stream is being captured, or there is no memory) the members run with what there is, one by one if need be.
+    if (group_size != 32) {
+        const size_t most = half_need > need ? half_need : need;
+        int rc = AQ_ERR_NOMEM;
+        if (aq::workspace_may_grow(&ctx->ws, most, ctx->stream)) rc = aq::workspace_reserve(ctx->stream, &ctx->ws, most, fail);
+        if (rc != AQ_OK && rc != AQ_ERR_NOMEM) return rc;
+        if (ctx->ws.bytes < half_need) in_grid = 0, q.nseg = 0;
     }
     int x_state = aq::kXReadyNone;
     if (q.nseg > 0) {

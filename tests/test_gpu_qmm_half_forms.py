@@ -143,3 +143,46 @@ def test_reserved_by_rows_and_columns_a_call_is_captured_on_its_kernels(bits, gs
             t.free()
     finally:
         fresh.close()
+
+
+@pytest.mark.parametrize("bytes_too", [0, 1 << 20])
+def test_several_matrices_captured_after_reserving(bytes_too):
+    """aq_qmm_multi in a graph: with room for one matrix at a time (aq_reserve_workspace) or only for the copy of x and small
+    shares of K, every member has the bytes of its own eager call or the call is refused, and nothing allocates."""
+    import aq_mi355
+    M, K, Ns = 200, 4096, (4096, 1024, 520)
+    say("qmm multi in a graph", bytes_too)
+    fresh = aq_mi355.Context(0)
+    try:
+        x = F.synthetic_x(M, K, seed=2730)
+        dws = [DeviceAffine(fresh, *F.synthetic_affine(n, K, 4, 64, seed=2731 + i)) for i, n in enumerate(Ns)]
+        dx, ys = fresh.to_device(x), [fresh.alloc(M * n * 4) for n in Ns]
+        if bytes_too:
+            fresh.reserve_workspace_bytes(M * K * 2 + bytes_too)
+        else:
+            fresh.reserve_workspace(M, K)
+        held = fresh.workspace_bytes()
+        call = lambda: fresh.qmm_multi(dx, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, list(Ns), M, K, 64, 4, aq_mi355.AQ_OUT_F32)
+        fresh.capture_begin()
+        refused = False
+        try:
+            call()
+        except aq_mi355.AqError as e:
+            assert bytes_too and e.code == aq_mi355.AQ_ERR_UNSUPPORTED
+            refused = True
+        graph = fresh.capture_end()
+        assert fresh.workspace_bytes() == held and refused == bool(bytes_too)
+        if not refused:
+            for _ in range(3):
+                for y in ys:
+                    fresh.fill_zero(y)
+                fresh.graph_launch(graph)
+                fresh.sync()
+                got = [y.download(np.uint32) for y in ys]
+                for d, n, one in zip(dws, Ns, got):
+                    assert np.array_equal(run_qmv(fresh, x, d, M, K, n, 64, 4, True, fn="qmm").view(np.uint32).reshape(-1), one)
+        fresh.graph_destroy(graph)
+        for t in [dx] + ys + dws:
+            t.free()
+    finally:
+        fresh.close()
