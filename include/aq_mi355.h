@@ -166,7 +166,7 @@ int aq_qmm_multi(aq_ctx *ctx, const void *x, int count, const void *const *packe
  * tiles of a matrix leave CUs idle, the fp32 partial tiles of shares of K.  The workspace grows on demand, which
  * drains the stream and allocates: not allowed while a capture is open and unwelcome in a serving
  * loop.  This call sizes it ahead of time for one matrix of any N and activations of up to M x K (the copy and at most
- * 16 KiB * min(M, 256) * CUs of partial tiles: 268 MB at M >= 256 on 256 CUs).  The reference sizes its
+ * 4 KiB * min(M, 256) * CUs of partial tiles: 268 MB at M >= 256 on 256 CUs).  The reference sizes its
  * own scratch the same way at model load (hipMLXQ4DeviceWeightConfig and the batch scratch of
  * go/engine/hip/hip_projection_launch.go:2671-2720). */
 int aq_reserve_workspace(aq_ctx *ctx, int M, int K);
