@@ -82,11 +82,25 @@ struct aq_ctx {
     void* head_fold = nullptr;     // aq_qmv_greedy's fold tickets and slots (aq::kHeadFoldBytes, kept zeroed by the kernel)
     unsigned char* static_scratch = nullptr;  // this device's copy of `scratch` (hipGetSymbolAddress at creation)
     char name[256] = {0};
+    bool leaves_streams = false;  // a caller's stream has been left: uses of the scratch blocks on such streams are noted
     std::mutex host_mu;     // one staged host call at a time
     aq::HostStage* host = nullptr;
 };
 
 namespace {
+
+// The context's lock, held while a call selects and launches.  What the call gave a caller's stream to do over the scratch
+// blocks is noted before the lock is let go: another call may leave that stream, and its owner destroy it, right after.
+struct CallLock {
+    aq_ctx* ctx;
+    std::lock_guard<std::mutex> held;
+    explicit CallLock(aq_ctx* c) : ctx(c), held(c->mu) {}
+    ~CallLock() {
+        if (ctx->stream == ctx->own_stream) return;
+        (void)aq::workspace_note(ctx->stream, &ctx->ws, ctx->leaves_streams);
+        (void)aq::workspace_note(ctx->stream, &ctx->head_ws, ctx->leaves_streams);
+    }
+};
 
 // Widths every path accepts (MLX affine widths the reference dispatches,
 // go/model/quant_weight.go:11-13); 1-bit packs are widened to 2-bit by the
@@ -537,21 +551,27 @@ int go_to_stream(aq_ctx* ctx, hipStream_t stream) {
     const hipStream_t old = ctx->stream;
     ctx->stream = stream;
     if (stream == old) return AQ_OK;
-    const hipError_t rc = aq::workspace_leave(old, &ctx->ws), rc_head = aq::workspace_leave(old, &ctx->head_ws);
-    if (rc != hipSuccess || rc_head != hipSuccess) return hip_fail(rc != hipSuccess ? rc : rc_head, "hipEventRecord");
-    return AQ_OK;
+    hipError_t first = hipSuccess;
+    for (aq::Workspace* ws : {&ctx->ws, &ctx->head_ws}) {
+        hipError_t rc = old == ctx->own_stream ? aq::workspace_note(old, ws) : hipSuccess;  // (others: CallLock)
+        const hipError_t left = aq::workspace_leave(ws);
+        rc = rc == hipSuccess ? left : rc;
+        first = first == hipSuccess ? rc : first;
+    }
+    ctx->leaves_streams = ctx->leaves_streams || old != ctx->own_stream;
+    return first == hipSuccess ? AQ_OK : hip_fail(first, "hipEventRecord");
 }
 }  // namespace
 
 int aq_use_stream(aq_ctx* ctx, void* hip_stream) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_use_stream: ctx is null");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     return go_to_stream(ctx, static_cast<hipStream_t>(hip_stream));
 }
 
 int aq_use_own_stream(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_use_own_stream: ctx is null");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     return go_to_stream(ctx, ctx->own_stream);
 }
 
@@ -580,7 +600,7 @@ int aq_free(aq_ctx* ctx, void* dptr) {
 int aq_h2d(aq_ctx* ctx, void* dst_dev, const void* src_host, size_t bytes) {
     if (!ctx || (bytes && (!dst_dev || !src_host))) return fail(AQ_ERR_ARG, "aq_h2d: bad argument");
     if (!bytes) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipMemcpyAsync(dst_dev, src_host, bytes, hipMemcpyHostToDevice, ctx->stream), "hipMemcpyHtoD");
     AQ_HIP(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     return AQ_OK;
@@ -589,7 +609,7 @@ int aq_h2d(aq_ctx* ctx, void* dst_dev, const void* src_host, size_t bytes) {
 int aq_d2h(aq_ctx* ctx, void* dst_host, const void* src_dev, size_t bytes) {
     if (!ctx || (bytes && (!dst_host || !src_dev))) return fail(AQ_ERR_ARG, "aq_d2h: bad argument");
     if (!bytes) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipMemcpyAsync(dst_host, src_dev, bytes, hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyDtoH");
     AQ_HIP(hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     return AQ_OK;
@@ -598,7 +618,7 @@ int aq_d2h(aq_ctx* ctx, void* dst_host, const void* src_dev, size_t bytes) {
 int aq_d2d(aq_ctx* ctx, void* dst_dev, const void* src_dev, size_t bytes) {
     if (!ctx || (bytes && (!dst_dev || !src_dev))) return fail(AQ_ERR_ARG, "aq_d2d: bad argument");
     if (!bytes) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipMemcpyAsync(dst_dev, src_dev, bytes, hipMemcpyDeviceToDevice, ctx->stream), "hipMemcpyDtoD");
     return AQ_OK;
 }
@@ -606,7 +626,7 @@ int aq_d2d(aq_ctx* ctx, void* dst_dev, const void* src_dev, size_t bytes) {
 int aq_fill_zero(aq_ctx* ctx, void* dptr, size_t bytes) {
     if (!ctx || (bytes && !dptr)) return fail(AQ_ERR_ARG, "aq_fill_zero: bad argument");
     if (!bytes) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::fill_zero_launch(dptr, bytes, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -619,14 +639,14 @@ int aq_sync(aq_ctx* ctx) {
 
 int aq_timer_start(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_timer_start: ctx is null");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipEventRecord(ctx->ev0, ctx->stream), "hipEventRecord");
     return AQ_OK;
 }
 
 int aq_timer_stop(aq_ctx* ctx, float* elapsed_ms) {
     if (!ctx || !elapsed_ms) return fail(AQ_ERR_ARG, "aq_timer_stop: bad argument");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipEventRecord(ctx->ev1, ctx->stream), "hipEventRecord");
     AQ_HIP(hipEventSynchronize(ctx->ev1), "hipEventSynchronize");
     AQ_HIP(hipEventElapsedTime(elapsed_ms, ctx->ev0, ctx->ev1), "hipEventElapsedTime");
@@ -654,10 +674,12 @@ struct aq_graph {
 
 int aq_capture_begin(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_capture_begin: ctx is null");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     if (ctx->stream == nullptr) return fail(AQ_ERR_UNSUPPORTED, "aq_capture_begin: the legacy default stream cannot be captured");
-    AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->ws), "hipEventRecord");
-    AQ_HIP(aq::workspace_leave(ctx->stream, &ctx->head_ws), "hipEventRecord");
+    for (aq::Workspace* ws : {&ctx->ws, &ctx->head_ws}) {
+        AQ_HIP(aq::workspace_note(ctx->stream, ws), "hipEventRecord");
+        AQ_HIP(aq::workspace_leave(ws), "hipDeviceSynchronize");
+    }
     AQ_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
     ctx->ws.touched = ctx->ws.required = ctx->head_ws.touched = ctx->head_ws.required = false;
     return AQ_OK;
@@ -666,7 +688,7 @@ int aq_capture_begin(aq_ctx* ctx) {
 int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
     if (!ctx || !out) return fail(AQ_ERR_ARG, "aq_capture_end: bad argument");
     *out = nullptr;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     hipGraph_t g = nullptr;
     AQ_HIP(hipStreamEndCapture(ctx->stream, &g), "hipStreamEndCapture");
     aq_graph* ag = new (std::nothrow) aq_graph();
@@ -688,7 +710,7 @@ int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
 
 int aq_graph_launch(aq_ctx* ctx, aq_graph* graph) {
     if (!ctx || !graph || !graph->exec) return fail(AQ_ERR_ARG, "aq_graph_launch: bad argument");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     if (graph->ws.stale(ctx->ws) || graph->head_ws.stale(ctx->head_ws))
         return fail(AQ_ERR_UNSUPPORTED,
                     "aq_graph_launch: the context's workspace was reallocated after this graph was captured (a later call "
@@ -714,7 +736,7 @@ int aq_probe_read(aq_ctx* ctx, const void* packed, const void* scales, const voi
     if (!packed || (mode != 2 && (!scales || !biases))) return fail(AQ_ERR_ARG, "aq_probe_read: null operand");
     if (!aligned(packed, 16) || !aligned(scales, 8) || !aligned(biases, 8))
         return fail(AQ_ERR_ARG, "aq_probe_read: packed must be 16-byte, scales and biases 8-byte aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::read_probe_launch(packed, scales, biases, N, K / 2, K / 32, mode, nullptr, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -735,7 +757,7 @@ int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, c
     if (!x || !packed || (!tiled && (!scales || !biases)) || !y) return fail(AQ_ERR_ARG, "aq_qmv: null operand");
     if (!aligned(x, 2) || !aligned(packed, 4) || !aligned(scales, 2) || !aligned(biases, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_qmv: operand pointer is not element-aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     aq::QmvArgs a{};
     a.x = static_cast<const uint16_t*>(x);
     a.w = static_cast<const uint32_t*>(packed);
@@ -815,7 +837,7 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         }
         fused = fused && total < (int64_t)1 << 30;
         if (fused) {
-            std::lock_guard<std::mutex> lk(ctx->mu);
+            CallLock lk(ctx);
             // the kernels aq_qmv would pick for each member, in one grid
             // (every variant with the same split of K computes the same bytes, whatever the rows per workgroup)
             const int di = (ctx->families_off >> kFamDiag & 1) ? -1 : aq::qmvd_pick(M, K, (int)total);
@@ -848,7 +870,7 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     int members = 0, ti = -1;
     aq::QmvMultiArgs grid{};
     if (tok) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
         grid.common = all.common;
@@ -875,7 +897,7 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         if (int rc = aq_qmv(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
     }
     if (in_grid) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
         AQ_HIP(aq::qmvt_multi_launch(ti, grid, ctx->stream), "hipLaunchKernel");
     }
@@ -891,7 +913,7 @@ int aq_qmm(aq_ctx* ctx, const void* x, const void* packed, const void* scales, c
     if (!x || !packed || !scales || !biases || !y) return fail(AQ_ERR_ARG, "aq_qmm: null operand");
     if (!aligned(x, 2) || !aligned(packed, 4) || !aligned(scales, 2) || !aligned(biases, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_qmm: operand pointer is not element-aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     if (M <= aq::kQmvMaxRows && ctx->forced[1] < 0) {
         // a matmul of up to four rows is a matvec: the matvec selection runs it (no pass over x, no workspace)
         aq::QmvArgs a{};
@@ -940,7 +962,7 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         ctx->last_variant[1] = ctx->last_variant[0];
         return AQ_OK;
     }
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     // the members that the fp16-operand kernels take run as one grid (same bytes as on their own, see qmmh_split): narrow
     // matrices (k and v beside q) then fill the rounds of tiles that the wide ones leave part-empty
@@ -997,7 +1019,7 @@ int aq_reserve_workspace(aq_ctx* ctx, int M, int K) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_reserve_workspace: ctx is null");
     if (M < 0 || K < 0) return fail(AQ_ERR_SHAPE, "aq_reserve_workspace: M and K must be non-negative");
     if (M == 0 || K == 0) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     return aq::qmm_reserve(ctx->stream, &ctx->ws, M, K, ctx->cu_count, fail);
 }
@@ -1005,7 +1027,7 @@ int aq_reserve_workspace(aq_ctx* ctx, int M, int K) {
 int aq_reserve_workspace_bytes(aq_ctx* ctx, size_t bytes) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_reserve_workspace_bytes: ctx is null");
     if (bytes == 0) return AQ_OK;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     return aq::workspace_reserve(ctx->stream, &ctx->ws, bytes, fail);
 }
@@ -1013,7 +1035,7 @@ int aq_reserve_workspace_bytes(aq_ctx* ctx, size_t bytes) {
 size_t aq_workspace_bytes(aq_ctx* ctx) {
     if (!ctx) return 0;
     std::lock_guard<std::mutex> host_lk(ctx->host_mu);
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     return ctx->ws.bytes + ctx->head_ws.bytes + (ctx->host ? ctx->host->device_bytes() : 0);
 }
 
@@ -1142,7 +1164,7 @@ int gather_call(aq_ctx* ctx, const void* x, const void* packed, const void* scal
         !aligned(rhs, 4) || (lhs && !aligned(lhs, 4)))
         return fail(AQ_ERR_ARG, "aq_gather_qmv: operand pointer is not element-aligned");
     if (routes > 65535) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv: at most 65535 routes per call");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     aq::QmvArgs a{};
     a.x = static_cast<const uint16_t*>(x);
     a.w = static_cast<const uint32_t*>(packed);
@@ -1203,7 +1225,7 @@ int aq_act_mul(aq_ctx* ctx, const void* gate, const void* up, void* y, int64_t n
     if (!gate || !up || !y) return fail(AQ_ERR_ARG, "aq_act_mul: null operand");
     if (!aligned(gate, 2) || !aligned(up, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_act_mul: operand pointer is not element-aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::act_mul_launch(static_cast<const uint16_t*>(gate), static_cast<const uint16_t*>(up),
                               static_cast<uint16_t*>(y), n, act, ctx->stream),
            "hipLaunchKernel");
@@ -1261,7 +1283,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, false, di) &&
             aq::qmvd_fits(up, bits, group_size, false, di) &&
             (size_t)M * K * 2 + (size_t)M * ((K + 255) / 256) * 48 + 128 + (size_t)2 * aq::qmvd_variant(di)->waves * 256 <= 96 * 1024) {
-            std::lock_guard<std::mutex> lk(ctx->mu);
+            CallLock lk(ctx);
             ctx->last_variant[0] = "qmv_gate_up_diag";
             AQ_HIP(aq::qmvd_pair_launch(di, a, false, ctx->stream), "hipLaunchKernel");
             return AQ_OK;
@@ -1272,7 +1294,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         // of the unfused route, which then runs as for any other call
         // (a pair's partial tiles are twice a single matrix's)
         const size_t region = 2 * qmm_region(ctx, M, K, N) + 2 * align256((size_t)M * N * 4);
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * untiled_bytes(N, K), fail)) return rc;
         const uint32_t* w[2];
@@ -1284,7 +1306,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     }
     if (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) &&
         aligned(up_packed, 16)) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 1, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 1, rows, false)) {
             aq::QmvArgs a{};
@@ -1326,7 +1348,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         a.out_f32 = out_f32 ? 1 : 0;
         a.routes = 1;
         a.act = act;
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const int ti = aq::qmvt_pick_pair(bits, M, K, N, ctx->cu_count);
         if (ti >= 0 && aq::qmvt_pair_supported(ti) && aq::qmvt_fits(a, bits, group_size, ti, false)) {
             ctx->last_variant[0] = "qmv_gate_up_tok";
@@ -1339,7 +1361,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         aq::qmmh_runs(M, K, N, group_size, bits)) {
         // prefill sizes on the fp16-operand kernels: one launch, the tiles of which hold gate and up columns side by side; no
         // intermediate reaches memory
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         aq::QmmHalfCall q{};
         q.x = static_cast<const uint16_t*>(x);
         q.M = M;
@@ -1366,7 +1388,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     const size_t region = qmm_region(ctx, M, K, N);
     const size_t each = (((size_t)M * N * 4) + 255) & ~(size_t)255;
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * each, fail)) return rc;
     }
@@ -1378,7 +1400,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         // pass over x is skipped, and the stores of the `up` projection apply act(gate) * up on the way out
         // (rocm_mlx_q4_gelu_tanh_multiply_batch, go/engine/hip/kernels/quant/affine_gelu_tanh.hipinc:921-1109): one
         // [M, N] fp32 matrix is written and read instead of two written and two read.  Same bytes as the route below.
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         int x_state = aq::kXReadyNone;
         if (int rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], x, gate_packed,
                                       gate_scales, gate_biases, g, M, K, N, group_size, bits, true, fail, nullptr, 0, &x_state))
@@ -1390,7 +1412,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     }
     if (int rc = aq_qmv(ctx, x, gate_packed, gate_scales, gate_biases, g, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
     if (int rc = aq_qmv(ctx, x, up_packed, up_scales, up_biases, u, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::act_mul_f32_launch(g, u, y, (int64_t)M * N, act, out_f32 ? 1 : 0, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -1441,18 +1463,18 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
         a.routes = routes;
         a.act = act;
         {
-            std::lock_guard<std::mutex> lk(ctx->mu);
+            CallLock lk(ctx);
             if (const int rc = run_grouped(ctx, a, group_size, bits, true); rc != kPass) return rc;
         }
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, true, di)) {
-            std::lock_guard<std::mutex> lk(ctx->mu);
+            CallLock lk(ctx);
             ctx->last_variant[0] = "gather_gate_up_diag";
             AQ_HIP(aq::qmvd_pair_launch(di, a, true, ctx->stream), "hipLaunchKernel");
             return AQ_OK;
         }
     }
     if (ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, packed, (size_t)K * 2)) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 1, true, N, K, routes);
         if (aq::qmv_act_supported(bits, 1, rows, true)) {
             aq::QmvArgs a{};
@@ -1482,7 +1504,7 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
     }
     const size_t each = (((size_t)routes * N * 4) + 255) & ~(size_t)255;
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, 2 * each, fail)) return rc;
     }
@@ -1494,7 +1516,7 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
     if (int rc = gather_call(ctx, x, packed, scales, biases, lhs, rhs, u, routes, x_rows, K, N, num_experts, expert_rows,
                              up_row_base, group_size, bits, AQ_OUT_F32, false))
         return rc;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::act_mul_f32_launch(g, u, y, (int64_t)routes * N, act, out_f32 ? 1 : 0, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -1512,7 +1534,7 @@ int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* pa
         return fail(AQ_ERR_ARG, "aq_qmv_act: operand pointer is not element-aligned");
     if (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, gate_x, packed, (size_t)K * 2) &&
         aligned(up_x, 16)) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 2, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 2, rows, false)) {
             aq::QmvArgs a{};
@@ -1536,7 +1558,7 @@ int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* pa
     }
     const size_t region = qmm_region(ctx, M, K, N);
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * K * 2, fail)) return rc;
     }
@@ -1566,7 +1588,7 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
         return fail(AQ_ERR_ARG, "aq_gather_qmv_act: operand pointer is not element-aligned");
     if (routes > 65535) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv_act: at most 65535 routes per call");
     if (ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, gate_x, packed, (size_t)K * 2) && aligned(up_x, 16)) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 2, true, N, K, routes);
         if (aq::qmv_act_supported(bits, 2, rows, true)) {
             aq::QmvArgs a{};
@@ -1595,7 +1617,7 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
         }
     }
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, (size_t)x_rows * K * 2, fail)) return rc;
     }
@@ -1619,7 +1641,7 @@ int aq_moe_route(aq_ctx* ctx, const void* logits, int rows, int num_experts, int
     if (!aligned(logits, lb ? 2 : 4) || !aligned(ids, 4) || !aligned(weights, 4) ||
         (expert_scales && !aligned(expert_scales, 4)) || (token_of_route && !aligned(token_of_route, 4)))
         return fail(AQ_ERR_ARG, "aq_moe_route: operand pointer is not element-aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     aq::MoeRouteArgs a{};
     a.logits = logits;
     a.expert_scales = expert_scales;
@@ -1645,7 +1667,7 @@ int aq_moe_combine(aq_ctx* ctx, const void* route_rows, const float* weights, vo
     const bool in_f32 = (flags & AQ_IN_F32) != 0, out_f32 = (flags & AQ_OUT_F32) != 0;
     if (!aligned(route_rows, in_f32 ? 4 : 2) || !aligned(weights, 4) || !aligned(out, out_f32 ? 4 : 2))
         return fail(AQ_ERR_ARG, "aq_moe_combine: operand pointer is not element-aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     aq::MoeCombineArgs a{};
     a.route_rows = route_rows;
     a.weights = weights;
@@ -1700,7 +1722,7 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
                     "other shapes need scratch memory: use aq_qmv_greedy", op);
     if (fuse == 3 && !fused) {
         // the unfused reduction accumulates with atomics and starts from "no result"
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(aq::fill_zero_launch(out, (size_t)M * 8, ctx->stream), "hipLaunchKernel");
     }
     if (N == 0) return AQ_OK;
@@ -1710,7 +1732,7 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
     if (!aligned(x, 2) || !aligned(packed, 4) || !aligned(scales, 2) || !aligned(biases, 2))
         return fail(AQ_ERR_ARG, "%s: operand pointer is not element-aligned", op);
     if (fused) {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         {
             // the diagonal-MFMA kernel aq_qmv would pick for this projection, with the head epilogue
             const int di = bits != 4 || (ctx->families_off >> kFamDiag & 1) ? -1
@@ -1784,13 +1806,13 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
     // the projection as fp32 into scratch, then the same epilogue over it
     const size_t region = qmm_region(ctx, M, K, N);
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * N * 4, fail)) return rc;
     }
     float* logits = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + region);
     if (int rc = aq_qmv(ctx, x, packed, scales, biases, logits, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
     AQ_HIP(aq::pack_scores_launch(logits, M, N, suppress, suppress_count, fuse == 3 ? o : nullptr, fuse == 4 ? o : nullptr,
                                   ctx->stream),
@@ -1823,7 +1845,7 @@ int aq_qmv_greedy_selected(aq_ctx* ctx, const void* x, const void* packed, const
     if (count > 0 && !rows) return fail(AQ_ERR_ARG, "%s: count without a list of rows", op);
     if (rows && !aligned(rows, 4)) return fail(AQ_ERR_ARG, "%s: operand pointer is not element-aligned", op);
     if (count == 0 || N == 0) {  // nothing to choose from: "no result"
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(aq::fill_zero_launch(best, 8, ctx->stream), "hipLaunchKernel");
         return AQ_OK;
     }
@@ -1835,7 +1857,7 @@ int aq_qmv_greedy_selected(aq_ctx* ctx, const void* x, const void* packed, const
     if (count > 65535) return fail(AQ_ERR_UNSUPPORTED, "%s: at most 65535 candidates per call", op);
     const int width = N < 16 ? N : 16;
     const size_t start_bytes = align256((size_t)count * 4), need = start_bytes + (size_t)count * width * 4;
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, need, fail)) return rc;
     int32_t* start = static_cast<int32_t*>(ctx->ws.ptr);
@@ -1882,7 +1904,7 @@ int aq_packed_topk(aq_ctx* ctx, const uint64_t* scores, int64_t count, int top_k
     if (top_k > aq::kTopKMax) return fail(AQ_ERR_UNSUPPORTED, "aq_packed_topk: top-k is at most %d", aq::kTopKMax);
     if (!out || (count > 0 && !scores)) return fail(AQ_ERR_ARG, "aq_packed_topk: null operand");
     if (!aligned(out, 8) || !aligned(scores, 8)) return fail(AQ_ERR_ARG, "aq_packed_topk: operand pointer is not 8-byte aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     if (count == 0) {
         AQ_HIP(aq::fill_zero_launch(out, (size_t)top_k * 8, ctx->stream), "hipLaunchKernel");
         return AQ_OK;
@@ -1914,7 +1936,7 @@ int aq_packed_topk_sample(aq_ctx* ctx, const uint64_t* top, int top_k, float tem
     if (!(softcap >= 0.0f) || !std::isfinite(softcap))
         return fail(AQ_ERR_ARG, "aq_packed_topk_sample: softcap must be non-negative and finite");
     if (!std::isfinite(draw)) return fail(AQ_ERR_ARG, "aq_packed_topk_sample: draw must be finite");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::packed_topk_sample_launch(reinterpret_cast<const unsigned long long*>(top), top_k, temperature, top_p, softcap,
                                          draw, reinterpret_cast<unsigned long long*>(out), ctx->stream),
            "hipLaunchKernel");
@@ -2001,7 +2023,7 @@ int aq_upload_fused_gate_up(aq_ctx* ctx, const struct aqh_linear* gate, const st
     AQ_HIP(w.alloc(2 * gate->weight_len), "hipMalloc");
     AQ_HIP(s.alloc(2 * gate->scales_len), "hipMalloc");
     AQ_HIP(b.alloc(2 * gate->biases_len), "hipMalloc");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     // one strided copy per part and array: expert e's rows go to [e][part]
     struct Job {
         void* dst;
@@ -2045,7 +2067,7 @@ int aq_tile_weights(aq_ctx* ctx, const void* packed, const void* scales, const v
     if (!packed || !scales || !biases || !tiled) return fail(AQ_ERR_ARG, "aq_tile_weights: null operand");
     if (!aligned(packed, 16) || !aligned(tiled, 16) || !aligned(scales, 2) || !aligned(biases, 2))
         return fail(AQ_ERR_ARG, "aq_tile_weights: packed and tiled must be 16-byte aligned, scales and biases 2-byte aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::tile_repack_launch(packed, scales, biases, tiled, N, K, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -2062,7 +2084,7 @@ int aq_tile_device_linear(aq_ctx* ctx, aq_device_linear* lin) {
                     lin->group_size, lin->in_dim, lin->rows);
     void* tiled = nullptr;
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         AQ_HIP(hipMalloc(&tiled, (size_t)bytes), "hipMalloc");
     }
@@ -2088,7 +2110,7 @@ int aq_untile_weights(aq_ctx* ctx, const void* tiled, int64_t N, int K, int grou
     if (!packed || !scales || !biases || !tiled) return fail(AQ_ERR_ARG, "aq_untile_weights: null operand");
     if (!aligned(packed, 16) || !aligned(tiled, 16) || !aligned(scales, 2) || !aligned(biases, 2))
         return fail(AQ_ERR_ARG, "aq_untile_weights: packed and tiled must be 16-byte aligned, scales and biases 2-byte aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::tile_unpack_launch(tiled, packed, scales, biases, N, K, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -2103,7 +2125,7 @@ int aq_dequant_f32(aq_ctx* ctx, const void* packed, const void* scales, const vo
     if (((int64_t)K * bits) % 32 != 0) return fail(AQ_ERR_SHAPE, "aq_dequant_f32: cols*bits must be divisible by 32");
     if (!packed || !scales || !biases || !out_f32) return fail(AQ_ERR_ARG, "aq_dequant_f32: null operand");
     if (N * (int64_t)K / 8 > 0x7fffffffLL * 32) return fail(AQ_ERR_UNSUPPORTED, "aq_dequant_f32: tensor too large");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::dequant_launch(static_cast<const uint32_t*>(packed), static_cast<const uint16_t*>(scales),
                               static_cast<const uint16_t*>(biases), out_f32, N, K, group_size, bits, ctx->stream),
            "hipLaunchKernel");
@@ -2140,7 +2162,7 @@ int aq_gguf_to_affine(aq_ctx* ctx, int gguf_type, const void* src, uint64_t src_
     if (!src || !packed || !scales || !biases) return fail(AQ_ERR_ARG, "aq_gguf_to_affine: null operand");
     if (!aligned(packed, 16) || !aligned(scales, 2) || !aligned(biases, 2) || (gguf_type == aq::kGgufF32 && !aligned(src, 4)))
         return fail(AQ_ERR_ARG, "aq_gguf_to_affine: packed must be 16-byte, scales/biases 2-byte, F32 input 4-byte aligned");
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     AQ_HIP(aq::gguf_repack_launch(gguf_type, static_cast<const uint8_t*>(src), static_cast<uint32_t*>(packed),
                                   static_cast<uint16_t*>(scales), static_cast<uint16_t*>(biases), rows * (cols / 32),
                                   ctx->stream),
@@ -2163,7 +2185,7 @@ int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, con
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     hipStream_t stream;
     {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         stream = ctx->stream;
     }
     // small results are stored to pinned host memory by the kernel itself; larger ones cross in one copy, which fills the
@@ -2180,7 +2202,7 @@ int staged_host_call(aq_ctx* ctx, const char* op, const void* x, bool x_f32, con
     if (up != hipSuccess) {
         rc = hip_fail(up, "hipMemcpyHtoD");
     } else {
-        std::lock_guard<std::mutex> lk(ctx->mu);
+        CallLock lk(ctx);
         if (ctx->stream != stream) (void)hipStreamSynchronize(stream);  // (the caller moved the context meanwhile)
         stream = ctx->stream;
         aq::QmvArgs a{};
@@ -2286,7 +2308,7 @@ const char* aq_variant_name(int op, int variant) {
 int aq_force_variant(aq_ctx* ctx, int op, int variant) {
     if (!ctx || op < 0 || op > 1) return fail(AQ_ERR_ARG, "aq_force_variant: bad argument");
     if (variant >= aq_variant_count(op)) return fail(AQ_ERR_ARG, "aq_force_variant: variant %d out of range", variant);
-    std::lock_guard<std::mutex> lk(ctx->mu);
+    CallLock lk(ctx);
     ctx->forced[op] = variant < 0 ? -1 : variant;
     return AQ_OK;
 }

@@ -1,8 +1,11 @@
 // Scratch memory a context lends to its calls: one device block, grown on demand, never while a capture is open.
 //
 // Its users follow each other on the context's stream.  When the context moves to another stream, the work that the old
-// one still holds over the block is kept in order by an event: recorded when the stream is left (workspace_leave), waited for
-// by the first use on the new one.
+// one still holds over the block is kept in order by an event: recorded behind the last use (workspace_note), waited for by the
+// first use on the new one.  The context's own stream is noted when it is left.  A caller's stream may have been destroyed by
+// then, and the runtime must not be asked for it; noting every use on it as it ends costs 3 us of the stream (a marker; 40 best
+// of 262144 13.9 -> 17.0 us), which a program that stays on one stream would pay for nothing.  So the first time that one is
+// left the device is waited for, and from then on uses on callers' streams are noted (CallLock in aq_api.hip).
 #pragma once
 #include <hip/hip_runtime_api.h>
 #include <stddef.h>
@@ -32,6 +35,7 @@ struct Workspace {
     bool touched = false, required = false;
     hipEvent_t left = nullptr;
     bool used = false;          // work over the block was queued on the current stream since it became current
+    bool unnoted = false;       // ... since `left` was recorded
     bool left_pending = false;  // `left` stands for work on another stream that the current one has not waited for
 };
 
@@ -48,7 +52,11 @@ bool workspace_offer(hipStream_t stream, Workspace* ws, size_t need);
 bool workspace_may_grow(const Workspace* ws, size_t need, hipStream_t stream);
 // Orders a use of a block of ws (the current one or one that a graph keeps) on `stream` behind the earlier ones.
 hipError_t workspace_use(hipStream_t stream, Workspace* ws);
-// The context goes from `stream` to another one, or begins a capture on it.
-hipError_t workspace_leave(hipStream_t stream, Workspace* ws);
+// Notes the end of what `stream` (the current one) has been given to do over the block (record: with an event; else only that
+// recorded work needs none).
+hipError_t workspace_note(hipStream_t stream, Workspace* ws, bool record = true);
+// The context goes to another stream, or begins a capture: what was noted is for the next use to wait for, and the device is
+// waited for here if something was not.
+hipError_t workspace_leave(Workspace* ws);
 
 }  // namespace aq

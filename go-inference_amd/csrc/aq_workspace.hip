@@ -68,21 +68,34 @@ hipError_t workspace_use(hipStream_t stream, Workspace* ws) {
         if (rc != hipSuccess) return rc;
         ws->left_pending = false;
     }
-    ws->used = ws->touched = true;
+    ws->used = ws->unnoted = ws->touched = true;
     return hipSuccess;
 }
 
-hipError_t workspace_leave(hipStream_t stream, Workspace* ws) {
+hipError_t workspace_note(hipStream_t stream, Workspace* ws, bool record) {
+    if (!ws->unnoted) return hipSuccess;
+    if (capturing(stream)) {  // recorded, not run; what ran before the capture was noted when it began
+        ws->unnoted = false;
+        return hipSuccess;
+    }
+    if (!record) return hipSuccess;
+    ws->unnoted = false;
+    hipError_t rc = hipEventRecord(ws->left, stream);
+    if (rc != hipSuccess) {
+        (void)hipGetLastError();
+        rc = hipStreamSynchronize(stream);  // nothing is left to wait for
+    }
+    return rc;
+}
+
+hipError_t workspace_leave(Workspace* ws) {
     if (!ws->used) return hipSuccess;
     ws->used = false;
-    if (capturing(stream)) return hipSuccess;  // what ran before the capture was noted when it began
-    hipError_t rc = hipEventRecord(ws->left, stream);
-    if (rc == hipSuccess) {
+    if (!ws->unnoted) {
         ws->left_pending = true;
-        return rc;
+        return hipSuccess;
     }
-    // the caller has destroyed the stream already: what it still runs is waited for here
-    (void)hipGetLastError();
+    ws->unnoted = ws->left_pending = false;
     return hipDeviceSynchronize();
 }
 

@@ -66,7 +66,9 @@ void aq_destroy(aq_ctx *ctx);
  * (pass NULL for the legacy default stream the reference launches on,
  * go/engine/hip/hip_driver_cgo.go:452-478).  aq_use_own_stream() goes back.
  * Calls that go through the context's workspace stay in order across a switch: the first of them on the new stream waits
- * (on the device) for what the old one still does.  All other calls on the two streams are independent of each other. */
+ * (on the device) for what the old one still does.  All other calls on the two streams are independent of each other.
+ * The stream that is left may have been destroyed already.  (The first time that a caller's stream with such calls is left,
+ * the device is waited for; from then on each of them notes its end on the stream, 3 us.) */
 int aq_use_stream(aq_ctx *ctx, void *hip_stream);
 int aq_use_own_stream(aq_ctx *ctx);
 int aq_device_name(aq_ctx *ctx, char *buf, size_t buf_len);

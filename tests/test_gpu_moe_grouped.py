@@ -148,6 +148,34 @@ def test_two_streams_share_one_workspace(ctx):
             t.free()
 
 
+def test_stream_destroyed_before_the_context_leaves_it(ctx):
+    import ctypes
+    say("stream destroyed before it is left")
+    hip = ctypes.CDLL("libamdhip64.so")
+    M, K, N = 40, 512, 64
+    dw = DeviceAffine(ctx, *F.synthetic_affine(N, K, 4, 32, seed=2990))
+    dx, dy = ctx.to_device(F.synthetic_x(M, K, seed=2991)), ctx.alloc(M * N * 2)
+    call = lambda: ctx.qmm(dx, dw.w, dw.s, dw.b, dy, M, K, N, 32, 4)
+    call()
+    ctx.sync()
+    want = dy.download(np.uint16).copy()
+    for _ in range(3):
+        ctx.fill_zero(dy)
+        ctx.sync()
+        st = ctypes.c_void_p()
+        assert hip.hipStreamCreateWithFlags(ctypes.byref(st), 1) == 0
+        assert ctx.lib.aq_use_stream(ctx.handle, st) == 0
+        call()
+        assert hip.hipStreamSynchronize(st) == 0 and hip.hipStreamDestroy(st) == 0
+        assert ctx.lib.aq_use_own_stream(ctx.handle) == 0
+        assert np.array_equal(dy.download(np.uint16), want)
+        call()
+        ctx.sync()
+        assert np.array_equal(dy.download(np.uint16), want)
+    for t in (dx, dy, dw):
+        t.free()
+
+
 def test_recorded_calls_outlive_a_larger_workspace(orc):
     """A gather of many routes and matmuls in groups of 32, recorded over the workspace, are replayed after it has moved (other
     calls asked for more); recorded where it has no room they run on the kernels that need none."""

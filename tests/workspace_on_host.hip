@@ -14,7 +14,13 @@
 static std::vector<std::string> calls;  // in order
 static int live_blocks = 0, next_id = 1, record_fails = 0;
 static size_t memory = 1 << 20;  // bytes hipMalloc may still hand out
-static hipStream_t capturing_stream = nullptr;
+static hipStream_t capturing_stream = nullptr, destroyed_stream = nullptr;
+static void must_exist(hipStream_t s) {  // the runtime reads the object behind a handle without a look whether it is there
+    if (s && s == destroyed_stream) {
+        puts("a destroyed stream was asked for");
+        exit(1);
+    }
+}
 
 static void note(const char* fmt, ...) {
     char b[128];
@@ -50,15 +56,18 @@ hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
 }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t s) {
-    if (record_fails) return hipErrorContextIsDestroyed;
+    must_exist(s);
+    if (record_fails) return hipErrorUnknown;
     note("record %s", name(s).c_str());
     return hipSuccess;
 }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) {
+    must_exist(s);
     note("wait %s", name(s).c_str());
     return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t s) {
+    must_exist(s);
     note("sync %s", name(s).c_str());
     return hipSuccess;
 }
@@ -67,6 +76,7 @@ hipError_t hipDeviceSynchronize(void) {
     return hipSuccess;
 }
 hipError_t hipStreamIsCapturing(hipStream_t s, hipStreamCaptureStatus* cs) {
+    must_exist(s);
     *cs = s == capturing_stream && s ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
@@ -93,45 +103,69 @@ static bool seen(std::vector<std::string> want) {
 static const hipStream_t A = reinterpret_cast<hipStream_t>((uintptr_t)'A'), B = reinterpret_cast<hipStream_t>((uintptr_t)'B'),
                          C = reinterpret_cast<hipStream_t>((uintptr_t)'C');
 
+static hipError_t note_and_leave(hipStream_t stream, aq::Workspace* ws) {
+    const hipError_t rc = aq::workspace_note(stream, ws), left = aq::workspace_leave(ws);
+    return rc != hipSuccess ? rc : left;
+}
+
 static void use_on_another_stream_waits_for_the_last_one() {
     aq::Workspace ws;
     EXPECT(aq::workspace_open(&ws, 0) == hipSuccess);
     EXPECT(aq::workspace_reserve(A, &ws, 400, quiet) == 0 && ws.bytes == 500);
     EXPECT(seen({"sync A", "malloc 500"}));
-    EXPECT(aq::workspace_leave(A, &ws) == hipSuccess && seen({"record A"}));
+    EXPECT(note_and_leave(A, &ws) == hipSuccess && seen({"record A"}));
     EXPECT(aq::workspace_reserve(B, &ws, 100, quiet) == 0 && seen({"wait B"}));  // before any kernel of the call
     EXPECT(aq::workspace_reserve(B, &ws, 100, quiet) == 0 && seen({}));          // once
-    EXPECT(aq::workspace_leave(B, &ws) == hipSuccess && seen({"record B"}));
+    EXPECT(note_and_leave(B, &ws) == hipSuccess && seen({"record B"}));
     // a stream that never used the block is passed through: the one behind it still waits
-    EXPECT(aq::workspace_leave(A, &ws) == hipSuccess && seen({}));
+    EXPECT(note_and_leave(A, &ws) == hipSuccess && seen({}));
     EXPECT(aq::workspace_use(C, &ws) == hipSuccess && seen({"wait C"}));
     // growth frees the block behind everybody's work
-    EXPECT(aq::workspace_leave(C, &ws) == hipSuccess && seen({"record C"}));
+    EXPECT(note_and_leave(C, &ws) == hipSuccess && seen({"record C"}));
     EXPECT(aq::workspace_reserve(A, &ws, 800, quiet) == 0 && seen({"wait A", "sync A", "free", "malloc 1000"}));
-    // a stream that is gone when it is left: the device is waited for instead
+    // no event to be had: the stream is waited for instead
     record_fails = 1;
-    EXPECT(aq::workspace_leave(A, &ws) == hipSuccess && seen({"sync device"}));
+    EXPECT(note_and_leave(A, &ws) == hipSuccess && seen({"sync A"}));
     record_fails = 0;
-    EXPECT(aq::workspace_use(B, &ws) == hipSuccess && seen({}));
     aq::workspace_close(&ws);
     calls.clear();
     EXPECT(live_blocks == 0);
+}
+
+static void a_stream_may_be_destroyed_before_it_is_left() {
+    aq::Workspace ws;
+    EXPECT(aq::workspace_open(&ws, 1000) == hipSuccess && seen({"malloc 1000"}));
+    EXPECT(aq::workspace_use(A, &ws) == hipSuccess && aq::workspace_note(A, &ws) == hipSuccess && seen({"record A"}));  // a call
+    EXPECT(aq::workspace_note(A, &ws) == hipSuccess && seen({}));
+    destroyed_stream = A;
+    EXPECT(aq::workspace_leave(&ws) == hipSuccess && seen({}));
+    EXPECT(aq::workspace_use(B, &ws) == hipSuccess && seen({"wait B"}));
+    // uses that were not noted, captured ones aside: the device is waited for, once
+    EXPECT(aq::workspace_note(B, &ws, false) == hipSuccess && seen({}));
+    destroyed_stream = B;
+    EXPECT(aq::workspace_leave(&ws) == hipSuccess && seen({"sync device"}));
+    EXPECT(aq::workspace_leave(&ws) == hipSuccess && aq::workspace_use(C, &ws) == hipSuccess && seen({}));
+    capturing_stream = C;
+    EXPECT(aq::workspace_note(C, &ws, false) == hipSuccess && aq::workspace_leave(&ws) == hipSuccess && seen({}));
+    capturing_stream = destroyed_stream = nullptr;
+    aq::workspace_close(&ws);
+    calls.clear();
 }
 
 static void captured_uses_wait_for_nothing_and_are_ordered_when_replayed() {
     aq::Workspace ws;
     EXPECT(aq::workspace_open(&ws, 1000) == hipSuccess && seen({"malloc 1000"}));
     EXPECT(aq::workspace_use(A, &ws) == hipSuccess);
-    EXPECT(aq::workspace_leave(A, &ws) == hipSuccess && seen({"record A"}));
+    EXPECT(note_and_leave(A, &ws) == hipSuccess && seen({"record A"}));
     capturing_stream = B;
-    EXPECT(aq::workspace_reserve(B, &ws, 600, quiet) == 0 && seen({}));  // recorded, not run
+    EXPECT(aq::workspace_reserve(B, &ws, 600, quiet) == 0 && aq::workspace_note(B, &ws) == hipSuccess && seen({}));  // recorded, not run
     EXPECT(aq::workspace_reserve(B, &ws, 2000, quiet) != 0 && seen({}) && ws.bytes == 1000);
     capturing_stream = nullptr;
     EXPECT(aq::workspace_use(B, &ws) == hipSuccess && seen({"wait B"}));  // the replay
     // a capture begins on the stream in use, and the context leaves it while it is open
-    EXPECT(aq::workspace_leave(B, &ws) == hipSuccess && seen({"record B"}));
+    EXPECT(note_and_leave(B, &ws) == hipSuccess && seen({"record B"}));
     capturing_stream = B;
-    EXPECT(aq::workspace_use(B, &ws) == hipSuccess && aq::workspace_leave(B, &ws) == hipSuccess && seen({}));
+    EXPECT(aq::workspace_use(B, &ws) == hipSuccess && note_and_leave(B, &ws) == hipSuccess && seen({}));
     EXPECT(aq::workspace_use(C, &ws) == hipSuccess && seen({"wait C"}));
     capturing_stream = nullptr;
     aq::workspace_close(&ws);
@@ -187,6 +221,7 @@ int main() {
     an_offer_that_cannot_be_met_changes_nothing();
     a_block_that_a_graph_keeps_outlives_growth();
     use_on_another_stream_waits_for_the_last_one();
+    a_stream_may_be_destroyed_before_it_is_left();
     captured_uses_wait_for_nothing_and_are_ordered_when_replayed();
     puts("ok");
     return 0;
