@@ -1720,8 +1720,8 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
         return fail(AQ_ERR_UNSUPPORTED,
                     "%s: takes one activation row of 4- or 8-bit codes with 16-byte aligned rows (the fused kernels); "
                     "other shapes need scratch memory: use aq_qmv_greedy", op);
-    if (fuse == 3 && !fused) {
-        // the unfused reduction accumulates with atomics and starts from "no result"
+    if (fuse == 3 && !fused && !(K > 0 && aq::best_score_clears(N))) {
+        // the unfused reduction of long rows accumulates with atomics and starts from "no result"
         CallLock lk(ctx);
         AQ_HIP(aq::fill_zero_launch(out, (size_t)M * 8, ctx->stream), "hipLaunchKernel");
     }
@@ -1814,8 +1814,8 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
     if (int rc = aq_qmv(ctx, x, packed, scales, biases, logits, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
     CallLock lk(ctx);
     unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
-    AQ_HIP(aq::pack_scores_launch(logits, M, N, suppress, suppress_count, fuse == 3 ? o : nullptr, fuse == 4 ? o : nullptr,
-                                  ctx->stream),
+    AQ_HIP(fuse == 3 ? aq::best_score_launch(logits, M, N, suppress, suppress_count, o, ctx->stream)
+                     : aq::pack_scores_launch(logits, M, N, suppress, suppress_count, o, ctx->stream),
            "hipLaunchKernel");
     return AQ_OK;
 }

@@ -204,9 +204,13 @@ hipError_t qmv_head_launch(int bits, int fuse, int rows, const QmvArgs& a, hipSt
 hipError_t selected_windows_launch(const int32_t* rows, int count, int N, int width, int32_t* start, hipStream_t stream);
 hipError_t selected_pick_launch(const float* scores, const int32_t* rows, const int32_t* start, int count, int width,
                                 unsigned long long* best, hipStream_t stream);
-// The same two epilogues over fp32 scores that are already in memory: scores [M, N] -> best[M] / packed[M, N].
+// The same two epilogues over fp32 scores [M, N] that are already in memory: packed[M, N], or best[M], which has to be zero
+// beforehand unless best_score_clears(N).
 hipError_t pack_scores_launch(const float* scores, int M, int N, const int32_t* suppress, int suppress_count,
-                              unsigned long long* best_or_null, unsigned long long* packed_or_null, hipStream_t stream);
+                              unsigned long long* packed, hipStream_t stream);
+bool best_score_clears(int N);
+hipError_t best_score_launch(const float* scores, int M, int N, const int32_t* suppress, int suppress_count, unsigned long long* best,
+                             hipStream_t stream);
 // Largest top_k (<= kTopKMax) of `count` packed values, sorted descending, into out[top_k]; scratch holds
 // packed_topk_scratch_entries(count, top_k) values.
 constexpr int kTopKMax = 64;

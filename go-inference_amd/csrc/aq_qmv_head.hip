@@ -9,8 +9,8 @@
 //            (go/engine/hip/kernels/sampling/topk.hipinc:45-84) yields per chunk, here per wavefront segment
 //            and repeated until one segment is left.
 //
-// The streaming part is the dot2 body; only the epilogue differs.  pack_scores_kernel applies the same two
-// epilogues to fp32 scores already in memory (shapes the dot2 kernels do not take, several rows).
+// The streaming part is the dot2 body; only the epilogue differs.  best_score_kernel and pack_scores_kernel apply the same
+// two epilogues to fp32 scores already in memory (shapes the dot2 kernels do not take, several rows).
 #include "aq_qmv_body.h"
 
 namespace aq {
@@ -169,43 +169,82 @@ hipError_t head_fold_launch(const unsigned long long* partial, int count, unsign
     return hipGetLastError();
 }
 
-// grid.y = activation row; a workgroup folds its share of a row before touching the shared maximum
+// The epilogues over fp32 scores in memory.  scores: every value packed, a thread a value.
 __global__ __launch_bounds__(256) void pack_scores_kernel(const float* __restrict__ scores, int N, const int32_t* suppress,
-                                                          int suppress_count, unsigned long long* best,
-                                                          unsigned long long* packed_out) {
-    const int m = blockIdx.y;
-    const float* row_scores = scores + (int64_t)m * N;
-    unsigned long long mine = 0;
+                                                          int suppress_count, unsigned long long* packed_out) {
+    const int64_t row = (int64_t)blockIdx.y * N;
     for (int n = blockIdx.x * 256 + threadIdx.x; n < N; n += gridDim.x * 256) {
-        const float v = row_scores[n];
+        const float v = scores[row + n];
         unsigned long long p = 0;
         if (isfinite(v) && !token_suppressed((uint32_t)n, suppress, suppress_count)) p = pack_score_index(v, (uint32_t)n);
-        if (packed_out) packed_out[(int64_t)m * N + n] = p;
-        mine = p > mine ? p : mine;
+        packed_out[row + n] = p;
     }
-    if (!best) return;
+}
+
+// argmax: grid.y = activation row.  One workgroup a row (ONE) stores the row's best itself; several meet in an atomic maximum
+// on best[row], which starts at zero.  Atomics on one address are served one by one (about 12 ns each here): a workgroup
+// for every 256 scores spent 36 us on 6 x 128201 scores and 60 us on 8 x 164024 in them, for 4 MB that are read in 3.  So at
+// most kBestGroups of them per row, each thread with eight loads in flight; rows of up to kBestOneGroup scores in one
+// workgroup of 1024 threads, which needs no launch that clears best (a longer row is more than one CU reads in the time of
+// that launch: 128201 scores took it 18 us).  Whole greedy calls: 6 rows (128201 x 1152) 60.8 -> 29.6 us, 8 (164024 x 2048)
+// 108.8 -> 54.7, 15 (91522 x 2048, 8 bit) 105.8 -> 65.3, 3 (36934 x 1536) 30.6 -> 27.0.
+constexpr int kBestGroups = 32, kBestOneGroup = 16384;
+template <bool ONE>
+__global__ __launch_bounds__(ONE ? 1024 : 256) void best_score_kernel(const float* __restrict__ scores, int N, const int32_t* suppress,
+                                                                     int suppress_count, unsigned long long* best) {
+    constexpr int NT = ONE ? 1024 : 256, AHEAD = 8;
+    const int m = blockIdx.y;
+    const float* const row = scores + (int64_t)m * N;
+    unsigned long long mine = 0;
+    const int stride = (int)gridDim.x * NT;
+    for (int64_t n0 = (int64_t)blockIdx.x * NT + threadIdx.x; n0 < N; n0 += (int64_t)stride * AHEAD) {
+        float v[AHEAD];
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) v[i] = row[min(n0 + (int64_t)i * stride, (int64_t)N - 1)];
+#pragma unroll
+        for (int i = 0; i < AHEAD; i++) {
+            const int64_t n = n0 + (int64_t)i * stride;
+            if (n >= N || !isfinite(v[i])) continue;
+            const unsigned long long p = pack_score_index(v[i], (uint32_t)n);
+            if (p > mine && !token_suppressed((uint32_t)n, suppress, suppress_count)) mine = p;
+        }
+    }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const unsigned long long other = __shfl_xor(mine, o, kWave);
         mine = other > mine ? other : mine;
     }
-    __shared__ unsigned long long wave_best[4];
+    __shared__ unsigned long long wave_best[NT / kWave];
     if ((threadIdx.x & (kWave - 1)) == 0) wave_best[threadIdx.x >> 6] = mine;
     __syncthreads();
     if (threadIdx.x == 0) {
         unsigned long long b = wave_best[0];
-        for (int i = 1; i < 4; i++) b = wave_best[i] > b ? wave_best[i] : b;
-        if (b != 0) atomicMax(best + m, b);
+        for (int i = 1; i < NT / kWave; i++) b = wave_best[i] > b ? wave_best[i] : b;
+        if constexpr (ONE)
+            best[m] = b;
+        else if (b != 0)
+            atomicMax(best + m, b);
     }
 }
 
 hipError_t pack_scores_launch(const float* scores, int M, int N, const int32_t* suppress, int suppress_count,
-                              unsigned long long* best_or_null, unsigned long long* packed_or_null, hipStream_t stream) {
+                              unsigned long long* packed, hipStream_t stream) {
     if (M <= 0 || N <= 0) return hipSuccess;
     int bx = (N + 255) / 256;
     if (bx > 1024) bx = 1024;
     hipLaunchKernelGGL(pack_scores_kernel, dim3((unsigned)bx, (unsigned)M), dim3(256), 0, stream, scores, N, suppress,
-                       suppress_count, best_or_null, packed_or_null);
+                       suppress_count, packed);
+    return hipGetLastError();
+}
+bool best_score_clears(int N) { return N > 0 && N <= kBestOneGroup; }
+hipError_t best_score_launch(const float* scores, int M, int N, const int32_t* suppress, int suppress_count, unsigned long long* best,
+                             hipStream_t stream) {
+    if (M <= 0 || N <= 0) return hipSuccess;
+    if (best_score_clears(N))
+        hipLaunchKernelGGL(best_score_kernel<true>, dim3(1, (unsigned)M), dim3(1024), 0, stream, scores, N, suppress, suppress_count, best);
+    else
+        hipLaunchKernelGGL(best_score_kernel<false>, dim3((unsigned)min(kBestGroups, (N + 2047) / 2048), (unsigned)M), dim3(256), 0, stream, scores, N, suppress,
+                           suppress_count, best);
     return hipGetLastError();
 }
 
