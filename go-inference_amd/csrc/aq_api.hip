@@ -270,6 +270,7 @@ const QmvRule kQmvRules[] = {
     {4, 32, 0, 3, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
     {8, 32, 0, 2, 32, kFamTok},
     {0, 128, 0, 5, 32, kFamTok},
+    {0, 0, 0, 33, 64, kFamTok},
     {0, 0, 0, 9, 64, kFamTilesLarge},       // 16 Mi codes and more: the 16-row block-MFMA kernel is bound by its 4x4x4 MFMAs
     {0, 0, 0, 2, 16, kFamBlk},              // the whole call in one launch of up to 16 rows (4 where K is long)
     {8, 0, 0, 1, 1, kFamBlk},               // (a single row of 4-bit codes is faster on the dot2 kernels)
@@ -356,13 +357,48 @@ int run_diag(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool g
 bool tok_small(int bits, int group_size, int M, int K, int64_t rows) {
     return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20 && (bits == 8 ? M <= 4 : rows <= 528);
 }
+// 33..64 rows of x run as two halves in one grid.  They are ahead of the tiles (us, tiles / halves, 40 rows) while eight sets of 16
+// weight rows per workgroup fill each CU once at the most: 1024 x 14336 4 bit, groups of 64 / 32 / 128 17.0 / 11.4, 19.8 / 15.9,
+// 19.2 / 10.9, 8 bit 16.6 / 14.3, 21.2 / 15.6; 14336 x 4096 30.5 / 25.4, 39.7 / 33.2, 37.8 / 25.3, 32.8 / 30.5, 42.9 / 34.8.  With
+// two rounds they are ahead where the tiles are the slow ones, gate and up in groups of 64 (4096 x 14336 4 bit 52.7 / 43.6, 8 bit
+// 59.1 / 54.7) and groups of 128 (4096 x 28672 51.0 / 43.7), and behind elsewhere (4096 x 28672 groups of 64 41.7 / 44.0, 8 bit
+// 52.4 / 54.4, groups of 32 49.3 / 59.0, 60.6 / 62.6; gate and up in groups of 32 47.7 / 59.3).  Matrices of up to 528 rows stay
+// with the tiles, a choice that tests/test_gpu_selection.py states.
+bool tok_halves(const aq_ctx* ctx, int group_size, int M, int64_t rows, bool pair) {
+    if (M <= 32) return true;
+    if (rows <= 528) return false;
+    const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256, groups = ((rows + 15) / 16 * (pair ? 2 : 1) + 7) / 8 * 2;
+    return groups <= (group_size == 128 || (pair && group_size == 64) ? 2 : 1) * cus;
+}
+
+// Partial tiles for a token-tile call that shares K out: the context's workspace, if it is to be had (not while the stream is
+// being captured and it is too small: the call then runs without shares).
+bool tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
+    if (bytes == 0) return true;
+    if (hipSetDevice(ctx->device) != hipSuccess || !aq::workspace_offer(ctx->stream, &ctx->ws, bytes)) return false;
+    *tile = static_cast<float*>(ctx->ws.ptr);
+    return true;
+}
+int tok_pick(const aq_ctx* ctx, const aq::QmvArgs& t, int group_size, int bits, bool pair) {
+    const int64_t bands = (int64_t)((t.N + 15) / 16) * (pair ? 2 : 1) * (t.ksplit > 1 ? t.ksplit : 1);
+    return aq::qmvt_pick(bits, group_size, t.M, t.K, bands, t.ksplit > 1 ? t.share : (t.K + 255) / 256, pair, ctx->cu_count);
+}
 
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
-    const int ti = forced >= 0 ? forced : aq::qmvt_pick(bits, a.M, a.K, a.N, ctx->cu_count);
-    if (gather || ti < 0 || !aq::qmvt_fits(a, bits, group_size, ti, forced >= 0)) return kPass;
-    if (forced < 0 && tok_small(bits, group_size, a.M, a.K, a.N)) return kPass;
-    ctx->last_variant[0] = aq::qmvt_name(ti, a);
-    AQ_HIP(aq::qmvt_launch(ti, a, ctx->stream), "hipLaunchKernel");
+    if (gather) return kPass;
+    aq::QmvArgs t = a;
+    t.ksplit = 1;
+    t.tokens = forced < 0 ? aq::qmvt_tokens(a.M) : a.M;
+    if (forced < 0 && !tok_small(bits, group_size, a.M, a.K, a.N) && tok_halves(ctx, group_size, a.M, a.N, false)) {
+        aq::qmvt_split(bits, group_size, a.M, a.K, a.N, false, ctx->cu_count, &t.ksplit, &t.share);
+        if (!tok_tiles(ctx, aq::qmvt_tile_bytes(a.M, a.N, false, t.ksplit), &t.tile)) t.ksplit = 1;
+    } else if (forced < 0) {
+        return kPass;
+    }
+    const int ti = forced >= 0 ? forced : tok_pick(ctx, t, group_size, bits, false);
+    if (ti < 0 || !aq::qmvt_fits(t, bits, group_size, ti, forced >= 0)) return kPass;
+    ctx->last_variant[0] = aq::qmvt_name(ti, t);
+    AQ_HIP(aq::qmvt_launch(ti, t, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
 
@@ -416,11 +452,12 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
 
 // Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
 // the launch forms that put several matrices into one grid).
-bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows) {
+bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, bool pair) {
     if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(bits, group_size, M, K, rows)) return false;
-    if (bits == 4 && group_size == 64) return M >= 9 && M <= 32;
-    if (bits == 8 && group_size == 64) return (M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0) && M >= 2 && M <= 32;
-    return M <= 32 && M >= (group_size == 128 ? 5 : bits == 4 ? 3 : 2);
+    if (M > 64 || !tok_halves(ctx, group_size, M, rows, pair)) return false;
+    if (bits == 4 && group_size == 64) return M >= 9;
+    if (bits == 8 && group_size == 64) return (M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0) && M >= 2;
+    return M >= (group_size == 128 ? 5 : bits == 4 ? 3 : 2);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -873,23 +910,50 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         CallLock lk(ctx);
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
+        size_t bytes = 0;
         grid.common = all.common;
+        grid.common.tokens = aq::qmvt_tokens(M);
         for (int i = 0; i < count; i++) {
-            if (N[i] == 0 || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i])) continue;
-            const int own = aq::qmvt_pick(bits, M, K, N[i], ctx->cu_count);
-            if (own < 0 || !aq::qmvt_fits(multi_member(all, i), bits, group_size, own, false)) continue;
+            if (N[i] == 0 || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i], false)) continue;
+            aq::QmvArgs own = multi_member(grid, i);
+            own.w = all.w[i];
+            own.s = all.s[i];
+            own.b = all.b[i];
+            own.N = all.N[i];
+            aq::qmvt_split(bits, group_size, M, K, N[i], false, ctx->cu_count, &own.ksplit, &own.share);
+            const int oi = tok_pick(ctx, own, group_size, bits, false);
+            if (oi < 0 || !aq::qmvt_fits(own, bits, group_size, oi, false)) continue;
             in_grid |= 1u << i;
             grid.w[members] = all.w[i];
             grid.s[members] = all.s[i];
             grid.b[members] = all.b[i];
             grid.y[members] = all.y[i];
+            grid.ksplit[members] = own.ksplit;
+            grid.share[members] = own.share;
             grid.N[members++] = N[i];
+            bytes += aq::qmvt_tile_bytes(M, N[i], false, own.ksplit);
             total += N[i];
         }
         grid.count = members;
-        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, M, K, (int)total, ctx->cu_count) : -1;
-        for (int i = 0; ti >= 0 && i < members; i++)
-            if (!aq::qmvt_fits(multi_member(grid, i), bits, group_size, ti, false)) ti = -1;
+        float* tiles = nullptr;
+        const bool split = tok_tiles(ctx, bytes, &tiles);
+        int64_t bands = 0;
+        int runs = 1;
+        for (int i = 0; i < members; i++) {
+            if (!split) grid.ksplit[i] = 1;
+            const int ks = grid.ksplit[i], n = ks > 1 ? grid.share[i] : (K + 255) / 256;
+            grid.tile[i] = ks > 1 ? tiles : nullptr;
+            tiles += aq::qmvt_tile_bytes(M, grid.N[i], false, ks) / 4;
+            bands += (int64_t)((grid.N[i] + 15) / 16) * ks;
+            runs = n > runs ? n : runs;
+        }
+        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, group_size, M, K, bands, runs, false, ctx->cu_count) : -1;
+        for (int i = 0; ti >= 0 && i < members; i++) {
+            aq::QmvArgs one = multi_member(grid, i);
+            one.ksplit = grid.ksplit[i];
+            one.share = grid.share[i];
+            if (!aq::qmvt_fits(one, bits, group_size, ti, false)) ti = -1;
+        }
         if (ti < 0) in_grid = 0;
     }
     for (int i = 0; i < count; i++) {
@@ -899,7 +963,7 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     if (in_grid) {
         CallLock lk(ctx);
         ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
-        AQ_HIP(aq::qmvt_multi_launch(ti, grid, ctx->stream), "hipLaunchKernel");
+        AQ_HIP(aq::qmvt_multi_launch(ti, grid, bits, ctx->stream), "hipLaunchKernel");
     }
     return AQ_OK;
 }
@@ -1330,7 +1394,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
             return AQ_OK;
         }
     }
-    if (M > 1 && tok_runs(ctx, bits, group_size, M, K, N)) {
+    if (M > 1 && tok_runs(ctx, bits, group_size, M, K, N, true)) {
         // the token-tile kernels with half of a workgroup's rows in either matrix
         aq::QmvArgs a{};
         a.x = static_cast<const uint16_t*>(x);
@@ -1349,7 +1413,10 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         a.routes = 1;
         a.act = act;
         CallLock lk(ctx);
-        const int ti = aq::qmvt_pick_pair(bits, M, K, N, ctx->cu_count);
+        a.tokens = aq::qmvt_tokens(M);
+        aq::qmvt_split(bits, group_size, M, K, N, true, ctx->cu_count, &a.ksplit, &a.share);
+        if (!tok_tiles(ctx, aq::qmvt_tile_bytes(M, N, true, a.ksplit), &a.tile)) a.ksplit = 1;
+        const int ti = tok_pick(ctx, a, group_size, bits, true);
         if (ti >= 0 && aq::qmvt_pair_supported(ti) && aq::qmvt_fits(a, bits, group_size, ti, false)) {
             ctx->last_variant[0] = "qmv_gate_up_tok";
             AQ_HIP(aq::qmvt_pair_launch(ti, a, ctx->stream), "hipLaunchKernel");

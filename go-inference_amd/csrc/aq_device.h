@@ -121,6 +121,17 @@ __device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
     p[1] = high_halves(at(2), at(3));
 }
 
+// Eight 4-bit codes as four bf16 pairs (c0,c2)(c4,c6)(c1,c3)(c5,c7).  The bytes 0 .. 15 read as fp8 (e4m3) are 2^-9 times their
+// own value, subnormals and the first binade having one unit in the last place, so that the packed conversion to bf16 with a
+// scale of 2^9 yields two codes an instruction, exactly: seven instructions a word, against fourteen of unpack4_centred.
+__device__ __forceinline__ void unpack4_codes(uint32_t w, uint32_t p[4]) {
+    const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
+    p[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));
+    p[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, true));
+    p[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, false));
+    p[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(odd, 512.0f, true));
+}
+
 // scale * code + bias in two roundings.
 __device__ __forceinline__ float affine_weight(float scale, float code, float bias) {
 #pragma clang fp contract(off)

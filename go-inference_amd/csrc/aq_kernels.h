@@ -50,6 +50,10 @@ struct QmvArgs {
     const RouteChunk* chunks;
     const int32_t* route_x;
     const int32_t* route_of;
+    // token-tile kernels: shares of K (0, 1: none), 256-code runs per share, the fp32 partial tiles; rows of x per workgroup
+    int ksplit, share;
+    float* tile;
+    int tokens;
     int act;             // kActGeluTanh or kActSilu
     // head kernels only (aq_qmv_head.hip): y is uint64 best[M] (argmax) or uint64 scores[M, N]
     const int32_t* suppress;  // token ids that may not win, or nullptr
@@ -84,6 +88,8 @@ struct QmvMultiArgs {
     void* y[kQmvMultiMax];
     int N[kQmvMultiMax];
     int block_end[kQmvMultiMax];  // filled by the launcher: first workgroup past matrix i
+    int ksplit[kQmvMultiMax], share[kQmvMultiMax];  // token-tile kernels, as in QmvArgs
+    float* tile[kQmvMultiMax];
 };
 // dot2 kernels only: 4 wavefronts a workgroup, `rows` output rows per wavefront, m = 1..4 activation rows.
 bool qmv_multi_supported(int bits, int m, int rows);
@@ -167,25 +173,45 @@ hipError_t head_fold_launch(const unsigned long long* partial, int count, unsign
 bool qmvd_multi_supported(int idx);
 hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
 
-// Token-tile MFMA matvec kernels (aq_qmv_tok.hip; codes of 4 or 8 bits in groups of 32, 64 or 128, up to 32 activation rows
-// as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch, no scratch memory).  kind 6 in QmvVariant.
+// Token-tile MFMA matvec kernels (aq_qmv_tok.hip; codes of 4 or 8 bits in groups of 32, 64 or 128, up to 64 activation rows
+// as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch without scratch memory, or shares of K and a sum of
+// their partial tiles).  kind 6 in QmvVariant.
 int qmvt_variant_count();
 const QmvVariant* qmvt_variant(int idx);
 // (exact_only: groups of 64 with K a multiple of 256 only, what a forced variant takes)
 bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_only);
 const char* qmvt_name(int idx, const QmvArgs& a);  // the kernel qmvt_launch runs for this call
+// (a.ksplit, a.share and a.tile: see qmvt_split)
 hipError_t qmvt_launch(int idx, const QmvArgs& a, hipStream_t stream);
-int qmvt_pick(int bits, int M, int K, int rows, int cu_count);
+// Rows of x per workgroup (a.tokens): all of up to 32, else half of them.
+int qmvt_tokens(int M);
+// How a matrix of N rows (pair: two) shares K out over workgroups, a function of the matrix's own call alone so that it has the
+// same bytes in a grid of several: 1 share, or more whose partial tiles take qmvt_tile_bytes.
+void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share);
+size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit);
+// The variant for `sets` sets of 16 weight rows times their shares of K, the longest share being `runs` runs of 256 codes; or -1.
+int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count);
 // Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
 // sums are those of qmvt_launch.
-hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
-int qmvt_pick_pair(int bits, int M, int K, int N, int cu_count);
+hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t stream);
 bool qmvt_pair_supported(int idx);
 hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream);
 // Expert slabs with the routes grouped by expert (a.chunks, a.route_x, a.route_of; chunks of up to `tokens` = 16 or 32
 // routes; most_chunks entries in the list); pair as above.
 bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair);
 hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream);
+// Partial tiles [ksplit][M][N] ([ksplit][M][gate N | up N]) added in order, the activation applied for a pair, and dense groups
+// of 32 that are not finite formed again (plain_dot_g32).  Matrices with tile null are left alone.
+struct TokReduceArgs {
+    const uint16_t* x;
+    int M, K, bits, gs_shift, out_f32, act, pair, count;
+    const uint32_t* w[kQmvMultiMax];  // (pair: gate, up)
+    const uint16_t *s[kQmvMultiMax], *b[kQmvMultiMax];
+    void* y[kQmvMultiMax];
+    int N[kQmvMultiMax], ksplit[kQmvMultiMax];
+    const float* tile[kQmvMultiMax];
+};
+hipError_t tok_reduce_launch(const TokReduceArgs& a, hipStream_t stream);
 
 // lm_head kernels (aq_qmv_head.hip), one activation row: the projection with its epilogue replaced by
 //   fuse 3: best[0] = max over rows of pack(score, row): every wavefront stores its own maximum into

@@ -1,9 +1,12 @@
-// The token-tile kernels of aq_qmv_tok.h for 4-bit codes, and the host side of both widths: choice and launch.
+// The token-tile kernels of aq_qmv_tok.h for 4-bit codes, the sum of partial tiles, and the host side of both widths: choice and
+// launch.
 #include "aq_qmv_tok.h"
+
+#include <cmath>
 
 namespace aq {
 
-static const QmvTokEntry kEntries4[kTokPerWidth] = {AQ_QMVT_SET(4)};
+static const QmvTokEntry kEntries4[kTokPerWidth] = {AQ_QMVT_SET(4, 2)};
 const QmvTokEntry* tok_entries_4() { return kEntries4; }
 
 static const QmvTokEntry& tok_entry(int idx) { return idx < kTokPerWidth ? tok_entries_4()[idx] : tok_entries_8()[idx - kTokPerWidth]; }
@@ -14,89 +17,117 @@ const QmvVariant* qmvt_variant(int idx) {
     return &tok_entry(idx).v;
 }
 
-// (of a gated pair: one form for both matrices, so the alignment of either decides it)
-static int tok_form(const QmvArgs& a) {
-    const uintptr_t al8 = reinterpret_cast<uintptr_t>(a.s) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.s2) |
-                          reinterpret_cast<uintptr_t>(a.b2);
-    if (a.gs_shift == 6 && a.K % 256 == 0 && (al8 & 7) == 0) return kTokExact;
-    return a.gs_shift == 5 ? kTokG32 : kTokAny;
-}
-static size_t tok_lds_bytes(const QmvTokEntry& e, int K, int form) {
-    const size_t scales = (size_t)e.wg_rows * ((K + 255) / 256 + 1) * (form == kTokG32 ? 32 : 16);
-    if (form == kTokExact) return scales + (size_t)e.lds;
-    return scales > (size_t)e.lds ? scales : (size_t)e.lds;
+static bool tok_whole_runs(const QmvArgs& a) { return a.gs_shift == 6 && a.K % 256 == 0; }
+static int tok_runs_of(const QmvArgs& a) { return a.ksplit > 1 ? a.share : (a.K + 255) / 256; }
+static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs) {
+    const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.ts);
+    const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4;
+    return staged > sums ? staged : sums;
 }
 
 bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_only) {
     const QmvVariant* v = qmvt_variant(idx);
     if (!v || bits != v->bits || (group_size != 32 && group_size != 64 && group_size != 128)) return false;
-    // (K up to 16384, as qmvt_pick has it: what the tests cover; longer rows go to the kernels that split K)
-    if (a.M < 1 || a.M > v->m || a.N < 1 || a.K < 64 || a.K % 64 != 0 || a.K > kTokMaxK) return false;
+    // (K up to 16384: what the tests cover; longer rows go to the kernels that split K)
+    if (a.M < 1 || (a.M > v->m && (exact_only || a.M > kTokMax || a.tokens < 1 || a.tokens > v->m)) || a.N < 1 || a.K < 64 || a.K % 64 != 0 || a.K > kTokMaxK) return false;
     const uintptr_t al16 = reinterpret_cast<uintptr_t>(a.x) | reinterpret_cast<uintptr_t>(a.w) | reinterpret_cast<uintptr_t>(a.w2);
     if (al16 & 15) return false;
     // 32-bit byte offsets into the packed matrix and into x
     if ((uint64_t)a.N * (uint64_t)(a.K * bits / 8) >= (1ull << 32)) return false;
-    const QmvTokEntry& e = tok_entry(idx);
-    const int form = tok_form(a);
-    if (form == kTokExact) {
-        if (e.wg_rows * (a.K / 256) > tok16_stage_pieces(v->waves) * v->waves * kWave) return false;
-    } else {
-        const uintptr_t sb = reinterpret_cast<uintptr_t>(a.s) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.s2) |
-                             reinterpret_cast<uintptr_t>(a.b2);
-        if (exact_only || (sb & 15)) return false;
-    }
-    return tok_lds_bytes(e, a.K, form) <= 160 * 1024;
+    // (scales of any alignment would do; which calls run here by it is kept: 8 bytes where K is whole runs in groups of 64, else 16)
+    const uintptr_t sb = reinterpret_cast<uintptr_t>(a.s) | reinterpret_cast<uintptr_t>(a.b) | reinterpret_cast<uintptr_t>(a.s2) |
+                         reinterpret_cast<uintptr_t>(a.b2);
+    const bool exact = tok_whole_runs(a) && (sb & 7) == 0;
+    if (!exact && (exact_only || (sb & 15))) return false;
+    return tok_lds_bytes(tok_entry(idx), group_size == 32, tok_runs_of(a)) <= 160 * 1024;
 }
 
-const char* qmvt_name(int idx, const QmvArgs& a) { return tok_entry(idx).name[tok_form(a)]; }
+const char* qmvt_name(int idx, const QmvArgs& a) { return tok_entry(idx).name[a.gs_shift == 5 ? 2 : tok_whole_runs(a) ? 0 : 1]; }
+
+static int tok_blocks(const QmvTokEntry& e, int M, int tokens, int N, bool pair, int ksplit) {
+    const int outs = e.wg_rows / (pair ? 2 : 1);
+    const int blocks = (N + outs - 1) / outs * (ksplit > 1 ? ksplit : 1), parts = (M + tokens - 1) / tokens;
+    return parts > 1 ? (blocks + 7) / 8 * 8 * parts : blocks;
+}
+int qmvt_tokens(int M) { return M <= 32 ? M : (M + 1) / 2; }
+
+static hipError_t tok_reduce_one(const QmvArgs& a, int bits, bool pair, hipStream_t stream) {
+    if (a.ksplit <= 1) return hipSuccess;
+    TokReduceArgs r{};
+    r.x = a.x;
+    r.M = a.M;
+    r.K = a.K;
+    r.bits = bits;
+    r.gs_shift = a.gs_shift;
+    r.out_f32 = a.out_f32;
+    r.act = a.act;
+    r.pair = pair;
+    r.count = 1;
+    r.w[0] = a.w, r.s[0] = a.s, r.b[0] = a.b;
+    r.w[1] = a.w2, r.s[1] = a.s2, r.b[1] = a.b2;
+    r.y[0] = a.y;
+    r.N[0] = a.N;
+    r.ksplit[0] = a.ksplit;
+    r.tile[0] = a.tile;
+    return tok_reduce_launch(r, stream);
+}
+
+static hipError_t tok_launch(int idx, QmvArgs a, bool pair, hipStream_t stream) {
+    const QmvTokEntry& e = tok_entry(idx);
+    if (a.tokens < 1) a.tokens = a.M;
+    const bool g32 = a.gs_shift == 5;
+    const QmvTokKernel fn = pair ? e.pair[g32] : e.fn[g32];
+    const size_t lds = tok_lds_bytes(e, g32, tok_runs_of(a));
+    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
+    hipLaunchKernelGGL(fn, dim3((unsigned)tok_blocks(e, a.M, a.tokens, a.N, pair, a.ksplit)), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
+    if (hipError_t rc = hipGetLastError()) return rc;
+    return tok_reduce_one(a, e.v.bits, pair, stream);
+}
 
 hipError_t qmvt_launch(int idx, const QmvArgs& a, hipStream_t stream) {
     if (idx < 0 || idx >= qmvt_variant_count()) return hipErrorInvalidValue;
-    const QmvTokEntry& e = tok_entry(idx);
-    const int form = tok_form(a);
-    const QmvTokKernel fn = e.fn[form];
-    const size_t lds = tok_lds_bytes(e, a.K, form);
-    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
-    const int wg_rows = e.wg_rows;
-    hipLaunchKernelGGL(fn, dim3((unsigned)((a.N + wg_rows - 1) / wg_rows)), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
-    return hipGetLastError();
+    return tok_launch(idx, a, false, stream);
 }
 
-hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream) {
+hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t stream) {
     if (idx < 0 || idx >= qmvt_variant_count() || ma.count < 1 || ma.count > kQmvMultiMax) return hipErrorInvalidValue;
     const QmvTokEntry& e = tok_entry(idx);
-    int form = kTokExact;
+    const bool g32 = ma.common.gs_shift == 5;
+    const QmvTokMultiKernel fn = e.multi[g32];
+    int blocks = 0, runs = 1;
+    TokReduceArgs r{};
+    r.x = ma.common.x;
+    r.M = ma.common.M;
+    r.K = ma.common.K;
+    r.bits = bits;
+    r.gs_shift = ma.common.gs_shift;
+    r.out_f32 = ma.common.out_f32;
+    r.count = ma.count;
+    bool split = false;
     for (int i = 0; i < ma.count; i++) {
-        QmvArgs one = ma.common;
-        one.s = ma.s[i];
-        one.b = ma.b[i];
-        const int f = tok_form(one);
-        form = f > form ? f : form;
-    }
-    const QmvTokMultiKernel fn = e.multi[form];
-    const size_t lds = tok_lds_bytes(e, ma.common.K, form);
-    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
-    int blocks = 0;
-    for (int i = 0; i < ma.count; i++) {
-        blocks += (ma.N[i] + e.wg_rows - 1) / e.wg_rows;
+        blocks += tok_blocks(e, ma.common.M, ma.common.tokens, ma.N[i], false, ma.ksplit[i]);
         ma.block_end[i] = blocks;
+        const int n = ma.ksplit[i] > 1 ? ma.share[i] : (ma.common.K + 255) / 256;
+        runs = n > runs ? n : runs;
+        split |= ma.ksplit[i] > 1;
+        r.w[i] = ma.w[i], r.s[i] = ma.s[i], r.b[i] = ma.b[i];
+        r.y[i] = ma.y[i];
+        r.N[i] = ma.N[i];
+        r.ksplit[i] = ma.ksplit[i];
+        r.tile[i] = ma.ksplit[i] > 1 ? ma.tile[i] : nullptr;
     }
+    const size_t lds = tok_lds_bytes(e, g32, runs);
+    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, ma);
-    return hipGetLastError();
+    if (hipError_t rc = hipGetLastError()) return rc;
+    return split ? tok_reduce_launch(r, stream) : hipSuccess;
 }
 
 bool qmvt_pair_supported(int idx) { return idx >= 0 && idx < qmvt_variant_count() && tok_entry(idx).pair[0] != nullptr; }
 
 hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream) {
     if (!qmvt_pair_supported(idx)) return hipErrorInvalidValue;
-    const QmvTokEntry& e = tok_entry(idx);
-    const int form = tok_form(a);
-    const QmvTokKernel fn = e.pair[form];
-    const size_t lds = tok_lds_bytes(e, a.K, form);
-    if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
-    const int outs = e.wg_rows / 2;
-    hipLaunchKernelGGL(fn, dim3((unsigned)((a.N + outs - 1) / outs)), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
-    return hipGetLastError();
+    return tok_launch(idx, a, true, stream);
 }
 
 bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair) {
@@ -107,44 +138,154 @@ bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair) {
     if (al & 15) return false;
     // 32-bit byte offsets into an expert's rows and into x
     if ((uint64_t)a.expert_rows * (uint64_t)(a.K * bits / 8) >= (1ull << 32) || (uint64_t)a.x_rows * (uint64_t)a.K * 2 >= (1ull << 32)) return false;
-    // an expert's scales are read in 16-byte pieces from its first row on
+    // (which slabs run here is kept: those whose first row's scales lie on 16 bytes)
     const int64_t groups = a.K / group_size;
     if ((a.expert_rows * groups) % 8 || (a.row_base * groups) % 8 || (pair && (a.row_base2 * groups) % 8)) return false;
-    return tok_lds_bytes(tok_entry(0), a.K, group_size == 32 ? kTokG32 : kTokAny) <= 160 * 1024;
+    return tok_lds_bytes(tok_entry(1), group_size == 32, (a.K + 255) / 256) <= 160 * 1024;
 }
 
 hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream) {
-    const int idx = (bits == 8 ? kTokPerWidth : 0) + (tokens == 32 ? 3 : 0);  // (four sets of rows: the first of a token count)
+    const int idx = (bits == 8 ? kTokPerWidth : 0) + (tokens == 32 ? 5 : 1);  // (four sets of rows: the second of a token count)
     const QmvTokEntry& e = tok_entry(idx);
-    const int form = a.gs_shift == 5 ? kTokG32 : kTokAny;
-    const QmvTokKernel fn = e.grouped[form == kTokG32][pair ? 1 : 0];
+    const bool g32 = a.gs_shift == 5;
+    const QmvTokKernel fn = e.grouped[g32][pair ? 1 : 0];
     if (!fn || e.v.m != tokens) return hipErrorInvalidValue;
-    const size_t lds = tok_lds_bytes(e, a.K, form);
+    const size_t lds = tok_lds_bytes(e, g32, (a.K + 255) / 256);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     const int outs = e.wg_rows / (pair ? 2 : 1);
     hipLaunchKernelGGL(fn, dim3((unsigned)((a.N + outs - 1) / outs), (unsigned)most_chunks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
     return hipGetLastError();
 }
 
-// The variant for `rows` weight rows in all, or -1.
-int qmvt_pick(int bits, int M, int K, int rows, int cu_count) {
+size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit) {
+    return ksplit > 1 ? ((size_t)ksplit * M * N * (pair ? 2 : 1) * 4 + 255) & ~(size_t)255 : 0;
+}
+
+// Microseconds of a call: `fixed` (launch, first requests, the meeting in LDS and the store), and per pass of a workgroup (eight
+// runs of 256 codes) `pass` for x and `set` for each of its sets of 16 weight rows.  From runs at K = 1024 to 14336 with one to eight
+// sets per workgroup, 1024 to 28672 rows of weights, 12 and 24 rows of x.
+struct TokCost {
+    double fixed, pass, set;
+};
+static const TokCost& tok_cost(int bits, int group_size, int tokens) {
+    // [8 bit][groups of 32][more than 16 rows of x]
+    static const TokCost kCost[2][2][2] = {{{{3.0, 1.36, 0.62}, {2.8, 2.7, 0.85}}, {{3.8, 1.2, 0.79}, {5.2, 2.1, 1.29}}},
+                                           {{{3.7, 1.3, 1.04}, {3.7, 2.7, 1.18}}, {{4.0, 1.3, 1.15}, {4.0, 2.7, 1.35}}}};
+    return kCost[bits == 8][group_size == 32][tokens > 16];
+}
+// Sets of 16 weight rows per workgroup: the fewest that leave every CU at most one workgroup, for a second round costs more than
+// longer workgroups (us on one, two, four, eight sets; 24 rows of x, K = 2816, groups of 64: 4096 rows of weights 8.3 / 9.6 / 11.9 /
+// 17.2, 8192 15.1 / 10.0 / 12.1 / 17.2, 14336 27.9 / 18.1 / 12.3 / 17.4, 2 x 14336 35.1 / 23.9 / 18.3 from two on).
+static int tok_sets(int64_t sets, int cus) {
+    for (int rs = 1; rs < 8; rs *= 2)
+        if ((sets + rs - 1) / rs <= cus) return rs;
+    return 8;
+}
+
+// Shares of K where a workgroup would make several passes: the shares' workgroups carry more rows each, and a second launch adds
+// their partial tiles, which costs about 2.5 us and one more per megabyte (12 / 24 rows of x by 4096 x 14336 whole 16.9 / 27.9 us,
+// eight shares 13.5 / 18.0; 1024 x 14336 16.1 / 27.0, 10.2 / 12.8; at K = 4096, two passes, shares win nothing).
+void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share) {
+    const int cus = cu_count > 0 ? cu_count : 256, quads = (K + 255) / 256, tokens = qmvt_tokens(M);
+    const TokCost& c = tok_cost(bits, group_size, tokens);
+    *ksplit = 1;
+    *share = quads;
+    if ((bits != 4 && bits != 8) || M > kTokMax || K % 64 != 0 || K > kTokMaxK) return;  // (no call of these kernels)
+    const int64_t sets = (int64_t)((N + 15) / 16) * (pair ? 2 : 1) * ((M + tokens - 1) / tokens);
+    double best = 1e30;
+    for (int ks = 1; ks <= kTokShares && ks <= quads; ks++) {
+        const int sh = (quads + ks - 1) / ks, n = (quads + sh - 1) / sh;
+        if (n != ks) continue;
+        const int rs = tok_sets(sets * n, cus);
+        const double rounds = std::ceil((double)((sets * n + rs - 1) / rs) / cus);
+        const int whole = (sh + kTokWaves - 1) / kTokWaves;
+        const double passes = sh > kTokWaves ? 0.5 * (whole + (double)sh / kTokWaves) : 1.0;  // (a part of a pass costs more than its part)
+        double us = c.fixed + rounds * passes * (c.pass + rs * c.set);
+        if (n > 1) us = 1.1 * us + 2.5 + (double)qmvt_tile_bytes(M, N, pair, n) / 1e6;  // (a tenth: no shares for next to nothing)
+        if (us < best) best = us, *ksplit = n, *share = sh;
+    }
+}
+
+int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count) {
     if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK) return -1;
-    const int cus = cu_count > 0 ? cu_count : 256;
-    // eight wavefronts, one run each per pass; one set of 16 tokens up to 16 rows of x, else two; as many sets of 16
-    // weight rows per workgroup (fewer reads of x) as still leave three quarters of the CUs a workgroup
-    const int most = M <= 16 ? 16 : 32;
-    const int rs = (rows + 63) / 64 >= (cus * 3) / 4 ? 4 : (rows + 31) / 32 >= (cus * 3) / 4 ? 2 : 1;
-    for (int i = 0; i < qmvt_variant_count(); i++) {
-        const QmvVariant& v = tok_entry(i).v;
-        if (v.bits == bits && v.m == most && v.rows == rs) return i;
+    const int cus = cu_count > 0 ? cu_count : 256, tokens = qmvt_tokens(M), most = tokens <= 16 ? 16 : 32;
+    int rs = tok_sets(sets * ((M + tokens - 1) / tokens), cus);
+    if (pair && rs == 1) rs = 2;
+    for (int i = 0; i < qmvt_variant_count(); i++) {  // (listed with eight, four, two, one sets)
+        const QmvTokEntry& e = tok_entry(i);
+        if (e.v.bits != bits || e.v.m != most || e.v.rows > rs) continue;
+        if (tok_lds_bytes(e, group_size == 32, runs) <= 160 * 1024) return i;
     }
     return -1;
 }
-// The same for the gated pair of two matrices of N rows each (at least two sets of rows: one of either).
-int qmvt_pick_pair(int bits, int M, int K, int N, int cu_count) {
-    const int idx = qmvt_pick(bits, M, K, 2 * N, cu_count);
-    if (idx < 0 || qmvt_pair_supported(idx)) return idx;
-    return idx - 1;  // (the entries of a token count are listed with 4, 2, 1 sets)
+
+// V columns a thread.  grid.y: the matrices.
+template <int V>
+__global__ __launch_bounds__(256) void tok_reduce_kernel(const TokReduceArgs a) {
+    const int mi = blockIdx.y;
+    const float* const tile = a.tile[mi];
+    if (!tile) return;
+    const int N = a.N[mi], shares = a.ksplit[mi], stride = a.pair ? 2 * N : N;
+    const int64_t mn = (int64_t)a.M * stride;
+    const int per_row = N / V;
+    auto sum = [&](int64_t at, float (&v)[V]) {
+        float t[kTokShares][V];
+#pragma unroll
+        for (int s = 0; s < kTokShares; s++) {  // (requested together: a chain of loads is a chain of latencies)
+            if (s >= shares) break;
+            if constexpr (V == 4) {
+                const float4 f = *reinterpret_cast<const float4*>(tile + s * mn + at);
+                t[s][0] = f.x, t[s][1] = f.y, t[s][2] = f.z, t[s][3] = f.w;
+            } else {
+                t[s][0] = tile[s * mn + at];
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < kTokShares; s++)
+            if (s < shares)
+#pragma unroll
+                for (int e = 0; e < V; e++) v[e] = s ? v[e] + t[s][e] : t[s][e];
+    };
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= (int64_t)a.M * per_row) return;
+    const int m = (int)(i / per_row), c = (int)(i - (int64_t)m * per_row) * V;
+    float v[V], u[V];
+    sum((int64_t)m * stride + c, v);
+    if (a.pair) sum((int64_t)m * stride + N + c, u);
+#pragma unroll
+    for (int e = 0; e < V; e++) {
+        if (a.gs_shift == 5) {  // (dense groups of 32 keep what the any-width kernel makes of infinities)
+#pragma nounroll
+            for (int part = 0; part < (a.pair ? 2 : 1); part++) {
+                if (!not_finite(part ? u[e] : v[e])) continue;
+                const int mat = a.pair ? part : mi;
+                const size_t row = (size_t)(c + e), groups = (size_t)(a.K >> 5);
+                const float f = plain_dot_g32(a.x + (size_t)m * a.K, a.w[mat] + row * (size_t)(a.K / 32 * a.bits), a.s[mat] + row * groups,
+                                              a.b[mat] + row * groups, a.K, a.bits);
+                if (part) u[e] = f; else v[e] = f;
+            }
+        }
+        if (a.pair) v[e] = fmul_unfused(act_value(a.act, v[e]), u[e]);
+        const int64_t at = (int64_t)m * N + c + e;
+        if (a.out_f32)
+            static_cast<float*>(a.y[mi])[at] = v[e];
+        else
+            static_cast<uint16_t*>(a.y[mi])[at] = f32_to_bf16_bits(v[e]);
+    }
+}
+
+hipError_t tok_reduce_launch(const TokReduceArgs& a, hipStream_t stream) {
+    int64_t most = 0;
+    bool by4 = true;
+    for (int i = 0; i < a.count; i++) {
+        if (!a.tile[i]) continue;
+        most = (int64_t)a.M * a.N[i] > most ? (int64_t)a.M * a.N[i] : most;
+        by4 = by4 && a.N[i] % 4 == 0;
+    }
+    if (most == 0) return hipSuccess;
+    const int64_t grid = (most / (by4 ? 4 : 1) + 255) / 256;
+    hipLaunchKernelGGL(by4 ? tok_reduce_kernel<4> : tok_reduce_kernel<1>, dim3((unsigned)grid, (unsigned)a.count), dim3(256), 0, stream, a);
+    return hipGetLastError();
 }
 
 }  // namespace aq

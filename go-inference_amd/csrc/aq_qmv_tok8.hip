@@ -3,7 +3,7 @@
 
 namespace aq {
 
-static const QmvTokEntry kEntries8[kTokPerWidth] = {AQ_QMVT_SET(8)};
+static const QmvTokEntry kEntries8[kTokPerWidth] = {AQ_QMVT_SET(8, 1)};
 const QmvTokEntry* tok_entries_8() { return kEntries8; }
 
 }  // namespace aq
