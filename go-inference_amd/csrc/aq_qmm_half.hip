@@ -65,6 +65,23 @@ __device__ __forceinline__ f16x8_t expand_bytes(uint2 w) {
     return __builtin_bit_cast(f16x8_t, u);
 }
 
+// the value of lane `lane ^ BIT`
+template <int BIT>
+__device__ __forceinline__ float lane_xor(float v) {
+    const int i = __float_as_int(v);
+    if constexpr (BIT == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0xb1, 0xf, 0xf, false));  // quad_perm 1 0 3 2
+    if constexpr (BIT == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x4e, 0xf, 0xf, false));  // quad_perm 2 3 0 1
+    if constexpr (BIT == 4) return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x101f));
+    if constexpr (BIT == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x128, 0xf, 0xf, false));  // row_ror 8
+    if constexpr (BIT == 16) return __int_as_float(__builtin_amdgcn_permlane16_swap(i, i, false, false)[(threadIdx.x >> 4 & 1) ^ 1]);
+    return __int_as_float(__builtin_amdgcn_permlane32_swap(i, i, false, false)[(threadIdx.x >> 5 & 1) ^ 1]);
+}
+
+typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
+}
+
 __device__ __forceinline__ uint32_t dup16(uint32_t h) { return (h & 0xffffu) | (h << 16); }
 
 // 2^e for the largest finite magnitude `mag` (bf16 bits without the sign) such that mag * 2^e has binary
@@ -81,10 +98,13 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 }  // namespace
 
 // ---- pass over x ----------------------------------------------------------------------------
-// One workgroup per eight rows of x (rows padded to a multiple of 32 are written as zeros).  Thread (r = tid % 8,
-// p = tid / 8) works on 16-byte pieces p, p + 64, ... of row r: a load instruction then covers whole 128-byte lines of
-// eight rows, and the eight rows' slots of a fragment are 128 contiguous bytes of a store instruction (one row per
-// workgroup wrote 16 bytes per kilobyte and took 18 us for 34 MB).
+// One workgroup per ROWS rows of x (rows padded to a multiple of 32 are written as zeros).  Thread (r = tid % ROWS, p = tid /
+// ROWS) works on 16-byte pieces p, p + 512 / ROWS, ... of row r.  The slots of eight rows in a fragment are one 128-byte line;
+// with fewer rows a workgroup the others' run on the same XCD at about the same time, so that a line is put together in its L2
+// (spread over the XCDs two rows a workgroup took 33 us for 2048 x 15360, one row 56; here 22 and 32).
+// Bound: latency of two dependent passes in few workgroups, then memory (2048 x 15360: 126 MB in 22 us, 5.7 TB/s).  Eight rows a
+// workgroup from 1024 rows on, one below, magnitudes and block sums value by value -> here (us): 509 x 3840 8.0 -> 6.1, 509 x
+// 15360 16.8 -> 10.2, 777 x 10240 17.6 -> 10.1, 1024 x 15360 35.8 -> 13.3, 2048 x 4096 11.9 -> 9.9, 2048 x 15360 37.8 -> 22.4.
 // xf: [mblks][K/16][64 lanes][8] fp16, the A-fragment order of the tile kernels (4-bit slot order), values
 //     x * 2^e with e chosen per row;
 // xs: [mblks][ceil(G/4)][32 rows][4 blocks][hi, lo] bf16: 2^e * sum of x over each 64-code block, hi + lo (a wavefront's
@@ -92,8 +112,6 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // rs: [mblks * 32] fp32: 2^-e.
 //
 // GRP 32: xs holds the sums of the 32-code halves, [mblks][ceil(G/4)][half][32 rows][4 blocks][hi, lo].
-// ROWS rows of x per workgroup: eight, whose slots of a fragment are one 128-byte line of a store, or one where eight rows
-// a workgroup would leave most of the chip idle (21 x 15360: 4 workgroups).
 // GROUPED: row i of the fragments is row route_x[i] of x (the list of routes sorted by expert; negative: zeros), and rows
 // past *live_rows are left alone.
 constexpr int kPrepThreads = 512;
@@ -105,10 +123,12 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
                                                          uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K,
                                                          const int32_t* __restrict__ route_x, const int32_t* __restrict__ live_rows) {
     constexpr int STEP = kPrepThreads / ROWS;  // pieces of a row between a thread's pieces
-    if (live_rows && (int)blockIdx.x * ROWS >= *live_rows) return;
+    // the workgroups of eight rows, which fill the same lines of xf, on one XCD
+    const int seq = (int)blockIdx.x >> 3, row0 = (seq / (8 / ROWS) * 8 + ((int)blockIdx.x & 7)) * 8 + seq % (8 / ROWS) * ROWS;
+    if (row0 >= (M + 31) / 32 * 32 || (live_rows && row0 >= *live_rows)) return;
     const int tid = threadIdx.x;
     const int r = tid % ROWS, p0 = tid / ROWS;
-    const int row = (int)blockIdx.x * ROWS + r;
+    const int row = row0 + r;
     const int G = K / 64;
     const int G4 = (G + 3) / 4;
     const int pieces = K / 8;
@@ -116,31 +136,38 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
     const bool live = row < M && from >= 0;
     const uint16_t* const xrow = x + (int64_t)(live ? from : 0) * K;
     __shared__ uint32_t wave_mag[kPrepThreads / kWave][ROWS];
-    uint32_t mag = 0;
-    auto scan = [&](const uint4& v) {
-        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const uint32_t lo = w[i] & 0x7fffu, hi = (w[i] >> 16) & 0x7fffu;
-            if (lo < 0x7f80u) mag = max(mag, lo);  // inf and NaN do not set the scale
-            if (hi < 0x7f80u) mag = max(mag, hi);
-        }
-    };
-    // up to kPrepHold pieces per thread (K up to 4096 with eight rows) are requested together and stay in registers for the
-    // second pass
-    const bool held = pieces <= STEP * kPrepHold;
+    // kPrepHold pieces per thread are requested together; they stay in registers for the second pass if they are all there is
     uint4 hold[kPrepHold];
-    if (held) {
+    auto fetch = [&](int p) {
 #pragma unroll
         for (int i = 0; i < kPrepHold; i++) {
-            const int p = p0 + STEP * i;
             hold[i] = make_uint4(0u, 0u, 0u, 0u);
-            if (live && p < pieces) hold[i] = *reinterpret_cast<const uint4*>(xrow + p * 8);
+            if (live && p + p0 + STEP * i < pieces) hold[i] = *reinterpret_cast<const uint4*>(xrow + (p + p0 + STEP * i) * 8);
         }
+    };
+    // the largest magnitude, two values an instruction; inf and NaN do not set the scale, so a thread that has met one goes over
+    // its pieces again, value by value
+    uint32_t most = 0;
+    for (int p = 0; p < pieces; p += STEP * kPrepHold) {
+        fetch(p);
 #pragma unroll
-        for (int i = 0; i < kPrepHold; i++) scan(hold[i]);
-    } else if (live) {
-        for (int p = p0; p < pieces; p += STEP) scan(*reinterpret_cast<const uint4*>(xrow + p * 8));
+        for (int i = 0; i < kPrepHold; i++) {
+            const uint32_t w[4] = {hold[i].x, hold[i].y, hold[i].z, hold[i].w};
+#pragma unroll
+            for (int c = 0; c < 4; c++) most = max_u16x2(most, w[c] & 0x7fff7fffu);
+        }
+    }
+    uint32_t mag = max(most & 0xffffu, most >> 16);
+    if (mag >= 0x7f80u) {
+        mag = 0;
+#pragma nounroll
+        for (int p = p0; p < pieces; p += STEP) {
+#pragma nounroll
+            for (int c = 0; c < 8; c++) {
+                const uint32_t v = xrow[p * 8 + c] & 0x7fffu;
+                if (v < 0x7f80u) mag = max(mag, v);
+            }
+        }
     }
     // the threads of a wavefront that share a row are ROWS lanes apart
 #pragma unroll
@@ -162,9 +189,9 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
         sx = dot2_bf16(v.z, 0x3F803F80u, sx);
         sx = dot2_bf16(v.w, 0x3F803F80u, sx);
         // the 8 pieces of a block of this row sit in the 8 lanes ROWS apart
-        sx += __shfl_xor(sx, ROWS, kWave);
-        sx += __shfl_xor(sx, 2 * ROWS, kWave);
-        if (GRP == 64) sx += __shfl_xor(sx, 4 * ROWS, kWave);
+        sx += lane_xor<ROWS>(sx);
+        sx += lane_xor<2 * ROWS>(sx);
+        if (GRP == 64) sx += lane_xor<4 * ROWS>(sx);
         if ((c8 & (GRP / 8 - 1)) == 0) {
             const float scaled = sx * up;
             const uint32_t hi = f32_to_bf16_bits(scaled);
@@ -189,16 +216,12 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
         const int64_t frag = (int64_t)(row >> 5) * (K / 16) + g * 4 + t;
         *reinterpret_cast<f16x8_t*>(xf + (frag * 64 + h * 32 + (row & 31)) * 8) = o;
     };
-    if (held) {
+    const bool held = pieces <= STEP * kPrepHold;
+    for (int p = 0; p < pieces; p += STEP * kPrepHold) {
+        if (!held) fetch(p);
 #pragma unroll
         for (int i = 0; i < kPrepHold; i++)
-            if (p0 + STEP * i < pieces) emit(p0 + STEP * i, hold[i]);
-    } else {
-        for (int p = p0; p < pieces; p += STEP) {
-            uint4 v = {0u, 0u, 0u, 0u};
-            if (live) v = *reinterpret_cast<const uint4*>(xrow + p * 8);
-            emit(p, v);
-        }
+            if (p + p0 + STEP * i < pieces) emit(p + p0 + STEP * i, hold[i]);
     }
 }
 
@@ -1016,14 +1039,16 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     float* rs = reinterpret_cast<float*>(xs + (size_t)mblks * 32 * g4 * (g32 ? 16 : 8));
     hipError_t rc = hipSuccess;
     if (q.x_ready != qmmh_x_kind(q.bits, q.group_size)) {
-        // one row a workgroup while eight would leave CUs idle
-        const bool narrow = mblks * 4 < 128;
         typedef void (*PrepKernel)(const uint16_t*, uint16_t*, uint16_t*, float*, int, int, const int32_t*, const int32_t*);
-        static const PrepKernel kPrep[2][2][2] = {{{qmmh_prep_kernel<8, 64, 4>, qmmh_prep_kernel<8, 64, 8>}, {qmmh_prep_kernel<8, 32, 4>, qmmh_prep_kernel<8, 32, 8>}},
-                                                  {{qmmh_prep_kernel<1, 64, 4>, qmmh_prep_kernel<1, 64, 8>}, {qmmh_prep_kernel<1, 32, 4>, qmmh_prep_kernel<1, 32, 8>}}};
-        const PrepKernel fn = kPrep[narrow][g32][q.bits == 8];
-        hipLaunchKernelGGL(fn, dim3((unsigned)(narrow ? mblks * 32 : mblks * 4)), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows,
-                           q.K, q.route_x, q.live_rows);
+#define AQ_PREP(R) {{qmmh_prep_kernel<R, 64, 4>, qmmh_prep_kernel<R, 64, 8>}, {qmmh_prep_kernel<R, 32, 4>, qmmh_prep_kernel<R, 32, 8>}}
+        static const PrepKernel kPrep[3][2][2] = {AQ_PREP(1), AQ_PREP(2), AQ_PREP(8)};
+#undef AQ_PREP
+        // rows a workgroup (us, 1 / 2 / 8): 256 x 4096 4.9 / 5.2 / 7.9, 256 x 15360 8.9 / 10.1 / 26; 509 x 4096 6.8 / 6.2 / 9.0, 1024 x
+        // 15360 17.8 / 13.3 / 27; 2048 x 4096 14.7 / 11.9 / 9.9, 2048 x 15360 31.5 / 22.4 / 33
+        const int log_rows = rows <= 256 ? 0 : rows >= 1536 && q.K <= 4096 ? 3 : 1;
+        const PrepKernel fn = kPrep[log_rows == 3 ? 2 : log_rows][g32][q.bits == 8];
+        hipLaunchKernelGGL(fn, dim3((unsigned)((mblks * 4 + 7) / 8 * 8 << (3 - log_rows))), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows, q.K,
+                           q.route_x, q.live_rows);
         rc = hipGetLastError();
         if (rc != hipSuccess) return rc;
     }
