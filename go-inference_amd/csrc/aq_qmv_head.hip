@@ -317,50 +317,40 @@ __global__ __launch_bounds__(256) void packed_topk_kernel(const unsigned long lo
     topk_reduce_segment(in, count, top_k, out, (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6), threadIdx.x & (kWave - 1));
 }
 
-// Threshold path, for inputs of many segments.  The top_k-th largest of the segment maxima is a value T that
-// at least top_k entries reach (the maxima themselves), so the top_k largest entries all lie among the entries
-// >= T; for scores that are not arranged by rank that set is a little over top_k entries, and one workgroup
-// orders it by counting.  Three launches: maxima, filter, finish.  When more than kTopKCandidates entries
-// reach T (long runs of equal scores, an input sorted by score) the finish launch runs the segment-by-segment reduction
-// instead, all its rounds: as launches of their own, which left at once where there was nothing to do, the later ones took
-// 1.6 us each of every call.  Measured, us for 262144 entries and the best 40 in random order / sorted by score: rounds as
-// launches 16.8 / 53.4, in the workgroup that ends the first round last 13.7 / 83.0, as the tree 14.0 / 54.2 (best 8: 14.5 /
-// 27.9, 10.8 / 30.8, 10.9 / 29.6; best 64: 19.4 / 70.0, 16.4 / 127.5, 16.3 / 71.2).
-// A wavefront of these two kernels takes a piece of 64 * V entries: V is the largest of 16, 4, 1 that leaves at
-// least top_k pieces.
-// Head of the threshold path's scratch in 8-byte entries: the candidate counter and the tickets of the tree's nodes, 4 bytes
-// each (at most 1024 segments in nodes of 16 lists or more: 64 + 4 + 1).
+// Threshold path, for inputs of many segments: two launches.  The top_k-th largest of any set of maxima over disjoint parts of
+// the input is a value T that at least top_k entries reach (the maxima themselves), so the top_k largest entries all lie among
+// the entries >= T.
+//   lists   a workgroup takes 256 * V entries, finds T from the maxima of its 256 threads and lists the entries >= T, a little
+//           over top_k of them for scores that are not arranged by rank, beside the maxima of its four wavefronts;
+//   merge   T over all of those maxima leaves a little over top_k entries of the lists, which one workgroup orders by counting.
+// When a list overflows or more than kTopKCandidates entries are left (long runs of equal scores, an input sorted by score) the
+// second launch runs the segment-by-segment reduction instead, all its rounds: as launches of their own, which left at once where
+// there was nothing to do, the later ones took 1.6 us each of every call.
+// Bound: latency of the two launches (2 MB are read in a fraction of one).  Maxima, filter and finish as three launches -> here (us,
+// the best 40 / 64): 50220 entries 15.4 / 13.5 -> 11.0 / 11.0, 262144 13.6 / 16.3 -> 10.1 / 12.0, sorted by score 53.5 / 70.6 ->
+// 22.8 / 69.4.
+// V is the largest of 16, 4, 1 that leaves at least top_k wavefronts with a maximum each.
+// Head of the threshold path's scratch in 8-byte entries: the tickets of the tree's nodes, 4 bytes each (at most 1024 segments in
+// nodes of 16 lists or more: 64 + 4 + 1).
 constexpr int kTopKHeader = 40;
-static_assert(kTopKMax <= kTopKSegment / 16 && kTopKThresholdSegments <= 1024 && 1 + 64 + 4 + 1 <= 2 * kTopKHeader && 2 * kTopKHeader <= 256, "tickets");
-template <int V>
-__global__ __launch_bounds__(256) void topk_segment_max_kernel(const unsigned long long* __restrict__ in, int64_t count,
-                                                               unsigned long long* __restrict__ segmax, uint32_t* counter) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t segment = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t begin = segment * (kWave * V);
-    if (blockIdx.x == 0 && threadIdx.x < kTopKHeader * 2) counter[threadIdx.x] = 0;  // candidates, then the tickets of the tree
-    if (begin >= count) return;
-    unsigned long long m = 0;
-#pragma unroll
-    for (int j = 0; j < V; j++) {
-        const int64_t i = begin + j * kWave + lane;
-        const unsigned long long v = i < count ? in[i] : 0ull;
-        m = v > m ? v : m;
-    }
-    const uint32_t hi = (uint32_t)(m >> 32), lo = (uint32_t)m;
-    const uint32_t best_hi = wave_max_u32(hi);
-    const uint32_t best_lo = wave_max_u32(hi == best_hi ? lo : 0u);
-    if (lane == 0) segmax[segment] = ((unsigned long long)best_hi << 32) | best_lo;
-}
+constexpr int kTopKListMax = 2 * kTopKMax;             // entries a list holds
+static_assert(kTopKMax <= kTopKSegment / 16 && kTopKThresholdSegments <= 1024 && 64 + 4 + 1 <= 2 * kTopKHeader && 2 * kTopKHeader <= 256, "tickets");
+static_assert(kTopKMax <= kWave, "at least top_k lanes hold a maximum");
 
-// The largest t, a multiple of 2^kTopKThresholdShift, that at least top_k of the high words `key` (SV a lane, zero
-// where there is none) reach: built bit by bit from the top, every count one ballot.
-constexpr int kTopKThresholdShift = 8;
+// A t that at least top_k of the keys (SV a lane, zero where there is none) reach and no more than a multiple of
+// 2^kTopKThresholdShift below the largest such: built bit by bit from the top, every count one ballot.  The smallest of the
+// lanes' maxima is reached by 64 of them, so the bits that it shares with the largest are t's.
+constexpr int kTopKThresholdShift = 12;
 
 template <int SV>
 __device__ __forceinline__ uint32_t topk_threshold_key(const uint32_t (&key)[SV], int top_k) {
-    uint32_t t = 0;
-    for (int bit = 31; bit >= kTopKThresholdShift; bit--) {
+    uint32_t m = key[0];
+#pragma unroll
+    for (int j = 1; j < SV; j++) m = max(m, key[j]);
+    const uint32_t most = wave_max_u32(m), least = ~wave_max_u32(~m);
+    const int shared = most == least ? 32 : __builtin_clz(most ^ least);  // leading bits
+    uint32_t t = shared == 0 ? 0u : most & (0xffffffffu << (32 - shared));
+    for (int bit = 31 - shared; bit >= kTopKThresholdShift; bit--) {
         const uint32_t trial = t | (1u << bit);
         int reach = 0;
 #pragma unroll
@@ -370,34 +360,34 @@ __device__ __forceinline__ uint32_t topk_threshold_key(const uint32_t (&key)[SV]
     return t;
 }
 
-template <int SV>
-__device__ __forceinline__ uint32_t topk_threshold(const unsigned long long* __restrict__ segmax, int segments, int top_k,
-                                                   int lane) {
-    uint32_t key[SV];
-#pragma unroll
-    for (int j = 0; j < SV; j++) key[j] = j * kWave + lane < segments ? (uint32_t)(segmax[j * kWave + lane] >> 32) : 0u;
-    return topk_threshold_key<SV>(key, top_k);
-}
-
+// lists: [lists][kTopKListMax]; sizes: entries of each (more than kTopKListMax: it has overflowed); keys: the high words of the
+// wavefronts' maxima
 template <int V>
-__global__ __launch_bounds__(256) void topk_filter_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                          const unsigned long long* __restrict__ segmax, int segments,
-                                                          uint32_t* counter, unsigned long long* __restrict__ cand) {
-    const int lane = threadIdx.x & (kWave - 1);
-    const int64_t segment = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    const int64_t begin = segment * (kWave * V);
-    if (begin >= count) return;
-    unsigned long long v[V];
+__global__ __launch_bounds__(256) void topk_lists_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
+                                                         unsigned long long* __restrict__ lists, uint32_t* __restrict__ sizes,
+                                                         uint32_t* __restrict__ keys, uint32_t* tickets) {
+    __shared__ uint32_t thread_key[256];
+    __shared__ uint32_t filled;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int64_t begin = (int64_t)blockIdx.x * (256 * V);
+    if (blockIdx.x == 0 && tid < kTopKHeader * 2) tickets[tid] = 0;
+    if (tid == 0) filled = 0;
+    unsigned long long v[V], m = 0;
 #pragma unroll
     for (int j = 0; j < V; j++) {
-        const int64_t i = begin + j * kWave + lane;
+        const int64_t i = begin + j * 256 + tid;
         v[j] = i < count ? in[i] : 0ull;
     }
-    // T: at least top_k segment maxima have a high word (the score) >= T's, so at least top_k entries reach T
-    // and the top_k largest are among them; every wavefront works T out for itself from the same list
-    const uint32_t t_key = segments <= 4 * kWave ? topk_threshold<4>(segmax, segments, top_k, lane)
-                                                 : topk_threshold<kTopKThresholdSegments / kWave>(segmax, segments, top_k, lane);
-    const unsigned long long t = (unsigned long long)t_key << 32;
+#pragma unroll
+    for (int j = 0; j < V; j++) m = v[j] > m ? v[j] : m;
+    thread_key[tid] = (uint32_t)(m >> 32);
+    const uint32_t wave_key = wave_max_u32((uint32_t)(m >> 32));
+    if (lane == 0) keys[blockIdx.x * 4 + (tid >> 6)] = wave_key;
+    __syncthreads();
+    uint32_t key[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) key[j] = thread_key[j * kWave + lane];
+    const unsigned long long t = (unsigned long long)topk_threshold_key<4>(key, top_k) << 32;
     unsigned long long mask[V];
     int total = 0;
 #pragma unroll
@@ -405,77 +395,103 @@ __global__ __launch_bounds__(256) void topk_filter_kernel(const unsigned long lo
         mask[j] = __ballot(v[j] >= t && v[j] != 0);
         total += __popcll(mask[j]);
     }
-    if (total == 0) return;  // uniform over the wavefront
     uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(counter, (uint32_t)total);
+    if (lane == 0 && total) base = atomicAdd(&filled, (uint32_t)total);
     base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
     const unsigned long long below = (1ull << lane) - 1;
 #pragma unroll
     for (int j = 0; j < V; j++) {
         const uint32_t pos = base + (uint32_t)__popcll(mask[j] & below);
-        if (((mask[j] >> lane) & 1) && pos < (uint32_t)kTopKCandidates) cand[pos] = v[j];
+        if (((mask[j] >> lane) & 1) && pos < (uint32_t)kTopKListMax) lists[(int64_t)blockIdx.x * kTopKListMax + pos] = v[j];
         base += (uint32_t)__popcll(mask[j]);
     }
+    __syncthreads();
+    if (tid == 0) sizes[blockIdx.x] = filled;
 }
 
-// The candidates are distinct unless the input repeats a value, so an entry's place in the output is the number
-// of candidates above it (equal values take consecutive places in list order).
-__global__ __launch_bounds__(256) void topk_finish_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
-                                                          const uint32_t* counter, const unsigned long long* __restrict__ cand,
-                                                          unsigned long long* __restrict__ out, unsigned long long* tree,
-                                                          uint32_t* tickets) {
-    const uint32_t n = *counter;
+// Workgroup 0 merges; the others are there for the inputs that go through the tree, which all find out in the same way.
+// The candidates are distinct unless the input repeats a value, so an entry's place in the output is the number of candidates
+// above it (equal values take consecutive places).
+constexpr int kMergeThreads = 1024, kTreeWaves = 4;  // (the tree runs on a few wavefronts of many workgroups)
+template <int SV>
+__global__ __launch_bounds__(kMergeThreads) void topk_merge_kernel(const unsigned long long* __restrict__ in, int64_t count, int top_k,
+                                                                   const unsigned long long* __restrict__ lists,
+                                                                   const uint32_t* __restrict__ sizes, const uint32_t* __restrict__ keys,
+                                                                   int nlists, unsigned long long* __restrict__ out,
+                                                                   unsigned long long* tree, uint32_t* tickets) {
+    constexpr int WAVES = kMergeThreads / kWave;
+    constexpr int PER_WAVE = SV * 16 / WAVES;  // lists a wavefront takes (16 SV of them at the most)
+    __shared__ unsigned long long c[kTopKCandidates];
+    __shared__ uint32_t filled;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    if (tid == 0) filled = 0;
+    uint32_t key[SV], size[PER_WAVE];
+#pragma unroll
+    for (int j = 0; j < SV; j++) key[j] = j * kWave + lane < 4 * nlists ? keys[j * kWave + lane] : 0u;
+    unsigned long long v[PER_WAVE];  // the first 64 entries (past a list's size: unset); few lists have more
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; i++) {
+        const int l = wave + i * WAVES;
+        size[i] = l < nlists ? sizes[l] : 0u;
+        v[i] = l < nlists ? lists[(int64_t)l * kTopKListMax + lane] : 0ull;
+    }
+    __syncthreads();
+    const unsigned long long t = (unsigned long long)topk_threshold_key<SV>(key, top_k) << 32;
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; i++) {
+        if (size[i] > (uint32_t)kTopKListMax) {  // an overflow, seen by every workgroup alike
+            if (lane == 0) atomicAdd(&filled, (uint32_t)kTopKCandidates + 1);
+            continue;
+        }
+        for (uint32_t from = 0; from < size[i]; from += kWave) {
+            if (from) v[i] = lists[(int64_t)(wave + i * WAVES) * kTopKListMax + from + lane];
+            const unsigned long long mask = __ballot(from + lane < size[i] && v[i] >= t);
+            if (mask == 0) continue;
+            uint32_t base = 0;
+            if (lane == 0) base = atomicAdd(&filled, (uint32_t)__popcll(mask));
+            base = (uint32_t)__builtin_amdgcn_readfirstlane((int)base);
+            const uint32_t pos = base + (uint32_t)__popcll(mask & ((1ull << lane) - 1));
+            if (((mask >> lane) & 1) && pos < (uint32_t)kTopKCandidates) c[pos] = v[i];
+        }
+    }
+    __syncthreads();
+    const uint32_t n = filled;
     if (n > (uint32_t)kTopKCandidates) {
         // A tree of lists: every wavefront reduces its segment, and the one that completes the children of a node (as many
         // lists as fill a segment) reduces those too and goes on from there.  Every list has a place of its own.
-        const int lane = threadIdx.x & (kWave - 1), fan = kTopKSegment / top_k;
-        int64_t lists = (count + kTopKSegment - 1) / kTopKSegment, at = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-        if (at >= lists) return;
+        const int fan = kTopKSegment / top_k;
+        int64_t left = (count + kTopKSegment - 1) / kTopKSegment, at = (int64_t)blockIdx.x * kTreeWaves + wave;
+        if (wave >= kTreeWaves || at >= left) return;
         topk_reduce_segment(in, count, top_k, tree, at, lane);
         while (true) {
-            const int64_t node = at / fan, first = node * fan, nodes = (lists + fan - 1) / fan;
-            const int children = (int)(lists - first < fan ? lists - first : fan);
+            const int64_t node = at / fan, first = node * fan, nodes = (left + fan - 1) / fan;
+            const int children = (int)(left - first < fan ? left - first : fan);
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // this wavefront's list is visible before its ticket is
             uint32_t before = 0;
             if (lane == 0) before = atomicAdd(tickets + node, 1u);
             if (__builtin_amdgcn_readfirstlane((int)before) + 1 != children) return;
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-            unsigned long long* const dst = nodes == 1 ? out : tree + lists * top_k;
+            unsigned long long* const dst = nodes == 1 ? out : tree + left * top_k;
             topk_reduce_segment(tree + first * top_k, (int64_t)children * top_k, top_k, dst + node * top_k, 0, lane);
             if (nodes == 1) return;
             tree = dst;
             tickets += nodes;
-            lists = nodes;
+            left = nodes;
             at = node;
         }
     }
     if (blockIdx.x != 0) return;
-    constexpr int PER = kTopKCandidates / 256;
-    __shared__ unsigned long long c[kTopKCandidates];
-    unsigned long long mine[PER];
-    int rank[PER];
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const uint32_t idx = threadIdx.x + 256u * i;
-        mine[i] = idx < n ? cand[idx] : 0ull;
-        c[idx] = mine[i];
-        rank[i] = 0;
-    }
-    __syncthreads();
-    for (uint32_t o = 0; o < n; o++) {
-        const unsigned long long other = c[o];
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            const uint32_t idx = threadIdx.x + 256u * i;
-            rank[i] += (other > mine[i] || (other == mine[i] && o < idx)) ? 1 : 0;
+    for (uint32_t idx = tid; idx < n; idx += kMergeThreads) {
+        const unsigned long long mine = c[idx];
+        int rank = 0;
+#pragma unroll 8
+        for (uint32_t o = 0; o < n; o++) {
+            const unsigned long long other = c[o];
+            rank += (other > mine || (other == mine && o < idx)) ? 1 : 0;
         }
+        if (rank < top_k) out[rank] = mine;
     }
-#pragma unroll
-    for (int i = 0; i < PER; i++) {
-        const uint32_t idx = threadIdx.x + 256u * i;
-        if (idx < n && rank[i] < top_k) out[rank[i]] = mine[i];
-    }
-    if (threadIdx.x >= n && threadIdx.x < (uint32_t)top_k) out[threadIdx.x] = 0ull;  // fewer candidates than top_k
+    if ((uint32_t)tid >= n && tid < top_k) out[tid] = 0ull;  // fewer candidates than top_k
 }
 
 static int64_t topk_segments(int64_t count) { return (count + kTopKSegment - 1) / kTopKSegment; }
@@ -491,7 +507,12 @@ static int topk_threshold_per_lane(int64_t count, int top_k) {
     return 0;
 }
 
-// Entries of the tree of lists (topk_finish_kernel; the last list is the call's output).
+static int64_t topk_lists(int64_t count, int top_k) {
+    const int64_t entries = 256 * topk_threshold_per_lane(count, top_k);
+    return (count + entries - 1) / entries;
+}
+
+// Entries of the tree of lists (topk_merge_kernel; the last list is the call's output).
 static int64_t topk_tree_entries(int64_t count, int top_k) {
     const int64_t fan = kTopKSegment / top_k;
     int64_t total = 0;
@@ -505,17 +526,8 @@ size_t packed_topk_scratch_entries(int64_t count, int top_k) {
     const int64_t c1 = topk_segments(count) * top_k;
     const int64_t c2 = c1 > kTopKSegment ? topk_segments(c1) * top_k : 0;
     if (topk_threshold_per_lane(count, top_k))
-        return (size_t)(topk_tree_entries(count, top_k) + kTopKHeader + kTopKThresholdSegments + kTopKCandidates);
+        return (size_t)(topk_tree_entries(count, top_k) + kTopKHeader + kTopKThresholdSegments + topk_lists(count, top_k) * kTopKListMax);
     return (size_t)(c1 + c2);
-}
-
-template <int V>
-static void topk_threshold_launch(const unsigned long long* in, int64_t count, int top_k, unsigned long long* segmax,
-                                  uint32_t* counter, unsigned long long* cand, hipStream_t stream) {
-    const int64_t pieces = (count + kWave * V - 1) / (kWave * V);
-    const dim3 grid((unsigned)((pieces + 3) / 4));
-    hipLaunchKernelGGL(topk_segment_max_kernel<V>, grid, dim3(256), 0, stream, in, count, segmax, counter);
-    hipLaunchKernelGGL(topk_filter_kernel<V>, grid, dim3(256), 0, stream, in, count, top_k, segmax, (int)pieces, counter, cand);
 }
 
 hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int top_k, unsigned long long* out,
@@ -528,15 +540,17 @@ hipError_t packed_topk_launch(const unsigned long long* in, int64_t count, int t
     const unsigned long long* src = in;
     int64_t n = count;
     if (const int per_lane = topk_threshold_per_lane(count, top_k)) {
-        unsigned long long* extra = scratch + topk_tree_entries(count, top_k);
-        uint32_t* counter = reinterpret_cast<uint32_t*>(extra);
-        unsigned long long* segmax = extra + kTopKHeader;
-        unsigned long long* cand = segmax + kTopKThresholdSegments;
-        if (per_lane == 16) topk_threshold_launch<16>(in, count, top_k, segmax, counter, cand, stream);
-        else if (per_lane == 4) topk_threshold_launch<4>(in, count, top_k, segmax, counter, cand, stream);
-        else topk_threshold_launch<1>(in, count, top_k, segmax, counter, cand, stream);
-        hipLaunchKernelGGL(topk_finish_kernel, dim3((unsigned)((first + 3) / 4)), dim3(256), 0, stream, in, count, top_k, counter,
-                           cand, out, scratch, counter + 1);
+        unsigned long long* const extra = scratch + topk_tree_entries(count, top_k);
+        uint32_t* const tickets = reinterpret_cast<uint32_t*>(extra);
+        uint32_t* const keys = reinterpret_cast<uint32_t*>(extra + kTopKHeader);
+        uint32_t* const sizes = keys + kTopKThresholdSegments;
+        unsigned long long* const lists = extra + kTopKHeader + kTopKThresholdSegments;
+        const int nlists = (int)topk_lists(count, top_k);
+        hipLaunchKernelGGL(per_lane == 16 ? topk_lists_kernel<16> : per_lane == 4 ? topk_lists_kernel<4> : topk_lists_kernel<1>,
+                           dim3((unsigned)nlists), dim3(256), 0, stream, in, count, top_k, lists, sizes, keys, tickets);
+        hipLaunchKernelGGL(nlists <= 64 ? topk_merge_kernel<4> : topk_merge_kernel<kTopKThresholdSegments / kWave>,
+                           dim3((unsigned)((first + kTreeWaves - 1) / kTreeWaves)), dim3(kMergeThreads), 0, stream, in, count, top_k, lists, sizes,
+                           keys, nlists, out, scratch, tickets);
         return hipGetLastError();
     }
     while (true) {
@@ -606,11 +620,11 @@ __global__ __launch_bounds__(kSampleMax) void packed_topk_sample_kernel(const un
         return;
     }
     const double softcap = (double)softcap_f;
-    const double max_value = sample_score(vals[first_valid], softcap) / temperature;
-    wts[t] = (t >= first_valid && t < top_k && vals[t] != 0ull)
-                 ? exp(sample_score(vals[t], softcap) / temperature - max_value)
-                 : 0.0;
     const bool valid = t >= first_valid && t < top_k && vals[t] != 0ull;
+    const double score = valid ? sample_score(vals[t], softcap) / temperature : 0.0;
+    prefix[t] = score;  // (the first valid one's is every thread's maximum: tanh once, not twice in turn)
+    __syncthreads();
+    wts[t] = valid ? exp(score - prefix[first_valid]) : 0.0;
     if (valid && !isfinite(wts[t])) bad = 1;  // any non-finite weight: nothing is sampled
     __syncthreads();
     // The reference's four passes all add the same weights in the same order from 0.0: its total, its nucleus
