@@ -850,8 +850,8 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     if (count == 0) return AQ_OK;
     if (!packed || !y || !N) return fail(AQ_ERR_ARG, "aq_qmv_multi: null array");
     if (M < 0 || K < 0) return fail(AQ_ERR_SHAPE, "aq_qmv_multi: M, K must be non-negative");
-    bool fused = M >= 1 && M <= 4 && K > 0 && bits == 4 && ctx->forced[0] < 0;
     const bool tiled = (flags & AQ_W_TILED) != 0;  // every member is a tile-major tensor; scales and biases are not read
+    bool fused = M >= 1 && M <= 4 && K > 0 && (bits == 4 || (bits == 8 && !tiled)) && ctx->forced[0] < 0;
     if (!tiled && (!scales || !biases)) return fail(AQ_ERR_ARG, "aq_qmv_multi: null array");
     const void* const kNoArrays[aq::kQmvMultiMax] = {nullptr, nullptr, nullptr, nullptr};
     if (tiled) scales = biases = kNoArrays;
@@ -877,22 +877,32 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             CallLock lk(ctx);
             // the kernels aq_qmv would pick for each member, in one grid
             // (every variant with the same split of K computes the same bytes, whatever the rows per workgroup)
-            const int di = (ctx->families_off >> kFamDiag & 1) ? -1 : aq::qmvd_pick(M, K, (int)total);
+            const bool diag = !(ctx->families_off >> kFamDiag & 1);
+            int di = diag && bits == 4 ? aq::qmvd_pick(M, K, (int)total) : -1;
+            // 8 bit: the diagonal kernels stop at 40 Mi codes, so every member is asked by itself; members of both kinds run apart.
+            // (us, one by one / in one grid: one row of 4096 / 1024 / 1024 rows and K = 4096 14.7 / 8.6, 2048 / 512 / 512 and 2048 9.8 /
+            // 3.8, dot2: 5120 / 1024 / 1024 and 5120 17.9 / 9.6, 2 x 14336 and 4096 25.4 / 24.6; four rows of the first 18.1 / 10.3)
+            int on_diag = 0;
+            for (int i = 0; bits == 8 && diag && group_size == 64 && i < count; i++)
+                if (const int own = aq::qmvd_pick(M, K, N[i], 8); own >= 0) di = own, on_diag++;
+            if (on_diag == count && bits == 8)
+                if (const int all = aq::qmvd_pick(M, K, (int)total, 8); all >= 0) di = all;
+            if (on_diag < count && bits == 8) di = -1;
             if (di >= 0 && aq::qmvd_multi_supported(di)) {
                 bool fits = true;
                 const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
                 for (int i = 0; i < count; i++) fits = fits && aq::qmvd_fits(multi_member(ma, i), bits, group_size, false, di);
                 if (fits) {
-                    ctx->last_variant[0] = "qmv_multi_diag";
+                    ctx->last_variant[0] = bits == 4 ? "qmv_multi_diag" : aq::qmvd_variant(di)->name;
                     AQ_HIP(aq::qmvd_multi_launch(di, ma, ctx->stream), "hipLaunchKernel");
                     return AQ_OK;
                 }
             }
-            const int idx = M == 1 && !tiled ? pick_qmv_variant(ctx, bits, 1, false, (int)total, K, 1) : -1;
+            const int idx = M == 1 && !tiled && on_diag == 0 ? pick_qmv_variant(ctx, bits, 1, false, (int)total, K, 1) : -1;
             const int rows = idx >= 0 ? aq::qmv_variant(idx)->rows : 0;
             if (rows > 0 && aq::qmv_multi_supported(bits, 1, rows)) {
                 const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, 1, K, group_size, flags);
-                ctx->last_variant[0] = "qmv_multi_dot2";
+                ctx->last_variant[0] = bits == 4 ? "qmv_multi_dot2" : aq::qmv_variant(idx)->name;
                 AQ_HIP(aq::qmv_multi_launch(bits, 1, rows, ma, ctx->stream), "hipLaunchKernel");
                 return AQ_OK;
             }

@@ -710,6 +710,24 @@ __global__ __launch_bounds__(NR* NW* kWave, 4) void qmv_diag_multi_kernel(const 
     qmv_diag_dense<NW, SUP, NR, false, 1, CPS, false, MODE>(a, block);
 }
 
+// The same for 8-bit codes: at one row a launch of a 1024 x 4096 matrix is mostly its ramp (q|k|v of 4096 / 1024 / 1024 rows and
+// K = 4096: 14.7 us in three launches, 8.6 here).
+template <int NW, int SUP, int NR, int CPS, int MODE>
+__global__ __launch_bounds__(NR* NW* kWave, 4) void qmv_diag_b8_multi_kernel(const QmvMultiArgs ma) {
+    int set = 0;
+#pragma unroll
+    for (int i = 1; i < kQmvMultiMax; i++)
+        if (i < ma.count && (int)blockIdx.x >= ma.block_end[i - 1]) set = i;
+    QmvArgs a = ma.common;
+    a.w = ma.w[set];
+    a.s = ma.s[set];
+    a.b = ma.b[set];
+    a.y = ma.y[set];
+    a.N = ma.N[set];
+    const int block = (int)blockIdx.x - (set ? ma.block_end[set - 1] : 0);
+    qmv_diag_body<NW, SUP, NR, false, 1, false, CPS, false, 0, true, (MODE & 1) != 0, false, ((MODE & 4) != 0 ? 2 : 1), true>(a, block);
+}
+
 // ---- variant table --------------------------------------------------------
 
 // Packed bytes of a dense launch (all its matrices) from which the weights are loaded with the non-temporal hint; the
@@ -1038,33 +1056,32 @@ hipError_t qmvd_head_launch(int idx, int fuse, const QmvArgs& a, hipStream_t str
 
 typedef void (*QmvDiagMultiKernel)(const QmvMultiArgs);
 struct QmvDiagMultiEntry {
-    int nw, sup, nr, cps;
+    int bits, nw, sup, nr, cps;
     QmvDiagMultiKernel fn[8];
 };
-#define AQ_QMVD_MULTI(NW, SUP, NR) {NW, SUP, NR, 4, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 4)}
-#define AQ_QMVD_MULTI3(NW, SUP, NR) {NW, SUP, NR, 3, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 3)}
+#define AQ_QMVD_MULTI(NW, SUP, NR) {4, NW, SUP, NR, 4, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 4)}
+#define AQ_QMVD_MULTI3(NW, SUP, NR) {4, NW, SUP, NR, 3, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 3)}
+// (8 bit: whole steps of K only, what qmvd_pick takes)
+#define AQ_QMVDB_MULTI(NW, SUP, NR) {8, NW, SUP, NR, 4, {nullptr, nullptr, nullptr, nullptr, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 4>, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 5>, nullptr, nullptr}}
 static const QmvDiagMultiEntry kQmvDiagMultiTable[] = {
     AQ_QMVD_MULTI(4, 1, 1), AQ_QMVD_MULTI(4, 1, 2), AQ_QMVD_MULTI(4, 1, 4), AQ_QMVD_MULTI(2, 1, 2), AQ_QMVD_MULTI(2, 1, 4),
     AQ_QMVD_MULTI(6, 1, 1), AQ_QMVD_MULTI(8, 1, 1), AQ_QMVD_MULTI(10, 1, 1), AQ_QMVD_MULTI(12, 1, 1), AQ_QMVD_MULTI(14, 1, 1),
     AQ_QMVD_MULTI(16, 1, 1), AQ_QMVD_MULTI3(4, 1, 1), AQ_QMVD_MULTI3(4, 1, 2), AQ_QMVD_MULTI3(4, 1, 4), AQ_QMVD_MULTI3(2, 1, 2),
-    AQ_QMVD_MULTI3(2, 1, 4),
+    AQ_QMVD_MULTI3(2, 1, 4), AQ_QMVDB_MULTI(4, 1, 1), AQ_QMVDB_MULTI(4, 1, 2), AQ_QMVDB_MULTI(8, 1, 1), AQ_QMVDB_MULTI(16, 1, 1),
 };
-
-// The multi-matrix launch of variant idx (the same arithmetic, so the same bytes, as one launch per matrix).
-bool qmvd_multi_supported(int idx) {
+static const QmvDiagMultiEntry* find_multi(int idx) {
     const QmvVariant* v = qmvd_variant(idx);
-    if (!v || b8_of(*v)) return false;
-    for (const QmvDiagMultiEntry& e : kQmvDiagMultiTable)
-        if (e.nw == v->waves && e.sup == v->depth && e.nr == v->rows && e.cps == cps_of(*v) && !g32_of(*v)) return true;
-    return false;
+    if (v && !g32_of(*v))
+        for (const QmvDiagMultiEntry& e : kQmvDiagMultiTable)
+            if (e.bits == v->bits && e.nw == v->waves && e.sup == v->depth && e.nr == v->rows && e.cps == cps_of(*v)) return &e;
+    return nullptr;
 }
 
+// The multi-matrix launch of variant idx (the same arithmetic, so the same bytes, as one launch per matrix).
+bool qmvd_multi_supported(int idx) { return find_multi(idx) != nullptr; }
+
 hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream) {
-    const QmvVariant* v = qmvd_variant(idx);
-    const QmvDiagMultiEntry* e = nullptr;
-    if (v)
-        for (const QmvDiagMultiEntry& c : kQmvDiagMultiTable)
-            if (c.nw == v->waves && c.sup == v->depth && c.nr == v->rows && c.cps == cps_of(*v)) e = &c;
+    const QmvDiagMultiEntry* const e = find_multi(idx);
     if (!e || ma.count < 1 || ma.count > kQmvMultiMax) return hipErrorInvalidValue;
     const int wg_rows = kDiagRows * e->nr;
     int blocks = 0;
@@ -1072,12 +1089,14 @@ hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream) {
         blocks += (ma.N[i] + wg_rows - 1) / wg_rows;
         ma.block_end[i] = blocks;
     }
-    const size_t lds = qmvd_lds_bytes_for(ma.common.M, ma.common.K, e->nw * e->nr);
+    const int K4 = k4_of(ma.common.K, e->bits);
+    const size_t lds = qmvd_lds_bytes_for(ma.common.M, ma.common.K, e->nw * e->nr, 1, false, e->bits == 8);
     int64_t bytes = 0;
-    for (int i = 0; i < ma.count; i++) bytes += (int64_t)ma.N[i] * (ma.common.K / 2);
+    for (int i = 0; i < ma.count; i++) bytes += (int64_t)ma.N[i] * (K4 / 2);
     ma.common.stream_w = bytes >= kDiagStreamBytes ? 1 : 0;
     ma.common.early_wgs = diag_early_wgs(blocks);
-    const QmvDiagMultiKernel fn = e->fn[diag_mode(ma.common.K, e->cps, ma.common.tiled != 0, ma.common.stream_w != 0)];
+    const QmvDiagMultiKernel fn = e->fn[diag_mode(K4, e->cps, ma.common.tiled != 0, ma.common.stream_w != 0)];
+    if (!fn) return hipErrorInvalidValue;
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)(e->nw * e->nr * kWave)), lds, stream, ma);
     return hipGetLastError();
