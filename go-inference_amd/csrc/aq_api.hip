@@ -379,14 +379,14 @@ bool tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
     *tile = static_cast<float*>(ctx->ws.ptr);
     return true;
 }
-int tok_pick(const aq_ctx* ctx, const aq::QmvArgs& t, int group_size, int bits, bool pair) {
+int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, bool pair) {
     const int64_t bands = (int64_t)((t.N + 15) / 16) * (pair ? 2 : 1) * (t.ksplit > 1 ? t.ksplit : 1);
     return aq::qmvt_pick(bits, group_size, t.M, t.K, bands, t.ksplit > 1 ? t.share : (t.K + 255) / 256, pair, ctx->cu_count);
 }
 
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
     if (gather) return kPass;
-    aq::QmvArgs t = a;
+    aq::TokArgs t{a};
     t.ksplit = 1;
     t.tokens = forced < 0 ? aq::qmvt_tokens(a.M) : a.M;
     if (forced < 0 && !tok_small(bits, group_size, a.M, a.K, a.N) && tok_halves(ctx, group_size, a.M, a.N, false)) {
@@ -915,17 +915,18 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
                      check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK;
     unsigned in_grid = 0;
     int members = 0, ti = -1;
-    aq::QmvMultiArgs grid{};
+    aq::TokMultiArgs grid{};
     if (tok) {
         CallLock lk(ctx);
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
         size_t bytes = 0;
         grid.common = all.common;
-        grid.common.tokens = aq::qmvt_tokens(M);
+        grid.tokens = aq::qmvt_tokens(M);
         for (int i = 0; i < count; i++) {
             if (N[i] == 0 || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i], false)) continue;
-            aq::QmvArgs own = multi_member(grid, i);
+            aq::TokArgs own{multi_member(grid, i)};
+            own.tokens = grid.tokens;
             own.w = all.w[i];
             own.s = all.s[i];
             own.b = all.b[i];
@@ -959,7 +960,8 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         }
         ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, group_size, M, K, bands, runs, false, ctx->cu_count) : -1;
         for (int i = 0; ti >= 0 && i < members; i++) {
-            aq::QmvArgs one = multi_member(grid, i);
+            aq::TokArgs one{multi_member(grid, i)};
+            one.tokens = grid.tokens;
             one.ksplit = grid.ksplit[i];
             one.share = grid.share[i];
             if (!aq::qmvt_fits(one, bits, group_size, ti, false)) ti = -1;
@@ -1174,7 +1176,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
         a.route_x = g.route_x;
         a.route_of = g.route_of;
         ctx->last_variant[0] = pair ? "gather_gate_up_grouped_tok" : "gather_grouped_tok";
-        AQ_HIP(aq::qmvt_grouped_launch(bits, chunk, pair, most_chunks, a, ctx->stream), "hipLaunchKernel");
+        AQ_HIP(aq::qmvt_grouped_launch(bits, chunk, pair, most_chunks, aq::TokArgs{a}, ctx->stream), "hipLaunchKernel");
         return AQ_OK;
     }
     aq::QmmHalfCall q{};
@@ -1406,7 +1408,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     }
     if (M > 1 && tok_runs(ctx, bits, group_size, M, K, N, true)) {
         // the token-tile kernels with half of a workgroup's rows in either matrix
-        aq::QmvArgs a{};
+        aq::TokArgs a{};
         a.x = static_cast<const uint16_t*>(x);
         a.w = static_cast<const uint32_t*>(gate_packed);
         a.s = static_cast<const uint16_t*>(gate_scales);

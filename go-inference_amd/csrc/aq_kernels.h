@@ -50,10 +50,6 @@ struct QmvArgs {
     const RouteChunk* chunks;
     const int32_t* route_x;
     const int32_t* route_of;
-    // token-tile kernels: shares of K (0, 1: none), 256-code runs per share, the fp32 partial tiles; rows of x per workgroup
-    int ksplit, share;
-    float* tile;
-    int tokens;
     int act;             // kActGeluTanh or kActSilu
     // head kernels only (aq_qmv_head.hip): y is uint64 best[M] (argmax) or uint64 scores[M, N]
     const int32_t* suppress;  // token ids that may not win, or nullptr
@@ -88,8 +84,6 @@ struct QmvMultiArgs {
     void* y[kQmvMultiMax];
     int N[kQmvMultiMax];
     int block_end[kQmvMultiMax];  // filled by the launcher: first workgroup past matrix i
-    int ksplit[kQmvMultiMax], share[kQmvMultiMax];  // token-tile kernels, as in QmvArgs
-    float* tile[kQmvMultiMax];
 };
 // dot2 kernels only: 4 wavefronts a workgroup, `rows` output rows per wavefront, m = 1..4 activation rows.
 bool qmv_multi_supported(int bits, int m, int rows);
@@ -176,13 +170,24 @@ hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
 // Token-tile MFMA matvec kernels (aq_qmv_tok.hip; codes of 4 or 8 bits in groups of 32, 64 or 128, up to 64 activation rows
 // as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch without scratch memory, or shares of K and a sum of
 // their partial tiles).  kind 6 in QmvVariant.
+// Their arguments (apart from QmvArgs: those of the one-row kernels stay as short as they were, 0.04 us a launch).
+struct TokArgs : QmvArgs {
+    int ksplit, share;  // shares of K (0, 1: none), 256-code runs per share
+    float* tile;        // the fp32 partial tiles
+    int tokens;         // rows of x per workgroup
+};
+struct TokMultiArgs : QmvMultiArgs {
+    int ksplit[kQmvMultiMax], share[kQmvMultiMax];
+    float* tile[kQmvMultiMax];
+    int tokens;
+};
 int qmvt_variant_count();
 const QmvVariant* qmvt_variant(int idx);
 // (exact_only: groups of 64 with K a multiple of 256 only, what a forced variant takes)
-bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_only);
-const char* qmvt_name(int idx, const QmvArgs& a);  // the kernel qmvt_launch runs for this call
+bool qmvt_fits(const TokArgs& a, int bits, int group_size, int idx, bool exact_only);
+const char* qmvt_name(int idx, const TokArgs& a);  // the kernel qmvt_launch runs for this call
 // (a.ksplit, a.share and a.tile: see qmvt_split)
-hipError_t qmvt_launch(int idx, const QmvArgs& a, hipStream_t stream);
+hipError_t qmvt_launch(int idx, const TokArgs& a, hipStream_t stream);
 // Rows of x per workgroup (a.tokens): all of up to 32, else half of them.
 int qmvt_tokens(int M);
 // How a matrix of N rows (pair: two) shares K out over workgroups, a function of the matrix's own call alone so that it has the
@@ -193,13 +198,13 @@ size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit);
 int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count);
 // Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
 // sums are those of qmvt_launch.
-hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t stream);
+hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t stream);
 bool qmvt_pair_supported(int idx);
-hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream);
+hipError_t qmvt_pair_launch(int idx, const TokArgs& a, hipStream_t stream);
 // Expert slabs with the routes grouped by expert (a.chunks, a.route_x, a.route_of; chunks of up to `tokens` = 16 or 32
 // routes; most_chunks entries in the list); pair as above.
 bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair);
-hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream);
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const TokArgs& a, hipStream_t stream);
 // Partial tiles [ksplit][M][N] ([ksplit][M][gate N | up N]) added in order, the activation applied for a pair, and dense groups
 // of 32 that are not finite formed again (plain_dot_g32).  Matrices with tile null are left alone.
 struct TokReduceArgs {

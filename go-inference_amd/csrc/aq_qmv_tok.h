@@ -115,7 +115,7 @@ __device__ __forceinline__ void transpose4(uint32_t& s0, uint32_t& s1, uint32_t&
 }
 
 template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR, bool GROUPED>
-__device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block_of_all) {
+__device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block_of_all) {
     static_assert(BITS == 4 || BITS == 8, "code width");
     static_assert(GRP == 64 || GRP == 32, "group size (64: and 128)");
     constexpr int NW = kTokWaves;
@@ -577,19 +577,20 @@ __device__ __forceinline__ void qmv_tok16_body(const QmvArgs& a, const int block
 }
 
 template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR>
-__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_kernel(const QmvArgs a) {
+__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_kernel(const TokArgs a) {
     qmv_tok16_body<BITS, RS, RING, TS, GRP, PAIR, false>(a, (int)blockIdx.x);
 }
 template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR>
-__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_grouped_kernel(const QmvArgs a) {
+__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_grouped_kernel(const TokArgs a) {
     qmv_tok16_body<BITS, RS, RING, TS, GRP, PAIR, true>(a, (int)blockIdx.x);
 }
 // up to four matrices that share x in one grid: every workgroup belongs to one of them
 template <int BITS, int RS, int RING, int TS, int GRP>
-__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_multi_kernel(const QmvMultiArgs ma) {
+__global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_multi_kernel(const TokMultiArgs ma) {
     int i = 0, before = 0;
     while (i + 1 < ma.count && (int)blockIdx.x >= ma.block_end[i]) before = ma.block_end[i++];
-    QmvArgs a = ma.common;
+    TokArgs a{ma.common};
+    a.tokens = ma.tokens;
     a.w = ma.w[i];
     a.s = ma.s[i];
     a.b = ma.b[i];
@@ -603,8 +604,8 @@ __global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_multi_kernel(const
 
 // ---- kernels of one code width -------------------------------------------------------------------------------------
 
-typedef void (*QmvTokKernel)(const QmvArgs);
-typedef void (*QmvTokMultiKernel)(const QmvMultiArgs);
+typedef void (*QmvTokKernel)(const TokArgs);
+typedef void (*QmvTokMultiKernel)(const TokMultiArgs);
 struct QmvTokEntry {
     QmvVariant v;  // m = most activation rows, rows = sets of weight rows per workgroup, waves = wavefronts that share K
                    // (depth = sets of rows in flight, xmode = runs of 256 codes a wavefront holds per pass)

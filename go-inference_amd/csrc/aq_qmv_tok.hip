@@ -18,14 +18,14 @@ const QmvVariant* qmvt_variant(int idx) {
 }
 
 static bool tok_whole_runs(const QmvArgs& a) { return a.gs_shift == 6 && a.K % 256 == 0; }
-static int tok_runs_of(const QmvArgs& a) { return a.ksplit > 1 ? a.share : (a.K + 255) / 256; }
+static int tok_runs_of(const TokArgs& a) { return a.ksplit > 1 ? a.share : (a.K + 255) / 256; }
 static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs) {
     const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.ts);
     const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4;
     return staged > sums ? staged : sums;
 }
 
-bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_only) {
+bool qmvt_fits(const TokArgs& a, int bits, int group_size, int idx, bool exact_only) {
     const QmvVariant* v = qmvt_variant(idx);
     if (!v || bits != v->bits || (group_size != 32 && group_size != 64 && group_size != 128)) return false;
     // (K up to 16384: what the tests cover; longer rows go to the kernels that split K)
@@ -42,7 +42,7 @@ bool qmvt_fits(const QmvArgs& a, int bits, int group_size, int idx, bool exact_o
     return tok_lds_bytes(tok_entry(idx), group_size == 32, tok_runs_of(a)) <= 160 * 1024;
 }
 
-const char* qmvt_name(int idx, const QmvArgs& a) { return tok_entry(idx).name[a.gs_shift == 5 ? 2 : tok_whole_runs(a) ? 0 : 1]; }
+const char* qmvt_name(int idx, const TokArgs& a) { return tok_entry(idx).name[a.gs_shift == 5 ? 2 : tok_whole_runs(a) ? 0 : 1]; }
 
 static int tok_blocks(const QmvTokEntry& e, int M, int tokens, int N, bool pair, int ksplit) {
     const int outs = e.wg_rows / (pair ? 2 : 1);
@@ -51,7 +51,7 @@ static int tok_blocks(const QmvTokEntry& e, int M, int tokens, int N, bool pair,
 }
 int qmvt_tokens(int M) { return M <= 32 ? M : (M + 1) / 2; }
 
-static hipError_t tok_reduce_one(const QmvArgs& a, int bits, bool pair, hipStream_t stream) {
+static hipError_t tok_reduce_one(const TokArgs& a, int bits, bool pair, hipStream_t stream) {
     if (a.ksplit <= 1) return hipSuccess;
     TokReduceArgs r{};
     r.x = a.x;
@@ -72,7 +72,7 @@ static hipError_t tok_reduce_one(const QmvArgs& a, int bits, bool pair, hipStrea
     return tok_reduce_launch(r, stream);
 }
 
-static hipError_t tok_launch(int idx, QmvArgs a, bool pair, hipStream_t stream) {
+static hipError_t tok_launch(int idx, TokArgs a, bool pair, hipStream_t stream) {
     const QmvTokEntry& e = tok_entry(idx);
     if (a.tokens < 1) a.tokens = a.M;
     const bool g32 = a.gs_shift == 5;
@@ -84,12 +84,12 @@ static hipError_t tok_launch(int idx, QmvArgs a, bool pair, hipStream_t stream) 
     return tok_reduce_one(a, e.v.bits, pair, stream);
 }
 
-hipError_t qmvt_launch(int idx, const QmvArgs& a, hipStream_t stream) {
+hipError_t qmvt_launch(int idx, const TokArgs& a, hipStream_t stream) {
     if (idx < 0 || idx >= qmvt_variant_count()) return hipErrorInvalidValue;
     return tok_launch(idx, a, false, stream);
 }
 
-hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t stream) {
+hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t stream) {
     if (idx < 0 || idx >= qmvt_variant_count() || ma.count < 1 || ma.count > kQmvMultiMax) return hipErrorInvalidValue;
     const QmvTokEntry& e = tok_entry(idx);
     const bool g32 = ma.common.gs_shift == 5;
@@ -105,7 +105,7 @@ hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t str
     r.count = ma.count;
     bool split = false;
     for (int i = 0; i < ma.count; i++) {
-        blocks += tok_blocks(e, ma.common.M, ma.common.tokens, ma.N[i], false, ma.ksplit[i]);
+        blocks += tok_blocks(e, ma.common.M, ma.tokens, ma.N[i], false, ma.ksplit[i]);
         ma.block_end[i] = blocks;
         const int n = ma.ksplit[i] > 1 ? ma.share[i] : (ma.common.K + 255) / 256;
         runs = n > runs ? n : runs;
@@ -125,7 +125,7 @@ hipError_t qmvt_multi_launch(int idx, QmvMultiArgs ma, int bits, hipStream_t str
 
 bool qmvt_pair_supported(int idx) { return idx >= 0 && idx < qmvt_variant_count() && tok_entry(idx).pair[0] != nullptr; }
 
-hipError_t qmvt_pair_launch(int idx, const QmvArgs& a, hipStream_t stream) {
+hipError_t qmvt_pair_launch(int idx, const TokArgs& a, hipStream_t stream) {
     if (!qmvt_pair_supported(idx)) return hipErrorInvalidValue;
     return tok_launch(idx, a, true, stream);
 }
@@ -144,7 +144,7 @@ bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair) {
     return tok_lds_bytes(tok_entry(1), group_size == 32, (a.K + 255) / 256) <= 160 * 1024;
 }
 
-hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const QmvArgs& a, hipStream_t stream) {
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const TokArgs& a, hipStream_t stream) {
     const int idx = (bits == 8 ? kTokPerWidth : 0) + (tokens == 32 ? 5 : 1);  // (four sets of rows: the second of a token count)
     const QmvTokEntry& e = tok_entry(idx);
     const bool g32 = a.gs_shift == 5;
