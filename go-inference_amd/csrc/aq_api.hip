@@ -1165,6 +1165,7 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     g.chunk_rows = chunk;
     g.pad = pad;
     g.most_chunks = most_chunks;
+    g.most_rows = most_rows;
     g.chunks = reinterpret_cast<aq::RouteChunk*>(p);
     g.nchunks = reinterpret_cast<int32_t*>(p + list);
     g.live_rows = g.nchunks + 1;

@@ -279,7 +279,7 @@ hipError_t moe_route_launch(const MoeRouteArgs& a, hipStream_t stream);
 constexpr int kGroupMaxExperts = 4096;
 struct RouteGroupArgs {
     const int32_t *lhs, *rhs;  // lhs may be null (every route reads row 0)
-    int routes, x_rows, num_experts, chunk_rows, pad, most_chunks;
+    int routes, x_rows, num_experts, chunk_rows, pad, most_chunks, most_rows;
     RouteChunk* chunks;
     int32_t *nchunks, *live_rows, *route_x, *route_of;
 };

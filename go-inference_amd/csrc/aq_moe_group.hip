@@ -7,9 +7,9 @@
 // into chunks that one workgroup tile of the matmul (or token-tile) kernels takes as its rows of x.  The list has as many
 // entries as the ids ask for; the launches behind it are sized for the most there can be and read the count here.
 //
-// Bound: latency.  Two passes over 4 bytes a route with LDS counters and one scan over the experts, one workgroup because
-// the passes depend on each other through the counters (4096 routes over 128 experts: 11 us in a kernel trace; a grid-wide
-// meeting costs more than that).
+// Bound: latency, and the scattered places.  Two passes over 4 bytes a route with LDS counters and one scan over the experts, one
+// workgroup because the passes depend on each other through the counters (a grid-wide meeting costs more).  4096 routes over 128
+// experts in a kernel trace: places stored to memory one by one, loads each behind a branch 11.7 us -> 8.8.
 #include "aq_device.h"
 #include "aq_kernels.h"
 
@@ -17,8 +17,13 @@ namespace aq {
 
 constexpr int kGroupThreads = 1024;
 
+// STAGED: the two lists of places are put together in LDS and leave it in whole lines.  Places lie all over a list, and a store
+// instruction takes about four clocks per line that it touches: 8192 of them were most of this kernel's 11.5 us.
+template <bool STAGED>
 __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const RouteGroupArgs a) {
-    extern __shared__ int32_t counter[];  // [num_experts] routes of the expert, then the next free place of its run
+    extern __shared__ __attribute__((aligned(16))) int32_t counter[];  // [num_experts] routes of the expert, then the next free place of its run
+    int32_t* const list_x = STAGED ? counter + (a.num_experts + 3) / 4 * 4 : a.route_x;
+    int32_t* const list_of = STAGED ? list_x + (a.most_rows + 3) / 4 * 4 : a.route_of;
     __shared__ int32_t wave_rows[kGroupThreads / kWave], wave_chunks[kGroupThreads / kWave];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     const int E = a.num_experts;
@@ -32,11 +37,18 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const RouteGro
         return e < 0 || e >= E || x < 0 || x >= a.x_rows ? kBad : e;
     };
     constexpr int HOLD = 8;  // up to 8192 routes: the ids are read once and kept
-    int held[HOLD];
+    int held[HOLD], from[HOLD];
+    // (loads without a branch around each, or every one of them is waited for before the next is asked for)
 #pragma unroll
     for (int i = 0; i < HOLD; i++) {
-        const int r = tid + i * kGroupThreads;
-        held[i] = r < a.routes ? expert_of(r) : -1;
+        const int r = min(tid + i * kGroupThreads, a.routes - 1);
+        held[i] = a.rhs[r];
+        from[i] = a.lhs ? a.lhs[r] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < HOLD; i++) {
+        if (held[i] < 0 || held[i] >= E || from[i] < 0 || from[i] >= a.x_rows) held[i] = kBad;
+        if (tid + i * kGroupThreads >= a.routes) held[i] = -1;
     }
 #pragma unroll
     for (int i = 0; i < HOLD; i++)
@@ -62,6 +74,7 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const RouteGro
     if (lane == kWave - 1) wave_rows[wave] = rows_to, wave_chunks[wave] = chunks_to;
     __syncthreads();
     int row = rows_to - rows, chunk = chunks_to - chunks, all_rows = 0, all_chunks = 0;
+#pragma unroll
     for (int w = 0; w < kGroupThreads / kWave; w++) {
         if (w < wave) row += wave_rows[w], chunk += wave_chunks[w];
         all_rows += wave_rows[w];
@@ -70,7 +83,6 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const RouteGro
     for (int e = e0; e < e1; e++) {
         const int n = counter[e], end = row + padded(n);
         for (int c = 0; c < n; c += a.chunk_rows) a.chunks[chunk++] = RouteChunk{e, row + c, min(a.chunk_rows, n - c), 0};
-        for (int i = row + n; i < end; i++) a.route_x[i] = -1, a.route_of[i] = -1;
         counter[e] = row;
         row = end;
     }
@@ -78,20 +90,47 @@ __global__ __launch_bounds__(kGroupThreads) void moe_group_kernel(const RouteGro
     if (tid == 0) *a.nchunks = all_chunks, *a.live_rows = all_rows;
     __syncthreads();
 
-    auto place = [&](int r, int e) {
-        const int at = atomicAdd(&counter[e & (kBad - 1)], 1);
+    auto place = [&](int r, int e, int x, int at) {
         const bool bad = (e & kBad) != 0;
-        a.route_x[at] = bad ? -1 : a.lhs ? a.lhs[r] : 0;
-        a.route_of[at] = bad ? r | INT32_MIN : r;
+        list_x[at] = bad ? -1 : x;
+        list_of[at] = bad ? r | INT32_MIN : r;
     };
+    int at[HOLD];
 #pragma unroll
     for (int i = 0; i < HOLD; i++)
-        if (held[i] >= 0) place(tid + i * kGroupThreads, held[i]);
-    for (int r = tid + HOLD * kGroupThreads; r < a.routes; r += kGroupThreads) place(r, expert_of(r));
+        if (held[i] >= 0) at[i] = atomicAdd(&counter[held[i] & (kBad - 1)], 1);
+#pragma unroll
+    for (int i = 0; i < HOLD; i++)
+        if (held[i] >= 0) place(tid + i * kGroupThreads, held[i], from[i], at[i]);
+    for (int r = tid + HOLD * kGroupThreads; r < a.routes; r += kGroupThreads) {
+        const int e = expert_of(r);
+        place(r, e, a.lhs ? a.lhs[r] : 0, atomicAdd(&counter[e & (kBad - 1)], 1));
+    }
+    __syncthreads();
+    // Runs start at multiples of pad, and a counter is now where its run ends: -1 from there to the next multiple.
+    if (a.pad > 1)
+        for (int e = wave; e < E; e += kGroupThreads / kWave) {
+            const int begin = counter[e], end = padded(begin);
+            for (int i = begin + lane; i < end; i += kWave) list_x[i] = -1, list_of[i] = -1;
+        }
+    if constexpr (STAGED) {
+        __syncthreads();
+        // (lists in LDS and in memory have room for whole 16-byte pieces)
+        for (int i = tid; i < (all_rows + 3) / 4; i += kGroupThreads) {
+            reinterpret_cast<int4*>(a.route_x)[i] = reinterpret_cast<const int4*>(list_x)[i];
+            reinterpret_cast<int4*>(a.route_of)[i] = reinterpret_cast<const int4*>(list_of)[i];
+        }
+    }
 }
 
 hipError_t moe_group_launch(const RouteGroupArgs& a, hipStream_t stream) {
-    hipLaunchKernelGGL(moe_group_kernel, dim3(1), dim3(kGroupThreads), (size_t)a.num_experts * 4, stream, a);
+    const size_t counters = (size_t)(a.num_experts + 3) / 4 * 16, staged = counters + (size_t)(a.most_rows + 3) / 4 * 32;
+    if (staged > 128 * 1024) {
+        hipLaunchKernelGGL(moe_group_kernel<false>, dim3(1), dim3(kGroupThreads), counters, stream, a);
+    } else {
+        if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(moe_group_kernel<true>), staged)) return rc;
+        hipLaunchKernelGGL(moe_group_kernel<true>, dim3(1), dim3(kGroupThreads), staged, stream, a);
+    }
     return hipGetLastError();
 }
 
