@@ -5,6 +5,7 @@ arrays and device pointers into its C ABI (include/aq_mi355.h, include/aq_mi355_
 It raises if the library has not been built: there is no fallback path.
 """
 import ctypes
+import functools
 import os
 
 import numpy as np
@@ -183,6 +184,8 @@ def load():
 
 def _ptr(obj):
     """Device pointer (int / DeviceBuffer) or host numpy array -> void*."""
+    if type(obj) is int:  # a serving loop's case, ahead of the checks for the others: a call has 5 to 15 pointers
+        return obj
     if obj is None:
         return None
     if isinstance(obj, DeviceBuffer):
@@ -190,6 +193,12 @@ def _ptr(obj):
     if isinstance(obj, np.ndarray):
         return obj.ctypes.data
     return int(obj)
+
+
+@functools.lru_cache(maxsize=16)
+def _array_types(n):
+    """ctypes arrays of n pointers and n ints."""
+    return _vp * n, ctypes.c_int * n
 
 
 class DeviceBuffer:
@@ -297,16 +306,16 @@ class Context:
     def qmv_multi(self, x, ws, ss, bs, ys, Ns, M, K, group_size=64, bits=4, flags=0):
         """ws, ss, bs, ys: sequences of device buffers (one per weight matrix); Ns: their row counts."""
         n = len(ws)
-        arr = lambda seq: (_c.c_void_p * n)(*[_ptr(t) for t in seq])
-        self._check(self.lib.aq_qmv_multi(self.handle, _ptr(x), n, arr(ws), arr(ss), arr(bs), arr(ys),
-                                          (_c.c_int * n)(*Ns), M, K, group_size, bits, flags))
+        ptrs, ints = _array_types(n)
+        self._check(self.lib.aq_qmv_multi(self.handle, _ptr(x), n, ptrs(*map(_ptr, ws)), ptrs(*map(_ptr, ss)),
+                                          ptrs(*map(_ptr, bs)), ptrs(*map(_ptr, ys)), ints(*Ns), M, K, group_size, bits, flags))
 
     def qmm_multi(self, x, ws, ss, bs, ys, Ns, M, K, group_size=64, bits=4, flags=0):
         """aq_qmm over several weight matrices that share x: one pass over x for the members that need the same form."""
         n = len(ws)
-        arr = lambda seq: (_c.c_void_p * n)(*[_ptr(t) for t in seq])
-        self._check(self.lib.aq_qmm_multi(self.handle, _ptr(x), n, arr(ws), arr(ss), arr(bs), arr(ys),
-                                          (_c.c_int * n)(*Ns), M, K, group_size, bits, flags))
+        ptrs, ints = _array_types(n)
+        self._check(self.lib.aq_qmm_multi(self.handle, _ptr(x), n, ptrs(*map(_ptr, ws)), ptrs(*map(_ptr, ss)),
+                                          ptrs(*map(_ptr, bs)), ptrs(*map(_ptr, ys)), ints(*Ns), M, K, group_size, bits, flags))
 
     def prepared_qmv(self, x, w, s, b, y, M, K, N, group_size=64, bits=4, flags=0):
         """The same call as qmv with every argument converted once: returns a function of no arguments.  For loops
