@@ -915,12 +915,12 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
                      check_geometry("aq_qmv_multi", K, group_size, bits) == AQ_OK;
     unsigned in_grid = 0;
     int members = 0, ti = -1;
+    size_t bytes = 0;  // of the members' partial tiles
     aq::TokMultiArgs grid{};
     if (tok) {
         CallLock lk(ctx);
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
-        size_t bytes = 0;
         grid.common = all.common;
         grid.tokens = aq::qmvt_tokens(M);
         for (int i = 0; i < count; i++) {
@@ -946,15 +946,11 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             total += N[i];
         }
         grid.count = members;
-        float* tiles = nullptr;
-        const bool split = tok_tiles(ctx, bytes, &tiles);
+        float* room = nullptr;
         int64_t bands = 0;
         int runs = 1;
         for (int i = 0; i < members; i++) {
-            if (!split) grid.ksplit[i] = 1;
             const int ks = grid.ksplit[i], n = ks > 1 ? grid.share[i] : (K + 255) / 256;
-            grid.tile[i] = ks > 1 ? tiles : nullptr;
-            tiles += aq::qmvt_tile_bytes(M, grid.N[i], false, ks) / 4;
             bands += (int64_t)((grid.N[i] + 15) / 16) * ks;
             runs = n > runs ? n : runs;
         }
@@ -966,7 +962,8 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             one.share = grid.share[i];
             if (!aq::qmvt_fits(one, bits, group_size, ti, false)) ti = -1;
         }
-        if (ti < 0) in_grid = 0;
+        // without room for all the tiles every member decides by itself, as its own call does
+        if (ti < 0 || !tok_tiles(ctx, bytes, &room)) in_grid = 0;
     }
     for (int i = 0; i < count; i++) {
         if (in_grid >> i & 1) continue;
@@ -974,6 +971,13 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     }
     if (in_grid) {
         CallLock lk(ctx);
+        // (the calls in between may have moved the workspace; it has held the tiles once and does not shrink)
+        float* tiles = nullptr;
+        if (!tok_tiles(ctx, bytes, &tiles)) return fail(AQ_ERR_NOMEM, "aq_qmv_multi: %zu bytes of workspace for partial tiles", bytes);
+        for (int i = 0; i < grid.count; i++) {
+            grid.tile[i] = grid.ksplit[i] > 1 ? tiles : nullptr;
+            tiles += aq::qmvt_tile_bytes(M, grid.N[i], false, grid.ksplit[i]) / 4;
+        }
         ctx->last_variant[0] = aq::qmvt_variant(ti)->name;
         AQ_HIP(aq::qmvt_multi_launch(ti, grid, bits, ctx->stream), "hipLaunchKernel");
     }

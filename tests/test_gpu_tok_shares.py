@@ -111,3 +111,28 @@ def test_capture_without_a_workspace():
             t.free()
     finally:
         fresh.close()
+
+
+@pytest.mark.parametrize("reserve", [0, 1 << 20])
+def test_members_apart_move_the_workspace(reserve):
+    """A member that runs by itself, ahead of the grid, needs more workspace than the grid's partial tiles."""
+    import aq_mi355
+    M, K, Ns, gs, bits = 40, 14336, (600, 500, 1000), 64, 4
+    say("token tile shares, members apart", reserve)
+    x = F.synthetic_x(M, K, seed=2495)
+    mats = [F.synthetic_affine(n, K, bits, gs, seed=2496 + i) for i, n in enumerate(Ns)]
+    fresh = aq_mi355.Context(0)
+    try:
+        if reserve:
+            fresh.reserve_workspace_bytes(reserve)
+        dws = [DeviceAffine(fresh, *m) for m in mats]
+        dx, ys = fresh.to_device(x), [fresh.alloc(M * n * 4) for n in Ns]
+        fresh.qmv_multi(dx, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, list(Ns), M, K, gs, bits, aq_mi355.AQ_OUT_F32)
+        fresh.sync()
+        for n, d, y in zip(Ns, dws, ys):
+            alone = run_qmv(fresh, x, d, M, K, n, gs, bits, True)
+            assert np.array_equal(y.download(np.uint32, M * n), alone.view(np.uint32).reshape(-1)), "member of %d rows" % n
+        for t in [dx] + ys + dws:
+            t.free()
+    finally:
+        fresh.close()
