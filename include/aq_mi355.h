@@ -101,7 +101,8 @@ int aq_timer_stop(aq_ctx *ctx, float *elapsed_ms); /* records, waits, reports */
  * fails with a message), and when a later such call makes it grow, every graph captured over the old block is
  * refused by aq_graph_launch with AQ_ERR_UNSUPPORTED - reserve the largest workspace first
  * (aq_reserve_workspace / aq_reserve_workspace_bytes), or capture again.
- * Gathers of more than 64 routes (aq_gather_qmv, aq_gather_qmv_gate_up) and matmuls in groups of 32 use the workspace
+ * Gathers of more than 64 routes (aq_gather_qmv, aq_gather_qmv_gate_up), matmuls in groups of 32, and aq_qmv, aq_qmv_multi and
+ * aq_qmv_gate_up of 2 to 64 rows that share a long K out (partial tiles of up to 16 shares) use the workspace
  * where they can have it and run without it where they cannot (during a capture that would have to grow it, or for want of
  * memory): they are never refused for it, and neither is a graph of them.  A graph keeps the block that it was captured over
  * until it is destroyed. */
@@ -173,7 +174,7 @@ int aq_qmm_multi(aq_ctx *ctx, const void *x, int count, const void *const *packe
  * go/engine/hip/hip_projection_launch.go:2671-2720). */
 int aq_reserve_workspace(aq_ctx *ctx, int M, int K);
 /* The same by size.  Besides those the workspace holds: the partial tiles of the few-rows kernels (5..64 rows, up to 64*M*N
- * bytes), those of all members of an aq_qmm_multi call and of both matrices of an aq_qmv_gate_up call, the lists of gathers of
+ * bytes) and of the matvec kernels of 2..64 rows (up to as much, of a pair twice), those of all members of an aq_qmm_multi call and of both matrices of an aq_qmv_gate_up call, the lists of gathers of
  * more than 64 routes, the intermediates of the unfused
  * fallbacks of the fused MLP / lm_head entry points, and the scratch of aq_packed_topk.  A call that needs
  * more than is there grows it (not possible while a capture is open): run such a call once before capturing,
