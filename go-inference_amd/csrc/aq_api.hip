@@ -89,8 +89,10 @@ struct aq_ctx {
 
 namespace {
 
-// The context's lock, held while a call selects and launches.  What the call gave a caller's stream to do over the scratch
-// blocks is noted before the lock is let go: another call may leave that stream, and its owner destroy it, right after.
+// The context's lock, held while a call selects and launches: from the entry point to its last launch, so that no other thread's
+// call comes between a launch that fills scratch and the one that reads it (functions below that launch expect it held).  What the
+// call gave a caller's stream to do over the scratch blocks is noted before the lock is let go: another call may leave that
+// stream, and its owner destroy it, right after.
 struct CallLock {
     aq_ctx* ctx;
     std::lock_guard<std::mutex> held;
@@ -778,9 +780,9 @@ int aq_probe_read(aq_ctx* ctx, const void* packed, const void* scales, const voi
     return AQ_OK;
 }
 
-int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases, void* y, int M,
-           int K, int N, int group_size, int bits, unsigned flags) {
-    if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv: ctx is null");
+namespace {
+int qmv_call(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
+             int group_size, int bits, unsigned flags) {
     if (M < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_qmv: M, K, N must be non-negative");
     if (M == 0 || N == 0 || K == 0) return AQ_OK;
     if (int rc = check_geometry("aq_qmv", K, group_size, bits)) return rc;
@@ -794,7 +796,6 @@ int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, c
     if (!x || !packed || (!tiled && (!scales || !biases)) || !y) return fail(AQ_ERR_ARG, "aq_qmv: null operand");
     if (!aligned(x, 2) || !aligned(packed, 4) || !aligned(scales, 2) || !aligned(biases, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_qmv: operand pointer is not element-aligned");
-    CallLock lk(ctx);
     aq::QmvArgs a{};
     a.x = static_cast<const uint16_t*>(x);
     a.w = static_cast<const uint32_t*>(packed);
@@ -808,6 +809,14 @@ int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, c
     a.routes = 1;
     if (tiled) return launch_qmv_tiled(ctx, a, group_size, bits);
     return launch_qmv_rows(ctx, a, group_size, bits, false);
+}
+}  // namespace
+
+int aq_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases, void* y, int M,
+           int K, int N, int group_size, int bits, unsigned flags) {
+    if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv: ctx is null");
+    CallLock lk(ctx);
+    return qmv_call(ctx, x, packed, scales, biases, y, M, K, N, group_size, bits, flags);
 }
 
 namespace {
@@ -840,12 +849,9 @@ aq::QmvArgs multi_member(const aq::QmvMultiArgs& ma, int i) {
     one.N = ma.N[i];
     return one;
 }
-}  // namespace
 
-int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packed, const void* const* scales,
-                 const void* const* biases, void* const* y, const int* N, int M, int K, int group_size, int bits,
-                 unsigned flags) {
-    if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv_multi: ctx is null");
+int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* packed, const void* const* scales, const void* const* biases,
+                   void* const* y, const int* N, int M, int K, int group_size, int bits, unsigned flags) {
     if (count < 0 || count > aq::kQmvMultiMax) return fail(AQ_ERR_ARG, "aq_qmv_multi: count must be 0..%d", aq::kQmvMultiMax);
     if (count == 0) return AQ_OK;
     if (!packed || !y || !N) return fail(AQ_ERR_ARG, "aq_qmv_multi: null array");
@@ -874,7 +880,6 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         }
         fused = fused && total < (int64_t)1 << 30;
         if (fused) {
-            CallLock lk(ctx);
             // the kernels aq_qmv would pick for each member, in one grid
             // (every variant with the same split of K computes the same bytes, whatever the rows per workgroup)
             const bool diag = !(ctx->families_off >> kFamDiag & 1);
@@ -918,7 +923,6 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     size_t bytes = 0;  // of the members' partial tiles
     aq::TokMultiArgs grid{};
     if (tok) {
-        CallLock lk(ctx);
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
         grid.common = all.common;
@@ -967,10 +971,9 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
     }
     for (int i = 0; i < count; i++) {
         if (in_grid >> i & 1) continue;
-        if (int rc = aq_qmv(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
+        if (int rc = qmv_call(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
     }
     if (in_grid) {
-        CallLock lk(ctx);
         // (the calls in between may have moved the workspace; it has held the tiles once and does not shrink)
         float* tiles = nullptr;
         if (!tok_tiles(ctx, bytes, &tiles)) return fail(AQ_ERR_NOMEM, "aq_qmv_multi: %zu bytes of workspace for partial tiles", bytes);
@@ -982,6 +985,15 @@ int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         AQ_HIP(aq::qmvt_multi_launch(ti, grid, bits, ctx->stream), "hipLaunchKernel");
     }
     return AQ_OK;
+}
+}  // namespace
+
+int aq_qmv_multi(aq_ctx* ctx, const void* x, int count, const void* const* packed, const void* const* scales,
+                 const void* const* biases, void* const* y, const int* N, int M, int K, int group_size, int bits,
+                 unsigned flags) {
+    if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv_multi: ctx is null");
+    CallLock lk(ctx);
+    return qmv_multi_call(ctx, x, count, packed, scales, biases, y, N, M, K, group_size, bits, flags);
 }
 
 int aq_qmm(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases, void* y, int M,
@@ -1019,6 +1031,7 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
                  const void* const* biases, void* const* y, const int* N, int M, int K, int group_size, int bits,
                  unsigned flags) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_qmm_multi: ctx is null");
+    CallLock lk(ctx);
     if (count < 1 || count > 8) return fail(AQ_ERR_ARG, "aq_qmm_multi: count must be 1..8");
     if (!packed || !scales || !biases || !y || !N) return fail(AQ_ERR_ARG, "aq_qmm_multi: null array");
     if (M <= 0 || K <= 0) return fail(AQ_ERR_SHAPE, "aq_qmm_multi: M, N, K must be positive");
@@ -1037,12 +1050,11 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
         // up to four rows: matvec calls (one launch per four members where the fused kernels take the shape)
         for (int i = 0; i < count; i += aq::kQmvMultiMax) {
             const int n = count - i < aq::kQmvMultiMax ? count - i : aq::kQmvMultiMax;
-            if (int rc = aq_qmv_multi(ctx, x, n, packed + i, scales + i, biases + i, y + i, N + i, M, K, group_size, bits, flags)) return rc;
+            if (int rc = qmv_multi_call(ctx, x, n, packed + i, scales + i, biases + i, y + i, N + i, M, K, group_size, bits, flags)) return rc;
         }
         ctx->last_variant[1] = ctx->last_variant[0];
         return AQ_OK;
     }
-    CallLock lk(ctx);
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
     // the members that the fp16-operand kernels take run as one grid (same bytes as on their own, see qmmh_split): narrow
     // matrices (k and v beside q) then fill the rounds of tiles that the wide ones leave part-empty
@@ -1231,7 +1243,6 @@ namespace {
 int gather_call(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
                 const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
                 int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags, bool grouped) {
-    if (!ctx) return fail(AQ_ERR_ARG, "aq_gather_qmv: ctx is null");
     if (routes < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_gather_qmv: routes, K, N must be non-negative");
     if (routes == 0 || N == 0 || K == 0) return AQ_OK;  // qmv_gather.go:422-424
     if (num_experts <= 0 || expert_rows <= 0 || x_rows <= 0)
@@ -1245,7 +1256,6 @@ int gather_call(aq_ctx* ctx, const void* x, const void* packed, const void* scal
         !aligned(rhs, 4) || (lhs && !aligned(lhs, 4)))
         return fail(AQ_ERR_ARG, "aq_gather_qmv: operand pointer is not element-aligned");
     if (routes > 65535) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv: at most 65535 routes per call");
-    CallLock lk(ctx);
     aq::QmvArgs a{};
     a.x = static_cast<const uint16_t*>(x);
     a.w = static_cast<const uint32_t*>(packed);
@@ -1273,6 +1283,8 @@ int gather_call(aq_ctx* ctx, const void* x, const void* packed, const void* scal
 int aq_gather_qmv(aq_ctx* ctx, const void* x, const void* packed, const void* scales, const void* biases,
                   const int32_t* lhs, const int32_t* rhs, void* y, int routes, int x_rows, int K, int N,
                   int num_experts, int expert_rows, int row_base, int group_size, int bits, unsigned flags) {
+    if (!ctx) return fail(AQ_ERR_ARG, "aq_gather_qmv: ctx is null");
+    CallLock lk(ctx);
     return gather_call(ctx, x, packed, scales, biases, lhs, rhs, y, routes, x_rows, K, N, num_experts, expert_rows, row_base,
                        group_size, bits, flags, true);
 }
@@ -1298,25 +1310,32 @@ int act_rows(const aq_ctx* ctx, int bits, int fuse, bool gather, int64_t N, int 
 
 }  // namespace
 
-int aq_act_mul(aq_ctx* ctx, const void* gate, const void* up, void* y, int64_t n, int act) {
-    if (!ctx) return fail(AQ_ERR_ARG, "aq_act_mul: ctx is null");
+namespace {
+int act_mul_call(aq_ctx* ctx, const void* gate, const void* up, void* y, int64_t n, int act) {
     if (n < 0) return fail(AQ_ERR_SHAPE, "aq_act_mul: n must be non-negative");
     if (!act_ok(act)) return fail(AQ_ERR_UNSUPPORTED, "aq_act_mul: unknown activation %d", act);
     if (n == 0) return AQ_OK;
     if (!gate || !up || !y) return fail(AQ_ERR_ARG, "aq_act_mul: null operand");
     if (!aligned(gate, 2) || !aligned(up, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_act_mul: operand pointer is not element-aligned");
-    CallLock lk(ctx);
     AQ_HIP(aq::act_mul_launch(static_cast<const uint16_t*>(gate), static_cast<const uint16_t*>(up),
                               static_cast<uint16_t*>(y), n, act, ctx->stream),
            "hipLaunchKernel");
     return AQ_OK;
+}
+}  // namespace
+
+int aq_act_mul(aq_ctx* ctx, const void* gate, const void* up, void* y, int64_t n, int act) {
+    if (!ctx) return fail(AQ_ERR_ARG, "aq_act_mul: ctx is null");
+    CallLock lk(ctx);
+    return act_mul_call(ctx, gate, up, y, n, act);
 }
 
 int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const void* gate_scales, const void* gate_biases,
                    const void* up_packed, const void* up_scales, const void* up_biases, void* y, int M, int K, int N,
                    int group_size, int bits, int act, unsigned flags) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv_gate_up: ctx is null");
+    CallLock lk(ctx);
     if (M < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_qmv_gate_up: M, K, N must be non-negative");
     if (!act_ok(act)) return fail(AQ_ERR_UNSUPPORTED, "aq_qmv_gate_up: unknown activation %d", act);
     if (M == 0 || N == 0) return AQ_OK;
@@ -1364,7 +1383,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, false, di) &&
             aq::qmvd_fits(up, bits, group_size, false, di) &&
             (size_t)M * K * 2 + (size_t)M * ((K + 255) / 256) * 48 + 128 + (size_t)2 * aq::qmvd_variant(di)->waves * 256 <= 96 * 1024) {
-            CallLock lk(ctx);
             ctx->last_variant[0] = "qmv_gate_up_diag";
             AQ_HIP(aq::qmvd_pair_launch(di, a, false, ctx->stream), "hipLaunchKernel");
             return AQ_OK;
@@ -1375,7 +1393,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         // of the unfused route, which then runs as for any other call
         // (a pair's partial tiles are twice a single matrix's)
         const size_t region = 2 * qmm_region(ctx, M, K, N) + 2 * align256((size_t)M * N * 4);
-        CallLock lk(ctx);
         AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
         if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * untiled_bytes(N, K), fail)) return rc;
         const uint32_t* w[2];
@@ -1387,7 +1404,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     }
     if (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) &&
         aligned(up_packed, 16)) {
-        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 1, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 1, rows, false)) {
             aq::QmvArgs a{};
@@ -1429,7 +1445,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         a.out_f32 = out_f32 ? 1 : 0;
         a.routes = 1;
         a.act = act;
-        CallLock lk(ctx);
         a.tokens = aq::qmvt_tokens(M);
         aq::qmvt_split(bits, group_size, M, K, N, true, ctx->cu_count, &a.ksplit, &a.share);
         if (!tok_tiles(ctx, aq::qmvt_tile_bytes(M, N, true, a.ksplit), &a.tile)) a.ksplit = 1;
@@ -1445,7 +1460,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         aq::qmmh_runs(M, K, N, group_size, bits)) {
         // prefill sizes on the fp16-operand kernels: one launch, the tiles of which hold gate and up columns side by side; no
         // intermediate reaches memory
-        CallLock lk(ctx);
         aq::QmmHalfCall q{};
         q.x = static_cast<const uint16_t*>(x);
         q.M = M;
@@ -1471,11 +1485,8 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
     // two projections into fp32 scratch, then the element-wise step
     const size_t region = qmm_region(ctx, M, K, N);
     const size_t each = (((size_t)M * N * 4) + 255) & ~(size_t)255;
-    {
-        CallLock lk(ctx);
-        AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * each, fail)) return rc;
-    }
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + 2 * each, fail)) return rc;
     float* g = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + region);
     float* u = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + region + each);
     if (M > 32 && ctx->forced[0] < 0 && !(ctx->families_off >> kFamTiles & 1) &&
@@ -1484,7 +1495,6 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         // pass over x is skipped, and the stores of the `up` projection apply act(gate) * up on the way out
         // (rocm_mlx_q4_gelu_tanh_multiply_batch, go/engine/hip/kernels/quant/affine_gelu_tanh.hipinc:921-1109): one
         // [M, N] fp32 matrix is written and read instead of two written and two read.  Same bytes as the route below.
-        CallLock lk(ctx);
         int x_state = aq::kXReadyNone;
         if (int rc = aq::qmm_dispatch(ctx->stream, &ctx->ws, ctx->cu_count, ctx->forced[1], &ctx->last_variant[1], x, gate_packed,
                                       gate_scales, gate_biases, g, M, K, N, group_size, bits, true, fail, nullptr, 0, &x_state))
@@ -1494,9 +1504,8 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         if (rc == AQ_OK) ctx->last_variant[0] = "qmv_gate_up_tiles";
         return rc;
     }
-    if (int rc = aq_qmv(ctx, x, gate_packed, gate_scales, gate_biases, g, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
-    if (int rc = aq_qmv(ctx, x, up_packed, up_scales, up_biases, u, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
-    CallLock lk(ctx);
+    if (int rc = qmv_call(ctx, x, gate_packed, gate_scales, gate_biases, g, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
+    if (int rc = qmv_call(ctx, x, up_packed, up_scales, up_biases, u, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
     AQ_HIP(aq::act_mul_f32_launch(g, u, y, (int64_t)M * N, act, out_f32 ? 1 : 0, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -1506,6 +1515,7 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
                           int num_experts, int expert_rows, int gate_row_base, int up_row_base, int group_size,
                           int bits, int act, unsigned flags) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_gather_qmv_gate_up: ctx is null");
+    CallLock lk(ctx);
     if (routes < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_gather_qmv_gate_up: routes, K, N must be non-negative");
     if (!act_ok(act)) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv_gate_up: unknown activation %d", act);
     if (routes == 0 || N == 0) return AQ_OK;
@@ -1546,19 +1556,14 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
         a.x_rows = x_rows;
         a.routes = routes;
         a.act = act;
-        {
-            CallLock lk(ctx);
-            if (const int rc = run_grouped(ctx, a, group_size, bits, true); rc != kPass) return rc;
-        }
+        if (const int rc = run_grouped(ctx, a, group_size, bits, true); rc != kPass) return rc;
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, true, di)) {
-            CallLock lk(ctx);
             ctx->last_variant[0] = "gather_gate_up_diag";
             AQ_HIP(aq::qmvd_pair_launch(di, a, true, ctx->stream), "hipLaunchKernel");
             return AQ_OK;
         }
     }
     if (ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, packed, (size_t)K * 2)) {
-        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 1, true, N, K, routes);
         if (aq::qmv_act_supported(bits, 1, rows, true)) {
             aq::QmvArgs a{};
@@ -1587,11 +1592,8 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
         }
     }
     const size_t each = (((size_t)routes * N * 4) + 255) & ~(size_t)255;
-    {
-        CallLock lk(ctx);
-        AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, 2 * each, fail)) return rc;
-    }
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, 2 * each, fail)) return rc;
     float* g = static_cast<float*>(ctx->ws.ptr);
     float* u = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + each);
     if (int rc = gather_call(ctx, x, packed, scales, biases, lhs, rhs, g, routes, x_rows, K, N, num_experts, expert_rows,
@@ -1600,7 +1602,6 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
     if (int rc = gather_call(ctx, x, packed, scales, biases, lhs, rhs, u, routes, x_rows, K, N, num_experts, expert_rows,
                              up_row_base, group_size, bits, AQ_OUT_F32, false))
         return rc;
-    CallLock lk(ctx);
     AQ_HIP(aq::act_mul_f32_launch(g, u, y, (int64_t)routes * N, act, out_f32 ? 1 : 0, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
 }
@@ -1608,6 +1609,7 @@ int aq_gather_qmv_gate_up(aq_ctx* ctx, const void* x, const void* packed, const 
 int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* packed, const void* scales,
                const void* biases, void* y, int M, int K, int N, int group_size, int bits, int act, unsigned flags) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_qmv_act: ctx is null");
+    CallLock lk(ctx);
     if (M < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_qmv_act: M, K, N must be non-negative");
     if (!act_ok(act)) return fail(AQ_ERR_UNSUPPORTED, "aq_qmv_act: unknown activation %d", act);
     if (M == 0 || N == 0 || K == 0) return AQ_OK;
@@ -1618,7 +1620,6 @@ int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* pa
         return fail(AQ_ERR_ARG, "aq_qmv_act: operand pointer is not element-aligned");
     if (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, gate_x, packed, (size_t)K * 2) &&
         aligned(up_x, 16)) {
-        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 2, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 2, rows, false)) {
             aq::QmvArgs a{};
@@ -1641,14 +1642,11 @@ int aq_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* pa
         }
     }
     const size_t region = qmm_region(ctx, M, K, N);
-    {
-        CallLock lk(ctx);
-        AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * K * 2, fail)) return rc;
-    }
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * K * 2, fail)) return rc;
     void* gated = static_cast<char*>(ctx->ws.ptr) + region;
-    if (int rc = aq_act_mul(ctx, gate_x, up_x, gated, (int64_t)M * K, act)) return rc;
-    return aq_qmv(ctx, gated, packed, scales, biases, y, M, K, N, group_size, bits, flags);
+    if (int rc = act_mul_call(ctx, gate_x, up_x, gated, (int64_t)M * K, act)) return rc;
+    return qmv_call(ctx, gated, packed, scales, biases, y, M, K, N, group_size, bits, flags);
 }
 
 int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const void* packed, const void* scales,
@@ -1656,6 +1654,7 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
                       int N, int num_experts, int expert_rows, int row_base, int group_size, int bits, int act,
                       unsigned flags) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_gather_qmv_act: ctx is null");
+    CallLock lk(ctx);
     if (routes < 0 || K < 0 || N < 0) return fail(AQ_ERR_SHAPE, "aq_gather_qmv_act: routes, K, N must be non-negative");
     if (!act_ok(act)) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv_act: unknown activation %d", act);
     if (routes == 0 || N == 0 || K == 0) return AQ_OK;
@@ -1672,7 +1671,6 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
         return fail(AQ_ERR_ARG, "aq_gather_qmv_act: operand pointer is not element-aligned");
     if (routes > 65535) return fail(AQ_ERR_UNSUPPORTED, "aq_gather_qmv_act: at most 65535 routes per call");
     if (ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, gate_x, packed, (size_t)K * 2) && aligned(up_x, 16)) {
-        CallLock lk(ctx);
         const int rows = act_rows(ctx, bits, 2, true, N, K, routes);
         if (aq::qmv_act_supported(bits, 2, rows, true)) {
             aq::QmvArgs a{};
@@ -1700,12 +1698,9 @@ int aq_gather_qmv_act(aq_ctx* ctx, const void* gate_x, const void* up_x, const v
             return AQ_OK;
         }
     }
-    {
-        CallLock lk(ctx);
-        AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, (size_t)x_rows * K * 2, fail)) return rc;
-    }
-    if (int rc = aq_act_mul(ctx, gate_x, up_x, ctx->ws.ptr, (int64_t)x_rows * K, act)) return rc;
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, (size_t)x_rows * K * 2, fail)) return rc;
+    if (int rc = act_mul_call(ctx, gate_x, up_x, ctx->ws.ptr, (int64_t)x_rows * K, act)) return rc;
     return gather_call(ctx, ctx->ws.ptr, packed, scales, biases, lhs, rhs, y, routes, x_rows, K, N, num_experts, expert_rows,
                        row_base, group_size, bits, flags, false);
 }
@@ -1790,6 +1785,7 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
               const void* biases, const int32_t* suppress, int suppress_count, uint64_t* out, int M, int K, int N,
               int group_size, int bits, bool no_alloc = false) {
     if (!ctx) return fail(AQ_ERR_ARG, "%s: ctx is null", op);
+    CallLock lk(ctx);
     if (M < 0 || K < 0 || N < 0 || suppress_count < 0) return fail(AQ_ERR_SHAPE, "%s: M, K, N, suppress_count must be non-negative", op);
     if (M == 0) return AQ_OK;
     if (!out) return fail(AQ_ERR_ARG, "%s: null output", op);
@@ -1806,7 +1802,6 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
                     "other shapes need scratch memory: use aq_qmv_greedy", op);
     if (fuse == 3 && !fused && !(K > 0 && aq::best_score_clears(N))) {
         // the unfused reduction of long rows accumulates with atomics and starts from "no result"
-        CallLock lk(ctx);
         AQ_HIP(aq::fill_zero_launch(out, (size_t)M * 8, ctx->stream), "hipLaunchKernel");
     }
     if (N == 0) return AQ_OK;
@@ -1816,7 +1811,6 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
     if (!aligned(x, 2) || !aligned(packed, 4) || !aligned(scales, 2) || !aligned(biases, 2))
         return fail(AQ_ERR_ARG, "%s: operand pointer is not element-aligned", op);
     if (fused) {
-        CallLock lk(ctx);
         {
             // the diagonal-MFMA kernel aq_qmv would pick for this projection, with the head epilogue
             const int di = bits != 4 || (ctx->families_off >> kFamDiag & 1) ? -1
@@ -1889,14 +1883,10 @@ int head_call(aq_ctx* ctx, const char* op, int fuse, const void* x, const void* 
     }
     // the projection as fp32 into scratch, then the same epilogue over it
     const size_t region = qmm_region(ctx, M, K, N);
-    {
-        CallLock lk(ctx);
-        AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-        if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * N * 4, fail)) return rc;
-    }
+    AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
+    if (int rc = aq::workspace_reserve(ctx->stream, &ctx->ws, region + (size_t)M * N * 4, fail)) return rc;
     float* logits = reinterpret_cast<float*>(static_cast<char*>(ctx->ws.ptr) + region);
-    if (int rc = aq_qmv(ctx, x, packed, scales, biases, logits, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
-    CallLock lk(ctx);
+    if (int rc = qmv_call(ctx, x, packed, scales, biases, logits, M, K, N, group_size, bits, AQ_OUT_F32)) return rc;
     unsigned long long* o = reinterpret_cast<unsigned long long*>(out);
     AQ_HIP(fuse == 3 ? aq::best_score_launch(logits, M, N, suppress, suppress_count, o, ctx->stream)
                      : aq::pack_scores_launch(logits, M, N, suppress, suppress_count, o, ctx->stream),

@@ -20,9 +20,10 @@
  * conditions as Go errors ("HIP returned <rc>", go/engine/hip/hip_driver_cgo.go:1728-1730;
  * shape errors, go/engine/hip/hip_projection_reference.go:122-144).
  *
- * Threading: calls on one aq_ctx are serialised by an internal mutex; kernels
- * are enqueued on the context's stream and are asynchronous with respect to
- * the host unless the entry point says otherwise.
+ * Threading: calls on one aq_ctx are serialised by an internal mutex, held
+ * until a call's last launch; kernels are enqueued on the context's stream and
+ * are asynchronous with respect to the host unless the entry point says
+ * otherwise.
  */
 #ifndef AQ_MI355_H
 #define AQ_MI355_H

@@ -1,0 +1,190 @@
+// The library's entry points against a HIP runtime of this program's own, which launches nothing and writes down what it is
+// asked: which call of which thread launched which kernel, and what memory was asked for.  So order and scratch can be checked
+// without a GPU.  The definitions here take the place of the runtime's when the program loads libaq_mi355.so.
+#include "aq_mi355.h"
+
+#include <dlfcn.h>
+#include <hip/hip_runtime_api.h>
+#include <pthread.h>
+#include <unistd.h>
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <thread>
+#include <vector>
+
+struct Launch {
+    int thread, call;
+    std::string kernel;
+};
+static std::vector<Launch> log_;
+static std::mutex log_mu;
+static thread_local int this_thread = 0, this_call = 0;
+static std::map<const void*, std::string>& names() {  // (filled while the library is being loaded)
+    static std::map<const void*, std::string> m;
+    return m;
+}
+static uintptr_t next_address = 1ull << 32;
+static void* address(size_t n) {
+    const uintptr_t p = next_address;
+    next_address += (n + 511) & ~(size_t)255;
+    return reinterpret_cast<void*>(p);
+}
+
+// Other threads get their turn wherever a lock is let go.
+extern "C" int pthread_mutex_unlock(pthread_mutex_t* m) {
+    static int (*const real)(pthread_mutex_t*) = reinterpret_cast<int (*)(pthread_mutex_t*)>(dlsym(RTLD_NEXT, "pthread_mutex_unlock"));
+    const int rc = real(m);
+    if (this_thread) usleep(20);
+    return rc;
+}
+
+extern "C" {
+void** __hipRegisterFatBinary(const void*) {
+    static void* handle = nullptr;
+    return &handle;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*, void*, void*, void*, int*) { names()[host] = name; }
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+static thread_local dim3 grid_, block_;
+static thread_local size_t lds_;
+static thread_local hipStream_t stream_;
+hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {
+    grid_ = g, block_ = b, lds_ = lds, stream_ = s;
+    return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t* s) {
+    *g = grid_, *b = block_, *lds = lds_, *s = stream_;
+    return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void**, size_t, hipStream_t) {
+    std::lock_guard<std::mutex> lk(log_mu);
+    log_.push_back({this_thread, this_call, names()[fn]});
+    return hipSuccess;
+}
+hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
+hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {  // (the header's name for the versioned symbol)
+    memset(p, 0, sizeof *p);
+    strcpy(p->gcnArchName, "gfx950");
+    p->multiProcessorCount = 256;
+    return hipSuccess;
+}
+hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
+hipError_t hipFuncSetAttribute(const void*, hipFuncAttribute, int) { return hipSuccess; }
+hipError_t hipGetSymbolAddress(void** p, const void*) { return *p = address(4 << 20), hipSuccess; }
+static size_t allocated = 0;
+hipError_t hipMalloc(void** p, size_t n) {
+    allocated += n;
+    return *p = address(n), hipSuccess;
+}
+hipError_t hipFree(void*) { return hipSuccess; }
+hipError_t hipMemset(void*, int, size_t) { return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "?"; }
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) { return *s = reinterpret_cast<hipStream_t>(16), hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+static int drains = 0;
+hipError_t hipStreamSynchronize(hipStream_t) { return drains++, hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
+static bool capturing = false;
+hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus* s) {
+    return *s = capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone, hipSuccess;
+}
+hipError_t hipDeviceSynchronize(void) { return hipSuccess; }
+hipError_t hipEventCreate(hipEvent_t* e) { return *e = reinterpret_cast<hipEvent_t>(32), hipSuccess; }
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { return hipEventCreate(e); }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+}
+
+static int failures = 0;
+#define CHECK(what, ...)                   \
+    do {                                   \
+        if (!(what)) {                     \
+            failures++;                    \
+            printf("%s: ", #what);         \
+            printf(__VA_ARGS__);           \
+            puts("");                      \
+        }                                  \
+    } while (0)
+
+static aq_ctx* ctx;
+static void* const X = address(1 << 24);
+static void* const W = address((size_t)1 << 32);
+static void* const S = address(1 << 28);
+static void* const B = address(1 << 28);
+static void* const Y = address(1 << 28);
+static int qmv(int M, int K, int N, int group, int bits) { return aq_qmv(ctx, X, W, S, B, Y, M, K, N, group, bits, 0); }
+
+// The launches of a call follow each other: with another thread's call between the one that fills scratch and the one that reads
+// it, the reader finds what that call left there.
+static void test_calls_stay_whole() {
+    typedef int (*Call)();
+    static const Call calls[] = {
+        [] { return aq_qmv_greedy(ctx, X, W, S, B, nullptr, 0, static_cast<uint64_t*>(Y), 4, 1536, 3000, 32, 4); },
+        [] { return aq_qmv_scores(ctx, X, W, S, B, nullptr, 0, static_cast<uint64_t*>(Y), 20, 14336, 700, 64, 4); },
+        [] { return aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, 3, 768, 500, 64, 6, AQ_ACT_SILU, 0); },
+        [] { return aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, 100, 768, 500, 64, 8, AQ_ACT_SILU, 0); },
+        [] { return aq_qmv_act(ctx, X, Y, W, S, B, Y, 24, 14336, 640, 64, 4, AQ_ACT_SILU, 0); },
+        [] { return aq_gather_qmv_gate_up(ctx, X, W, S, B, nullptr, static_cast<int32_t*>(S), Y, 9, 1, 768, 96, 4, 192, 0, 96, 64, 6, AQ_ACT_SILU, 0); },
+        [] { return aq_gather_qmv_act(ctx, X, Y, W, S, B, nullptr, static_cast<int32_t*>(S), Y, 9, 1, 768, 96, 4, 96, 0, 64, 6, AQ_ACT_SILU, 0); },
+        [] {
+            const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+            void* y[3] = {Y, Y, Y};
+            const int N[3] = {600, 500, 1000};
+            return aq_qmv_multi(ctx, X, 3, w, s, b, y, N, 40, 14336, 64, 4, 0);
+        },
+        [] {
+            const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+            void* y[3] = {Y, Y, Y};
+            const int N[3] = {600, 500, 1000};
+            return aq_qmm_multi(ctx, X, 3, w, s, b, y, N, 3, 768, 32, 4, 0);
+        },
+    };
+    int several = 0;
+    auto body = [&](int thread) {
+        this_thread = thread;
+        for (int round = 0; round < 4; round++)
+            for (const Call& c : calls) {
+                this_call++;
+                const int rc = thread == 1 ? c() : qmv(24, 14336, 4096, 64, 4);
+                std::lock_guard<std::mutex> lk(log_mu);
+                CHECK(rc == AQ_OK, "thread %d call %d: %d %s", thread, this_call, rc, aq_last_error());
+            }
+        this_thread = 0;
+    };
+    log_.clear();
+    std::thread one(body, 1), two(body, 2);
+    one.join();
+    two.join();
+    std::map<std::pair<int, int>, size_t> last;
+    for (size_t i = 0; i < log_.size(); i++) {
+        const std::pair<int, int> call{log_[i].thread, log_[i].call};
+        const auto before = last.find(call);
+        if (before != last.end()) {
+            several++;
+            CHECK(before->second + 1 == i, "thread %d call %d: %s, then %s of thread %d, then %s", call.first, call.second,
+                  log_[before->second].kernel.c_str(), log_[i - 1].kernel.c_str(), log_[i - 1].thread, log_[i].kernel.c_str());
+        }
+        last[call] = i;
+    }
+    CHECK(several >= 4 * 9, "%d launches behind another of their call", several);
+}
+
+int main() {
+    if (aq_create(0, &ctx) != AQ_OK) {
+        printf("aq_create: %s\n", aq_last_error());
+        return 1;
+    }
+    test_calls_stay_whole();
+    aq_destroy(ctx);
+    if (!failures) puts("ok");
+    return failures ? 1 : 0;
+}
