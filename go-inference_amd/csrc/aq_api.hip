@@ -6,6 +6,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <array>
 #include <climits>
 #include <cmath>
 #include <cstdarg>
@@ -79,6 +80,9 @@ struct aq_ctx {
     int cu_count = 0;
     aq::Workspace ws;       // scratch of the matmul path and of the unfused fallbacks (aq_qmm.h)
     aq::Workspace head_ws;         // per-wavefront maxima of aq_qmv_greedy; sized at creation for common vocabularies
+    aq::Workspace tok_ws;   // partial tiles of the token-tile kernels: aq::kTokTileBytes from creation on, so that their calls
+                            // neither allocate nor go without, and leave what other calls keep in `ws` alone
+    std::array<aq::Workspace*, 3> blocks() { return {&ws, &head_ws, &tok_ws}; }
     void* head_fold = nullptr;     // aq_qmv_greedy's fold tickets and slots (aq::kHeadFoldBytes, kept zeroed by the kernel)
     unsigned char* static_scratch = nullptr;  // this device's copy of `scratch` (hipGetSymbolAddress at creation)
     char name[256] = {0};
@@ -99,8 +103,7 @@ struct CallLock {
     explicit CallLock(aq_ctx* c) : ctx(c), held(c->mu) {}
     ~CallLock() {
         if (ctx->stream == ctx->own_stream) return;
-        (void)aq::workspace_note(ctx->stream, &ctx->ws, ctx->leaves_streams);
-        (void)aq::workspace_note(ctx->stream, &ctx->head_ws, ctx->leaves_streams);
+        for (aq::Workspace* ws : ctx->blocks()) (void)aq::workspace_note(ctx->stream, ws, ctx->leaves_streams);
     }
 };
 
@@ -260,7 +263,8 @@ const QmvRule kQmvRules[] = {
                                             // has the bytes of a call with that row alone
     {8, 0, 0, 1, 1, kFamDot2},              // one row of 8-bit codes: the dot2 kernel with its non-temporal loads, 12.4 us for
                                             // 4096 x 14336 (63 % of the HBM peak) against 14.2 us on the block-MFMA kernel
-    {8, 64, 0, 2, 32, kFamTok},             // K a multiple of 256 up to 16384: one launch, weights streamed once, no scratch
+    {8, 64, 0, 2, 32, kFamTok},             // K a multiple of 64 up to 16384: weights streamed once in one launch, and a sum of
+                                            // partial tiles behind it where workgroups share K out
                                             // (4 rows of 4096 x 14336: 14.3 us against 15.0 on the block-MFMA kernels, 21.5 on
                                             // the dot2 kernels; the reference states its rows-equal-single-rows contract for
                                             // 4-bit codes only, qmv_rows_test.go:36-41)
@@ -373,13 +377,11 @@ bool tok_halves(const aq_ctx* ctx, int group_size, int M, int64_t rows, bool pai
     return groups <= (group_size == 128 || (pair && group_size == 64) ? 2 : 1) * cus;
 }
 
-// Partial tiles for a token-tile call that shares K out: the context's workspace, if it is to be had (not while the stream is
-// being captured and it is too small: the call then runs without shares).
-bool tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
-    if (bytes == 0) return true;
-    if (hipSetDevice(ctx->device) != hipSuccess || !aq::workspace_offer(ctx->stream, &ctx->ws, bytes)) return false;
-    *tile = static_cast<float*>(ctx->ws.ptr);
-    return true;
+// Room for the partial tiles of a token-tile call that shares K out (qmvt_split keeps them inside the block).
+hipError_t tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
+    if (bytes == 0) return hipSuccess;
+    *tile = static_cast<float*>(ctx->tok_ws.ptr);
+    return aq::workspace_use(ctx->stream, &ctx->tok_ws);
 }
 int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, bool pair) {
     const int64_t bands = (int64_t)((t.N + 15) / 16) * (pair ? 2 : 1) * (t.ksplit > 1 ? t.ksplit : 1);
@@ -393,12 +395,12 @@ int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool ga
     t.tokens = forced < 0 ? aq::qmvt_tokens(a.M) : a.M;
     if (forced < 0 && !tok_small(bits, group_size, a.M, a.K, a.N) && tok_halves(ctx, group_size, a.M, a.N, false)) {
         aq::qmvt_split(bits, group_size, a.M, a.K, a.N, false, ctx->cu_count, &t.ksplit, &t.share);
-        if (!tok_tiles(ctx, aq::qmvt_tile_bytes(a.M, a.N, false, t.ksplit), &t.tile)) t.ksplit = 1;
     } else if (forced < 0) {
         return kPass;
     }
     const int ti = forced >= 0 ? forced : tok_pick(ctx, t, group_size, bits, false);
     if (ti < 0 || !aq::qmvt_fits(t, bits, group_size, ti, forced >= 0)) return kPass;
+    AQ_HIP(tok_tiles(ctx, aq::qmvt_tile_bytes(a.M, a.N, false, t.ksplit), &t.tile), "hipStreamWaitEvent");
     ctx->last_variant[0] = aq::qmvt_name(ti, t);
     AQ_HIP(aq::qmvt_launch(ti, t, ctx->stream), "hipLaunchKernel");
     return AQ_OK;
@@ -553,6 +555,7 @@ int aq_create(int device, aq_ctx** out) {
         rc = aq::workspace_open(&ctx->head_ws, (size_t)4 << 20);
     }
     if (rc == hipSuccess) rc = aq::workspace_open(&ctx->ws, 0);
+    if (rc == hipSuccess) rc = aq::workspace_open(&ctx->tok_ws, aq::kTokTileBytes);
     if (rc != hipSuccess) {
         aq_destroy(ctx);
         return hip_fail(rc, "hipStreamCreate");
@@ -575,8 +578,7 @@ void aq_destroy(aq_ctx* ctx) {
         (void)hipStreamDestroy(ctx->own_stream);
     }
     delete ctx->host;
-    aq::workspace_close(&ctx->ws);
-    aq::workspace_close(&ctx->head_ws);
+    for (aq::Workspace* ws : ctx->blocks()) aq::workspace_close(ws);
     if (ctx->head_fold) (void)hipFree(ctx->head_fold);
     if (ctx->ev0) (void)hipEventDestroy(ctx->ev0);
     if (ctx->ev1) (void)hipEventDestroy(ctx->ev1);
@@ -591,7 +593,7 @@ int go_to_stream(aq_ctx* ctx, hipStream_t stream) {
     ctx->stream = stream;
     if (stream == old) return AQ_OK;
     hipError_t first = hipSuccess;
-    for (aq::Workspace* ws : {&ctx->ws, &ctx->head_ws}) {
+    for (aq::Workspace* ws : ctx->blocks()) {
         hipError_t rc = old == ctx->own_stream ? aq::workspace_note(old, ws) : hipSuccess;  // (others: CallLock)
         const hipError_t left = aq::workspace_leave(ws);
         rc = rc == hipSuccess ? left : rc;
@@ -708,19 +710,20 @@ struct aq_graph {
             if (used) block = ws.block;
         }
         bool stale(const aq::Workspace& ws) const { return required && generation != ws.generation; }
-    } ws, head_ws;
+    };
+    std::array<Scratch, 3> scratch;  // of aq_ctx::blocks
 };
 
 int aq_capture_begin(aq_ctx* ctx) {
     if (!ctx) return fail(AQ_ERR_ARG, "aq_capture_begin: ctx is null");
     CallLock lk(ctx);
     if (ctx->stream == nullptr) return fail(AQ_ERR_UNSUPPORTED, "aq_capture_begin: the legacy default stream cannot be captured");
-    for (aq::Workspace* ws : {&ctx->ws, &ctx->head_ws}) {
+    for (aq::Workspace* ws : ctx->blocks()) {
         AQ_HIP(aq::workspace_note(ctx->stream, ws), "hipEventRecord");
         AQ_HIP(aq::workspace_leave(ws), "hipDeviceSynchronize");
     }
     AQ_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal), "hipStreamBeginCapture");
-    ctx->ws.touched = ctx->ws.required = ctx->head_ws.touched = ctx->head_ws.required = false;
+    for (aq::Workspace* ws : ctx->blocks()) ws->touched = ws->required = false;
     return AQ_OK;
 }
 
@@ -736,8 +739,7 @@ int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
         return fail(AQ_ERR_NOMEM, "aq_capture_end: out of host memory");
     }
     ag->graph = g;
-    ag->ws.note(ctx->ws);
-    ag->head_ws.note(ctx->head_ws);
+    for (size_t i = 0; i < ag->scratch.size(); i++) ag->scratch[i].note(*ctx->blocks()[i]);
     hipError_t rc = hipGraphInstantiate(&ag->exec, g, nullptr, nullptr, 0);
     if (rc != hipSuccess) {
         aq_graph_destroy(ag);
@@ -750,13 +752,14 @@ int aq_capture_end(aq_ctx* ctx, aq_graph** out) {
 int aq_graph_launch(aq_ctx* ctx, aq_graph* graph) {
     if (!ctx || !graph || !graph->exec) return fail(AQ_ERR_ARG, "aq_graph_launch: bad argument");
     CallLock lk(ctx);
-    if (graph->ws.stale(ctx->ws) || graph->head_ws.stale(ctx->head_ws))
-        return fail(AQ_ERR_UNSUPPORTED,
-                    "aq_graph_launch: the context's workspace was reallocated after this graph was captured (a later call "
-                    "needed more room); the graph's kernels still point at the old block: capture it again, and reserve "
-                    "the largest workspace first (aq_reserve_workspace / aq_reserve_workspace_bytes)");
-    if (graph->ws.used) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->ws), "hipStreamWaitEvent");
-    if (graph->head_ws.used) AQ_HIP(aq::workspace_use(ctx->stream, &ctx->head_ws), "hipStreamWaitEvent");
+    for (size_t i = 0; i < graph->scratch.size(); i++)
+        if (graph->scratch[i].stale(*ctx->blocks()[i]))
+            return fail(AQ_ERR_UNSUPPORTED,
+                        "aq_graph_launch: the context's workspace was reallocated after this graph was captured (a later call "
+                        "needed more room); the graph's kernels still point at the old block: capture it again, and reserve "
+                        "the largest workspace first (aq_reserve_workspace / aq_reserve_workspace_bytes)");
+    for (size_t i = 0; i < graph->scratch.size(); i++)
+        if (graph->scratch[i].used) AQ_HIP(aq::workspace_use(ctx->stream, ctx->blocks()[i]), "hipStreamWaitEvent");
     AQ_HIP(hipGraphLaunch(graph->exec, ctx->stream), "hipGraphLaunch");
     return AQ_OK;
 }
@@ -950,7 +953,6 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             total += N[i];
         }
         grid.count = members;
-        float* room = nullptr;
         int64_t bands = 0;
         int runs = 1;
         for (int i = 0; i < members; i++) {
@@ -966,17 +968,15 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             one.share = grid.share[i];
             if (!aq::qmvt_fits(one, bits, group_size, ti, false)) ti = -1;
         }
-        // without room for all the tiles every member decides by itself, as its own call does
-        if (ti < 0 || !tok_tiles(ctx, bytes, &room)) in_grid = 0;
+        if (ti < 0 || bytes > aq::kTokTileBytes) in_grid = 0;  // (members apart have the block to themselves, one after another)
     }
     for (int i = 0; i < count; i++) {
         if (in_grid >> i & 1) continue;
         if (int rc = qmv_call(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
     }
     if (in_grid) {
-        // (the calls in between may have moved the workspace; it has held the tiles once and does not shrink)
         float* tiles = nullptr;
-        if (!tok_tiles(ctx, bytes, &tiles)) return fail(AQ_ERR_NOMEM, "aq_qmv_multi: %zu bytes of workspace for partial tiles", bytes);
+        AQ_HIP(tok_tiles(ctx, bytes, &tiles), "hipStreamWaitEvent");
         for (int i = 0; i < grid.count; i++) {
             grid.tile[i] = grid.ksplit[i] > 1 ? tiles : nullptr;
             tiles += aq::qmvt_tile_bytes(M, grid.N[i], false, grid.ksplit[i]) / 4;
@@ -1128,7 +1128,9 @@ size_t aq_workspace_bytes(aq_ctx* ctx) {
     if (!ctx) return 0;
     std::lock_guard<std::mutex> host_lk(ctx->host_mu);
     CallLock lk(ctx);
-    return ctx->ws.bytes + ctx->head_ws.bytes + (ctx->host ? ctx->host->device_bytes() : 0);
+    size_t bytes = ctx->host ? ctx->host->device_bytes() : 0;
+    for (const aq::Workspace* ws : ctx->blocks()) bytes += ws->bytes;
+    return bytes;
 }
 
 namespace {
@@ -1447,9 +1449,9 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         a.act = act;
         a.tokens = aq::qmvt_tokens(M);
         aq::qmvt_split(bits, group_size, M, K, N, true, ctx->cu_count, &a.ksplit, &a.share);
-        if (!tok_tiles(ctx, aq::qmvt_tile_bytes(M, N, true, a.ksplit), &a.tile)) a.ksplit = 1;
         const int ti = tok_pick(ctx, a, group_size, bits, true);
         if (ti >= 0 && aq::qmvt_pair_supported(ti) && aq::qmvt_fits(a, bits, group_size, ti, false)) {
+            AQ_HIP(tok_tiles(ctx, aq::qmvt_tile_bytes(M, N, true, a.ksplit), &a.tile), "hipStreamWaitEvent");
             ctx->last_variant[0] = "qmv_gate_up_tok";
             AQ_HIP(aq::qmvt_pair_launch(ti, a, ctx->stream), "hipLaunchKernel");
             return AQ_OK;

@@ -168,8 +168,8 @@ bool qmvd_multi_supported(int idx);
 hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream);
 
 // Token-tile MFMA matvec kernels (aq_qmv_tok.hip; codes of 4 or 8 bits in groups of 32, 64 or 128, up to 64 activation rows
-// as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch without scratch memory, or shares of K and a sum of
-// their partial tiles).  kind 6 in QmvVariant.
+// as the rows of 16x16x32 MFMAs, K a multiple of 64 up to 16384; one launch, or shares of K and a sum of their partial tiles in
+// a block of scratch that the context makes when it is made).  kind 6 in QmvVariant.
 // Their arguments (apart from QmvArgs: those of the one-row kernels stay as short as they were, 0.04 us a launch).
 struct TokArgs : QmvArgs {
     int ksplit, share;  // shares of K (0, 1: none), 256-code runs per share
@@ -190,14 +190,16 @@ const char* qmvt_name(int idx, const TokArgs& a);  // the kernel qmvt_launch run
 hipError_t qmvt_launch(int idx, const TokArgs& a, hipStream_t stream);
 // Rows of x per workgroup (a.tokens): all of up to 32, else half of them.
 int qmvt_tokens(int M);
-// How a matrix of N rows (pair: two) shares K out over workgroups, a function of the matrix's own call alone so that it has the
-// same bytes in a grid of several: 1 share, or more whose partial tiles take qmvt_tile_bytes.
+// How a matrix of N rows (pair: two) shares K out over workgroups: 1 share, or more whose partial tiles take qmvt_tile_bytes, at
+// most kTokTileBytes.  A function of the width, the group size, K, N and whether x has more than 32 rows, so that a row of x has
+// the same bytes in calls of any up to 32 rows (any 33..64), and a matrix the same in a grid of several as by itself.
+constexpr size_t kTokTileBytes = (size_t)32 << 20;
 void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share);
 size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit);
 // The variant for `sets` sets of 16 weight rows times their shares of K, the longest share being `runs` runs of 256 codes; or -1.
 int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count);
 // Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
-// sums are those of qmvt_launch.
+// sums are those of qmvt_launch with the same shares (the pair has its own: twice the workgroups a share).
 hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t stream);
 bool qmvt_pair_supported(int idx);
 hipError_t qmvt_pair_launch(int idx, const TokArgs& a, hipStream_t stream);

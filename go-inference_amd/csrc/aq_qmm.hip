@@ -59,15 +59,6 @@ size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
             partial = half > partial ? half : partial;
         }
     }
-    // the token-tile kernels' shares of K (callers keep rows of theirs behind this region while aq_qmv runs, behind two of them
-    // while aq_qmv_gate_up does)
-    for (int form = 0; form < 8; form++) {
-        const bool pair = form & 1;
-        int ksplit, share;
-        qmvt_split(form & 2 ? 8 : 4, form & 4 ? 32 : 64, M, K, N, pair, cu_count, &ksplit, &share);
-        const size_t tiles = qmvt_tile_bytes(M, N, pair, ksplit) / (pair ? 2 : 1);
-        partial = tiles > partial ? tiles : partial;
-    }
     return xbytes + ((partial + 255) & ~(size_t)255);
 }
 

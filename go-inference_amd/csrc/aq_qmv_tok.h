@@ -74,7 +74,7 @@ typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) u32x2_a2_t;
 //     with ones, which leave them in every lane of their token.
 //   * a wavefront keeps the A operands of its run in registers and streams the sets of rows past them, RING sets in
 //     flight (see the loop); the wavefronts' partial sums meet in LDS.
-// Token t of an M-row call equals token t of any other call on the same variant with the same shares of K, bit for bit.
+// Token t of an M-row call equals token t of any other call with the same shares of K (qmvt_split), bit for bit.
 // Any K that is a multiple of 64: a run that K ends inside reads its last 16 bytes again and multiplies them with zeros of x
 // under scales of zero.
 // What the operand holds of a code, and why.  A weight is near zero on average: what the operand has beside it comes off again,

@@ -102,11 +102,12 @@ int aq_timer_stop(aq_ctx *ctx, float *elapsed_ms); /* records, waits, reports */
  * fails with a message), and when a later such call makes it grow, every graph captured over the old block is
  * refused by aq_graph_launch with AQ_ERR_UNSUPPORTED - reserve the largest workspace first
  * (aq_reserve_workspace / aq_reserve_workspace_bytes), or capture again.
- * Gathers of more than 64 routes (aq_gather_qmv, aq_gather_qmv_gate_up), matmuls in groups of 32, and aq_qmv, aq_qmv_multi and
- * aq_qmv_gate_up of 2 to 64 rows that share a long K out (partial tiles of up to 16 shares) use the workspace
+ * Gathers of more than 64 routes (aq_gather_qmv, aq_gather_qmv_gate_up) and matmuls in groups of 32 use the workspace
  * where they can have it and run without it where they cannot (during a capture that would have to grow it, or for want of
  * memory): they are never refused for it, and neither is a graph of them.  A graph keeps the block that it was captured over
- * until it is destroyed. */
+ * until it is destroyed.  The token-tile kernels (aq_qmv, aq_qmv_multi and aq_qmv_gate_up of 2 to 64 rows, see aq_qmv) keep the
+ * partial tiles of a long K in 32 MB of their own that are there from aq_create on: such a call never allocates, and a graph of
+ * it has the bytes of the eager call. */
 typedef struct aq_graph aq_graph;
 int aq_capture_begin(aq_ctx *ctx);
 int aq_capture_end(aq_ctx *ctx, aq_graph **out);
@@ -132,19 +133,24 @@ int aq_probe_read(aq_ctx *ctx, const void *packed, const void *scales, const voi
  * (go/engine/hip/hip_projection_launch.go:1306-1406, 2671-2720, 4907-5287) with the bf16
  * semantics of MLX affine_qmv (go/engine/metal/qmv.go:354-421) and the M-row
  * form (go/engine/metal/qmv_rows.go:14-60).  M >= 1; rows of x are contiguous.
- * N == 0 or K == 0 is a no-op returning AQ_OK (qmv.go:365-371). */
+ * N == 0 or K == 0 is a no-op returning AQ_OK (qmv.go:365-371).
+ * 4- and 8-bit codes, K a multiple of 64 up to 16384, operands 16-byte aligned: up to 32 rows of x, from 9 on in groups of 64
+ * (8 bit: from 2, or 5 where K is 2048, 4096 or 8192), from 5 in groups of 128, from 3 in groups of 32 (8 bit: 2), the
+ * token-tile kernels run the call (small matrices with K no multiple of 256 excepted): one launch, or two where workgroups share
+ * a long K out, and a row of x has the same bytes whatever the number of rows beside it.  33 to 64 rows run there too on
+ * matrices of more than 528 rows that are not too wide, with the same identity among themselves. */
 int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, const void *biases, void *y, int M,
            int K, int N, int group_size, int bits, unsigned flags);
 
-/* `count` (1..4) independent aq_qmv calls that share x, M, K, group size and width, in ONE launch:
+/* `count` (1..4) independent aq_qmv calls that share x, M, K, group size and width, in ONE launch where that pays (below):
  * y[i][M, N[i]] = x . dequant(packed[i], scales[i], biases[i])^T.  The arrays are host arrays of device
  * pointers.  Results are byte-identical to `count` separate aq_qmv calls.  This is the no-copy form of
  * running q|k|v or gate|up over model.ConcatQuantRows (go/model/quant_weight.go:32-62): at batch 1 the
  * narrow projections are bound by launch latency, not bandwidth, and one grid over all of them fills
- * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384), and for
- * the row counts the token-tile kernels run (9..32 rows of 4-bit group-64 codes, 3..32 of group 32, 5..32 of group 128,
- * 2..32 of 8-bit codes) over those members whose own call runs on them; other shapes and members are run as separate
- * launches. */
+ * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384; 8-bit codes:
+ * up to four where every member's own call runs on the diagonal kernels), and for the row counts the token-tile kernels run
+ * (see aq_qmv) over those members whose own call runs on them, with one more launch where a member shares K out; other shapes
+ * and members are run as separate launches. */
 int aq_qmv_multi(aq_ctx *ctx, const void *x, int count, const void *const *packed, const void *const *scales,
                  const void *const *biases, void *const *y, const int *N, int M, int K, int group_size, int bits,
                  unsigned flags);
@@ -175,14 +181,14 @@ int aq_qmm_multi(aq_ctx *ctx, const void *x, int count, const void *const *packe
  * go/engine/hip/hip_projection_launch.go:2671-2720). */
 int aq_reserve_workspace(aq_ctx *ctx, int M, int K);
 /* The same by size.  Besides those the workspace holds: the partial tiles of the few-rows kernels (5..64 rows, up to 64*M*N
- * bytes) and of the matvec kernels of 2..64 rows (up to as much, of a pair twice), those of all members of an aq_qmm_multi call and of both matrices of an aq_qmv_gate_up call, the lists of gathers of
- * more than 64 routes, the intermediates of the unfused
+ * bytes), those of all members of an aq_qmm_multi call and of both matrices of an aq_qmv_gate_up call on the tiles, the
+ * lists of gathers of more than 64 routes, the intermediates of the unfused
  * fallbacks of the fused MLP / lm_head entry points, and the scratch of aq_packed_topk.  A call that needs
  * more than is there grows it (not possible while a capture is open): run such a call once before capturing,
  * or reserve its bytes here. */
 int aq_reserve_workspace_bytes(aq_ctx *ctx, size_t bytes);
 /* Device bytes the context holds as scratch right now (the workspace above, the partial maxima of
- * aq_qmv_greedy, and the block that host-slice calls upload to, of which up to 256 MB stay between calls): lets a caller, or a
+ * aq_qmv_greedy, the partial tiles of the token-tile kernels, and the block that host-slice calls upload to, of which up to 256 MB stay between calls): lets a caller, or a
  * test, see whether a call made any of them grow.  No reference counterpart. */
 size_t aq_workspace_bytes(aq_ctx *ctx);
 
@@ -218,10 +224,11 @@ int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *sc
  * launch go/engine/hip/hip_projection_launch.go:3086-3160, packet contract/launch_abi.hipinc:634-657).
  * gate and up are [N, K*bits/32] with their own scales/biases; for a row-concatenated gate|up slab
  * (model.ConcatQuantRows, go/model/quant_weight.go:32-62) pass the slab for gate and slab + N rows for up.
- * M == 1 with 4/8-bit codes (up to 4 rows of 4-bit group-64 codes when K is a multiple of 256 between 1280 and 8192; up to 32
- * rows where aq_qmv runs its token-tile kernels) runs as ONE launch that reads every weight once; other shapes run the two
- * projections and the element-wise step as separate launches through the context's workspace (which grows
- * on demand like aq_qmm's; not while a capture is open). */
+ * M == 1 with 4/8-bit codes (up to 4 rows of 4-bit group-64 codes when K is a multiple of 256 between 1280 and 8192) runs as ONE
+ * launch that reads every weight once.  So do rows up to 64 where aq_qmv runs its token-tile kernels, from 33 on reading every
+ * weight twice, with a second launch where workgroups share a long K out; and more rows on the tiles of aq_qmm behind a pass
+ * over x.  Other shapes run the two projections and the element-wise step as separate launches through the context's
+ * workspace (which grows on demand like aq_qmm's; not while a capture is open). */
 int aq_qmv_gate_up(aq_ctx *ctx, const void *x, const void *gate_packed, const void *gate_scales,
                    const void *gate_biases, const void *up_packed, const void *up_scales, const void *up_biases,
                    void *y, int M, int K, int N, int group_size, int bits, int act, unsigned flags);

@@ -1,6 +1,7 @@
 // The library's entry points against a HIP runtime of this program's own, which launches nothing and writes down what it is
 // asked: which call of which thread launched which kernel, and what memory was asked for.  So order and scratch can be checked
 // without a GPU.  The definitions here take the place of the runtime's when the program loads libaq_mi355.so.
+#include "aq_kernels.h"
 #include "aq_mi355.h"
 
 #include <dlfcn.h>
@@ -20,6 +21,9 @@
 struct Launch {
     int thread, call;
     std::string kernel;
+    aq::TokArgs tok;  // of the token-tile kernels
+    aq::TokMultiArgs multi;
+    bool is(const char* part) const { return kernel.find(part) != std::string::npos; }
 };
 static std::vector<Launch> log_;
 static std::mutex log_mu;
@@ -62,18 +66,22 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
     *g = grid_, *b = block_, *lds = lds_, *s = stream_;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void**, size_t, hipStream_t) {
+hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void** args, size_t, hipStream_t) {
     std::lock_guard<std::mutex> lk(log_mu);
-    log_.push_back({this_thread, this_call, names()[fn]});
+    Launch l{this_thread, this_call, names()[fn], {}, {}};
+    if (l.is("qmv_tok16_kernel")) l.tok = *static_cast<const aq::TokArgs*>(args[0]);
+    if (l.is("qmv_tok16_multi_kernel")) l.multi = *static_cast<const aq::TokMultiArgs*>(args[0]);
+    log_.push_back(l);
     return hipSuccess;
 }
 hipError_t hipGetDeviceCount(int* n) { return *n = 1, hipSuccess; }
 hipError_t hipGetDevice(int* d) { return *d = 0, hipSuccess; }
 hipError_t hipSetDevice(int) { return hipSuccess; }
+static int compute_units = 256;
 hipError_t hipGetDeviceProperties(hipDeviceProp_t* p, int) {  // (the header's name for the versioned symbol)
     memset(p, 0, sizeof *p);
     strcpy(p->gcnArchName, "gfx950");
-    p->multiProcessorCount = 256;
+    p->multiProcessorCount = compute_units;
     return hipSuccess;
 }
 hipError_t hipDeviceGetAttribute(int* v, hipDeviceAttribute_t, int) { return *v = 256, hipSuccess; }
@@ -178,13 +186,79 @@ static void test_calls_stay_whole() {
     CHECK(several >= 4 * 9, "%d launches behind another of their call", several);
 }
 
-int main() {
-    if (aq_create(0, &ctx) != AQ_OK) {
-        printf("aq_create: %s\n", aq_last_error());
-        return 1;
+// A row of x meets the same sums in a call of 9 rows as in one of 32 (and of 33 as of 64), recorded or not: the shares of K do not
+// depend on the number of rows, and their partial tiles lie in a block that is there from the start, apart from each other.
+static uintptr_t tiles_lo, tiles_hi;
+static void tiles_used(const float* tile, size_t bytes) {
+    const uintptr_t p = reinterpret_cast<uintptr_t>(tile);
+    tiles_lo = p < tiles_lo ? p : tiles_lo;
+    tiles_hi = p + bytes > tiles_hi ? p + bytes : tiles_hi;
+}
+static void test_shares() {
+    int shared = 0, calls = 0;
+    tiles_lo = UINTPTR_MAX, tiles_hi = 0;
+    unsigned seed = 1;
+    auto rnd = [&](int n) { return (int)((seed = seed * 1664525u + 1013904223u) >> 8) % n; };
+    for (int i = 0; i < 1500; i++) {
+        const int bits = i % 3 ? 4 : 8, group = 32 << rnd(3), K = 128 * (1 + rnd(128)), N = 16 + rnd(1 << (4 + rnd(12)));
+        const bool pair = i % 4 == 3;
+        for (int from : {9, 33}) {
+            int ksplit = -1, share = 0;
+            for (int M = from; M <= from + (from == 9 ? 23 : 31); M += 1 + rnd(7)) {
+                log_.clear();
+                capturing = (M + i) % 2;
+                const size_t before = allocated;
+                const int drained = drains;
+                const int rc = pair ? aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, M, K, N, group, bits, AQ_ACT_SILU, 0) : qmv(M, K, N, group, bits);
+                if (log_.empty() || !log_[0].is("qmv_tok16_kernel")) continue;  // (other kernels: they may want scratch, and be refused it)
+                CHECK(rc == AQ_OK && allocated == before && drains == drained, "%d, %zu bytes allocated, the stream drained %d times", rc, allocated - before,
+                      drains - drained);
+                const aq::TokArgs& a = log_[0].tok;
+                calls++;
+                if (ksplit < 0) ksplit = a.ksplit, share = a.share;
+                CHECK(a.ksplit == ksplit && a.share == share, "bits %d group %d K %d N %d pair %d: %d shares from %d rows, %d at %d", bits, group, K, N,
+                      pair, ksplit, from, a.ksplit, M);
+                if (a.ksplit <= 1) continue;
+                shared++;
+                tiles_used(a.tile, (size_t)a.ksplit * M * N * (pair ? 8 : 4));
+                CHECK(log_.size() == 2 && log_[1].is("tok_reduce"), "%zu launches", log_.size());
+            }
+        }
     }
-    test_calls_stay_whole();
-    aq_destroy(ctx);
+    capturing = false;
+    CHECK(calls > 5000 && shared > 1000, "%d calls, %d of them shared K out", calls, shared);
+    for (int i = 0; i < 300; i++) {
+        const int M = 9 + rnd(24), K = 4096 + 256 * rnd(48);
+        const void *w[4] = {W, W, W, W}, *s[4] = {S, S, S, S}, *b[4] = {B, B, B, B};
+        void* y[4] = {Y, Y, Y, Y};
+        const int N[4] = {16 + rnd(4096), 1 + rnd(20000), 16 + rnd(20000), 1 + rnd(4096)};
+        log_.clear();
+        CHECK(aq_qmv_multi(ctx, X, 4, w, s, b, y, N, M, K, 64, 4, 0) == AQ_OK, "%s", aq_last_error());
+        for (const Launch& l : log_) {
+            if (l.is("qmv_tok16_kernel") && l.tok.ksplit > 1) tiles_used(l.tok.tile, (size_t)l.tok.ksplit * M * l.tok.N * 4);
+            uintptr_t end = 0;
+            for (int m = 0; l.is("qmv_tok16_multi") && m < l.multi.count; m++) {
+                if (l.multi.ksplit[m] <= 1) continue;
+                CHECK(reinterpret_cast<uintptr_t>(l.multi.tile[m]) >= end, "member %d overlaps the one before it", m);
+                end = reinterpret_cast<uintptr_t>(l.multi.tile[m]) + (size_t)l.multi.ksplit[m] * M * l.multi.N[m] * 4;
+                tiles_used(l.multi.tile[m], (size_t)l.multi.ksplit[m] * M * l.multi.N[m] * 4);
+            }
+        }
+    }
+    CHECK(tiles_hi - tiles_lo <= aq::kTokTileBytes, "partial tiles over %zu bytes", (size_t)(tiles_hi - tiles_lo));
+}
+
+int main() {
+    for (int cus : {128, 512, 256}) {
+        compute_units = cus;
+        if (aq_create(0, &ctx) != AQ_OK) {
+            printf("aq_create: %s\n", aq_last_error());
+            return 1;
+        }
+        test_shares();
+        if (cus == 256) test_calls_stay_whole();
+        aq_destroy(ctx);
+    }
     if (!failures) puts("ok");
     return failures ? 1 : 0;
 }

@@ -80,33 +80,39 @@ def test_gated_pair(ctx, orc, bits, gs, M, K, N):
         t.free()
 
 
-def test_capture_without_a_workspace():
-    """A call that would share K out is captured on a context that has never run anything: it runs whole, and again after eager
-    calls have made room."""
+@pytest.mark.parametrize("bits,gs,K,N", [(4, 64, 8192, 4096), (4, 64, 4736, 1985), (8, 64, 14336, 700), (4, 32, 15360, 545)])
+def test_a_row_has_the_same_bytes_in_calls_of_9_to_32_rows(bits, gs, K, N):
+    """... and of 33 to 64; eager, and recorded on a context that has never run anything."""
     import aq_mi355
-    M, K, N = 24, 14336, 700
-    say("token tile shares in a graph", M, K, N)
-    words, s, b = F.synthetic_affine(N, K, 4, 64, seed=2490)
-    x = F.synthetic_x(M, K, seed=2491)
-    ref = F.reference_f64(x, words, s, b, 4, 64, K)
+    say("token tiles, rows across row counts", bits, gs, K, N)
+    words, s, b = F.synthetic_affine(N, K, bits, gs, seed=2490)
+    x = F.synthetic_x(64, K, seed=2491)
     fresh = aq_mi355.Context(0)
     try:
-        dw = DeviceAffine(fresh, words, s, b)
-        dx, dy = fresh.to_device(x), fresh.alloc(M * N * 4)
-        call = lambda: fresh.qmv(dx, dw.w, dw.s, dw.b, dy, M, K, N, 64, 4, aq_mi355.AQ_OUT_F32)
-        for _ in range(2):
-            fresh.capture_begin()
-            call()
-            graph = fresh.capture_end()
-            for _ in range(3):
-                fresh.fill_zero(dy)
-                fresh.graph_launch(graph)
-                fresh.sync()
-                check_accumulators(dy.download(np.float32, M * N).copy(), ref, "replay")
-            fresh.graph_destroy(graph)
-            call()
-            fresh.sync()
-            check_accumulators(dy.download(np.float32, M * N).copy(), ref, "eager")
+        dw, dx, dy = DeviceAffine(fresh, words, s, b), fresh.to_device(x), fresh.alloc(64 * N * 4)
+        call = lambda m: fresh.qmv(dx, dw.w, dw.s, dw.b, dy, m, K, N, gs, bits, aq_mi355.AQ_OUT_F32)
+        held = fresh.workspace_bytes()
+        for counts in ((9, 12, 16, 17, 24, 28, 32), (33, 48, 64)):
+            want = None
+            for m in counts:
+                fresh.capture_begin()
+                call(m)
+                graph = fresh.capture_end()
+                assert fresh.last_variant(0).startswith("qmvt_"), fresh.last_variant(0)
+                for replay in range(3):
+                    fresh.fill_zero(dy)
+                    fresh.graph_launch(graph)
+                    fresh.sync()
+                    got = dy.download(np.uint32, m * N).reshape(m, N)
+                    want = got if want is None else want
+                    assert np.array_equal(got[:len(want)], want[:m]), (m, replay)
+                    call(m)
+                    fresh.sync()
+                    assert np.array_equal(dy.download(np.uint32, m * N).reshape(m, N), got), (m, replay)
+                want = got
+                fresh.graph_destroy(graph)
+        assert fresh.workspace_bytes() == held
+        check_accumulators(want.view(np.float32), F.reference_f64(x, words, s, b, bits, gs, K), "64 rows")
         for t in (dw, dx, dy):
             t.free()
     finally:
