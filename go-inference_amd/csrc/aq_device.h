@@ -99,20 +99,10 @@ __device__ __forceinline__ uint4 unpack_word4(uint32_t w, uint32_t mask_s, uint3
     return v;
 }
 
-// Codes centred on zero, for sums that must not lose what the bias takes off again: (code - 8) / 16 of the eight 4-bit codes in
-// the order of unpack4_word, code - 128 of four 8-bit codes.  Both have at most 8 significant bits: exact in bf16.
+// Codes centred on zero, for sums that must not lose what the bias takes off again: code - 128 of four 8-bit codes, which has at
+// most 8 significant bits: exact in bf16.
 __device__ __forceinline__ uint32_t high_halves(float lo, float hi) {
     return __builtin_amdgcn_perm(__float_as_uint(hi), __float_as_uint(lo), 0x07060302u);
-}
-__device__ __forceinline__ void unpack4_centred(uint32_t w, uint32_t p[4]) {
-    w ^= 0x88888888u;  // signed nibbles
-    uint32_t odd = w >> 4;
-    asm("" : "+v"(odd));  // (or eight shifts take the place of the byte selections)
-    auto at = [](uint32_t v, int byte) { return __builtin_amdgcn_cvt_off_f32_i4(byte ? (int)((v >> (8 * byte)) & 0xffu) : (int)v); };
-    p[0] = high_halves(at(w, 0), at(w, 2));
-    p[1] = high_halves(at(odd, 0), at(odd, 2));
-    p[2] = high_halves(at(w, 1), at(w, 3));
-    p[3] = high_halves(at(odd, 1), at(odd, 3));
 }
 __device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
     w ^= 0x80808080u;  // signed bytes
@@ -123,7 +113,7 @@ __device__ __forceinline__ void unpack8_centred(uint32_t w, uint32_t p[2]) {
 
 // Eight 4-bit codes as four bf16 pairs (c0,c2)(c4,c6)(c1,c3)(c5,c7).  The bytes 0 .. 15 read as fp8 (e4m3) are 2^-9 times their
 // own value, subnormals and the first binade having one unit in the last place, so that the packed conversion to bf16 with a
-// scale of 2^9 yields two codes an instruction, exactly: seven instructions a word, against fourteen of unpack4_centred.
+// scale of 2^9 yields two codes an instruction, exactly: seven instructions a word (fourteen by signed-nibble conversions).
 __device__ __forceinline__ void unpack4_codes(uint32_t w, uint32_t p[4]) {
     const uint32_t even = w & 0x0f0f0f0fu, odd = (w >> 4) & 0x0f0f0f0fu;
     p[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(even, 512.0f, false));

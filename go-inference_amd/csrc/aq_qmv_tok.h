@@ -24,7 +24,6 @@ __device__ __forceinline__ gptr_t uniform_ptr(const void* p) {
     return reinterpret_cast<gptr_t>(((uint64_t)hi << 32) | lo);
 }
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint4 load_u128_at(gptr_t base, uint32_t off) {
     const u32x4_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x4_t*>(base + off);
     return make_uint4(v[0], v[1], v[2], v[3]);
@@ -34,10 +33,6 @@ __device__ __forceinline__ uint4 load_u128_at(gptr_t base, uint32_t off) {
 __device__ __forceinline__ uint4 load_u128_stream_at(gptr_t base, uint32_t off) {
     const u32x4_t v = __builtin_nontemporal_load(reinterpret_cast<const __attribute__((address_space(1))) u32x4_t*>(base + off));
     return make_uint4(v[0], v[1], v[2], v[3]);
-}
-__device__ __forceinline__ uint2 load_u64_at(gptr_t base, uint32_t off) {
-    const u32x2_t v = *reinterpret_cast<const __attribute__((address_space(1))) u32x2_t*>(base + off);
-    return make_uint2(v[0], v[1]);
 }
 __device__ __forceinline__ bf16x8_t as_bf16x8(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
     const uint4 v = make_uint4(a, b, c, d);
@@ -56,9 +51,11 @@ typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) u32x2_a2_t;
 // v_mfma_f32_16x16x32_bf16 with 16 tokens as the rows of A (TS such sets per expanded weight: up to 16 TS rows of x) and
 // 16 weight rows as the columns of B.  A workgroup of eight wavefronts owns RS sets of 16 weight rows; wavefront w takes
 // the runs of 256 codes w, w + 8, ... of all of them, one run a pass.
-//   * A load instruction covers whole 128-byte lines of 8 rows; the lines then go through LDS (a wavefront's own 2.3 KiB), out of
-//     which lane (n = lane % 16, q = lane / 16) reads the codes 8 q .. 8 q + 7 of row n for every step of 32 codes.  (Moves and
-//     swaps between lanes instead took 125 clocks of the vector unit per set and run.)
+//   * A load instruction covers whole 128-byte lines of 8 rows.  4 bit: the lines go through LDS (a wavefront's own 2.3 KiB), out
+//     of which lane (n = lane % 16, q = lane / 16) reads the codes 8 q .. 8 q + 7 of row n for every step of 32 codes.  (Moves and
+//     swaps between lanes instead took 125 clocks of the vector unit per set and run.)  8 bit: two DPP moves per register pair
+//     give lane (n, q) the codes 16 q .. 16 q + 15 of a block of 64 of row n, whose halves are its operands of the block's two
+//     steps, x being loaded to match; groups of 32, where a step is a group, swap 32-lane halves besides.
 //   * x is read a whole 128-byte line of each of 8 tokens per instruction: lanes i = lane % 16 < 8 take the first 64
 //     bytes of token i (an even step), lanes i >= 8 the second 64 bytes of token i - 8 (the odd step behind it); a
 //     second instruction does the same for tokens 8..15, and two DPP moves per register pair put the halves where the
@@ -99,20 +96,10 @@ constexpr int kTokRowPitch = 144;  // LDS bytes between the 128-byte lines of a 
 // rows a wavefront reads at once fall into different banks
 __host__ __device__ constexpr int tok_sb_pitch(bool g32, int runs) { return g32 ? 2 * runs + 1 : runs | 1; }
 __host__ __device__ constexpr size_t tok_sb_bytes(bool g32, int rows, int runs) { return (size_t)rows * tok_sb_pitch(g32, runs) * 16; }
-// ... of a wavefront's lines of weights, and its sums of x
-__host__ __device__ constexpr int tok_own_bytes(int ts) { return 16 * kTokRowPitch + ts * 512; }
-
-// Registers s0 .. s3 of the four 16-lane blocks as a 4 x 4 matrix, transposed.
-__device__ __forceinline__ void transpose4(uint32_t& s0, uint32_t& s1, uint32_t& s2, uint32_t& s3) {
-    const auto p = __builtin_amdgcn_permlane16_swap(s0, s1, false, false);
-    const auto r = __builtin_amdgcn_permlane16_swap(s2, s3, false, false);
-    const auto e = __builtin_amdgcn_permlane32_swap(p[0], r[0], false, false);
-    const auto o = __builtin_amdgcn_permlane32_swap(p[1], r[1], false, false);
-    s0 = e[0];
-    s1 = o[0];
-    s2 = e[1];
-    s3 = o[1];
-}
+// ... of a wavefront's lines of weights (4 bit), and its sums of x where a group's sum starts from them
+__host__ __device__ constexpr int tok_line_bytes(int bits) { return bits == 4 ? 16 * kTokRowPitch : 0; }
+__host__ __device__ constexpr bool tok_from_sum(int bits, bool g32) { return bits == 4 && g32; }
+__host__ __device__ constexpr int tok_own_bytes(int bits, bool g32, int ts) { return tok_line_bytes(bits) + (tok_from_sum(bits, g32) ? ts * 512 : 0); }
 
 template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR, bool GROUPED>
 __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block_of_all) {
@@ -121,7 +108,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
     constexpr int NW = kTokWaves;
     constexpr bool G32 = GRP == 32;
     constexpr int GPR = 256 / GRP;  // groups of a run (groups of 128: two, each held twice)
-    constexpr bool FROM_SUM = BITS == 4 && G32;
+    constexpr bool FROM_SUM = tok_from_sum(BITS, G32);
     constexpr float kLacks = BITS == 8 ? 128.0f : G32 ? 8.0f : 0.0f;  // in codes
     static_assert(!PAIR || RS % 2 == 0, "a pair shares its sets of rows between two matrices");
     constexpr int PAIRS = PAIR ? 2 : 1;
@@ -184,10 +171,9 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
     const uint32_t part16 = (uint32_t)(n >> 3) * 64u + (uint32_t)q * 16u;
     const uint32_t w_lane = (uint32_t)(row0 + (n & 7)) * row_bytes, w_last = (uint32_t)(N - 1) * row_bytes;
     // x: lane (i, q) of load `ab` of token set ts reads token 16 ts + (i % 8) + 8 ab, bytes 64 (i / 8) + 16 q of a
-    // 128-byte step pair (TS sets of 16 tokens share every expanded weight); 8-bit codes moved between lanes: a step takes 8 of
-    // the 16 codes that lane block q has of a block of 64, so bytes 32 q + 16 (i / 8)
-    constexpr bool VIA_LDS = BITS == 4;
-    const uint32_t x_part = BITS == 4 || VIA_LDS ? part16 : (uint32_t)q * 32u + (uint32_t)(n >> 3) * 16u;
+    // 128-byte step pair (TS sets of 16 tokens share every expanded weight); 8 bit: a step takes 8 of the 16 codes that lane
+    // block q has of a block of 64, so bytes 32 q + 16 (i / 8)
+    const uint32_t x_part = BITS == 4 ? part16 : (uint32_t)q * 32u + (uint32_t)(n >> 3) * 16u;
     auto x_row = [&](int t) { return GROUPED ? (uint32_t)max(a.route_x[first_route + t], 0) : (uint32_t)t; };
     uint32_t x_lane[TS][2];
 #pragma unroll
@@ -274,8 +260,8 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         if (tid + i * NT < pieces) load_piece(tid + i * NT, sv[i], bv[i]);
     __builtin_amdgcn_sched_barrier(0);
 
-    unsigned char* const w_own = lds_raw + tok_sb_bytes(G32, ROWS, runs) + wave * tok_own_bytes(TS);
-    float* const sums_own = reinterpret_cast<float*>(w_own + 16 * kTokRowPitch);  // groups of 32, 4 bit: [set of tokens][step][token]
+    [[maybe_unused]] unsigned char* const w_own = lds_raw + tok_sb_bytes(G32, ROWS, runs) + wave * tok_own_bytes(BITS, G32, TS);
+    [[maybe_unused]] float* const sums_own = reinterpret_cast<float*>(w_own + tok_line_bytes(BITS));  // [set of tokens][step][token]
 
     // A pass: one run of this wavefront, its A operands in registers, and the RS sets of rows streamed
     // past them one set at a time through a ring of RING register slots.  Loads return in the order they were issued, and
@@ -360,7 +346,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 if constexpr (BITS == 4)  // the order the expansion leaves the codes of a word in: 0 2 4 6 1 3 5 7
                     v = make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
                                    __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
-                if constexpr (BITS == 8 && G32 && !VIA_LDS) {  // (as the codes: the even step's upper lanes against the odd one's lower)
+                if constexpr (BITS == 8 && G32) {  // (as the codes: the even step's upper lanes against the odd one's lower)
                     if ((st & 1) == 0) {
                         held = v;
                         continue;
@@ -406,24 +392,17 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 sbv = sbq[(rs * 16 + n) * sb_pitch + at];
                 bbv = make_uint4(sbv.z, sbv.w, 0u, 0u);
             }
-            // the codes of a line: 4 bit the words of the set's eight steps, 8 bit the two words each of four steps
+            // the codes of a line: 4 bit the words of the set's eight steps, 8 bit the two words of each of four steps
             uint32_t ww[8];
             auto fetch_line = [&](int ln) {
                 const uint4 la = ring[SL][ln][0], lb = ring[SL][ln][1];
-                if constexpr (VIA_LDS) {
+                if constexpr (BITS == 4) {
                     unsigned char* const to = w_own + (n & 7) * kTokRowPitch + part16;
                     *reinterpret_cast<uint4*>(to) = la;
                     *reinterpret_cast<uint4*>(to + 8 * kTokRowPitch) = lb;
                     const unsigned char* const from = w_own + n * kTokRowPitch;
 #pragma unroll
-                    for (int i = 0; i < (BITS == 4 ? 8 : 4); i++) {
-                        if constexpr (BITS == 4) {
-                            ww[i] = *reinterpret_cast<const uint32_t*>(from + i * 16 + q * 4);
-                        } else {
-                            const uint2 v = *reinterpret_cast<const uint2*>(from + i * 32 + q * 8);
-                            ww[2 * i] = v.x, ww[2 * i + 1] = v.y;
-                        }
-                    }
+                    for (int i = 0; i < 8; i++) ww[i] = *reinterpret_cast<const uint32_t*>(from + i * 16 + q * 4);
                 } else {
                     // first 64 bytes of all 16 rows (lanes i >= 8 from the second load's lanes i - 8), second 64 bytes (lanes
                     // i < 8 from the first load's lanes i + 8): as for x
@@ -435,10 +414,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                     ww[5] = __builtin_amdgcn_update_dpp(lb.y, la.y, 0x108, 0xf, 0x3, false);
                     ww[6] = __builtin_amdgcn_update_dpp(lb.z, la.z, 0x108, 0xf, 0x3, false);
                     ww[7] = __builtin_amdgcn_update_dpp(lb.w, la.w, 0x108, 0xf, 0x3, false);
-                    if constexpr (BITS == 4) {
-                        transpose4(ww[0], ww[1], ww[2], ww[3]);
-                        transpose4(ww[4], ww[5], ww[6], ww[7]);
-                    } else if constexpr (G32) {  // a step is one half of a block of 64: the second 8 codes of its lanes move across
+                    if constexpr (G32) {  // a step is one half of a block of 64: the second 8 codes of its lanes move across
 #pragma unroll
                         for (int g = 0; g < 2; g++)
 #pragma unroll

@@ -20,7 +20,7 @@ const QmvVariant* qmvt_variant(int idx) {
 static bool tok_whole_runs(const QmvArgs& a) { return a.gs_shift == 6 && a.K % 256 == 0; }
 static int tok_runs_of(const TokArgs& a) { return a.ksplit > 1 ? a.share : (a.K + 255) / 256; }
 static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs) {
-    const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.ts);
+    const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.v.bits, g32, e.ts);
     const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4;
     return staged > sums ? staged : sums;
 }
