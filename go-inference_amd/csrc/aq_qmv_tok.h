@@ -281,11 +281,25 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 ring[SL][ln][ab] = load_u128_stream_at(PAIR && rs >= RS / 2 ? wg2 : wg, row + in_row);
             }
     };
+    // (A wavefront without a run of its own takes its share of the staging and requests nothing.  When it went through the loop with
+    // the first run's x and weights, unused: 9 / 24 rows of 768 x 1024 3.7 / 5.3 us against 3.3 / 4.2, 24 of 1024 x 2048 5.4
+    // against 4.5, of 1536 x 2048 in groups of 32 7.2 against 6.5.  A condition around the loop's loads instead of a loop that is
+    // not entered: the kernels of eight sets and two sets of tokens spill, 32 rows of 15360 x 3840 24.9 -> 50.7.)
     bool staged = false;
-    // (a wavefront without a run of its own goes through the loop once as well, to take its share of the staging)
-    for (int at = wave; at < runs || at == wave; at += NW) {
-        const bool live = at < runs;
-        const int run = qfirst + (live ? at : 0);
+    auto stage = [&]() {
+#pragma unroll
+        for (int i = 0; i < PRE; i++)
+            if (tid + i * NT < pieces) store_piece(tid + i * NT, sv[i], bv[i]);
+        for (int p = tid + PRE * NT; p < pieces; p += NT) {
+            uint4 s, b;
+            load_piece(p, s, b);
+            store_piece(p, s, b);
+        }
+        __syncthreads();
+        staged = true;
+    };
+    for (int at = wave; at < runs; at += NW) {
+        const int run = qfirst + at;
         uint4 xa[TS][4], xb[TS][4];
 #pragma unroll
         for (int ts = 0; ts < TS; ts++)
@@ -299,19 +313,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         issue_set(std::integral_constant<int, 0>{}, run);
         if constexpr (RING > 1 && RS > 1) issue_set(std::integral_constant<int, 1>{}, run);
         __builtin_amdgcn_sched_barrier(0);
-        if (!staged) {
-#pragma unroll
-            for (int i = 0; i < PRE; i++)
-                if (tid + i * NT < pieces) store_piece(tid + i * NT, sv[i], bv[i]);
-            for (int p = tid + PRE * NT; p < pieces; p += NT) {
-                uint4 s, b;
-                load_piece(p, s, b);
-                store_piece(p, s, b);
-            }
-            __syncthreads();
-            staged = true;
-        }
-        if (!live) break;
+        if (!staged) stage();
 
         // A operands of the run, and the three-way split of the lane block's group sum of x
         bf16x8_t af[TS][8], a2[TS][GPR / 4];
@@ -496,6 +498,8 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         if constexpr (RS > 7) run_set(std::integral_constant<int, 7>{});
         static_assert(RS <= 8 && RS % RING == 0, "sets of rows per workgroup");
     }
+
+    if (!staged) stage();  // a wavefront without a run of its own
 
     // ---- the wavefronts' partial sums meet in LDS, in the scales' place: red[wave][token][row]; thread (token, row) adds them in
     // wave order ----
