@@ -175,11 +175,13 @@ struct TokArgs : QmvArgs {
     int ksplit, share;  // shares of K (0, 1: none), 256-code runs per share
     float* tile;        // the fp32 partial tiles
     int tokens;         // rows of x per workgroup
+    uint32_t red_at;    // filled by the launcher: where in LDS the wavefronts' sums meet
 };
 struct TokMultiArgs : QmvMultiArgs {
     int ksplit[kQmvMultiMax], share[kQmvMultiMax];
     float* tile[kQmvMultiMax];
     int tokens;
+    uint32_t red_at;
 };
 int qmvt_variant_count();
 const QmvVariant* qmvt_variant(int idx);
@@ -206,7 +208,7 @@ hipError_t qmvt_pair_launch(int idx, const TokArgs& a, hipStream_t stream);
 // Expert slabs with the routes grouped by expert (a.chunks, a.route_x, a.route_of; chunks of up to `tokens` = 16 or 32
 // routes; most_chunks entries in the list); pair as above.
 bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair);
-hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const TokArgs& a, hipStream_t stream);
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, TokArgs a, hipStream_t stream);
 // Partial tiles [ksplit][M][N] ([ksplit][M][gate N | up N]) added in order, the activation applied for a pair, and dense groups
 // of 32 that are not finite formed again (plain_dot_g32).  Matrices with tile null are left alone.
 struct TokReduceArgs {

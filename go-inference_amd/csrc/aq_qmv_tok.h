@@ -501,10 +501,10 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
 
     if (!staged) stage();  // a wavefront without a run of its own
 
-    // ---- the wavefronts' partial sums meet in LDS, in the scales' place: red[wave][token][row]; thread (token, row) adds them in
-    // wave order ----
-    float* red = reinterpret_cast<float*>(lds_raw);
-    __syncthreads();
+    // ---- the wavefronts' partial sums meet in LDS: red[wave][token][row]; thread (token, row) adds them in wave order.  Behind
+    // what is staged, so that a wavefront need not wait before it puts its own there, or in its place (tok_lds_bytes) ----
+    float* red = reinterpret_cast<float*>(lds_raw + a.red_at);
+    if (a.red_at == 0) __syncthreads();
     // D layout of the 16x16 MFMA: lane (n, q), register r -> token 4 q + r (of its set), weight row n
 #pragma unroll
     for (int rs = 0; rs < RS; rs++)
@@ -579,6 +579,7 @@ __global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_multi_kernel(const
     a.ksplit = ma.ksplit[i];
     a.share = ma.share[i];
     a.tile = ma.tile[i];
+    a.red_at = ma.red_at;
     qmv_tok16_body<BITS, RS, RING, TS, GRP, false, false>(a, (int)blockIdx.x - before);
 }
 

@@ -19,10 +19,16 @@ const QmvVariant* qmvt_variant(int idx) {
 
 static bool tok_whole_runs(const QmvArgs& a) { return a.gs_shift == 6 && a.K % 256 == 0; }
 static int tok_runs_of(const TokArgs& a) { return a.ksplit > 1 ? a.share : (a.K + 255) / 256; }
-static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs) {
+// LDS of a workgroup whose longest share is `runs` runs.  The wavefronts' sums meet behind what is staged (red_at) where that costs no
+// workgroup of a CU, else in its place, behind a barrier (us, in its place / behind: 4 / 16 / 32 rows of 4096 x 14336, 8 bit 14.6 /
+// 16.3 / 20.2 against 14.4 / 16.1 / 19.9, 4 bit 16 / 32 rows 11.6 / 16.3 against 11.5 / 16.1).
+static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs, uint32_t* red_at = nullptr) {
     const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.v.bits, g32, e.ts);
-    const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4;
-    return staged > sums ? staged : sums;
+    const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4, cu = 160 * 1024;
+    const int of_a_cu = e.v.rows * e.ts <= 2 ? 2 : 1;  // workgroups that a CU's registers hold
+    const bool behind = staged + sums <= cu / of_a_cu;
+    if (red_at) *red_at = behind ? (uint32_t)staged : 0;
+    return behind ? staged + sums : staged > sums ? staged : sums;
 }
 
 bool qmvt_fits(const TokArgs& a, int bits, int group_size, int idx, bool exact_only) {
@@ -77,7 +83,7 @@ static hipError_t tok_launch(int idx, TokArgs a, bool pair, hipStream_t stream) 
     if (a.tokens < 1) a.tokens = a.M;
     const bool g32 = a.gs_shift == 5;
     const QmvTokKernel fn = pair ? e.pair[g32] : e.fn[g32];
-    const size_t lds = tok_lds_bytes(e, g32, tok_runs_of(a));
+    const size_t lds = tok_lds_bytes(e, g32, tok_runs_of(a), &a.red_at);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     hipLaunchKernelGGL(fn, dim3((unsigned)tok_blocks(e, a.M, a.tokens, a.N, pair, a.ksplit)), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
     if (hipError_t rc = hipGetLastError()) return rc;
@@ -116,7 +122,7 @@ hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t str
         r.ksplit[i] = ma.ksplit[i];
         r.tile[i] = ma.ksplit[i] > 1 ? ma.tile[i] : nullptr;
     }
-    const size_t lds = tok_lds_bytes(e, g32, runs);
+    const size_t lds = tok_lds_bytes(e, g32, runs, &ma.red_at);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, ma);
     if (hipError_t rc = hipGetLastError()) return rc;
@@ -144,13 +150,13 @@ bool qmvt_grouped_fits(const QmvArgs& a, int bits, int group_size, bool pair) {
     return tok_lds_bytes(tok_entry(1), group_size == 32, (a.K + 255) / 256) <= 160 * 1024;
 }
 
-hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, const TokArgs& a, hipStream_t stream) {
+hipError_t qmvt_grouped_launch(int bits, int tokens, bool pair, int most_chunks, TokArgs a, hipStream_t stream) {
     const int idx = (bits == 8 ? kTokPerWidth : 0) + (tokens == 32 ? 5 : 1);  // (four sets of rows: the second of a token count)
     const QmvTokEntry& e = tok_entry(idx);
     const bool g32 = a.gs_shift == 5;
     const QmvTokKernel fn = e.grouped[g32][pair ? 1 : 0];
     if (!fn || e.v.m != tokens) return hipErrorInvalidValue;
-    const size_t lds = tok_lds_bytes(e, g32, (a.K + 255) / 256);
+    const size_t lds = tok_lds_bytes(e, g32, (a.K + 255) / 256, &a.red_at);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     const int outs = e.wg_rows / (pair ? 2 : 1);
     hipLaunchKernelGGL(fn, dim3((unsigned)((a.N + outs - 1) / outs), (unsigned)most_chunks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, a);
