@@ -395,8 +395,14 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 bbv = make_uint4(sbv.z, sbv.w, 0u, 0u);
             }
             // the codes of a line: 4 bit the words of the set's eight steps, 8 bit the two words of each of four steps
-            uint32_t ww[8];
+            // (8 bit, two sets of tokens, in groups of 32 or with eight sets of rows: both lines at once, so that the next set is
+            // requested before the first product; us, line by line / at once: 32 rows of 4096 x 14336 in groups of 32 22.0 / 21.7, of
+            // 2560 x (10240 | 10240) 24.0 / 22.2, of 14336 x 4096 22.0 / 21.2; but 32 rows of 4096 x 14336 in groups of 64 20.0 / 20.6,
+            // and one set of tokens, 4 rows, 14.6 / 15.3)
+            constexpr int HELD = TS == 2 && (G32 || RS == 8) ? LINES : 1;
+            uint32_t ww[8 * HELD];
             auto fetch_line = [&](int ln) {
+                const int w0 = ln % HELD * 8;
                 const uint4 la = ring[SL][ln][0], lb = ring[SL][ln][1];
                 if constexpr (BITS == 4) {
                     unsigned char* const to = w_own + (n & 7) * kTokRowPitch + part16;
@@ -408,22 +414,22 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 } else {
                     // first 64 bytes of all 16 rows (lanes i >= 8 from the second load's lanes i - 8), second 64 bytes (lanes
                     // i < 8 from the first load's lanes i + 8): as for x
-                    ww[0] = __builtin_amdgcn_update_dpp(la.x, lb.x, 0x118, 0xf, 0xc, false);
-                    ww[1] = __builtin_amdgcn_update_dpp(la.y, lb.y, 0x118, 0xf, 0xc, false);
-                    ww[2] = __builtin_amdgcn_update_dpp(la.z, lb.z, 0x118, 0xf, 0xc, false);
-                    ww[3] = __builtin_amdgcn_update_dpp(la.w, lb.w, 0x118, 0xf, 0xc, false);
-                    ww[4] = __builtin_amdgcn_update_dpp(lb.x, la.x, 0x108, 0xf, 0x3, false);
-                    ww[5] = __builtin_amdgcn_update_dpp(lb.y, la.y, 0x108, 0xf, 0x3, false);
-                    ww[6] = __builtin_amdgcn_update_dpp(lb.z, la.z, 0x108, 0xf, 0x3, false);
-                    ww[7] = __builtin_amdgcn_update_dpp(lb.w, la.w, 0x108, 0xf, 0x3, false);
+                    ww[w0] = __builtin_amdgcn_update_dpp(la.x, lb.x, 0x118, 0xf, 0xc, false);
+                    ww[w0 + 1] = __builtin_amdgcn_update_dpp(la.y, lb.y, 0x118, 0xf, 0xc, false);
+                    ww[w0 + 2] = __builtin_amdgcn_update_dpp(la.z, lb.z, 0x118, 0xf, 0xc, false);
+                    ww[w0 + 3] = __builtin_amdgcn_update_dpp(la.w, lb.w, 0x118, 0xf, 0xc, false);
+                    ww[w0 + 4] = __builtin_amdgcn_update_dpp(lb.x, la.x, 0x108, 0xf, 0x3, false);
+                    ww[w0 + 5] = __builtin_amdgcn_update_dpp(lb.y, la.y, 0x108, 0xf, 0x3, false);
+                    ww[w0 + 6] = __builtin_amdgcn_update_dpp(lb.z, la.z, 0x108, 0xf, 0x3, false);
+                    ww[w0 + 7] = __builtin_amdgcn_update_dpp(lb.w, la.w, 0x108, 0xf, 0x3, false);
                     if constexpr (G32) {  // a step is one half of a block of 64: the second 8 codes of its lanes move across
 #pragma unroll
                         for (int g = 0; g < 2; g++)
 #pragma unroll
                             for (int k = 0; k < 2; k++) {
-                                const auto p = __builtin_amdgcn_permlane32_swap(ww[4 * g + k], ww[4 * g + 2 + k], false, false);
-                                ww[4 * g + k] = p[0];
-                                ww[4 * g + 2 + k] = p[1];
+                                const auto p = __builtin_amdgcn_permlane32_swap(ww[w0 + 4 * g + k], ww[w0 + 4 * g + 2 + k], false, false);
+                                ww[w0 + 4 * g + k] = p[0];
+                                ww[w0 + 4 * g + 2 + k] = p[1];
                             }
                     }
                 }
@@ -438,13 +444,16 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
             for (int ts = 0; ts < TS; ts++) part[ts] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
             auto step = [&](auto st_tag) {
                 constexpr int st = decltype(st_tag)::value;
-                if constexpr (st % (8 / LINES) == 0) fetch_line(st / (8 / LINES));
+                if constexpr (st % (8 * HELD / LINES) == 0)
+#pragma unroll
+                    for (int ln = st * LINES / 8; ln < st * LINES / 8 + HELD; ln++) fetch_line(ln);
                 uint32_t e[4];
                 if constexpr (BITS == 4) {
                     unpack4_codes(ww[st], e);
                 } else {
-                    unpack8_centred(ww[2 * (st & 3)], e);
-                    unpack8_centred(ww[2 * (st & 3) + 1], e + 2);
+                    constexpr int w0 = 2 * (st % (4 * HELD));
+                    unpack8_centred(ww[w0], e);
+                    unpack8_centred(ww[w0 + 1], e + 2);
                 }
                 const bf16x8_t bop = as_bf16x8(e[0], e[1], e[2], e[3]);
                 constexpr int g = st / (8 / GPR);
