@@ -14,6 +14,14 @@ typedef __attribute__((ext_vector_type(16))) float f32x16_t;
 
 constexpr int kWave = 64;
 
+// What the lanes of a wavefront have written to LDS is there for its other lanes, and what they have read may be written over.  The
+// LDS operations of one wavefront complete in the order they were issued: this keeps the compiler from issuing them in another.
+__device__ __forceinline__ void order_wave_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+}
+
 // bf16 -> f32 is a 16-bit left shift (go/model/quant/mlxaffine/mlxaffine.go:239-241).
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h) { return __uint_as_float(h << 16); }
 

@@ -316,6 +316,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         if (!staged) stage();
 
         // A operands of the run, and the three-way split of the lane block's group sum of x
+        if constexpr (FROM_SUM) order_wave_lds();  // (the sums of the last run have been read)
         bf16x8_t af[TS][8], a2[TS][GPR / 4];
         const uint32_t one2 = 0x3f803f80u;
         const bf16x8_t ones = as_bf16x8(one2, one2, one2, one2);
@@ -406,8 +407,10 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 const uint4 la = ring[SL][ln][0], lb = ring[SL][ln][1];
                 if constexpr (BITS == 4) {
                     unsigned char* const to = w_own + (n & 7) * kTokRowPitch + part16;
+                    order_wave_lds();  // (the last set's words have been read)
                     *reinterpret_cast<uint4*>(to) = la;
                     *reinterpret_cast<uint4*>(to + 8 * kTokRowPitch) = lb;
+                    order_wave_lds();  // the lines, and the sums above, are there for other lanes to read
                     const unsigned char* const from = w_own + n * kTokRowPitch;
 #pragma unroll
                     for (int i = 0; i < 8; i++) ww[i] = *reinterpret_cast<const uint32_t*>(from + i * 16 + q * 4);
