@@ -901,7 +901,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
                 const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
                 for (int i = 0; i < count; i++) fits = fits && aq::qmvd_fits(multi_member(ma, i), bits, group_size, false, di);
                 if (fits) {
-                    ctx->last_variant[0] = bits == 4 ? "qmv_multi_diag" : aq::qmvd_variant(di)->name;
+                    ctx->last_variant[0] = bits == 4 ? "qmv_multi_diag" : "qmv8_multi_diag";
                     AQ_HIP(aq::qmvd_multi_launch(di, ma, ctx->stream), "hipLaunchKernel");
                     return AQ_OK;
                 }
@@ -910,7 +910,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             const int rows = idx >= 0 ? aq::qmv_variant(idx)->rows : 0;
             if (rows > 0 && aq::qmv_multi_supported(bits, 1, rows)) {
                 const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, 1, K, group_size, flags);
-                ctx->last_variant[0] = bits == 4 ? "qmv_multi_dot2" : aq::qmv_variant(idx)->name;
+                ctx->last_variant[0] = bits == 4 ? "qmv_multi_dot2" : "qmv8_multi_dot2";
                 AQ_HIP(aq::qmv_multi_launch(bits, 1, rows, ma, ctx->stream), "hipLaunchKernel");
                 return AQ_OK;
             }

@@ -28,6 +28,14 @@ def test_members_have_the_bytes_of_their_own_calls(ctx, M, gs, Ns, K, offset):
     one, ys = ctx.alloc(M * max(Ns) * 4), [ctx.alloc(M * n * 4) for n in Ns]
     ctx.qmv_multi(x, [m[0] for m in mats], [m[1] for m in mats], [m[2] for m in mats], ys, list(Ns), M, K, gs, 8, aq_mi355.AQ_OUT_F32)
     ctx.sync()
+    diag = [gs == 64 and n * K <= 40 << 20 and (K in (4096, 8192) or (K == 2048 and M <= 2)) for n in Ns]
+    name = ctx.last_variant(0)
+    if all(diag) and offset == 0:
+        assert name == "qmv8_multi_diag", name
+    elif M == 1 and not any(diag):
+        assert name == "qmv8_multi_dot2", name
+    else:  # in the token tiles' grid, or apart
+        assert not name.startswith("qmv8_multi"), name
     for n, m, y in zip(Ns, mats, ys):
         ctx.qmv(x, m[0], m[1], m[2], one, M, K, n, gs, 8, aq_mi355.AQ_OUT_F32)
         ctx.sync()
