@@ -9,6 +9,7 @@
 #include <pthread.h>
 #include <unistd.h>
 
+#include <array>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -248,6 +249,30 @@ static void test_shares() {
     CHECK(tiles_hi - tiles_lo <= aq::kTokTileBytes, "partial tiles over %zu bytes", (size_t)(tiles_hi - tiles_lo));
 }
 
+// The calls that tests/test_gpu_group32_infinities.py makes for the launch that adds partial tiles.
+static void test_shares_of_the_infinities() {
+    auto tiles = [](int i) { return i < (int)log_.size() && log_[i].is("tok_reduce"); };
+    for (int bits : {4, 8}) {
+        for (auto [M, K, N] : {std::array{21, 15360, 100}, {21, 15360, 101}, {40, 15360, 600}, {63, 15360, 545}}) {
+            log_.clear();
+            CHECK(qmv(M, K, N, 32, bits) == AQ_OK && tiles(1), "%d bit, %d x %d x %d", bits, M, K, N);
+            if (M == 63) continue;
+            log_.clear();
+            CHECK(aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, M, K, N, 32, bits, AQ_ACT_SILU, 0) == AQ_OK && tiles(1), "gate|up, %d bit, %d x %d x %d",
+                  bits, M, K, N);
+        }
+        for (auto [M, K, wide] : {std::array{21, 5120, 12000}, {40, 5120, 6000}}) {
+            const void *w[2] = {W, W}, *s[2] = {S, S}, *b[2] = {B, B};
+            void* y[2] = {Y, Y};
+            const int N[2] = {wide, M == 21 ? 100 : 600};
+            log_.clear();
+            CHECK(aq_qmv_multi(ctx, X, 2, w, s, b, y, N, M, K, 32, bits, 0) == AQ_OK && tiles(1), "members, %d bit, %d x %d", bits, M, K);
+            CHECK(log_[0].multi.count == 2 && log_[0].multi.ksplit[0] == 1 && log_[0].multi.ksplit[1] > 1, "members, %d bit, %d x %d: %d and %d shares", bits,
+                  M, K, log_[0].multi.ksplit[0], log_[0].multi.ksplit[1]);
+        }
+    }
+}
+
 int main() {
     for (int cus : {128, 512, 256}) {
         compute_units = cus;
@@ -256,7 +281,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole();
+        if (cus == 256) test_calls_stay_whole(), test_shares_of_the_infinities();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");

@@ -119,6 +119,38 @@ def test_a_row_has_the_same_bytes_in_calls_of_9_to_32_rows(bits, gs, K, N):
         fresh.close()
 
 
+def test_capture_without_a_workspace():
+    """A call that shares K out is captured on a context that has never run anything, and again after eager calls."""
+    import aq_mi355
+    M, K, N = 24, 14336, 700
+    say("token tile shares in a graph", M, K, N)
+    words, s, b = F.synthetic_affine(N, K, 4, 64, seed=2490)
+    x = F.synthetic_x(M, K, seed=2491)
+    ref = F.reference_f64(x, words, s, b, 4, 64, K)
+    fresh = aq_mi355.Context(0)
+    try:
+        dw = DeviceAffine(fresh, words, s, b)
+        dx, dy = fresh.to_device(x), fresh.alloc(M * N * 4)
+        call = lambda: fresh.qmv(dx, dw.w, dw.s, dw.b, dy, M, K, N, 64, 4, aq_mi355.AQ_OUT_F32)
+        for _ in range(2):
+            fresh.capture_begin()
+            call()
+            graph = fresh.capture_end()
+            for _ in range(3):
+                fresh.fill_zero(dy)
+                fresh.graph_launch(graph)
+                fresh.sync()
+                check_accumulators(dy.download(np.float32, M * N).copy(), ref, "replay")
+            fresh.graph_destroy(graph)
+            call()
+            fresh.sync()
+            check_accumulators(dy.download(np.float32, M * N).copy(), ref, "eager")
+        for t in (dw, dx, dy):
+            t.free()
+    finally:
+        fresh.close()
+
+
 @pytest.mark.parametrize("reserve", [0, 1 << 20])
 def test_members_apart_move_the_workspace(reserve):
     """A member that runs by itself, ahead of the grid, needs more workspace than the grid's partial tiles."""
