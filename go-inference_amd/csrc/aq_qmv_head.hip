@@ -337,9 +337,9 @@ constexpr int kTopKListMax = 2 * kTopKMax;             // entries a list holds
 static_assert(kTopKMax <= kTopKSegment / 16 && kTopKThresholdSegments <= 1024 && 64 + 4 + 1 <= 2 * kTopKHeader && 2 * kTopKHeader <= 256, "tickets");
 static_assert(kTopKMax <= kWave, "at least top_k lanes hold a maximum");
 
-// A t that at least top_k of the keys (SV a lane, zero where there is none) reach and no more than a multiple of
-// 2^kTopKThresholdShift below the largest such: built bit by bit from the top, every count one ballot.  The smallest of the
-// lanes' maxima is reached by 64 of them, so the bits that it shares with the largest are t's.
+// A t that at least top_k of the keys (SV a lane, zero where there is none) reach, and few more unless it is the largest such: built
+// bit by bit from the top, every count one ballot.  The smallest of the lanes' maxima is reached by 64 of them, so the bits that
+// it shares with the largest are t's.  The last bits are only asked for where the scores agree in the others.
 constexpr int kTopKThresholdShift = 12;
 
 template <int SV>
@@ -350,13 +350,18 @@ __device__ __forceinline__ uint32_t topk_threshold_key(const uint32_t (&key)[SV]
     const uint32_t most = wave_max_u32(m), least = ~wave_max_u32(~m);
     const int shared = most == least ? 32 : __builtin_clz(most ^ least);  // leading bits
     uint32_t t = shared == 0 ? 0u : most & (0xffffffffu << (32 - shared));
-    for (int bit = 31 - shared; bit >= kTopKThresholdShift; bit--) {
+    int reached = SV * kWave;  // (or more than anyone asks for, where t is what all of them share)
+    auto try_bit = [&](int bit) {
         const uint32_t trial = t | (1u << bit);
         int reach = 0;
 #pragma unroll
         for (int j = 0; j < SV; j++) reach += __popcll(__ballot(key[j] >= trial));
-        if (reach >= top_k) t = trial;
-    }
+        if (reach >= top_k) t = trial, reached = reach;
+    };
+    int bit = 31 - shared;
+    for (; bit >= kTopKThresholdShift; bit--) try_bit(bit);
+    if (__builtin_expect(t != 0 && reached > max(top_k + 8, 48), 0))
+        for (; bit >= 0; bit--) try_bit(bit);
     return t;
 }
 

@@ -24,3 +24,20 @@ def test_lists(ctx, count, top_k, planted):
     assert np.array_equal(_u64(dout, top_k), np.sort(packed)[::-1][:top_k])
     din.free()
     dout.free()
+
+
+@pytest.mark.parametrize("count,top_k", [(6000, 40), (6000, 64), (64 * 1024, 1), (64 * 4096 + 1, 64)])
+@pytest.mark.parametrize("step", [1, 1 << 9, 1 << 14])
+def test_scores_that_agree_in_their_high_bits(ctx, count, top_k, step):
+    """... and differ in the last ones, or are a few values many times over."""
+    say("packed topk, close scores", count, top_k, step)
+    rng = np.random.default_rng(count + top_k + step)
+    near = (np.float32(1000) + rng.standard_normal(count).astype(np.float32) * np.float32(0.3)).view(np.uint32)
+    key = near // np.uint32(step) * np.uint32(step) | np.uint32(0x80000000)
+    packed = (key.astype(np.uint64) << np.uint64(32)) | np.arange(count, dtype=np.uint64)
+    din, dout = ctx.to_device(packed), ctx.to_device(np.full(top_k, 0xDEADBEEF, np.uint64))
+    ctx.packed_topk(din, count, top_k, dout)
+    ctx.sync()
+    assert np.array_equal(_u64(dout, top_k), np.sort(packed)[::-1][:top_k])
+    din.free()
+    dout.free()
