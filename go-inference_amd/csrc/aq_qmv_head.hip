@@ -189,7 +189,12 @@ __global__ __launch_bounds__(256) void pack_scores_kernel(const float* __restric
 // that launch: 128201 scores took it 18 us).  Whole greedy calls: 6 rows (128201 x 1152) 60.8 -> 29.6 us, 8 (164024 x 2048)
 // 108.8 -> 54.7, 15 (91522 x 2048, 8 bit) 105.8 -> 65.3, 3 (36934 x 1536) 30.6 -> 27.0.
 constexpr int kBestGroups = 32, kBestOneGroup = 16384;
-template <bool ONE>
+// Suppressed tokens are bits of the workgroup's own scores, put down while the first scores are on their way.  (With the list looked
+// through for every score that was a thread's largest so far, 2 x 16384 scores took 15.4 us with 3 entries, 70 with 40 and 453 with
+// 300, beside 11 without a list; as bits 12.1, 12.3 and 12.5.)  Only rows of more than kBestBitsScores go through the list.
+constexpr int kBestBitsScores = kBestOneGroup * kBestGroups;
+enum { kNoList, kListAsBits, kListInMemory };
+template <bool ONE, int LIST>
 __global__ __launch_bounds__(ONE ? 1024 : 256) void best_score_kernel(const float* __restrict__ scores, int N, const int32_t* suppress,
                                                                      int suppress_count, unsigned long long* best) {
     constexpr int NT = ONE ? 1024 : 256, AHEAD = 8;
@@ -197,17 +202,42 @@ __global__ __launch_bounds__(ONE ? 1024 : 256) void best_score_kernel(const floa
     const float* const row = scores + (int64_t)m * N;
     unsigned long long mine = 0;
     const int stride = (int)gridDim.x * NT;
-    for (int64_t n0 = (int64_t)blockIdx.x * NT + threadIdx.x; n0 < N; n0 += (int64_t)stride * AHEAD) {
-        float v[AHEAD];
+    float v[AHEAD];
+    auto fetch = [&](int64_t n0) {
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) v[i] = row[min(n0 + (int64_t)i * stride, (int64_t)N - 1)];
+    };
+    const int64_t first = (int64_t)blockIdx.x * NT + threadIdx.x;
+    fetch(first);
+    // bit: round * NT + thread, kBestOneGroup of them at the most
+    __shared__ uint32_t gone[LIST == kListAsBits ? kBestOneGroup / 32 : 1];
+    if constexpr (LIST == kListAsBits) {
+        for (int i = threadIdx.x; i < kBestOneGroup / 32; i += NT) gone[i] = 0;
+        __syncthreads();
+        for (int i = threadIdx.x; i < suppress_count; i += NT) {
+            const int s = suppress[i];
+            if (s < 0 || s >= N) continue;
+            const int round = s / stride, thread = s - round * stride - (int)blockIdx.x * NT;
+            if (thread < 0 || thread >= NT) continue;
+            const int bit = round * NT + thread;
+            atomicOr(&gone[bit >> 5], 1u << (bit & 31));
+        }
+        __syncthreads();
+    }
+    int bit = threadIdx.x;
+    for (int64_t n0 = first; n0 < N; n0 += (int64_t)stride * AHEAD, bit += NT * AHEAD) {
+        uint32_t word[AHEAD] = {};
+        if constexpr (LIST == kListAsBits)
+#pragma unroll
+            for (int i = 0; i < AHEAD; i++) word[i] = gone[min(bit + i * NT, kBestOneGroup - 1) >> 5];
 #pragma unroll
         for (int i = 0; i < AHEAD; i++) {
             const int64_t n = n0 + (int64_t)i * stride;
-            if (n >= N || !isfinite(v[i])) continue;
+            if (n >= N || !isfinite(v[i]) || (word[i] >> (bit & 31) & 1u)) continue;
             const unsigned long long p = pack_score_index(v[i], (uint32_t)n);
-            if (p > mine && !token_suppressed((uint32_t)n, suppress, suppress_count)) mine = p;
+            if (p > mine && (LIST != kListInMemory || !token_suppressed((uint32_t)n, suppress, suppress_count))) mine = p;
         }
+        if (n0 + (int64_t)stride * AHEAD < N) fetch(n0 + (int64_t)stride * AHEAD);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -240,11 +270,13 @@ bool best_score_clears(int N) { return N > 0 && N <= kBestOneGroup; }
 hipError_t best_score_launch(const float* scores, int M, int N, const int32_t* suppress, int suppress_count, unsigned long long* best,
                              hipStream_t stream) {
     if (M <= 0 || N <= 0) return hipSuccess;
-    if (best_score_clears(N))
-        hipLaunchKernelGGL(best_score_kernel<true>, dim3(1, (unsigned)M), dim3(1024), 0, stream, scores, N, suppress, suppress_count, best);
-    else
-        hipLaunchKernelGGL(best_score_kernel<false>, dim3((unsigned)min(kBestGroups, (N + 2047) / 2048), (unsigned)M), dim3(256), 0, stream, scores, N, suppress,
-                           suppress_count, best);
+    typedef void (*BestKernel)(const float*, int, const int32_t*, int, unsigned long long*);
+    static const BestKernel kBest[2][3] = {{best_score_kernel<false, kNoList>, best_score_kernel<false, kListAsBits>, best_score_kernel<false, kListInMemory>},
+                                           {best_score_kernel<true, kNoList>, best_score_kernel<true, kListAsBits>, nullptr}};
+    const bool one = best_score_clears(N);
+    const int list = suppress_count == 0 ? kNoList : N <= kBestBitsScores ? kListAsBits : kListInMemory;
+    hipLaunchKernelGGL(kBest[one][list], dim3(one ? 1u : (unsigned)min(kBestGroups, (N + 2047) / 2048), (unsigned)M), dim3(one ? 1024 : 256), 0, stream,
+                       scores, N, suppress, suppress_count, best);
     return hipGetLastError();
 }
 

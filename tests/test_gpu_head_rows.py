@@ -27,3 +27,19 @@ def test_best_of_every_row(ctx, M, N):
     packed = _scores(ctx, x, dw, M, K, N, gs, bits, winners)
     assert np.array_equal(_greedy(ctx, x, dw, M, K, N, gs, bits, winners), packed.max(axis=1))
     dw.free()
+
+
+# one workgroup a row and several with the list as bits, its longest row, and the first that goes through the list
+@pytest.mark.parametrize("M,N,count", [(2, 16384, 300), (3, 16385, 1100), (1, 524288, 70), (2, 524288, 70), (2, 524289, 70)])
+def test_best_behind_a_long_list(ctx, M, N, count):
+    say("greedy rows, suppressed", M, N, count)
+    K, gs, bits = 64, 64, 4
+    words, s, b = F.synthetic_affine(N, K, bits, gs, seed=F.BASE_SEED + 112)
+    x = F.synthetic_x(M, K, seed=F.BASE_SEED + 113)
+    dw = DeviceAffine(ctx, words, s, b)
+    packed = _scores(ctx, x, dw, M, K, N, gs, bits)
+    gone = np.unique(np.concatenate([np.argsort(p)[::-1][:count] for p in packed] + [[0, N - 1]]))
+    listed = list(map(int, gone)) + [-1, N, N + 5, int(gone[0])]   # tokens that there are not, one twice
+    packed[:, gone] = 0
+    assert np.array_equal(_greedy(ctx, x, dw, M, K, N, gs, bits, listed), packed.max(axis=1))
+    dw.free()
