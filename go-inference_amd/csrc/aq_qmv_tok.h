@@ -126,7 +126,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
     int block = block_of_all, split = 0, M = a.M, m0 = 0;
     if constexpr (!GROUPED) {
         const int bands = (N + OUTS - 1) / OUTS;
-        if (M > a.tokens) {
+        if (__builtin_expect(M > a.tokens, 0)) {
             // more rows of x than a workgroup takes: eight bands for the first of them, then the same eight for the next, so that
             // the workgroups of a band run side by side on one XCD (every eighth workgroup) and share its weights in L2
             const int parts = (M + a.tokens - 1) / a.tokens, round = block / (8 * parts), in = block - round * 8 * parts;
@@ -135,7 +135,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
             block = round * 8 + in % 8;
             if (block >= bands * max(a.ksplit, 1)) return;
         }
-        if (a.ksplit > 1) {
+        if (__builtin_expect(a.ksplit > 1, 0)) {
             split = block / bands;
             block -= split * bands;
         }
@@ -196,20 +196,15 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
     constexpr uint32_t LD = G32 ? 8 : 4;  // groups a load brings
     constexpr int PRE = 2;
     const int pieces = ROWS * runs;
+    const float per_run = __builtin_amdgcn_rcpf((float)runs);
     uint4 sv[PRE], bv[PRE];
     auto piece_at = [&](int p, int& r, int& c) {
-        r = p / runs;
+        r = (int)(((float)p + 0.5f) * per_run);  // (p / runs: p below 2^13 and runs up to 64, far from where rounding matters)
         c = p - r * runs;
         return (uint32_t)min(row0 + r % OUTS, N - 1) * (uint32_t)groups + (uint32_t)((qfirst + c) * per);
     };
     auto load_one = [&](gptr_t base, uint32_t at, uint32_t end) {
-        if (end < LD) {  // (a matrix of fewer groups than one load brings)
-            uint32_t v[4] = {0u, 0u, 0u, 0u};
-            for (uint32_t i = 0; at + i < end; i++)
-                v[i >> 1] |= (uint32_t)*reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(base + (at + i) * 2u) << (16u * (i & 1u));
-            return make_uint4(v[0], v[1], v[2], v[3]);
-        }
-        const gptr_t from = base + (size_t)min(at, end - LD) * 2u;
+        const gptr_t from = base + min(at, end - LD) * 2u;
         if constexpr (G32) {
             const u32x4_a2_t u = *reinterpret_cast<const __attribute__((address_space(1))) u32x4_a2_t*>(from);
             return make_uint4(u[0], u[1], u[2], u[3]);
@@ -225,13 +220,24 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         s = load_one(second ? sg2 : sg, at, sb_end[second ? 1 : 0]);
         b = load_one(second ? bg2 : bg, at, sb_end[second ? 1 : 0]);
     };
+    auto put_piece = [&](int r, int c, const uint32_t (&v)[2][4]) {
+        if constexpr (G32) {
+            sbq[r * sb_pitch + 2 * c] = make_uint4(v[0][0], v[0][1], v[0][2], v[0][3]);
+            sbq[r * sb_pitch + 2 * c + 1] = make_uint4(v[1][0], v[1][1], v[1][2], v[1][3]);
+        } else if (a.gs_shift == 7) {  // groups of 128 fill two places of 64
+            sbq[r * sb_pitch + c] = make_uint4((v[0][0] & 0xffffu) * 0x10001u, (v[0][0] >> 16) * 0x10001u, (v[1][0] & 0xffffu) * 0x10001u,
+                                               (v[1][0] >> 16) * 0x10001u);
+        } else {
+            sbq[r * sb_pitch + c] = make_uint4(v[0][0], v[0][1], v[1][0], v[1][1]);
+        }
+    };
     auto store_piece = [&](int p, const uint4& s, const uint4& b) {
         int r, c;
         const uint32_t at = piece_at(p, r, c), end = sb_end[PAIR && r >= OUTS ? 1 : 0];
         const int live = min(per, groups - (qfirst + c) * per);
-        const int down = end >= LD && at > end - LD ? (int)(at - (end - LD)) : 0;
+        const int down = at > end - LD ? (int)(at - (end - LD)) : 0;
         uint32_t v[2][4] = {{s.x, s.y, s.z, s.w}, {b.x, b.y, b.z, b.w}};
-        if (live != per || down != 0) {
+        if (__builtin_expect(live != per || down != 0, 0)) {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
 #pragma nounroll
@@ -245,16 +251,29 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
                 for (int e = 0; e < 4; e++) v[i][e] = 2 * e + 1 < live ? v[i][e] : 2 * e < live ? v[i][e] & 0xffffu : 0u;
             }
         }
-        if constexpr (G32) {
-            sbq[r * sb_pitch + 2 * c] = make_uint4(v[0][0], v[0][1], v[0][2], v[0][3]);
-            sbq[r * sb_pitch + 2 * c + 1] = make_uint4(v[1][0], v[1][1], v[1][2], v[1][3]);
-        } else if (a.gs_shift == 7) {  // groups of 128 fill two places of 64
-            sbq[r * sb_pitch + c] = make_uint4((v[0][0] & 0xffffu) * 0x10001u, (v[0][0] >> 16) * 0x10001u, (v[1][0] & 0xffffu) * 0x10001u,
-                                               (v[1][0] >> 16) * 0x10001u);
-        } else {
-            sbq[r * sb_pitch + c] = make_uint4(v[0][0], v[0][1], v[1][0], v[1][1]);
+        put_piece(r, c, v);
+    };
+    // A matrix of fewer groups than one load brings (up to three rows): value by value, in a place of its own, away from the code that
+    // every workgroup has to fetch.
+    const bool tiny = min(sb_end[0], sb_end[1]) < LD;
+    auto stage_tiny = [&](int from) {
+#pragma nounroll
+        for (int p = from; p < pieces; p += NT) {
+            int r, c;
+            const uint32_t at = piece_at(p, r, c);
+            const bool second = PAIR && r >= OUTS;
+            uint32_t v[2][4] = {};
+#pragma unroll
+            for (int i = 0; i < (int)LD; i++) {
+                if (i >= per || (qfirst + c) * per + i >= groups) break;
+                typedef const __attribute__((address_space(1))) uint16_t* value_ptr;
+                v[0][i >> 1] |= (uint32_t)*reinterpret_cast<value_ptr>((second ? sg2 : sg) + (at + i) * 2u) << (16 * (i & 1));
+                v[1][i >> 1] |= (uint32_t)*reinterpret_cast<value_ptr>((second ? bg2 : bg) + (at + i) * 2u) << (16 * (i & 1));
+            }
+            put_piece(r, c, v);
         }
     };
+    if (__builtin_expect(!tiny, 1))
 #pragma unroll
     for (int i = 0; i < PRE; i++)
         if (tid + i * NT < pieces) load_piece(tid + i * NT, sv[i], bv[i]);
@@ -287,13 +306,19 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
     // not entered: the kernels of eight sets and two sets of tokens spill, 32 rows of 15360 x 3840 24.9 -> 50.7.)
     bool staged = false;
     auto stage = [&]() {
+        int from = tid;
+        asm volatile("" : "+v"(from));  // (or what the stores need is worked out ahead of the loop, before its loads are requested)
+        if (__builtin_expect(tiny, 0)) {
+            stage_tiny(from);
+        } else {
 #pragma unroll
-        for (int i = 0; i < PRE; i++)
-            if (tid + i * NT < pieces) store_piece(tid + i * NT, sv[i], bv[i]);
-        for (int p = tid + PRE * NT; p < pieces; p += NT) {
-            uint4 s, b;
-            load_piece(p, s, b);
-            store_piece(p, s, b);
+            for (int i = 0; i < PRE; i++)
+                if (from + i * NT < pieces) store_piece(from + i * NT, sv[i], bv[i]);
+            for (int p = from + PRE * NT; __builtin_expect(p < pieces, 0); p += NT) {
+                uint4 s, b;
+                load_piece(p, s, b);
+                store_piece(p, s, b);
+            }
         }
         __syncthreads();
         staged = true;
@@ -322,7 +347,7 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         const bf16x8_t ones = as_bf16x8(one2, one2, one2, one2);
 #pragma unroll
         for (int ts = 0; ts < TS; ts++) {
-            if ((run + 1) * 256 > K) {
+            if (__builtin_expect((run + 1) * 256 > K, 0)) {
 #pragma unroll
                 for (int sp = 0; sp < 4; sp++)
                     if (run * 256 + sp * 64 >= K) xa[ts][sp] = xb[ts][sp] = make_uint4(0u, 0u, 0u, 0u);

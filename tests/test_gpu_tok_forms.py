@@ -155,3 +155,24 @@ def test_sums_keep_fp32_accuracy(ctx, bits, gs, M, K, N):
     print("error %.2e" % err)
     assert err <= 2.0 ** -21
     dw.free()
+
+
+@pytest.mark.parametrize("bits,gs,M,K,N", [(8, 64, 9, 64, 1), (8, 64, 17, 64, 3), (8, 64, 5, 192, 1), (4, 32, 5, 64, 1), (4, 32, 20, 64, 3), (8, 32, 9, 192, 1),
+                                           (8, 32, 2, 64, 4), (4, 128, 9, 128, 3), (4, 128, 18, 384, 1), (8, 128, 6, 384, 1), (4, 128, 6, 128, 4)])
+def test_matrices_of_fewer_groups_than_a_load_of_scales(ctx, bits, gs, M, K, N):
+    import aq_mi355
+    say("tok tiny", bits, gs, M, K, N)
+    mats = [F.synthetic_affine(N, K, bits, gs, seed=2600 + K + i) for i in range(2)]
+    x = F.synthetic_x(M, K, seed=2602)
+    dws = [DeviceAffine(ctx, *m) for m in mats]
+    acc = run_qmv(ctx, x, dws[0], M, K, N, gs, bits, True)
+    assert ctx.last_variant(0).startswith("qmvt_"), ctx.last_variant(0)
+    g, u = (F.reference_f64(x, *m, bits, gs, K) for m in mats)
+    check_accumulators(acc, g, "tiny")
+    dx, dy = ctx.to_device(x), ctx.alloc(M * N * 4)
+    ctx.qmv_gate_up(dx, *((d.w, d.s, d.b) for d in dws), dy, M, K, N, gs, bits, aq_mi355.AQ_ACT_SILU, aq_mi355.AQ_OUT_F32)
+    ctx.sync()
+    assert ctx.last_variant(0) == "qmv_gate_up_tok"
+    check_accumulators(dy.download(np.float32, M * N), g / (1.0 + np.exp(-g)) * u, "tiny pair")
+    for t in [dx, dy] + dws:
+        t.free()
