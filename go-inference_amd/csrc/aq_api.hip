@@ -383,9 +383,12 @@ hipError_t tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
     *tile = static_cast<float*>(ctx->tok_ws.ptr);
     return aq::workspace_use(ctx->stream, &ctx->tok_ws);
 }
+aq::TokPart tok_part(int K, int N, bool pair, int ksplit, int share) {
+    return {(int64_t)((N + 15) / 16) * (pair ? 2 : 1), ksplit > 1 ? ksplit : 1, ksplit > 1 ? share : (K + 255) / 256};
+}
 int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, bool pair) {
-    const int64_t bands = (int64_t)((t.N + 15) / 16) * (pair ? 2 : 1) * (t.ksplit > 1 ? t.ksplit : 1);
-    return aq::qmvt_pick(bits, group_size, t.M, t.K, bands, t.ksplit > 1 ? t.share : (t.K + 255) / 256, pair, ctx->cu_count);
+    const aq::TokPart part = tok_part(t.K, t.N, pair, t.ksplit, t.share);
+    return aq::qmvt_pick(bits, group_size, t.M, t.K, &part, 1, pair, ctx->cu_count);
 }
 
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
@@ -926,6 +929,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
     size_t bytes = 0;  // of the members' partial tiles
     aq::TokMultiArgs grid{};
     if (tok) {
+        aq::TokPart parts[aq::kQmvMultiMax];
         const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         int64_t total = 0;
         grid.common = all.common;
@@ -942,25 +946,22 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             const int oi = tok_pick(ctx, own, group_size, bits, false);
             if (oi < 0 || !aq::qmvt_fits(own, bits, group_size, oi, false)) continue;
             in_grid |= 1u << i;
-            grid.w[members] = all.w[i];
-            grid.s[members] = all.s[i];
-            grid.b[members] = all.b[i];
-            grid.y[members] = all.y[i];
-            grid.ksplit[members] = own.ksplit;
-            grid.share[members] = own.share;
-            grid.N[members++] = N[i];
+            // the longest workgroups first, or they outlast the others
+            const aq::TokPart part = tok_part(K, N[i], false, own.ksplit, own.share);
+            int at = members++;
+            for (; at > 0 && parts[at - 1].runs < part.runs; at--) {
+                grid.w[at] = grid.w[at - 1], grid.s[at] = grid.s[at - 1], grid.b[at] = grid.b[at - 1], grid.y[at] = grid.y[at - 1];
+                grid.N[at] = grid.N[at - 1], grid.ksplit[at] = grid.ksplit[at - 1], grid.share[at] = grid.share[at - 1];
+                parts[at] = parts[at - 1];
+            }
+            grid.w[at] = all.w[i], grid.s[at] = all.s[i], grid.b[at] = all.b[i], grid.y[at] = all.y[i];
+            grid.N[at] = N[i], grid.ksplit[at] = own.ksplit, grid.share[at] = own.share;
+            parts[at] = part;
             bytes += aq::qmvt_tile_bytes(M, N[i], false, own.ksplit);
             total += N[i];
         }
         grid.count = members;
-        int64_t bands = 0;
-        int runs = 1;
-        for (int i = 0; i < members; i++) {
-            const int ks = grid.ksplit[i], n = ks > 1 ? grid.share[i] : (K + 255) / 256;
-            bands += (int64_t)((grid.N[i] + 15) / 16) * ks;
-            runs = n > runs ? n : runs;
-        }
-        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, group_size, M, K, bands, runs, false, ctx->cu_count) : -1;
+        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, group_size, M, K, parts, members, false, ctx->cu_count) : -1;
         for (int i = 0; ti >= 0 && i < members; i++) {
             aq::TokArgs one{multi_member(grid, i)};
             one.tokens = grid.tokens;

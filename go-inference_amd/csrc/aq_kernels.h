@@ -198,8 +198,12 @@ int qmvt_tokens(int M);
 constexpr size_t kTokTileBytes = (size_t)32 << 20;
 void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share);
 size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit);
-// The variant for `sets` sets of 16 weight rows times their shares of K, the longest share being `runs` runs of 256 codes; or -1.
-int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count);
+// The variant for a launch of these matrices (sets of 16 weight rows, shares of K, runs of 256 codes of the longest share); or -1.
+struct TokPart {
+    int64_t sets;
+    int shares, runs;
+};
+int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count);
 // Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
 // sums are those of qmvt_launch with the same shares (the pair has its own: twice the workgroups a share).
 hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t stream);

@@ -168,59 +168,115 @@ size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit) {
 }
 
 // Microseconds of a call: `fixed` (launch, first requests, the meeting in LDS and the store), and per pass of a workgroup (eight
-// runs of 256 codes) `pass` for x and `set` for each of its sets of 16 weight rows.  From runs at K = 1024 to 14336 with one to eight
-// sets per workgroup, 1024 to 28672 rows of weights, 12 and 24 rows of x.
+// runs of 256 codes) `pass` for x and `set` for each of its sets of 16 weight rows.  From runs at K = 2048 to 12288 with one to eight
+// sets in 208 workgroups, 12 and 24 rows of x (graph replay over 640 MB of weights; off by 2.5 to 5.5 % rms, 14 % at most).
 struct TokCost {
     double fixed, pass, set;
 };
 static const TokCost& tok_cost(int bits, int group_size, int tokens) {
     // [8 bit][groups of 32][more than 16 rows of x]
-    static const TokCost kCost[2][2][2] = {{{{3.0, 1.36, 0.62}, {2.8, 2.7, 0.85}}, {{3.8, 1.2, 0.79}, {5.2, 2.1, 1.29}}},
-                                           {{{3.7, 1.3, 1.04}, {3.7, 2.7, 1.18}}, {{4.0, 1.3, 1.15}, {4.0, 2.7, 1.35}}}};
+    static const TokCost kCost[2][2][2] = {{{{2.6, 1.25, 0.72}, {2.8, 2.5, 0.89}}, {{3.0, 1.13, 0.93}, {3.85, 2.1, 1.43}}},
+                                           {{{2.3, 1.34, 1.27}, {2.45, 2.6, 1.37}}, {{2.6, 1.4, 1.35}, {2.9, 2.8, 1.5}}}};
     return kCost[bits == 8][group_size == 32][tokens > 16];
 }
-// Sets of 16 weight rows per workgroup: the fewest that leave every CU at most one workgroup, for a second round costs more than
-// longer workgroups (us on one, two, four, eight sets; 24 rows of x, K = 2816, groups of 64: 4096 rows of weights 8.3 / 9.6 / 11.9 /
-// 17.2, 8192 15.1 / 10.0 / 12.1 / 17.2, 14336 27.9 / 18.1 / 12.3 / 17.4, 2 x 14336 35.1 / 23.9 / 18.3 from two on).
-static int tok_sets(int64_t sets, int cus) {
-    for (int rs = 1; rs < 8; rs *= 2)
-        if ((sets + rs - 1) / rs <= cus) return rs;
-    return 8;
+// Passes of a workgroup whose share is `runs` runs (a part of a pass costs more than its part).
+static double tok_passes(int runs) {
+    return runs > kTokWaves ? 0.5 * ((runs + kTokWaves - 1) / kTokWaves + (double)runs / kTokWaves) : 1.0;
+}
+// When the last CU is done with these matrices on `rs` sets a workgroup, one workgroup a CU at a time, in the order of the grid.
+static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count, int parts_of_x, int cus) {
+    struct Level {  // CUs that are free at a time, earliest first
+        double at;
+        int64_t cus;
+    };
+    if (count == 1)
+        return (double)(((parts[0].sets + rs - 1) / rs * parts[0].shares * parts_of_x + cus - 1) / cus) * tok_passes(parts[0].runs) * (c.pass + rs * c.set);
+    Level levels[4 * kQmvMultiMax] = {{0.0, cus}};
+    int n = 1;
+    for (int i = 0; i < count; i++) {
+        const double t = tok_passes(parts[i].runs) * (c.pass + rs * c.set);
+        int64_t groups = (parts[i].sets + rs - 1) / rs * parts[i].shares * parts_of_x;
+        while (groups > 0) {
+            if (n == 1) {  // whole rounds
+                levels[0].at += (double)(groups / cus) * t;
+                groups %= cus;
+                if (groups == 0) break;
+            }
+            const int64_t now = groups < levels[0].cus ? groups : levels[0].cus;
+            const Level next = {levels[0].at + t, now};
+            if ((levels[0].cus -= now) == 0) {
+                n--;
+                for (int l = 0; l < n; l++) levels[l] = levels[l + 1];
+            }
+            int at = 0;
+            while (at < n && levels[at].at < next.at) at++;
+            if (at < n && levels[at].at == next.at) {
+                levels[at].cus += now;
+            } else if (n == 4 * kQmvMultiMax) {  // (not seen: as if they were done when those above are)
+                levels[at < n ? at : n - 1].cus += now;
+            } else {
+                for (int l = n++; l > at; l--) levels[l] = levels[l - 1];
+                levels[at] = next;
+            }
+            groups -= now;
+        }
+    }
+    return levels[n - 1].at;
+}
+// Sets of 16 weight rows per workgroup, by the same figures.  Mostly the fewest that leave every CU one workgroup (us on one, two,
+// four, eight sets; 24 rows of x, K = 2816, groups of 64: 4096 rows of weights 8.3 / 9.6 / 11.9 / 17.2, 8192 15.1 / 10.0 / 12.1 /
+// 17.2, 14336 27.9 / 18.1 / 12.3 / 17.4, 2 x 14336 35.1 / 23.9 / 18.3 from two on); fewer where a second round would be nearly empty,
+// and where members of a grid differ in length, so that the ones that are not shared out do not outlast the rest.
+static int tok_sets(const TokCost& c, const TokPart* parts, int count, int parts_of_x, int cus, double* us = nullptr) {
+    double best = 1e30;
+    int best_rs = 1;
+    for (int rs = 1; rs <= 8; rs *= 2) {
+        const double t = tok_span(c, rs, parts, count, parts_of_x, cus);
+        if (t < best) best = t, best_rs = rs;
+    }
+    if (us) *us = c.fixed + best;
+    return best_rs;
 }
 
-// Shares of K where a workgroup would make several passes: the shares' workgroups carry more rows each, and a second launch adds
-// their partial tiles, which costs about 2.5 us and one more per megabyte (12 / 24 rows of x by 4096 x 14336 whole 16.9 / 27.9 us,
-// eight shares 13.5 / 18.0; 1024 x 14336 16.1 / 27.0, 10.2 / 12.8; at K = 4096, two passes, shares win nothing).
-// Asked for 24 rows of x for every call of up to 32 and for 48 beyond, so that shares, and with them the bytes of a row, do not
-// depend on the number of rows; against a choice for each number the model
-// loses 0.04 % on average (27 shapes where the two differ: 2 % faster on average, 8 bit 5 x 6528 x 3408 at worst 9.2 -> 11.2 us).
+// Shares of K where a workgroup would make three passes or more: the shares' workgroups carry more rows each, and a second launch
+// adds their partial tiles, which costs about 2.5 us and one more per megabyte (us, whole / shares, 12 and 24 rows of x: 4096 x 14336
+// 16.3 / 13.3 and 26.6 / 17.8, 1024 x 14336 16.3 / 8.6 and 26.6 / 10.7, 1536 x 6144 8.5 / 8.4 and 13.0 / 10.4).  With two passes they
+// win at more than 16 rows what they lose at fewer, and lose where a matrix is one of several in a grid (1024 x 4096 6.5 / 7.2 and
+// 9.6 / 8.6; 32 rows of 4096 x (4096 | 1024 | 1024) 13.2 / 16.3).
+// The choice for every call of up to 32 rows is the one that 12 and 24 rows are fastest with together, and the one for 48 rows beyond,
+// so that shares, and with them the bytes of a row, do not depend on the number of rows.
 void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share) {
-    const int cus = cu_count > 0 ? cu_count : 256, quads = (K + 255) / 256;
-    const int rows = M <= 32 ? 24 : 48, most = M <= 32 ? 32 : 64, tokens = qmvt_tokens(rows);
-    const TokCost& c = tok_cost(bits, group_size, tokens);
+    const int cus = cu_count > 0 ? cu_count : 256, quads = (K + 255) / 256, most = M <= 32 ? 32 : 64;
     *ksplit = 1;
     *share = quads;
     if ((bits != 4 && bits != 8) || M > kTokMax || K % 64 != 0 || K > kTokMaxK) return;  // (no call of these kernels)
-    const int64_t sets = (int64_t)((N + 15) / 16) * (pair ? 2 : 1) * ((rows + tokens - 1) / tokens);
+    if (quads <= 2 * kTokWaves) return;
     double best = 1e30;
     for (int ks = 1; ks <= kTokShares && ks <= quads; ks++) {
         const int sh = (quads + ks - 1) / ks, n = (quads + sh - 1) / sh;
         if (n != ks || qmvt_tile_bytes(most, N, pair, n) > kTokTileBytes) continue;
-        const int rs = tok_sets(sets * n, cus);
-        const double rounds = std::ceil((double)((sets * n + rs - 1) / rs) / cus);
-        const int whole = (sh + kTokWaves - 1) / kTokWaves;
-        const double passes = sh > kTokWaves ? 0.5 * (whole + (double)sh / kTokWaves) : 1.0;  // (a part of a pass costs more than its part)
-        double us = c.fixed + rounds * passes * (c.pass + rs * c.set);
-        if (n > 1) us = 1.1 * us + 2.5 + (double)qmvt_tile_bytes(rows, N, pair, n) / 1e6;  // (a tenth: no shares for next to nothing)
-        if (us < best) best = us, *ksplit = n, *share = sh;
+        double sum = 0.0;
+        for (const int rows : {12, 24, 48}) {
+            if ((rows > 32) != (M > 32)) continue;
+            const int tokens = qmvt_tokens(rows);
+            const TokPart part{(int64_t)((N + 15) / 16) * (pair ? 2 : 1), n, sh};
+            double us;
+            tok_sets(tok_cost(bits, group_size, tokens), &part, 1, (rows + tokens - 1) / tokens, cus, &us);
+            // (a tenth: no shares for next to nothing, see above)
+            if (n > 1) us = (M <= 32 ? 1.1 : 1.0) * us + 2.5 + (double)qmvt_tile_bytes(rows, N, pair, n) / 1e6;
+            sum += us;
+        }
+        if (sum < best) best = sum, *ksplit = n, *share = sh;
+        if (sh <= kTokWaves) break;  // (one pass: more shares have nothing to win)
     }
 }
 
-int qmvt_pick(int bits, int group_size, int M, int K, int64_t sets, int runs, bool pair, int cu_count) {
-    if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK) return -1;
+int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count) {
+    if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK || count < 1) return -1;
     const int cus = cu_count > 0 ? cu_count : 256, tokens = qmvt_tokens(M), most = tokens <= 16 ? 16 : 32;
-    int rs = tok_sets(sets * ((M + tokens - 1) / tokens), cus);
+    int rs = tok_sets(tok_cost(bits, group_size, tokens), parts, count, (M + tokens - 1) / tokens, cus), runs = 1;
     if (pair && rs == 1) rs = 2;
+    for (int i = 0; i < count; i++) runs = parts[i].runs > runs ? parts[i].runs : runs;
     for (int i = 0; i < qmvt_variant_count(); i++) {  // (listed with eight, four, two, one sets)
         const QmvTokEntry& e = tok_entry(i);
         if (e.v.bits != bits || e.v.m != most || e.v.rows > rs) continue;
