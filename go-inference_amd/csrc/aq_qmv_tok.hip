@@ -312,7 +312,7 @@ __global__ __launch_bounds__(256) void tok_reduce_kernel(const TokReduceArgs a) 
 #pragma unroll
                 for (int e = 0; e < V; e++) v[e] = s ? v[e] + t[s][e] : t[s][e];
     };
-    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (int64_t)a.M * per_row) return;
     const int m = (int)(i / per_row), c = (int)(i - (int64_t)m * per_row) * V;
     float v[V], u[V];
@@ -342,15 +342,18 @@ __global__ __launch_bounds__(256) void tok_reduce_kernel(const TokReduceArgs a) 
 
 hipError_t tok_reduce_launch(const TokReduceArgs& a, hipStream_t stream) {
     int64_t most = 0;
-    bool by4 = true;
+    // (groups of 32: outputs that are formed again take a thread each, on as many CUs as there are wavefronts; us, by fours in
+    // workgroups of 256 / so: 4 rows with an infinity by 2684 x 10112 3810 / 734, 25 by 625 x 15616 1790 / 1281)
+    bool by4 = a.gs_shift != 5;
     for (int i = 0; i < a.count; i++) {
         if (!a.tile[i]) continue;
         most = (int64_t)a.M * a.N[i] > most ? (int64_t)a.M * a.N[i] : most;
         by4 = by4 && a.N[i] % 4 == 0;
     }
     if (most == 0) return hipSuccess;
-    const int64_t grid = (most / (by4 ? 4 : 1) + 255) / 256;
-    hipLaunchKernelGGL(by4 ? tok_reduce_kernel<4> : tok_reduce_kernel<1>, dim3((unsigned)grid, (unsigned)a.count), dim3(256), 0, stream, a);
+    const int threads = a.gs_shift == 5 ? 64 : 256;
+    const int64_t grid = (most / (by4 ? 4 : 1) + threads - 1) / threads;
+    hipLaunchKernelGGL(by4 ? tok_reduce_kernel<4> : tok_reduce_kernel<1>, dim3((unsigned)grid, (unsigned)a.count), dim3((unsigned)threads), 0, stream, a);
     return hipGetLastError();
 }
 
