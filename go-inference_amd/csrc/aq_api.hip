@@ -384,7 +384,7 @@ hipError_t tok_tiles(aq_ctx* ctx, size_t bytes, float** tile) {
     return aq::workspace_use(ctx->stream, &ctx->tok_ws);
 }
 aq::TokPart tok_part(int K, int N, bool pair, int ksplit, int share) {
-    return {(int64_t)((N + 15) / 16) * (pair ? 2 : 1), ksplit > 1 ? ksplit : 1, ksplit > 1 ? share : (K + 255) / 256};
+    return {(int64_t)((N + 15) / 16) * (pair ? 2 : 1), ksplit > 1 ? ksplit : 1, ksplit > 1 ? share : (K + 255) / 256, 0};
 }
 int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, bool pair) {
     const aq::TokPart part = tok_part(t.K, t.N, pair, t.ksplit, t.share);
@@ -961,12 +961,32 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             total += N[i];
         }
         grid.count = members;
-        ti = members > 0 && total < (int64_t)1 << 30 ? aq::qmvt_pick(bits, group_size, M, K, parts, members, false, ctx->cu_count) : -1;
+        if (members > 0 && total < (int64_t)1 << 30) {
+            double shared = 0, whole = 0;
+            ti = aq::qmvt_pick(bits, group_size, M, K, parts, members, false, ctx->cu_count, &shared);
+            if (bytes > 0) {
+                // Workgroups that share K out, with a launch that adds their tiles, or that work through the shares by themselves:
+                // the others may fill the chip without them (us, shared out / by themselves: 9 / 32 rows of 5376 x (4096 | 2048 |
+                // 2048) 13.6 / 11.7 and 24.1 / 19.0, of 6144 x (6144 | 1024 | 1024) 14.6 / 12.4 and 26.0 / 20.7)
+                aq::TokPart alone[aq::kQmvMultiMax];
+                for (int i = 0; i < members; i++) {
+                    alone[i] = parts[i];
+                    if (grid.ksplit[i] > 1) alone[i].shares = 1, alone[i].inside = grid.ksplit[i];
+                }
+                const int own = aq::qmvt_pick(bits, group_size, M, K, alone, members, false, ctx->cu_count, &whole);
+                if (own >= 0 && whole < shared + 2.5 + (double)bytes / 1e6) {
+                    ti = own;
+                    bytes = 0;
+                    for (int i = 0; i < members; i++) grid.inside[i] = grid.ksplit[i] > 1 ? grid.ksplit[i] : 0, grid.ksplit[i] = 1;
+                }
+            }
+        }
         for (int i = 0; ti >= 0 && i < members; i++) {
             aq::TokArgs one{multi_member(grid, i)};
             one.tokens = grid.tokens;
             one.ksplit = grid.ksplit[i];
             one.share = grid.share[i];
+            one.inside = grid.inside[i];
             if (!aq::qmvt_fits(one, bits, group_size, ti, false)) ti = -1;
         }
         if (ti < 0 || bytes > aq::kTokTileBytes) in_grid = 0;  // (members apart have the block to themselves, one after another)

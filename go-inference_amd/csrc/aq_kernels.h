@@ -175,10 +175,11 @@ struct TokArgs : QmvArgs {
     int ksplit, share;  // shares of K (0, 1: none), 256-code runs per share
     float* tile;        // the fp32 partial tiles
     int tokens;         // rows of x per workgroup
+    int inside;         // shares of K that a workgroup works through by itself (0, 1: none; several matrices in one grid only)
     uint32_t red_at;    // filled by the launcher: where in LDS the wavefronts' sums meet
 };
 struct TokMultiArgs : QmvMultiArgs {
-    int ksplit[kQmvMultiMax], share[kQmvMultiMax];
+    int ksplit[kQmvMultiMax], share[kQmvMultiMax], inside[kQmvMultiMax];
     float* tile[kQmvMultiMax];
     int tokens;
     uint32_t red_at;
@@ -198,12 +199,13 @@ int qmvt_tokens(int M);
 constexpr size_t kTokTileBytes = (size_t)32 << 20;
 void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu_count, int* ksplit, int* share);
 size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit);
-// The variant for a launch of these matrices (sets of 16 weight rows, shares of K, runs of 256 codes of the longest share); or -1.
+// The variant for a launch of these matrices, and its microseconds; or -1.
 struct TokPart {
-    int64_t sets;
-    int shares, runs;
+    int64_t sets;      // of 16 weight rows
+    int shares, runs;  // shares of K, runs of 256 codes of the longest
+    int inside;        // ... that a workgroup works through by itself: `shares` is 1 then, `runs` that of a share
 };
-int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count);
+int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count, double* us = nullptr);
 // Several matrices that share x in one grid, and the gated pair act(gate . x) * (up . x) (a.w2, a.s2, a.b2, a.act): the
 // sums are those of qmvt_launch with the same shares (the pair has its own: twice the workgroups a share).
 hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t stream);

@@ -43,6 +43,7 @@ constexpr int kTokMax = 64;   // activation rows per launch (the M side), 32 per
 constexpr int kTokMaxK = 16384;
 constexpr int kTokWaves = 8;  // wavefronts of a workgroup, which share K
 constexpr int kTokShares = 16;  // most shares of K
+constexpr int kTokInsideSets = 4;  // most sets of rows of a workgroup that works through shares by itself (eight, with two sets of tokens, spill)
 typedef uint32_t __attribute__((ext_vector_type(4), aligned(2))) u32x4_a2_t;  // loads of any alignment
 typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) u32x2_a2_t;
 
@@ -90,7 +91,8 @@ typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) u32x2_a2_t;
 // GROUPED (expert slabs): the rows of x of a launch are the routes of one chunk of the list a.chunks (aq_moe_group.hip):
 // up to 16 TS routes that name the same expert, which then streams its weights once for all of them.
 // a.ksplit > 1: the workgroups of a band of rows share K out, a.share runs each, and store fp32 partial tiles [ksplit][M][N]
-// ([ksplit][M][gate N | up N] for a pair) that tok_reduce_kernel adds in order.
+// ([ksplit][M][gate N | up N] for a pair) that tok_reduce_kernel adds in order.  a.inside > 1 (INSIDE): a workgroup works through
+// that many shares by itself and adds their sums in the same order.
 constexpr int kTokRowPitch = 144;  // LDS bytes between the 128-byte lines of a wavefront's rows: reads of 4 q + 16 step fall into different banks
 // LDS bytes of the staged scales and biases of `rows` weight rows over `runs` runs, 16-byte pieces at an odd pitch so that the 16
 // rows a wavefront reads at once fall into different banks
@@ -101,7 +103,7 @@ __host__ __device__ constexpr int tok_line_bytes(int bits) { return bits == 4 ? 
 __host__ __device__ constexpr bool tok_from_sum(int bits, bool g32) { return bits == 4 && g32; }
 __host__ __device__ constexpr int tok_own_bytes(int bits, bool g32, int ts) { return tok_line_bytes(bits) + (tok_from_sum(bits, g32) ? ts * 512 : 0); }
 
-template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR, bool GROUPED>
+template <int BITS, int RS, int RING, int TS, int GRP, bool PAIR, bool GROUPED, bool INSIDE = false>
 __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block_of_all) {
     static_assert(BITS == 4 || BITS == 8, "code width");
     static_assert(GRP == 64 || GRP == 32, "group size (64: and 128)");
@@ -323,273 +325,294 @@ __device__ __forceinline__ void qmv_tok16_body(const TokArgs& a, const int block
         __syncthreads();
         staged = true;
     };
-    for (int at = wave; at < runs; at += NW) {
-        const int run = qfirst + at;
-        uint4 xa[TS][4], xb[TS][4];
-#pragma unroll
-        for (int ts = 0; ts < TS; ts++)
-#pragma unroll
-            for (int sp = 0; sp < 4; sp++) {
-                const uint32_t in_row = run * 256 + sp * 64 < K ? (uint32_t)run * 512u + (uint32_t)sp * 128u : 0u;  // uniform
-                xa[ts][sp] = load_u128_at(xg, x_lane[ts][0] + in_row);
-                xb[ts][sp] = load_u128_at(xg, x_lane[ts][1] + in_row);
-            }
-        __builtin_amdgcn_sched_barrier(0);
-        issue_set(std::integral_constant<int, 0>{}, run);
-        if constexpr (RING > 1 && RS > 1) issue_set(std::integral_constant<int, 1>{}, run);
-        __builtin_amdgcn_sched_barrier(0);
-        if (!staged) stage();
-
-        // A operands of the run, and the three-way split of the lane block's group sum of x
-        if constexpr (FROM_SUM) order_wave_lds();  // (the sums of the last run have been read)
-        bf16x8_t af[TS][8], a2[TS][GPR / 4];
-        const uint32_t one2 = 0x3f803f80u;
-        const bf16x8_t ones = as_bf16x8(one2, one2, one2, one2);
-#pragma unroll
-        for (int ts = 0; ts < TS; ts++) {
-            if (__builtin_expect((run + 1) * 256 > K, 0)) {
-#pragma unroll
-                for (int sp = 0; sp < 4; sp++)
-                    if (run * 256 + sp * 64 >= K) xa[ts][sp] = xb[ts][sp] = make_uint4(0u, 0u, 0u, 0u);
-            }
-            f32x4_t sum[GPR];  // (every register of lane (t, q) is token t's)
-            [[maybe_unused]] uint4 held = {0u, 0u, 0u, 0u};
-#pragma unroll
-            for (int st = 0; st < 8; st++) {
-                // even step: lanes i >= 8 take tokens 8..15 from the second load's lanes i - 8; odd step: lanes i < 8 take
-                // tokens 0..7 from the first load's lanes i + 8
-                const uint4 va = xa[ts][st >> 1], vb = xb[ts][st >> 1];
-                uint4 v;
-                if ((st & 1) == 0) {
-                    v.x = __builtin_amdgcn_update_dpp(va.x, vb.x, 0x118, 0xf, 0xc, false);
-                    v.y = __builtin_amdgcn_update_dpp(va.y, vb.y, 0x118, 0xf, 0xc, false);
-                    v.z = __builtin_amdgcn_update_dpp(va.z, vb.z, 0x118, 0xf, 0xc, false);
-                    v.w = __builtin_amdgcn_update_dpp(va.w, vb.w, 0x118, 0xf, 0xc, false);
-                } else {
-                    v.x = __builtin_amdgcn_update_dpp(vb.x, va.x, 0x108, 0xf, 0x3, false);
-                    v.y = __builtin_amdgcn_update_dpp(vb.y, va.y, 0x108, 0xf, 0x3, false);
-                    v.z = __builtin_amdgcn_update_dpp(vb.z, va.z, 0x108, 0xf, 0x3, false);
-                    v.w = __builtin_amdgcn_update_dpp(vb.w, va.w, 0x108, 0xf, 0x3, false);
-                }
-                if constexpr (BITS == 4)  // the order the expansion leaves the codes of a word in: 0 2 4 6 1 3 5 7
-                    v = make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
-                                   __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
-                if constexpr (BITS == 8 && G32) {  // (as the codes: the even step's upper lanes against the odd one's lower)
-                    if ((st & 1) == 0) {
-                        held = v;
-                        continue;
-                    }
-                    const auto x = __builtin_amdgcn_permlane32_swap(held.x, v.x, false, false);
-                    const auto y = __builtin_amdgcn_permlane32_swap(held.y, v.y, false, false);
-                    const auto z = __builtin_amdgcn_permlane32_swap(held.z, v.z, false, false);
-                    const auto w = __builtin_amdgcn_permlane32_swap(held.w, v.w, false, false);
-                    af[ts][st - 1] = as_bf16x8(x[0], y[0], z[0], w[0]);
-                    sum[st - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[ts][st - 1], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    v = make_uint4(x[1], y[1], z[1], w[1]);
-                }
-                af[ts][st] = as_bf16x8(v.x, v.y, v.z, v.w);
-                const int g = st / (8 / GPR);
-                const bool begins = st % (8 / GPR) == 0;
-                sum[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[ts][st], begins ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : sum[g], 0, 0, 0);
-            }
-#pragma unroll
-            for (int g4 = 0; g4 < GPR / 4; g4++) {
-                const float X = q == 0 ? sum[4 * g4][0] : q == 1 ? sum[4 * g4 + 1][0] : q == 2 ? sum[4 * g4 + 2][0] : sum[4 * g4 + 3][0];
-                if constexpr (FROM_SUM) sums_own[(ts * 8 + 4 * g4 + q) * 16 + n] = -8.0f * X;
-                const uint32_t u0 = __float_as_uint(X) & 0xffff0000u;
-                const float r1 = X - __uint_as_float(u0);
-                const uint32_t u1 = __float_as_uint(r1) & 0xffff0000u;
-                const uint32_t u2 = __float_as_uint(r1 - __uint_as_float(u1)) & 0xffff0000u;
-                const uint32_t m0 = __float_as_uint(kLacks * __uint_as_float(u0));
-                const uint32_t m1 = __float_as_uint(kLacks * __uint_as_float(u1));
-                const uint32_t m2 = __float_as_uint(kLacks * __uint_as_float(u2));
-                a2[ts][g4] = as_bf16x8((u0 >> 16) | u1, (u2 >> 16) | m0, (m1 >> 16) | m2, 0u);
-            }
-        }
-        // picks element q of four bf16 values in two registers, twice
-        const uint32_t sel_q = 0x01000100u + 0x02020202u * (uint32_t)q;
-
-        auto run_set = [&](auto rs_tag) {
-            constexpr int rs = decltype(rs_tag)::value, SL = rs % RING;
-            // scales, then biases, of the run's groups
-            uint4 sbv, bbv;
-            if constexpr (G32) {
-                sbv = sbq[(rs * 16 + n) * sb_pitch + 2 * at];
-                bbv = sbq[(rs * 16 + n) * sb_pitch + 2 * at + 1];
-            } else {
-                sbv = sbq[(rs * 16 + n) * sb_pitch + at];
-                bbv = make_uint4(sbv.z, sbv.w, 0u, 0u);
-            }
-            // the codes of a line: 4 bit the words of the set's eight steps, 8 bit the two words of each of four steps
-            // (8 bit, two sets of tokens, in groups of 32 or with eight sets of rows: both lines at once, so that the next set is
-            // requested before the first product; us, line by line / at once: 32 rows of 4096 x 14336 in groups of 32 22.0 / 21.7, of
-            // 2560 x (10240 | 10240) 24.0 / 22.2, of 14336 x 4096 22.0 / 21.2; but 32 rows of 4096 x 14336 in groups of 64 20.0 / 20.6,
-            // and one set of tokens, 4 rows, 14.6 / 15.3)
-            constexpr int HELD = TS == 2 && (G32 || RS == 8) ? LINES : 1;
-            uint32_t ww[8 * HELD];
-            auto fetch_line = [&](int ln) {
-                const int w0 = ln % HELD * 8;
-                const uint4 la = ring[SL][ln][0], lb = ring[SL][ln][1];
-                if constexpr (BITS == 4) {
-                    unsigned char* const to = w_own + (n & 7) * kTokRowPitch + part16;
-                    order_wave_lds();  // (the last set's words have been read)
-                    *reinterpret_cast<uint4*>(to) = la;
-                    *reinterpret_cast<uint4*>(to + 8 * kTokRowPitch) = lb;
-                    order_wave_lds();  // the lines, and the sums above, are there for other lanes to read
-                    const unsigned char* const from = w_own + n * kTokRowPitch;
-#pragma unroll
-                    for (int i = 0; i < 8; i++) ww[i] = *reinterpret_cast<const uint32_t*>(from + i * 16 + q * 4);
-                } else {
-                    // first 64 bytes of all 16 rows (lanes i >= 8 from the second load's lanes i - 8), second 64 bytes (lanes
-                    // i < 8 from the first load's lanes i + 8): as for x
-                    ww[w0] = __builtin_amdgcn_update_dpp(la.x, lb.x, 0x118, 0xf, 0xc, false);
-                    ww[w0 + 1] = __builtin_amdgcn_update_dpp(la.y, lb.y, 0x118, 0xf, 0xc, false);
-                    ww[w0 + 2] = __builtin_amdgcn_update_dpp(la.z, lb.z, 0x118, 0xf, 0xc, false);
-                    ww[w0 + 3] = __builtin_amdgcn_update_dpp(la.w, lb.w, 0x118, 0xf, 0xc, false);
-                    ww[w0 + 4] = __builtin_amdgcn_update_dpp(lb.x, la.x, 0x108, 0xf, 0x3, false);
-                    ww[w0 + 5] = __builtin_amdgcn_update_dpp(lb.y, la.y, 0x108, 0xf, 0x3, false);
-                    ww[w0 + 6] = __builtin_amdgcn_update_dpp(lb.z, la.z, 0x108, 0xf, 0x3, false);
-                    ww[w0 + 7] = __builtin_amdgcn_update_dpp(lb.w, la.w, 0x108, 0xf, 0x3, false);
-                    if constexpr (G32) {  // a step is one half of a block of 64: the second 8 codes of its lanes move across
-#pragma unroll
-                        for (int g = 0; g < 2; g++)
-#pragma unroll
-                            for (int k = 0; k < 2; k++) {
-                                const auto p = __builtin_amdgcn_permlane32_swap(ww[w0 + 4 * g + k], ww[w0 + 4 * g + 2 + k], false, false);
-                                ww[w0 + 4 * g + k] = p[0];
-                                ww[w0 + 4 * g + 2 + k] = p[1];
-                            }
-                    }
-                }
-                if (ln == LINES - 1) {  // (into the registers that are free now)
-                    __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (rs + RING < RS) issue_set(std::integral_constant<int, rs + RING>{}, run);
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            };
-            f32x4_t part[TS], d[TS];
-#pragma unroll
-            for (int ts = 0; ts < TS; ts++) part[ts] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
-            auto step = [&](auto st_tag) {
-                constexpr int st = decltype(st_tag)::value;
-                if constexpr (st % (8 * HELD / LINES) == 0)
-#pragma unroll
-                    for (int ln = st * LINES / 8; ln < st * LINES / 8 + HELD; ln++) fetch_line(ln);
-                uint32_t e[4];
-                if constexpr (BITS == 4) {
-                    unpack4_codes(ww[st], e);
-                } else {
-                    constexpr int w0 = 2 * (st % (4 * HELD));
-                    unpack8_centred(ww[w0], e);
-                    unpack8_centred(ww[w0 + 1], e + 2);
-                }
-                const bf16x8_t bop = as_bf16x8(e[0], e[1], e[2], e[3]);
-                constexpr int g = st / (8 / GPR);
-                constexpr bool begins = st % (8 / GPR) == 0, ends = (st + 1) % (8 / GPR) == 0;
-                const uint32_t sw = g < 2 ? sbv.x : g < 4 ? sbv.y : g < 6 ? sbv.z : sbv.w;
-                const float sc = (g & 1) ? __uint_as_float(sw & 0xffff0000u) : __uint_as_float(sw << 16);
-#pragma unroll
-                for (int ts = 0; ts < TS; ts++) {
-                    f32x4_t from = {0.0f, 0.0f, 0.0f, 0.0f};
-                    if constexpr (FROM_SUM) from = *reinterpret_cast<const f32x4_t*>(sums_own + (ts * 8 + st) * 16 + 4 * q);
-                    d[ts] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[ts][st], bop, begins ? from : d[ts], 0, 0, 0);
-                    if (ends)
-#pragma unroll
-                        for (int r = 0; r < 4; r++) {
-                            float v = __builtin_fmaf(sc, d[ts][r], part[ts][r]);
-                            if constexpr (G32) asm volatile("" : "+v"(v));  // here, not behind all the steps: their products would be held until then
-                            part[ts][r] = v;
-                        }
-                }
-            };
-            step(std::integral_constant<int, 0>{});
-            step(std::integral_constant<int, 1>{});
-            step(std::integral_constant<int, 2>{});
-            step(std::integral_constant<int, 3>{});
-            step(std::integral_constant<int, 4>{});
-            step(std::integral_constant<int, 5>{});
-            step(std::integral_constant<int, 6>{});
-            step(std::integral_constant<int, 7>{});
-#pragma unroll
-            for (int g4 = 0; g4 < GPR / 4; g4++) {
-                const uint32_t bb = __builtin_amdgcn_perm(g4 ? bbv.w : bbv.y, g4 ? bbv.z : bbv.x, sel_q);
-                const uint32_t ss = __builtin_amdgcn_perm(g4 ? sbv.w : sbv.y, g4 ? sbv.z : sbv.x, sel_q);
-                const bf16x8_t b2 = as_bf16x8(bb, __builtin_amdgcn_perm(ss, bb, 0x05040100u), ss, 0u);
-#pragma unroll
-                for (int ts = 0; ts < TS; ts++)
-                    part[ts] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[ts][g4], b2, part[ts], 0, 0, 0);
-            }
+    // INSIDE: a.inside shares of K one after another, each with a meeting of its own, so that the sums are those of workgroups that
+    // share K out.
+    int share_from = 0, share_end = INSIDE && a.inside > 1 ? a.share : runs;
+    float* const red = reinterpret_cast<float*>(lds_raw + a.red_at);
+    [[maybe_unused]] float* const kept = red + NW * 16 * TS * ROWS;  // the sums of the shares so far
+    while (true) {
+        for (int at = share_from + wave; at < share_end; at += NW) {
+            const int run = qfirst + at;
+            uint4 xa[TS][4], xb[TS][4];
 #pragma unroll
             for (int ts = 0; ts < TS; ts++)
 #pragma unroll
-                for (int r = 0; r < 4; r++) acc[rs][ts][r] += part[ts][r];
+                for (int sp = 0; sp < 4; sp++) {
+                    const uint32_t in_row = run * 256 + sp * 64 < K ? (uint32_t)run * 512u + (uint32_t)sp * 128u : 0u;  // uniform
+                    xa[ts][sp] = load_u128_at(xg, x_lane[ts][0] + in_row);
+                    xb[ts][sp] = load_u128_at(xg, x_lane[ts][1] + in_row);
+                }
             __builtin_amdgcn_sched_barrier(0);
-        };
-        run_set(std::integral_constant<int, 0>{});
-        if constexpr (RS > 1) run_set(std::integral_constant<int, 1>{});
-        if constexpr (RS > 2) run_set(std::integral_constant<int, 2>{});
-        if constexpr (RS > 3) run_set(std::integral_constant<int, 3>{});
-        if constexpr (RS > 4) run_set(std::integral_constant<int, 4>{});
-        if constexpr (RS > 5) run_set(std::integral_constant<int, 5>{});
-        if constexpr (RS > 6) run_set(std::integral_constant<int, 6>{});
-        if constexpr (RS > 7) run_set(std::integral_constant<int, 7>{});
-        static_assert(RS <= 8 && RS % RING == 0, "sets of rows per workgroup");
-    }
+            issue_set(std::integral_constant<int, 0>{}, run);
+            if constexpr (RING > 1 && RS > 1) issue_set(std::integral_constant<int, 1>{}, run);
+            __builtin_amdgcn_sched_barrier(0);
+            if (!staged) stage();
 
-    if (!staged) stage();  // a wavefront without a run of its own
+            // A operands of the run, and the three-way split of the lane block's group sum of x
+            if constexpr (FROM_SUM) order_wave_lds();  // (the sums of the last run have been read)
+            bf16x8_t af[TS][8], a2[TS][GPR / 4];
+            const uint32_t one2 = 0x3f803f80u;
+            const bf16x8_t ones = as_bf16x8(one2, one2, one2, one2);
+#pragma unroll
+            for (int ts = 0; ts < TS; ts++) {
+                if (__builtin_expect((run + 1) * 256 > K, 0)) {
+#pragma unroll
+                    for (int sp = 0; sp < 4; sp++)
+                        if (run * 256 + sp * 64 >= K) xa[ts][sp] = xb[ts][sp] = make_uint4(0u, 0u, 0u, 0u);
+                }
+                f32x4_t sum[GPR];  // (every register of lane (t, q) is token t's)
+                [[maybe_unused]] uint4 held = {0u, 0u, 0u, 0u};
+#pragma unroll
+                for (int st = 0; st < 8; st++) {
+                    // even step: lanes i >= 8 take tokens 8..15 from the second load's lanes i - 8; odd step: lanes i < 8 take
+                    // tokens 0..7 from the first load's lanes i + 8
+                    const uint4 va = xa[ts][st >> 1], vb = xb[ts][st >> 1];
+                    uint4 v;
+                    if ((st & 1) == 0) {
+                        v.x = __builtin_amdgcn_update_dpp(va.x, vb.x, 0x118, 0xf, 0xc, false);
+                        v.y = __builtin_amdgcn_update_dpp(va.y, vb.y, 0x118, 0xf, 0xc, false);
+                        v.z = __builtin_amdgcn_update_dpp(va.z, vb.z, 0x118, 0xf, 0xc, false);
+                        v.w = __builtin_amdgcn_update_dpp(va.w, vb.w, 0x118, 0xf, 0xc, false);
+                    } else {
+                        v.x = __builtin_amdgcn_update_dpp(vb.x, va.x, 0x108, 0xf, 0x3, false);
+                        v.y = __builtin_amdgcn_update_dpp(vb.y, va.y, 0x108, 0xf, 0x3, false);
+                        v.z = __builtin_amdgcn_update_dpp(vb.z, va.z, 0x108, 0xf, 0x3, false);
+                        v.w = __builtin_amdgcn_update_dpp(vb.w, va.w, 0x108, 0xf, 0x3, false);
+                    }
+                    if constexpr (BITS == 4)  // the order the expansion leaves the codes of a word in: 0 2 4 6 1 3 5 7
+                        v = make_uint4(__builtin_amdgcn_perm(v.y, v.x, 0x05040100u), __builtin_amdgcn_perm(v.w, v.z, 0x05040100u),
+                                       __builtin_amdgcn_perm(v.y, v.x, 0x07060302u), __builtin_amdgcn_perm(v.w, v.z, 0x07060302u));
+                    if constexpr (BITS == 8 && G32) {  // (as the codes: the even step's upper lanes against the odd one's lower)
+                        if ((st & 1) == 0) {
+                            held = v;
+                            continue;
+                        }
+                        const auto x = __builtin_amdgcn_permlane32_swap(held.x, v.x, false, false);
+                        const auto y = __builtin_amdgcn_permlane32_swap(held.y, v.y, false, false);
+                        const auto z = __builtin_amdgcn_permlane32_swap(held.z, v.z, false, false);
+                        const auto w = __builtin_amdgcn_permlane32_swap(held.w, v.w, false, false);
+                        af[ts][st - 1] = as_bf16x8(x[0], y[0], z[0], w[0]);
+                        sum[st - 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[ts][st - 1], f32x4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+                        v = make_uint4(x[1], y[1], z[1], w[1]);
+                    }
+                    af[ts][st] = as_bf16x8(v.x, v.y, v.z, v.w);
+                    const int g = st / (8 / GPR);
+                    const bool begins = st % (8 / GPR) == 0;
+                    sum[g] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, af[ts][st], begins ? f32x4_t{0.0f, 0.0f, 0.0f, 0.0f} : sum[g], 0, 0, 0);
+                }
+#pragma unroll
+                for (int g4 = 0; g4 < GPR / 4; g4++) {
+                    const float X = q == 0 ? sum[4 * g4][0] : q == 1 ? sum[4 * g4 + 1][0] : q == 2 ? sum[4 * g4 + 2][0] : sum[4 * g4 + 3][0];
+                    if constexpr (FROM_SUM) sums_own[(ts * 8 + 4 * g4 + q) * 16 + n] = -8.0f * X;
+                    const uint32_t u0 = __float_as_uint(X) & 0xffff0000u;
+                    const float r1 = X - __uint_as_float(u0);
+                    const uint32_t u1 = __float_as_uint(r1) & 0xffff0000u;
+                    const uint32_t u2 = __float_as_uint(r1 - __uint_as_float(u1)) & 0xffff0000u;
+                    const uint32_t m0 = __float_as_uint(kLacks * __uint_as_float(u0));
+                    const uint32_t m1 = __float_as_uint(kLacks * __uint_as_float(u1));
+                    const uint32_t m2 = __float_as_uint(kLacks * __uint_as_float(u2));
+                    a2[ts][g4] = as_bf16x8((u0 >> 16) | u1, (u2 >> 16) | m0, (m1 >> 16) | m2, 0u);
+                }
+            }
+            // picks element q of four bf16 values in two registers, twice
+            const uint32_t sel_q = 0x01000100u + 0x02020202u * (uint32_t)q;
 
-    // ---- the wavefronts' partial sums meet in LDS: red[wave][token][row]; thread (token, row) adds them in wave order.  Behind
-    // what is staged, so that a wavefront need not wait before it puts its own there, or in its place (tok_lds_bytes) ----
-    float* red = reinterpret_cast<float*>(lds_raw + a.red_at);
-    if (a.red_at == 0) __syncthreads();
-    // D layout of the 16x16 MFMA: lane (n, q), register r -> token 4 q + r (of its set), weight row n
+            auto run_set = [&](auto rs_tag) {
+                constexpr int rs = decltype(rs_tag)::value, SL = rs % RING;
+                // scales, then biases, of the run's groups
+                uint4 sbv, bbv;
+                if constexpr (G32) {
+                    sbv = sbq[(rs * 16 + n) * sb_pitch + 2 * at];
+                    bbv = sbq[(rs * 16 + n) * sb_pitch + 2 * at + 1];
+                } else {
+                    sbv = sbq[(rs * 16 + n) * sb_pitch + at];
+                    bbv = make_uint4(sbv.z, sbv.w, 0u, 0u);
+                }
+                // the codes of a line: 4 bit the words of the set's eight steps, 8 bit the two words of each of four steps
+                // (8 bit, two sets of tokens, in groups of 32 or with eight sets of rows: both lines at once, so that the next set is
+                // requested before the first product; us, line by line / at once: 32 rows of 4096 x 14336 in groups of 32 22.0 / 21.7, of
+                // 2560 x (10240 | 10240) 24.0 / 22.2, of 14336 x 4096 22.0 / 21.2; but 32 rows of 4096 x 14336 in groups of 64 20.0 / 20.6,
+                // and one set of tokens, 4 rows, 14.6 / 15.3)
+                constexpr int HELD = TS == 2 && (G32 || RS == 8) ? LINES : 1;
+                uint32_t ww[8 * HELD];
+                auto fetch_line = [&](int ln) {
+                    const int w0 = ln % HELD * 8;
+                    const uint4 la = ring[SL][ln][0], lb = ring[SL][ln][1];
+                    if constexpr (BITS == 4) {
+                        unsigned char* const to = w_own + (n & 7) * kTokRowPitch + part16;
+                        order_wave_lds();  // (the last set's words have been read)
+                        *reinterpret_cast<uint4*>(to) = la;
+                        *reinterpret_cast<uint4*>(to + 8 * kTokRowPitch) = lb;
+                        order_wave_lds();  // the lines, and the sums above, are there for other lanes to read
+                        const unsigned char* const from = w_own + n * kTokRowPitch;
 #pragma unroll
-    for (int rs = 0; rs < RS; rs++)
+                        for (int i = 0; i < 8; i++) ww[i] = *reinterpret_cast<const uint32_t*>(from + i * 16 + q * 4);
+                    } else {
+                        // first 64 bytes of all 16 rows (lanes i >= 8 from the second load's lanes i - 8), second 64 bytes (lanes
+                        // i < 8 from the first load's lanes i + 8): as for x
+                        ww[w0] = __builtin_amdgcn_update_dpp(la.x, lb.x, 0x118, 0xf, 0xc, false);
+                        ww[w0 + 1] = __builtin_amdgcn_update_dpp(la.y, lb.y, 0x118, 0xf, 0xc, false);
+                        ww[w0 + 2] = __builtin_amdgcn_update_dpp(la.z, lb.z, 0x118, 0xf, 0xc, false);
+                        ww[w0 + 3] = __builtin_amdgcn_update_dpp(la.w, lb.w, 0x118, 0xf, 0xc, false);
+                        ww[w0 + 4] = __builtin_amdgcn_update_dpp(lb.x, la.x, 0x108, 0xf, 0x3, false);
+                        ww[w0 + 5] = __builtin_amdgcn_update_dpp(lb.y, la.y, 0x108, 0xf, 0x3, false);
+                        ww[w0 + 6] = __builtin_amdgcn_update_dpp(lb.z, la.z, 0x108, 0xf, 0x3, false);
+                        ww[w0 + 7] = __builtin_amdgcn_update_dpp(lb.w, la.w, 0x108, 0xf, 0x3, false);
+                        if constexpr (G32) {  // a step is one half of a block of 64: the second 8 codes of its lanes move across
 #pragma unroll
-        for (int ts = 0; ts < TS; ts++)
+                            for (int g = 0; g < 2; g++)
 #pragma unroll
-            for (int r = 0; r < 4; r++) red[(wave * 16 * TS + 16 * ts + 4 * q + r) * ROWS + rs * 16 + n] = acc[rs][ts][r];
-    __syncthreads();
-    auto total_of = [&](int t, int column) {
-        float total = red[t * ROWS + column];
+                                for (int k = 0; k < 2; k++) {
+                                    const auto p = __builtin_amdgcn_permlane32_swap(ww[w0 + 4 * g + k], ww[w0 + 4 * g + 2 + k], false, false);
+                                    ww[w0 + 4 * g + k] = p[0];
+                                    ww[w0 + 4 * g + 2 + k] = p[1];
+                                }
+                        }
+                    }
+                    if (ln == LINES - 1) {  // (into the registers that are free now)
+                        __builtin_amdgcn_sched_barrier(0);
+                        if constexpr (rs + RING < RS) issue_set(std::integral_constant<int, rs + RING>{}, run);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                };
+                f32x4_t part[TS], d[TS];
 #pragma unroll
-        for (int p = 1; p < NW; p++) total += red[(p * 16 * TS + t) * ROWS + column];
-        return total;
-    };
-    for (int o = tid; o < min(M, 16 * TS) * OUTS; o += NT) {
-        const int t = o / OUTS, rl = o - t * OUTS;
-        const int row = row0 + rl;
-        if (row >= N) continue;
-        float total = total_of(t, rl);
-        [[maybe_unused]] float up = PAIR ? total_of(t, OUTS + rl) : 0.0f;
-        if (!GROUPED && a.ksplit > 1) {
-            float* const dst = a.tile + ((size_t)split * a.M + m0 + t) * (size_t)(PAIRS * N);
-            dst[row] = total;
-            if constexpr (PAIR) dst[N + row] = up;
-            continue;
+                for (int ts = 0; ts < TS; ts++) part[ts] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+                auto step = [&](auto st_tag) {
+                    constexpr int st = decltype(st_tag)::value;
+                    if constexpr (st % (8 * HELD / LINES) == 0)
+#pragma unroll
+                        for (int ln = st * LINES / 8; ln < st * LINES / 8 + HELD; ln++) fetch_line(ln);
+                    uint32_t e[4];
+                    if constexpr (BITS == 4) {
+                        unpack4_codes(ww[st], e);
+                    } else {
+                        constexpr int w0 = 2 * (st % (4 * HELD));
+                        unpack8_centred(ww[w0], e);
+                        unpack8_centred(ww[w0 + 1], e + 2);
+                    }
+                    const bf16x8_t bop = as_bf16x8(e[0], e[1], e[2], e[3]);
+                    constexpr int g = st / (8 / GPR);
+                    constexpr bool begins = st % (8 / GPR) == 0, ends = (st + 1) % (8 / GPR) == 0;
+                    const uint32_t sw = g < 2 ? sbv.x : g < 4 ? sbv.y : g < 6 ? sbv.z : sbv.w;
+                    const float sc = (g & 1) ? __uint_as_float(sw & 0xffff0000u) : __uint_as_float(sw << 16);
+#pragma unroll
+                    for (int ts = 0; ts < TS; ts++) {
+                        f32x4_t from = {0.0f, 0.0f, 0.0f, 0.0f};
+                        if constexpr (FROM_SUM) from = *reinterpret_cast<const f32x4_t*>(sums_own + (ts * 8 + st) * 16 + 4 * q);
+                        d[ts] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[ts][st], bop, begins ? from : d[ts], 0, 0, 0);
+                        if (ends)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                float v = __builtin_fmaf(sc, d[ts][r], part[ts][r]);
+                                if constexpr (G32) asm volatile("" : "+v"(v));  // here, not behind all the steps: their products would be held until then
+                                part[ts][r] = v;
+                            }
+                    }
+                };
+                step(std::integral_constant<int, 0>{});
+                step(std::integral_constant<int, 1>{});
+                step(std::integral_constant<int, 2>{});
+                step(std::integral_constant<int, 3>{});
+                step(std::integral_constant<int, 4>{});
+                step(std::integral_constant<int, 5>{});
+                step(std::integral_constant<int, 6>{});
+                step(std::integral_constant<int, 7>{});
+#pragma unroll
+                for (int g4 = 0; g4 < GPR / 4; g4++) {
+                    const uint32_t bb = __builtin_amdgcn_perm(g4 ? bbv.w : bbv.y, g4 ? bbv.z : bbv.x, sel_q);
+                    const uint32_t ss = __builtin_amdgcn_perm(g4 ? sbv.w : sbv.y, g4 ? sbv.z : sbv.x, sel_q);
+                    const bf16x8_t b2 = as_bf16x8(bb, __builtin_amdgcn_perm(ss, bb, 0x05040100u), ss, 0u);
+#pragma unroll
+                    for (int ts = 0; ts < TS; ts++)
+                        part[ts] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[ts][g4], b2, part[ts], 0, 0, 0);
+                }
+#pragma unroll
+                for (int ts = 0; ts < TS; ts++)
+#pragma unroll
+                    for (int r = 0; r < 4; r++) acc[rs][ts][r] += part[ts][r];
+                __builtin_amdgcn_sched_barrier(0);
+            };
+            run_set(std::integral_constant<int, 0>{});
+            if constexpr (RS > 1) run_set(std::integral_constant<int, 1>{});
+            if constexpr (RS > 2) run_set(std::integral_constant<int, 2>{});
+            if constexpr (RS > 3) run_set(std::integral_constant<int, 3>{});
+            if constexpr (RS > 4) run_set(std::integral_constant<int, 4>{});
+            if constexpr (RS > 5) run_set(std::integral_constant<int, 5>{});
+            if constexpr (RS > 6) run_set(std::integral_constant<int, 6>{});
+            if constexpr (RS > 7) run_set(std::integral_constant<int, 7>{});
+            static_assert(RS <= 8 && RS % RING == 0, "sets of rows per workgroup");
         }
-        if constexpr (G32 && !GROUPED) {  // (dense groups of 32 keep what the any-width kernel makes of infinities)
+
+        if (!staged) stage();  // a wavefront without a run of its own
+
+        // ---- the wavefronts' partial sums meet in LDS: red[wave][token][row]; thread (token, row) adds them in wave order.  Behind
+        // what is staged, so that a wavefront need not wait before it puts its own there, or in its place (tok_lds_bytes) ----
+        if (a.red_at == 0) __syncthreads();
+        // D layout of the 16x16 MFMA: lane (n, q), register r -> token 4 q + r (of its set), weight row n
+#pragma unroll
+        for (int rs = 0; rs < RS; rs++)
+#pragma unroll
+            for (int ts = 0; ts < TS; ts++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) red[(wave * 16 * TS + 16 * ts + 4 * q + r) * ROWS + rs * 16 + n] = acc[rs][ts][r];
+        __syncthreads();
+        auto total_of = [&](int t, int column) {
+            float total = red[t * ROWS + column];
+#pragma unroll
+            for (int p = 1; p < NW; p++) total += red[(p * 16 * TS + t) * ROWS + column];
+            return total;
+        };
+        for (int o = tid; o < min(M, 16 * TS) * OUTS; o += NT) {
+            const int t = o / OUTS, rl = o - t * OUTS;
+            const int row = row0 + rl;
+            if (row >= N) continue;
+            float total = total_of(t, rl);
+            [[maybe_unused]] float up = PAIR ? total_of(t, OUTS + rl) : 0.0f;
+            if constexpr (INSIDE) {
+                if (share_from > 0) total = kept[o] + total;
+                if (share_end < runs) {
+                    kept[o] = total;
+                    continue;
+                }
+            }
+            if (!GROUPED && a.ksplit > 1) {
+                float* const dst = a.tile + ((size_t)split * a.M + m0 + t) * (size_t)(PAIRS * N);
+                dst[row] = total;
+                if constexpr (PAIR) dst[N + row] = up;
+                continue;
+            }
+            if constexpr (G32 && !GROUPED) {  // (dense groups of 32 keep what the any-width kernel makes of infinities)
 #pragma nounroll
-            for (int part = 0; part < PAIRS; part++) {
-                if (!not_finite(part ? up : total)) continue;
-                const float v = plain_dot_g32(a.x + (size_t)(m0 + t) * K, (PAIR && part ? a.w2 : a.w) + (size_t)row * (row_bytes / 4),
-                                              (PAIR && part ? a.s2 : a.s) + (size_t)row * groups, (PAIR && part ? a.b2 : a.b) + (size_t)row * groups, K, BITS);
-                if (part) up = v; else total = v;
+                for (int part = 0; part < PAIRS; part++) {
+                    if (!not_finite(part ? up : total)) continue;
+                    const float v = plain_dot_g32(a.x + (size_t)(m0 + t) * K, (PAIR && part ? a.w2 : a.w) + (size_t)row * (row_bytes / 4),
+                                                  (PAIR && part ? a.s2 : a.s) + (size_t)row * groups, (PAIR && part ? a.b2 : a.b) + (size_t)row * groups, K, BITS);
+                    if (part) up = v; else total = v;
+                }
+            }
+            if constexpr (PAIR) total = fmul_unfused(act_value(a.act, total), up);
+            size_t y_row = (size_t)(m0 + t);
+            if constexpr (GROUPED) {
+                const int route = a.route_of[first_route + t];
+                if (route < 0) total = 0.0f;  // an expert id or a row of x out of range
+                y_row = (size_t)(route & INT32_MAX);
+            }
+            const size_t at = y_row * N + row;
+            if (a.out_f32) {
+                static_cast<float*>(a.y)[at] = total;
+            } else {
+                static_cast<uint16_t*>(a.y)[at] = f32_to_bf16_bits(total);
             }
         }
-        if constexpr (PAIR) total = fmul_unfused(act_value(a.act, total), up);
-        size_t y_row = (size_t)(m0 + t);
-        if constexpr (GROUPED) {
-            const int route = a.route_of[first_route + t];
-            if (route < 0) total = 0.0f;  // an expert id or a row of x out of range
-            y_row = (size_t)(route & INT32_MAX);
-        }
-        const size_t at = y_row * N + row;
-        if (a.out_f32) {
-            static_cast<float*>(a.y)[at] = total;
-        } else {
-            static_cast<uint16_t*>(a.y)[at] = f32_to_bf16_bits(total);
-        }
+        if (!INSIDE || share_end >= runs) break;
+        share_from = share_end;
+        share_end = min(runs, share_end + a.share);
+#pragma unroll
+        for (int rs = 0; rs < RS; rs++)
+#pragma unroll
+            for (int ts = 0; ts < TS; ts++) acc[rs][ts] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        __syncthreads();  // the last share's sums have been read
     }
 }
 
@@ -615,9 +638,10 @@ __global__ __launch_bounds__(kTokWaves* kWave) void qmv_tok16_multi_kernel(const
     a.N = ma.N[i];
     a.ksplit = ma.ksplit[i];
     a.share = ma.share[i];
+    a.inside = ma.inside[i];
     a.tile = ma.tile[i];
     a.red_at = ma.red_at;
-    qmv_tok16_body<BITS, RS, RING, TS, GRP, false, false>(a, (int)blockIdx.x - before);
+    qmv_tok16_body<BITS, RS, RING, TS, GRP, false, false, RS <= kTokInsideSets>(a, (int)blockIdx.x - before);
 }
 
 // ---- kernels of one code width -------------------------------------------------------------------------------------

@@ -22,10 +22,15 @@ static int tok_runs_of(const TokArgs& a) { return a.ksplit > 1 ? a.share : (a.K 
 // LDS of a workgroup whose longest share is `runs` runs.  The wavefronts' sums meet behind what is staged (red_at) where that costs no
 // workgroup of a CU, else in its place, behind a barrier (us, in its place / behind: 4 / 16 / 32 rows of 4096 x 14336, 8 bit 14.6 /
 // 16.3 / 20.2 against 14.4 / 16.1 / 19.9, 4 bit 16 / 32 rows 11.6 / 16.3 against 11.5 / 16.1).
-static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs, uint32_t* red_at = nullptr) {
+// (inside: the sums of shares that a workgroup works through by itself lie behind, for the scales are needed again)
+static size_t tok_lds_bytes(const QmvTokEntry& e, bool g32, int runs, uint32_t* red_at = nullptr, bool inside = false) {
     const size_t staged = tok_sb_bytes(g32, e.wg_rows, runs) + (size_t)kTokWaves * tok_own_bytes(e.v.bits, g32, e.ts);
     const size_t sums = (size_t)kTokWaves * 16 * e.ts * e.wg_rows * 4, cu = 160 * 1024;
     const int of_a_cu = e.v.rows * e.ts <= 2 ? 2 : 1;  // workgroups that a CU's registers hold
+    if (inside) {
+        if (red_at) *red_at = (uint32_t)staged;
+        return staged + sums + sums / kTokWaves;
+    }
     const bool behind = staged + sums <= cu / of_a_cu;
     if (red_at) *red_at = behind ? (uint32_t)staged : 0;
     return behind ? staged + sums : staged > sums ? staged : sums;
@@ -45,7 +50,7 @@ bool qmvt_fits(const TokArgs& a, int bits, int group_size, int idx, bool exact_o
                          reinterpret_cast<uintptr_t>(a.b2);
     const bool exact = tok_whole_runs(a) && (sb & 7) == 0;
     if (!exact && (exact_only || (sb & 15))) return false;
-    return tok_lds_bytes(tok_entry(idx), group_size == 32, tok_runs_of(a)) <= 160 * 1024;
+    return tok_lds_bytes(tok_entry(idx), group_size == 32, tok_runs_of(a), nullptr, a.inside > 1) <= 160 * 1024;
 }
 
 const char* qmvt_name(int idx, const TokArgs& a) { return tok_entry(idx).name[a.gs_shift == 5 ? 2 : tok_whole_runs(a) ? 0 : 1]; }
@@ -109,20 +114,22 @@ hipError_t qmvt_multi_launch(int idx, TokMultiArgs ma, int bits, hipStream_t str
     r.gs_shift = ma.common.gs_shift;
     r.out_f32 = ma.common.out_f32;
     r.count = ma.count;
-    bool split = false;
+    bool split = false, inside = false;
     for (int i = 0; i < ma.count; i++) {
         blocks += tok_blocks(e, ma.common.M, ma.tokens, ma.N[i], false, ma.ksplit[i]);
         ma.block_end[i] = blocks;
         const int n = ma.ksplit[i] > 1 ? ma.share[i] : (ma.common.K + 255) / 256;
         runs = n > runs ? n : runs;
         split |= ma.ksplit[i] > 1;
+        inside |= ma.inside[i] > 1;
         r.w[i] = ma.w[i], r.s[i] = ma.s[i], r.b[i] = ma.b[i];
         r.y[i] = ma.y[i];
         r.N[i] = ma.N[i];
         r.ksplit[i] = ma.ksplit[i];
         r.tile[i] = ma.ksplit[i] > 1 ? ma.tile[i] : nullptr;
     }
-    const size_t lds = tok_lds_bytes(e, g32, runs, &ma.red_at);
+    const size_t lds = tok_lds_bytes(e, g32, runs, &ma.red_at, inside);
+    if (lds > 160 * 1024 || (inside && e.v.rows > kTokInsideSets)) return hipErrorInvalidValue;
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     hipLaunchKernelGGL(fn, dim3((unsigned)blocks), dim3((unsigned)(e.v.waves * kWave)), lds, stream, ma);
     if (hipError_t rc = hipGetLastError()) return rc;
@@ -173,6 +180,7 @@ size_t qmvt_tile_bytes(int M, int N, bool pair, int ksplit) {
 struct TokCost {
     double fixed, pass, set;
 };
+constexpr double kMeetFixed = 0.4, kMeetSet = 0.15;  // a meeting in LDS between shares that a workgroup works through by itself
 static const TokCost& tok_cost(int bits, int group_size, int tokens) {
     // [8 bit][groups of 32][more than 16 rows of x]
     static const TokCost kCost[2][2][2] = {{{{2.6, 1.25, 0.72}, {2.8, 2.5, 0.89}}, {{3.0, 1.13, 0.93}, {3.85, 2.1, 1.43}}},
@@ -183,18 +191,23 @@ static const TokCost& tok_cost(int bits, int group_size, int tokens) {
 static double tok_passes(int runs) {
     return runs > kTokWaves ? 0.5 * ((runs + kTokWaves - 1) / kTokWaves + (double)runs / kTokWaves) : 1.0;
 }
+static double tok_time(const TokCost& c, int rs, const TokPart& p, int K) {
+    if (p.inside <= 1) return tok_passes(p.runs) * (c.pass + rs * c.set);
+    const int last = (K + 255) / 256 - (p.inside - 1) * p.runs;
+    return ((p.inside - 1) * tok_passes(p.runs) + tok_passes(last)) * (c.pass + rs * c.set) + (p.inside - 1) * (kMeetFixed + kMeetSet * rs);
+}
 // When the last CU is done with these matrices on `rs` sets a workgroup, one workgroup a CU at a time, in the order of the grid.
-static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count, int parts_of_x, int cus) {
+static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count, int K, int parts_of_x, int cus) {
     struct Level {  // CUs that are free at a time, earliest first
         double at;
         int64_t cus;
     };
     if (count == 1)
-        return (double)(((parts[0].sets + rs - 1) / rs * parts[0].shares * parts_of_x + cus - 1) / cus) * tok_passes(parts[0].runs) * (c.pass + rs * c.set);
+        return (double)(((parts[0].sets + rs - 1) / rs * parts[0].shares * parts_of_x + cus - 1) / cus) * tok_time(c, rs, parts[0], K);
     Level levels[4 * kQmvMultiMax] = {{0.0, cus}};
     int n = 1;
     for (int i = 0; i < count; i++) {
-        const double t = tok_passes(parts[i].runs) * (c.pass + rs * c.set);
+        const double t = tok_time(c, rs, parts[i], K);
         int64_t groups = (parts[i].sets + rs - 1) / rs * parts[i].shares * parts_of_x;
         while (groups > 0) {
             if (n == 1) {  // whole rounds
@@ -227,11 +240,13 @@ static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count
 // four, eight sets; 24 rows of x, K = 2816, groups of 64: 4096 rows of weights 8.3 / 9.6 / 11.9 / 17.2, 8192 15.1 / 10.0 / 12.1 /
 // 17.2, 14336 27.9 / 18.1 / 12.3 / 17.4, 2 x 14336 35.1 / 23.9 / 18.3 from two on); fewer where a second round would be nearly empty,
 // and where members of a grid differ in length, so that the ones that are not shared out do not outlast the rest.
-static int tok_sets(const TokCost& c, const TokPart* parts, int count, int parts_of_x, int cus, double* us = nullptr) {
+static int tok_sets(const TokCost& c, const TokPart* parts, int count, int K, int parts_of_x, int cus, double* us = nullptr) {
     double best = 1e30;
-    int best_rs = 1;
-    for (int rs = 1; rs <= 8; rs *= 2) {
-        const double t = tok_span(c, rs, parts, count, parts_of_x, cus);
+    int best_rs = 1, most = 8;
+    for (int i = 0; i < count; i++)
+        if (parts[i].inside > 1) most = kTokInsideSets;
+    for (int rs = 1; rs <= most; rs *= 2) {
+        const double t = tok_span(c, rs, parts, count, K, parts_of_x, cus);
         if (t < best) best = t, best_rs = rs;
     }
     if (us) *us = c.fixed + best;
@@ -259,9 +274,9 @@ void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu
         for (const int rows : {12, 24, 48}) {
             if ((rows > 32) != (M > 32)) continue;
             const int tokens = qmvt_tokens(rows);
-            const TokPart part{(int64_t)((N + 15) / 16) * (pair ? 2 : 1), n, sh};
+            const TokPart part{(int64_t)((N + 15) / 16) * (pair ? 2 : 1), n, sh, 0};
             double us;
-            tok_sets(tok_cost(bits, group_size, tokens), &part, 1, (rows + tokens - 1) / tokens, cus, &us);
+            tok_sets(tok_cost(bits, group_size, tokens), &part, 1, K, (rows + tokens - 1) / tokens, cus, &us);
             // (a tenth: no shares for next to nothing, see above)
             if (n > 1) us = (M <= 32 ? 1.1 : 1.0) * us + 2.5 + (double)qmvt_tile_bytes(rows, N, pair, n) / 1e6;
             sum += us;
@@ -271,16 +286,21 @@ void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu
     }
 }
 
-int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count) {
+int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count, double* us) {
     if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK || count < 1) return -1;
     const int cus = cu_count > 0 ? cu_count : 256, tokens = qmvt_tokens(M), most = tokens <= 16 ? 16 : 32;
-    int rs = tok_sets(tok_cost(bits, group_size, tokens), parts, count, (M + tokens - 1) / tokens, cus), runs = 1;
+    int rs = tok_sets(tok_cost(bits, group_size, tokens), parts, count, K, (M + tokens - 1) / tokens, cus, us), runs = 1;
     if (pair && rs == 1) rs = 2;
-    for (int i = 0; i < count; i++) runs = parts[i].runs > runs ? parts[i].runs : runs;
+    bool inside = false;
+    for (int i = 0; i < count; i++) {
+        const int n = parts[i].inside > 1 ? (K + 255) / 256 : parts[i].runs;
+        runs = n > runs ? n : runs;
+        inside |= parts[i].inside > 1;
+    }
     for (int i = 0; i < qmvt_variant_count(); i++) {  // (listed with eight, four, two, one sets)
         const QmvTokEntry& e = tok_entry(i);
         if (e.v.bits != bits || e.v.m != most || e.v.rows > rs) continue;
-        if (tok_lds_bytes(e, group_size == 32, runs) <= 160 * 1024) return i;
+        if (tok_lds_bytes(e, group_size == 32, runs, nullptr, inside) <= 160 * 1024) return i;
     }
     return -1;
 }

@@ -249,6 +249,24 @@ static void test_shares() {
     CHECK(tiles_hi - tiles_lo <= aq::kTokTileBytes, "partial tiles over %zu bytes", (size_t)(tiles_hi - tiles_lo));
 }
 
+// Members of a grid that fills the chip work through their shares by themselves: no tiles, no second launch.
+static void test_shares_inside() {
+    struct Case {
+        int bits, group, M, K, N[3];
+    };
+    static const Case cases[] = {{4, 64, 9, 5376, {4096, 2048, 2048}}, {8, 64, 32, 5312, {2047, 4090, 2048}}, {8, 32, 8, 5376, {4096, 2048, 2048}},
+                                 {4, 32, 21, 5376, {4096, 2048, 2048}}, {8, 32, 21, 5376, {4096, 2048, 2048}}, {4, 32, 21, 6144, {1024, 6144, 1001}}};
+    for (const Case& c : cases) {
+        const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+        void* y[3] = {Y, Y, Y};
+        log_.clear();
+        CHECK(aq_qmv_multi(ctx, X, 3, w, s, b, y, c.N, c.M, c.K, c.group, c.bits, 0) == AQ_OK, "%s", aq_last_error());
+        int inside = 0;
+        for (const int n : log_[0].multi.inside) inside += n > 1;
+        CHECK(log_.size() == 1 && inside > 0, "%d rows of %d: %zu launches, %d members with shares of their own", c.M, c.K, log_.size(), inside);
+    }
+}
+
 // The calls that tests/test_gpu_group32_infinities.py makes for the launch that adds partial tiles.
 static void test_shares_of_the_infinities() {
     auto tiles = [](int i) { return i < (int)log_.size() && log_[i].is("tok_reduce"); };
@@ -281,7 +299,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole(), test_shares_of_the_infinities();
+        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_the_infinities();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");

@@ -154,7 +154,7 @@ def test_gated_pair_in_shares(ctx, bits, M, K, N):
         t.free()
 
 
-@pytest.mark.parametrize("M,K,Ns", [(21, 5120, (12000, 100, 64)), (40, 5120, (6000, 600)), (21, 15360, (130, 65, 1))])
+@pytest.mark.parametrize("M,K,Ns", [(21, 5120, (12000, 100, 64)), (40, 5120, (6000, 600)), (21, 15360, (130, 65, 1)), (21, 5376, (4096, 2048, 2048))])
 @pytest.mark.parametrize("bits", [4, 8])
 def test_members_in_shares(ctx, bits, M, K, Ns):
     import aq_mi355

@@ -42,7 +42,8 @@ def test_sums(ctx, bits, gs, M, K, N):
 
 
 @pytest.mark.parametrize("bits,gs,M,K,Ns", [(4, 64, 12, 14336, (1000, 17, 4096)), (4, 64, 24, 8192, (2048, 530)), (4, 32, 21, 15360, (130, 64, 1)),
-                                            (8, 64, 20, 9728, (512, 96)), (4, 64, 48, 4096, (1000, 530)), (8, 32, 33, 1024, (600, 700, 540))])
+                                            (8, 64, 20, 9728, (512, 96)), (4, 64, 9, 5376, (4096, 2048, 2048)), (8, 64, 32, 5312, (2047, 4090, 2048)),
+                                            (4, 32, 21, 6144, (1024, 6144, 1001)), (8, 32, 8, 5376, (4096, 2048, 2048)), (4, 128, 17, 8192, (8192, 1024)), (4, 64, 48, 4096, (1000, 530)), (8, 32, 33, 1024, (600, 700, 540))])
 def test_members_have_the_bytes_of_their_own_calls(ctx, bits, gs, M, K, Ns):
     import aq_mi355
     say("token tile shares, members", bits, gs, M, K, Ns)
