@@ -240,12 +240,13 @@ static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count
 // four, eight sets; 24 rows of x, K = 2816, groups of 64: 4096 rows of weights 8.3 / 9.6 / 11.9 / 17.2, 8192 15.1 / 10.0 / 12.1 /
 // 17.2, 14336 27.9 / 18.1 / 12.3 / 17.4, 2 x 14336 35.1 / 23.9 / 18.3 from two on); fewer where a second round would be nearly empty,
 // and where members of a grid differ in length, so that the ones that are not shared out do not outlast the rest.
-static int tok_sets(const TokCost& c, const TokPart* parts, int count, int K, int parts_of_x, int cus, double* us = nullptr) {
+// (a pair has two or more, one of each matrix)
+static int tok_sets(const TokCost& c, const TokPart* parts, int count, int K, int parts_of_x, bool pair, int cus, double* us = nullptr) {
     double best = 1e30;
     int best_rs = 1, most = 8;
     for (int i = 0; i < count; i++)
         if (parts[i].inside > 1) most = kTokInsideSets;
-    for (int rs = 1; rs <= most; rs *= 2) {
+    for (int rs = pair ? 2 : 1; rs <= most; rs *= 2) {
         const double t = tok_span(c, rs, parts, count, K, parts_of_x, cus);
         if (t < best) best = t, best_rs = rs;
     }
@@ -276,7 +277,7 @@ void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu
             const int tokens = qmvt_tokens(rows);
             const TokPart part{(int64_t)((N + 15) / 16) * (pair ? 2 : 1), n, sh, 0};
             double us;
-            tok_sets(tok_cost(bits, group_size, tokens), &part, 1, K, (rows + tokens - 1) / tokens, cus, &us);
+            tok_sets(tok_cost(bits, group_size, tokens), &part, 1, K, (rows + tokens - 1) / tokens, pair, cus, &us);
             // (a tenth: no shares for next to nothing, see above)
             if (n > 1) us = (M <= 32 ? 1.1 : 1.0) * us + 2.5 + (double)qmvt_tile_bytes(rows, N, pair, n) / 1e6;
             sum += us;
@@ -289,8 +290,7 @@ void qmvt_split(int bits, int group_size, int M, int K, int N, bool pair, int cu
 int qmvt_pick(int bits, int group_size, int M, int K, const TokPart* parts, int count, bool pair, int cu_count, double* us) {
     if (M < 1 || M > kTokMax || K < 64 || K % 64 != 0 || K > kTokMaxK || count < 1) return -1;
     const int cus = cu_count > 0 ? cu_count : 256, tokens = qmvt_tokens(M), most = tokens <= 16 ? 16 : 32;
-    int rs = tok_sets(tok_cost(bits, group_size, tokens), parts, count, K, (M + tokens - 1) / tokens, cus, us), runs = 1;
-    if (pair && rs == 1) rs = 2;
+    int rs = tok_sets(tok_cost(bits, group_size, tokens), parts, count, K, (M + tokens - 1) / tokens, pair, cus, us), runs = 1;
     bool inside = false;
     for (int i = 0; i < count; i++) {
         const int n = parts[i].inside > 1 ? (K + 255) / 256 : parts[i].runs;

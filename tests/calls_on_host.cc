@@ -267,6 +267,15 @@ static void test_shares_inside() {
     }
 }
 
+// A pair has two sets of rows a workgroup or more: what one would take is no reason to leave K whole.
+static void test_shares_of_pairs() {
+    for (auto [bits, M, K, N] : {std::array{8, 32, 6208, 1920}, {4, 24, 6208, 1920}, {8, 9, 5120, 2048}}) {
+        log_.clear();
+        CHECK(aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, M, K, N, 64, bits, AQ_ACT_SILU, 0) == AQ_OK, "%s", aq_last_error());
+        CHECK(log_.size() == 2 && log_[1].is("tok_reduce"), "gate|up, %d bit, %d x %d x %d: %zu launches", bits, M, K, N, log_.size());
+    }
+}
+
 // The calls that tests/test_gpu_group32_infinities.py makes for the launch that adds partial tiles.
 static void test_shares_of_the_infinities() {
     auto tiles = [](int i) { return i < (int)log_.size() && log_[i].is("tok_reduce"); };
@@ -299,7 +308,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_the_infinities();
+        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");
