@@ -204,11 +204,15 @@ static double tok_span(const TokCost& c, int rs, const TokPart* parts, int count
     };
     if (count == 1)
         return (double)(((parts[0].sets + rs - 1) / rs * parts[0].shares * parts_of_x + cus - 1) / cus) * tok_time(c, rs, parts[0], K);
+    // Halves of the rows of x: the two workgroups of a band are on one XCD, and every member begins at the first, which therefore has
+    // the most of them (64 rows of 9600 x (5248 | 1344 | 1344): 248 workgroups, but 34 of them on the 32 CUs there, 74 us for 37)
+    const int xcds = parts_of_x > 1 ? 8 : 1;
+    cus = cus > xcds ? cus / xcds : 1;
     Level levels[4 * kQmvMultiMax] = {{0.0, cus}};
     int n = 1;
     for (int i = 0; i < count; i++) {
         const double t = tok_time(c, rs, parts[i], K);
-        int64_t groups = (parts[i].sets + rs - 1) / rs * parts[i].shares * parts_of_x;
+        int64_t groups = ((parts[i].sets + rs - 1) / rs * parts[i].shares + xcds - 1) / xcds * parts_of_x;
         while (groups > 0) {
             if (n == 1) {  // whole rounds
                 levels[0].at += (double)(groups / cus) * t;

@@ -265,6 +265,15 @@ static void test_shares_inside() {
         for (const int n : log_[0].multi.inside) inside += n > 1;
         CHECK(log_.size() == 1 && inside > 0, "%d rows of %d: %zu launches, %d members with shares of their own", c.M, c.K, log_.size(), inside);
     }
+    // Halves of 64 rows: bands of all members begin on the first XCD, whose CUs would have two of these workgroups after another.
+    for (auto [group, K, wide, narrow] : {std::array{64, 9600, 5248, 1344}, {128, 13568, 6272, 832}}) {
+        const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+        void* y[3] = {Y, Y, Y};
+        const int N[3] = {wide, narrow, narrow};
+        log_.clear();
+        CHECK(aq_qmv_multi(ctx, X, 3, w, s, b, y, N, 64, K, group, 4, 0) == AQ_OK, "%s", aq_last_error());
+        CHECK(log_.size() == 2 && log_[1].is("tok_reduce"), "64 rows of %d: %zu launches", K, log_.size());
+    }
 }
 
 // A pair has two sets of rows a workgroup or more: what one would take is no reason to leave K whole.
