@@ -44,14 +44,12 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 constexpr uint32_t kMaskH = 0x03C003C0u;   // a nibble moved to fp16 mantissa bits [9:6]
 constexpr uint32_t kMagicH = 0x4C004C00u;  // fp16 16.0 in both halves: 16 + code, exact
 
-// 8 codes of one packed word -> 8 fp16 values s * (code - 8) in slot order (c0,c4)(c1,c5)(c2,c6)(c3,c7)
-__device__ __forceinline__ uint4 expand_word(uint32_t w, uint32_t mask_s, uint32_t magic_v, f16x2_t s2, f16x2_t m24) {
-    uint4 v;
-    v.x = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_or(w << 6, mask_s, magic_v)), s2, m24));
-    v.y = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_or(w << 2, mask_s, magic_v)), s2, m24));
-    v.z = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_or(w >> 2, mask_s, magic_v)), s2, m24));
-    v.w = __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_or(w >> 6, mask_s, magic_v)), s2, m24));
-    return v;
+// Pair I (codes I and I + 4) of a packed word -> fp16 values s * (code - 8); the pairs of a word in order are its slot order
+// (c0,c4)(c1,c5)(c2,c6)(c3,c7)
+template <int I>
+__device__ __forceinline__ uint32_t expand_pair(uint32_t w, uint32_t mask_s, uint32_t magic_v, f16x2_t s2, f16x2_t m24) {
+    const uint32_t at = I == 0 ? w << 6 : I == 1 ? w << 2 : I == 2 ? w >> 2 : w >> 6;
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_or(at, mask_s, magic_v)), s2, m24));
 }
 
 // 8 codes of two packed words of 8-bit codes -> 8 fp16 values code - 128 in their natural order: the bytes go into the
@@ -80,6 +78,37 @@ __device__ __forceinline__ float lane_xor(float v) {
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
+}
+
+// Elements off .. off + 7 of an array of `total`; what lies past its end is anything.  Rows of scales start at any even address
+// (K of 704: 22 bytes a row), and one 16-byte load from there beats eight of two bytes, each of which touches as many lines.
+// load_eight reads eight elements that lie inside the array, moved_down brings the asked for to the front.  (TINY: an array of
+// fewer than eight.)
+typedef uint32_t u32x4_at2_t __attribute__((ext_vector_type(4), aligned(2)));
+template <bool TINY>
+__device__ __forceinline__ uint4 load_eight(const uint16_t* base, uint32_t off, uint32_t total) {
+    if constexpr (TINY) {
+        uint64_t lo = 0, hi = 0;
+#pragma nounroll
+        for (uint32_t i = 0; i < 4; i++) {
+            lo |= (uint64_t)base[min(off + i, total - 1)] << (16 * i);
+            hi |= (uint64_t)base[min(off + 4 + i, total - 1)] << (16 * i);
+        }
+        return make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+    }
+    const u32x4_at2_t v = *reinterpret_cast<const u32x4_at2_t*>(base + min(off, total - 8));
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+__device__ __forceinline__ uint4 moved_down(uint4 v, uint32_t off, uint32_t total) {
+    const uint32_t by = total >= 8 && off > total - 8 ? min(off - (total - 8), 7u) : 0u;
+    v.x = by & 4 ? v.z : v.x;
+    v.y = by & 4 ? v.w : v.y;
+    v.x = by & 2 ? v.y : v.x;
+    v.y = by & 2 ? v.z : v.y;
+    v.z = by & 2 ? v.w : v.z;
+    const uint32_t half = (by & 1) * 16;
+    return make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, half), __builtin_amdgcn_alignbit(v.z, v.y, half), __builtin_amdgcn_alignbit(v.w, v.z, half),
+                      v.w >> half);
 }
 
 __device__ __forceinline__ uint32_t dup16(uint32_t h) { return (h & 0xffffu) | (h << 16); }
@@ -209,7 +238,7 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
             hv[2 * i] = (_Float16)(bf16_bits_to_f32(w[i] & 0xffffu) * up);
             hv[2 * i + 1] = (_Float16)(bf16_bits_to_f32(w[i] >> 16) * up);
         }
-        // slot order (x0,x4)(x1,x5)(x2,x6)(x3,x7): the order in which expand_word emits the codes of a word
+        // slot order (x0,x4)(x1,x5)(x2,x6)(x3,x7): the order in which expand_pair emits the codes of a word
         const f16x8_t o = BITS == 4 ? f16x8_t{hv[0], hv[4], hv[1], hv[5], hv[2], hv[6], hv[3], hv[7]}
                                     : f16x8_t{hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], hv[6], hv[7]};
         const int t = BITS == 4 ? c8 & 3 : c8 >> 1, h = BITS == 4 ? c8 >> 2 : c8 & 1;
@@ -278,14 +307,16 @@ __device__ __forceinline__ void fix_output(const QmmHalfArgs& a, const QmmSegmen
 // rows (1472 / 4032) 274 -> 125, of 300 rows in groups of 32 (2048 / 8192) 24.7 ms on the any-width kernel -> 159, 512 tokens
 // through 128 experts (2816 / 704) 3692 -> 314.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
 // instructions of expansion and 64 of scaling; a block takes 0.72 us of a CU for 0.23 us of matrix pipe.
-template <int BITS, int MB, int NB, int WM, int WN, int STAGES, int OCC, bool SPREAD, int GRP>
-__global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfArgs a) {
+// Scales and biases go through LDS as well, SE of each row at a time (a segment).  Loaded by the lanes that use them, four blocks at
+// a time, every load touched a line per row, in either wavefront row again: as many lines as the copies of A and of the packed
+// weights together.
+template <int BITS, int MB, int NB, int WM, int WN, int STAGES, int SE, int GRP>
+__global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArgs a) {
     constexpr bool G32 = GRP == 32;
     constexpr bool B8 = BITS == 8;
     constexpr float CENTRE = B8 ? 128.0f : 8.0f;  // the operand's codes are code - CENTRE
     static_assert(NB == 2, "a pair is two column blocks");
     static_assert(STAGES == 2 || STAGES == 3 || STAGES == 4, "LDS stages");
-    constexpr int AHEAD = STAGES - 1;  // iteration g requests block g + AHEAD
     constexpr int BM = WM * MB * 32;
     constexpr int BN = WN * NB * 32;
     constexpr int NWAVE = WM * WN;
@@ -300,17 +331,22 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     constexpr int NBC = B_STAGE / 1024 / NWAVE;  // B copies a wavefront issues per stage
     static_assert(A_BLOCKS % NWAVE == 0, "A fragments must divide among the wavefronts");
     static_assert(B_STAGE % (1024 * NWAVE) == 0 && NBC >= 1, "weight pieces must divide among the wavefronts");
+    constexpr bool XS_LDS = !B8 && MB >= 3;  // the sums of x of a quad go through LDS
+    constexpr int NX = (BM / 32 + NWAVE - 1) / NWAVE;  // copies of them a wavefront issues
     constexpr int NA = A_BLOCKS / NWAVE;  // A copies a wavefront issues per block
-    // B's next stage is issued in a stage's first block, behind that iteration's A copies.  still_out: the copies that may be
-    // on their way at the end of the iteration of block Q of a quad, which are those newer than A of the next block, and in a
-    // stage's second block none of B's.
-    static_assert(AHEAD <= 2, "waits are counted for one or two blocks ahead");
-    // BITS 8: iteration g requests A and B of block g + AHEAD.
-    auto still_out = [=](int q) constexpr { return B8 ? (AHEAD - 1) * (NA + NBC) : (AHEAD - 1) * NA + ((q & 1) == 0 ? NBC : 0); };
+    // Behind the barrier of block g the copies of A's block g + STAGES are issued.  BITS 4: and, in a stage's first block, those of B's
+    // stage after the next, two blocks before its codes are read; BITS 8: and B's block g + STAGES.  still_out: the copies that may
+    // be on their way at the barrier of block Q of a quad: A of block g + 1 has to have landed and with it the codes that are
+    // read up to the next barrier.
+    static_assert(STAGES <= 3, "waits are counted for two or three stages");
+    auto still_out = [=](int q) constexpr {
+        return B8 ? (STAGES - 2) * (NA + NBC) : (STAGES - 2) * NA + ((q & 1) ? NBC : 0) + (XS_LDS && q == 1 ? NX : 0);
+    };
 
     extern __shared__ __align__(16) uint8_t lds[];
     uint8_t* const abuf = lds;                     // [STAGES][A_STAGE]
     uint8_t* const bbuf = lds + STAGES * A_STAGE;  // [B_BUFS][B_STAGE]
+    uint16_t* const sbuf = reinterpret_cast<uint16_t*>(bbuf + B_BUFS * B_STAGE);  // [scales, biases][BN][SE]
     // the same as LDS byte addresses: the copy instructions take theirs from a scalar register, and plain integer
     // arithmetic keeps it on the scalar unit (a pointer would be converted, null check included, per copy)
     const uint32_t abuf_at = __builtin_amdgcn_readfirstlane(lds_offset(lds));
@@ -349,8 +385,8 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
 
     const int K = a.K, N = a.seg[seg].N;
     const int Gall = K / 64;
-    const int gb = split * a.seg[seg].gsplit;         // first block of K this workgroup multiplies (a multiple of 4)
-    const int G = min(Gall, gb + a.seg[seg].gsplit);  // one past its last block
+    const int gb = __builtin_amdgcn_readfirstlane(split * a.seg[seg].gsplit);  // first block of K this workgroup multiplies (a multiple of 4)
+    const int G = __builtin_amdgcn_readfirstlane(min(Gall, gb + a.seg[seg].gsplit));  // one past its last block
     const int G4 = (Gall + 3) / 4;
     const int ksteps = K / 16;
     const int sb_per_row = G32 ? Gall * 2 : Gall / a.gs_blocks;
@@ -397,13 +433,13 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         wpiece[c] = (uint32_t)((lane % PPR) ^ turn(r)) * 16u;
     }
     // copy c of stage st (64-code blocks QB * st ..) into buffer `buf`
-    auto issue_b = [&](int c, int st, int buf) {
+    auto issue_b = [&](int c, int st, int buf) __attribute__((always_inline)) {
         const uint32_t in_row = min((uint32_t)(st * B_ROW) + wpiece[c], row_bytes - 16u);
         const int block = (c * NWAVE + wave) * RPI >> 5;
         copy16_to_lds((block & 1) ? wtile2 : wtile1, wrow[c] + in_row, bbuf_at + (uint32_t)(buf * B_STAGE + (c * NWAVE + wave) * 1024));
     };
     // copy c of A's block g
-    auto issue_a1 = [&](int c, int g, int stage) {
+    auto issue_a1 = [&](int c, int g, int stage) __attribute__((always_inline)) {
         const int blk = wave + c * NWAVE;
         int mblk = m0 / 32 + (blk >> 2);
         mblk = mblk < a.mblks ? mblk : a.mblks - 1;  // past the end: any valid rows, never stored
@@ -415,9 +451,11 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
     // the first blocks are on their way while the prologue scans the scale rows
     if constexpr (!B8)
 #pragma unroll
-        for (int c = 0; c < NBC; c++) issue_b(c, gb / QB, 0);
+        for (int st = 0; st < 2; st++)
 #pragma unroll
-    for (int d = 0; d < AHEAD; d++) {
+            for (int c = 0; c < NBC; c++) issue_b(c, min(gb / QB + st, (Gall - 1) / QB), st);
+#pragma unroll
+    for (int d = 0; d < STAGES; d++) {
 #pragma unroll
         for (int c = 0; c < NA; c++) issue_a1(c, gb + d < G ? gb + d : G - 1, d);
         if constexpr (B8)
@@ -425,76 +463,135 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
             for (int c = 0; c < NBC; c++) issue_b(c, gb + d < G ? gb + d : G - 1, d);
     }
 
-    // this lane's weight rows (one per column block), and the power of two that brings the row's largest scale (of this
-    // workgroup's range of K) into [2^10, 2^11): lane half h scans its half of the row's scales
-    uint32_t sboff[NB];  // element offset of the row's scales (and biases): a 32-bit lane part next to a uniform base
-    float col_up[NB];
-#pragma unroll
-    for (int nb = 0; nb < NB; nb++) {
-        const uint16_t* const sbase = nb ? sb2[0] : sb1[0];
-        const int n = weight_row(wave_n, nb, j);
-        sboff[nb] = (uint32_t)n * (uint32_t)sb_per_row;
-        if constexpr (B8) {  // the scales stay fp32
-            col_up[nb] = 1.0f;
-            continue;
-        }
-        const uint16_t* srow = sbase + sboff[nb];
-        uint32_t mag = 0;
-        const int first = G32 ? gb * 2 : gb / a.gs_blocks, last = G32 ? G * 2 : (G + a.gs_blocks - 1) / a.gs_blocks;
-        if (((sb_per_row | first | last) & 7) == 0 && ((uintptr_t)sbase & 15) == 0) {
-            const uint4* p = reinterpret_cast<const uint4*>(srow);
-            for (int i = (first >> 3) + h; i < (last >> 3); i += 2) {
-                const uint4 v = p[i];
-                const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    const uint32_t lo = w[c] & 0x7fffu, hi = (w[c] >> 16) & 0x7fffu;
-                    if (lo < 0x7f80u) mag = max(mag, lo);
-                    if (hi < 0x7f80u) mag = max(mag, hi);
-                }
-            }
-        } else {
-            for (int i = first + h; i < last; i += 2) {
-                const uint32_t v = srow[i] & 0x7fffu;
-                if (v < 0x7f80u) mag = max(mag, v);
-            }
-        }
-        mag = max(mag, (uint32_t)__shfl_xor((int)mag, 32, kWave));
-        col_up[nb] = pow2f(exponent_shift(mag, 10));
-    }
+    // A row of scales (or biases) in pieces of eight elements.  Eight lanes share a row: a load touches eight lines.
+    const uint32_t sb_total = (uint32_t)N * (uint32_t)sb_per_row;
+    const int per_quad = G32 ? 8 : 4 / a.gs_blocks;                       // elements of a quad of four 64-code blocks
+    const int first = gb / 4 * per_quad, last = min((G + 3) / 4 * per_quad, sb_per_row);  // of this workgroup's range of K
+    auto sb_row = [&](int r) { return (uint32_t)weight_row((r >> 5) / NB, (r >> 5) % NB, r & 31) * (uint32_t)sb_per_row; };
+    constexpr int THREADS = NWAVE * kWave;
 
-    // Scales are fetched per QUAD of four 64-code blocks, one quad ahead: the bf16 bits of the quad's four blocks
-    // in two words per column block (8-byte loads where the rows allow it).  Biases and the (hi, lo) block sums
-    // of x are needed once per quad, by the affine MFMA behind its last block, and are fetched for the quad under
-    // way.
-    // (groups of 32: this lane half's four of the quad's eight, picked out of one 16-byte load)
-    const uintptr_t sb_bits = (uintptr_t)sb1[0] | (uintptr_t)sb1[1] | (uintptr_t)sb2[0] | (uintptr_t)sb2[1];
-    const bool quad_loads = (Gall & 3) == 0 && (G32 ? (sb_bits & 15) == 0 : a.gs_blocks == 1 && (sb_bits & 7) == 0);
-    const uint32_t half_sel = h ? 0x07060302u : 0x05040100u;
-    uint2 s_cur[NB], s_nxt[NB], b_cur[NB];
-    auto load_quad = [&](int which, int quad, uint2 (&dst)[NB]) {
-        if (quad_loads) {
+    // Segment n of the scales and biases: SE elements of each row from first + n * SE on.  A thread loads its pieces (whose rows
+    // lie in one matrix or, eight elements a segment, in two) and stores them later.
+    constexpr int PPS = SE / 8;  // pieces of a row
+    constexpr int NP = 2 * BN * PPS / THREADS;
+    static_assert(2 * BN * PPS % THREADS == 0 && NP >= 1 && THREADS % kWave == 0, "pieces must divide among the threads");
+    const int quads = G32 ? SE / 8 : a.gs_blocks == 1 ? SE / 4 : SE / 2;  // of a segment
+    // (the thread's number is hidden from the compiler, which would keep every piece's address in registers)
+    auto piece_off = [&](int i, int n, bool& bias, bool& second) __attribute__((always_inline)) {
+        int t = tid;
+        asm volatile("" : "+v"(t));
+        const int at = i * THREADS + t, r = at / PPS % BN;
+        bias = i * THREADS >= BN * PPS || ((i + 1) * THREADS > BN * PPS && at >= BN * PPS);
+        second = (r >> 5) % NB != 0;
+        return sb_row(r) + (uint32_t)(first + n * SE + at % PPS * 8);
+    };
+    auto load_segment = [&](auto tiny, int n, uint4 (&to)[NP]) __attribute__((always_inline)) {
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                const uint16_t* const base = nb ? sb2[which] : sb1[which];
-                if constexpr (G32) {
-                    const uint4 v = *reinterpret_cast<const uint4*>(base + sboff[nb] + quad * 8);
-                    dst[nb] = make_uint2(__builtin_amdgcn_perm(v.y, v.x, half_sel), __builtin_amdgcn_perm(v.w, v.z, half_sel));
-                } else {
-                    dst[nb] = *reinterpret_cast<const uint2*>(base + sboff[nb] + quad * 4);
-                }
+        for (int i = 0; i < NP; i++) {
+            bool bias, second;
+            const uint32_t off = piece_off(i, n, bias, second);
+            to[i] = load_eight<decltype(tiny)::value>(bias ? (second ? sb2[1] : sb1[1]) : second ? sb2[0] : sb1[0], off, sb_total);
+        }
+    };
+    auto store_segment = [&](int n, const uint4 (&from)[NP]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < NP; i++) {
+            bool bias, second;
+            const uint32_t off = piece_off(i, n, bias, second);
+            *reinterpret_cast<uint4*>(sbuf + (i * THREADS + tid) * 8) = moved_down(from[i], off, sb_total);
+        }
+    };
+    uint4 piece[NP];
+
+    // Ahead of the loop: the first segment, and the power of two that brings a row's largest scale (of this workgroup's range of K)
+    // into [2^10, 2^11).  Everything is asked for before anything is waited for.
+    float col_up[NB];
+    auto scan = [&](auto tiny) __attribute__((always_inline)) {
+        constexpr int ROWS = BN * 8 / THREADS;  // of a thread
+        static_assert(BN * 8 % THREADS == 0, "rows of scales must divide among the threads");
+        uint4 v[ROWS];
+        uint32_t mag[ROWS];
+        auto at = [&](int i, int e, const uint16_t*& base) {
+            const int r = (i * THREADS + tid) >> 3;
+            base = (r >> 5) % NB ? sb2[0] : sb1[0];
+            return sb_row(r) + (uint32_t)e;
+        };
+        for (int e = first + (tid & 7) * 8, more = first; more < last; e += 64, more += 64) {
+#pragma unroll
+            for (int i = 0; i < ROWS; i++) {
+                const uint16_t* base;
+                const uint32_t off = at(i, e, base);
+                v[i] = load_eight<decltype(tiny)::value>(base, off, sb_total);
             }
-        } else {
+            if (more == first) {
 #pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                uint32_t v[4];
+                for (int i = 0; i < ROWS; i++) mag[i] = 0;
+                load_segment(tiny, 0, piece);
+            }
+            const int n = last - e;  // elements that count
 #pragma unroll
-                for (int k = 0; k < 4; k++) {
-                    int idx = G32 ? (quad * 4 + k) * 2 + h : (quad * 4 + k) / a.gs_blocks;
-                    idx = idx < sb_per_row ? idx : sb_per_row - 1;  // blocks past K: never used
-                    v[k] = (nb ? sb2[which] : sb1[which])[sboff[nb] + idx];
+            for (int i = 0; i < ROWS; i++) {
+                const uint16_t* base;
+                const uint32_t off = at(i, e, base);
+                v[i] = moved_down(v[i], off, sb_total);
+                const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+                uint32_t most = 0;
+#pragma unroll
+                for (int c = 0; c < 4; c++) most = max_u16x2(most, w[c] & (n > 2 * c + 1 ? 0x7fff7fffu : n > 2 * c ? 0x7fffu : 0u));
+                uint32_t one = max(most & 0xffffu, most >> 16);
+                if (one >= 0x7f80u) {  // inf and NaN do not set the scale
+                    one = 0;
+#pragma nounroll
+                    for (int c = 0; c < 8 && c < n; c++) {
+                        const uint32_t m = (c < 4 ? (c < 2 ? w[0] : w[1]) : c < 6 ? w[2] : w[3]) >> (c & 1) * 16 & 0x7fffu;
+                        if (m < 0x7f80u) one = max(one, m);
+                    }
                 }
-                dst[nb] = make_uint2(v[0] | (v[1] << 16), v[2] | (v[3] << 16));
+                mag[i] = max(mag[i], one);
+            }
+        }
+        uint32_t* const mags = reinterpret_cast<uint32_t*>(sbuf);
+#pragma unroll
+        for (int i = 0; i < ROWS; i++) {
+            mag[i] = max(mag[i], (uint32_t)__builtin_amdgcn_mov_dpp((int)mag[i], 0xb1, 0xf, 0xf, false));   // quad_perm 1 0 3 2
+            mag[i] = max(mag[i], (uint32_t)__builtin_amdgcn_mov_dpp((int)mag[i], 0x4e, 0xf, 0xf, false));   // quad_perm 2 3 0 1
+            mag[i] = max(mag[i], (uint32_t)__builtin_amdgcn_mov_dpp((int)mag[i], 0x141, 0xf, 0xf, false));  // eight lanes mirrored
+            if ((tid & 7) == 0) mags[(i * THREADS + tid) >> 3] = mag[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) col_up[nb] = pow2f(exponent_shift(mags[(wave_n * NB + nb) * 32 + j], 10));
+        __syncthreads();
+    };
+    auto prologue = [&](auto tiny) __attribute__((always_inline)) {
+        if constexpr (B8) {  // the scales stay fp32
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) col_up[nb] = 1.0f;
+            load_segment(tiny, 0, piece);
+        } else {
+            scan(tiny);
+        }
+    };
+    if (sb_total < 8)
+        prologue(std::true_type{});
+    else
+        prologue(std::false_type{});
+    store_segment(0, piece);
+    // A quad's scales (which 0) or biases (1) of this lane's rows: the bf16 bits of its four blocks in two words per column block
+    // (groups of 32: this lane half's four of the quad's eight).
+    const uint32_t half_sel = h ? 0x07060302u : 0x05040100u;
+    const uint32_t sel_01 = a.gs_blocks == 1 ? 0x03020100u : 0x01000100u, sel_23 = a.gs_blocks == 1 ? 0x07060504u : 0x03020302u;
+    uint2 s_cur[NB], s_nxt[NB], b_cur[NB];
+    auto read_quad = [&](int which, int quad, uint2 (&dst)[NB]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+            const uint16_t* const at = sbuf + ((which * BN + (wave_n * NB + nb) * 32 + j) * SE + quad * per_quad);
+            if constexpr (G32) {
+                const uint4 v = *reinterpret_cast<const uint4*>(at);
+                dst[nb] = make_uint2(__builtin_amdgcn_perm(v.y, v.x, half_sel), __builtin_amdgcn_perm(v.w, v.z, half_sel));
+            } else {  // (groups of 128: two elements, each for two blocks)
+                const uint32_t lo = *reinterpret_cast<const uint32_t*>(at), hi = *reinterpret_cast<const uint32_t*>(at + per_quad - 2);
+                dst[nb] = make_uint2(__builtin_amdgcn_perm(hi, lo, sel_01), __builtin_amdgcn_perm(hi, lo, sel_23));
             }
         }
     };
@@ -503,16 +600,31 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
         const uint32_t w = q < 2 ? v.x : v.y;
         return (q & 1) ? (w & 0xffff0000u) : (w << 16);
     };
-    uint32_t xsoff[MB];  // in 16-byte units
+    int quad_at = 0;  // place of the quad under way in its segment
+    int segment = 0;
+    // Sums of x: loaded a quad at a time, or, where registers are short, copied into LDS, a row block a copy
+    // (several wavefronts the same one where there are fewer): 512 bytes a quad, groups of 32 1024.
+    constexpr int XS_BLOCK = G32 ? 1024 : 512;
+    const uint32_t xbuf_at = bbuf_at + B_BUFS * B_STAGE + 2 * BN * SE * 2;
+    const uint8_t* const xbuf = reinterpret_cast<const uint8_t*>(sbuf) + 2 * BN * SE * 2;
+    [[maybe_unused]] auto issue_xs = [&](int quad) __attribute__((always_inline)) {
+#pragma unroll
+        for (int c = 0; c < NX; c++) {
+            const int blk = (wave + c * NWAVE) % (BM / 32), mblk = min(m0 / 32 + blk, a.mblks - 1);
+            copy16_to_lds(reinterpret_cast<const uint8_t*>(a.xs) + ((int64_t)mblk * G4 + quad) * XS_BLOCK, (uint32_t)(G32 ? lane : lane & 31) * 16u,
+                          xbuf_at + (uint32_t)(blk * 1024));
+        }
+    };
+    [[maybe_unused]] uint32_t xsoff[MB];  // in 16-byte units
 #pragma unroll
     for (int mb = 0; mb < MB; mb++) {
         const int mblk = min(m0 / 32 + wave_m * MB + mb, a.mblks - 1);
         xsoff[mb] = (uint32_t)mblk * (uint32_t)(G32 ? 2 * G4 : G4) * 32u + (G32 ? (uint32_t)h * 32u : 0u) + (uint32_t)j;
     }
-    uint4 xs_cur[MB];
+    uint4 xs_cur[XS_LDS ? 1 : MB];
     auto load_xs = [&](int quad) {
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + (G32 ? 64 * quad : 32 * quad)];
+        for (int mb = 0; mb < (XS_LDS ? 0 : MB); mb++) xs_cur[mb] = reinterpret_cast<const uint4*>(a.xs)[xsoff[mb] + (G32 ? 64 * quad : 32 * quad)];
     };
 
     f32x16_t out[MB][NB];
@@ -523,18 +635,17 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
 #pragma unroll
             for (int r = 0; r < 16; r++) out[mb][nb][r] = 0.0f;
 
-    // Affine terms of a quad's blocks 0..Q in one bf16 MFMA per output tile: k-slots (2q, 2q+1) carry
+    // Affine terms of a quad's blocks 0..qlast in one bf16 MFMA per output tile: k-slots (2q, 2q+1) carry
     // (Sx_hi, Sx_lo) of block q on the A side; lanes h=0 pair them with the bias, lanes h=1 with 8 * scale
-    // (both times the row's power of two: exact); blocks past Q (only at the end of K) contribute zeros.
-    auto affine = [&](auto q_tag) {
-        constexpr int Q = decltype(q_tag)::value;
+    // (both times the row's power of two: exact); blocks past qlast (only at the end of K) contribute zeros.
+    auto affine = [&](int qlast) __attribute__((always_inline)) {
         bf16x8_t bbf[NB], ebf[NB];
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) {
             uint32_t v[4], ve[4];
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                if (q <= Q) {
+                if (q <= qlast) {
                     const uint32_t eight = __float_as_uint(__uint_as_float(quad_hi(s_cur[nb], q)) * (CENTRE * col_up[nb])) >> 16;
                     const uint32_t bia = __float_as_uint(__uint_as_float(quad_hi(b_cur[nb], q)) * col_up[nb]) >> 16;
                     v[q] = dup16(!G32 && h ? eight : bia);
@@ -547,9 +658,11 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
             bbf[nb] = __builtin_bit_cast(bf16x8_t, u);
             ebf[nb] = __builtin_bit_cast(bf16x8_t, ue);
         }
+        if constexpr (XS_LDS) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) {
-            const bf16x8_t aa = __builtin_bit_cast(bf16x8_t, xs_cur[mb]);
+            const uint4 sums = XS_LDS ? *reinterpret_cast<const uint4*>(xbuf + (wave_m * MB + mb) * 1024 + (G32 ? lane : j) * 16) : xs_cur[XS_LDS ? 0 : mb];
+            const bf16x8_t aa = __builtin_bit_cast(bf16x8_t, sums);
 #pragma unroll
             for (int nb = 0; nb < NB; nb++)
                 out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aa, bbf[nb], out[mb][nb], 0, 0, 0);
@@ -558,177 +671,318 @@ __global__ __launch_bounds__(WM* WN* kWave, OCC) void qmmh_kernel(const QmmHalfA
                 for (int nb = 0; nb < NB; nb++)
                     out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(aa, ebf[nb], out[mb][nb], 0, 0, 0);
             }
+            if constexpr (XS_LDS) __builtin_amdgcn_sched_barrier(0);
         }
     };
 
     // One 64-code block per iteration; Q = g & 3 is static so that everything indexed by it stays in fixed
     // registers.  Iteration g requests block g + AHEAD.  Past the end of K the last block is requested again.
     //
-    // The next quad's scales and the current quad's biases and sums are fetched at Q = 1 with ordinary loads.
+    // The segment after this one (in its last quad) and the quad's sums of x are fetched at Q = 1 with ordinary loads.
     // The compiler cannot count the copy instructions, so wherever it first uses a loaded register it waits
     // until NOTHING is outstanding, copies included.  Iteration Q = 1 is therefore ordered: loads, MFMAs, first
     // use of the loaded registers (forced), and only then this iteration's copies - the forced wait then covers
     // the loads, a block of MFMAs old, and the copies of block g+1, which the end of the iteration needs anyway.
-    // (Loads at Q = 0, or the forced use at Q = 2, measured 3 to 4 % slower on the large tiles and no better on the small.)
+    // A segment is replaced where it lies: its last quad's scales and biases have been read by every wavefront before the
+    // barrier of Q = 0, and the next are first read at Q = 3, behind the barrier of Q = 1.
     // With two or four stages the stage of block g is g & 3 modulo the stages, static like Q, and every LDS address
     // of the loop is a constant; with three it is carried along.
-    const int glast = G - 1;
     constexpr bool STATIC_STAGE = STAGES == 2 || STAGES == 4;
     int sa_carried = 0;  // LDS stage that holds block g
-    auto iteration = [&](auto q_tag, int g) {
+    // whether the quad of block g is the last of its segment, with more of K behind it
+    auto refills = [&](int g) { return quad_at + 1 == quads && (g | 3) + 1 < G; };
+    auto next_quad = [&] {
+        if (++quad_at == quads) quad_at = 0, segment++;
+    };
+    // BITS 4: the loop as a pipeline of steps of 16 codes.  Step t of a block multiplies the fragments that step t - 1 has made
+    // ready, while the words of step t + 1 are expanded and A's fragments of step t + 1 are read, both a few instructions at a
+    // time between the MFMAs of one row block and the next: a wavefront then keeps matrix cores, vector unit and LDS busy by
+    // itself, where expanding a whole block ahead of its MFMAs left the matrix cores to the one other wavefront of the SIMD.
+    // The only barrier of a block is in the middle of its last step, behind MFMAs that need nothing of the next block.
+    constexpr bool TWO_A = MB <= 3;  // A's next fragments in registers of their own; else over those just multiplied
+    f16x8_t afr[TWO_A ? 2 : 1][MB];
+    uint32_t bfr[2][NB][4];
+    uint4 cw[NB];               // the block's words of this lane
+    f16x2_t s2[NB], m24[NB];    // its scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
+    auto read_a = [&](int mb, int t, int stage) {
+        afr[TWO_A ? t & 1 : 0][mb] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
+    };
+    // row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3, of block Q of a quad
+    auto read_codes = [&](int q) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+            cw[nb] = *reinterpret_cast<const uint4*>(bbuf + (q >> 1) * B_STAGE + ((wave_n * NB + nb) * 32 + j) * B_ROW + (((q % 2 * 2 + h) ^ turn(j)) * 16));
+    };
+    auto take_scale = [&](const uint2 (&from)[NB], int q) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+            const float sv = __uint_as_float(quad_hi(from[nb], q)) * col_up[nb], mv = sv * -24.0f;
+            s2[nb] = f16x2_t{(_Float16)sv, (_Float16)sv};
+            m24[nb] = f16x2_t{(_Float16)mv, (_Float16)mv};
+        }
+    };
+    // pairs [from, to) of the NB * 4 of word t
+    auto expand_some = [&](int t, int from, int to) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = from; i < to; i++) {
+            const int nb = i >> 2;
+            const uint32_t w = t == 0 ? cw[nb].x : t == 1 ? cw[nb].y : t == 2 ? cw[nb].z : cw[nb].w;
+            uint32_t& to_reg = bfr[t & 1][nb][i & 3];
+            if ((i & 3) == 0) to_reg = expand_pair<0>(w, mask_s, magic_v, s2[nb], m24[nb]);
+            if ((i & 3) == 1) to_reg = expand_pair<1>(w, mask_s, magic_v, s2[nb], m24[nb]);
+            if ((i & 3) == 2) to_reg = expand_pair<2>(w, mask_s, magic_v, s2[nb], m24[nb]);
+            if ((i & 3) == 3) to_reg = expand_pair<3>(w, mask_s, magic_v, s2[nb], m24[nb]);
+        }
+    };
+    auto block = [&](auto q_tag, int g) __attribute__((always_inline)) {
         constexpr int Q = decltype(q_tag)::value;
-        constexpr bool LATE = Q == 1;  // copies behind the MFMAs
-        const bool more = g + 1 < G;
         const int sa = STATIC_STAGE ? Q % STAGES : sa_carried;
-        if constexpr (Q == 0) {
+        const int sa_next = sa == STAGES - 1 ? 0 : sa + 1;
+        constexpr int PRE = MB / 2;  // row blocks of the last step ahead of the barrier
+        constexpr int PAIRS = NB * 4;
+        const bool refill = Q == 1 && refills(g);
+        if constexpr (Q == 0) read_quad(1, quad_at, b_cur);
+        if constexpr (Q == 1) {
+            if (refill) load_segment(std::false_type{}, segment + 1, piece);
+            if constexpr (!XS_LDS) load_xs(g >> 2);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (Q == 3) read_quad(0, quad_at + 1 == quads ? 0 : quad_at + 1, s_nxt);  // (behind the end of K: anything)
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int tn = (t + 1) & 3;  // the step that is made ready
+            if (t == 3) {  // the last word of this block is expanded
+                read_codes((Q + 1) & 3);
+                if (Q == 3) take_scale(s_nxt, 0); else take_scale(s_cur, Q + 1);
+            }
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) {
+                if (t == 3 && mb == PRE) {
+                    // The ordinary loads of block 1 are first used here, ahead of new copies: the compiler, which cannot count
+                    // the copies, waits for everything.
+                    if constexpr (Q == 1) {
+                        if (refill) store_segment(segment + 1, piece);
+#pragma unroll
+                        for (int m = 0; m < (XS_LDS ? 0 : MB); m++)
+                            asm volatile("" : "+v"(xs_cur[m].x), "+v"(xs_cur[m].y), "+v"(xs_cur[m].z), "+v"(xs_cur[m].w));
+                    }
+                    // What the next block needs has landed once only newer copies are outstanding, and every read of this block
+                    // has returned.  A bare s_barrier on purpose: __syncthreads() carries a workgroup fence, for which the
+                    // compiler drains ALL outstanding copies into LDS.
+                    __builtin_amdgcn_sched_barrier(0);
+                    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(still_out(Q)) : "memory");
+                    __builtin_amdgcn_s_barrier();
+                    asm volatile("" ::: "memory");
+                    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                    for (int m = 0; m < PRE; m++) read_a(m, 0, sa_next);
+                }
+                const bool reads = t < 3 || mb >= PRE;
+                if (TWO_A && reads) read_a(mb, tn, t == 3 ? sa_next : sa);
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++)
+                    out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[TWO_A ? t & 1 : 0][mb], __builtin_bit_cast(f16x8_t, make_uint4(bfr[t & 1][nb][0], bfr[t & 1][nb][1], bfr[t & 1][nb][2], bfr[t & 1][nb][3])),
+                                                                         out[mb][nb], 0, 0, 0);
+                if (!TWO_A && reads) read_a(mb, tn, t == 3 ? sa_next : sa);
+                expand_some(tn, mb * PAIRS / MB, (mb + 1) * PAIRS / MB);
+                if (t == 3 && mb >= PRE) {
+                    constexpr int COPIES = NA + ((Q & 1) == 0 ? NBC : 0), OVER = MB - PRE;
+#pragma unroll
+                    for (int c = (mb - PRE) * COPIES / OVER; c < (mb - PRE + 1) * COPIES / OVER; c++) {
+                        if (c < NA)
+                            issue_a1(c, min(g + STAGES, G - 1), sa);
+                        else
+                            issue_b(c - NA, min(g / QB + 2, (Gall - 1) / QB), Q >> 1);
+                    }
+                    // (the last quad's sums have been read before this barrier)
+                    if (XS_LDS && Q == 0 && mb == MB - 1) issue_xs(g >> 2);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (Q == 3) {
+            affine(3);
 #pragma unroll
             for (int nb = 0; nb < NB; nb++) s_cur[nb] = s_nxt[nb];
+            next_quad();
         }
-        if constexpr (Q == 1) {
-            const int nq = (g >> 2) + 1 < G4 ? (g >> 2) + 1 : G4 - 1;
-            load_quad(0, nq, s_nxt);
-            load_quad(1, g >> 2, b_cur);
-            load_xs(g >> 2);
-        }
-        // the copies of block g + AHEAD: together at the top, or (SPREAD) a few in front of every row block's
-        // MFMAs, so that they do not queue up behind those of the other wavefronts
-        const int g2 = g + AHEAD < G ? g + AHEAD : glast;
-        const int st2 = sa == 0 ? STAGES - 1 : sa - 1;  // stage (sa + AHEAD) % STAGES: read last in iteration g-1
-        // B's next stage into the buffer that was read last in the stage before this one (past the end of K: the last again)
-        constexpr int NBQ = B8 || (Q & 1) == 0 ? NBC : 0;
-        const int bcur = B8 ? sa : Q >> 1, bnxt = B8 ? st2 : (Q >> 1) ^ 1;
-        const int bst = B8 ? g2 : min(g / QB + 1, (Gall - 1) / QB);
-        auto issue_some = [&](int from, int to) {  // A's copies first, then B's
-#pragma unroll
-            for (int c = from; c < to; c++) {
-                if (c < NA)
-                    issue_a1(c, g2, st2);
-                else
-                    issue_b(c - NA, bst, bnxt);
-            }
-        };
-        if constexpr (!SPREAD && !LATE) issue_some(0, NA + NBQ);
-        const uint8_t* ab = abuf + sa * A_STAGE + (wave_m * MB) * 4096 + lane * 16;
-        const uint8_t* const brow = bbuf + bcur * B_STAGE + ((wave_n * NB) * 32 + j) * B_ROW;
-        f16x8_t bfrag[NB][4];
-        [[maybe_unused]] float scale[NB][G32 ? 2 : 1];  // BITS 8: of the block's groups
-        if constexpr (B8) {
-            // row (wave_n * NB + nb) * 32 + j, eight codes from 16 t + 8 h on for step t
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    bfrag[nb][t] = expand_bytes(*reinterpret_cast<const uint2*>(brow + nb * 32 * B_ROW + ((t ^ turn(j)) * 16) + h * 8));
-                const uint32_t sv = quad_hi(s_cur[nb], Q);
-                if constexpr (G32) {  // the lane halves hold the two groups' scales
-                    const auto both = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
-                    scale[nb][0] = __uint_as_float(both[0]);
-                    scale[nb][1] = __uint_as_float(both[1]);
-                } else {
-                    scale[nb][0] = __uint_as_float(sv);
-                }
-            }
-        } else {
-            // this lane's codes: row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3
-            const uint8_t* bb = brow + (((Q % QB * 2 + h) ^ turn(j)) * 16);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++) {
-                const uint4 cw = *reinterpret_cast<const uint4*>(bb + nb * 32 * B_ROW);
-                // the block's scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
-                const float sv = __uint_as_float(quad_hi(s_cur[nb], Q)) * col_up[nb];
-                const f16x2_t s2 = {(_Float16)sv, (_Float16)sv};
-                const float mv = sv * -24.0f;
-                const f16x2_t m24 = {(_Float16)mv, (_Float16)mv};
-                bfrag[nb][0] = __builtin_bit_cast(f16x8_t, expand_word(cw.x, mask_s, magic_v, s2, m24));
-                bfrag[nb][1] = __builtin_bit_cast(f16x8_t, expand_word(cw.y, mask_s, magic_v, s2, m24));
-                bfrag[nb][2] = __builtin_bit_cast(f16x8_t, expand_word(cw.z, mask_s, magic_v, s2, m24));
-                bfrag[nb][3] = __builtin_bit_cast(f16x8_t, expand_word(cw.w, mask_s, magic_v, s2, m24));
-            }
-        }
-        constexpr int GROUPS = G32 ? 2 : 1;  // of a block
-        [[maybe_unused]] f32x16_t part[2][NB];
-        [[maybe_unused]] auto scale_part = [&](int u) {
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-#pragma unroll
-                for (int r = 0; r < 16; r++)
-                    out[u / GROUPS][nb][r] = __builtin_fmaf(scale[nb][u % GROUPS], part[u & 1][nb][r], out[u / GROUPS][nb][r]);
-        };
-        // the A fragments of row block mb+1 are read while row block mb is multiplied
-        f16x8_t afrag[2][4];
-#pragma unroll
-        for (int t = 0; t < 4; t++) afrag[0][t] = *reinterpret_cast<const f16x8_t*>(ab + t * 1024);
-#pragma unroll
-        for (int mb = 0; mb < MB; mb++) {
-            if (mb + 1 < MB) {
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-                    afrag[(mb + 1) & 1][t] = *reinterpret_cast<const f16x8_t*>(ab + ((mb + 1) * 4 + t) * 1024);
-                __builtin_amdgcn_sched_barrier(0);  // or the scheduler sinks the reads back to their first use
-            }
-            if constexpr (SPREAD && !LATE) issue_some(mb * (NA + NBQ) / MB, (mb + 1) * (NA + NBQ) / MB);
-            if constexpr (B8) {
-                // a group's sums are scaled while the matrix cores work on the next group's
-#pragma unroll
-                for (int grp = 0; grp < GROUPS; grp++) {
-                    constexpr int STEPS = 4 / GROUPS;
-                    const int u = mb * GROUPS + grp;
-#pragma unroll
-                    for (int t = 0; t < STEPS; t++)
-#pragma unroll
-                        for (int nb = 0; nb < NB; nb++)
-                            part[u & 1][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag[mb & 1][grp * STEPS + t], bfrag[nb][grp * STEPS + t],
-                                                                                     t ? part[u & 1][nb] : f32x16_t{}, 0, 0, 0);
-                    if (u > 0) scale_part(u - 1);
-                }
-                if (mb == MB - 1) scale_part(MB * GROUPS - 1);
-            } else {
-#pragma unroll
-                for (int t = 0; t < 4; t++)
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++)
-                        out[mb][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afrag[mb & 1][t], bfrag[nb][t], out[mb][nb], 0, 0, 0);
-            }
-        }
-        if constexpr (LATE) {
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int nb = 0; nb < NB; nb++)
-                asm volatile("" : "+v"(s_nxt[nb].x), "+v"(s_nxt[nb].y), "+v"(b_cur[nb].x), "+v"(b_cur[nb].y));
-#pragma unroll
-            for (int mb = 0; mb < MB; mb++)
-                asm volatile("" : "+v"(xs_cur[mb].x), "+v"(xs_cur[mb].y), "+v"(xs_cur[mb].z), "+v"(xs_cur[mb].w));
-            __builtin_amdgcn_sched_barrier(0);
-            issue_some(0, NA + NBQ);
-        }
-        if (Q == 3 || !more) {
-            if (Q < 1) {  // K ends inside a quad before its biases and sums were asked for
-                load_quad(1, g >> 2, b_cur);
-                load_xs(g >> 2);
-            }
-            affine(q_tag);
-        }
-        sa_carried = sa == STAGES - 1 ? 0 : sa + 1;
-        // Block g+1 has landed once only newer copies are outstanding (still_out); this iteration's LDS reads have returned.  A bare s_barrier on purpose: __syncthreads() carries a workgroup
-        // fence, for which the compiler drains ALL outstanding copies into LDS.
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(still_out(Q)) : "memory");
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
+        sa_carried = sa_next;
     };
-    // the first quad's scales; blocks 0 .. AHEAD-1 were requested before the scan of the scale rows (any wait of
-    // the compiler's for the loads since then has drained those copies too: all the better)
-    load_quad(0, gb >> 2, s_nxt);
+    // BITS 8: units of the MFMAs of a row block and group, into partial sums of their own.  While a unit is multiplied the sums of the
+    // unit before it are scaled; in a block's last row block, behind the barrier, each step's fragments of B are replaced by the next
+    // block's as soon as they have been multiplied, and A's always by the next row block's.  A quad ends with its sums scaled.
+    constexpr int GROUPS = G32 ? 2 : 1;  // of a block
+    constexpr int UNITS = MB * GROUPS, STEPS = 4 / GROUPS;
+    f16x8_t a8[4], b8[NB][4];
+    uint2 codes8[NB];
+    constexpr int PARTS = G32 ? 1 : 2;  // (groups of 32 have no registers for a second unit's sums: scaled behind their own MFMAs)
+    f32x16_t part[PARTS][NB];
+    float scale[NB][GROUPS], scale_before[NB];  // of the block's groups; of the last group of the block before
+    // (the compiler would move what it can of the work above a branch behind it, with everything that this work reads)
+    auto pin8 = [&]() __attribute__((always_inline)) {
 #pragma unroll
-    for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(s_nxt[nb].x), "+v"(s_nxt[nb].y));
+        for (int nb = 0; nb < NB; nb++) {
+#pragma unroll
+            for (int mb = 0; mb < MB; mb++) asm volatile("" : "+v"(out[mb][nb]));
+#pragma unroll
+            for (int t = 0; t < 4; t++) asm volatile("" : "+v"(b8[nb][t]));
+        }
+    };
+    auto read_a8 = [&](int t, int mb, int stage) __attribute__((always_inline)) {
+        a8[t] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
+    };
+    // row (wave_n * NB + nb) * 32 + j, eight codes from 16 t + 8 h on for step t
+    auto read_codes8 = [&](int t, int stage) __attribute__((always_inline)) {
+        const uint8_t* const at = bbuf + (stage * B_STAGE + (wave_n * NB * 32 + j) * B_ROW + h * 8 + ((t ^ turn(j)) * 16));
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) codes8[nb] = *reinterpret_cast<const uint2*>(at + nb * 32 * B_ROW);
+    };
+    auto expand8 = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) b8[nb][t] = expand_bytes(codes8[nb]);
+    };
+    // registers [from, to) of the sums of the unit before unit u of block Q of a quad
+    auto scale_part = [&](auto q_tag, int u, int from, int to) __attribute__((always_inline)) {
+        constexpr int Q = decltype(q_tag)::value;
+        const int last = u == 0 ? UNITS - 1 : u - 1;
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+            for (int r = from; r < to; r++)
+                out[last / GROUPS][nb][r] = __builtin_fmaf(u == 0 ? scale_before[nb] : scale[nb][last % GROUPS], part[(Q * UNITS + u + 1) % PARTS][nb][r],
+                                                           out[last / GROUPS][nb][r]);
+    };
+    [[maybe_unused]] auto block8 = [&](auto q_tag, int g) __attribute__((always_inline)) {
+        constexpr int Q = decltype(q_tag)::value;
+        const int sa = sa_carried, sa_next = sa == STAGES - 1 ? 0 : sa + 1;
+        const bool refill = Q == 1 && refills(g);
+        if constexpr (Q == 0) {
+            read_quad(0, quad_at, s_cur);
+            read_quad(1, quad_at, b_cur);
+        }
+        if constexpr (Q == 1) pin8();
+        if (refill) load_segment(std::false_type{}, segment + 1, piece);
+        if constexpr (Q == 2) load_xs(g >> 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UNITS; u++) {
+            const int mb = u / GROUPS;
+            const bool last_mb = mb == MB - 1;
+            if (u == (MB - 1) * GROUPS) {  // (as in BITS 4's)
+                if constexpr (Q == 1) pin8();
+                if (refill) store_segment(segment + 1, piece);
+                if constexpr (Q == 2) {
+#pragma unroll
+                    for (int m = 0; m < MB; m++)
+                        asm volatile("" : "+v"(xs_cur[m].x), "+v"(xs_cur[m].y), "+v"(xs_cur[m].z), "+v"(xs_cur[m].w));
+                }
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(still_out(Q)) : "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int step = 0; step < STEPS; step++) {
+                const int t = u % GROUPS * STEPS + step;
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++)
+                    part[(Q * UNITS + u) % PARTS][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a8[t], b8[nb][t], step ? part[(Q * UNITS + u) % PARTS][nb] : f32x16_t{}, 0, 0, 0);
+                read_a8(t, last_mb ? 0 : mb + 1, last_mb ? sa_next : sa);
+                if (PARTS == 2 && (Q > 0 || u > 0)) scale_part(q_tag, u, step * 16 / STEPS, (step + 1) * 16 / STEPS);
+                if (u == 0 && step == STEPS - 1) {
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++) {
+                        const uint32_t sv = quad_hi(s_cur[nb], Q);
+                        if constexpr (G32) {  // the lane halves hold the two groups' scales
+                            const auto both = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
+                            scale[nb][0] = __uint_as_float(both[0]);
+                            scale[nb][1] = __uint_as_float(both[1]);
+                        } else {
+                            scale[nb][0] = __uint_as_float(sv);
+                        }
+                    }
+                }
+                if (last_mb) {
+                    if (t > 0) expand8(t - 1);
+                    read_codes8(t, sa_next);
+#pragma unroll
+                    for (int c = t * (NA + NBC) / 4; c < (t + 1) * (NA + NBC) / 4; c++) {
+                        if (c < NA)
+                            issue_a1(c, min(g + STAGES, G - 1), sa);
+                        else
+                            issue_b(c - NA, min(g + STAGES, G - 1), sa);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            if (PARTS == 1) {
+                scale_part(q_tag, u + 1, 0, 16);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        expand8(3);
+        if constexpr (Q == 3) {
+            if (PARTS == 2) scale_part(q_tag, UNITS, 0, 16);
+            affine(3);
+            next_quad();
+        } else {
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++) scale_before[nb] = scale[nb][GROUPS - 1];
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        sa_carried = sa_next;
+    };
+    // blocks 0 .. STAGES-1 were requested before the scan of the scale rows (any wait of the compiler's for the loads since then has
+    // drained those copies too)
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * (B8 ? NA + NBC : NA)) : "memory");  // block 0 has landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 1) * (B8 ? NA + NBC : NA)) : "memory");  // block 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    for (int g = gb; g < G; g += 4) {
-        iteration(std::integral_constant<int, 0>{}, g);
-        if (g + 1 < G) iteration(std::integral_constant<int, 1>{}, g + 1);
-        if (g + 2 < G) iteration(std::integral_constant<int, 2>{}, g + 2);
-        if (g + 3 < G) iteration(std::integral_constant<int, 3>{}, g + 3);
+    auto run = [&](auto q_tag, int g) __attribute__((always_inline)) {
+        if constexpr (B8) block8(q_tag, g); else block(q_tag, g);
+    };
+    if constexpr (B8) {
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            read_codes8(t, 0);
+            expand8(t);
+            read_a8(t, 0, 0);
+        }
+    } else {
+        read_quad(0, 0, s_cur);
+        read_codes(0);
+        take_scale(s_cur, 0);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) read_a(mb, 0, 0);
+        expand_some(0, 0, NB * 4);
+    }
+    int g = gb;
+    for (; g + 4 <= G; g += 4) {
+        run(std::integral_constant<int, 0>{}, g);
+        run(std::integral_constant<int, 1>{}, g + 1);
+        run(std::integral_constant<int, 2>{}, g + 2);
+        run(std::integral_constant<int, 3>{}, g + 3);
+    }
+    g = __builtin_amdgcn_readfirstlane(g);
+    if (g < G) {  // K ends inside a quad
+        run(std::integral_constant<int, 0>{}, g);
+        if constexpr (B8 && PARTS == 2)
+            if (g + 1 == G) scale_part(std::integral_constant<int, 0>{}, UNITS, 0, 16);
+        if (g + 1 < G) run(std::integral_constant<int, 1>{}, g + 1);
+        if constexpr (B8 && PARTS == 2)
+            if (g + 2 == G) scale_part(std::integral_constant<int, 1>{}, UNITS, 0, 16);
+        if (g + 2 < G) run(std::integral_constant<int, 2>{}, g + 2);
+        if constexpr (B8 && PARTS == 2)
+            if (g + 3 == G) scale_part(std::integral_constant<int, 2>{}, UNITS, 0, 16);
+        if constexpr (XS_LDS) {  // its sums are asked for in its first block, and may be on their way
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+        } else if (g + (B8 ? 2 : 1) >= G) {
+            load_xs(g >> 2);
+        }
+        affine(G - 1 - g);
     }
     // the copies requested past the end of K must not outlive the wavefront's use of LDS
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -909,30 +1163,32 @@ struct QmmHalfEntry {
     int lds_bytes;
 };
 
-#define AQ_QMMH(PREFIX, BITS, MB, NB, WM, WN, ST, OCC, SPREAD, SUFFIX)                                                        \
-    {                                                                                                                        \
-        {PREFIX #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, BITS, MB, NB, WM, WN},                                             \
-            qmmh_kernel<BITS, MB, NB, WM, WN, ST, OCC, SPREAD, 64>, qmmh_kernel<BITS, MB, NB, WM, WN, ST, OCC, SPREAD, 32>,  \
-            ST*(WM * MB * 4096) + (BITS == 8 ? ST : 2) * (WN * NB * 32 * 64)                                                  \
+#define AQ_QMMH(PREFIX, BITS, MB, NB, WM, WN, ST, SE, SUFFIX)                                                        \
+    {                                                                                                                            \
+        {PREFIX #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, BITS, MB, NB, WM, WN},                                                 \
+            qmmh_kernel<BITS, MB, NB, WM, WN, ST, SE, 64>, qmmh_kernel<BITS, MB, NB, WM, WN, ST, SE, 32>, \
+            ST*(WM * MB * 4096) + (BITS == 8 ? ST : 2) * (WN * NB * 32 * 64) + 2 * (WN * NB * 32) * SE * 2 +                      \
+                (BITS == 4 && MB >= 3 ? WM * MB * 1024 : 0)                                                                      \
     }
 #define AQ_QMMH4(...) AQ_QMMH("qmmh_b4_mb", 4, __VA_ARGS__)
 #define AQ_QMMH8(...) AQ_QMMH("qmmh8_b8_mb", 8, __VA_ARGS__)
 
 static const QmmHalfEntry kQmmHalfTable[] = {
-    AQ_QMMH4(4, 2, 2, 2, 2, 2, true, "_s2c"),  // 256 x 128, four wavefronts, two stages (every LDS address a constant)
-    AQ_QMMH4(4, 2, 2, 4, 3, 2, false, ""),     // 256 x 256, eight wavefronts, three stages (120 KiB): an A tile feeds twice the MFMAs
-    AQ_QMMH4(3, 2, 2, 4, 3, 2, false, ""),     // 192 x 256: a round of these takes 0.82 of a round of those; for row counts
-                                              // that fill their rounds better (1536 rows: 8 bands instead of 6 of 256)
-    AQ_QMMH4(2, 2, 2, 2, 3, 2, false, ""),     // 128 x 128
-    AQ_QMMH4(2, 2, 1, 4, 3, 2, false, ""),     // 64 x 256
-    AQ_QMMH4(1, 2, 1, 4, 3, 2, false, ""),     // 32 x 256
+    AQ_QMMH4(4, 2, 2, 2, 2, 16, "_s2c"),  // 256 x 128, four wavefronts, two stages (every LDS address a constant), one a CU
+    AQ_QMMH4(4, 2, 1, 4, 2, 8, "_s2c"),  // 128 x 256, four wavefronts, two stages (every LDS address a constant), two a CU
+    AQ_QMMH4(4, 2, 2, 4, 3, 16, ""),     // 256 x 256, eight wavefronts, three stages: an A tile feeds twice the MFMAs
+    AQ_QMMH4(3, 2, 2, 4, 3, 16, ""),     // 192 x 256: a round of these takes 0.82 of a round of those; for row counts
+                                                  // that fill their rounds better (1536 rows: 8 bands instead of 6 of 256)
+    AQ_QMMH4(2, 2, 2, 2, 3, 16, ""),     // 128 x 128
+    AQ_QMMH4(2, 2, 1, 4, 3, 16, ""),     // 64 x 256
+    AQ_QMMH4(1, 2, 1, 4, 3, 8, ""),      // 32 x 256, three a CU
     // 8-bit codes (a wavefront's partial sums take 64 registers: 96 or 128 rows a wavefront would spill)
-    AQ_QMMH8(2, 2, 2, 2, 3, 2, true, ""),      // (copies spread: 343 -> 329 us on 2048 x 4096 x 14336)
-    AQ_QMMH8(2, 2, 2, 4, 3, 2, false, ""),     // 128 x 256, eight wavefronts
-    AQ_QMMH8(2, 2, 1, 4, 3, 2, false, ""),
-    AQ_QMMH8(1, 2, 1, 4, 3, 2, false, ""),
-    AQ_QMMH8(1, 2, 2, 2, 3, 2, false, ""),     // 64 x 128 (4-bit tiles of that size, unsplit 167 -> 152 us on 509 x 15360 x 3840, lost to
-                                               // 128 x 128 and 192 x 256 with shares of K: 117 -> 142)
+    AQ_QMMH8(2, 2, 2, 2, 3, 16, ""),      // (copies spread: 343 -> 329 us on 2048 x 4096 x 14336)
+    AQ_QMMH8(2, 2, 2, 4, 3, 16, ""),     // 128 x 256, eight wavefronts
+    AQ_QMMH8(2, 2, 1, 4, 3, 8, ""),
+    AQ_QMMH8(1, 2, 1, 4, 3, 16, ""),
+    AQ_QMMH8(1, 2, 2, 2, 3, 8, ""),      // 64 x 128 (4-bit tiles of that size, unsplit 167 -> 152 us on 509 x 15360 x 3840, lost to
+                                                  // 128 x 128 and 192 x 256 with shares of K: 117 -> 142)
 };
 
 int qmmh_variant_count() { return (int)(sizeof(kQmmHalfTable) / sizeof(kQmmHalfTable[0])); }
@@ -953,17 +1209,16 @@ size_t qmmh_partial_bytes(const QmmHalfCall& q) {
 
 // What a workgroup tile of each kernel takes: microseconds per 64-code block of K alone on its CU, the same per tile when the
 // CU has more of them, and outside the loop.  From runs at K = 1024 and 4096 with 1/2, 1, 2, 3 and 4 tiles per CU (a CU's
-// clock and its share of L2 depend on how busy the rest of the chip is: 256 x 256 tiles take 1.77 on half the CUs, 2.2 on all).
+// clock and its share of L2 depend on how busy the rest of the chip is: 256 x 256 tiles take 1.73 alone and 1.95 in a row).
 struct QmmHalfCost {
     double solo, full, fixed;
 };
-static const QmmHalfCost kQmmHalfCost[] = {{1.35, 1.17, 8.0}, {1.77, 2.2, 8.0}, {1.48, 1.78, 7.0}, {0.9, 0.735, 5.0}, {0.9, 0.74, 5.0}, {0.75, 0.55, 4.0},
-                                           {1.02, 0.72, 5.0}, {1.25, 1.35, 6.0}, {1.01, 0.74, 5.0}, {0.78, 0.51, 4.0}, {0.66, 0.41, 4.0}};
+static const QmmHalfCost kQmmHalfCost[] = {{0.99, 1.12, 8.5}, {0.95, 1.0, 10.0}, {1.73, 1.95, 12.0}, {1.37, 1.4, 10.0}, {0.65, 0.61, 5.0}, {0.67, 0.62, 5.0}, {0.61, 0.44, 3.0},
+                                           {0.75, 0.65, 5.0}, {1.17, 1.27, 6.5}, {0.77, 0.69, 5.0}, {0.66, 0.49, 3.0}, {0.58, 0.435, 3.0}};
 
 // Microseconds of kernel i over `tiles` tiles of `blocks` blocks each.
 static double half_cost(int i, int64_t tiles, int blocks, int cus) {
-    const double load = (double)tiles / cus, per_cu = load > 1.0 ? ceil(load) : load;
-    const double work = kQmmHalfCost[i].full * per_cu, least = kQmmHalfCost[i].solo;
+    const double work = tiles > cus ? kQmmHalfCost[i].full * ceil((double)tiles / cus) : 0.0, least = kQmmHalfCost[i].solo;
     return kQmmHalfCost[i].fixed + blocks * (work > least ? work : least);
 }
 static int64_t half_strips(int i, int N, bool pair) {
