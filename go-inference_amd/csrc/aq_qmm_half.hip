@@ -277,10 +277,7 @@ __device__ __forceinline__ void fix_output(const QmmHalfArgs& a, const QmmSegmen
 }
 
 // ---- main kernel ----------------------------------------------------------------------------
-// OCC: wavefronts per SIMD the register budget is cut for (2: 256 registers, 1: 512, the accumulators then live in
-// the accumulation half of the register file).
-// SPREAD: the copies of the block requested in an iteration are issued a few at a time in front of every row block's
-// MFMAs instead of together at the top.
+// SE: elements of a row of scales (and of biases) in LDS at a time.
 // GRP 32: the codes a lane half h expands are those of one group (block g's half h), so that only its scale and bias differ:
 // the lane half keeps its own four scales per quad; the affine term takes its own sums on the A side and two MFMAs per quad
 // (sum x bias, sum x 8 scale) instead of one.
@@ -1183,7 +1180,7 @@ static const QmmHalfEntry kQmmHalfTable[] = {
     AQ_QMMH4(2, 2, 1, 4, 3, 16, ""),     // 64 x 256
     AQ_QMMH4(1, 2, 1, 4, 3, 8, ""),      // 32 x 256, three a CU
     // 8-bit codes (a wavefront's partial sums take 64 registers: 96 or 128 rows a wavefront would spill)
-    AQ_QMMH8(2, 2, 2, 2, 3, 16, ""),      // (copies spread: 343 -> 329 us on 2048 x 4096 x 14336)
+    AQ_QMMH8(2, 2, 2, 2, 3, 16, ""),      // 128 x 128
     AQ_QMMH8(2, 2, 2, 4, 3, 16, ""),     // 128 x 256, eight wavefronts
     AQ_QMMH8(2, 2, 1, 4, 3, 8, ""),
     AQ_QMMH8(1, 2, 1, 4, 3, 16, ""),
