@@ -160,9 +160,14 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(const MoeCombineArgs a
     }
 }
 
-// The same for bf16 route rows of whole 16-byte pieces: one row per grid row, eight columns a thread, the rows of all ranks
-// requested together (one element a thread: 18 us for 512 x 8 x 2816, 23 MB; here 6).
-constexpr int kCombineAhead = 8;
+// The same for bf16 route rows of whole 16-byte pieces: one row per grid row, eight columns a thread, AHEAD ranks at a time.
+// Bound: latency; rows and weights of the AHEAD ranks are requested together, ahead of any use and with no branch between them
+// (ranks past the last repeat it and are not added).
+// Roundings by instruction and chosen at compile time: with f32_to_bf16_bits and its NaN case inside, and a break after the last
+// rank, the weights were loaded rank by rank between thousands of branches (us a pass: 8 tokens, 8 of 128 experts, 2816 columns
+// 79.6 -> 77.8, 512 tokens 243.8 -> 241.0; one element a thread: 18 for the kernel alone at 512 tokens).
+// As many ranks at a time as there are, up to eight: repeated ones cost their loads.
+template <int AHEAD, bool STEPS>
 __global__ __launch_bounds__(kWave) void moe_combine_wide_kernel(const MoeCombineArgs a) {
 #pragma clang fp contract(off)  // as above
     const int col = ((int)blockIdx.x * kWave + (int)threadIdx.x) * 8;
@@ -170,26 +175,35 @@ __global__ __launch_bounds__(kWave) void moe_combine_wide_kernel(const MoeCombin
     const int64_t row = blockIdx.y, first = row * a.top_k;
     const uint16_t* const src = static_cast<const uint16_t*>(a.route_rows) + first * a.n + col;
     float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    for (int r0 = 0; r0 < a.top_k; r0 += kCombineAhead) {
-        uint4 v[kCombineAhead];
+    auto rounded = [](float (&v)[2]) {
+        const uint32_t u = pack_bf16x2(v[0], v[1]);
+        v[0] = __uint_as_float(u << 16), v[1] = __uint_as_float(u & 0xffff0000u);
+    };
+    for (int r0 = 0; r0 < a.top_k; r0 += AHEAD) {
+        uint4 v[AHEAD];
+        float w[AHEAD];
 #pragma unroll
-        for (int i = 0; i < kCombineAhead; i++)
-            if (r0 + i < a.top_k) v[i] = *reinterpret_cast<const uint4*>(src + (int64_t)(r0 + i) * a.n);
+        for (int i = 0; i < AHEAD; i++) {
+            const int r = min(r0 + i, a.top_k - 1);
+            v[i] = *reinterpret_cast<const uint4*>(src + (int64_t)r * a.n);
+            w[i] = a.weights[first + r];
+        }
 #pragma unroll
-        for (int i = 0; i < kCombineAhead; i++) {
-            if (r0 + i >= a.top_k) break;
-            float w = a.weights[first + r0 + i];
-            if (a.bf16_steps) w = bf16_bits_to_f32(f32_to_bf16_bits(w));
+        for (int i = 0; i < AHEAD; i++) {
+            const bool counts = r0 + i < a.top_k;  // (a break here, and every load moves down to its use)
+            float wi = w[i];
+            if (STEPS) wi = bf16_bits_to_f32(f32_to_bf16_bits(wi));
             const uint32_t words[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                const float scaled = bf16_bits_to_f32((words[c >> 1] >> (16 * (c & 1))) & 0xffffu) * w;
-                if (a.bf16_steps) {
-                    const float term = bf16_bits_to_f32(f32_to_bf16_bits(scaled));
-                    acc[c] = r0 + i == 0 ? term : bf16_bits_to_f32(f32_to_bf16_bits(acc[c] + term));
-                } else {
-                    acc[c] = acc[c] + scaled;
+            for (int c = 0; c < 4; c++) {
+                float term[2] = {__uint_as_float(words[c] << 16) * wi, __uint_as_float(words[c] & 0xffff0000u) * wi};
+                if (STEPS) rounded(term);
+                float sum[2] = {acc[2 * c] + term[0], acc[2 * c + 1] + term[1]};
+                if (STEPS) {
+                    rounded(sum);
+                    if (r0 + i == 0) sum[0] = term[0], sum[1] = term[1];  // (not 0 + term: minus zero stays)
                 }
+                acc[2 * c] = counts ? sum[0] : acc[2 * c], acc[2 * c + 1] = counts ? sum[1] : acc[2 * c + 1];
             }
         }
     }
@@ -229,7 +243,12 @@ hipError_t moe_combine_launch(const MoeCombineArgs& a, hipStream_t stream) {
     if (total <= 0) return hipSuccess;
     const uintptr_t at = reinterpret_cast<uintptr_t>(a.route_rows) | reinterpret_cast<uintptr_t>(a.out);
     if (!a.in_f32 && a.n % 8 == 0 && (at & 15) == 0 && a.rows <= 65535) {
-        hipLaunchKernelGGL(moe_combine_wide_kernel, dim3((unsigned)((a.n / 8 + kWave - 1) / kWave), (unsigned)a.rows), dim3(kWave), 0, stream, a);
+        typedef void (*CombineKernel)(MoeCombineArgs);
+        static const CombineKernel kWide[3][2] = {{moe_combine_wide_kernel<2, false>, moe_combine_wide_kernel<2, true>},
+                                                  {moe_combine_wide_kernel<4, false>, moe_combine_wide_kernel<4, true>},
+                                                  {moe_combine_wide_kernel<8, false>, moe_combine_wide_kernel<8, true>}};
+        const CombineKernel fn = kWide[a.top_k <= 2 ? 0 : a.top_k <= 4 ? 1 : 2][a.bf16_steps ? 1 : 0];
+        hipLaunchKernelGGL(fn, dim3((unsigned)((a.n / 8 + kWave - 1) / kWave), (unsigned)a.rows), dim3(kWave), 0, stream, a);
         return hipGetLastError();
     }
     int64_t blocks = (total + 255) / 256;
