@@ -331,8 +331,11 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     constexpr bool XS_LDS = !B8 && MB >= 3;  // the sums of x of a quad go through LDS
     constexpr int NX = (BM / 32 + NWAVE - 1) / NWAVE;  // copies of them a wavefront issues
     constexpr int NA = A_BLOCKS / NWAVE;  // A copies a wavefront issues per block
+    constexpr bool WHOLE = B8 && MB == 1;               // a block at a time (whole8)
+    constexpr int DEPTH = WHOLE ? STAGES - 1 : STAGES;  // blocks requested ahead of the loop
     // Behind the barrier of block g the copies of A's block g + STAGES are issued.  BITS 4: and, in a stage's first block, those of B's
-    // stage after the next, two blocks before its codes are read; BITS 8: and B's block g + STAGES.  still_out: the copies that may
+    // stage after the next, two blocks before its codes are read; BITS 8: and B's block g + STAGES (WHOLE: ahead of the barrier of
+    // block g, of block g + STAGES - 1).  still_out: the copies that may
     // be on their way at the barrier of block Q of a quad: A of block g + 1 has to have landed and with it the codes that are
     // read up to the next barrier.
     static_assert(STAGES <= 3, "waits are counted for two or three stages");
@@ -452,7 +455,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
 #pragma unroll
             for (int c = 0; c < NBC; c++) issue_b(c, min(gb / QB + st, (Gall - 1) / QB), st);
 #pragma unroll
-    for (int d = 0; d < STAGES; d++) {
+    for (int d = 0; d < DEPTH; d++) {
 #pragma unroll
         for (int c = 0; c < NA; c++) issue_a1(c, gb + d < G ? gb + d : G - 1, d);
         if constexpr (B8)
@@ -812,7 +815,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     constexpr int UNITS = MB * GROUPS, STEPS = 4 / GROUPS;
     f16x8_t a8[4], b8[NB][4];
     uint2 codes8[NB];
-    constexpr int PARTS = G32 ? 1 : 2;  // (groups of 32 have no registers for a second unit's sums: scaled behind their own MFMAs)
+    constexpr int PARTS = G32 || WHOLE ? 1 : 2;  // (groups of 32 have no registers for a second unit's sums: scaled behind their own MFMAs)
     f32x16_t part[PARTS][NB];
     float scale[NB][GROUPS], scale_before[NB];  // of the block's groups; of the last group of the block before
     // (the compiler would move what it can of the work above a branch behind it, with everything that this work reads)
@@ -837,6 +840,19 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     auto expand8 = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) b8[nb][t] = expand_bytes(codes8[nb]);
+    };
+    auto take_scales8 = [&](int q) __attribute__((always_inline)) {  // of block q of a quad
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) {
+            const uint32_t sv = quad_hi(s_cur[nb], q);
+            if constexpr (G32) {  // the lane halves hold the two groups' scales
+                const auto both = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
+                scale[nb][0] = __uint_as_float(both[0]);
+                scale[nb][1] = __uint_as_float(both[1]);
+            } else {
+                scale[nb][0] = __uint_as_float(sv);
+            }
+        }
     };
     // registers [from, to) of the sums of the unit before unit u of block Q of a quad
     auto scale_part = [&](auto q_tag, int u, int from, int to) __attribute__((always_inline)) {
@@ -887,19 +903,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
                     part[(Q * UNITS + u) % PARTS][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a8[t], b8[nb][t], step ? part[(Q * UNITS + u) % PARTS][nb] : f32x16_t{}, 0, 0, 0);
                 read_a8(t, last_mb ? 0 : mb + 1, last_mb ? sa_next : sa);
                 if (PARTS == 2 && (Q > 0 || u > 0)) scale_part(q_tag, u, step * 16 / STEPS, (step + 1) * 16 / STEPS);
-                if (u == 0 && step == STEPS - 1) {
-#pragma unroll
-                    for (int nb = 0; nb < NB; nb++) {
-                        const uint32_t sv = quad_hi(s_cur[nb], Q);
-                        if constexpr (G32) {  // the lane halves hold the two groups' scales
-                            const auto both = __builtin_amdgcn_permlane32_swap(sv, sv, false, false);
-                            scale[nb][0] = __uint_as_float(both[0]);
-                            scale[nb][1] = __uint_as_float(both[1]);
-                        } else {
-                            scale[nb][0] = __uint_as_float(sv);
-                        }
-                    }
-                }
+                if (u == 0 && step == STEPS - 1) take_scales8(Q);
                 if (last_mb) {
                     if (t > 0) expand8(t - 1);
                     read_codes8(t, sa_next);
@@ -930,23 +934,86 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         __builtin_amdgcn_sched_barrier(0);
         sa_carried = sa_next;
     };
-    // blocks 0 .. STAGES-1 were requested before the scan of the scale rows (any wait of the compiler's for the loads since then has
+    // BITS 8 with 32 rows a wavefront: a block's codes are expanded, then multiplied, then its sums scaled, while the other two
+    // wavefronts of the SIMD fill the matrix cores.  block8's pipeline takes 196 registers for 64 x 128 tiles (groups of 32 178), which
+    // leaves two wavefronts a SIMD where LDS has room for three; here 136 (164).  us, pipeline -> here: 777 x 2560 x 3072 on 64 x 128
+    // tiles 63.6 -> 53.4, 512 tokens through 128 experts (2816 / 704) gate|up 160.9 -> 151.5, down 100.3 -> 85.7, groups of 32 182.5 ->
+    // 179.1 and 105.7 -> 89.7; 777 x 2048 x 2560 on 32 x 256 tiles, one a CU, 29.0 -> 28.1, 777 x 2560 x 20480 188 -> 172.
+    // The copies of block g + STAGES - 1 go to the stage that was last read in block g - 1; in block 1 they follow the first use of
+    // its ordinary loads.
+    [[maybe_unused]] auto whole8 = [&](auto q_tag, int g) __attribute__((always_inline)) {
+        constexpr int Q = decltype(q_tag)::value;
+        const int sa = sa_carried, st2 = sa == 0 ? STAGES - 1 : sa - 1, g2 = min(g + STAGES - 1, G - 1);
+        const bool refill = Q == 1 && refills(g);
+        auto request = [&]() __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < NA; c++) issue_a1(c, g2, st2);
+#pragma unroll
+            for (int c = 0; c < NBC; c++) issue_b(c, g2, st2);
+        };
+        if constexpr (Q == 0) {
+            read_quad(0, quad_at, s_cur);
+            read_quad(1, quad_at, b_cur);
+        }
+        if constexpr (Q == 1) {
+            if (refill) load_segment(std::false_type{}, segment + 1, piece);
+            load_xs(g >> 2);
+        } else {
+            request();
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            read_codes8(t, sa);
+            expand8(t);
+        }
+        take_scales8(Q);
+#pragma unroll
+        for (int t = 0; t < 4; t++) read_a8(t, 0, sa);
+#pragma unroll
+        for (int u = 0; u < GROUPS; u++) {
+#pragma unroll
+            for (int step = 0; step < STEPS; step++)
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++)
+                    part[0][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a8[u * STEPS + step], b8[nb][u * STEPS + step], step ? part[0][nb] : f32x16_t{}, 0, 0, 0);
+            scale_part(q_tag, u + 1, 0, 16);
+        }
+        if constexpr (Q == 1) {
+            __builtin_amdgcn_sched_barrier(0);
+            if (refill) store_segment(segment + 1, piece);
+            asm volatile("" : "+v"(xs_cur[0].x), "+v"(xs_cur[0].y), "+v"(xs_cur[0].z), "+v"(xs_cur[0].w));
+            __builtin_amdgcn_sched_barrier(0);
+            request();
+        }
+        if constexpr (Q == 3) {
+            affine(3);
+            next_quad();
+        }
+        // (or the compiler moves the scaling behind the next branch, and the partial sums stay in registers until there)
+#pragma unroll
+        for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(out[0][nb]));
+        sa_carried = sa == STAGES - 1 ? 0 : sa + 1;
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(still_out(Q)) : "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // blocks 0 .. DEPTH-1 were requested before the scan of the scale rows (any wait of the compiler's for the loads since then has
     // drained those copies too)
     __builtin_amdgcn_sched_barrier(0);
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((STAGES - 1) * (B8 ? NA + NBC : NA)) : "memory");  // block 0 has landed
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((DEPTH - 1) * (B8 ? NA + NBC : NA)) : "memory");  // block 0 has landed
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     auto run = [&](auto q_tag, int g) __attribute__((always_inline)) {
-        if constexpr (B8) block8(q_tag, g); else block(q_tag, g);
+        if constexpr (WHOLE) whole8(q_tag, g); else if constexpr (B8) block8(q_tag, g); else block(q_tag, g);
     };
-    if constexpr (B8) {
+    if constexpr (B8 && !WHOLE) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
             read_codes8(t, 0);
             expand8(t);
             read_a8(t, 0, 0);
         }
-    } else {
+    } else if constexpr (!B8) {
         read_quad(0, 0, s_cur);
         read_codes(0);
         take_scale(s_cur, 0);
@@ -976,7 +1043,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-        } else if (g + (B8 ? 2 : 1) >= G) {
+        } else if (g + (B8 && !WHOLE ? 2 : 1) >= G) {
             load_xs(g >> 2);
         }
         affine(G - 1 - g);
@@ -1183,7 +1250,7 @@ static const QmmHalfEntry kQmmHalfTable[] = {
     AQ_QMMH8(2, 2, 2, 2, 3, 16, ""),      // 128 x 128
     AQ_QMMH8(2, 2, 2, 4, 3, 16, ""),     // 128 x 256, eight wavefronts
     AQ_QMMH8(2, 2, 1, 4, 3, 8, ""),
-    AQ_QMMH8(1, 2, 1, 4, 3, 16, ""),
+    AQ_QMMH8(1, 2, 1, 4, 3, 8, ""),
     AQ_QMMH8(1, 2, 2, 2, 3, 8, ""),      // 64 x 128 (4-bit tiles of that size, unsplit 167 -> 152 us on 509 x 15360 x 3840, lost to
                                                   // 128 x 128 and 192 x 256 with shares of K: 117 -> 142)
 };
