@@ -331,16 +331,16 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     constexpr bool XS_LDS = !B8 && MB >= 3;  // the sums of x of a quad go through LDS
     constexpr int NX = (BM / 32 + NWAVE - 1) / NWAVE;  // copies of them a wavefront issues
     constexpr int NA = A_BLOCKS / NWAVE;  // A copies a wavefront issues per block
-    constexpr bool WHOLE = B8 && MB == 1;               // a block at a time (whole8)
+    constexpr bool WHOLE = MB == 1;                     // a block at a time (whole)
     constexpr int DEPTH = WHOLE ? STAGES - 1 : STAGES;  // blocks requested ahead of the loop
     // Behind the barrier of block g the copies of A's block g + STAGES are issued.  BITS 4: and, in a stage's first block, those of B's
-    // stage after the next, two blocks before its codes are read; BITS 8: and B's block g + STAGES (WHOLE: ahead of the barrier of
-    // block g, of block g + STAGES - 1).  still_out: the copies that may
-    // be on their way at the barrier of block Q of a quad: A of block g + 1 has to have landed and with it the codes that are
-    // read up to the next barrier.
+    // stage after the next, two blocks before its codes are read; BITS 8: and B's block g + STAGES.  WHOLE: ahead of the barrier of
+    // block g those of A's (and BITS 8's) block g + STAGES - 1 and, in a stage's first block, of BITS 4's next stage.  still_out: the
+    // copies that may be on their way at the barrier of block Q of a quad: A of block g + 1 has to have landed and with it the codes
+    // that are read up to the next barrier.
     static_assert(STAGES <= 3, "waits are counted for two or three stages");
     auto still_out = [=](int q) constexpr {
-        return B8 ? (STAGES - 2) * (NA + NBC) : (STAGES - 2) * NA + ((q & 1) ? NBC : 0) + (XS_LDS && q == 1 ? NX : 0);
+        return B8 ? (STAGES - 2) * (NA + NBC) : (STAGES - 2) * NA + ((q & 1) != WHOLE ? NBC : 0) + (XS_LDS && q == 1 ? NX : 0);
     };
 
     extern __shared__ __align__(16) uint8_t lds[];
@@ -451,7 +451,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     // the first blocks are on their way while the prologue scans the scale rows
     if constexpr (!B8)
 #pragma unroll
-        for (int st = 0; st < 2; st++)
+        for (int st = 0; st < (WHOLE ? 1 : 2); st++)
 #pragma unroll
             for (int c = 0; c < NBC; c++) issue_b(c, min(gb / QB + st, (Gall - 1) / QB), st);
 #pragma unroll
@@ -700,12 +700,12 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     // itself, where expanding a whole block ahead of its MFMAs left the matrix cores to the one other wavefront of the SIMD.
     // The only barrier of a block is in the middle of its last step, behind MFMAs that need nothing of the next block.
     constexpr bool TWO_A = MB <= 3;  // A's next fragments in registers of their own; else over those just multiplied
-    f16x8_t afr[TWO_A ? 2 : 1][MB];
-    uint32_t bfr[2][NB][4];
+    f16x8_t afr[WHOLE ? 4 : TWO_A ? 2 : 1][MB];
+    uint32_t bfr[WHOLE ? 4 : 2][NB][4];
     uint4 cw[NB];               // the block's words of this lane
     f16x2_t s2[NB], m24[NB];    // its scale, brought into fp16 range (8 significant bits: exact), and -24 times it (10 bits)
     auto read_a = [&](int mb, int t, int stage) {
-        afr[TWO_A ? t & 1 : 0][mb] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
+        afr[WHOLE ? t : TWO_A ? t & 1 : 0][mb] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
     };
     // row (wave_n * NB + nb) * 32 + j, words 4h .. 4h+3, of block Q of a quad
     auto read_codes = [&](int q) {
@@ -727,7 +727,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         for (int i = from; i < to; i++) {
             const int nb = i >> 2;
             const uint32_t w = t == 0 ? cw[nb].x : t == 1 ? cw[nb].y : t == 2 ? cw[nb].z : cw[nb].w;
-            uint32_t& to_reg = bfr[t & 1][nb][i & 3];
+            uint32_t& to_reg = bfr[WHOLE ? t : t & 1][nb][i & 3];
             if ((i & 3) == 0) to_reg = expand_pair<0>(w, mask_s, magic_v, s2[nb], m24[nb]);
             if ((i & 3) == 1) to_reg = expand_pair<1>(w, mask_s, magic_v, s2[nb], m24[nb]);
             if ((i & 3) == 2) to_reg = expand_pair<2>(w, mask_s, magic_v, s2[nb], m24[nb]);
@@ -934,49 +934,68 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         __builtin_amdgcn_sched_barrier(0);
         sa_carried = sa_next;
     };
-    // BITS 8 with 32 rows a wavefront: a block's codes are expanded, then multiplied, then its sums scaled, while the other two
-    // wavefronts of the SIMD fill the matrix cores.  block8's pipeline takes 196 registers for 64 x 128 tiles (groups of 32 178), which
-    // leaves two wavefronts a SIMD where LDS has room for three; here 136 (164).  us, pipeline -> here: 777 x 2560 x 3072 on 64 x 128
-    // tiles 63.6 -> 53.4, 512 tokens through 128 experts (2816 / 704) gate|up 160.9 -> 151.5, down 100.3 -> 85.7, groups of 32 182.5 ->
-    // 179.1 and 105.7 -> 89.7; 777 x 2048 x 2560 on 32 x 256 tiles, one a CU, 29.0 -> 28.1, 777 x 2560 x 20480 188 -> 172.
-    // The copies of block g + STAGES - 1 go to the stage that was last read in block g - 1; in block 1 they follow the first use of
-    // its ordinary loads.
-    [[maybe_unused]] auto whole8 = [&](auto q_tag, int g) __attribute__((always_inline)) {
+    // 32 rows a wavefront: a block's codes are expanded, then multiplied (BITS 8: then its sums scaled), while the other wavefronts of
+    // the SIMD fill the matrix cores.  With two MFMAs a step the pipelines above have too little to hide LDS latency behind.  us,
+    // pipeline -> here.  BITS 4, 32 x 256 tiles: 413 x 4096 x 3328 46.0 -> 39.7, 413 x 1024 x 3328 17.4 -> 15.7, in groups of 32 300 x
+    // 2048 x 3328 28.6 -> 25.2; 512 tokens through 128 experts (2816 / 704) gate|up 121.8 -> 114.6, down 74.7 -> 72.4; level at three
+    // tiles a CU.  BITS 8: block8 takes 196 registers for 64 x 128 tiles (groups of 32 178), which leaves two wavefronts a SIMD where
+    // LDS has room for three; here 136 (164): 777 x 2560 x 3072 63.6 -> 53.4, the experts 160.9 -> 151.5 and 100.3 -> 85.7, in groups
+    // of 32 182.5 -> 179.1 and 105.7 -> 89.7; 32 x 256 tiles 777 x 2048 x 2560 29.0 -> 28.1, 777 x 2560 x 20480 188 -> 172.
+    // The copies of block g + STAGES - 1 go to the stage that was last read in block g - 1, BITS 4's next stage of B likewise; in
+    // block 1 they follow the first use of its ordinary loads.
+    [[maybe_unused]] auto whole = [&](auto q_tag, int g) __attribute__((always_inline)) {
         constexpr int Q = decltype(q_tag)::value;
         const int sa = sa_carried, st2 = sa == 0 ? STAGES - 1 : sa - 1, g2 = min(g + STAGES - 1, G - 1);
         const bool refill = Q == 1 && refills(g);
         auto request = [&]() __attribute__((always_inline)) {
 #pragma unroll
             for (int c = 0; c < NA; c++) issue_a1(c, g2, st2);
+            if constexpr (B8 || Q % 2 == 0)
 #pragma unroll
-            for (int c = 0; c < NBC; c++) issue_b(c, g2, st2);
+                for (int c = 0; c < NBC; c++) B8 ? issue_b(c, g2, st2) : issue_b(c, min(g / QB + 1, (Gall - 1) / QB), (Q >> 1) ^ 1);
         };
         if constexpr (Q == 0) {
-            read_quad(0, quad_at, s_cur);
+            if constexpr (B8) read_quad(0, quad_at, s_cur);
             read_quad(1, quad_at, b_cur);
         }
+        if constexpr (Q == 3 && !B8) read_quad(0, quad_at + 1 == quads ? 0 : quad_at + 1, s_nxt);  // (behind the end of K: anything)
         if constexpr (Q == 1) {
             if (refill) load_segment(std::false_type{}, segment + 1, piece);
             load_xs(g >> 2);
         } else {
             request();
         }
+        if constexpr (B8) {
 #pragma unroll
-        for (int t = 0; t < 4; t++) {
-            read_codes8(t, sa);
-            expand8(t);
-        }
-        take_scales8(Q);
+            for (int t = 0; t < 4; t++) {
+                read_codes8(t, sa);
+                expand8(t);
+            }
+            take_scales8(Q);
 #pragma unroll
-        for (int t = 0; t < 4; t++) read_a8(t, 0, sa);
+            for (int t = 0; t < 4; t++) read_a8(t, 0, sa);
 #pragma unroll
-        for (int u = 0; u < GROUPS; u++) {
+            for (int u = 0; u < GROUPS; u++) {
 #pragma unroll
-            for (int step = 0; step < STEPS; step++)
+                for (int step = 0; step < STEPS; step++)
+#pragma unroll
+                    for (int nb = 0; nb < NB; nb++)
+                        part[0][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a8[u * STEPS + step], b8[nb][u * STEPS + step], step ? part[0][nb] : f32x16_t{}, 0, 0, 0);
+                scale_part(q_tag, u + 1, 0, 16);
+            }
+        } else {
+            read_codes(Q);
+            take_scale(s_cur, Q);
+#pragma unroll
+            for (int t = 0; t < 4; t++) read_a(0, t, sa);
+#pragma unroll
+            for (int t = 0; t < 4; t++) {
+                expand_some(t, 0, NB * 4);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++)
-                    part[0][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a8[u * STEPS + step], b8[nb][u * STEPS + step], step ? part[0][nb] : f32x16_t{}, 0, 0, 0);
-            scale_part(q_tag, u + 1, 0, 16);
+                    out[0][nb] = __builtin_amdgcn_mfma_f32_32x32x16_f16(afr[t][0], __builtin_bit_cast(f16x8_t, make_uint4(bfr[t][nb][0], bfr[t][nb][1], bfr[t][nb][2], bfr[t][nb][3])),
+                                                                        out[0][nb], 0, 0, 0);
+            }
         }
         if constexpr (Q == 1) {
             __builtin_amdgcn_sched_barrier(0);
@@ -987,9 +1006,12 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         }
         if constexpr (Q == 3) {
             affine(3);
+            if constexpr (!B8)
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++) s_cur[nb] = s_nxt[nb];
             next_quad();
         }
-        // (or the compiler moves the scaling behind the next branch, and the partial sums stay in registers until there)
+        // (or the compiler moves work behind the next branch, and what it reads stays in registers until there: BITS 8's partial sums)
 #pragma unroll
         for (int nb = 0; nb < NB; nb++) asm volatile("" : "+v"(out[0][nb]));
         sa_carried = sa == STAGES - 1 ? 0 : sa + 1;
@@ -1004,7 +1026,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     auto run = [&](auto q_tag, int g) __attribute__((always_inline)) {
-        if constexpr (WHOLE) whole8(q_tag, g); else if constexpr (B8) block8(q_tag, g); else block(q_tag, g);
+        if constexpr (WHOLE) whole(q_tag, g); else if constexpr (B8) block8(q_tag, g); else block(q_tag, g);
     };
     if constexpr (B8 && !WHOLE) {
 #pragma unroll
@@ -1015,11 +1037,13 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         }
     } else if constexpr (!B8) {
         read_quad(0, 0, s_cur);
-        read_codes(0);
-        take_scale(s_cur, 0);
+        if constexpr (!WHOLE) {
+            read_codes(0);
+            take_scale(s_cur, 0);
 #pragma unroll
-        for (int mb = 0; mb < MB; mb++) read_a(mb, 0, 0);
-        expand_some(0, 0, NB * 4);
+            for (int mb = 0; mb < MB; mb++) read_a(mb, 0, 0);
+            expand_some(0, 0, NB * 4);
+        }
     }
     int g = gb;
     for (; g + 4 <= G; g += 4) {
