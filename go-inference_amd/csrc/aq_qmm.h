@@ -87,7 +87,7 @@ struct QmmSegment {
     void* y;
     int N;
     int ksplit, gsplit;    // workgroups that share a tile along K, 64-code blocks of K each takes (qmmh_split)
-    int strips, unit_end;  // filled by the launcher: column strips, and column units (strips x ksplit) up to and with this matrix
+    int strips;            // filled by the launcher: column strips
     float* partial;        // filled by the launcher: partial tiles of a K split
 };
 struct QmmHalfArgs {
@@ -100,7 +100,6 @@ struct QmmHalfArgs {
     int M, K;
     int bits, gs_blocks, out_f32, act;
     int mblks, tiles_m;
-    int units;    // column units of all matrices
     int group_m;  // row bands of a group of tiles
     // routes grouped by expert (aq_moe_group.hip), or null
     const RouteChunk* chunks;
@@ -118,6 +117,26 @@ struct QmmHalfCall {
     const int32_t *nchunks, *route_x, *route_of, *live_rows;
     int most_chunks, most_rows, expert_rows, row_base, row_base2;
 };
+// The tile that workgroup `place` of a grid works on: the matrix (negative: none), the tile's number in it, the matrix's column units
+// (strips x shares of K: each share stores fp32 partial tiles).  Workgroups are dealt to the 8 XCDs round-robin, so every 8th one
+// shares an L2.  Each XCD has a contiguous run of the tiles of every matrix; what is left over of a matrix goes to the XCDs behind
+// those that the one before it ended with.  (One run over the tiles of all matrices gave q's long ones to the first XCDs and the short
+// shares of k and v to the others.  us with the sums of shares, that -> this, 8 bit on 64 x 128 tiles: 777 x 2560 x (2048, 512, 512),
+// k and v in five shares, 58 -> 38; 562 x 2816 x (2496, 1152, 1152) in six 93 -> 46.)
+struct QmmTileAt {
+    int seg, id, units;
+};
+__host__ __device__ inline QmmTileAt qmmh_tile_at(const QmmSegment* seg, int nseg, int row_bands, int place) {
+    int in_run = place >> 3, ends = 0;
+    for (int i = 0; i < nseg; i++) {
+        const int units = seg[i].strips * seg[i].ksplit, tiles = row_bands * units, left = tiles & 7;
+        const int xcd = (place - ends) & 7, run = (tiles >> 3) + (xcd < left);
+        if (in_run < run) return {i, xcd * (tiles >> 3) + (xcd < left ? xcd : left) + in_run, units};
+        in_run -= run;
+        ends += left;
+    }
+    return {-1, 0, 0};
+}
 int qmmh_variant_count();
 const QmmVariant* qmmh_variant(int idx);
 int qmmh_x_kind(int bits, int group_size);  // the pass over x their kernels need (kXReady*)

@@ -31,6 +31,7 @@
 #include "aq_lds_copy.h"
 #include "aq_qmm.h"
 
+#include <algorithm>
 #include <cmath>
 #include <type_traits>
 
@@ -352,24 +353,18 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     const uint32_t abuf_at = __builtin_amdgcn_readfirstlane(lds_offset(lds));
     const uint32_t bbuf_at = abuf_at + STAGES * A_STAGE;
 
-    // workgroups are dealt to the 8 XCDs round-robin, so every 8th one shares an L2; give each XCD a
-    // contiguous run of tiles in row-band-major order
-    // (a matrix with K shared out has ksplit column units per column strip: each stores fp32 partial tiles)
-    const int T = __builtin_amdgcn_readfirstlane((a.chunks ? *a.nchunks : a.tiles_m) * a.units);
-    const int per_xcd = (T + 7) / 8;
-    const int id = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per_xcd || id >= T) return;
+    const int row_bands = __builtin_amdgcn_readfirstlane(a.chunks ? *a.nchunks : a.tiles_m);
+    const QmmTileAt at = qmmh_tile_at(a.seg, a.nseg, row_bands, (int)blockIdx.x);
+    if (at.seg < 0) return;
+    const int seg = __builtin_amdgcn_readfirstlane(at.seg);
+    const int id = at.id, units = __builtin_amdgcn_readfirstlane(at.units);
     // tiles in groups of a.group_m row bands, column unit by column unit inside a group: the tiles an XCD works on at a
     // time then cover a patch of the output that is about as tall as it is wide in bytes read
-    const int group = __builtin_amdgcn_readfirstlane(id / (a.group_m * a.units));
-    const int in_group = id - group * a.group_m * a.units;
-    const int bands = min(a.group_m, T / a.units - group * a.group_m);
-    int unit = __builtin_amdgcn_readfirstlane(in_group / bands);
+    const int group = __builtin_amdgcn_readfirstlane(id / (a.group_m * units));
+    const int in_group = id - group * a.group_m * units;
+    const int bands = min(a.group_m, row_bands - group * a.group_m);
+    const int unit = __builtin_amdgcn_readfirstlane(in_group / bands);
     const int tm = __builtin_amdgcn_readfirstlane(group * a.group_m + in_group - unit * bands);
-    int seg = 0;
-    while (seg + 1 < a.nseg && unit >= a.seg[seg].unit_end) seg++;
-    seg = __builtin_amdgcn_readfirstlane(seg);
-    if (seg > 0) unit -= a.seg[seg - 1].unit_end;
     const int split = __builtin_amdgcn_readfirstlane(unit / a.seg[seg].strips);
     const int tn = __builtin_amdgcn_readfirstlane(unit - split * a.seg[seg].strips);
     float* const partial = a.seg[seg].partial;  // null: this workgroup's sums are whole
@@ -1412,18 +1407,22 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     a.mblks = mblks;
     const int bm = qmmh_rows(idx), bn = e.v.wn * e.v.nb * 32;
     char* partial = static_cast<char*>(workspace) + ((qmmt_workspace_bytes(rows, q.K) + 255) & ~(size_t)255);
-    int units = 0, split_segments = 0;
+    int split_segments = 0;
     int64_t split_work = 0;
     bool by4 = true;
     for (int i = 0; i < q.nseg; i++) {
+        a.seg[i] = q.seg[i];
+        if (a.seg[i].ksplit <= 1) a.seg[i].ksplit = 1, a.seg[i].gsplit = (q.K / 64 + 3) / 4 * 4;
+    }
+    if (!q.pair) std::stable_sort(a.seg, a.seg + q.nseg, [](const QmmSegment& l, const QmmSegment& r) { return l.gsplit > r.gsplit; });
+    a.tiles_m = (rows + bm - 1) / bm;
+    int64_t T = 0;  // tiles
+    for (int i = 0; i < q.nseg; i++) {
         QmmSegment& seg = a.seg[i];
-        seg = q.seg[i];
         seg.partial = nullptr;
         seg.strips = (int)half_strips(idx, seg.N, q.pair);
-        if (seg.ksplit <= 1) seg.ksplit = 1, seg.gsplit = (q.K / 64 + 3) / 4 * 4;
         if (q.pair && i == 1) break;
-        units += seg.strips * seg.ksplit;
-        seg.unit_end = units;
+        T += (int64_t)(q.chunks ? q.most_chunks : a.tiles_m) * seg.strips * seg.ksplit;
         if (seg.ksplit > 1) {
             if (q.chunks || seg.gsplit % 4 != 0 || (int64_t)(seg.ksplit - 1) * seg.gsplit * 64 >= q.K) return hipErrorInvalidValue;
             seg.partial = reinterpret_cast<float*>(partial);
@@ -1433,8 +1432,6 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
             by4 = by4 && seg.N % 4 == 0;
         }
     }
-    a.units = units;
-    a.tiles_m = (rows + bm - 1) / bm;
     {
         // the patch an XCD's 32 CUs work on at a time: group_m row bands by the rest in column strips, fewest bytes per step
         // of K (4096 x 4096 x 16384: 598 -> 571 us against one band, 1024 x 4096 x 16384 on 64-row tiles 284 -> 201 us)
@@ -1452,8 +1449,7 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     a.expert_rows = q.expert_rows;
     a.row_base = q.row_base;
     a.row_base2 = q.row_base2;
-    const int T = (q.chunks ? q.most_chunks : a.tiles_m) * units;
-    const unsigned grid = (unsigned)(((T + 7) / 8) * 8);
+    const unsigned grid = (unsigned)((T + 7) / 8 * 8);
     const QmmHalfKernel fn = g32 ? e.fn32 : e.fn;
     rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), (size_t)e.lds_bytes);
     if (rc != hipSuccess) return rc;

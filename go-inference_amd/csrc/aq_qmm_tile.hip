@@ -541,7 +541,7 @@ hipError_t qmmt_launch_splitk(int idx, const QmmArgs& q, void* workspace, int ks
         c.K = q.K;
         c.group_size = q.gs_blocks * 64;
         c.bits = qmmt_variant(idx)->bits;
-        c.seg[0] = {q.w, q.s, q.b, q.y, q.N, 1, 0, 0, 0, nullptr};
+        c.seg[0] = {q.w, q.s, q.b, q.y, q.N, 1, 0, 0, nullptr};
         c.nseg = 1;
         c.out_f32 = q.out_f32;
         c.x_ready = q.x_ready;
