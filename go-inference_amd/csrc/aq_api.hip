@@ -1090,7 +1090,7 @@ int aq_qmm_multi(aq_ctx* ctx, const void* x, int count, const void* const* packe
             seg.b = static_cast<const uint16_t*>(biases[i]);
             seg.y = y[i];
             seg.N = N[i];
-            aq::qmmh_split(M, K, bits, &seg, ctx->cu_count);
+            aq::qmmh_split(M, K, group_size, bits, &seg, ctx->cu_count);
             in_grid |= 1u << i;
         }
     if (q.nseg > 0) {

@@ -142,9 +142,9 @@ const QmmVariant* qmmh_variant(int idx);
 int qmmh_x_kind(int bits, int group_size);  // the pass over x their kernels need (kXReady*)
 int qmmh_rows(int idx);  // rows of x of a workgroup tile
 hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream);
-// How a matrix of seg->N columns shares K out for M rows of x: a function of M, K, N and the code width alone, so that the call of several
-// matrices, the gated pair and a call of its own add in the same order and give the same bytes.
-void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count);
+// How a matrix of seg->N columns shares K out for M rows of x: a function of M, K, N, the group size and the code width alone, so that
+// the call of several matrices, the gated pair and a call of its own add in the same order and give the same bytes.
+void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_count);
 // The kernel for these matrices (the bytes of a result do not depend on it).
 int qmmh_pick(const QmmHalfCall& q, int cu_count);
 size_t qmmh_partial_bytes(const QmmHalfCall& q);

@@ -53,11 +53,12 @@ size_t qmm_scratch_bytes(int M, int K, int N, int cu_count) {
         q.M = M;
         q.nseg = 1;
         q.seg[0].N = N;
-        for (int bits : {4, 8}) {
-            qmmh_split(M, K, bits, &q.seg[0], cu_count);
-            const size_t half = qmmh_partial_bytes(q);
-            partial = half > partial ? half : partial;
-        }
+        for (int bits : {4, 8})
+            for (int group : {32, 64}) {
+                qmmh_split(M, K, group, bits, &q.seg[0], cu_count);
+                const size_t half = qmmh_partial_bytes(q);
+                partial = half > partial ? half : partial;
+            }
     }
     return xbytes + ((partial + 255) & ~(size_t)255);
 }
@@ -102,7 +103,7 @@ bool qmmh_runs(int M, int K, int N, int group_size, int bits) {
 
 int qmmh_run(hipStream_t stream, Workspace* ws, int cu_count, int idx, QmmHalfCall& q, const char** last_variant, FailFn fail, int* x_state) {
     if (!q.chunks)
-        for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, q.bits, &q.seg[i], cu_count);
+        for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) qmmh_split(q.M, q.K, q.group_size, q.bits, &q.seg[i], cu_count);
     const size_t xbytes = (qmmt_workspace_bytes(q.chunks ? q.most_rows : q.M, q.K) + 255) & ~(size_t)255;
     const size_t need = xbytes + qmmh_partial_bytes(q);
     const uint64_t moves = ws->moves;

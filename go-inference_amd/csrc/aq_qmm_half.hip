@@ -1290,19 +1290,30 @@ size_t qmmh_partial_bytes(const QmmHalfCall& q) {
     return bytes;
 }
 
-// What a workgroup tile of each kernel takes: microseconds per 64-code block of K alone on its CU, the same per tile when the
-// CU has more of them, and outside the loop.  From runs at K = 1024 and 4096 with 1/2, 1, 2, 3 and 4 tiles per CU (a CU's
-// clock and its share of L2 depend on how busy the rest of the chip is: 256 x 256 tiles take 1.73 alone and 1.95 in a row).
+// What a workgroup tile of each kernel takes: microseconds per 64-code block of K with one tile a CU on all CUs, the same per tile
+// when CUs have more of them, outside the loop, and by how much of itself the loop is shorter when the rest of the chip idles (its
+// clock and its share of L2).  First row: groups of 64 and 128, second: of 32.  Fitted to 2000 launches on weights from memory, 66 to
+// 2048 rows (groups of 32: 509), K of 768 to 15360, 256 to 17664 columns, in 1 to 16 shares of K: predicted within 4 to 5 % (rms).
+// What this picks takes 1 % longer than the best of a shape's measured forms; constants from K of 1024 and 4096, without groups of
+// 32 and with shares at twice their cost took 2 to 4 %: 2048 x 14336 x 4096 unsplit 255 -> 234 in two shares, 509 x 15360 x 3840 in
+// groups of 32 99 -> 94, 999 x 9920 x 4032 of 8 bit 159 -> 121.
 struct QmmHalfCost {
-    double solo, full, fixed;
+    double solo, full, fixed, idle;
 };
-static const QmmHalfCost kQmmHalfCost[] = {{0.99, 1.12, 8.5}, {0.95, 1.0, 10.0}, {1.73, 1.95, 12.0}, {1.37, 1.4, 10.0}, {0.65, 0.61, 5.0}, {0.67, 0.62, 5.0}, {0.61, 0.44, 3.0},
-                                           {0.75, 0.65, 5.0}, {1.17, 1.27, 6.5}, {0.77, 0.69, 5.0}, {0.66, 0.49, 3.0}, {0.58, 0.435, 3.0}};
+static const QmmHalfCost kQmmHalfCost[2][12] = {
+    {{1.01, 1.13, 11.5, 0.21}, {1.00, 0.95, 12.0, 0.23}, {1.72, 1.98, 11.5, 0.38}, {1.23, 1.45, 12.5, 0.24}, {0.74, 0.59, 9.0, 0.26}, {0.78, 0.61, 9.5, 0.27},
+     {0.55, 0.44, 8.5, 0.22}, {0.92, 0.65, 8.0, 0.21}, {1.22, 1.29, 9.5, 0.19}, {0.94, 0.69, 8.0, 0.23}, {0.73, 0.54, 7.0, 0.21}, {0.62, 0.43, 7.0, 0.20}},
+    {{1.10, 1.19, 10.5, 0.13}, {1.16, 0.98, 11.5, 0.14}, {1.79, 1.92, 10.0, 0.24}, {1.29, 1.25, 11.0, 0.14}, {0.75, 0.62, 8.0, 0.18}, {0.87, 0.67, 8.5, 0.21},
+     {0.65, 0.49, 7.5, 0.22}, {1.01, 0.71, 8.0, 0.14}, {1.38, 1.46, 10.0, 0.16}, {1.12, 0.80, 8.5, 0.16}, {0.89, 0.63, 7.0, 0.17}, {0.71, 0.50, 7.0, 0.18}}};
+static_assert(sizeof(kQmmHalfCost[0]) / sizeof(kQmmHalfCost[0][0]) == sizeof(kQmmHalfTable) / sizeof(kQmmHalfTable[0]), "a cost for each kernel");
 
-// Microseconds of kernel i over `tiles` tiles of `blocks` blocks each.
-static double half_cost(int i, int64_t tiles, int blocks, int cus) {
-    const double work = tiles > cus ? kQmmHalfCost[i].full * ceil((double)tiles / cus) : 0.0, least = kQmmHalfCost[i].solo;
-    return kQmmHalfCost[i].fixed + blocks * (work > least ? work : least);
+// Microseconds of kernel i over `tiles` tiles of `most` blocks at most and `all` blocks together.  (Matrices in one grid with different
+// shares: at the most blocks for every tile, what this picked took 2 to 7 % longer than the best tile; here 0.2 to 1.5 %.)
+static double half_cost(int i, int group_size, int64_t tiles, int most, int64_t all, int cus) {
+    const QmmHalfCost& c = kQmmHalfCost[group_size == 32][i];
+    const double load = (double)tiles / cus, per_cu = load > 1.0 ? ceil(load) : 1.0;
+    const double longest = c.solo * most, full = per_cu > 1.0 ? c.full * per_cu * ((double)all / tiles) : 0.0;
+    return c.fixed + (full > longest ? full : longest) * (1.0 - c.idle * (1.0 - load / per_cu));
 }
 static int64_t half_strips(int i, int N, bool pair) {
     const int bn = kQmmHalfTable[i].v.wn * kQmmHalfTable[i].v.nb * 32 / (pair ? 2 : 1);
@@ -1310,7 +1321,7 @@ static int64_t half_strips(int i, int N, bool pair) {
 }
 static int64_t half_bands(int i, int M) { return (M + qmmh_rows(i) - 1) / qmmh_rows(i); }
 
-void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count) {
+void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_count) {
     const int cus = cu_count > 0 ? cu_count : 256;
     const int G = K / 64;
     double best_us = 1e30;
@@ -1321,10 +1332,12 @@ void qmmh_split(int M, int K, int bits, QmmSegment* seg, int cu_count) {
         const int64_t tiles = half_bands(i, M) * half_strips(i, seg->N, false);
         for (int ks = 1; ks <= 16; ks++) {
             const int gsplit = ((G + ks - 1) / ks + 3) / 4 * 4;
-            if (ks > 1 && (gsplit < 8 || (int64_t)(ks - 1) * gsplit >= G || (int64_t)tiles * ks > 4 * cus)) continue;
-            double us = half_cost(i, tiles * ks, ks > 1 ? gsplit : G, cus);
-            // partial tiles: written and read once at about 3 bytes per nanosecond, one more launch
-            if (ks > 1) us += 3.0 + (double)ks * M * (double)seg->N * 8 / 3e6;
+            if (ks > 1 && (gsplit < 8 || tiles * ks > 4 * cus)) break;
+            if (ks > 1 && (int64_t)(ks - 1) * gsplit >= G) continue;
+            const int blocks = ks > 1 ? gsplit : G;
+            double us = half_cost(i, group_size, tiles * ks, blocks, tiles * ks * blocks, cus);
+            // partial tiles: one more launch, and their bytes (two of 2048 x 4096: 14 us for the sums, 10 for the stores)
+            if (ks > 1) us += 3.0 + (double)ks * M * (double)seg->N * 4 / 2.4e6;
             if (us < best_us) best_us = us, seg->ksplit = ks, seg->gsplit = gsplit;
         }
     }
@@ -1349,14 +1362,16 @@ int qmmh_pick(const QmmHalfCall& q, int cu_count) {
     double best_us = 1e30;
     for (int i = 0; i < qmmh_variant_count(); i++) {
         if (kQmmHalfTable[i].v.bits != q.bits) continue;
-        int64_t tiles = 0;
-        int blocks = 0;
+        int64_t tiles = 0, all = 0;
+        int most = 0;
         for (int k = 0; k < (q.pair ? 1 : q.nseg); k++) {
-            tiles += half_bands(i, q.M) * half_strips(i, q.seg[k].N, q.pair) * q.seg[k].ksplit;
+            const int64_t t = half_bands(i, q.M) * half_strips(i, q.seg[k].N, q.pair) * q.seg[k].ksplit;
             const int b = q.seg[k].ksplit > 1 ? q.seg[k].gsplit : q.K / 64;
-            blocks = b > blocks ? b : blocks;
+            tiles += t;
+            all += t * b;
+            most = b > most ? b : most;
         }
-        const double us = half_cost(i, tiles, blocks, cus);
+        const double us = half_cost(i, q.group_size, tiles, most, all, cus);
         if (us < best_us) best_us = us, best = i;
     }
     return best;

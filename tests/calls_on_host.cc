@@ -309,6 +309,26 @@ static void test_shares_of_the_infinities() {
     }
 }
 
+// Tiles and shares of K of prompts, where the costs of the tiles decide and measured far apart (us, the other form -> this one).
+static void test_tiles_of_prompts() {
+    auto prompt = [](int M, int K, int N, int group, int bits) {
+        log_.clear();
+        CHECK(aq_qmm(ctx, X, W, S, B, Y, M, K, N, group, bits, 0) == AQ_OK, "%s", aq_last_error());
+        return log_.size();
+    };
+    // (pass over x, tiles, sums of shares)
+    for (auto [M, K, N, group, bits] : {std::array{2048, 14336, 4096, 64, 4}, {999, 9920, 4032, 64, 8}, {509, 15360, 3840, 32, 4}})  // 255 -> 234, 159 -> 121
+        CHECK(prompt(M, K, N, group, bits) == 3 && log_[2].is("qmmh_reduce"), "%d x %d x %d, %d bit: %zu launches", M, K, N, bits, log_.size());
+    CHECK(prompt(333, 1024, 1024, 64, 8) == 2, "333 rows: %zu launches", log_.size());  // 15 -> 14
+    // q|k|v of a prompt of 8 bit: 64 x 128 tiles, three workgroups a CU (55 -> 52)
+    const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+    void* y[3] = {Y, Y, Y};
+    const int N[3] = {2048, 512, 512};
+    log_.clear();
+    CHECK(aq_qmm_multi(ctx, X, 3, w, s, b, y, N, 777, 2560, 64, 8, 0) == AQ_OK && log_.size() > 1, "%s", aq_last_error());
+    CHECK(log_[1].is("qmmh_kernelILi8ELi1ELi2ELi2ELi2E"), "q|k|v of 777 rows: %s", log_[1].kernel.c_str());
+}
+
 int main() {
     for (int cus : {128, 512, 256}) {
         compute_units = cus;
@@ -317,7 +337,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities();
+        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities(), test_tiles_of_prompts();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");
