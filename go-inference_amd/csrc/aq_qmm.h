@@ -66,6 +66,7 @@ size_t qmmt_workspace_bytes(int M, int K);
 hipError_t qmmt_launch(int idx, const QmmArgs& a, void* workspace, hipStream_t stream);
 // The pass over x variant idx needs (kXReady*).
 int qmmt_x_kind(int idx);
+int qmmt_half_index(int idx);  // the fp16-operand kernel (qmmh_variant) that a tile variant is, or -1
 // The same with K shared out over ksplit workgroups per tile and a second kernel that adds the partial
 // tiles: for few rows of x, where M x N tiles alone leave most of the chip idle.
 size_t qmmt_splitk_bytes(int M, int N, int ksplit);

@@ -135,7 +135,10 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
                  const void* packed, const void* scales, const void* biases, void* y, int M, int K, int N,
                  int group_size, int bits, bool out_f32, FailFn fail, const float* gate, int act, int* x_state) {
     const bool mfma_ok = qmm_takes_gate(x, packed, K, group_size, bits);
-    if (forced < 0 && !gate && qmmh_takes(x, packed, K, group_size, bits) && qmmh_runs(M, K, N, group_size, bits)) {
+    // (a forced tile of theirs: groups of 32 here, in the shares of an unforced call; groups of 64 and 128 below, whole)
+    const int half = forced >= 0 && group_size == 32 ? qmmt_half_index(forced) : -1;
+    const bool half_runs = forced < 0 ? qmmh_runs(M, K, N, group_size, bits) : half >= 0 && qmmh_variant(half)->bits == bits;
+    if (half_runs && !gate && qmmh_takes(x, packed, K, group_size, bits)) {
         QmmHalfCall q{};
         q.x = static_cast<const uint16_t*>(x);
         q.M = M;
@@ -149,7 +152,7 @@ int qmm_dispatch(hipStream_t stream, Workspace* ws, int cu_count, int forced, co
         q.seg[0].N = N;
         q.nseg = 1;
         q.out_f32 = out_f32 ? 1 : 0;
-        const int rc = qmmh_run(stream, ws, cu_count, -1, q, last_variant, fail, x_state);
+        const int rc = qmmh_run(stream, ws, cu_count, half, q, last_variant, fail, x_state);
         if (rc != kQmmhNoScratch) return rc;
     }
     if (!mfma_ok) {

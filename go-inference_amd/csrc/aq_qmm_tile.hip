@@ -517,6 +517,11 @@ hipError_t qmmt_launch(int idx, const QmmArgs& q, void* workspace, hipStream_t s
     return qmmt_launch_splitk(idx, q, workspace, 1, stream);
 }
 
+int qmmt_half_index(int idx) {
+    idx -= tile_variants();
+    return idx >= 0 && idx < qmmh_variant_count() ? idx : -1;
+}
+
 int qmmt_x_kind(int idx) {
     const QmmVariant* v = qmmt_variant(idx);
     if (!v) return kXReadyNone;

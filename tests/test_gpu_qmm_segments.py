@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 # a segment is 8 or 16 elements of a row, 4 / gs_blocks of them (groups of 32: 8) a quad of four 64-code blocks.  Ends: one block, a
 # whole segment, one block into the next, the middle of a quad of the third; fewer than eight scales in all
 @pytest.mark.parametrize("bits", [4, 8])
-@pytest.mark.parametrize("gs,M,K,N", [(32, 33, 64, 3), (32, 97, 512, 67), (32, 40, 832, 131), (64, 65, 64, 5), (64, 97, 1024, 67), (64, 40, 1088, 131),
+@pytest.mark.parametrize("gs,M,K,N", [(32, 33, 64, 3), (32, 97, 512, 67), (32, 40, 832, 131), (32, 300, 1984, 131), (64, 65, 64, 5), (64, 97, 1024, 67), (64, 40, 1088, 131),
                                       (64, 130, 2240, 35), (128, 33, 128, 1), (128, 97, 2048, 67), (128, 40, 2176, 35)])
 def test_every_tile_over_segments_of_scales(ctx, bits, gs, M, K, N):
     import aq_mi355
@@ -21,8 +21,8 @@ def test_every_tile_over_segments_of_scales(ctx, bits, gs, M, K, N):
     dw = DeviceAffine(ctx, words, s, b)
     ref, first = F.reference_f64(x, words, s, b, bits, gs, K), None
     prefix = "qmmh_" if bits == 4 else "qmmh8_"
-    # (groups of 32 take the tile that the rule picks)
-    tiles = [(i, n) for i, n in enumerate(aq_mi355.variant_names(1)) if n.startswith(prefix)] if gs != 32 else [(-1, prefix)]
+    # (the rule's tile too: groups of 32 have its shares of K on every tile)
+    tiles = [(i, n) for i, n in enumerate(aq_mi355.variant_names(1)) if n.startswith(prefix)] + ([(-1, prefix)] if gs == 32 else [])
     for i, name in tiles:
         say("segments", name, gs, M, K, N)
         ctx.force_variant(1, i)
