@@ -301,10 +301,10 @@ __device__ __forceinline__ void fix_output(const QmmHalfArgs& a, const QmmSegmen
 // tile kernels of aq_qmm_tile.hip.  Against those: two vector instructions per pair of codes instead of three, several
 // matrices in one grid, the gated pair, groups of 32 and expert slabs.  A step of the MFMA is 16 consecutive codes, so that
 // groups of 32 are two steps each; bytes are staged one 64-code block at a time, in as many stages as A.
-// Measured (us; bf16-code tiles -> here): 2048 x 4096 x 14336 395 -> 329, a layer of 777 rows (2560 / 10240) 453 -> 358, of 400
+// Measured (us; bf16-code tiles -> here): 2048 x 4096 x 14336 395 -> 329, a layer of 777 rows (2560 / 10240) 453 -> 332, of 400
 // rows (1472 / 4032) 274 -> 125, of 300 rows in groups of 32 (2048 / 8192) 24.7 ms on the any-width kernel -> 159, 512 tokens
-// through 128 experts (2816 / 704) 3692 -> 314.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
-// instructions of expansion and 64 of scaling; a block takes 0.72 us of a CU for 0.23 us of matrix pipe.
+// through 128 experts (2816 / 704) 3692 -> 285.  Bound: with 64 rows a wavefront, 16 MFMAs a block stand against 64 vector
+// instructions of expansion and 64 of scaling; with two 128 x 128 tiles on a CU a block takes 0.65 us of it for 0.23 us of matrix pipe.
 // Scales and biases go through LDS as well, SE of each row at a time (a segment).  Loaded by the lanes that use them, four blocks at
 // a time, every load touched a line per row, in either wavefront row again: as many lines as the copies of A and of the packed
 // weights together.
@@ -314,7 +314,6 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     constexpr bool B8 = BITS == 8;
     constexpr float CENTRE = B8 ? 128.0f : 8.0f;  // the operand's codes are code - CENTRE
     static_assert(NB == 2, "a pair is two column blocks");
-    static_assert(STAGES == 2 || STAGES == 3 || STAGES == 4, "LDS stages");
     constexpr int BM = WM * MB * 32;
     constexpr int BN = WN * NB * 32;
     constexpr int NWAVE = WM * WN;
@@ -339,7 +338,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     // block g those of A's (and BITS 8's) block g + STAGES - 1 and, in a stage's first block, of BITS 4's next stage.  still_out: the
     // copies that may be on their way at the barrier of block Q of a quad: A of block g + 1 has to have landed and with it the codes
     // that are read up to the next barrier.
-    static_assert(STAGES <= 3, "waits are counted for two or three stages");
+    static_assert(STAGES == 2 || STAGES == 3, "waits are counted for two or three stages");
     auto still_out = [=](int q) constexpr {
         return B8 ? (STAGES - 2) * (NA + NBC) : (STAGES - 2) * NA + ((q & 1) != WHOLE ? NBC : 0) + (XS_LDS && q == 1 ? NX : 0);
     };
@@ -670,19 +669,22 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         }
     };
 
-    // One 64-code block per iteration; Q = g & 3 is static so that everything indexed by it stays in fixed
-    // registers.  Iteration g requests block g + AHEAD.  Past the end of K the last block is requested again.
-    //
-    // The segment after this one (in its last quad) and the quad's sums of x are fetched at Q = 1 with ordinary loads.
-    // The compiler cannot count the copy instructions, so wherever it first uses a loaded register it waits
-    // until NOTHING is outstanding, copies included.  Iteration Q = 1 is therefore ordered: loads, MFMAs, first
-    // use of the loaded registers (forced), and only then this iteration's copies - the forced wait then covers
-    // the loads, a block of MFMAs old, and the copies of block g+1, which the end of the iteration needs anyway.
-    // A segment is replaced where it lies: its last quad's scales and biases have been read by every wavefront before the
-    // barrier of Q = 0, and the next are first read at Q = 3, behind the barrier of Q = 1.
-    // With two or four stages the stage of block g is g & 3 modulo the stages, static like Q, and every LDS address
-    // of the loop is a constant; with three it is carried along.
-    constexpr bool STATIC_STAGE = STAGES == 2 || STAGES == 4;
+    // A 64-code block at a time; Q = g & 3 is static so that everything indexed by it stays in fixed registers.  Past the end of K the
+    // last block is requested again.  Who asks for what, which barrier publishes it and which frees its place:
+    //   copies of A and of the packed weights: see still_out;
+    //   the segment of scales and biases after this one, in the last quad of a segment: ordinary loads at the start of block Q = 1, stored
+    //     over the old segment ahead of that block's barrier.  The old one's last scales and biases have been read by every wavefront
+    //     before the barrier of Q = 0 (or of the Q = 3 before it); the new ones are first read at Q = 3 (BITS 8: at the next Q = 0);
+    //   a quad's sums of x: BITS 4 ordinary loads at Q = 1, or with XS_LDS copies behind the barrier of Q = 0, which has freed their
+    //     place (the last quad's are read at the end of Q = 3) and which the barrier of Q = 2 publishes; BITS 8 ordinary loads at Q = 2
+    //     (WHOLE: at Q = 1).
+    // The compiler cannot count the copy instructions, so wherever it first uses a register of an ordinary load it waits until NOTHING is
+    // outstanding, copies included.  A block with ordinary loads is therefore ordered: loads, MFMAs, first use of the loaded registers
+    // (forced), and only then new copies - the forced wait then covers the loads, most of a block of MFMAs old, and the copies that the
+    // barrier waits for anyway.
+    // With two stages the stage of block g is g & 1, static like Q, and every LDS address of the loop is a constant; with three it is
+    // carried along.
+    constexpr bool STATIC_STAGE = STAGES == 2;
     int sa_carried = 0;  // LDS stage that holds block g
     // whether the quad of block g is the last of its segment, with more of K behind it
     auto refills = [&](int g) { return quad_at + 1 == quads && (g | 3) + 1 < G; };
