@@ -1338,8 +1338,14 @@ void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_
             if (ks > 1 && (int64_t)(ks - 1) * gsplit >= G) continue;
             const int blocks = ks > 1 ? gsplit : G;
             double us = half_cost(i, group_size, tiles * ks, blocks, tiles * ks * blocks, cus);
-            // partial tiles: one more launch, and their bytes (two of 2048 x 4096: 14 us for the sums, 10 for the stores)
-            if (ks > 1) us += 3.0 + (double)ks * M * (double)seg->N * 4 / 2.4e6;
+            // Partial tiles: one more launch, and their bytes (two of 2048 x 4096: 14 us for the sums, 10 for the stores).  Matrices of
+            // few columns mostly stand in a grid beside wider ones, which fill the chip: there shares shorten little and cost the
+            // same, so their bytes count for more (below 768 columns it is k and v rather than a layer's output).  Over 320 layers of
+            // 66 to 2048 rows, against the bytes alone: q|k|v 1 to 2 % faster, o and down 0.1 % slower, the slowest layer against
+            // q|k|v whole 5 -> 3 %; 1966 x 1920 x (2688, 576, 576) in groups of 32 64 -> 53 us, 1905 x 3648 x (1664, 704, 704) of
+            // 8 bit 95 -> 80.  (1.6 up to 2048 columns: o and down 0.4 % slower again, 1053 x 2816 x 896 31 -> 37.)
+            const double bytes_us = (double)ks * M * (double)seg->N * 4 / 2.4e6;
+            if (ks > 1) us += 3.0 + bytes_us * (seg->N < 768 ? 1.6 : seg->N <= 2048 ? 1.3 : 1.0);
             if (us < best_us) best_us = us, seg->ksplit = ks, seg->gsplit = gsplit;
         }
     }
