@@ -1326,6 +1326,11 @@ static int64_t half_bands(int i, int M) { return (M + qmmh_rows(i) - 1) / qmmh_r
 void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_count) {
     const int cus = cu_count > 0 ? cu_count : 256;
     const int G = K / 64;
+    // Matrices much wider than deep are one of a gated pair as often as not, whose grid has twice the tiles and partial tiles: theirs
+    // cost the mean of the two.  150 pairs and as many single calls, against the single call's cost: pairs 1.1 % faster in the mean,
+    // single calls 0.4 % slower; pairs of 71 x 2944 x 9984 42.3 -> 35.3 us, in groups of 32 of 8 bit 85 x 3328 x 7232 49.8 -> 42.3 and
+    // 63 x 3840 x 15168 65.9 -> 59.3.  (At a pair's cost alone pairs are level with that and single calls another 1.5 % slower.)
+    const bool paired = seg->N >= K + K / 2;
     double best_us = 1e30;
     seg->ksplit = 1;
     seg->gsplit = (G + 3) / 4 * 4;
@@ -1338,6 +1343,10 @@ void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_
             if (ks > 1 && (int64_t)(ks - 1) * gsplit >= G) continue;
             const int blocks = ks > 1 ? gsplit : G;
             double us = half_cost(i, group_size, tiles * ks, blocks, tiles * ks * blocks, cus);
+            if (paired) {
+                const int64_t both = half_bands(i, M) * half_strips(i, seg->N, true) * ks;
+                us = 0.5 * (us + half_cost(i, group_size, both, blocks, both * blocks, cus));
+            }
             // Partial tiles: one more launch, and their bytes (two of 2048 x 4096: 14 us for the sums, 10 for the stores).  Matrices of
             // few columns mostly stand in a grid beside wider ones, which fill the chip: there shares shorten little and cost the
             // same, so their bytes count for more (below 768 columns it is k and v rather than a layer's output).  Over 320 layers of
@@ -1345,7 +1354,7 @@ void qmmh_split(int M, int K, int group_size, int bits, QmmSegment* seg, int cu_
             // q|k|v whole 5 -> 3 %; 1966 x 1920 x (2688, 576, 576) in groups of 32 64 -> 53 us, 1905 x 3648 x (1664, 704, 704) of
             // 8 bit 95 -> 80.  (1.6 up to 2048 columns: o and down 0.4 % slower again, 1053 x 2816 x 896 31 -> 37.)
             const double bytes_us = (double)ks * M * (double)seg->N * 4 / 2.4e6;
-            if (ks > 1) us += 3.0 + bytes_us * (seg->N < 768 ? 1.6 : seg->N <= 2048 ? 1.3 : 1.0);
+            if (ks > 1) us += 3.0 + bytes_us * (paired ? 1.5 : seg->N < 768 ? 1.6 : seg->N <= 2048 ? 1.3 : 1.0);
             if (us < best_us) best_us = us, seg->ksplit = ks, seg->gsplit = gsplit;
         }
     }

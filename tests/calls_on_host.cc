@@ -327,6 +327,9 @@ static void test_tiles_of_prompts() {
     log_.clear();
     CHECK(aq_qmm_multi(ctx, X, 3, w, s, b, y, N, 777, 2560, 64, 8, 0) == AQ_OK && log_.size() > 1, "%s", aq_last_error());
     CHECK(log_[1].is("qmmh_kernelILi8ELi1ELi2ELi2ELi2E"), "q|k|v of 777 rows: %s", log_[1].kernel.c_str());
+    // a pair that three shares of either matrix would not shorten (24.5 -> 22)
+    log_.clear();
+    CHECK(aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, 128, 1152, 3840, 32, 8, AQ_ACT_SILU, 0) == AQ_OK && log_.size() == 2, "gate|up of 128 rows: %zu launches", log_.size());
     // k and v beside a q that fills the chip stay whole (64 -> 53)
     const int wide[3] = {2688, 576, 576};
     log_.clear();

@@ -24,9 +24,9 @@ def _check_columns(acc, x, m, bits, gs, K, what):
 
 
 @pytest.mark.parametrize("bits,gs,M,K,N,tile", [(4, 32, 513, 1856, 3986, "256x128"), (4, 32, 200, 3904, 4758, "256x128"), (4, 32, 513, 3904, 5530, "128x256"),
-                                                (4, 32, 200, 3904, 4179, "256x256"), (4, 32, 130, 1856, 5530, "192x256"), (4, 64, 513, 1856, 3986, "128x256"),
-                                                (4, 64, 509, 1856, 4372, "256x128"), (4, 64, 130, 2112, 4372, "192x256"), (8, 32, 513, 3904, 6109, "128x256"),
-                                                (8, 32, 130, 2112, 3600, "64x256"), (8, 32, 513, 832, 3986, "128x128"), (8, 64, 200, 3904, 4758, "128x256")])
+                                                (4, 32, 200, 3904, 4179, "256x256"), (4, 32, 130, 3904, 2770, "192x256"), (4, 64, 513, 1856, 3986, "128x256"),
+                                                (4, 64, 509, 1856, 4372, "256x128"), (4, 64, 130, 3904, 3675, "192x256"), (8, 32, 513, 3904, 6109, "128x256"),
+                                                (8, 32, 130, 3904, 2147, "64x256"), (8, 32, 513, 832, 3986, "128x128"), (8, 64, 200, 3904, 4758, "128x256")])
 def test_gated_pair(ctx, orc, bits, gs, M, K, N, tile):
     import aq_mi355
     say("gate|up on large tiles", bits, gs, M, K, N, tile)
