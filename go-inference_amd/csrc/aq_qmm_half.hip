@@ -1388,7 +1388,11 @@ int qmmh_pick(const QmmHalfCall& q, int cu_count) {
             all += t * b;
             most = b > most ? b : most;
         }
-        const double us = half_cost(i, q.group_size, tiles, most, all, cus);
+        double us = half_cost(i, q.group_size, tiles, most, all, cus);
+        // Several 128 x 256 tiles of a pair a CU take 3 % longer than of one matrix (the costs come from single matrices; their epilogue has
+        // no activation).  Over 70 pairs of 500 to 1600 rows: 1274 x 2048 x 7296 122 -> 117 us on 192 x 256, 1676 x 1536 x 5376
+        // 99 -> 95, the largest loss against the costs before them 4 -> 2 %, the mean 0.1 % faster (at 5 and 7 % level).
+        if (q.pair && kQmmHalfTable[i].v.mb == 4 && kQmmHalfTable[i].v.wm == 1 && tiles > cus) us *= 1.03;
         if (us < best_us) best_us = us, best = i;
     }
     return best;
