@@ -83,8 +83,9 @@ typedef uint32_t __attribute__((ext_vector_type(2), aligned(2))) u32x2_a2_t;
 // Measured (us, graph replay over 640 MB of weights; moves between lanes, 14 or 8 instructions a word and at most 64 rows a
 // workgroup -> here): 21 rows of x, groups of 32: 3840 x (15360 | 15360) 49.5 -> 30.7, 15360 x 3840 29.6 -> 21.9; groups of 64:
 // 16 / 32 rows of 4096 x 14336 12.3 -> 11.7 / 17.2 -> 16.7, 32 of 14336 x 4096 30.8 -> 19.1, 8 bit 33.9 -> 22.5.
-// Bound by vector issue: 32 rows of 4096 x 14336 in groups of 64 spend 10 us on the instructions of the expansion, the MFMAs and
-// the epilogue, beside 6 to 7 us that any call takes (launch, the first requests, the sums over wavefronts, the store).
+// Bound by waits: 32 rows of 4096 x 14336 in groups of 64 take 10 us beside the 6 to 7 us of any call (launch, the first requests, the
+// sums over wavefronts, the store); by counters 5 of those are vector issue and 2 matrix cores, wavefronts stand at a counter or barrier
+// 35 % of their cycles (groups of 32, 21 rows of 3840 x (15360 | 15360): 53 %, vector issue 30 % of SIMD cycles, matrix cores 11 %).
 // Dense groups of 32 also test every sum for infinities, which the any-width kernel keeps (plain_dot_g32).
 // PAIR: the first half of the workgroup's sets of rows belongs to the gate matrix, the second half to the same rows of the
 // up matrix, and the store is act(gate) * up: one pass over x and one launch for a gated MLP's two projections.
