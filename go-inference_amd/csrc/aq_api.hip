@@ -1185,15 +1185,32 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     const bool tok_fits = aq::qmvt_grouped_fits(a, bits, group_size, pair) && !(ctx->families_off >> kFamTok & 1);
     if (!tiles_fit && !tok_fits) return kPass;
     const bool tiles = tiles_fit && !(tok_fits && per_expert <= 12 && a.K >= 2048);
-    const int chunk = !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= (bits == 4 ? 96 : 16) ? 32 : per_expert <= 384 ? 64 : bits == 8 ? 128 : 256;
-    const int pad = tiles ? 32 : 1;
-    const int most_chunks = a.routes / chunk + groups;
-    const int most_rows = a.routes + groups * (pad - 1);
-    const size_t xbytes = tiles ? (aq::qmmt_workspace_bytes(most_rows, a.K) + 255) & ~(size_t)255 : 0;
-    const size_t list = align256((size_t)most_chunks * sizeof(aq::RouteChunk)), places = align256((size_t)most_rows * 4);
-    const size_t need = xbytes + list + 256 + 2 * places;
+    // Tiles in blocks of 16 routes (4 bit), their copy of x one of its rows as they lie, or of a row per route where there are more of
+    // them.  They read and expand an expert's weights once for up to 48 routes, but a tile by itself takes 1.6 times as long as one of 32
+    // routes: they need a chip full of them (the same block on tiles of 32 -> here, us: 128 experts, 2816 / 704, 16 / 32 / 44 routes an
+    // expert 183 -> 159, 234 -> 186, 269 -> 248; 64 experts, 2048 / 704, 32 routes 111 -> 99, 60 routes 145 -> 142; 64 experts, 1536 /
+    // 1024, 6 routes 86 -> 76; below 1.4 tiles a CU 32 experts, 2048 / 704, 24 routes 69 -> 72, 50 routes 85 -> 95) and experts whose
+    // routes fit one chunk or two.
+    const bool by_route = a.lhs && a.x_rows > a.routes;
+    const int x_copy = !a.lhs ? 1 : by_route ? a.routes : a.x_rows;
+    bool blocks = tiles && bits == 4 && per_expert <= 64 && named * aq::qmmr_strips(a.N, pair) >= 1.4 * ctx->cu_count &&
+                  aq::qmmr_fits(x_copy, a.K, a.N, group_size, bits);
+    int chunk = 0, pad = 0, most_chunks = 0, most_rows = 0;
+    size_t xbytes = 0, list = 0, places = 0;
+    auto offered = [&] {
+        chunk = blocks ? aq::kRouteRows : !tiles ? (per_expert <= 12 ? 16 : 32) : per_expert <= (bits == 4 ? 96 : 16) ? 32 : per_expert <= 384 ? 64 : bits == 8 ? 128 : 256;
+        pad = tiles && !blocks ? 32 : 1;
+        most_chunks = a.routes / chunk + groups;
+        most_rows = a.routes + groups * (pad - 1);
+        xbytes = blocks ? aq::qmmr_workspace_bytes(x_copy, a.K, group_size) : tiles ? (aq::qmmt_workspace_bytes(most_rows, a.K) + 255) & ~(size_t)255 : 0;
+        list = align256((size_t)most_chunks * sizeof(aq::RouteChunk));
+        places = align256((size_t)most_rows * 4);
+        return aq::workspace_offer(ctx->stream, &ctx->ws, xbytes + list + 256 + 2 * places);
+    };
     AQ_HIP(hipSetDevice(ctx->device), "hipSetDevice");
-    if (!aq::workspace_offer(ctx->stream, &ctx->ws, need)) return kPass;  // the per-route kernels need no scratch
+    bool room = offered();
+    if (!room && blocks) blocks = false, room = offered();  // (short K is padded to 256 codes: the tiles of 32 may ask for less)
+    if (!room) return kPass;  // the per-route kernels need no scratch
     char* p = static_cast<char*>(ctx->ws.ptr) + xbytes;
     aq::RouteGroupArgs g{};
     g.lhs = a.lhs;
@@ -1210,6 +1227,29 @@ int run_grouped(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool pair)
     g.live_rows = g.nchunks + 1;
     g.route_x = reinterpret_cast<int32_t*>(p + list + 256);
     g.route_of = reinterpret_cast<int32_t*>(p + list + 256 + places);
+    if (blocks) {
+        aq::QmmRouteCall c{};
+        c.x = a.x;
+        c.rows = x_copy;
+        c.by_route = by_route;
+        c.lists = g;
+        c.w = a.w;
+        c.s = a.s;
+        c.b = a.b;
+        c.y = a.y;
+        c.K = a.K;
+        c.N = a.N;
+        c.group_size = group_size;
+        c.pair = pair ? 1 : 0;
+        c.act = a.act;
+        c.out_f32 = a.out_f32;
+        c.expert_rows = a.expert_rows;
+        c.row_base = a.row_base;
+        c.row_base2 = a.row_base2;
+        ctx->last_variant[0] = pair ? "gather_gate_up_grouped_blocks" : "gather_grouped_blocks";
+        AQ_HIP(aq::qmmr_launch(c, ctx->ws.ptr, ctx->stream), "hipLaunchKernel");
+        return AQ_OK;
+    }
     AQ_HIP(aq::moe_group_launch(g, ctx->stream), "hipLaunchKernel");
     if (!tiles) {
         a.chunks = g.chunks;

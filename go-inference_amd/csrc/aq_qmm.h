@@ -152,6 +152,37 @@ size_t qmmh_partial_bytes(const QmmHalfCall& q);
 // What one matrix of any N needs at most with up to M rows of up to K columns.
 size_t qmmh_partial_most(int M, int K, int cu_count);
 
+// Routes grouped by expert on tiles of up to 48 routes in blocks of 16 (aq_qmm_routes.hip), 4-bit codes.
+constexpr int kRouteRows = 48;  // routes of a chunk
+struct QmmRouteArgs {
+    const uint16_t* xf;  // [rows][K up to a multiple of 128] fp16
+    const uint32_t* xs;  // [rows][groups up to a multiple of 512 codes] sums of x, two bf16 each
+    const float* rs;     // [rows] the inverse of the power of two a row was scaled by
+    const uint32_t* w;
+    const uint16_t *s, *b;
+    void* y;
+    int K, N, pair, act, out_f32;
+    int by_route;  // rows of xf are the routes (else the rows of x)
+    int strips, most_chunks, expert_rows, row_base, row_base2;
+    const RouteChunk* chunks;
+    const int32_t *route_x, *route_of;
+};
+struct QmmRouteCall {
+    const uint16_t* x;
+    int rows, by_route;  // of the copy of x
+    const uint32_t* w;
+    const uint16_t *s, *b;
+    void* y;
+    int K, N, group_size, pair, act, out_f32, expert_rows, row_base, row_base2;
+    RouteGroupArgs lists;  // chunks of kRouteRows, runs side by side
+};
+// Whether the tiles of such a call take a matrix (rows: of the copy of x), and what they keep in scratch.
+int qmmr_strips(int N, bool pair);  // workgroups an expert's chunk of routes takes
+bool qmmr_fits(int rows, int K, int N, int group_size, int bits);
+size_t qmmr_workspace_bytes(int rows, int K, int group_size);
+// Lists, pass over x and tiles.
+hipError_t qmmr_launch(const QmmRouteCall& c, void* workspace, hipStream_t stream);
+
 hipError_t fill_zero_launch(void* p, size_t bytes, hipStream_t stream);
 
 // Upper bound (256-byte aligned) of the workspace bytes qmm_dispatch may use for an M x K by N call: the
