@@ -863,7 +863,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
     if (!packed || !y || !N) return fail(AQ_ERR_ARG, "aq_qmv_multi: null array");
     if (M < 0 || K < 0) return fail(AQ_ERR_SHAPE, "aq_qmv_multi: M, K must be non-negative");
     const bool tiled = (flags & AQ_W_TILED) != 0;  // every member is a tile-major tensor; scales and biases are not read
-    bool fused = M >= 1 && M <= 4 && K > 0 && (bits == 4 || (bits == 8 && !tiled)) && ctx->forced[0] < 0;
+    bool fused = M >= 1 && M <= (bits == 4 ? 8 : 4) && K > 0 && (bits == 4 || (bits == 8 && !tiled)) && ctx->forced[0] < 0;
     if (!tiled && (!scales || !biases)) return fail(AQ_ERR_ARG, "aq_qmv_multi: null array");
     const void* const kNoArrays[aq::kQmvMultiMax] = {nullptr, nullptr, nullptr, nullptr};
     if (tiled) scales = biases = kNoArrays;
@@ -1418,10 +1418,14 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         !aligned(gate_biases, 2) || !aligned(up_scales, 2) || !aligned(up_biases, 2) || !aligned(y, 2))
         return fail(AQ_ERR_ARG, "aq_qmv_gate_up: operand pointer is not element-aligned");
     const bool out_f32 = (flags & AQ_OUT_F32) != 0;
-    if (M <= 4 && ctx->forced[0] < 0) {
+    if (M <= 8 && ctx->forced[0] < 0) {
         // the diagonal-MFMA kernels with one set of wavefronts per matrix
-        // the split of K that a single row gets; any row count shares its bytes
-        const int di = (ctx->families_off >> kFamDiag & 1) ? -1 : aq::qmvd_pick(1, K, 1 << 20);
+        // The split of K that a single row gets; any row count shares its bytes.  Five to eight rows in one launch up to four steps
+        // of K, else in two.  (As a launch or two for either matrix and one for the activation, and q, k and v apart, a layer of 6 rows
+        // took, us, before -> here: 2048 / 8192 56.6 -> 37.7, 3072 / 8192 58.8 -> 39.9, of 8 rows 4096 / 14336 81.5 -> 65.6.)
+        const bool diag = !(ctx->families_off >> kFamDiag & 1);
+        int di = diag ? aq::qmvd_pick(M, K, 1 << 20) : -1, per = M;
+        if (diag && M > 4 && di < 0) di = aq::qmvd_pick(4, K, 1 << 20), per = 4;
         aq::QmvArgs a{};
         a.x = static_cast<const uint16_t*>(x);
         a.w = static_cast<const uint32_t*>(gate_packed);
@@ -1433,7 +1437,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         a.y = y;
         a.K = K;
         a.N = N;
-        a.M = M;
+        a.M = per;
         a.gs_shift = is_pow2(group_size) ? ilog2(group_size) : 0;
         a.out_f32 = out_f32 ? 1 : 0;
         a.routes = 1;
@@ -1444,10 +1448,14 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         up.s = a.s2;
         up.b = a.b2;
         if (di >= 0 && aq::qmvd_pair_supported(di) && aq::qmvd_fits(a, bits, group_size, false, di) &&
-            aq::qmvd_fits(up, bits, group_size, false, di) &&
-            (size_t)M * K * 2 + (size_t)M * ((K + 255) / 256) * 48 + 128 + (size_t)2 * aq::qmvd_variant(di)->waves * 256 <= 96 * 1024) {
+            aq::qmvd_fits(up, bits, group_size, false, di) && aq::qmvd_pair_room(di, per, K)) {
             ctx->last_variant[0] = "qmv_gate_up_diag";
-            AQ_HIP(aq::qmvd_pair_launch(di, a, false, ctx->stream), "hipLaunchKernel");
+            for (int m0 = 0; m0 < M; m0 += per) {
+                a.M = M - m0 < per ? M - m0 : per;
+                a.x = static_cast<const uint16_t*>(x) + (size_t)m0 * K;
+                a.y = static_cast<char*>(y) + (size_t)m0 * N * (out_f32 ? 4 : 2);
+                AQ_HIP(aq::qmvd_pair_launch(di, a, false, ctx->stream), "hipLaunchKernel");
+            }
             return AQ_OK;
         }
     }

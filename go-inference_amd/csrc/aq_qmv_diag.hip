@@ -652,9 +652,9 @@ __global__ __launch_bounds__(NR* NW* kWave, 4) void qmv_diag_kernel(const QmvArg
         qmv_diag_dense<NW, SUP, NR, false, MT, CPS, false, MODE>(a, (int)blockIdx.x);
 }
 
-template <int NW, int SUP, int CPS, int MODE>
+template <int NW, int SUP, int CPS, int MT, int MODE>
 __global__ __launch_bounds__(2 * NW* kWave, 4) void qmv_diag_pair_kernel(const QmvArgs a) {
-    qmv_diag_dense<NW, SUP, 2, true, 1, CPS, false, MODE>(a, (int)blockIdx.x);
+    qmv_diag_dense<NW, SUP, 2, true, MT, CPS, false, MODE>(a, (int)blockIdx.x);
 }
 
 // Quantisation groups of 32 codes, up to two activation rows.
@@ -694,7 +694,7 @@ __global__ __launch_bounds__(2 * NW* kWave, 4) void qmv_diag_gather_pair_kernel(
 
 // Several weight matrices against the same activations in one launch (q|k|v, gate|up): the workgroups of all
 // matrices form one grid, and each looks up which matrix it belongs to.
-template <int NW, int SUP, int NR, int CPS, int MODE>
+template <int NW, int SUP, int NR, int CPS, int MT, int MODE>
 __global__ __launch_bounds__(NR* NW* kWave, 4) void qmv_diag_multi_kernel(const QmvMultiArgs ma) {
     int set = 0;
 #pragma unroll
@@ -707,7 +707,7 @@ __global__ __launch_bounds__(NR* NW* kWave, 4) void qmv_diag_multi_kernel(const 
     a.y = ma.y[set];
     a.N = ma.N[set];
     const int block = (int)blockIdx.x - (set ? ma.block_end[set - 1] : 0);
-    qmv_diag_dense<NW, SUP, NR, false, 1, CPS, false, MODE>(a, block);
+    qmv_diag_dense<NW, SUP, NR, false, MT, CPS, false, MODE>(a, block);
 }
 
 // The same for 8-bit codes: at one row a launch of a 1024 x 4096 matrix is mostly its ramp (q|k|v of 4096 / 1024 / 1024 rows and
@@ -965,29 +965,36 @@ int qmvd_pick_g32(int M, int K, int N) {
 
 // act(gate . x) * (up . x) with the variant's (wavefronts, steps) split of K; a.w2 / a.s2 / a.b2 are the `up` matrix.
 struct QmvDiagPairEntry {
-    int nw, sup, cps;
+    int nw, sup, cps, mt;
     QmvDiagKernel fn[8], gather_fn[2];  // gather_fn[1]: K a whole number of chunks
 };
-#define AQ_QMVD_PAIR(NW, SUP, CPS) {NW, SUP, CPS, AQ_DIAG_MODES(qmv_diag_pair_kernel, NW, SUP, CPS), {qmv_diag_gather_pair_kernel<NW, SUP, CPS, false>, qmv_diag_gather_pair_kernel<NW, SUP, CPS, true>}}
+#define AQ_QMVD_PAIR(NW, SUP, CPS) {NW, SUP, CPS, 1, AQ_DIAG_MODES(qmv_diag_pair_kernel, NW, SUP, CPS, 1), {qmv_diag_gather_pair_kernel<NW, SUP, CPS, false>, qmv_diag_gather_pair_kernel<NW, SUP, CPS, true>}}
+// five to eight rows, where one launch takes them (the variants of 8 rows)
+#define AQ_QMVD_PAIR8(NW, SUP, CPS) {NW, SUP, CPS, 2, AQ_DIAG_MODES(qmv_diag_pair_kernel, NW, SUP, CPS, 2), {nullptr, nullptr}}
 static const QmvDiagPairEntry kQmvDiagPairTable[] = {
     AQ_QMVD_PAIR(2, 1, 4), AQ_QMVD_PAIR(4, 1, 4), AQ_QMVD_PAIR(6, 1, 4), AQ_QMVD_PAIR(8, 1, 4),
-    AQ_QMVD_PAIR(2, 1, 3), AQ_QMVD_PAIR(4, 1, 3),
+    AQ_QMVD_PAIR(2, 1, 3), AQ_QMVD_PAIR(4, 1, 3), AQ_QMVD_PAIR8(2, 1, 4), AQ_QMVD_PAIR8(4, 1, 4), AQ_QMVD_PAIR8(2, 1, 3), AQ_QMVD_PAIR8(4, 1, 3),
 };
 static const QmvDiagPairEntry* find_pair(int idx) {
     const QmvVariant* v = qmvd_variant(idx);
     if (v)
         for (const QmvDiagPairEntry& e : kQmvDiagPairTable)
-            if (e.nw == v->waves && e.sup == v->depth && e.cps == cps_of(*v) && !g32_of(*v) && !b8_of(*v)) return &e;
+            if (e.nw == v->waves && e.sup == v->depth && e.cps == cps_of(*v) && e.mt == (v->m + 3) / 4 && !g32_of(*v) && !b8_of(*v)) return &e;
     return nullptr;
 }
 bool qmvd_pair_supported(int idx) { return find_pair(idx) != nullptr; }
+bool qmvd_pair_room(int idx, int M, int K) {
+    const QmvDiagPairEntry* e = find_pair(idx);
+    return e && qmvd_lds_bytes_for(M, K, 2 * e->nw, e->mt) <= 96 * 1024;
+}
 
 hipError_t qmvd_pair_launch(int idx, const QmvArgs& a, bool gather, hipStream_t stream) {
     const QmvDiagPairEntry* e = find_pair(idx);
     if (!e) return hipErrorInvalidValue;
     const int stream_w = !gather && (int64_t)2 * a.N * (a.K / 2) >= kDiagStreamBytes ? 1 : 0;
     const QmvDiagKernel fn = gather ? e->gather_fn[a.K % kDiagChunk == 0 ? 1 : 0] : e->fn[diag_mode(a.K, e->cps, a.tiled != 0, stream_w != 0)];
-    const size_t lds = qmvd_lds_bytes_for(gather ? 1 : a.M, a.K, 2 * e->nw);
+    if (!fn) return hipErrorInvalidValue;
+    const size_t lds = qmvd_lds_bytes_for(gather ? 1 : a.M, a.K, 2 * e->nw, e->mt);
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(fn), lds)) return rc;
     dim3 grid((unsigned)((a.N + kDiagRows - 1) / kDiagRows), gather ? (unsigned)a.routes : 1u, 1u);
     QmvArgs b = a;
@@ -1056,24 +1063,27 @@ hipError_t qmvd_head_launch(int idx, int fuse, const QmvArgs& a, hipStream_t str
 
 typedef void (*QmvDiagMultiKernel)(const QmvMultiArgs);
 struct QmvDiagMultiEntry {
-    int bits, nw, sup, nr, cps;
+    int bits, nw, sup, nr, cps, mt;
     QmvDiagMultiKernel fn[8];
 };
-#define AQ_QMVD_MULTI(NW, SUP, NR) {4, NW, SUP, NR, 4, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 4)}
-#define AQ_QMVD_MULTI3(NW, SUP, NR) {4, NW, SUP, NR, 3, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 3)}
+#define AQ_QMVD_MULTI(NW, SUP, NR) {4, NW, SUP, NR, 4, 1, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 4, 1)}
+#define AQ_QMVD_MULTI3(NW, SUP, NR) {4, NW, SUP, NR, 3, 1, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, 3, 1)}
+#define AQ_QMVD_MULTI8(NW, SUP, NR, CPS) {4, NW, SUP, NR, CPS, 2, AQ_DIAG_MODES(qmv_diag_multi_kernel, NW, SUP, NR, CPS, 2)}  // five to eight rows
 // (8 bit: whole steps of K only, what qmvd_pick takes)
-#define AQ_QMVDB_MULTI(NW, SUP, NR) {8, NW, SUP, NR, 4, {nullptr, nullptr, nullptr, nullptr, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 4>, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 5>, nullptr, nullptr}}
+#define AQ_QMVDB_MULTI(NW, SUP, NR) {8, NW, SUP, NR, 4, 1, {nullptr, nullptr, nullptr, nullptr, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 4>, qmv_diag_b8_multi_kernel<NW, SUP, NR, 4, 5>, nullptr, nullptr}}
 static const QmvDiagMultiEntry kQmvDiagMultiTable[] = {
     AQ_QMVD_MULTI(4, 1, 1), AQ_QMVD_MULTI(4, 1, 2), AQ_QMVD_MULTI(4, 1, 4), AQ_QMVD_MULTI(2, 1, 2), AQ_QMVD_MULTI(2, 1, 4),
     AQ_QMVD_MULTI(6, 1, 1), AQ_QMVD_MULTI(8, 1, 1), AQ_QMVD_MULTI(10, 1, 1), AQ_QMVD_MULTI(12, 1, 1), AQ_QMVD_MULTI(14, 1, 1),
     AQ_QMVD_MULTI(16, 1, 1), AQ_QMVD_MULTI3(4, 1, 1), AQ_QMVD_MULTI3(4, 1, 2), AQ_QMVD_MULTI3(4, 1, 4), AQ_QMVD_MULTI3(2, 1, 2),
-    AQ_QMVD_MULTI3(2, 1, 4), AQ_QMVDB_MULTI(4, 1, 1), AQ_QMVDB_MULTI(4, 1, 2), AQ_QMVDB_MULTI(8, 1, 1), AQ_QMVDB_MULTI(16, 1, 1),
+    AQ_QMVD_MULTI8(4, 1, 4, 4), AQ_QMVD_MULTI8(4, 1, 2, 4), AQ_QMVD_MULTI8(2, 1, 4, 4), AQ_QMVD_MULTI8(4, 1, 4, 3), AQ_QMVD_MULTI8(4, 1, 2, 3),
+    AQ_QMVD_MULTI8(2, 1, 4, 3), AQ_QMVD_MULTI3(2, 1, 4), AQ_QMVDB_MULTI(4, 1, 1), AQ_QMVDB_MULTI(4, 1, 2), AQ_QMVDB_MULTI(8, 1, 1), AQ_QMVDB_MULTI(16, 1, 1),
 };
 static const QmvDiagMultiEntry* find_multi(int idx) {
     const QmvVariant* v = qmvd_variant(idx);
     if (v && !g32_of(*v))
         for (const QmvDiagMultiEntry& e : kQmvDiagMultiTable)
-            if (e.bits == v->bits && e.nw == v->waves && e.sup == v->depth && e.nr == v->rows && e.cps == cps_of(*v)) return &e;
+            if (e.bits == v->bits && e.nw == v->waves && e.sup == v->depth && e.nr == v->rows && e.cps == cps_of(*v) && e.mt == (v->m + 3) / 4)
+                return &e;
     return nullptr;
 }
 
@@ -1090,7 +1100,7 @@ hipError_t qmvd_multi_launch(int idx, QmvMultiArgs ma, hipStream_t stream) {
         ma.block_end[i] = blocks;
     }
     const int K4 = k4_of(ma.common.K, e->bits);
-    const size_t lds = qmvd_lds_bytes_for(ma.common.M, ma.common.K, e->nw * e->nr, 1, false, e->bits == 8);
+    const size_t lds = qmvd_lds_bytes_for(ma.common.M, ma.common.K, e->nw * e->nr, e->mt, false, e->bits == 8);
     int64_t bytes = 0;
     for (int i = 0; i < ma.count; i++) bytes += (int64_t)ma.N[i] * (K4 / 2);
     ma.common.stream_w = bytes >= kDiagStreamBytes ? 1 : 0;
