@@ -146,8 +146,8 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // past *live_rows are left alone.
 constexpr int kPrepThreads = 512;
 constexpr int kPrepHold = 8;
-// BITS 8: the order in which the 8-bit kernels take x: a step of 16 codes is 16 consecutive ones (half h the second eight),
-// values in their natural order.
+// BITS 8: the order in which the 8-bit kernels take x: lane half h has codes 32 i + 16 h .. + 15 of a block in steps 2 i and 2 i + 1
+// (one 16-byte read of the weights), values in their natural order.
 template <int ROWS, int GRP, int BITS>
 __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xf,
                                                          uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K,
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t*
         // slot order (x0,x4)(x1,x5)(x2,x6)(x3,x7): the order in which expand_pair emits the codes of a word
         const f16x8_t o = BITS == 4 ? f16x8_t{hv[0], hv[4], hv[1], hv[5], hv[2], hv[6], hv[3], hv[7]}
                                     : f16x8_t{hv[0], hv[1], hv[2], hv[3], hv[4], hv[5], hv[6], hv[7]};
-        const int t = BITS == 4 ? c8 & 3 : c8 >> 1, h = BITS == 4 ? c8 >> 2 : c8 & 1;
+        const int t = BITS == 4 ? c8 & 3 : (c8 >> 2) * 2 + (c8 & 1), h = BITS == 4 ? c8 >> 2 : c8 >> 1 & 1;
         const int64_t frag = (int64_t)(row >> 5) * (K / 16) + g * 4 + t;
         *reinterpret_cast<f16x8_t*>(xf + (frag * 64 + h * 32 + (row & 31)) * 8) = o;
     };
@@ -811,7 +811,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     constexpr int GROUPS = G32 ? 2 : 1;  // of a block
     constexpr int UNITS = MB * GROUPS, STEPS = 4 / GROUPS;
     f16x8_t a8[4], b8[NB][4];
-    uint2 codes8[NB];
+    uint4 codes8[NB];  // of two steps
     constexpr int PARTS = G32 || WHOLE ? 1 : 2;  // (groups of 32 have no registers for a second unit's sums: scaled behind their own MFMAs)
     f32x16_t part[PARTS][NB];
     float scale[NB][GROUPS], scale_before[NB];  // of the block's groups; of the last group of the block before
@@ -828,15 +828,16 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     auto read_a8 = [&](int t, int mb, int stage) __attribute__((always_inline)) {
         a8[t] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
     };
-    // row (wave_n * NB + nb) * 32 + j, eight codes from 16 t + 8 h on for step t
-    auto read_codes8 = [&](int t, int stage) __attribute__((always_inline)) {
-        const uint8_t* const at = bbuf + (stage * B_STAGE + (wave_n * NB * 32 + j) * B_ROW + h * 8 + ((t ^ turn(j)) * 16));
+    // Row (wave_n * NB + nb) * 32 + j: the sixteen codes of steps 2 i and 2 i + 1, whole 16-byte pieces of 16 rows that lie in different
+    // banks.  (Eight codes a read, one half of each piece: rows j and j + 16 met in the same banks, 13 % of the CU's cycles.)
+    auto read_codes8 = [&](int i, int stage) __attribute__((always_inline)) {
+        const uint8_t* const at = bbuf + (stage * B_STAGE + (wave_n * NB * 32 + j) * B_ROW + (((2 * i + h) ^ turn(j)) * 16));
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) codes8[nb] = *reinterpret_cast<const uint2*>(at + nb * 32 * B_ROW);
+        for (int nb = 0; nb < NB; nb++) codes8[nb] = *reinterpret_cast<const uint4*>(at + nb * 32 * B_ROW);
     };
     auto expand8 = [&](int t) __attribute__((always_inline)) {
 #pragma unroll
-        for (int nb = 0; nb < NB; nb++) b8[nb][t] = expand_bytes(codes8[nb]);
+        for (int nb = 0; nb < NB; nb++) b8[nb][t] = expand_bytes(t & 1 ? make_uint2(codes8[nb].z, codes8[nb].w) : make_uint2(codes8[nb].x, codes8[nb].y));
     };
     auto take_scales8 = [&](int q) __attribute__((always_inline)) {  // of block q of a quad
 #pragma unroll
@@ -903,7 +904,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
                 if (u == 0 && step == STEPS - 1) take_scales8(Q);
                 if (last_mb) {
                     if (t > 0) expand8(t - 1);
-                    read_codes8(t, sa_next);
+                    if (t % 2 == 0) read_codes8(t / 2, sa_next);
 #pragma unroll
                     for (int c = t * (NA + NBC) / 4; c < (t + 1) * (NA + NBC) / 4; c++) {
                         if (c < NA)
@@ -965,7 +966,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         if constexpr (B8) {
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                read_codes8(t, sa);
+                if (t % 2 == 0) read_codes8(t / 2, sa);
                 expand8(t);
             }
             take_scales8(Q);
@@ -1028,7 +1029,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     if constexpr (B8 && !WHOLE) {
 #pragma unroll
         for (int t = 0; t < 4; t++) {
-            read_codes8(t, 0);
+            if (t % 2 == 0) read_codes8(t / 2, 0);
             expand8(t);
             read_a8(t, 0, 0);
         }
