@@ -904,7 +904,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
                 const aq::QmvMultiArgs ma = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
                 for (int i = 0; i < count; i++) fits = fits && aq::qmvd_fits(multi_member(ma, i), bits, group_size, false, di);
                 if (fits) {
-                    ctx->last_variant[0] = bits == 4 ? "qmv_multi_diag" : "qmv8_multi_diag";
+                    ctx->last_variant[0] = bits == 8 ? "qmv8_multi_diag" : M > 4 ? "qmvd_multi_m8" : "qmv_multi_diag";
                     AQ_HIP(aq::qmvd_multi_launch(di, ma, ctx->stream), "hipLaunchKernel");
                     return AQ_OK;
                 }

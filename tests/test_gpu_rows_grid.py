@@ -22,7 +22,7 @@ def test_members_and_pair(ctx, M, K, N, N2):
     for flags, w, s, b in [(0, [d.w for d in mats], [d.s for d in mats], [d.b for d in mats])] + ([(aq_mi355.AQ_W_TILED, tiled, [None] * 3, [None] * 3)] if tiled else []):
         ctx.qmv_multi(x, w, s, b, ys, Ns, M, K, 64, 4, flags | f32)
         ctx.sync()
-        assert K > 4096 or ctx.last_variant(0) == "qmv_multi_diag", ctx.last_variant(0)
+        assert K > 4096 or ctx.last_variant(0) == "qmvd_multi_m8", ctx.last_variant(0)
         for d, n, y in zip(mats, Ns, ys):
             ctx.qmv(x, d.w, d.s, d.b, one, M, K, n, 64, 4, f32)
             ctx.sync()
