@@ -257,7 +257,8 @@ const QmvRule kQmvRules[] = {
     {4, 64, 0, 2, 8, kFamDot2},             // K the diagonal kernels do not take (up to 1024, no multiple of 128, beyond
                                             // 16384): the kernel a single row of such a K runs on, four rows a launch, so
                                             // that rows keep the bytes of single-row calls here too
-    {4, 32, 0, 1, 2, kFamDiag},             // groups of 32: two tokens x eight groups as MFMA rows
+    {4, 32, 0, 1, 2, kFamDiag},             // groups of 32: two tokens x eight groups as MFMA rows (K a multiple of 256; two rows of another
+                                            // K: token tile, a layer of 1216 / 4032 23.4 us on dot2 kernels, 16.8 here)
     {8, 64, 0, 1, 4, kFamDiag},             // up to four rows of 8-bit codes, K of 2048, 4096 or 8192, up to 40 Mi codes (where
                                             // measured ahead of the next two rules, see qmvd_pick); a row of such a call
                                             // has the bytes of a call with that row alone
@@ -273,9 +274,9 @@ const QmvRule kQmvRules[] = {
                                             // calls have passed, e.g. on operands that are not 16-byte aligned, or with the
                                             // diagonal and dot2 families switched off: this kernel is faster at long K,
                                             // 15.6 against 2 x 9 us at 8 rows of 14336 x 4096, but not row by row the same bytes)
-    {4, 32, 0, 3, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
+    {4, 32, 0, 2, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
     {8, 32, 0, 2, 32, kFamTok},
-    {0, 128, 0, 5, 32, kFamTok},
+    {0, 128, 0, 2, 32, kFamTok},            // (2..4 rows of a layer of 2048 / 7168 29-32 us on the block-MFMA kernels, 19-21 here, of 8 bit 26-30 / 19-21)
     {0, 0, 0, 33, 64, kFamTok},
     {0, 0, 0, 9, 64, kFamTilesLarge},       // 16 Mi codes and more: the 16-row block-MFMA kernel is bound by its 4x4x4 MFMAs
     {0, 0, 0, 2, 16, kFamBlk},              // the whole call in one launch of up to 16 rows (4 where K is long)
@@ -358,21 +359,26 @@ int run_diag(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool g
 // families behind.  8 bit: up to four rows, where the dot2 kernels are ahead (us, dot2 / here: 2 rows of 960 x 512 2.8 / 4.5, of
 // 4032 x 1024 4.4 / 6.7; 4 rows 3.2 / 4.5, 5.8 / 7.0); from five rows on what is behind are tiles, a pass over x and a sum of
 // shares of K in three launches (8 rows 14.6 / 4.6, 17.6 / 7.3; 32 rows 15.0 / 6.7, 18.1 / 11.9).  4 bit: up to 528 rows of
-// weights; the tiles are behind there as well (9 rows of x by 960 x 512 13.6 / 4.6, by 960 x 2048 14.3 / 4.6, 32 by 4032 x 1024
-// 17.4 / 11.1), but the choice for those sizes is one that tests/test_gpu_selection.py states.
+// weights that are no whole sets of 16; the tiles are behind there as well (9 rows of x by 960 x 512 13.6 / 4.6, by 960 x 2048 14.3 /
+// 4.6, 32 by 4032 x 1024 17.4 / 11.1), but the choice is one that tests/test_gpu_selection.py states, at 520 rows.  Whole sets, what k
+// and v of a layer have, run here, in one grid with q (a layer of 1216 / 4032 with 448 rows of k and v, tiles / here: 9 rows of x
+// 30.0 / 17.6, 32 rows 35.9 / 20.6).
 bool tok_small(int bits, int group_size, int M, int K, int64_t rows) {
-    return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20 && (bits == 8 ? M <= 4 : rows <= 528);
+    return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20 && (bits == 8 ? M <= 4 : rows <= 528 && rows % 16 != 0);
 }
 // 33..64 rows of x run as two halves in one grid.  They are ahead of the tiles (us, tiles / halves, 40 rows) while eight sets of 16
 // weight rows per workgroup fill each CU once at the most: 1024 x 14336 4 bit, groups of 64 / 32 / 128 17.0 / 11.4, 19.8 / 15.9,
 // 19.2 / 10.9, 8 bit 16.6 / 14.3, 21.2 / 15.6; 14336 x 4096 30.5 / 25.4, 39.7 / 33.2, 37.8 / 25.3, 32.8 / 30.5, 42.9 / 34.8.  With
 // two rounds they are ahead where the tiles are the slow ones, gate and up in groups of 64 (4096 x 14336 4 bit 52.7 / 43.6, 8 bit
 // 59.1 / 54.7) and groups of 128 (4096 x 28672 51.0 / 43.7), and behind elsewhere (4096 x 28672 groups of 64 41.7 / 44.0, 8 bit
-// 52.4 / 54.4, groups of 32 49.3 / 59.0, 60.6 / 62.6; gate and up in groups of 32 47.7 / 59.3).  Matrices of up to 528 rows stay
-// with the tiles, a choice that tests/test_gpu_selection.py states.
+// 52.4 / 54.4, groups of 32 49.3 / 59.0, 60.6 / 62.6; gate and up in groups of 32 47.7 / 59.3).  Matrices of up to 528 rows that are no
+// whole sets of 16, and those of fewer than 256, stay with the tiles, choices that tests/test_gpu_selection.py (520 rows) and
+// tests/test_gpu_fused_act.py (pairs of 96, and their own calls) state; k and v of a layer are larger whole
+// sets (a layer of 2048 / 7168 with 512 rows of them, 48 rows of x, tiles / halves: 45.6 / 27.5, groups of 32 53.5 / 32.4, of 128 52.6
+// / 27.5, 8 bit 46.3 / 30.1; of 1216 / 4032 with 448, 8 bit, 64 rows 55.9 / 24.0).
 bool tok_halves(const aq_ctx* ctx, int group_size, int M, int64_t rows, bool pair) {
     if (M <= 32) return true;
-    if (rows <= 528) return false;
+    if (rows <= 528 && (rows < 256 || rows % 16 != 0)) return false;
     const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256, groups = ((rows + 15) / 16 * (pair ? 2 : 1) + 7) / 8 * 2;
     return groups <= (group_size == 128 || (pair && group_size == 64) ? 2 : 1) * cus;
 }
@@ -391,12 +397,19 @@ int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, 
     return aq::qmvt_pick(bits, group_size, t.M, t.K, &part, 1, pair, ctx->cu_count);
 }
 
+// Two to four rows of x that other kernels keep: two rows in groups of 32 at a K of whole steps of the diagonal kernels, where a row
+// has the bytes of a call with that row alone, and groups of 128 beyond 64 Mi codes, as far as both sides were timed.
+bool tok_few(int bits, int group_size, int M, int K, int64_t rows) {
+    return (bits == 4 && group_size == 32 && M == 2 && K % 256 == 0) || (group_size == 128 && M <= 4 && rows * K > (int64_t)64 << 20);
+}
+
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
     if (gather) return kPass;
     aq::TokArgs t{a};
     t.ksplit = 1;
     t.tokens = forced < 0 ? aq::qmvt_tokens(a.M) : a.M;
-    if (forced < 0 && !tok_small(bits, group_size, a.M, a.K, a.N) && tok_halves(ctx, group_size, a.M, a.N, false)) {
+    const bool left = tok_small(bits, group_size, a.M, a.K, a.N) || tok_few(bits, group_size, a.M, a.K, a.N);
+    if (forced < 0 && !left && tok_halves(ctx, group_size, a.M, a.N, false)) {
         aq::qmvt_split(bits, group_size, a.M, a.K, a.N, false, ctx->cu_count, &t.ksplit, &t.share);
     } else if (forced < 0) {
         return kPass;
@@ -461,10 +474,10 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
 // the launch forms that put several matrices into one grid).
 bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, bool pair) {
     if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(bits, group_size, M, K, rows)) return false;
-    if (M > 64 || !tok_halves(ctx, group_size, M, rows, pair)) return false;
+    if (M < 2 || M > 64 || tok_few(bits, group_size, M, K, rows) || !tok_halves(ctx, group_size, M, rows, pair)) return false;
     if (bits == 4 && group_size == 64) return M >= 9;
-    if (bits == 8 && group_size == 64) return (M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0) && M >= 2;
-    return M >= (group_size == 128 ? 5 : bits == 4 ? 3 : 2);
+    if (bits == 8 && group_size == 64) return M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0;
+    return true;
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
