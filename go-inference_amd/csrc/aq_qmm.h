@@ -89,7 +89,8 @@ struct QmmSegment {
     int N;
     int ksplit, gsplit;    // workgroups that share a tile along K, 64-code blocks of K each takes (qmmh_split)
     int strips;            // filled by the launcher: column strips
-    float* partial;        // filled by the launcher: partial tiles of a K split
+    float* partial;        // filled by the launcher: partial sums of shares of K, or null
+    uint32_t* tickets;     // one for each tile
 };
 struct QmmHalfArgs {
     const uint16_t* xf;  // as in QmmTileArgs, fp16

@@ -30,6 +30,7 @@
 #include "aq_kernels.h"
 #include "aq_lds_copy.h"
 #include "aq_qmm.h"
+#include "aq_share_sum.h"
 
 #include <algorithm>
 #include <cmath>
@@ -144,6 +145,7 @@ __device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t
 // GRP 32: xs holds the sums of the 32-code halves, [mblks][ceil(G/4)][half][32 rows][4 blocks][hi, lo].
 // GROUPED: row i of the fragments is row route_x[i] of x (the list of routes sorted by expert; negative: zeros), and rows
 // past *live_rows are left alone.
+// tickets: `count` words that the tiles of shared K start from at zero.
 constexpr int kPrepThreads = 512;
 constexpr int kPrepHold = 8;
 // BITS 8: the order in which the 8-bit kernels take x: lane half h has codes 32 i + 16 h .. + 15 of a block in steps 2 i and 2 i + 1
@@ -151,7 +153,9 @@ constexpr int kPrepHold = 8;
 template <int ROWS, int GRP, int BITS>
 __global__ __launch_bounds__(kPrepThreads) void qmmh_prep_kernel(const uint16_t* __restrict__ x, uint16_t* __restrict__ xf,
                                                          uint16_t* __restrict__ xs, float* __restrict__ rs, int M, int K,
-                                                         const int32_t* __restrict__ route_x, const int32_t* __restrict__ live_rows) {
+                                                         const int32_t* __restrict__ route_x, const int32_t* __restrict__ live_rows,
+                                                         uint32_t* __restrict__ tickets, int count) {
+    for (int i = (int)(blockIdx.x * kPrepThreads + threadIdx.x); i < count; i += (int)gridDim.x * kPrepThreads) tickets[i] = 0u;
     constexpr int STEP = kPrepThreads / ROWS;  // pieces of a row between a thread's pieces
     // the workgroups of eight rows, which fill the same lines of xf, on one XCD
     const int seq = (int)blockIdx.x >> 3, row0 = (seq / (8 / ROWS) * 8 + ((int)blockIdx.x & 7)) * 8 + seq % (8 / ROWS) * ROWS;
@@ -364,9 +368,11 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     const int bands = min(a.group_m, row_bands - group * a.group_m);
     const int unit = __builtin_amdgcn_readfirstlane(in_group / bands);
     const int tm = __builtin_amdgcn_readfirstlane(group * a.group_m + in_group - unit * bands);
-    const int split = __builtin_amdgcn_readfirstlane(unit / a.seg[seg].strips);
-    const int tn = __builtin_amdgcn_readfirstlane(unit - split * a.seg[seg].strips);
+    // shares of K from the last to the first, which then mostly is the one to add them up and still holds its own
+    const int turns = __builtin_amdgcn_readfirstlane(unit / a.seg[seg].strips), split = a.seg[seg].ksplit - 1 - turns;
+    const int tn = __builtin_amdgcn_readfirstlane(unit - turns * a.seg[seg].strips);
     float* const partial = a.seg[seg].partial;  // null: this workgroup's sums are whole
+    uint32_t* const tickets = a.seg[seg].tickets;  // not null: partial sums are added here
     const bool pair = a.pair != 0;  // gate: seg[0], up: seg[1]
 
     const int tid = threadIdx.x;
@@ -1075,19 +1081,101 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
 
     // D layout of v_mfma_f32_32x32x*: lane (j, h), register r -> row 8*(r/4) + 4*h + r%4, column j: a lane holds
     // single elements of 16 rows, and storing them as they lie means 2-byte stores to 64-byte pieces of rows
-    // (measured: a third of a tile's time).  Each 32-row block of the wavefront's tile therefore goes through a
+    // (measured: a third of a tile's time).  Each 32-row block of the wavefront's tile, scaled by the two inverse powers of two
+    // (exact, whatever the order; that of the column belongs to the share of K, whose scales it comes from), therefore goes through a
     // staging area in LDS that belongs to the wavefront (the stages are free: every copy has landed, every read of
-    // the loop has returned, and the barrier says so for all wavefronts), scaled by the two inverse powers of two
-    // (exact, whatever the order), and leaves it row-major, eight consecutive columns per lane: 16-byte bf16
+    // the loop has returned, and the barrier says so for all wavefronts) and leaves it row-major, eight consecutive columns per lane: 16-byte bf16
     // stores, whole 128-byte lines per eight lanes.
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
+    {
+        const float col_down[2] = {1.0f / col_up[0], 1.0f / col_up[1]};
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++) {
+            const int mtop = m0 + (wave_m * MB + mb) * 32;  // < mblks * 32 unless the whole block lies past the last row
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int m = mtop + 4 * h + 8 * q;
+                const float4 down = m < a.mblks * 32 ? *reinterpret_cast<const float4*>(a.rs + m) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+                for (int nb = 0; nb < NB; nb++) {
+                    out[mb][nb][4 * q] = out[mb][nb][4 * q] * down.x * col_down[nb];
+                    out[mb][nb][4 * q + 1] = out[mb][nb][4 * q + 1] * down.y * col_down[nb];
+                    out[mb][nb][4 * q + 2] = out[mb][nb][4 * q + 2] * down.z * col_down[nb];
+                    out[mb][nb][4 * q + 3] = out[mb][nb][4 * q + 3] * down.w * col_down[nb];
+                }
+            }
+        }
+    }
+    if (tickets) {
+        // Shares of K (aq_share_sum.h): the sums of 32 x 32 blocks as the accumulators hold them, [share][block row][block column,
+        // gate then up][four accumulators][lane].
+        const int cols = (N + 31) / 32, all_cols = pair ? 2 * cols : cols, shares = a.seg[seg].ksplit;
+        const uint32_t share = (uint32_t)a.mblks * all_cols * 4096;
+        auto of = [&](int s) { return partial_sums(uniform(partial + (int64_t)s * (share / 4)), share); };
+        // block (mb, nb) of this wavefront's tile; past the last row or column: past the end
+        auto block_at = [&](int mb, int nb) {
+            const int br = m0 / 32 + wave_m * MB + mb, bc = pair ? n0 / 32 + wave_n : n0 / 32 + wave_n * NB + nb;
+            return br < a.mblks && bc < cols ? (uint32_t)(br * all_cols + (pair ? nb * cols : 0) + bc) * 4096 + lane * 16 : share;
+        };
+        const __amdgpu_buffer_rsrc_t own = of(split);
+#pragma unroll
+        for (int mb = 0; mb < MB; mb++)
+#pragma unroll
+            for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                for (int r = 0; r < 16; r += 4)
+                    put_partial(own, block_at(mb, nb) + r * 256, make_float4(out[mb][nb][r], out[mb][nb][r + 1], out[mb][nb][r + 2], out[mb][nb][r + 3]));
+        if (!last_share(tickets + tm * a.seg[seg].strips + tn, shares, reinterpret_cast<uint32_t*>(sbuf))) return;
+        // Shares 0 and 1 add in either order, so one of them stays where it is; a later one's sums are read back in their turn.  IN_FLIGHT
+        // block rows of sums are requested at a time, of one share (one block row a wavefront: of as many shares).
+        constexpr int IN_FLIGHT = MB == 4 ? 2 : 3;
+        auto add = [&](int s, bool fresh, auto shares_tag) __attribute__((always_inline)) {
+            constexpr int S = decltype(shares_tag)::value, ROWS = S > 1 ? 1 : MB < IN_FLIGHT ? MB : IN_FLIGHT;
+#pragma unroll
+            for (int mb0 = 0; mb0 < MB; mb0 += ROWS) {
+                float4 v[S][ROWS][NB][4];
+#pragma unroll
+                for (int t = 0; t < S; t++)
+#pragma unroll
+                    for (int i = 0; i < ROWS; i++)
+#pragma unroll
+                        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) v[t][i][nb][r] = get_partial(of(s + t), block_at(mb0 + i, nb) + r * 1024);
+#pragma unroll
+                for (int t = 0; t < S; t++)
+#pragma unroll
+                    for (int i = 0; i < ROWS; i++)
+#pragma unroll
+                        for (int nb = 0; nb < NB; nb++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) {
+                                const float4 f = v[t][i][nb][r];
+                                f32x16_t& o = out[mb0 + i][nb];
+                                o[4 * r] = fresh ? f.x : o[4 * r] + f.x;
+                                o[4 * r + 1] = fresh ? f.y : o[4 * r + 1] + f.y;
+                                o[4 * r + 2] = fresh ? f.z : o[4 * r + 2] + f.z;
+                                o[4 * r + 3] = fresh ? f.w : o[4 * r + 3] + f.w;
+                            }
+            }
+        };
+        typedef std::integral_constant<int, 1> One;
+        add(split == 0 ? 1 : 0, split > 1, One{});
+        int s = split <= 1 ? 2 : 1;
+        if constexpr (MB == 1)
+#pragma nounroll
+            for (; s + IN_FLIGHT <= shares; s += IN_FLIGHT) add(s, false, std::integral_constant<int, IN_FLIGHT>{});
+#pragma nounroll
+        for (; s < shares; s++) add(s, false, One{});
+    }
     constexpr int CW = NB * 32;  // columns of the wavefront's tile
     static_assert(NWAVE * 32 * CW * 4 <= STAGES * A_STAGE + B_BUFS * B_STAGE, "staging area fits the stages");
     float* const stage = reinterpret_cast<float*>(lds) + wave * (32 * CW);
-    const int stride = partial && pair ? 2 * N : N;
-    void* const ybase = partial ? static_cast<void*>(partial + (int64_t)split * a.M * stride) : a.seg[seg].y;
-    const bool y_f32 = partial != nullptr || a.out_f32 != 0;
+    const bool parts = partial && !tickets;  // partial tiles, for qmmh_reduce_kernel
+    const int stride = parts && pair ? 2 * N : N;
+    void* const ybase = parts ? static_cast<void*>(partial + (int64_t)split * a.M * stride) : a.seg[seg].y;
+    const bool y_f32 = parts || a.out_f32 != 0;
     // COLS columns of the wavefront's tile leave together, eight consecutive ones per lane; `gated`: act(gate) * up of the two
     // column blocks.  (Partial tiles of a pair keep both sums: the gate columns of all outputs, then the up columns.)
     [[maybe_unused]] bool odd_one = false;  // this lane has stored a value that may not be finite
@@ -1104,23 +1192,14 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) {
             const int mtop = m0 + (wave_m * MB + mb) * 32;  // < mblks * 32 unless the whole block lies past the last row
-            float4 down[4];
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int m = mtop + 4 * h + 8 * q;
-                down[q] = m < a.mblks * 32 ? *reinterpret_cast<const float4*>(a.rs + m) : make_float4(0.f, 0.f, 0.f, 0.f);
-            }
-            const float col_down[2] = {1.0f / col_up[0], 1.0f / col_up[1]};
 #pragma unroll
             for (int r = 0; r < 16; r++) {
-                const float4 d4 = down[r >> 2];
-                const float dm = (r & 3) == 0 ? d4.x : (r & 3) == 1 ? d4.y : (r & 3) == 2 ? d4.z : d4.w;
                 const int at = (8 * (r >> 2) + 4 * h + (r & 3)) * COLS + j;
                 if constexpr (GATED) {
-                    stage[at] = fmul_unfused(act_value(a.act, out[mb][0][r] * dm * col_down[0]), out[mb][1][r] * dm * col_down[1]);
+                    stage[at] = fmul_unfused(act_value(a.act, out[mb][0][r]), out[mb][1][r]);
                 } else {
 #pragma unroll
-                    for (int nb = 0; nb < NB; nb++) stage[at + nb * 32] = out[mb][nb][r] * dm * col_down[nb];
+                    for (int nb = 0; nb < NB; nb++) stage[at + nb * 32] = out[mb][nb][r];
                 }
             }
 #pragma unroll
@@ -1136,7 +1215,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
                     if (route < 0) lo = hi = make_float4(0.f, 0.f, 0.f, 0.f);  // an expert id or a row of x out of range
                     y_row = route & INT32_MAX;
                 }
-                if (G32 && !partial)  // (one test for the eight; fix_output looks at each)
+                if (G32 && !parts)  // (one test for the eight; fix_output looks at each)
                     odd_one |= not_finite(((fabsf(lo.x) + fabsf(lo.y)) + (fabsf(lo.z) + fabsf(lo.w))) + ((fabsf(hi.x) + fabsf(hi.y)) + (fabsf(hi.z) + fabsf(hi.w))));
                 const int64_t o = y_row * stride + col;
                 if (wide && n + 8 <= N) {
@@ -1168,7 +1247,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
             }
         }
     };
-    if (pair && !partial) {
+    if (pair && !parts) {
         store_tile(std::true_type{});
     } else {
         store_tile(std::false_type{});
@@ -1176,7 +1255,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
     if constexpr (G32) {
         // Dense groups of 32 keep what the any-width kernel makes of infinities: a lane goes over what it has stored once more.
         // (Partial tiles: qmmh_reduce_kernel does.)
-        if (a.x && !partial && odd_one) {
+        if (a.x && !parts && odd_one) {
             const int lanes = pair ? 4 : 8, row_in = lane / lanes, c8 = (lane % lanes) * 8;
             const int first = n0 + wave_n * (pair ? 32 : CW) + c8;
 #pragma nounroll
@@ -1195,7 +1274,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
 template <int V>
 __global__ __launch_bounds__(256) void qmmh_reduce_kernel(const QmmHalfArgs a) {
     const QmmSegment& seg = a.seg[blockIdx.y];
-    if (!seg.partial) return;
+    if (!seg.partial || seg.tickets) return;
     const int N = seg.N, stride = a.pair ? 2 * N : N, per_row = N / V;
     const int64_t total = (int64_t)a.M * per_row;
     const int64_t mn = (int64_t)a.M * stride;
@@ -1286,10 +1365,15 @@ int qmmh_x_kind(int bits, int group_size) {
     return bits == 8 ? (group_size == 32 ? kXReadyHalf8G32 : kXReadyHalf8) : (group_size == 32 ? kXReadyHalf32 : kXReadyHalf);
 }
 int qmmh_rows(int idx) { return kQmmHalfTable[idx].v.wm * kQmmHalfTable[idx].v.mb * 32; }
+// One share's partial sums of a matrix in 32 x 32 blocks, and a ticket for each of its tiles on the smallest kernels.
+static size_t half_share_bytes(const QmmHalfCall& q, int i) {
+    return (size_t)((q.M + 31) / 32) * ((q.seg[i].N + 31) / 32) * (q.pair ? 2 : 1) * 4096;
+}
+static size_t half_ticket_bytes(int M, int N) { return ((size_t)((M + 31) / 32) * ((N + 63) / 64) * 4 + 255) & ~(size_t)255; }
 size_t qmmh_partial_bytes(const QmmHalfCall& q) {
     size_t bytes = 0;
     for (int i = 0; i < (q.pair ? 1 : q.nseg); i++)
-        if (q.seg[i].ksplit > 1) bytes += ((size_t)q.seg[i].ksplit * q.M * q.seg[i].N * (q.pair ? 2 : 1) * 4 + 255) & ~(size_t)255;
+        if (q.seg[i].ksplit > 1) bytes += half_share_bytes(q, i) * q.seg[i].ksplit + half_ticket_bytes(q.M, q.seg[i].N);
     return bytes;
 }
 
@@ -1367,8 +1451,8 @@ size_t qmmh_partial_most(int M, int K, int cu_count) {
     // qmmh_split: strips x bands x shares <= 4 CUs, so that shares x N <= 4 CUs x columns of a tile / bands of M rows
     size_t most = 0;
     for (int i = 0; i < qmmh_variant_count(); i++) {
-        const size_t rows = qmmh_rows(i), bn = (size_t)kQmmHalfTable[i].v.wn * kQmmHalfTable[i].v.nb * 32;
-        const size_t bytes = (size_t)4 * cus * bn * ((size_t)M < rows ? (size_t)M : rows) * 4;
+        const size_t rows = qmmh_rows(i), bn = (size_t)kQmmHalfTable[i].v.wn * kQmmHalfTable[i].v.nb * 32, blocks = ((size_t)M + 31) / 32 * 32;
+        const size_t bytes = (size_t)4 * cus * bn * (blocks < rows ? blocks : rows) * 4 + half_ticket_bytes(M, (int)((size_t)4 * cus * bn / half_bands(i, M)) + 64);
         most = bytes > most ? bytes : most;
     }
     return (most + 255) & ~(size_t)255;
@@ -1400,7 +1484,7 @@ int qmmh_pick(const QmmHalfCall& q, int cu_count) {
 }
 
 
-// workspace: fragments, block sums, row factors (qmmt_workspace_bytes sizes them), then the partial tiles of a K split
+// workspace: fragments, block sums, row factors (qmmt_workspace_bytes sizes them), then tickets and partial sums of shares of K
 hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream_t stream) {
     if (idx < 0 || idx >= qmmh_variant_count() || q.nseg < 1 || q.nseg > kQmmSegments || (q.pair && q.nseg != 2)) return hipErrorInvalidValue;
     const QmmHalfEntry& e = kQmmHalfTable[idx];
@@ -1413,21 +1497,6 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     uint16_t* xs = xf + (size_t)mblks * 32 * q.K;
     float* rs = reinterpret_cast<float*>(xs + (size_t)mblks * 32 * g4 * (g32 ? 16 : 8));
     hipError_t rc = hipSuccess;
-    if (q.x_ready != qmmh_x_kind(q.bits, q.group_size)) {
-        typedef void (*PrepKernel)(const uint16_t*, uint16_t*, uint16_t*, float*, int, int, const int32_t*, const int32_t*);
-#define AQ_PREP(R) {{qmmh_prep_kernel<R, 64, 4>, qmmh_prep_kernel<R, 64, 8>}, {qmmh_prep_kernel<R, 32, 4>, qmmh_prep_kernel<R, 32, 8>}}
-        static const PrepKernel kPrep[3][2][2] = {AQ_PREP(1), AQ_PREP(2), AQ_PREP(8)};
-#undef AQ_PREP
-        // rows a workgroup (us, 1 / 2 / 8): 256 x 4096 4.9 / 5.2 / 7.9, 256 x 15360 8.9 / 10.1 / 26; 509 x 4096 6.8 / 6.2 / 9.0, 1024 x
-        // 15360 17.8 / 13.3 / 27; 2048 x 4096 14.7 / 11.9 / 9.9, 2048 x 15360 31.5 / 22.4 / 33
-        const int log_rows = rows <= 256 ? 0 : rows >= 1536 && q.K <= 4096 ? 3 : 1;
-        const PrepKernel fn = kPrep[log_rows == 3 ? 2 : log_rows][g32][q.bits == 8];
-        hipLaunchKernelGGL(fn, dim3((unsigned)((mblks * 4 + 7) / 8 * 8 << (3 - log_rows))), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows, q.K,
-                           q.route_x, q.live_rows);
-        rc = hipGetLastError();
-        if (rc != hipSuccess) return rc;
-    }
-
     QmmHalfArgs a{};
     a.xf = xf;
     a.xs = xs;
@@ -1443,8 +1512,11 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     a.act = q.act;
     a.mblks = mblks;
     const int bm = qmmh_rows(idx), bn = e.v.wn * e.v.nb * 32;
-    char* partial = static_cast<char*>(workspace) + ((qmmt_workspace_bytes(rows, q.K) + 255) & ~(size_t)255);
-    int split_segments = 0;
+    char* const behind = static_cast<char*>(workspace) + ((qmmt_workspace_bytes(rows, q.K) + 255) & ~(size_t)255);
+    uint32_t* const tickets = reinterpret_cast<uint32_t*>(behind);
+    int count = 0;            // tickets
+    size_t ticket_bytes = 0;  // that qmmh_partial_bytes has for them
+    int split_segments = 0;   // whose partial tiles a second kernel adds
     int64_t split_work = 0;
     bool by4 = true;
     for (int i = 0; i < q.nseg; i++) {
@@ -1457,17 +1529,50 @@ hipError_t qmmh_launch(int idx, const QmmHalfCall& q, void* workspace, hipStream
     for (int i = 0; i < q.nseg; i++) {
         QmmSegment& seg = a.seg[i];
         seg.partial = nullptr;
+        seg.tickets = nullptr;
         seg.strips = (int)half_strips(idx, seg.N, q.pair);
         if (q.pair && i == 1) break;
         T += (int64_t)(q.chunks ? q.most_chunks : a.tiles_m) * seg.strips * seg.ksplit;
         if (seg.ksplit > 1) {
             if (q.chunks || seg.gsplit % 4 != 0 || (int64_t)(seg.ksplit - 1) * seg.gsplit * 64 >= q.K) return hipErrorInvalidValue;
-            seg.partial = reinterpret_cast<float*>(partial);
-            partial += ((size_t)seg.ksplit * q.M * seg.N * (q.pair ? 2 : 1) * 4 + 255) & ~(size_t)255;
-            split_segments++;
-            split_work = (int64_t)q.M * seg.N > split_work ? (int64_t)q.M * seg.N : split_work;
-            by4 = by4 && seg.N % 4 == 0;
+            ticket_bytes += half_ticket_bytes(q.M, seg.N);
+            // Who adds the shares: the last workgroup of a tile where the others' sums are up to 100 KiB, else a kernel behind this one.  (A
+            // CU reads some 18 KB a microsecond, the whole chip 4.5 TB/s behind a launch: 240 tiles of 128 x 128 in two shares 31.6 + 6.0
+            // us -> 34.3, 116 of 192 x 256 82 + 10 -> 102.)  Over 40 layers of 66 to 2048 rows, against that kernel for all: limits of 48 / 64 / 100 /
+            // 128 / 160 KiB 1.2 / 1.7 / 2.4 / 2.3 / 2.3 % faster, the slowest layer 1 / 1 / 0 / 1 / 5 % slower.
+            if ((int64_t)(seg.ksplit - 1) * (bm < mblks * 32 ? bm : mblks * 32) * bn * 4 <= 100 << 10) {
+                seg.tickets = tickets + count;
+                count += a.tiles_m * seg.strips;
+            } else {
+                split_segments++;
+                split_work = (int64_t)q.M * seg.N > split_work ? (int64_t)q.M * seg.N : split_work;
+                by4 = by4 && seg.N % 4 == 0;
+            }
         }
+    }
+    char* partial = behind + ticket_bytes;
+    for (int i = 0; i < (q.pair ? 1 : q.nseg); i++) {
+        QmmSegment& seg = a.seg[i];
+        if (seg.ksplit <= 1) continue;
+        seg.partial = reinterpret_cast<float*>(partial);
+        partial += (size_t)mblks * ((seg.N + 31) / 32) * (q.pair ? 2 : 1) * 4096 * seg.ksplit;
+    }
+    if (q.x_ready != qmmh_x_kind(q.bits, q.group_size)) {
+        typedef void (*PrepKernel)(const uint16_t*, uint16_t*, uint16_t*, float*, int, int, const int32_t*, const int32_t*, uint32_t*, int);
+#define AQ_PREP(R) {{qmmh_prep_kernel<R, 64, 4>, qmmh_prep_kernel<R, 64, 8>}, {qmmh_prep_kernel<R, 32, 4>, qmmh_prep_kernel<R, 32, 8>}}
+        static const PrepKernel kPrep[3][2][2] = {AQ_PREP(1), AQ_PREP(2), AQ_PREP(8)};
+#undef AQ_PREP
+        // rows a workgroup (us, 1 / 2 / 8): 256 x 4096 4.9 / 5.2 / 7.9, 256 x 15360 8.9 / 10.1 / 26; 509 x 4096 6.8 / 6.2 / 9.0, 1024 x
+        // 15360 17.8 / 13.3 / 27; 2048 x 4096 14.7 / 11.9 / 9.9, 2048 x 15360 31.5 / 22.4 / 33
+        const int log_rows = rows <= 256 ? 0 : rows >= 1536 && q.K <= 4096 ? 3 : 1;
+        const PrepKernel fn = kPrep[log_rows == 3 ? 2 : log_rows][g32][q.bits == 8];
+        hipLaunchKernelGGL(fn, dim3((unsigned)((mblks * 4 + 7) / 8 * 8 << (3 - log_rows))), dim3(kPrepThreads), 0, stream, q.x, xf, xs, rs, rows, q.K,
+                           q.route_x, q.live_rows, tickets, count);
+        rc = hipGetLastError();
+        if (rc != hipSuccess) return rc;
+    } else if (count > 0) {
+        rc = fill_zero_launch(tickets, (size_t)count * 4, stream);
+        if (rc != hipSuccess) return rc;
     }
     {
         // the patch an XCD's 32 CUs work on at a time: group_m row bands by the rest in column strips, fewest bytes per step

@@ -64,7 +64,6 @@ template <typename T>
 __device__ __forceinline__ T load_at(global_t base, uint32_t off) {
     return *reinterpret_cast<const __attribute__((address_space(1))) T*>(base + hidden(off));
 }
-__device__ __forceinline__ global_t in_memory(const void* p) { return (global_t)(const uint8_t*)p; }
 // largest finite magnitude (bf16 bits) of the halves of a word and of `most`
 __device__ __forceinline__ uint32_t most_of(uint32_t most, uint32_t w) {
     const uint32_t lo = w & 0x7fffu, hi = w >> 16 & 0x7fffu;
