@@ -470,6 +470,13 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
     return fail(AQ_ERR_UNSUPPORTED, "aq_qmv: no kernel for bits=%d group=%d rows=%d K=%d N=%d", bits, group_size, a.M, a.K, a.N);
 }
 
+// Whether two to eight rows of x run on the dot2 kernels, four a launch, whatever the number of rows of weights: groups of 64 of 4
+// bit at a K that the diagonal kernels do not take.
+bool dot2_rows(const aq_ctx* ctx, int bits, int group_size, int M, int K, const void* x, const void* w) {
+    return bits == 4 && group_size == 64 && M >= 2 && M <= 8 && ctx->forced[0] < 0 && !(ctx->families_off >> kFamDot2 & 1) &&
+           aq::qmvd_pick(1, K, 1) < 0 && dot2_eligible(K, group_size, bits, x, w, (size_t)(M < 4 ? M : 4) * K * 2);
+}
+
 // Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
 // the launch forms that put several matrices into one grid).
 bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, bool pair) {
@@ -931,6 +938,23 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
                 return AQ_OK;
             }
         }
+    }
+    if (fused && M > 1 && !tiled) {
+        // The dot2 kernels over all matrices, as many launches as one matrix by itself takes.  (One by one, with a pair as two matvec calls
+        // and the activation, a layer took, us, before -> here: two rows of 1216 / 4032 41.7 -> 27.3, four of 896 / 3584 38.2 -> 26.0, of
+        // 3008 / 9024 69.5 -> 54.5, eight of 1024 / 3072 60.0 -> 38.1, of 3008 / 9024 128 -> 102.)
+        bool takes = true;
+        for (int i = 0; i < count; i++) takes = takes && N[i] > 0 && dot2_rows(ctx, bits, group_size, M, K, x, packed[i]);
+        for (int m0 = 0; takes && m0 < M; m0 += 4) {
+            const int m = M - m0 < 4 ? M - m0 : 4;
+            const size_t row_bytes = (flags & AQ_OUT_F32) ? 4 : 2;
+            void* at[aq::kQmvMultiMax];
+            for (int i = 0; i < count; i++) at[i] = static_cast<char*>(y[i]) + (size_t)m0 * N[i] * row_bytes;
+            const aq::QmvMultiArgs ma = multi_args(static_cast<const uint16_t*>(x) + (size_t)m0 * K, count, packed, scales, biases, at, N, m, K, group_size, flags);
+            ctx->last_variant[0] = "qmvr_multi_dot2";
+            AQ_HIP(aq::qmv_multi_launch(bits, m, m > 1 ? 2 : 1, ma, ctx->stream), "hipLaunchKernel");
+        }
+        if (takes) return AQ_OK;
     }
     // several rows: the token-tile kernels over all matrices in one grid (aq_qmv names what is wrong with a call).  A member
     // belongs to it if its own call runs on them: the choice by the rows of all members together would move members across a
@@ -1486,8 +1510,8 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         gate_packed = w[0], gate_scales = sc[0], gate_biases = bi[0];
         up_packed = w[1], up_scales = sc[1], up_biases = bi[1];
     }
-    if (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) &&
-        aligned(up_packed, 16)) {
+    const bool pair_rows = M > 1 && dot2_rows(ctx, bits, group_size, M, K, x, gate_packed) && dot2_rows(ctx, bits, group_size, M, K, x, up_packed);
+    if (pair_rows || (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) && aligned(up_packed, 16))) {
         const int rows = act_rows(ctx, bits, 1, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 1, rows, false)) {
             aq::QmvArgs a{};
@@ -1507,7 +1531,12 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
             a.routes = 1;
             a.act = act;
             ctx->last_variant[0] = "qmv_gate_up_dot2";
-            AQ_HIP(aq::qmv_act_launch(bits, 1, rows, false, a, ctx->stream), "hipLaunchKernel");
+            for (int m0 = 0; m0 < M; m0 += 4) {
+                a.M = M - m0 < 4 ? M - m0 : 4;
+                a.x = static_cast<const uint16_t*>(x) + (size_t)m0 * K;
+                a.y = static_cast<char*>(y) + (size_t)m0 * N * (out_f32 ? 4 : 2);
+                AQ_HIP(aq::qmv_act_launch(bits, 1, rows, false, a, ctx->stream), "hipLaunchKernel");
+            }
             return AQ_OK;
         }
     }

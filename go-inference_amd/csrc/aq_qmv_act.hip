@@ -1,4 +1,4 @@
-// Activation-fused matvec kernels for the MLP of a decode step (one activation row).
+// Activation-fused matvec kernels for the MLP of a decode step (one activation row; the dense pair of 4 bit up to four).
 //
 //   pair fusion    y[n] = act(gate[n,:] . x) * (up[n,:] . x): both projections and the activation in one
 //                  launch, as rocm_mlx_q4_gelu_tanh_multiply does
@@ -17,36 +17,38 @@
 
 namespace aq {
 
-template <int BITS, int R, bool GATHER, int FUSE>
+template <int BITS, int R, bool GATHER, int FUSE, int M = 1>
 __global__ __launch_bounds__(4 * kWave) void qmv_act_kernel(const QmvArgs a) {
-    qmv_dot2_body<BITS, 1, R, 4, 2, GATHER, FUSE>(a, blockIdx.x);
+    qmv_dot2_body<BITS, M, R, 4, 2, GATHER, FUSE>(a, blockIdx.x);
 }
 
 typedef void (*QmvActKernel)(const QmvArgs);
 struct QmvActEntry {
-    int bits, fuse, rows, gather;
+    int bits, fuse, rows, gather, m;
     QmvActKernel fn;
 };
-#define AQ_ACT(BITS, FUSE, R, G) {BITS, FUSE, R, G, qmv_act_kernel<BITS, R, (G != 0), FUSE>}
+#define AQ_ACT(BITS, FUSE, R, G) {BITS, FUSE, R, G, 1, qmv_act_kernel<BITS, R, (G != 0), FUSE>}
+#define AQ_ACT_M(M) {4, 1, 1, 0, M, qmv_act_kernel<4, 1, false, 1, M>}, {4, 1, 2, 0, M, qmv_act_kernel<4, 2, false, 1, M>}
 #define AQ_ACT_SET(BITS, G)                                                                            \
     AQ_ACT(BITS, 1, 1, G), AQ_ACT(BITS, 1, 2, G), AQ_ACT(BITS, 2, 1, G), AQ_ACT(BITS, 2, 2, G), \
         AQ_ACT(BITS, 2, 4, G)
-static const QmvActEntry kActTable[] = {AQ_ACT_SET(4, 0), AQ_ACT_SET(4, 1), AQ_ACT_SET(8, 0), AQ_ACT_SET(8, 1)};
+static const QmvActEntry kActTable[] = {AQ_ACT_SET(4, 0), AQ_ACT_SET(4, 1), AQ_ACT_SET(8, 0), AQ_ACT_SET(8, 1),
+                                         AQ_ACT_M(2), AQ_ACT_M(3), AQ_ACT_M(4)};
 
-static const QmvActEntry* find_act(int bits, int fuse, int rows, bool gather) {
+static const QmvActEntry* find_act(int bits, int fuse, int rows, bool gather, int m) {
     for (const QmvActEntry& e : kActTable)
-        if (e.bits == bits && e.fuse == fuse && e.rows == rows && (e.gather != 0) == gather) return &e;
+        if (e.bits == bits && e.fuse == fuse && e.rows == rows && (e.gather != 0) == gather && e.m == m) return &e;
     return nullptr;
 }
 
-bool qmv_act_supported(int bits, int fuse, int rows, bool gather) { return find_act(bits, fuse, rows, gather) != nullptr; }
+bool qmv_act_supported(int bits, int fuse, int rows, bool gather, int m) { return find_act(bits, fuse, rows, gather, m) != nullptr; }
 
 hipError_t qmv_act_launch(int bits, int fuse, int rows, bool gather, const QmvArgs& a, hipStream_t stream) {
-    const QmvActEntry* e = find_act(bits, fuse, rows, gather);
-    if (!e || a.M != 1) return hipErrorInvalidValue;
+    const QmvActEntry* e = find_act(bits, fuse, rows, gather, a.M);
+    if (!e) return hipErrorInvalidValue;
     const int rows_per_wg = rows * 4;
     dim3 grid((unsigned)((a.N + rows_per_wg - 1) / rows_per_wg), gather ? (unsigned)a.routes : 1u, 1u);
-    const size_t lds = (size_t)a.K * 2;
+    const size_t lds = (size_t)a.M * a.K * 2;
     if (hipError_t rc = ensure_dynamic_lds(reinterpret_cast<const void*>(e->fn), (size_t)lds)) return rc;
     hipLaunchKernelGGL(e->fn, grid, dim3(4 * kWave), lds, stream, a);
     return hipGetLastError();
