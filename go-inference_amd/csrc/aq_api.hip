@@ -470,11 +470,12 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
     return fail(AQ_ERR_UNSUPPORTED, "aq_qmv: no kernel for bits=%d group=%d rows=%d K=%d N=%d", bits, group_size, a.M, a.K, a.N);
 }
 
-// Whether two to eight rows of x run on the dot2 kernels, four a launch, whatever the number of rows of weights: groups of 64 of 4
-// bit at a K that the diagonal kernels do not take.
-bool dot2_rows(const aq_ctx* ctx, int bits, int group_size, int M, int K, const void* x, const void* w) {
-    return bits == 4 && group_size == 64 && M >= 2 && M <= 8 && ctx->forced[0] < 0 && !(ctx->families_off >> kFamDot2 & 1) &&
-           aq::qmvd_pick(1, K, 1) < 0 && dot2_eligible(K, group_size, bits, x, w, (size_t)(M < 4 ? M : 4) * K * 2);
+// Whether several rows of x run on the dot2 kernels, four a launch: groups of 64 at a K that the diagonal kernels do not take, two to
+// eight rows of 4-bit codes, two to four of 8 bit where the matrix is small (tok_small).
+bool dot2_rows(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, const void* x, const void* w) {
+    if (group_size != 64 || M < 2 || ctx->forced[0] >= 0 || (ctx->families_off >> kFamDot2 & 1)) return false;
+    if (bits == 8 ? M > 4 || !tok_small(8, 64, M, K, rows) : bits != 4 || M > 8 || aq::qmvd_pick(1, K, 1) >= 0) return false;
+    return dot2_eligible(K, group_size, bits, x, w, (size_t)(M < 4 ? M : 4) * K * 2);
 }
 
 // Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
@@ -939,22 +940,28 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
             }
         }
     }
+    // The members that the dot2 kernels run, all in one grid, as many launches as one of them by itself takes.  (One by one, with a pair as
+    // two matvec calls and the activation, a layer took, us, before -> here: two rows of 1216 / 4032 41.7 -> 27.3, four of 896 / 3584 38.2 ->
+    // 26.0, of 3008 / 9024 69.5 -> 54.5, eight of 1024 / 3072 60.0 -> 38.1, of 3008 / 9024 128 -> 102; 8 bit, two
+    // rows of 832 / 2368 40.9 -> 27.0, four of 1984 / 5952 38.1 -> 30.6.)
+    unsigned done = 0;
     if (fused && M > 1 && !tiled) {
-        // The dot2 kernels over all matrices, as many launches as one matrix by itself takes.  (One by one, with a pair as two matvec calls
-        // and the activation, a layer took, us, before -> here: two rows of 1216 / 4032 41.7 -> 27.3, four of 896 / 3584 38.2 -> 26.0, of
-        // 3008 / 9024 69.5 -> 54.5, eight of 1024 / 3072 60.0 -> 38.1, of 3008 / 9024 128 -> 102.)
-        bool takes = true;
-        for (int i = 0; i < count; i++) takes = takes && N[i] > 0 && dot2_rows(ctx, bits, group_size, M, K, x, packed[i]);
-        for (int m0 = 0; takes && m0 < M; m0 += 4) {
+        const void *w[aq::kQmvMultiMax], *sc[aq::kQmvMultiMax], *bi[aq::kQmvMultiMax];
+        void* to[aq::kQmvMultiMax];
+        int n[aq::kQmvMultiMax], some = 0;
+        for (int i = 0; i < count; i++) {
+            if (N[i] == 0 || !dot2_rows(ctx, bits, group_size, M, K, N[i], x, packed[i])) continue;
+            w[some] = packed[i], sc[some] = scales[i], bi[some] = biases[i], to[some] = y[i], n[some++] = N[i];
+            done |= 1u << i;
+        }
+        for (int m0 = 0; some > 0 && m0 < M; m0 += 4) {
             const int m = M - m0 < 4 ? M - m0 : 4;
-            const size_t row_bytes = (flags & AQ_OUT_F32) ? 4 : 2;
-            void* at[aq::kQmvMultiMax];
-            for (int i = 0; i < count; i++) at[i] = static_cast<char*>(y[i]) + (size_t)m0 * N[i] * row_bytes;
-            const aq::QmvMultiArgs ma = multi_args(static_cast<const uint16_t*>(x) + (size_t)m0 * K, count, packed, scales, biases, at, N, m, K, group_size, flags);
-            ctx->last_variant[0] = "qmvr_multi_dot2";
+            aq::QmvMultiArgs ma = multi_args(static_cast<const uint16_t*>(x) + (size_t)m0 * K, some, w, sc, bi, to, n, m, K, group_size, flags);
+            for (int i = 0; i < some; i++) ma.y[i] = static_cast<char*>(to[i]) + (size_t)m0 * n[i] * ((flags & AQ_OUT_F32) ? 4 : 2);
+            ctx->last_variant[0] = bits == 4 ? "qmvr_multi_dot2" : "qmvr8_multi_dot2";
             AQ_HIP(aq::qmv_multi_launch(bits, m, m > 1 ? 2 : 1, ma, ctx->stream), "hipLaunchKernel");
         }
-        if (takes) return AQ_OK;
+        if (done + 1 == 1u << count) return AQ_OK;
     }
     // several rows: the token-tile kernels over all matrices in one grid (aq_qmv names what is wrong with a call).  A member
     // belongs to it if its own call runs on them: the choice by the rows of all members together would move members across a
@@ -972,7 +979,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
         grid.common = all.common;
         grid.tokens = aq::qmvt_tokens(M);
         for (int i = 0; i < count; i++) {
-            if (N[i] == 0 || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i], false)) continue;
+            if (N[i] == 0 || (done >> i & 1) || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i], false)) continue;
             aq::TokArgs own{multi_member(grid, i)};
             own.tokens = grid.tokens;
             own.w = all.w[i];
@@ -1029,7 +1036,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
         if (ti < 0 || bytes > aq::kTokTileBytes) in_grid = 0;  // (members apart have the block to themselves, one after another)
     }
     for (int i = 0; i < count; i++) {
-        if (in_grid >> i & 1) continue;
+        if ((in_grid | done) >> i & 1) continue;
         if (int rc = qmv_call(ctx, x, packed[i], scales[i], biases[i], y[i], M, K, N[i], group_size, bits, flags)) return rc;
     }
     if (in_grid) {
@@ -1510,7 +1517,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         gate_packed = w[0], gate_scales = sc[0], gate_biases = bi[0];
         up_packed = w[1], up_scales = sc[1], up_biases = bi[1];
     }
-    const bool pair_rows = M > 1 && dot2_rows(ctx, bits, group_size, M, K, x, gate_packed) && dot2_rows(ctx, bits, group_size, M, K, x, up_packed);
+    const bool pair_rows = M > 1 && dot2_rows(ctx, bits, group_size, M, K, N, x, gate_packed) && dot2_rows(ctx, bits, group_size, M, K, N, x, up_packed);
     if (pair_rows || (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) && aligned(up_packed, 16))) {
         const int rows = act_rows(ctx, bits, 1, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 1, rows, false)) {

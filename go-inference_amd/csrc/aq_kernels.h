@@ -65,7 +65,7 @@ constexpr int kActSilu = 2;
 //   fuse 1: y[n] = act(gate[n,:] . x) * (up[n,:] . x)          (two matrices, one output)
 //   fuse 2: y[n] = w[n,:] . bf16(act(x[k]) * x2[k])            (activation applied while x is staged)
 // rows: output rows per wavefront (fuse 1: of each matrix).  False / error when no kernel fits.
-bool qmv_act_supported(int bits, int fuse, int rows, bool gather, int m = 1);  // (m > 1: the dense pair of 4 bit)
+bool qmv_act_supported(int bits, int fuse, int rows, bool gather, int m = 1);  // (m > 1: the dense pair)
 hipError_t qmv_act_launch(int bits, int fuse, int rows, bool gather, const QmvArgs& a, hipStream_t stream);
 // y[i] = bf16(act(gate[i]) * up[i]) over n bf16 values.
 hipError_t act_mul_launch(const uint16_t* gate, const uint16_t* up, uint16_t* y, int64_t n, int act, hipStream_t stream);

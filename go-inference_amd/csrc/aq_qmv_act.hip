@@ -1,4 +1,4 @@
-// Activation-fused matvec kernels for the MLP of a decode step (one activation row; the dense pair of 4 bit up to four).
+// Activation-fused matvec kernels for the MLP of a decode step (one activation row; the dense pair up to four).
 //
 //   pair fusion    y[n] = act(gate[n,:] . x) * (up[n,:] . x): both projections and the activation in one
 //                  launch, as rocm_mlx_q4_gelu_tanh_multiply does
@@ -28,12 +28,12 @@ struct QmvActEntry {
     QmvActKernel fn;
 };
 #define AQ_ACT(BITS, FUSE, R, G) {BITS, FUSE, R, G, 1, qmv_act_kernel<BITS, R, (G != 0), FUSE>}
-#define AQ_ACT_M(M) {4, 1, 1, 0, M, qmv_act_kernel<4, 1, false, 1, M>}, {4, 1, 2, 0, M, qmv_act_kernel<4, 2, false, 1, M>}
+#define AQ_ACT_M(BITS, M) {BITS, 1, 1, 0, M, qmv_act_kernel<BITS, 1, false, 1, M>}, {BITS, 1, 2, 0, M, qmv_act_kernel<BITS, 2, false, 1, M>}
 #define AQ_ACT_SET(BITS, G)                                                                            \
     AQ_ACT(BITS, 1, 1, G), AQ_ACT(BITS, 1, 2, G), AQ_ACT(BITS, 2, 1, G), AQ_ACT(BITS, 2, 2, G), \
         AQ_ACT(BITS, 2, 4, G)
 static const QmvActEntry kActTable[] = {AQ_ACT_SET(4, 0), AQ_ACT_SET(4, 1), AQ_ACT_SET(8, 0), AQ_ACT_SET(8, 1),
-                                         AQ_ACT_M(2), AQ_ACT_M(3), AQ_ACT_M(4)};
+                                         AQ_ACT_M(4, 2), AQ_ACT_M(4, 3), AQ_ACT_M(4, 4), AQ_ACT_M(8, 2), AQ_ACT_M(8, 3), AQ_ACT_M(8, 4)};
 
 static const QmvActEntry* find_act(int bits, int fuse, int rows, bool gather, int m) {
     for (const QmvActEntry& e : kActTable)
