@@ -135,10 +135,11 @@ int aq_probe_read(aq_ctx *ctx, const void *packed, const void *scales, const voi
  * form (go/engine/metal/qmv_rows.go:14-60).  M >= 1; rows of x are contiguous.
  * N == 0 or K == 0 is a no-op returning AQ_OK (qmv.go:365-371).
  * 4- and 8-bit codes, K a multiple of 64 up to 16384, operands 16-byte aligned: up to 32 rows of x, from 9 on in groups of 64
- * (8 bit: from 2, or 5 where K is 2048, 4096 or 8192), from 5 in groups of 128, from 3 in groups of 32 (8 bit: 2), the
- * token-tile kernels run the call (small matrices with K no multiple of 256 excepted): one launch, or two where workgroups share
- * a long K out, and a row of x has the same bytes whatever the number of rows beside it.  33 to 64 rows run there too on
- * matrices of more than 528 rows that are not too wide, with the same identity among themselves. */
+ * (8 bit: from 2, or 5 where K is 2048, 4096 or 8192), from 2 in groups of 128 (from 5 beyond 64 Mi codes), from 3 in groups of
+ * 32 (8 bit, and K no multiple of 256: 2), the token-tile kernels run the call (small matrices with K no multiple of 256 excepted, but
+ * for 4 bit in whole sets of 16 rows): one launch, or two where workgroups share a long K out, and a row of x has the same bytes
+ * whatever the number of rows beside it.  33 to 64 rows run there too on matrices of more than 528 rows, or of 256 and more in whole sets
+ * of 16, that are not too wide, with the same identity among themselves. */
 int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, const void *biases, void *y, int M,
            int K, int N, int group_size, int bits, unsigned flags);
 
@@ -147,8 +148,9 @@ int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, c
  * pointers.  Results are byte-identical to `count` separate aq_qmv calls.  This is the no-copy form of
  * running q|k|v or gate|up over model.ConcatQuantRows (go/model/quant_weight.go:32-62): at batch 1 the
  * narrow projections are bound by launch latency, not bandwidth, and one grid over all of them fills
- * the machine.  One launch for one activation row (up to four when K is a multiple of 128 between 1152 and 16384; 8-bit codes:
- * up to four where every member's own call runs on the diagonal kernels), and for the row counts the token-tile kernels run
+ * the machine.  One launch for one activation row (4-bit codes in groups of 64: up to eight rows, or one launch per four of them where
+ * aq_qmv takes as many; 8-bit codes: up to four where every member's own call runs on the diagonal kernels, or those members that run
+ * on the dot2 kernels), and for the row counts the token-tile kernels run
  * (see aq_qmv) over those members whose own call runs on them, with one more launch where a member shares K out; other shapes
  * and members are run as separate launches. */
 int aq_qmv_multi(aq_ctx *ctx, const void *x, int count, const void *const *packed, const void *const *scales,
@@ -224,8 +226,8 @@ int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *sc
  * launch go/engine/hip/hip_projection_launch.go:3086-3160, packet contract/launch_abi.hipinc:634-657).
  * gate and up are [N, K*bits/32] with their own scales/biases; for a row-concatenated gate|up slab
  * (model.ConcatQuantRows, go/model/quant_weight.go:32-62) pass the slab for gate and slab + N rows for up.
- * M == 1 with 4/8-bit codes (up to 4 rows of 4-bit group-64 codes when K is a multiple of 256 between 1280 and 8192) runs as ONE
- * launch that reads every weight once.  So do rows up to 64 where aq_qmv runs its token-tile kernels, from 33 on reading every
+ * M == 1 with 4/8-bit codes runs as ONE launch that reads every weight once, up to 8 rows of 4-bit group-64 codes (up to 4 of small
+ * 8-bit ones with K no multiple of 256) as one or two.  So do rows up to 64 where aq_qmv runs its token-tile kernels, from 33 on reading every
  * weight twice, with a second launch where workgroups share a long K out; and more rows on the tiles of aq_qmm behind a pass
  * over x.  Other shapes run the two projections and the element-wise step as separate launches through the context's
  * workspace (which grows on demand like aq_qmm's; not while a capture is open). */
