@@ -281,6 +281,9 @@ __device__ __forceinline__ void fix_output(const QmmHalfArgs& a, const QmmSegmen
         static_cast<uint16_t*>(seg.y)[at] = f32_to_bf16_bits(y);
 }
 
+// Whether a tile has LDS for its rows' factors (two of the 8-bit kernels fill half a CU's with their stages).
+__host__ __device__ constexpr bool half_rows_in_lds(int bits, int mb, int waves) { return !(bits == 8 && mb == 2 && waves == 4); }
+
 // ---- main kernel ----------------------------------------------------------------------------
 // SE: elements of a row of scales (and of biases) in LDS at a time.
 // GRP 32: the codes a lane half h expands are those of one group (block g's half h), so that only its scale and bias differ:
@@ -572,11 +575,21 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
             scan(tiny);
         }
     };
+    // The rows' factors wait in LDS for the epilogue, whose first loads they were, behind all of K and ahead of every store (2048 rows of 4096 /
+    // 14336 949 -> 936 us with the sums of shares, 958 -> 942 by this alone; 40 layers of 66 to 2048 rows 0.7 % faster).
+    constexpr bool RS_LDS = half_rows_in_lds(BITS, MB, NWAVE);
+    static_assert(BM <= THREADS, "a row's factor a thread");
+    float* const rbuf = reinterpret_cast<float*>(sbuf + 2 * BN * SE) + (XS_LDS ? BM / 32 * 256 : 0);
+    [[maybe_unused]] float row_down = 0.0f;
+    if constexpr (RS_LDS)
+        if (tid < BM) row_down = a.rs[min(m0 + tid, a.mblks * 32 - 1)];
     if (sb_total < 8)
         prologue(std::true_type{});
     else
         prologue(std::false_type{});
     store_segment(0, piece);
+    if constexpr (RS_LDS)
+        if (tid < BM) rbuf[tid] = row_down;
     // A quad's scales (which 0) or biases (1) of this lane's rows: the bf16 bits of its four blocks in two words per column block
     // (groups of 32: this lane half's four of the quad's eight).
     const uint32_t half_sel = h ? 0x07060302u : 0x05040100u;
@@ -1092,11 +1105,15 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         const float col_down[2] = {1.0f / col_up[0], 1.0f / col_up[1]};
 #pragma unroll
         for (int mb = 0; mb < MB; mb++) {
-            const int mtop = m0 + (wave_m * MB + mb) * 32;  // < mblks * 32 unless the whole block lies past the last row
+            const int in_tile = (wave_m * MB + mb) * 32;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const int m = mtop + 4 * h + 8 * q;
-                const float4 down = m < a.mblks * 32 ? *reinterpret_cast<const float4*>(a.rs + m) : make_float4(0.f, 0.f, 0.f, 0.f);
+                const int r = in_tile + 4 * h + 8 * q, m = m0 + r;  // m < mblks * 32 unless the whole block lies past the last row
+                float4 down = make_float4(0.f, 0.f, 0.f, 0.f);
+                if constexpr (RS_LDS)
+                    down = *reinterpret_cast<const float4*>(rbuf + r);
+                else if (m < a.mblks * 32)
+                    down = *reinterpret_cast<const float4*>(a.rs + m);
 #pragma unroll
                 for (int nb = 0; nb < NB; nb++) {
                     out[mb][nb][4 * q] = out[mb][nb][4 * q] * down.x * col_down[nb];
@@ -1333,7 +1350,7 @@ struct QmmHalfEntry {
         {PREFIX #MB "_nb" #NB "_wm" #WM "_wn" #WN SUFFIX, BITS, MB, NB, WM, WN},                                                 \
             qmmh_kernel<BITS, MB, NB, WM, WN, ST, SE, 64>, qmmh_kernel<BITS, MB, NB, WM, WN, ST, SE, 32>, \
             ST*(WM * MB * 4096) + (BITS == 8 ? ST : 2) * (WN * NB * 32 * 64) + 2 * (WN * NB * 32) * SE * 2 +                      \
-                (BITS == 4 && MB >= 3 ? WM * MB * 1024 : 0)                                                                      \
+                (BITS == 4 && MB >= 3 ? WM * MB * 1024 : 0) + (half_rows_in_lds(BITS, MB, WM * WN) ? WM * MB * 128 : 0)          \
     }
 #define AQ_QMMH4(...) AQ_QMMH("qmmh_b4_mb", 4, __VA_ARGS__)
 #define AQ_QMMH8(...) AQ_QMMH("qmmh8_b8_mb", 8, __VA_ARGS__)
