@@ -335,7 +335,10 @@ __global__ __launch_bounds__(kThreads, GRP == 32 ? 2 : 3) void qmmr_kernel(const
             const uint32_t l = hidden((uint32_t)lane);
             copy16_to_lds(a.xs, sum_at[wave * 16 + (l & 15)] + ((uint32_t)(seg * kElements) + (l >> 4) * 4) * 4, sums_at + (uint32_t)wave * 1024);
         };
-        // bias and 8 * scale, each times the sums of x over the segment (two bf16 a sum: two slots of the product a group)
+        // bias and 8 * scale times the sums of x over the segment (two bf16 a sum: two slots of a product for either).  The two nearly cancel,
+        // so a product takes both of eight groups.  (All biases in one and all scales in the next left the accumulator with the large half
+        // in between.  fp32 error against float64, tiles of 32 routes / so / here: groups of 64, K of 704 1.69e-7 / 1.84e-7 / 1.63e-7, of
+        // 4096 4.04e-7 / 4.15e-7 / 4.02e-7, of 32, K of 576 1.70e-7 / 1.82e-7 / 1.53e-7, of 128, K of 1280 2.24e-7 / 2.35e-7 / 2.17e-7; 173 us the block both ways.)
         auto affine = [&](int cp) __attribute__((always_inline)) {
 #pragma unroll
             for (int i = 0; i < 2; i++) {
@@ -350,9 +353,11 @@ __global__ __launch_bounds__(kThreads, GRP == 32 ? 2 : 3) void qmmr_kernel(const
                 }
 #pragma unroll
                 for (int rb = 0; rb < RB; rb++) {
-                    const bf16x8_t x8 = *reinterpret_cast<const bf16x8_t*>(sums + rb * 256 + lane * 4);
-                    acc[rb][cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x8, __builtin_bit_cast(bf16x8_t, make_uint4(bw[0], bw[1], bw[2], bw[3])), acc[rb][cg], 0, 0, 0);
-                    acc[rb][cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x8, __builtin_bit_cast(bf16x8_t, make_uint4(ew[0], ew[1], ew[2], ew[3])), acc[rb][cg], 0, 0, 0);
+                    const uint4 x4 = *reinterpret_cast<const uint4*>(sums + rb * 256 + lane * 4);
+                    acc[rb][cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, make_uint4(x4.x, x4.x, x4.y, x4.y)),
+                                                                          __builtin_bit_cast(bf16x8_t, make_uint4(bw[0], ew[0], bw[1], ew[1])), acc[rb][cg], 0, 0, 0);
+                    acc[rb][cg] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, make_uint4(x4.z, x4.z, x4.w, x4.w)),
+                                                                          __builtin_bit_cast(bf16x8_t, make_uint4(bw[2], ew[2], bw[3], ew[3])), acc[rb][cg], 0, 0, 0);
                 }
             }
         };

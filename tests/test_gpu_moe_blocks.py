@@ -48,3 +48,39 @@ def test_rows_of_x(ctx, x_rows, use_lhs):
     check_accumulators(got[plain], ref[plain], "blocks of routes")
     for t in (dx, dl, dr, dy, dw):
         t.free()
+
+
+@pytest.mark.parametrize("gs,K", [(64, 704), (32, 576), (128, 1280)])
+def test_no_further_from_float64_than_tiles_of_32_routes(ctx, gs, K):
+    """The first experts' routes once among those of many experts (blocks of 16) and once by themselves, too few workgroups for blocks: the
+    fp32 results of the blocks are no further from float64."""
+    import aq_mi355
+    routes, E, few, N = 2600, 80, 8, 1280
+    say("error of blocks of routes", gs, K)
+    rng = np.random.default_rng(K)
+    words, s, b = F.synthetic_affine(E * N, K, 4, gs, seed=K)
+    x = F.synthetic_x(routes // 2, K, seed=5)
+    rhs, lhs = rng.integers(0, E, routes).astype(np.int32), rng.integers(0, routes // 2, routes).astype(np.int32)
+    mine = np.nonzero(rhs < few)[0]
+    dw, dx = DeviceAffine(ctx, words, s, b), ctx.to_device(x)
+
+    def run(ids, rows, experts):
+        dr, dl, dy = ctx.to_device(ids), ctx.to_device(rows), ctx.alloc(len(ids) * N * 4)
+        ctx.gather_qmv(dx, dw.w, dw.s, dw.b, dl, dr, dy, len(ids), routes // 2, K, N, experts, N, 0, gs, 4, aq_mi355.AQ_OUT_F32)
+        ctx.sync()
+        got = dy.download(np.float32, len(ids) * N).reshape(len(ids), N).astype(np.float64)
+        for t in (dr, dl, dy):
+            t.free()
+        return got, ctx.last_variant(0)
+
+    blocks, name = run(rhs, lhs, E)
+    assert name == "gather_grouped_blocks", name
+    tiles, name = run(rhs[mine], lhs[mine], few)
+    assert name == "gather_grouped_tiles", name
+    ref = np.zeros_like(tiles)
+    for e in range(few):
+        z, rows = np.nonzero(rhs[mine] == e)[0], slice(e * N, (e + 1) * N)
+        ref[z] = F.reference_f64(x[lhs[mine][z]], words[rows], s[rows], b[rows], 4, gs, K)
+    assert np.linalg.norm(blocks[mine] - ref) <= np.linalg.norm(tiles - ref)
+    for t in (dx, dw):
+        t.free()
