@@ -257,8 +257,8 @@ const QmvRule kQmvRules[] = {
     {4, 64, 0, 2, 8, kFamDot2},             // K the diagonal kernels do not take (up to 1024, no multiple of 128, beyond
                                             // 16384): the kernel a single row of such a K runs on, four rows a launch, so
                                             // that rows keep the bytes of single-row calls here too
-    {4, 32, 0, 1, 2, kFamDiag},             // groups of 32: two tokens x eight groups as MFMA rows (K a multiple of 256; two rows of another
-                                            // K: token tile, a layer of 1216 / 4032 23.4 us on dot2 kernels, 16.8 here)
+    {4, 32, 0, 1, 2, kFamDiag},             // groups of 32: two tokens x eight groups as MFMA rows (K a multiple of 256; two rows of
+                                            // another K: the dot2 kernels, see dot2_rows)
     {8, 64, 0, 1, 4, kFamDiag},             // up to four rows of 8-bit codes, K of 2048, 4096 or 8192, up to 40 Mi codes (where
                                             // measured ahead of the next two rules, see qmvd_pick); a row of such a call
                                             // has the bytes of a call with that row alone
@@ -274,9 +274,10 @@ const QmvRule kQmvRules[] = {
                                             // calls have passed, e.g. on operands that are not 16-byte aligned, or with the
                                             // diagonal and dot2 families switched off: this kernel is faster at long K,
                                             // 15.6 against 2 x 9 us at 8 rows of 14336 x 4096, but not row by row the same bytes)
-    {4, 32, 0, 2, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
+    {4, 32, 0, 3, 32, kFamTok},             // groups of 32 (GGUF-derived layouts): a step of the MFMA is one group
     {8, 32, 0, 2, 32, kFamTok},
-    {0, 128, 0, 2, 32, kFamTok},            // (2..4 rows of a layer of 2048 / 7168 29-32 us on the block-MFMA kernels, 19-21 here, of 8 bit 26-30 / 19-21)
+    {0, 128, 0, 2, 32, kFamTok},            // (2..4 rows of a layer of 2048 / 7168 29-32 us on the block-MFMA kernels, 19-21 here; where the
+                                            // dot2 kernels give them the bytes of single-row calls, dot2_rows, they stay there)
     {0, 0, 0, 33, 64, kFamTok},
     {0, 0, 0, 9, 64, kFamTilesLarge},       // 16 Mi codes and more: the 16-row block-MFMA kernel is bound by its 4x4x4 MFMAs
     {0, 0, 0, 2, 16, kFamBlk},              // the whole call in one launch of up to 16 rows (4 where K is long)
@@ -397,10 +398,26 @@ int tok_pick(const aq_ctx* ctx, const aq::TokArgs& t, int group_size, int bits, 
     return aq::qmvt_pick(bits, group_size, t.M, t.K, &part, 1, pair, ctx->cu_count);
 }
 
-// Two to four rows of x that other kernels keep: two rows in groups of 32 at a K of whole steps of the diagonal kernels, where a row
-// has the bytes of a call with that row alone, and groups of 128 beyond 64 Mi codes, as far as both sides were timed.
-bool tok_few(int bits, int group_size, int M, int K, int64_t rows) {
-    return (bits == 4 && group_size == 32 && M == 2 && K % 256 == 0) || (group_size == 128 && M <= 4 && rows * K > (int64_t)64 << 20);
+// Two to four rows of x in groups of 128 that other kernels keep: matrices beyond 64 Mi codes, as far as both sides were timed.
+bool tok_few(int group_size, int M, int K, int64_t rows) { return group_size == 128 && M <= 4 && rows * K > (int64_t)64 << 20; }
+
+// Whether several rows of x run on the dot2 kernels, four a launch, where a row has the bytes of a call with that row alone: groups
+// of 64 at a K that the diagonal kernels do not take, two to eight rows of 4-bit codes, two to four of 8 bit where the matrix is small
+// (tok_small); two rows of 4 bit in groups of 32 at such a K; two to four rows in groups of 128 but for the shapes of the block-MFMA
+// kernels, which never gave them those bytes (4 bit, K a multiple of 512, a multiple of four rows of weights; token tiles now).
+// The bytes decide for groups of 32 and 128, not the time.  (us, one by one with a pair as three launches / a grid or a pair here / token
+// tiles: two rows by 4096 / 1024 / 1024, 4 bit, groups of 32, K of 1216 10.1 / 4.8 / 5.7, of 14528 35.6 / 26.4 / 23.0; four rows in groups
+// of 128, K of 1152 12.2 / 6.2 / 5.1, of 7296 27.4 / 18.9 / 12.7, 8 bit, K of 4096 20.5 / 11.4 / 10.7, of 14336 68 / 53 / 27.)
+bool dot2_rows(const aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits) {
+    const int M = a.M, K = a.K;
+    if (M < 2 || ctx->forced[0] >= 0 || (ctx->families_off >> kFamDot2 & 1) || (bits != 4 && bits != 8)) return false;
+    if (group_size == 64 && (bits == 8 ? M > 4 || !tok_small(8, 64, M, K, a.N) : M > 8 || aq::qmvd_pick(1, K, 1) >= 0)) return false;
+    if (group_size == 32 && (bits == 8 || M > 2 || K % 256 == 0)) return false;
+    if (group_size == 128) {
+        aq::BlkPlan plan;
+        if (M > 4 || (!(ctx->families_off >> kFamBlk & 1) && aq::qmvb_plan(a, bits, group_size, false, ctx->cu_count, -1, &plan))) return false;
+    }
+    return dot2_eligible(K, group_size, bits, a.x, a.w, (size_t)(M < 4 ? M : 4) * K * 2);
 }
 
 int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool gather, int forced) {
@@ -408,7 +425,7 @@ int run_tok(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool ga
     aq::TokArgs t{a};
     t.ksplit = 1;
     t.tokens = forced < 0 ? aq::qmvt_tokens(a.M) : a.M;
-    const bool left = tok_small(bits, group_size, a.M, a.K, a.N) || tok_few(bits, group_size, a.M, a.K, a.N);
+    const bool left = tok_small(bits, group_size, a.M, a.K, a.N) || tok_few(group_size, a.M, a.K, a.N) || dot2_rows(ctx, a, group_size, bits);
     if (forced < 0 && !left && tok_halves(ctx, group_size, a.M, a.N, false)) {
         aq::qmvt_split(bits, group_size, a.M, a.K, a.N, false, ctx->cu_count, &t.ksplit, &t.share);
     } else if (forced < 0) {
@@ -470,22 +487,15 @@ int launch_qmv_rows(aq_ctx* ctx, aq::QmvArgs a, int group_size, int bits, bool g
     return fail(AQ_ERR_UNSUPPORTED, "aq_qmv: no kernel for bits=%d group=%d rows=%d K=%d N=%d", bits, group_size, a.M, a.K, a.N);
 }
 
-// Whether several rows of x run on the dot2 kernels, four a launch: groups of 64 at a K that the diagonal kernels do not take, two to
-// eight rows of 4-bit codes, two to four of 8 bit where the matrix is small (tok_small).
-bool dot2_rows(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, const void* x, const void* w) {
-    if (group_size != 64 || M < 2 || ctx->forced[0] >= 0 || (ctx->families_off >> kFamDot2 & 1)) return false;
-    if (bits == 8 ? M > 4 || !tok_small(8, 64, M, K, rows) : bits != 4 || M > 8 || aq::qmvd_pick(1, K, 1) >= 0) return false;
-    return dot2_eligible(K, group_size, bits, x, w, (size_t)(M < 4 ? M : 4) * K * 2);
-}
-
-// Whether the token-tile kernels run an unforced dense call of this kind on a matrix of `rows` rows (the rules above, for
+// Whether the token-tile kernels run an unforced dense call of this kind, a.w alone or as one of a pair (the rules above, for
 // the launch forms that put several matrices into one grid).
-bool tok_runs(const aq_ctx* ctx, int bits, int group_size, int M, int K, int64_t rows, bool pair) {
-    if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(bits, group_size, M, K, rows)) return false;
-    if (M < 2 || M > 64 || tok_few(bits, group_size, M, K, rows) || !tok_halves(ctx, group_size, M, rows, pair)) return false;
+bool tok_runs(const aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool pair) {
+    const int M = a.M, K = a.K;
+    if (ctx->forced[0] >= 0 || (ctx->families_off >> kFamTok & 1) || tok_small(bits, group_size, M, K, a.N)) return false;
+    if (M < 2 || M > 64 || tok_few(group_size, M, K, a.N) || dot2_rows(ctx, a, group_size, bits) || !tok_halves(ctx, group_size, M, a.N, pair)) return false;
     if (bits == 4 && group_size == 64) return M >= 9;
-    if (bits == 8 && group_size == 64) return M >= 5 || aq::qmvd_pick(M, K, (int)rows, 8) < 0;
-    return true;
+    if (bits == 8 && group_size == 64) return M >= 5 || aq::qmvd_pick(M, K, a.N, 8) < 0;
+    return M >= (bits == 4 && group_size == 32 ? 3 : 2);
 }
 
 size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
@@ -949,8 +959,9 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
         const void *w[aq::kQmvMultiMax], *sc[aq::kQmvMultiMax], *bi[aq::kQmvMultiMax];
         void* to[aq::kQmvMultiMax];
         int n[aq::kQmvMultiMax], some = 0;
+        const aq::QmvMultiArgs all = multi_args(x, count, packed, scales, biases, y, N, M, K, group_size, flags);
         for (int i = 0; i < count; i++) {
-            if (N[i] == 0 || !dot2_rows(ctx, bits, group_size, M, K, N[i], x, packed[i])) continue;
+            if (N[i] == 0 || !dot2_rows(ctx, multi_member(all, i), group_size, bits)) continue;
             w[some] = packed[i], sc[some] = scales[i], bi[some] = biases[i], to[some] = y[i], n[some++] = N[i];
             done |= 1u << i;
         }
@@ -979,7 +990,7 @@ int qmv_multi_call(aq_ctx* ctx, const void* x, int count, const void* const* pac
         grid.common = all.common;
         grid.tokens = aq::qmvt_tokens(M);
         for (int i = 0; i < count; i++) {
-            if (N[i] == 0 || (done >> i & 1) || !aligned(y[i], 2) || !tok_runs(ctx, bits, group_size, M, K, N[i], false)) continue;
+            if (N[i] == 0 || (done >> i & 1) || !aligned(y[i], 2) || !tok_runs(ctx, multi_member(all, i), group_size, bits, false)) continue;
             aq::TokArgs own{multi_member(grid, i)};
             own.tokens = grid.tokens;
             own.w = all.w[i];
@@ -1517,7 +1528,17 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
         gate_packed = w[0], gate_scales = sc[0], gate_biases = bi[0];
         up_packed = w[1], up_scales = sc[1], up_biases = bi[1];
     }
-    const bool pair_rows = M > 1 && dot2_rows(ctx, bits, group_size, M, K, N, x, gate_packed) && dot2_rows(ctx, bits, group_size, M, K, N, x, up_packed);
+    aq::QmvArgs own[2]{};  // the calls of either matrix by itself, as far as the rules look at them
+    for (int i = 0; i < 2; i++) {
+        own[i].x = static_cast<const uint16_t*>(x);
+        own[i].w = static_cast<const uint32_t*>(i ? up_packed : gate_packed);
+        own[i].s = static_cast<const uint16_t*>(i ? up_scales : gate_scales);
+        own[i].b = static_cast<const uint16_t*>(i ? up_biases : gate_biases);
+        own[i].M = M;
+        own[i].K = K;
+        own[i].N = N;
+    }
+    const bool pair_rows = dot2_rows(ctx, own[0], group_size, bits) && dot2_rows(ctx, own[1], group_size, bits);
     if (pair_rows || (M == 1 && ctx->forced[0] < 0 && dot2_eligible(K, group_size, bits, x, gate_packed, (size_t)K * 2) && aligned(up_packed, 16))) {
         const int rows = act_rows(ctx, bits, 1, false, N, K, 1);
         if (aq::qmv_act_supported(bits, 1, rows, false)) {
@@ -1547,7 +1568,7 @@ int aq_qmv_gate_up(aq_ctx* ctx, const void* x, const void* gate_packed, const vo
             return AQ_OK;
         }
     }
-    if (M > 1 && tok_runs(ctx, bits, group_size, M, K, N, true)) {
+    if (tok_runs(ctx, own[0], group_size, bits, true) && tok_runs(ctx, own[1], group_size, bits, true)) {
         // the token-tile kernels with half of a workgroup's rows in either matrix
         aq::TokArgs a{};
         a.x = static_cast<const uint16_t*>(x);

@@ -1,5 +1,5 @@
 """Matrices of up to 528 rows in whole sets of 16 on the token tiles: k and v beside q in one grid with the bytes of their own calls, at
-the numbers of rows of x where a call changes form; groups of 128 and of 32 from two rows on."""
+the numbers of rows of x where a call changes form; groups of 128 from two rows on (4 bit, K a multiple of 512), of 32 from three."""
 import numpy as np
 import pytest
 
@@ -11,8 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("bits,gs,M,K,Ns", [(4, 64, 9, 1216, (1040, 448, 528)), (4, 64, 32, 832, (640, 16, 512)), (4, 64, 33, 2048, (2064, 512, 256)),
                                             (8, 64, 64, 1216, (1536, 448, 448)), (4, 32, 48, 960, (600, 256, 528)), (8, 32, 40, 512, (544, 512, 512)),
-                                            (4, 128, 2, 1152, (1537, 384, 33)), (8, 128, 4, 896, (1024, 256, 7)), (4, 128, 64, 384, (531, 512, 272)),
-                                            (4, 32, 2, 1216, (1537, 448, 33))])
+                                            (4, 128, 2, 1536, (1536, 384, 32)), (8, 128, 5, 896, (1024, 256, 7)), (4, 128, 64, 384, (531, 512, 272)),
+                                            (4, 32, 3, 1216, (1537, 448, 33))])
 def test_members_beside_a_wide_matrix(ctx, bits, gs, M, K, Ns):
     import aq_mi355
     say("small members", bits, gs, M, K, Ns)
