@@ -149,11 +149,13 @@ int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, c
  * pointers.  Results are byte-identical to `count` separate aq_qmv calls.  This is the no-copy form of
  * running q|k|v or gate|up over model.ConcatQuantRows (go/model/quant_weight.go:32-62): at batch 1 the
  * narrow projections are bound by launch latency, not bandwidth, and one grid over all of them fills
- * the machine.  One launch for one activation row (4-bit codes in groups of 64: up to eight rows, or one launch per four of them where
- * aq_qmv takes as many; 8-bit codes: up to four where every member's own call runs on the diagonal kernels, or those members that run
- * on the dot2 kernels), and for the row counts the token-tile kernels run
- * (see aq_qmv) over those members whose own call runs on them, with one more launch where a member shares K out; other shapes
- * and members are run as separate launches. */
+ * the machine.  One launch for one activation row; for 4-bit codes in groups of 64 with K a multiple of 128 from 1152 on, up to four rows
+ * with K up to 16384 and up to eight with K up to 4096 (five to eight rows of longer K: every member by itself, two launches each); for
+ * 8-bit codes, up to four rows where every member's own call runs on the diagonal kernels.  One launch per four rows over those members
+ * whose own call runs on the dot2 kernels, up to eight rows of 4 bit in groups of 64 (K up to 1024, no multiple of 128, or beyond
+ * 16384), two in groups of 32 (K no multiple of 256), up to four in groups of 128 or of small 8-bit matrices (see aq_qmv).  For the row
+ * counts the token-tile kernels run (see aq_qmv) one launch over those members whose own call runs on them, with one more where a
+ * member shares K out.  Other shapes and members are run as separate launches. */
 int aq_qmv_multi(aq_ctx *ctx, const void *x, int count, const void *const *packed, const void *const *scales,
                  const void *const *biases, void *const *y, const int *N, int M, int K, int group_size, int bits,
                  unsigned flags);
@@ -227,8 +229,9 @@ int aq_gather_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *sc
  * launch go/engine/hip/hip_projection_launch.go:3086-3160, packet contract/launch_abi.hipinc:634-657).
  * gate and up are [N, K*bits/32] with their own scales/biases; for a row-concatenated gate|up slab
  * (model.ConcatQuantRows, go/model/quant_weight.go:32-62) pass the slab for gate and slab + N rows for up.
- * M == 1 with 4/8-bit codes runs as ONE launch that reads every weight once, up to 8 rows of 4-bit group-64 codes (up to 4 of small
- * 8-bit ones with K no multiple of 256) as one or two.  So do rows up to 64 where aq_qmv runs its token-tile kernels, from 33 on reading every
+ * M == 1 with 4/8-bit codes runs as ONE launch that reads every weight once.  So do up to four rows of 4-bit codes in groups of 64 with K
+ * a multiple of 128 from 1152 to 8192 (five to eight: one launch up to K = 4096, two beyond; K from 8193 to 16384: the projections
+ * apart), and up to four rows of what aq_qmv_multi runs on the dot2 kernels (eight of 4 bit in groups of 64: two launches).  So do rows up to 64 where aq_qmv runs its token-tile kernels, from 33 on reading every
  * weight twice, with a second launch where workgroups share a long K out; and more rows on the tiles of aq_qmm behind a pass
  * over x.  Other shapes run the two projections and the element-wise step as separate launches through the context's
  * workspace (which grows on demand like aq_qmm's; not while a capture is open). */

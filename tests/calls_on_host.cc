@@ -336,6 +336,32 @@ static void test_tiles_of_prompts() {
     CHECK(aq_qmm_multi(ctx, X, 3, w, s, b, y, wide, 1966, 1920, 32, 4, 0) == AQ_OK && log_.size() == 2, "q|k|v of 1966 rows: %zu launches", log_.size());
 }
 
+// What include/aq_mi355.h says of the launches of a few rows: of q|k|v, and of the gated pair (0: the projections apart).
+static void test_launches_of_few_rows() {
+    struct Case {
+        int bits, group, M, K, members, pair;
+    };
+    static const Case cases[] = {
+        {4, 64, 1, 4096, 1, 1}, {4, 64, 4, 1152, 1, 1}, {4, 64, 4, 8192, 1, 1}, {4, 64, 4, 16384, 1, 0}, {4, 64, 2, 8320, 1, 0}, {4, 64, 5, 1152, 1, 1},
+        {4, 64, 8, 4096, 1, 1}, {4, 64, 5, 4224, 6, 2}, {4, 64, 8, 8192, 6, 2}, {4, 64, 8, 8320, 6, 0}, {4, 64, 6, 16384, 6, 0}, {4, 64, 4, 1024, 1, 1},
+        {4, 64, 8, 1024, 2, 2}, {4, 64, 5, 4160, 2, 2}, {4, 64, 8, 16448, 2, 2}, {4, 64, 3, 14400, 1, 1}, {4, 32, 2, 1216, 1, 1}, {4, 32, 2, 1536, 3, 0},
+        {4, 128, 4, 1152, 1, 1}, {4, 128, 4, 2048, 1, 1}, {8, 128, 4, 2048, 1, 1}, {8, 64, 4, 896, 1, 1}, {8, 64, 4, 4096, 1, 0}, {8, 64, 4, 3072, 1, 1},
+        {8, 64, 5, 4096, 1, 1}, {4, 64, 32, 4096, 1, 1}, {4, 32, 3, 1216, 1, 1}};
+    for (const Case& c : cases) {
+        const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+        void* y[3] = {Y, Y, Y};
+        const int N[3] = {2048, 512, 512};
+        log_.clear();
+        CHECK(aq_qmv_multi(ctx, X, 3, w, s, b, y, N, c.M, c.K, c.group, c.bits, 0) == AQ_OK && (int)log_.size() == c.members,
+              "q|k|v, %d bit, groups of %d, %d rows of %d: %zu launches", c.bits, c.group, c.M, c.K, log_.size());
+        log_.clear();
+        CHECK(aq_qmv_gate_up(ctx, X, W, S, B, W, S, B, Y, c.M, c.K, 2048, c.group, c.bits, AQ_ACT_SILU, 0) == AQ_OK, "%s", aq_last_error());
+        const bool apart = log_.back().is("act_mul");
+        CHECK(apart ? c.pair == 0 : (int)log_.size() == c.pair, "gate|up, %d bit, groups of %d, %d rows of %d: %zu launches, the last %s", c.bits, c.group,
+              c.M, c.K, log_.size(), log_.back().kernel.c_str());
+    }
+}
+
 int main() {
     for (int cus : {128, 512, 256}) {
         compute_units = cus;
@@ -344,7 +370,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities(), test_tiles_of_prompts();
+        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities(), test_tiles_of_prompts(), test_launches_of_few_rows();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");
