@@ -3,6 +3,7 @@
 // without a GPU.  The definitions here take the place of the runtime's when the program loads libaq_mi355.so.
 #include "aq_kernels.h"
 #include "aq_mi355.h"
+#include "aq_qmm.h"
 
 #include <dlfcn.h>
 #include <hip/hip_runtime_api.h>
@@ -24,6 +25,7 @@ struct Launch {
     std::string kernel;
     aq::TokArgs tok;  // of the token-tile kernels
     aq::TokMultiArgs multi;
+    aq::QmmHalfArgs half;  // of the fp16-operand tiles
     bool is(const char* part) const { return kernel.find(part) != std::string::npos; }
 };
 static std::vector<Launch> log_;
@@ -69,9 +71,10 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* fn, dim3, dim3, void** args, size_t, hipStream_t) {
     std::lock_guard<std::mutex> lk(log_mu);
-    Launch l{this_thread, this_call, names()[fn], {}, {}};
+    Launch l{this_thread, this_call, names()[fn], {}, {}, {}};
     if (l.is("qmv_tok16_kernel")) l.tok = *static_cast<const aq::TokArgs*>(args[0]);
     if (l.is("qmv_tok16_multi_kernel")) l.multi = *static_cast<const aq::TokMultiArgs*>(args[0]);
+    if (l.is("qmmh_kernel")) l.half = *static_cast<const aq::QmmHalfArgs*>(args[0]);
     log_.push_back(l);
     return hipSuccess;
 }
@@ -336,6 +339,60 @@ static void test_tiles_of_prompts() {
     CHECK(aq_qmm_multi(ctx, X, 3, w, s, b, y, wide, 1966, 1920, 32, 4, 0) == AQ_OK && log_.size() == 2, "q|k|v of 1966 rows: %zu launches", log_.size());
 }
 
+// Who adds the shares of K in the calls of tests/test_gpu_share_sums.py: of each of the members, the last workgroup of a tile (T), a
+// second kernel (K), or nobody (-).
+static void test_who_adds_shares() {
+    struct Case {
+        int bits, group, M, K, N[3];
+        const char* adds;
+    };
+    static const Case cases[] = {
+        {4, 64, 65, 4096, {515, 130, 64}, "KKK"}, {4, 32, 96, 3840, {1100, 33, 257}, "KKK"}, {4, 128, 129, 8192, {1024, 512, 31}, "KKK"},
+        {8, 64, 66, 3072, {3072, 96, 1000}, "KKK"}, {8, 32, 200, 2048, {640, 513, 64}, "TTT"}, {4, 64, 300, 2816, {704, 2050, 1}, "KKK"},
+        {4, 32, 500, 8192, {2048, 72, 95}, "KKK"}, {8, 64, 777, 10240, {2560, 256, 17}, "KKK"}, {4, 64, 129, 2816, {3072, 96, 1000}, "TKK"},
+        {4, 32, 300, 2048, {4096, 1024, 33}, "-TT"}, {4, 128, 777, 2048, {1100, 33, 257}, "TKK"}, {4, 64, 500, 4096, {3072, 96, 1000}, "TKK"},
+        {4, 64, 777, 2048, {4096, 1024, 33}, "-TK"}, {8, 64, 300, 4096, {2048, 513, 513}, "TKK"}, {8, 32, 500, 2816, {3072, 96, 1000}, "-TK"}};
+    for (const Case& c : cases) {
+        const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+        void* y[3] = {Y, Y, Y};
+        log_.clear();
+        CHECK(aq_qmm_multi(ctx, X, 3, w, s, b, y, c.N, c.M, c.K, c.group, c.bits, 0) == AQ_OK && log_.size() >= 2 && log_[1].is("qmmh_kernel"), "%s", aq_last_error());
+        std::string adds;
+        for (int i = 0; i < 3; i++) adds += !log_[1].half.seg[i].partial ? '-' : log_[1].half.seg[i].tickets ? 'T' : 'K';
+        CHECK(adds == c.adds && log_.size() == (adds.find('K') == std::string::npos ? 2 : 3), "%d bit, %d rows of %d: %s, %zu launches", c.bits, c.M, c.K, adds.c_str(),
+              log_.size());
+    }
+}
+
+// A recorded call whose workspace holds a member at a time, not the grid: one pass over x, and a launch that clears the tickets ahead of a later
+// member's tiles (tests/test_gpu_share_sums.py runs it).
+static void test_tickets_of_members_one_by_one() {
+    aq_ctx* own = nullptr;
+    CHECK(aq_create(0, &own) == AQ_OK, "%s", aq_last_error());
+    const void *w[3] = {W, W, W}, *s[3] = {S, S, S}, *b[3] = {B, B, B};
+    void* y[3] = {Y, Y, Y};
+    const int N[3] = {515, 500, 130};
+    CHECK(aq_qmm(own, X, W, S, B, Y, 65, 2048, N[0], 64, 4, 0) == AQ_OK, "%s", aq_last_error());
+    log_.clear();
+    capturing = true;
+    CHECK(aq_qmm_multi(own, X, 3, w, s, b, y, N, 65, 2048, 64, 4, 0) == AQ_OK, "%s", aq_last_error());
+    capturing = false;
+    std::string kernels;
+    for (const Launch& l : log_) kernels += l.is("prep") ? 'x' : l.is("qmmh_kernel") ? l.half.seg[0].tickets ? 'T' : '-' : l.is("fill") ? '0' : '?';
+    CHECK(kernels == "xT0T0T", "%s, the last %s", kernels.c_str(), log_.back().kernel.c_str());
+    aq_destroy(own);
+}
+
+// The list of an expert block's routes: beside the pass over x while it takes up to 40 KiB of LDS, behind that a launch of its own.
+static void test_lists_of_routes() {
+    for (auto [routes, launches] : {std::array{5056, 2}, {5057, 3}}) {
+        log_.clear();
+        CHECK(aq_gather_qmv_gate_up(ctx, X, W, S, B, static_cast<int32_t*>(S), static_cast<int32_t*>(S), Y, routes, 1000, 256, 776, 128, 2 * 776, 0, 776, 64, 4, AQ_ACT_SILU, 0) == AQ_OK,
+              "%s", aq_last_error());
+        CHECK((int)log_.size() == launches && log_.back().is("qmmr_kernel"), "%d routes: %zu launches, the last %s", routes, log_.size(), log_.back().kernel.c_str());
+    }
+}
+
 // What include/aq_mi355.h says of the launches of a few rows: of q|k|v, and of the gated pair (0: the projections apart).
 static void test_launches_of_few_rows() {
     struct Case {
@@ -370,7 +427,7 @@ int main() {
             return 1;
         }
         test_shares();
-        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities(), test_tiles_of_prompts(), test_launches_of_few_rows();
+        if (cus == 256) test_calls_stay_whole(), test_shares_inside(), test_shares_of_pairs(), test_shares_of_the_infinities(), test_tiles_of_prompts(), test_launches_of_few_rows(), test_who_adds_shares(), test_tickets_of_members_one_by_one(), test_lists_of_routes();
         aq_destroy(ctx);
     }
     if (!failures) puts("ok");

@@ -1,6 +1,6 @@
 """Shares of K added by the last workgroup of a tile: matrices and pairs at the edges of the tiles (rows and columns that are no whole
-blocks of 32), two to many shares, beside matrices whose shares a second kernel adds; the same bytes in every repetition, between other
-calls over the same workspace, from a call of the matrix alone and from replays of a graph."""
+blocks of 32), two to many shares, beside matrices whose shares a second kernel adds (which of the members: tests/calls_on_host.cc); the
+same bytes in every repetition, between other calls over the same workspace, from a call of the matrix alone and from replays of a graph."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,9 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("bits,gs,M,K,Ns", [(4, 64, 65, 4096, (515, 130, 64)), (4, 32, 96, 3840, (1100, 33, 257)), (4, 128, 129, 8192, (1024, 512, 31)),
                                             (8, 64, 66, 3072, (3072, 96, 1000)), (8, 32, 200, 2048, (640, 513, 64)), (4, 64, 300, 2816, (704, 2050, 1)),
-                                            (4, 32, 500, 8192, (2048, 72, 95)), (8, 64, 777, 10240, (2560, 256, 17))])
+                                            (4, 32, 500, 8192, (2048, 72, 95)), (8, 64, 777, 10240, (2560, 256, 17)), (4, 64, 129, 2816, (3072, 96, 1000)),
+                                            (4, 32, 300, 2048, (4096, 1024, 33)), (4, 128, 777, 2048, (1100, 33, 257)), (4, 64, 500, 4096, (3072, 96, 1000)),
+                                            (4, 64, 777, 2048, (4096, 1024, 33)), (8, 64, 300, 4096, (2048, 513, 513)), (8, 32, 500, 2816, (3072, 96, 1000))])
 def test_repeated(ctx, bits, gs, M, K, Ns):
     import aq_mi355
     say("share sums", bits, gs, M, K, Ns)
@@ -55,3 +57,38 @@ def test_repeated(ctx, bits, gs, M, K, Ns):
     ctx.graph_destroy(graph)
     for t in [dx, gated] + ys + dws:
         t.free()
+
+
+def test_members_one_by_one():
+    """A recorded call whose workspace holds a member at a time: the tickets of a later member are cleared by a launch of their own
+    (tests/calls_on_host.cc looks at the launches), in every replay, whatever the workspace holds by then."""
+    import aq_mi355
+    M, K, Ns = 65, 2048, (515, 500, 130)
+    say("share sums one by one")
+    c = aq_mi355.Context(0)
+    try:
+        x = F.synthetic_x(M, K, seed=3500)
+        mats = [F.synthetic_affine(n, K, 4, 64, seed=3501 + i) for i, n in enumerate(Ns)]
+        dws = [DeviceAffine(c, *m) for m in mats]
+        want = [run_qmv(c, x, d, M, K, n, 64, 4, True, fn="qmm") for d, n in zip(dws, Ns)]
+        for m, got in zip(mats, want):
+            check_accumulators(got, F.reference_f64(x, *m, 4, 64, K), "a member alone")
+        dx, ys = c.to_device(x), [c.alloc(M * n * 4) for n in Ns]
+        before = c.workspace_bytes()
+        c.capture_begin()
+        c.qmm_multi(dx, [d.w for d in dws], [d.s for d in dws], [d.b for d in dws], ys, list(Ns), M, K, 64, 4, aq_mi355.AQ_OUT_F32)
+        graph = c.capture_end()
+        assert c.workspace_bytes() == before
+        for _ in range(4):
+            for y in ys:
+                c.fill_zero(y)
+            c.graph_launch(graph)
+            c.sync()
+            for y, n, one in zip(ys, Ns, want):
+                assert np.array_equal(y.download(np.uint32, M * n), one.view(np.uint32).reshape(-1))
+            run_qmv(c, x[::-1], dws[0], M, K, Ns[0], 64, 4, True, fn="qmm")  # other contents for the workspace
+        c.graph_destroy(graph)
+        for t in [dx] + ys + dws:
+            t.free()
+    finally:
+        c.close()
