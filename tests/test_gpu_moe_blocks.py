@@ -14,7 +14,9 @@ pytestmark = pytest.mark.gpu
 # routes, experts, K, N (1.4 tiles a CU of 256 columns and more)
 @pytest.mark.parametrize("gs,routes,E,K,N,skew", [(64, 260, 80, 256, 1030, False), (64, 1900, 80, 320, 1033, False), (64, 700, 128, 704, 776, True),
                                                   (64, 2600, 80, 1088, 1030, True), (32, 1900, 80, 128, 1030, False), (32, 1200, 100, 576, 1028, True),
-                                                  (128, 1900, 80, 640, 1030, False), (128, 1500, 100, 2176, 1024, False)])
+                                                  (128, 1900, 80, 640, 1030, False), (128, 1500, 100, 2176, 1024, False),
+                                                  # the longest list beside the pass over x, and one in a launch of its own (tests/calls_on_host.cc)
+                                                  (64, 5056, 128, 256, 776, False), (64, 5057, 128, 256, 776, True)])
 def test_blocks(ctx, orc, gs, routes, E, K, N, skew):
     grouped.test_grouped_gather(ctx, orc, 4, gs, routes, E, K, N, skew)
     assert ctx.last_variant(0) == "gather_gate_up_grouped_blocks", ctx.last_variant(0)
