@@ -156,8 +156,8 @@ size_t qmmh_partial_most(int M, int K, int cu_count);
 // Routes grouped by expert on tiles of up to 48 routes in blocks of 16 (aq_qmm_routes.hip), 4-bit codes.
 constexpr int kRouteRows = 48;  // routes of a chunk
 struct QmmRouteArgs {
-    const uint16_t* xf;  // [rows][K up to a multiple of 128] fp16
-    const uint32_t* xs;  // [rows][groups up to a multiple of 512 codes] sums of x, two bf16 each
+    const uint16_t* xf;  // [rows][K up to a multiple of 256] fp16
+    const uint32_t* xs;  // [rows][groups up to a multiple of 16] sums of x, two bf16 each
     const float* rs;     // [rows] the inverse of the power of two a row was scaled by
     const uint32_t* w;
     const uint16_t *s, *b;
