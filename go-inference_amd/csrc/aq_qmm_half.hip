@@ -27,6 +27,7 @@
 // one workgroup per row so that the row's largest magnitude is known), A tiles and PACKED weights copied
 // global -> LDS by copy instructions three blocks deep, one barrier per block, XCD-aware tile order.
 #include "aq_device.h"
+#include "aq_fp16_operands.h"
 #include "aq_kernels.h"
 #include "aq_lds_copy.h"
 #include "aq_qmm.h"
@@ -65,28 +66,6 @@ __device__ __forceinline__ f16x8_t expand_bytes(uint2 w) {
     return __builtin_bit_cast(f16x8_t, u);
 }
 
-// the value of lane `lane ^ BIT`
-template <int BIT>
-__device__ __forceinline__ float lane_xor(float v) {
-    const int i = __float_as_int(v);
-    if constexpr (BIT == 1) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0xb1, 0xf, 0xf, false));  // quad_perm 1 0 3 2
-    if constexpr (BIT == 2) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x4e, 0xf, 0xf, false));  // quad_perm 2 3 0 1
-    if constexpr (BIT == 4) return __int_as_float(__builtin_amdgcn_ds_swizzle(i, 0x101f));
-    if constexpr (BIT == 8) return __int_as_float(__builtin_amdgcn_mov_dpp(i, 0x128, 0xf, 0xf, false));  // row_ror 8
-    if constexpr (BIT == 16) return __int_as_float(__builtin_amdgcn_permlane16_swap(i, i, false, false)[(threadIdx.x >> 4 & 1) ^ 1]);
-    return __int_as_float(__builtin_amdgcn_permlane32_swap(i, i, false, false)[(threadIdx.x >> 5 & 1) ^ 1]);
-}
-
-// the largest value of the lanes that are BIT, 2 BIT, ... apart (by shuffles through LDS: 29 layers of 66 to 414 rows 0.6 % slower)
-template <int BIT>
-__device__ __forceinline__ uint32_t max_lanes(uint32_t v) {
-    if constexpr (BIT < kWave) {
-        v = max(v, __float_as_uint(lane_xor<BIT>(__uint_as_float(v))));
-        return max_lanes<2 * BIT>(v);
-    }
-    return v;
-}
-
 typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ uint32_t max_u16x2(uint32_t a, uint32_t b) {
     return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
@@ -122,19 +101,6 @@ __device__ __forceinline__ uint4 moved_down(uint4 v, uint32_t off, uint32_t tota
     return make_uint4(__builtin_amdgcn_alignbit(v.y, v.x, half), __builtin_amdgcn_alignbit(v.z, v.y, half), __builtin_amdgcn_alignbit(v.w, v.z, half),
                       v.w >> half);
 }
-
-__device__ __forceinline__ uint32_t dup16(uint32_t h) { return (h & 0xffffu) | (h << 16); }
-
-// 2^e for the largest finite magnitude `mag` (bf16 bits without the sign) such that mag * 2^e has binary
-// exponent `target`; 1 for an all-zero row.  e is kept inside what fp32 powers of two hold.
-__device__ __forceinline__ int exponent_shift(uint32_t mag, int target) {
-    if (mag == 0) return 0;
-    int e = target + 127 - (int)(mag >> 7);
-    e = e > 120 ? 120 : e;
-    e = e < -120 ? -120 : e;
-    return e;
-}
-__device__ __forceinline__ float pow2f(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
 
 }  // namespace
 

@@ -21,6 +21,7 @@
 // in 90 us, 4.9 TB/s; vector issue 45 % of SIMD cycles, matrix cores 20 %.  The first 10 us of a round are its first lines on their way,
 // of all tiles at once.  Codes with the non-temporal hint: 194 -> 198 us the block.
 #include "aq_device.h"
+#include "aq_fp16_operands.h"
 #include "aq_kernels.h"
 #include "aq_lds_copy.h"
 #include "aq_moe_group.h"
@@ -46,13 +47,6 @@ constexpr int kThreads = 256, kWaves = kThreads / kWave;
 constexpr int kCols = kWaves * 64;
 constexpr int kStage = 16 * kStep * 2;  // bytes of 16 rows of x
 
-__device__ __forceinline__ int shift_to(uint32_t mag, int target) {
-    if (mag == 0) return 0;
-    const int e = target + 127 - (int)(mag >> 7);
-    return e > 120 ? 120 : e < -120 ? -120 : e;
-}
-__device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(127 + e) << 23); }
-__device__ __forceinline__ uint32_t dup16(uint32_t h) { return (h & 0xffffu) | (h << 16); }
 // A load at a uniform base and a 32-bit offset of the lane.  (The offset is hidden from the compiler, which would carry a 64-bit address
 // per load through the loop: 36 registers of 154 with one row block.)
 __device__ __forceinline__ uint32_t hidden(uint32_t v) {
@@ -110,11 +104,10 @@ __global__ __launch_bounds__(kPrepThreads) void qmmr_prep_kernel(const uint16_t*
 #pragma unroll
         for (int i = 0; i < HOLD; i++) mag = most_of(most_of(most_of(most_of(mag, hold[i].x), hold[i].y), hold[i].z), hold[i].w);
     }
-#pragma unroll
-    for (int o = 1; o < kWave; o <<= 1) mag = max(mag, (uint32_t)__shfl_xor((int)mag, o, kWave));
-    const int e = shift_to(mag, 14);
-    const float up = pow2(e);
-    if (lane == 0) rs[row] = pow2(-e);
+    mag = max_lanes<1>(mag);
+    const int e = exponent_shift(mag, 14);
+    const float up = pow2f(e);
+    if (lane == 0) rs[row] = pow2f(-e);
     uint16_t* const to = xf + (int64_t)row * padded * 8;
     uint32_t* const sums = xs + (int64_t)row * (all * 8 / GRP);
     for (int p0 = 0; p0 < all; p0 += HOLD * kWave) {
@@ -291,10 +284,7 @@ __global__ __launch_bounds__(kThreads, GRP == 32 ? 2 : 3) void qmmr_kernel(const
     uint32_t up = 0;  // its biased exponents, a byte for each column block
 #pragma unroll
     for (int cg = 0; cg < 4; cg++) {
-        uint32_t m = mag[cg];
-        m = max(m, (uint32_t)__shfl_xor((int)m, 16, kWave));
-        m = max(m, (uint32_t)__shfl_xor((int)m, 32, kWave));
-        up |= (uint32_t)(127 + shift_to(m, 10)) << (8 * cg);
+        up |= (uint32_t)(127 + exponent_shift(max_lanes<16>(mag[cg]), 10)) << (8 * cg);
     }
     auto col_up = [&](int cg) { return __uint_as_float((hidden(up) >> (8 * cg) & 0xffu) << 23); };
     const uint32_t mask_s = opaque_s(0x03C003C0u), magic_v = opaque_v(0x4C004C00u);
