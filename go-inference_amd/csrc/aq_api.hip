@@ -360,10 +360,11 @@ int run_diag(aq_ctx* ctx, const aq::QmvArgs& a, int group_size, int bits, bool g
 // families behind.  8 bit: up to four rows, where the dot2 kernels are ahead (us, dot2 / here: 2 rows of 960 x 512 2.8 / 4.5, of
 // 4032 x 1024 4.4 / 6.7; 4 rows 3.2 / 4.5, 5.8 / 7.0); from five rows on what is behind are tiles, a pass over x and a sum of
 // shares of K in three launches (8 rows 14.6 / 4.6, 17.6 / 7.3; 32 rows 15.0 / 6.7, 18.1 / 11.9).  4 bit: up to 528 rows of
-// weights that are no whole sets of 16; the tiles are behind there as well (9 rows of x by 960 x 512 13.6 / 4.6, by 960 x 2048 14.3 /
-// 4.6, 32 by 4032 x 1024 17.4 / 11.1), but the choice is one that tests/test_gpu_selection.py states, at 520 rows.  Whole sets, what k
-// and v of a layer have, run here, in one grid with q (a layer of 1216 / 4032 with 448 rows of k and v, tiles / here: 9 rows of x
-// 30.0 / 17.6, 32 rows 35.9 / 20.6).
+// weights that are no whole sets of 16, which tests/test_gpu_selection.py states for 520 of them; neither the time nor the width is a
+// reason: the token tiles are ahead at every one (us, tiles / here, ragged 17, 203, 450, 520 rows and whole sets 48, 256, 512: 9 rows of
+// x, K of 1216 11.3 / 3.5, 12.2 / 3.6, 12.7 / 3.8, 12.5 / 3.9 and 11.5 / 3.6, 11.8 / 3.5, 12.2 / 3.8; 32 rows, K of 4032 14.2 / 10.0, 16.8 /
+// 10.2, 19.2 / 10.2, 17.2 / 10.2 and 13.6 / 10.1, 16.6 / 10.1, 17.4 / 10.2).  Whole sets, what k and v of a layer have, run here, in one
+// grid with q (a layer of 1216 / 4032 with 448 rows of k and v, tiles / here: 9 rows of x 30.0 / 17.6, 32 rows 35.9 / 20.6).
 bool tok_small(int bits, int group_size, int M, int K, int64_t rows) {
     return group_size == 64 && K % 256 != 0 && rows * K < (int64_t)4 << 20 && (bits == 8 ? M <= 4 : rows <= 528 && rows % 16 != 0);
 }
@@ -373,10 +374,12 @@ bool tok_small(int bits, int group_size, int M, int K, int64_t rows) {
 // two rounds they are ahead where the tiles are the slow ones, gate and up in groups of 64 (4096 x 14336 4 bit 52.7 / 43.6, 8 bit
 // 59.1 / 54.7) and groups of 128 (4096 x 28672 51.0 / 43.7), and behind elsewhere (4096 x 28672 groups of 64 41.7 / 44.0, 8 bit
 // 52.4 / 54.4, groups of 32 49.3 / 59.0, 60.6 / 62.6; gate and up in groups of 32 47.7 / 59.3).  Matrices of up to 528 rows that are no
-// whole sets of 16, and those of fewer than 256, stay with the tiles, choices that tests/test_gpu_selection.py (520 rows) and
-// tests/test_gpu_fused_act.py (pairs of 96, and their own calls) state; k and v of a layer are larger whole
-// sets (a layer of 2048 / 7168 with 512 rows of them, 48 rows of x, tiles / halves: 45.6 / 27.5, groups of 32 53.5 / 32.4, of 128 52.6
-// / 27.5, 8 bit 46.3 / 30.1; of 1216 / 4032 with 448, 8 bit, 64 rows 55.9 / 24.0).
+// whole sets of 16, and those of fewer than 256, stay with the tiles: tests/test_gpu_selection.py (520 rows) and
+// tests/test_gpu_fused_act.py (pairs of 77, 96 and 300) state it, the time does not (ragged 17, 203, 450, 520 rows and whole sets 48, 256,
+// 512, 64 rows of x, K of 4096: 14.8 / 10.4, 18.4 / 10.6, 21.8 / 10.7, 17.4 / 10.7 and 14.3 / 10.5, 16.5 / 10.5, 17.5 / 10.6, 8 bit 14.3 / 11.1 to
+// 17.2 / 11.4 and 13.6 / 11.2 to 15.5 / 11.3, groups of 32 17.2 / 12.0 to 20.7 / 12.3 and 16.2 / 12.1 to 18.9 / 12.3; pairs of 48 to 520, 40 rows
+// of x, K of 2048 24-29 / 7.3).  k and v of a layer are larger whole sets (a layer of 2048 / 7168 with 512 rows of them, 48 rows of x, tiles /
+// halves: 45.6 / 27.5, groups of 32 53.5 / 32.4, of 128 52.6 / 27.5, 8 bit 46.3 / 30.1; of 1216 / 4032 with 448, 8 bit, 64 rows 55.9 / 24.0).
 bool tok_halves(const aq_ctx* ctx, int group_size, int M, int64_t rows, bool pair) {
     if (M <= 32) return true;
     if (rows <= 528 && (rows < 256 || rows % 16 != 0)) return false;

@@ -135,12 +135,12 @@ int aq_probe_read(aq_ctx *ctx, const void *packed, const void *scales, const voi
  * form (go/engine/metal/qmv_rows.go:14-60).  M >= 1; rows of x are contiguous.
  * N == 0 or K == 0 is a no-op returning AQ_OK (qmv.go:365-371).
  * 4- and 8-bit codes, K a multiple of 64 up to 16384, operands 16-byte aligned: up to 32 rows of x, from 9 on in groups of 64
- * (8 bit: from 2, or 5 where K is 2048, 4096 or 8192), from 5 in groups of 128 (from 2 of 4 bit with K a multiple of 512, N of 4, up to
- * 64 Mi codes), from 3 in groups of 32 (8 bit: 2), the token-tile kernels run the call (small matrices with K no multiple of 256
- * excepted, but for 4 bit in whole sets of 16 rows): one launch, or two where workgroups share a long K out, and a row of x has the same
- * bytes whatever the number of rows beside it.  Fewer rows have the bytes of a call with that row alone (but for 4 bit in groups of 128
- * beyond 64 Mi codes).  33 to 64 rows run there too on matrices of more than 528 rows, or of 256 and more in whole sets
- * of 16, that are not too wide, with the same identity among themselves. */
+ * (8 bit: from 2; up to 40 Mi codes from 3 where K is 2048, from 5 where it is 4096 or 8192), from 5 in groups of 128 (from 2 of 4 bit with K a multiple of 512,
+ * N of 4, up to 64 Mi codes), from 3 in groups of 32 (8 bit: 2), the token-tile kernels run the call (small matrices with K no multiple of
+ * 256 excepted, but for 4 bit in whole sets of 16 rows): one launch, or two where workgroups share a long K out, and a row of x has the
+ * same bytes in every call of so many rows.  A row of a call of fewer has the bytes of a call with that row alone, which are those of
+ * other kernels (4 bit in groups of 128 beyond 64 Mi codes excepted).  33 to 64 rows run there too on matrices of more than 528 rows, or
+ * of 256 and more in whole sets of 16, that are not too wide, with the same identity among themselves. */
 int aq_qmv(aq_ctx *ctx, const void *x, const void *packed, const void *scales, const void *biases, void *y, int M,
            int K, int N, int group_size, int bits, unsigned flags);
 
