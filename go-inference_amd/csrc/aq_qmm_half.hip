@@ -551,7 +551,7 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         }
     };
     // The rows' factors wait in LDS for the epilogue, whose first loads they were, behind all of K and ahead of every store (2048 rows of 4096 /
-    // 14336 949 -> 936 us with the sums of shares, 958 -> 942 by this alone; 40 layers of 66 to 2048 rows 0.7 % faster).
+    // 14336 937 -> 926 us, 777 rows of 8 bit 322 -> 318, 509 rows in groups of 32 359 -> 357; 40 layers of 66 to 2048 rows 0.7 % faster).
     constexpr bool RS_LDS = half_rows_in_lds(BITS, MB, NWAVE);
     static_assert(BM <= THREADS, "a row's factor a thread");
     float* const rbuf = reinterpret_cast<float*>(sbuf + 2 * BN * SE) + (XS_LDS ? BM / 32 * 256 : 0);
@@ -823,7 +823,8 @@ __global__ __launch_bounds__(WM* WN* kWave, 2) void qmmh_kernel(const QmmHalfArg
         a8[t] = *reinterpret_cast<const f16x8_t*>(abuf + stage * A_STAGE + (wave_m * MB + mb) * 4096 + t * 1024 + lane * 16);
     };
     // Row (wave_n * NB + nb) * 32 + j: the sixteen codes of steps 2 i and 2 i + 1, whole 16-byte pieces of 16 rows that lie in different
-    // banks.  (Eight codes a read, one half of each piece: rows j and j + 16 met in the same banks, 13 % of the CU's cycles.)
+    // banks.  (Eight codes a read, one half of each piece: rows j and j + 16 met in the same banks; conflicts took
+    // 13 % of a CU's cycles in gate and up of 777 rows, 6 % so.)
     auto read_codes8 = [&](int i, int stage) __attribute__((always_inline)) {
         const uint8_t* const at = bbuf + (stage * B_STAGE + (wave_n * NB * 32 + j) * B_ROW + (((2 * i + h) ^ turn(j)) * 16));
 #pragma unroll

@@ -17,9 +17,9 @@
 // left each row: that runs over the rows of x as the caller has them, once each however many routes read it, and beside the
 // list of routes (per route and behind the list: 7.8 + 13.9 us of gate and up -> 8.8).
 //
-// Bound (gate and up above): 437 MB past the L2s, 285 of them the weights (the lines of the scales are fetched again in every segment),
-// in 90 us, 4.9 TB/s; vector issue 45 % of SIMD cycles, matrix cores 20 %.  The first 10 us of a round are its first lines on their way,
-// of all tiles at once.  Codes with the non-temporal hint: 194 -> 198 us the block.
+// Bound (gate and up above): 391 MB past the L2s, 285 of them the weights (the lines of the scales are fetched again in every segment),
+// in 88 us, 4.4 TB/s; vector issue 64 % of SIMD cycles, matrix cores 21 %, wavefronts wait 26 % of theirs.  The first 10 us of a round
+// are its first lines on their way, of all tiles at once.  Codes with the non-temporal hint: 194 -> 198 us the block.
 #include "aq_device.h"
 #include "aq_fp16_operands.h"
 #include "aq_kernels.h"
